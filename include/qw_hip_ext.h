@@ -3,14 +3,17 @@
  *
  * Host shadow rules (qw_buf.ptr is host memory, the kernels read HBM):
  *   - host -> device, when a batch is submitted, for every buffer a dispatch of the batch binds:
- *       a buffer of at most QW_HIP_SMALL_BYTES is copied every time;
+ *       a buffer of at most QW_HIP_SMALL_BYTES is copied every time (once its whole has been: the bytes that the batch's
+ *       dispatches can touch; a copy out of HBM, or its address asked for, brings the rest into step first);
  *       a larger one is copied the first time it is bound and again only after qw_hip_buf_mark_dirty();
  *       qw_buf_wrap() buffers are copied once; device-only buffers never;
+ *       not the bytes that the batch's kernels write whole before anything reads them (a product's result, say): what the
+ *       host side held there is about to be replaced;
  *       none of this for a buffer that a submitted batch (or an earlier, flushed part of this one) binds in an
  *       output role and that has not been waited for yet: HBM then holds the newer contents (a layer's output that the
  *       next layer reads), and they stay until the wait copies them back.
- *   - device -> host, when the batch completes, for every buffer bound in an output role:
- *       always, unless the buffer is device-only or larger than QW_HIP_BIG_OUT_BYTES (then: qw_hip_buf_download()).
+ *   - device -> host, when the batch completes, for every buffer bound in an output role: the bytes its dispatches may have
+ *       written, always, unless the buffer is device-only or larger than QW_HIP_BIG_OUT_BYTES (then: qw_hip_buf_download()).
  */
 #pragma once
 #include "gpu.h"

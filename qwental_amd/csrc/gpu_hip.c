@@ -65,6 +65,9 @@ typedef struct qw_hbuf {
     unsigned mark;   // scratch for de-duplication while a batch is submitted
     int pending_out; // submitted batches that bind it in an output role and have not been waited for: HBM is newer than the shadow
     uint64_t out_seq; // the last batch that counted itself in pending_out
+    size_t plo, phi;  // the bytes that those batches' dispatches may write (the least range that holds them all)
+    bool part;        // the last upload carried [slo, shi) only, the bytes its batch could touch: HBM may lack what the host wrote elsewhere
+    size_t slo, shi;
     struct qw_gpu *g;
     int npack;       // packed copies made from this buffer (dropped when its contents change)
     bool released;   // the device bytes were freed (qw_hip_buf_release_source): dptr is only the key of its tile-major copies
@@ -92,7 +95,14 @@ typedef struct {
     bool join; // needs the side stream's results: the main stream waits for them first
 } qw_launch;
 
-typedef struct { qw_hbuf *b; bool out; } qw_use;
+// A buffer as a dispatch binds it, and the bytes it may touch. whole: every byte of [lo, hi) is written, whatever they held.
+typedef struct { qw_hbuf *b; bool out, whole; size_t lo, hi; } qw_use;
+
+// What the host and the device exchange about a batch in flight beside its data: pinned, one per batch at a time. t0 / t1:
+// the device clock at the start and the end of every submitted segment (0: not taken); done, copied: the batch's number
+// once its kernels have finished (where it was submitted without waiting) and once its outputs are in the shadows.
+typedef struct { volatile uint64_t t0[9], t1[9]; volatile uint32_t done, copied; uint32_t pad[26]; } qw_ioslot;
+enum { QW_IO_SLOTS = 32 };
 
 // measurement switches: read from the environment by qw_gpu_open (and again by qw_hip_reload_switches), never per batch
 typedef struct { unsigned dnc_nb, dnq_min, spin_limit, hc_rows; int side, load_threads; bool dn_any, nl_c4, no_swiglu_matvec, shared_in_gu, split_select, pk_split, kq_own, no_fuse, ablate, verbose, quiet; } qw_switches;
@@ -115,8 +125,11 @@ struct qw_batch {
     uint64_t seq;      // this batch's number (qw_hbuf.out_seq)
     qw_hbuf **outs;    // buffers whose pending_out this batch raised
     int nouts, capouts;
-    hipEvent_t ev[2 * 9]; // start/stop per submitted segment (end + at most 8 flushes)
     int nseg;
+    qw_ioslot *io;       // stamps and flags of this batch (NULL until its first submit)
+    int io_idx;
+    hipEvent_t ev[2 * 9]; // profiled batches, and those for which no slot was free: start/stop per submitted segment (end + at most 8 flushes)
+    bool events;
     hipEvent_t *pev;      // profiling: 2 events per launch
     int npev;
     // Work deferred from one dispatch of a layer to the next (the reference's front part also computes the shared
@@ -189,6 +202,11 @@ struct qw_gpu {
     uint32_t *sync_host; // pinned: the error word of those launches, copied back when a batch is waited for
     bool fuse_broken;    // such a launch gave up once: the layers stay separate launches from then on
     float *shgu;         // [2 streams][2][16][QW_SHGU_MAXI] gate and up results of a shared expert in the K-quant format family
+    qw_ioslot *io;       // QW_IO_SLOTS of them, pinned; io_used: bit per slot taken by a batch
+    uint32_t io_used;
+    uint32_t *io_count;  // device: a zero word per slot for qwk_io
+    hipFunction_t io_func;
+    double tick;         // seconds of the device clock's unit
     bool repack;         // make packed copies (QW_HIP_REPACK=0 in the environment or qw_hip_set_repack turn it off)
     size_t pack_bytes, released_bytes;
 };
@@ -292,8 +310,10 @@ qw_gpu *qw_gpu_open(void) {
         if (hipMalloc(&g->tabs, QW_TAB_BYTES) != hipSuccess || hipMemset(g->tabs, 0, QW_TAB_BYTES) != hipSuccess ||
             hipMalloc((void **)&g->shgu, (size_t)2 * 2 * 16 * 4096 * 4) != hipSuccess ||
             hipMalloc((void **)&g->sync, QW_SYNC_ALLOC) != hipSuccess || hipMemset(g->sync, 0, QW_SYNC_ALLOC) != hipSuccess ||
-            hipHostMalloc((void **)&g->sync_host, 64, hipHostMallocDefault) != hipSuccess ||
-            !(f = find_func(g, "qwk_tab_init"))) { free(g->kernels); free(g); return NULL; }
+            hipHostMalloc((void **)&g->sync_host, 64, hipHostMallocCoherent) != hipSuccess ||
+            hipHostMalloc((void **)&g->io, sizeof(qw_ioslot) * QW_IO_SLOTS, hipHostMallocCoherent) != hipSuccess ||
+            hipMalloc((void **)&g->io_count, QW_IO_SLOTS * 4) != hipSuccess || hipMemset(g->io_count, 0, QW_IO_SLOTS * 4) != hipSuccess ||
+            !(g->io_func = find_func(g, "qwk_io")) || !(f = find_func(g, "qwk_tab_init"))) { free(g->kernels); free(g); return NULL; }
         ta = (qwk_tab_args){.tab = g->tabs, .slot_order = 1};
         if (hipDeviceSynchronize() != hipSuccess || hipModuleLaunchKernel(f, 32, 1, 1, 256, 1, 1, 0, g->stream[0], params, NULL) != hipSuccess ||
             hipStreamSynchronize(g->stream[0]) != hipSuccess) {
@@ -302,6 +322,10 @@ qw_gpu *qw_gpu_open(void) {
             free(g);
             return NULL;
         }
+    }
+    {
+        int khz = 0;
+        g->tick = 1e-3 / (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, 0) == hipSuccess && khz > 0 ? khz : 100000);
     }
     // the entry point that allocates nothing: its scratch array's address on this device and its recorder, made now
     if (!qw_noalloc_scratch(g->dev, &g->na_scratch, &g->na_bytes, &g->na_err)) g->na_scratch = NULL;
@@ -350,6 +374,8 @@ void qw_gpu_close(qw_gpu *g) {
     (void)hipFree(g->shgu);
     (void)hipFree(g->sync);
     (void)hipHostFree(g->sync_host);
+    (void)hipHostFree(g->io);
+    (void)hipFree(g->io_count);
     if (g->na_batch) { free(g->na_batch->l); free(g->na_batch->use); free(g->na_batch); }
     (void)hipModuleUnload(g->mod);
     free(g->kernels);
@@ -633,7 +659,7 @@ static qw_hbuf *hbuf_new(qw_gpu *g, size_t size) {
 bool qw_buf_new(qw_gpu *g, size_t size, qw_buf *out) {
     qw_hbuf *h = hbuf_new(g, size);
     if (!h) return false;
-    if (size <= ((size_t)64 << 20) && hipHostMalloc(&h->host, size ? size : 1, hipHostMallocDefault) == hipSuccess) {
+    if (size <= ((size_t)64 << 20) && hipHostMalloc(&h->host, size ? size : 1, hipHostMallocCoherent) == hipSuccess) {
         h->pinned = true;
         memset(h->host, 0, size);
     } else {
@@ -721,8 +747,15 @@ void qw_hip_set_repack(qw_gpu *g, bool on) { g->repack = on; }
 unsigned qw_hip_graph_launches(const qw_gpu *g) { return g->ngraph_launches; }
 void qw_hip_set_graphs(qw_gpu *g, bool on) { g->use_graphs = on; }
 size_t qw_hip_packed_bytes(const qw_gpu *g) { return g->pack_bytes; }
-void *qw_hip_buf_devptr(const qw_buf *b) { return b && b->handle && !((qw_hbuf *)b->handle)->released ? ((qw_hbuf *)b->handle)->dptr : NULL; }
+// Before HBM is looked at from outside a batch: what the host wrote beyond the range of the last upload.
+static bool rest_up(qw_hbuf *h) {
+    if (!h || !h->part || h->pending_out || h->released || h->dirty || !h->host) return true;
+    h->part = false;
+    return (!h->slo || hipMemcpy(h->dptr, h->host, h->slo, hipMemcpyHostToDevice) == hipSuccess) &&
+           (h->shi >= h->size || hipMemcpy((char *)h->dptr + h->shi, (char *)h->host + h->shi, h->size - h->shi, hipMemcpyHostToDevice) == hipSuccess);
+}
 static bool range_ok(const qw_hbuf *h, size_t off, size_t len) { return !h->released && off <= h->size && len <= h->size - off; } // a released buffer has no bytes to copy
+void *qw_hip_buf_devptr(const qw_buf *b) { return b && b->handle && !((qw_hbuf *)b->handle)->released && rest_up(b->handle) ? ((qw_hbuf *)b->handle)->dptr : NULL; }
 // Free the device bytes of a weight buffer and keep its tile-major copies (include/qw_hip_ext.h).
 // Bytes of h that some tile-major copy was made from: the union of the copies' source ranges inside the buffer.
 static size_t packed_source_bytes(const qw_hbuf *h) {
@@ -775,7 +808,7 @@ bool qw_hip_buf_upload(qw_buf *b, size_t off, size_t len) {
 }
 bool qw_hip_buf_download(qw_buf *b, size_t off, size_t len) {
     qw_hbuf *h = b ? b->handle : NULL;
-    return h && h->host && !h->wrapped && range_ok(h, off, len) && hipMemcpy((char *)h->host + off, (char *)h->dptr + off, len, hipMemcpyDeviceToHost) == hipSuccess;
+    return h && h->host && !h->wrapped && range_ok(h, off, len) && rest_up(h) && hipMemcpy((char *)h->host + off, (char *)h->dptr + off, len, hipMemcpyDeviceToHost) == hipSuccess;
 }
 bool qw_hip_buf_write(qw_buf *b, size_t off, const void *src, size_t len) {
     qw_hbuf *h = b ? b->handle : NULL;
@@ -867,8 +900,8 @@ bool qw_hip_buf_write_fd(qw_buf *b, size_t off, int fd, uint64_t foff, size_t le
     return ok; // (a host side got the same bytes; whether it still holds others that HBM lacks stays as it was)
 }
 bool qw_hip_buf_read(const qw_buf *b, size_t off, void *dst, size_t len) {
-    const qw_hbuf *h = b ? b->handle : NULL;
-    return h && range_ok(h, off, len) && hipMemcpy(dst, (const char *)h->dptr + off, len, hipMemcpyDeviceToHost) == hipSuccess;
+    qw_hbuf *h = b ? b->handle : NULL;
+    return h && range_ok(h, off, len) && rest_up(h) && hipMemcpy(dst, (const char *)h->dptr + off, len, hipMemcpyDeviceToHost) == hipSuccess;
 }
 
 // ---------------------------------------------------------------- batches: recording
@@ -935,7 +968,13 @@ static bool bind_ptr(qw_batch *b, unsigned index, size_t need, bool out, const c
         b->capuse = b->capuse ? 2 * b->capuse : 64;
         b->use = realloc(b->use, sizeof *b->use * (size_t)b->capuse);
     }
-    b->use[b->nuse++] = (qw_use){h, out};
+    b->use[b->nuse++] = (qw_use){h, out, false, off, off + need};
+    return true;
+}
+// The same for an output of which the dispatch writes every byte of the range: what the range held before does not matter.
+static bool bind_whole(qw_batch *b, unsigned index, size_t need, const char *what, void **p) {
+    if (!bind_ptr(b, index, need, true, what, p)) return false;
+    b->use[b->nuse - 1].whole = true;
     return true;
 }
 static bool bind_bytes(qw_batch *b, unsigned index, void *dst, size_t len, const char *what) {
@@ -1070,7 +1109,7 @@ static bool tr_qmvm(qw_batch *b) { // src/engine.c:752-771: 0..3 W, 4 x, 5..8 y,
         if (!in.N[j]) return fail(b, "qmv_ggm: matrix %d has no rows", j);
         if (b->buf[j].h && b->buf[j].off % 16) return fail(b, "qmv_ggm: offset %zu of matrix %d is not 16-byte aligned", b->buf[j].off, j);
         if (!bind_ptr(b, (unsigned)j, (size_t)a.N[j] * a.rowbytes[j], false, "W", (void **)&a.W[j]) ||
-            !bind_ptr(b, 5u + (unsigned)j, (size_t)a.nb * a.N[j] * (a.yfloat ? 4 : 2), true, "y", &a.y[j])) return false;
+            !bind_whole(b, 5u + (unsigned)j, (size_t)a.nb * a.N[j] * (a.yfloat ? 4 : 2), "y", &a.y[j])) return false;
     }
     if (in.total != total) return fail(b, "qmv_ggm: total %u, the matrices have %u rows", in.total, total);
     qw_hbuf *hm[4] = {b->buf[0].h, b->buf[1].h, b->buf[2].h, b->buf[3].h};
@@ -1090,6 +1129,7 @@ static bool tr_qmv(qw_batch *b) { // src/engine.c:717-723: 0 W, 3 x, 4 y, 5 {N, 
         if (!bind_ptr(b, 0, (size_t)m.N[0] * m.rowbytes[0], false, "W", (void **)&m.W[0]) ||
             !bind_ptr(b, 3, ((size_t)(m.nb - 1) * m.xstride + m.K) * 2, false, "x", (void **)&m.x) ||
             !bind_ptr(b, 4, ((size_t)(m.nb - 1) * m.ystride[0] + m.N[0]) * (m.yfloat ? 4 : 2), true, "y", &m.y[0])) return false;
+        b->use[b->nuse - 1].whole = m.nb == 1 || m.ystride[0] == m.N[0];
         qw_hbuf *hm[4] = {b->buf[0].h};
         return launch_qmvm(b, &m, hm);
     }
@@ -1104,6 +1144,7 @@ static bool tr_qmv(qw_batch *b) { // src/engine.c:717-723: 0 W, 3 x, 4 y, 5 {N, 
     b->allow_released = false;
     if (!bound || !bind_ptr(b, 3, ((size_t)(a.nb - 1) * a.xstride + a.K) * 2, false, "x", (void **)&a.x) ||
         !bind_ptr(b, 4, ((size_t)(a.nb - 1) * a.ystride + a.N) * (a.yfloat ? 4 : 2), true, "y", &a.y)) return false;
+    b->use[b->nuse - 1].whole = a.nb == 1 || a.ystride == a.N;
     char fn[48];
     int F = p->F;
     if (F == 21 && p->K <= 2560 && a.N % 16 == 0) { // tile-major copy of the rows, made at first use
@@ -1132,7 +1173,7 @@ static bool fill_router(qw_batch *b, qwk_router_args *a, unsigned iWr, unsigned 
     const qw_kparams *p = &b->k->p;
     *a = (qwk_router_args){.E = (uint32_t)p->E, .D = (uint32_t)p->D, .nb = nbr};
     return bind_ptr(b, iWr, (size_t)p->E * p->D * 2, false, "router weights", (void **)&a->Wr) && bind_ptr(b, iWsg, (size_t)p->D * 2, false, "shared gate vector", (void **)&a->Wsg) &&
-           bind_ptr(b, ix, (size_t)nbr * p->D * 2, false, "x", (void **)&a->x) && bind_ptr(b, ilg, (size_t)nbr * (p->E + 1) * 4, true, "logits", (void **)&a->logits);
+           bind_ptr(b, ix, (size_t)nbr * p->D * 2, false, "x", (void **)&a->x) && bind_whole(b, ilg, (size_t)nbr * (p->E + 1) * 4, "logits", (void **)&a->logits);
 }
 
 static bool fill_select(qw_batch *b, qwk_select_args *a, unsigned ilg, unsigned isel, uint32_t nbr) {
@@ -1359,7 +1400,7 @@ static bool tr_gu(qw_batch *b) {
     if (!bind_ptr(b, 5, QW_SEL_BYTES((size_t)p->gnb, (size_t)p->topk), false, "selection", (void **)&a.sel)) return false;
     b->pend_sd.valid = false;
     b->pend_sd.rowbytes = (uint32_t)fmt_rb(p->fsd, p->I);
-    if (!bind_ptr(b, 2, (size_t)p->D * b->pend_sd.rowbytes, false, "shared down weights", (void **)&b->pend_sd.Wsd) || !bind_ptr(b, 3, (size_t)nbr * p->D * 4, true, "Psh", (void **)&b->pend_sd.Psh)) return false;
+    if (!bind_ptr(b, 2, (size_t)p->D * b->pend_sd.rowbytes, false, "shared down weights", (void **)&b->pend_sd.Wsd) || !bind_whole(b, 3, (size_t)nbr * p->D * 4, "Psh", (void **)&b->pend_sd.Psh)) return false;
     b->pend_sd.valid = true;
     b->pend_sd.hd = b->buf[2].h;
     b->pend_sd.fmt = p->fsd;
@@ -1602,7 +1643,7 @@ static bool tr_cmb(qw_batch *b) {
     if (!bind_bytes(b, 8, &nbr, 4, "nbr") || !nbr_ok(b, nbr)) return false;
     qwk_cmb_args a = {.D = (uint32_t)p->D, .nbr = nbr, .topk = (uint32_t)p->topk, .gnb = (uint32_t)p->gnb};
     if (!bind_ptr(b, 9, (size_t)nbr * p->topk * p->D * 4, false, "Pg", (void **)&a.Pg) || !bind_ptr(b, 1, (size_t)nbr * p->D * 4, false, "Psh", (void **)&a.Psh) ||
-        !bind_ptr(b, 3, QW_SEL_BYTES((size_t)p->gnb, (size_t)p->topk), false, "selection", (void **)&a.sel) || !bind_ptr(b, 4, (size_t)nbr * p->D * 2, true, "out", (void **)&a.out)) return false;
+        !bind_ptr(b, 3, QW_SEL_BYTES((size_t)p->gnb, (size_t)p->topk), false, "selection", (void **)&a.sel) || !bind_whole(b, 4, (size_t)nbr * p->D * 2, "out", (void **)&a.out)) return false;
     if (b->pend_dn.valid) {
         qwk_dn_args *d = &b->pend_dn.a;
         // the down dispatch counts tokens by its compiled NB, the combine by the bound count: the masks carry the rest
@@ -1736,7 +1777,7 @@ static bool tr_pk_combine(qw_batch *b, unsigned gy) { // 0 D, 1 pos_of, 2 w, 3 Y
     const qw_kparams *p = &b->k->p;
     qwk_combine_args a = {.KD = (uint32_t)p->K, .topk = (uint32_t)p->topk, .T = gy, .P = gy * (uint32_t)p->topk};
     if (!bind_ptr(b, 0, (size_t)a.P * p->K * 2, false, "D", (void **)&a.Dm) || !bind_ptr(b, 1, (size_t)a.P * 4, false, "pos_of", (void **)&a.pos_of) ||
-        !bind_ptr(b, 2, (size_t)a.P * 4, false, "w", (void **)&a.w) || !bind_ptr(b, 3, (size_t)gy * p->K * 2, true, "Y", (void **)&a.Y)) return false;
+        !bind_ptr(b, 2, (size_t)a.P * 4, false, "w", (void **)&a.w) || !bind_whole(b, 3, (size_t)gy * p->K * 2, "Y", (void **)&a.Y)) return false;
     if (!add_launch(b, "qwk_moe_combine", cdiv((unsigned)p->K / 4, 64), 64, &a, sizeof a)) return false;
     if (gy) b->l[b->nl - 1].gy = gy;
     return true;
@@ -1889,10 +1930,10 @@ static bool tr_hc(qw_batch *b) {
     }
     if (!bind_ptr(b, 4, HCD * QW_HC_LR * 2, false, "mix_up", (void **)&a.Wu)) return false;
     if (f == FAM_HC_UP) {
-        if (!bind_ptr(b, 5, nb * QW_HC * QW_HC_PDS * 4, false, "partial sums", (void **)&a.pd) || !bind_ptr(b, 6, nb * D * 2, true, "x", (void **)&a.x)) return false;
-        if (a.want_inj && !bind_ptr(b, 7, nb * QW_HC * QW_HC * 4, true, "new inject sums", (void **)&a.injo)) return false;
+        if (!bind_ptr(b, 5, nb * QW_HC * QW_HC_PDS * 4, false, "partial sums", (void **)&a.pd) || !bind_whole(b, 6, nb * D * 2, "x", (void **)&a.x)) return false;
+        if (a.want_inj && !bind_whole(b, 7, nb * QW_HC * QW_HC * 4, "new inject sums", (void **)&a.injo)) return false;
     } else if (!bind_ptr(b, 5, nb * QW_HC_LR * 4, false, "sx", (void **)&a.sx) || !bind_ptr(b, 6, nb * QW_HC * 4, false, "rs", (void **)&a.rs) ||
-               !bind_ptr(b, 7, nb * D * 2, true, "x", (void **)&a.x)) return false;
+               !bind_whole(b, 7, nb * D * 2, "x", (void **)&a.x)) return false;
     if (!add_launch(b, f == FAM_HC_UP ? "qwk_hc_up" : "qwk_hc_upv", (unsigned)(D / 8), 256, &a, sizeof a)) return false;
     b->l[b->nl - 1].gy = (unsigned)(nb + QW_HC_TG - 1) / QW_HC_TG; // tokens four at a time
     return true;
@@ -2051,30 +2092,144 @@ static int graph_run(qw_batch *b, hipStream_t st) {
     return HIPOK(g, hipGraphLaunch(exec, st)) ? 1 : -1;
 }
 
-static bool submit_segment(qw_batch *b) {
+// ---- the copies between shadows and HBM, the stamps and the flags (qwk_io)
+typedef struct { qwk_io_args a; unsigned grid; } qw_io;
+static bool io_launch(qw_batch *b, qw_io *io) {
+    void *params[] = {&io->a};
+    io->a.count = b->g->io_count + b->io_idx;
+    if (!io->a.n) io->grid = 1;
+    if (!HIPOK(b->g, hipModuleLaunchKernel(b->g->io_func, io->grid, 1, 1, 256, 1, 1, 0, b->g->stream[b->stream], params, NULL))) return b->failed = true, false;
+    const uint32_t to_host = io->a.to_host;
+    *io = (qw_io){.a = {.to_host = to_host}};
+    return true;
+}
+static bool io_add(qw_batch *b, qw_io *io, const void *src, void *dst, size_t bytes) {
+    if (!bytes) return true;
+    if (io->a.n == QW_IO_MAX && !io_launch(b, io)) return false;
+    const size_t wgs = (bytes + QW_IO_WG - 1) / QW_IO_WG;
+    io->a.src[io->a.n] = src, io->a.dst[io->a.n] = dst, io->a.bytes[io->a.n] = (uint32_t)bytes;
+    io->grid += wgs < 64 ? (unsigned)wgs : 64; // reading over PCIe with 256 workgroups or more is slower than with 64 (1 MB: 33 against 27 us)
+    io->a.first[++io->a.n] = io->grid;
+    return true;
+}
+// Batches with stamps and flags; the others (profiled ones, and when more than QW_IO_SLOTS batches are in flight) time
+// themselves with events and wait for the stream.
+static bool io_take(qw_batch *b) {
+    qw_gpu *g = b->g;
+    if (b->io || b->events) return true;
+    if (b->prof || g->io_used == ~0u) return b->events = true;
+    b->io_idx = __builtin_ctz(~g->io_used);
+    g->io_used |= 1u << b->io_idx;
+    b->io = &g->io[b->io_idx];
+    memset((void *)b->io, 0, sizeof *b->io);
+    return true;
+}
+// Until the kernel has raised the flag: polling sees it 5 us sooner than hipStreamSynchronize returns. A long wait, and one
+// for a kernel that never comes to its end, is left to the runtime, which also knows about errors.
+static bool io_wait(qw_batch *b, const volatile uint32_t *flag) {
+    qw_gpu *g = b->g;
+    for (double t0 = 0;;) {
+        for (int i = 0; i < 512; i++) {
+            if (*flag == (uint32_t)b->seq) {
+                __atomic_thread_fence(__ATOMIC_ACQUIRE);
+                return true;
+            }
+            __builtin_ia32_pause();
+        }
+        if (t0 == 0) t0 = qw_now();
+        else if (qw_now() - t0 > 20e-3) break;
+    }
+    if (!HIPOK(g, hipStreamSynchronize(g->stream[b->stream]))) return false;
+    if (*flag == (uint32_t)b->seq) return true;
+    set_err(g, "a batch ended without its last launch");
+    return false;
+}
+// The part of h that this segment's dispatches write whole before anything reads it: [*lo, *hi), in units of 16 bytes (the
+// end of the buffer apart). Those bytes need no upload.
+static void whole_range(const qw_batch *b, int first, const qw_hbuf *h, size_t *lo, size_t *hi) {
+    *lo = *hi = 0;
+    for (int i = first; i < b->nuse; i++) {
+        const qw_use *u = &b->use[i];
+        if (u->b != h || u->lo == u->hi) continue;
+        if (u->out && u->whole) {
+            if (*lo == *hi) *lo = u->lo, *hi = u->hi;
+            else if (u->lo <= *hi && u->hi >= *lo) { // touches or overlaps
+                if (u->lo < *lo) *lo = u->lo;
+                if (u->hi > *hi) *hi = u->hi;
+            }
+        } else if (u->lo < *lo || u->hi > *hi) { // reads, or may leave alone, bytes that the host provides
+            *lo = *hi = 0;
+            return;
+        }
+    }
+    *lo = (*lo + 15) & ~(size_t)15;
+    if (*hi != h->size) *hi &= ~(size_t)15;
+    if (*hi < *lo) *lo = *hi = 0;
+}
+
+// The least range of h, in units of 16 bytes, that holds what dispatches from use `first` on may touch (out: may write).
+static void touched_range(const qw_batch *b, int first, const qw_hbuf *h, bool out, size_t *lo, size_t *hi) {
+    *lo = h->size, *hi = 0;
+    for (int i = first; i < b->nuse; i++) {
+        const qw_use *u = &b->use[i];
+        if (u->b != h || (out && !u->out)) continue;
+        if (u->lo < *lo) *lo = u->lo;
+        if (u->hi > *hi) *hi = u->hi;
+    }
+    *lo &= ~(size_t)15;
+    *hi = *hi + 15 > h->size ? h->size : (*hi + 15) & ~(size_t)15;
+    if (*hi < *lo) *hi = *lo;
+}
+
+// last: the caller waits for the batch at once, and its last launch also carries the outputs back (qw_batch_wait).
+static bool submit_segment(qw_batch *b, bool last) {
     qw_gpu *g = b->g;
     hipStream_t st = g->stream[b->stream];
     if (b->failed || !flush_select(b) || !flush_tw(b, NULL, NULL) || !flush_pf(b) || !flush_gu(b) || !flush_dn(b) || !flush_pk(b)) return false;
     if (b->nseg >= 9) return fail(b, "too many flushes in one batch");
+    io_take(b);
     // host -> device for what this segment binds
     const unsigned mark = ++g->mark;
+    qw_io up = {0};
     for (int i = b->done_use; i < b->nuse; i++) {
         qw_hbuf *h = b->use[i].b;
         if (h->mark == mark) continue;
         h->mark = mark;
         if (h->device_only || !h->host) continue;
-        // A kernel of a batch that was submitted (or of an earlier segment of this one) and not yet waited for wrote
-        // this buffer: HBM holds the newer contents, and the shadow must not overwrite them.
         if (h->released) continue; // no device bytes: its tile-major copies are what the kernels read
-        if (h->pending_out > 0 && !h->dirty) continue;
-        if (h->dirty || (!h->wrapped && h->size <= QW_HIP_SMALL_BYTES)) {
-            if (!HIPOK(g, hipMemcpyAsync(h->dptr, h->host, h->size, hipMemcpyHostToDevice, st))) { b->failed = true; return false; }
-            h->dirty = false;
+        const bool small = !h->wrapped && h->size <= QW_HIP_SMALL_BYTES;
+        if (!h->dirty && !small) continue;
+        // [lo, hi): needs no upload. [tlo, thi): what this segment can touch; a buffer that was in step goes up no further.
+        size_t lo, hi, tlo = 0, thi = h->size;
+        whole_range(b, b->done_use, h, &lo, &hi);
+        if (h->size > QW_HIP_BIG_OUT_BYTES) lo = hi = 0; // (its results are not carried back: the shadow must not be taken for them later)
+        if (!h->dirty) {
+            touched_range(b, i, h, false, &tlo, &thi);
+            // A kernel of a batch that was submitted (or of an earlier segment of this one) and not yet waited for wrote
+            // this buffer: HBM holds the newer contents there, and the shadow must not overwrite them.
+            if (h->pending_out > 0) lo = h->plo, hi = h->phi;
         }
+        h->part = tlo > 0 || thi < h->size, h->slo = tlo, h->shi = thi;
+        if (lo < tlo) lo = tlo;
+        if (hi > thi) hi = thi;
+        if (hi <= lo) lo = hi = thi;
+        char *d = h->dptr, *s = h->host;
+        if (b->io && h->pinned && small) {
+            if (!io_add(b, &up, s + tlo, d + tlo, lo - tlo) || !io_add(b, &up, s + hi, d + hi, thi - hi)) return false;
+        } else {
+            if (lo > tlo && !HIPOK(g, hipMemcpyAsync(d + tlo, s + tlo, lo - tlo, hipMemcpyHostToDevice, st))) { b->failed = true; return false; }
+            if (thi > hi && !HIPOK(g, hipMemcpyAsync(d + hi, s + hi, thi - hi, hipMemcpyHostToDevice, st))) { b->failed = true; return false; }
+        }
+        h->dirty = false;
     }
     for (int i = b->done_use; i < b->nuse; i++) { // outputs of this segment: the device side is the newer one until the batch is waited for
         qw_hbuf *h = b->use[i].b;
-        if (!b->use[i].out || h->device_only || !h->host || h->wrapped || h->out_seq == b->seq) continue;
+        if (!b->use[i].out || h->device_only || !h->host || h->wrapped) continue;
+        if (!h->pending_out) h->plo = h->size, h->phi = 0;
+        size_t lo = b->use[i].lo & ~(size_t)15, hi = (b->use[i].hi + 15) & ~(size_t)15;
+        if (lo < h->plo) h->plo = lo;
+        if (hi > h->phi) h->phi = hi < h->size ? hi : h->size;
+        if (h->out_seq == b->seq) continue;
         if (b->nouts == b->capouts) {
             b->capouts = b->capouts ? 2 * b->capouts : 16;
             b->outs = realloc(b->outs, sizeof *b->outs * (size_t)b->capouts);
@@ -2083,10 +2238,14 @@ static bool submit_segment(qw_batch *b) {
         h->pending_out++;
         b->outs[b->nouts++] = h;
     }
-    hipEvent_t *ev = &b->ev[2 * b->nseg];
-    if (!HIPOK(g, hipEventCreate(&ev[0])) || !HIPOK(g, hipEventCreate(&ev[1]))) { b->failed = true; return false; }
-    b->nseg++;
-    if (!HIPOK(g, hipEventRecord(ev[0], st))) { b->failed = true; return false; }
+    const int seg = b->nseg++;
+    hipEvent_t *ev = &b->ev[2 * seg];
+    if (b->events) {
+        if (!HIPOK(g, hipEventCreate(&ev[0])) || !HIPOK(g, hipEventCreate(&ev[1])) || !HIPOK(g, hipEventRecord(ev[0], st))) { b->failed = true; return false; }
+    } else if (up.a.n || seg == 0 || b->io->t1[seg - 1]) { // (a segment that follows on a running one starts where that one ends)
+        up.a.t_done = (uint64_t *)&b->io->t0[seg];
+        if (!io_launch(b, &up)) return false;
+    }
     const int as_graph = graph_run(b, st);
     if (as_graph < 0) { b->failed = true; return false; }
     bool side_open = false;
@@ -2114,7 +2273,12 @@ static bool submit_segment(qw_batch *b) {
         }
     }
     if (side_open && !side_link(g, g->side[b->stream], st)) { b->failed = true; return false; }
-    if (!HIPOK(g, hipEventRecord(ev[1], st))) { b->failed = true; return false; }
+    if (b->events) {
+        if (!HIPOK(g, hipEventRecord(ev[1], st))) { b->failed = true; return false; }
+    } else if (!last) { // the segment's end, and for qw_batch_poll the batch's
+        qw_io end = {.a = {.t_enter = (uint64_t *)&b->io->t1[seg], .flag = b->submitted ? (uint32_t *)&b->io->done : NULL, .flagval = (uint32_t)b->seq}};
+        if (!io_launch(b, &end)) return false;
+    }
     b->done_l = b->nl;
     b->done_use = b->nuse;
     return true;
@@ -2123,35 +2287,38 @@ static bool submit_segment(qw_batch *b) {
 void qw_batch_flush(qw_batch *b) {
     if (b->prof) return; // as in the reference: a profiled batch is not split
     if (b->nseg >= 8) return;
-    submit_segment(b);
+    submit_segment(b, false);
 }
 
 void qw_batch_submit(qw_batch *b) {
     if (b->submitted) return;
     b->submitted = true;
-    submit_segment(b);
+    submit_segment(b, false);
 }
 
 bool qw_batch_poll(qw_batch *b) {
     if (b->failed || !b->submitted) return true;
-    return hipEventQuery(b->ev[2 * b->nseg - 1]) != hipErrorNotReady;
+    if (b->events) return hipEventQuery(b->ev[2 * b->nseg - 1]) != hipErrorNotReady;
+    return b->io->done == (uint32_t)b->seq || hipStreamQuery(b->g->stream[b->stream]) != hipErrorNotReady; // (an error counts as done: the wait reports it)
 }
 
 static void batch_free(qw_batch *b) {
     for (int i = 0; i < b->nouts; i++) b->outs[i]->pending_out--;
     free(b->outs);
-    for (int i = 0; i < 2 * b->nseg; i++) (void)hipEventDestroy(b->ev[i]);
+    if (b->events)
+        for (int i = 0; i < 2 * b->nseg; i++)
+            if (b->ev[i]) (void)hipEventDestroy(b->ev[i]);
     for (int i = 0; i < b->npev; i++) (void)hipEventDestroy(b->pev[i]);
+    if (b->io) b->g->io_used &= ~(1u << b->io_idx);
     free(b->pev);
     free(b->l);
     free(b->use);
     free(b);
 }
 
-double qw_batch_wait(qw_batch *b) {
+static double batch_wait(qw_batch *b, bool ended) { // ended: submitted by qw_batch_end, whose last segment left its end to this
     qw_gpu *g = b->g;
     hipStream_t st = g->stream[b->stream];
-    if (!b->submitted) qw_batch_submit(b);
     double secs = -1;
     if (b->failed) {
         (void)hipStreamSynchronize(st);
@@ -2162,23 +2329,47 @@ double qw_batch_wait(qw_batch *b) {
     }
     // device -> host for everything bound in an output role
     const unsigned mark = ++g->mark;
-    bool ok = true;
+    bool ok = true, sync = b->events;
+    qw_io down = {.a = {.to_host = 1}};
     for (int i = 0; i < b->nuse && ok; i++) {
         qw_hbuf *h = b->use[i].b;
         if (!b->use[i].out || h->mark == mark) continue;
         h->mark = mark;
         if (h->device_only || !h->host || h->wrapped || h->size > QW_HIP_BIG_OUT_BYTES) continue;
-        ok = HIPOK(g, hipMemcpyAsync(h->host, h->dptr, h->size, hipMemcpyDeviceToHost, st));
+        size_t lo, hi; // only what its dispatches may have written: the rest of the shadow is the host's own
+        touched_range(b, i, h, true, &lo, &hi);
+        if (hi <= lo) continue;
+        if (b->io && h->pinned) ok = io_add(b, &down, (char *)h->dptr + lo, (char *)h->host + lo, hi - lo);
+        else ok = HIPOK(g, hipMemcpyAsync((char *)h->host + lo, (char *)h->dptr + lo, hi - lo, hipMemcpyDeviceToHost, st)), sync = true;
     }
-    if (ok && b->uses_sync) ok = HIPOK(g, hipMemcpyAsync(g->sync_host, g->sync + QW_SYNC_ERR_WORD, 4, hipMemcpyDeviceToHost, st));
-    ok = ok && HIPOK(g, hipStreamSynchronize(st));
+    if (ok && b->uses_sync) {
+        if (b->io) ok = io_add(b, &down, g->sync + QW_SYNC_ERR_WORD, g->sync_host, 4);
+        else ok = HIPOK(g, hipMemcpyAsync(g->sync_host, g->sync + QW_SYNC_ERR_WORD, 4, hipMemcpyDeviceToHost, st));
+    }
+    if (ok && b->io) {
+        const volatile uint32_t *flag = &b->io->done;
+        if (ended || down.a.n) {
+            flag = &b->io->copied;
+            if (ended) down.a.t_enter = (uint64_t *)&b->io->t1[b->nseg - 1];
+            down.a.flag = (uint32_t *)flag, down.a.flagval = (uint32_t)b->seq;
+            ok = io_launch(b, &down);
+        }
+        ok = ok && (sync ? HIPOK(g, hipStreamSynchronize(st)) : io_wait(b, flag));
+    } else ok = ok && HIPOK(g, hipStreamSynchronize(st));
+    if (!ok) (void)hipStreamSynchronize(st); // nothing of this batch may still be on its way when its slot and its buffers go
     if (ok && b->uses_sync && g->sync_host[0]) { // a launch whose workgroups wait for one another gave up: its results are not valid
         (void)hipMemset(g->sync, 0, QW_SYNC_BYTES);
         g->fuse_broken = true;
         set_err(g, "a fused layer launch timed out waiting for its workgroups (are other kernels running on this device?); layers run as separate launches from now on");
         ok = false;
     }
-    if (ok) {
+    if (ok && b->io) {
+        secs = 0;
+        for (int s = 0; s < b->nseg; s++) {
+            const uint64_t t0 = b->io->t0[s] ? b->io->t0[s] : s ? b->io->t1[s - 1] : 0, t1 = b->io->t1[s];
+            if (t1 > t0) secs += (double)(t1 - t0) * g->tick;
+        }
+    } else if (ok) {
         secs = 0;
         for (int s = 0; s < b->nseg; s++) {
             float ms = 0;
@@ -2204,9 +2395,16 @@ double qw_batch_wait(qw_batch *b) {
     return secs;
 }
 
+double qw_batch_wait(qw_batch *b) {
+    if (b->submitted) return batch_wait(b, false);
+    return qw_batch_end(b);
+}
+
 double qw_batch_end(qw_batch *b) {
-    qw_batch_submit(b);
-    return qw_batch_wait(b);
+    if (b->submitted) return batch_wait(b, false);
+    b->submitted = true;
+    submit_segment(b, true);
+    return batch_wait(b, true);
 }
 
 void qw_gpu_set_stream(qw_gpu *g, int s) { g->cur_stream = s == 1 ? 1 : 0; }

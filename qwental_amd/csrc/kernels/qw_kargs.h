@@ -306,3 +306,21 @@ typedef struct { /* synthetic weights: nblocks GGUF blocks of one type, scale d 
     uint32_t type; /* 8 or 21 */
     float sigma;
 } qwk_fill_args;
+
+/* qwk_io: the host side of a batch, one launch in front of its kernels (host shadows -> HBM) and one behind them (HBM ->
+ * host shadows). Piece i is copied by workgroups [first[i], first[i + 1]) of the launch, QW_IO_WG bytes each and round
+ * again. Host pointers are pinned, coherent memory. */
+#define QW_IO_MAX 24u        /* pieces of one launch */
+#define QW_IO_WG 16384u      /* bytes a workgroup has in flight: 256 threads x 4 x 16 */
+typedef struct {
+    const void *src[QW_IO_MAX];
+    void *dst[QW_IO_MAX];
+    uint32_t bytes[QW_IO_MAX], first[QW_IO_MAX + 1];
+    uint32_t n;         /* pieces (may be 0: stamps and the flag only, one workgroup) */
+    uint32_t *count;    /* device word, zero before and after the launch: workgroups that are done */
+    uint64_t *t_enter;  /* host, may be NULL: the device clock when the launch's first workgroup starts */
+    uint64_t *t_done;   /* host, may be NULL: the device clock when every piece has been copied */
+    uint32_t *flag;     /* host, may be NULL: receives flagval when everything above has reached the host */
+    uint32_t flagval;
+    uint32_t to_host;   /* the destinations are host memory */
+} qwk_io_args;

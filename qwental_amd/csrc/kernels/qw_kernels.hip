@@ -2912,6 +2912,44 @@ extern "C" __global__ __launch_bounds__(256) void qwk_copy(qwk_mem_args a) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += step) q[i] = p[i];
 }
 #endif
+#if QW_IN_PART(5)
+// The host side of a batch (qwk_io_args). A batch over host-shadowed buffers used to issue one hipMemcpyAsync a buffer and
+// a timing event at either end; each of those is a packet of its own with a signal behind it. Bound by the round trip over
+// PCIe (about 2 us) and, from some 100 KB on, by its rate (45 to 50 GB/s, the same as the copy engines'): a workgroup asks
+// for its 16 KB at once, pieces run beside each other, and the last workgroup done raises the flag the host polls.
+// Measured, an empty kernel between host and back: 4 KB up + 16 KB down + two events + stream synchronisation 25.5 us,
+// with two of these launches 11 to 12 us; 256 KB down 25.1 us by hipMemcpyAsync, 14.5 by this kernel.
+extern "C" __global__ __launch_bounds__(256) void qwk_io(qwk_io_args a) {
+    if (a.t_enter && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(a.t_enter, __builtin_amdgcn_s_memrealtime(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    uint32_t p = 0;
+    while (p + 1 < a.n && blockIdx.x >= a.first[p + 1]) p++;
+    if (p < a.n) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, ""); // what the host wrote since an earlier launch read the same lines
+        const uint32_t n16 = a.bytes[p] / 16, wg = blockIdx.x - a.first[p], nwg = a.first[p + 1] - a.first[p];
+        const u4 *src = (const u4 *)a.src[p];
+        u4 *dst = (u4 *)a.dst[p];
+        for (uint32_t base = wg * (QW_IO_WG / 16); base < n16; base += nwg * (QW_IO_WG / 16)) {
+            u4 v[4];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++)
+                if (base + k * 256 + threadIdx.x < n16) v[k] = src[base + k * 256 + threadIdx.x];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++)
+                if (base + k * 256 + threadIdx.x < n16) dst[base + k * 256 + threadIdx.x] = v[k];
+        }
+        if (wg == 0 && threadIdx.x < a.bytes[p] % 16) ((uint8_t *)dst)[n16 * 16 + threadIdx.x] = ((const uint8_t *)src)[n16 * 16 + threadIdx.x];
+    }
+    if (a.to_host || a.flag) __builtin_amdgcn_fence(__ATOMIC_RELEASE, ""); // this wave's stores have reached the host
+    else __builtin_amdgcn_s_waitcnt(0);
+    if (!a.flag && !a.t_done) return;
+    __syncthreads();
+    if (threadIdx.x == 0 && __hip_atomic_fetch_add(a.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+        __hip_atomic_store(a.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); // for the next launch
+        if (a.t_done) __hip_atomic_store(a.t_done, __builtin_amdgcn_s_memrealtime(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (a.flag) __hip_atomic_store(a.flag, a.flagval, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+#endif
 // Fill n 16-byte units with a counter-based hash of (seed, index): uniform random bytes.
 __device__ __forceinline__ uint32_t qw_mix(uint64_t x) {
     x ^= x >> 33; x *= 0xff51afd7ed558ccdull; x ^= x >> 33; x *= 0xc4ceb9fe1a85ec53ull; x ^= x >> 33;

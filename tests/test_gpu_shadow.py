@@ -1,0 +1,101 @@
+"""The copies between host shadows and HBM around a batch (qwk_io in front of the kernels and behind them): what the host
+wrote goes up, what the kernels wrote comes back, and nothing else of a buffer changes on either side."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import qwental_amd as q
+from qwental_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def product(oracle, ft, W, N, K, x):
+    return oracle.qmv(ft, W, N, K, x, f64=True)
+
+
+@pytest.mark.parametrize("N,K,nb,yoff,slack", [(16, 256, 1, 0, 0), (33, 512, 3, 52, 7), (640, 256, 16, 16, 100), (9, 256, 2, 4, 1), (4096, 256, 5, 0, 20000)])
+def test_rows_inside_a_larger_buffer_leave_the_rest_alone(gpu, oracle, N, K, nb, yoff, slack):
+    """y at an offset of a buffer full of the host's own bytes: only the product's bytes change, on the host and in HBM."""
+    rng = np.random.default_rng(N + K + nb)
+    W = synth.matrix(rng, 8, N, K)
+    path = q.Path(gpu, 2048, 512, 512, 10, 16)
+    wb, y = gpu.buf_from(W, device_only=True), gpu.buf(yoff + nb * N * 4 + slack)
+    xb = gpu.buf(nb * K * 2)
+    for it in range(3):  # the input changes under the same address from call to call
+        x = synth.activations(rng, nb, K)
+        fence = rng.integers(0, 256, y.size, dtype=np.uint8)
+        y.view()[:] = fence
+        C.memmove(xb.c.ptr, x.ctypes.data, x.nbytes)  # straight into the shadow
+        b = gpu.batch()
+        path.qmv_gg(b, q.Tensor(wb, 8), N, K, xb, y, nb, yoff=yoff)
+        assert b.end() > 0
+        got = y.view().copy()
+        res = got[yoff:yoff + nb * N * 4].view(np.float32).reshape(nb, N)
+        ref = product(oracle, 8, W, N, K, x)
+        assert np.abs(res - ref).max() <= 1e-5 * np.abs(ref).max()
+        keep = np.ones(y.size, bool)
+        keep[yoff:yoff + nb * N * 4] = False
+        assert np.array_equal(got[keep], fence[keep])
+        assert np.array_equal(y.read(), got)  # HBM holds what the host sees
+    for bb in (wb, xb, y):
+        bb.free()
+    path.close()
+
+
+def test_gaps_between_strided_rows_keep_the_hosts_bytes(gpu, oracle):
+    N, K, nb, stride = 20, 256, 4, 37
+    rng = np.random.default_rng(5)
+    W, x = synth.matrix(rng, 21, N, K), synth.activations(rng, nb, K)
+    ok, err = gpu.compile("#define qmv_gg qmv_gg_gaps\n#define GF 21\n#define KD %d\n#define RB %d\n#define NB %d\n#define YT float\n" % (K, synth.row_bytes(21, K), nb))
+    assert ok, err
+    wb, xb, y = gpu.buf_from(W, device_only=True), gpu.buf_from(x), gpu.buf(nb * stride * 4)
+    v = y.view(np.float32).reshape(nb, stride)
+    v[:] = -7.5
+    b = gpu.batch()
+    b.kernel(gpu.kernel("qmv_gg_gaps"))
+    b.buf(0, wb)
+    b.buf(3, xb)
+    b.buf(4, y)
+    b.bytes(5, np.array([N, K, stride, 0], np.uint32))
+    b.dispatch(1)
+    assert b.end() > 0
+    ref = product(oracle, 21, W, N, K, x)
+    assert np.abs(v[:, :N] - ref).max() <= 1e-5 * np.abs(ref).max() and (v[:, N:] == -7.5).all()
+    for bb in (wb, xb, y):
+        bb.free()
+
+
+@pytest.mark.parametrize("nbuf", [3, 24, 25, 60])
+def test_many_buffers_and_many_batches_in_flight(gpu, oracle, nbuf):
+    """More pieces than one launch carries, more batches in flight than there are slots, polled and waited for out of order."""
+    N, K = 48, 256
+    rng = np.random.default_rng(nbuf)
+    W = synth.matrix(rng, 8, N, K)
+    path = q.Path(gpu, 2048, 512, 512, 10, 16)
+    wb = gpu.buf_from(W, device_only=True)
+    xs = [synth.activations(rng, 1, K) for _ in range(nbuf)]
+    xb, yb = [gpu.buf_from(x) for x in xs], [gpu.buf(N * 4) for _ in xs]
+    refs = [product(oracle, 8, W, N, K, x)[0] for x in xs]
+    b = gpu.batch()
+    for x, y in zip(xb, yb):
+        path.qmv_gg(b, q.Tensor(wb, 8), N, K, x, y, 1)
+    assert b.end() > 0
+    for y, r in zip(yb, refs):
+        assert np.abs(y.view(np.float32)[:N] - r).max() <= 1e-5 * np.abs(r).max()
+        y.view()[:] = 0
+    flight = []
+    for x, y in zip(xb, yb):
+        b = gpu.batch()
+        path.qmv_gg(b, q.Tensor(wb, 8), N, K, x, y, 1)
+        gpu.L.qw_batch_submit(b.b)
+        flight.append(b)
+    while not gpu.L.qw_batch_poll(flight[-1].b):
+        pass
+    for i in reversed(range(nbuf)):
+        assert gpu.L.qw_batch_wait(flight[i].b) > 0
+        assert np.abs(yb[i].view(np.float32)[:N] - refs[i]).max() <= 1e-5 * np.abs(refs[i]).max()
+    for bb in [wb] + xb + yb:
+        bb.free()
+    path.close()
