@@ -165,7 +165,7 @@ def test_reference_clients_link_against_the_library():
     import subprocess
     L = q.load_lib()
     exes = [os.path.join(ROOT, "oracle", "_ref", n) for n in ("dqtest_ref", "ggmtest_ref")]
-    if not os.path.isdir("/root/reference"):
+    if not os.path.exists("/root/reference/tools/dqtest.c"):  # (an empty mount point is no tree either)
         pytest.skip("no reference tree here")
     for exe in exes:
         assert os.path.exists(exe), "oracle/_ref is stale: run `make -C oracle ref` after building the library"
