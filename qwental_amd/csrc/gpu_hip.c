@@ -1743,10 +1743,13 @@ static bool tr_pk_scatter(qw_batch *b, unsigned gx) { // 0 X, 1 ids, 2 cursor, 3
     if (b->buf[0].off % 16 || b->buf[3].off % 16) return fail(b, "moe_scatter: row buffers must be 16-byte aligned");
     if (b->pend_pk.stage == 3 && b->pend_pk.pl.cursor == a.cursor && b->pend_pk.c.ids == a.ids && b->pend_pk.c.P == a.P && b->pend_pk.c.E == a.E && a.KD % 8 == 0) {
         const qwk_plan_args *pl = &b->pend_pk.pl;
-        const qwk_prep_args f = {.ids = a.ids, .counts = b->pend_pk.c.counts, .offs = pl->offs, .cursor = pl->cursor, .tiles = pl->tiles, .pos_of = a.pos_of, .X = a.X, .Xs = a.Xs,
-                                 .P = a.P, .E = a.E, .topk = a.topk, .KD = a.KD, .tm = pl->tm, .max_tiles = pl->max_tiles};
+        qwk_prep_args f = {.ids = a.ids, .counts = b->pend_pk.c.counts, .offs = pl->offs, .cursor = pl->cursor, .tiles = pl->tiles, .pos_of = a.pos_of, .X = a.X, .Xs = a.Xs,
+                                 .P = a.P, .E = a.E, .topk = a.topk, .KD = a.KD, .tm = pl->tm, .max_tiles = pl->max_tiles,
+                                 .slice = 1};
         b->pend_pk.stage = 0;
-        return add_launch(b, "qwk_moe_prep", a.P, 256, &f, sizeof f);
+        if (a.P <= QW_PREP_ONE) return add_launch(b, "qwk_moe_prep", a.P, 256, &f, sizeof f);
+        f.slice = umin(cdiv(a.P, 2 * (unsigned)b->g->ncu), QW_PREP_SLICE);
+        return add_launch(b, "qwk_moe_prep_slices", cdiv(a.P, f.slice), 512, &f, sizeof f);
     }
     if (!flush_pk(b)) return false;
     return add_launch(b, "qwk_moe_scatter", gx, 256, &a, sizeof a);
@@ -1778,7 +1781,7 @@ static bool tr_pk_combine(qw_batch *b, unsigned gy) { // 0 D, 1 pos_of, 2 w, 3 Y
     qwk_combine_args a = {.KD = (uint32_t)p->K, .topk = (uint32_t)p->topk, .T = gy, .P = gy * (uint32_t)p->topk};
     if (!bind_ptr(b, 0, (size_t)a.P * p->K * 2, false, "D", (void **)&a.Dm) || !bind_ptr(b, 1, (size_t)a.P * 4, false, "pos_of", (void **)&a.pos_of) ||
         !bind_ptr(b, 2, (size_t)a.P * 4, false, "w", (void **)&a.w) || !bind_whole(b, 3, (size_t)gy * p->K * 2, "Y", (void **)&a.Y)) return false;
-    if (!add_launch(b, "qwk_moe_combine", cdiv((unsigned)p->K / 4, 64), 64, &a, sizeof a)) return false;
+    if (!add_launch(b, "qwk_moe_combine", cdiv((unsigned)p->K / 8, 64), 64, &a, sizeof a)) return false;
     if (gy) b->l[b->nl - 1].gy = gy;
     return true;
 }
@@ -1789,12 +1792,26 @@ static bool launch_pf(qw_batch *b, qwk_pf_args *a, int F, int E, qw_hbuf *hw, qw
     a->split = 16, a->ntn = a->N / 16;
     if (!wb) a->H = NULL, a->Y1 = NULL; // SwiGLU rides only in a launch that holds both matrices
     char fn[32];
+    // The blocked kernel (qwk_pfg_*) wants its result rows 16-byte aligned. It takes IQ4_NL rows at any size (24 rows of the
+    // reference model's layer: down product 95 -> 51 us) and IQ3_S rows from entries of more than 16 rows on; with entries
+    // of 16 it passes the kernel that keeps an entry's rows in LDS once experts have several entries each (512 experts,
+    // top-10: 500 rows 154 + 83 against 151 + 83 us, 2048 rows 303 + 161 against 241 + 135, 250 rows 107 + 58 against 114 + 64).
+    const bool blocked = ((uintptr_t)a->Y | (uintptr_t)a->Y1 | (uintptr_t)a->H) % 16 == 0;
+    if (F == 20 && a->K % 320 == 0 && blocked) {
+        const uint32_t nch = a->K / 320;
+        const uint8_t *pk = get_pack(b, hw, a->W, NULL, NULL, (uint64_t)E * (a->N / 16), nch, a->rowbytes, QW_F_PACKED_NL);
+        if (pk) {
+            a->W = pk, a->rowbytes = nch * QW_NL_CHUNK_BYTES;
+            return add_launch(b, "qwk_pfg_f120", (unsigned)b->g->ncu, 512, a, sizeof *a);
+        }
+    }
     if (F == 21 && a->K % 256 == 0) {
         const uint32_t nblk = a->K / 256, split = wb ? 8 : 16;
         const uint64_t ntiles = (uint64_t)E * (a->N / split);
         const uint8_t *pk = get_pack(b, hw, a->W, wb ? hwb : NULL, wb, ntiles, nblk, a->rowbytes, split);
         if (pk) {
             a->W = pk, a->rowbytes = nblk * QW_SLAB_BYTES, a->split = split, a->ntn = a->N / split;
+            if (blocked && (a->tm > 16 || a->M > 5000)) return add_launch(b, "qwk_pfg_f121", (unsigned)b->g->ncu, 512, a, sizeof *a);
             if (a->tm <= 16 && a->K <= 2560) { // entries of one group of rows: the rows are staged in LDS per workgroup range
                 fname_fmt(fn, sizeof fn, "qwk_pfr_f121_c%d", a->K % 512 == 0 ? 2 : 1);
                 return add_launch(b, intern(fn), umin((unsigned)b->g->ncu, a->max_tiles * a->ntn), 64 * QW_WAVES_GU, a, sizeof *a);

@@ -71,6 +71,7 @@ __shared__ uint32_t qw_sst[12 * 16];
 // wave index in the workgroup, as a scalar (so that task indices and row bases stay in scalar registers)
 __device__ __forceinline__ uint32_t qw_wave() { return (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 __device__ __forceinline__ uint32_t qw_lane() { return threadIdx.x & 63; }
+#include "qw_grouped.hip.h"
 constexpr bool qw_has_lut(int f) { return f == 21 || f == QW_F_PACKED || f == QW_F_ABLATE; } // formats decoded through the LDS table (the ablation copies it too)
 __device__ __forceinline__ uint32_t qw_all_tokens(uint32_t nbr) { return nbr >= 32 ? 0xffffffffu : (1u << nbr) - 1; }
 
@@ -2270,7 +2271,7 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_scatter(qwk_scatter_ar
     for (uint32_t i = threadIdx.x; i < a.KD / 8; i += blockDim.x) dst[i] = src[i];
 }
 #endif
-// The four launches above as one, for a step of a few thousand pairs at most: a workgroup per pair, and every workgroup
+// The four launches above as one, for a step of about a thousand pairs at most: a workgroup per pair, and every workgroup
 // counts all pairs itself (LDS atomics over the P ids), which gives it its own packed row without a hand-over: the rows
 // of the experts below its own plus the earlier pairs of its own expert. The order inside an expert is therefore the
 // order of the pairs (the cursor form leaves whatever order the atomics came in; both are permutations the grouped
@@ -2340,6 +2341,91 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_prep(qwk_prep_args a) 
     for (uint32_t t = total_t + tid; t < a.max_tiles; t += 256) *(u4 *)(a.tiles + 4 * t) = u4{0, 0, 0, 0}; // unused entries
 }
 #endif
+// The same for more pairs: a workgroup takes a slice of them, two workgroups a compute unit, so that the counting is not
+// repeated for every pair (a workgroup per pair reads all ids P times: 13.0 us at 2500 pairs). Bound by latency (ids,
+// atomics, scan: about 8 us) and then by the rows' copy. Measured: 2500 pairs of 4 KB rows 13.0 -> 10.3 us; 20480 pairs
+// 72.5 (the four launches) -> 30.3, of which the copy's 168 MB are 32 us at the rate of a large copy.
+#if QW_IN_PART(5)
+extern "C" __global__ __launch_bounds__(512) void qwk_moe_prep_slices(qwk_prep_args a) {
+    __shared__ uint32_t cnt[1024], at[1024], wr[8], wt[8], id[QW_PREP_SLICE], pos[QW_PREP_SLICE];
+    const uint32_t tid = threadIdx.x, nth = blockDim.x, lane = tid & 63, wave = tid >> 6, nwv = nth >> 6;
+    const uint32_t p0 = blockIdx.x * a.slice < a.P ? blockIdx.x * a.slice : a.P, p1 = p0 + a.slice < a.P ? p0 + a.slice : a.P, np = p1 - p0;
+    for (uint32_t e = tid; e < 1024; e += nth) cnt[e] = 0;
+    if (tid < np) id[tid] = a.ids[p0 + tid];
+    __syncthreads();
+    auto count = [&](uint32_t from, uint32_t to) {
+        for (uint32_t q = from + tid; q < to; q += 8 * nth) { // eight ids under way at a time
+            uint32_t e[8];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++) e[i] = q + i * nth < to ? a.ids[q + i * nth] : ~0u;
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++)
+                if (e[i] < a.E) atomicAdd(&cnt[e[i]], 1u);
+        }
+    };
+    count(0, p0);
+    __syncthreads();
+    const uint32_t mine = tid < np ? id[tid] : ~0u;
+    uint32_t rank = mine < a.E ? cnt[mine] : 0; // earlier pairs of this pair's expert
+    for (uint32_t i = 0; i < np; i++) rank += i < tid && id[i] == mine;
+    __syncthreads();
+    count(p0, a.P);
+    __syncthreads();
+    // first packed row and first tile of every expert: thread t has experts per t .. per t + per - 1
+    const uint32_t per = 1024 / nth;
+    uint32_t sr = 0, st = 0;
+    for (uint32_t i = 0; i < per; i++) {
+        const uint32_t c = cnt[per * tid + i];
+        sr += c, st += (c + a.tm - 1) / a.tm;
+    }
+    uint32_t pr = sr, pt = st; // inclusive scans inside the wave
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t ur = __shfl_up(pr, o), ut = __shfl_up(pt, o);
+        if (lane >= (uint32_t)o) pr += ur, pt += ut;
+    }
+    if (lane == 63) wr[wave] = pr, wt[wave] = pt;
+    __syncthreads();
+    uint32_t row0 = pr - sr, tile0 = pt - st, total_t = 0;
+    for (uint32_t w = 0; w < nwv; w++) {
+        if (w < wave) row0 += wr[w], tile0 += wt[w];
+        total_t += wt[w];
+    }
+    for (uint32_t i = 0; i < per; i++) {
+        const uint32_t e = per * tid + i, c = cnt[e], nt = (c + a.tm - 1) / a.tm;
+        at[e] = row0;
+        if (blockIdx.x == 0 && e < a.E) {
+            a.counts[e] = c, a.offs[e] = row0, a.cursor[e] = row0 + c;
+            for (uint32_t t = 0; t < nt; t++) {
+                const uint32_t r = row0 + t * a.tm;
+                if (tile0 + t < a.max_tiles) *(u4 *)(a.tiles + 4 * (tile0 + t)) = u4{e, r, r + a.tm < row0 + c ? r + a.tm : row0 + c, 0};
+            }
+        }
+        row0 += c, tile0 += nt;
+    }
+    if (blockIdx.x == 0)
+        for (uint32_t t = total_t + tid; t < a.max_tiles; t += nth) *(u4 *)(a.tiles + 4 * t) = u4{0, 0, 0, 0}; // unused entries
+    __syncthreads();
+    if (tid < np) a.pos_of[p0 + tid] = pos[tid] = mine < a.E ? at[mine] + rank : 0xffffffffu; // an expert id outside the table: the pair is dropped
+    __syncthreads();
+    const uint32_t units = a.KD / 8; // a wave takes rows, four units of 16 bytes a lane under way at a time
+    for (uint32_t r = wave; r < np; r += nwv) {
+        const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)pos[r]);
+        if (to >= a.P) continue;
+        const u4 *src = (const u4 *)(a.X + (size_t)((p0 + r) / a.topk) * a.KD);
+        u4 *dst = (u4 *)(a.Xs + (size_t)to * a.KD);
+        for (uint32_t i = lane; i < units; i += 256) {
+            u4 v[4];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++)
+                if (i + 64 * k < units) v[k] = src[i + 64 * k];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++)
+                if (i + 64 * k < units) dst[i + 64 * k] = v[k];
+        }
+    }
+}
+#endif
 // H = SiLU(gate) * up, binary16 in and out, the product rounded once (kernels/moe_prefill.metal:95-103, kernels/prefill.metal:485-488)
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(256) void qwk_moe_act(qwk_act_args a) {
@@ -2354,24 +2440,34 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_act(qwk_act_args a) {
     a.H[i] = qw_f2h(g / (1.0f + __expf(-g)) * u);
 }
 #endif
-// y[t][c] = sum_s w[t][s] * D[pos_of[t][s]][c] in rank order; one thread per (token, 4 columns).
+// y[t][c] = sum_s w[t][s] * D[pos_of[t][s]][c] in rank order; one wave per (token, 512 columns), eight columns a lane. The
+// token's rows and weights arrive in one load (lane s: rank s), then all ranks' values are asked for before any is added
+// (as a loop over the ranks these were two dependent round trips a rank).
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(64) void qwk_moe_combine(qwk_combine_args a) {
-    const uint32_t c4 = blockIdx.x * blockDim.x + threadIdx.x, t = blockIdx.y;
-    if (c4 >= a.KD / 4 || t >= a.T) return;
-    float acc[4] = {0, 0, 0, 0};
-    for (uint32_t s = 0; s < a.topk; s++) {
-        const uint32_t p = t * a.topk + s, pos = a.pos_of[p];
-        if (pos >= a.P) continue;
-        const u2 v = *(const u2 *)(a.Dm + (size_t)pos * a.KD + 4 * c4);
-        const float w = a.w[p];
-        acc[0] += w * qw_h2f((uint16_t)v.x), acc[1] += w * qw_h2f((uint16_t)(v.x >> 16));
-        acc[2] += w * qw_h2f((uint16_t)v.y), acc[3] += w * qw_h2f((uint16_t)(v.y >> 16));
+    const uint32_t lane = threadIdx.x, t = blockIdx.y, c8 = blockIdx.x * 64 + lane;
+    const bool on = c8 < a.KD / 8;
+    const uint32_t pl = lane < a.topk ? a.pos_of[t * a.topk + lane] : ~0u;
+    const float wl = lane < a.topk ? a.w[t * a.topk + lane] : 0.0f;
+    const u4 *D = (const u4 *)a.Dm + (on ? c8 : 0);
+    u4 v[16];
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+        const uint32_t pos = (uint32_t)__builtin_amdgcn_readlane((int)pl, s);
+        if (pos < a.P) v[s] = D[(size_t)pos * (a.KD / 8)];
     }
-    u2 o;
-    o.x = (uint32_t)qw_f2h(acc[0]) | (uint32_t)qw_f2h(acc[1]) << 16;
-    o.y = (uint32_t)qw_f2h(acc[2]) | (uint32_t)qw_f2h(acc[3]) << 16;
-    *(u2 *)(a.Y + (size_t)t * a.KD + 4 * c4) = o;
+    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+        if ((uint32_t)__builtin_amdgcn_readlane((int)pl, s) >= a.P) continue;
+        const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wl), s));
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[2 * i] += w * qw_h2f((uint16_t)v[s][i]), acc[2 * i + 1] += w * qw_h2f((uint16_t)(v[s][i] >> 16));
+    }
+    u4 o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = (uint32_t)qw_f2h(acc[2 * i]) | (uint32_t)qw_f2h(acc[2 * i + 1]) << 16;
+    if (on) ((u4 *)a.Y)[(size_t)t * (a.KD / 8) + c8] = o;
 }
 #endif
 
@@ -2460,6 +2556,17 @@ template <int F, int CH> __device__ __forceinline__ void pf_body(const qwk_pf_ar
 QW_PF(21, 2, qwk_pf_f21_c2) QW_PF(21, 1, qwk_pf_f21_c1) QW_PF(8, 4, qwk_pf_f8_c4)
 QW_PF(20, 4, qwk_pf_f20_c4) // IQ4_NL rows (the down projection of the reference model's layer: K = 640)
 QW_PF(121, 2, qwk_pf_f121_c2) QW_PF(121, 1, qwk_pf_f121_c1) // tile-major IQ3_S: one matrix, or gate and up rows side by side
+#endif
+
+#if QW_IN_PART(5)
+extern "C" __global__ __launch_bounds__(64 * QW_PFG_WAVES) void qwk_pfg_f121(qwk_pf_args a) {
+    __shared__ qw_pfg_lds<QW_F_PACKED> L;
+    pfg_body<QW_F_PACKED>(a, L);
+}
+extern "C" __global__ __launch_bounds__(64 * QW_PFG_WAVES) void qwk_pfg_f120(qwk_pf_args a) {
+    __shared__ qw_pfg_lds<QW_F_PACKED_NL> L;
+    pfg_body<QW_F_PACKED_NL>(a, L);
+}
 #endif
 
 // The same product for entries of at most 16 packed rows over tile-major weights, the way the decode kernels work:
