@@ -27,7 +27,7 @@ static const unsigned char qw_code_object[] = {
 };
 
 #define QW_DNQ_MIN_DEFAULT 2u // token count from which down + combine run as one launch of token quarters (qwk_dnq_*)
-enum { QW_MAX_ARGS = 256, QW_MAX_KERNELS = 4096, QW_MAX_BIND = 32, QW_MAX_BYTES = 256, QW_PROF_MAX = 8192, QW_MAX_FUNCS = 256 };
+enum { QW_MAX_ARGS = 288, QW_MAX_KERNELS = 4096, QW_MAX_BIND = 32, QW_MAX_BYTES = 256, QW_PROF_MAX = 8192, QW_MAX_FUNCS = 256 };
 
 // ---------------------------------------------------------------- records
 typedef enum {
@@ -86,7 +86,7 @@ typedef struct {
 typedef struct {
     hipFunction_t f;
     const char *fname;
-    unsigned gx, gy, gz, bx;
+    unsigned gx, gy, gz, bx, lds; // lds: bytes of dynamic LDS
     unsigned char args[QW_MAX_ARGS];
     size_t argsz;
     const char *kname; // caller-visible kernel name (for profiling)
@@ -1064,7 +1064,40 @@ static unsigned pick_split(unsigned chunks, unsigned tiles, unsigned slots) {
         if (chunks % s == 0 && tiles * s <= slots) return s;
     return 1;
 }
-// hw: the buffers the matrices lie in (NULL: no tile-major copies are looked for)
+// A workgroup per tile, a wave per 256 values of K, everything in one round trip (qwk_qmvs). Measured against the
+// persistent kernels over 100 to 131072 rows of 256 to 4096 values, 1 to 16 tokens, it is 5 to 45 % faster while the waves
+// of the launch are on the device at once (32 a compute unit); beyond that the persistent kernels win, whose waves load
+// the next chunk while they multiply this one. With one wave a tile the line lies at two workgroups a compute unit.
+// IQ3_S, whose persistent kernels read a signed value from their table at once, leaves earlier: where a compute unit gets
+// more than four workgroups (each brings the 4 KB table), or more than its LDS holds.
+// unstaged: the persistent kernel would read activations from global memory (rows too long for its LDS) and is the slower
+// one at every size (Q8_0, 30000 x 4096: 100 against 40 us), but for one or two tokens of IQ3_S.
+#define QW_QMVS_WAVES 16u
+static unsigned qmvs_lds(const qwk_qmvm_args *a) { return 16 * a->tabu + a->K / 256 * (a->sh ? 512u << a->sh : 1024u); }
+static bool qmvs_fits(const qw_gpu *g, qwk_qmvm_args *a, unsigned tiles, bool unstaged) {
+    const unsigned ncu = (unsigned)g->ncu, waves = a->K / 256;
+    if (a->K % 256 || !a->K || waves > QW_QMVS_WAVES) return false;
+    bool iq3 = false, tab = false;
+    for (uint32_t j = 0; j < a->nmat; j++) {
+        const uint32_t f = a->fmt[j];
+        if (f == QW_F_PACKED_Q6) return false;
+        iq3 |= f == 21 || f == QW_F_PACKED;
+        tab |= f == 20 || f == 23;
+    }
+    a->tabu = iq3 || tab ? QW_SMALL_TABU : 0;
+    for (a->sh = 0; 1u << a->sh < a->nb; a->sh++) {}
+    if (unstaged && (!iq3 || a->nb > 2)) return true;
+    if (tiles * waves > 32 * ncu) return false;
+    if (iq3 && !unstaged) return tiles <= 4 * ncu && tiles <= 163840 / qmvs_lds(a) * ncu;
+    return tiles <= (waves > 1 ? 8 : 2) * ncu;
+}
+static bool launch_qmvs(qw_batch *b, qwk_qmvm_args *a, unsigned tiles) {
+    a->ctab = (const char *)b->g->tabs + QW_TAB_IQ3C;
+    if (!add_launch(b, a->nb <= 2 ? "qwk_qmvs_x1" : a->nb <= 4 ? "qwk_qmvs_x2" : a->nb <= 8 ? "qwk_qmvs_x4" : "qwk_qmvs_x8", tiles, a->K / 4, a, sizeof *a)) return false;
+    b->l[b->nl - 1].lds = qmvs_lds(a);
+    return true;
+}
+// hw: the buffers the matrices lie in (NULL, a shared expert's rows of one chunk: the persistent kernel, no tile-major copies)
 #define QW_Q6_PACK_MIN_ROWS 16384u
 static bool launch_qmvm(qw_batch *b, qwk_qmvm_args *a, qw_hbuf *const *hw) {
     unsigned tiles = 0;
@@ -1082,6 +1115,7 @@ static bool launch_qmvm(qw_batch *b, qwk_qmvm_args *a, qw_hbuf *const *hw) {
         if (a->fmt[j] == 12 || a->fmt[j] == 13) a->sums = 1;
     }
     if (!tiles) return true;
+    if (hw && qmvs_fits(b->g, a, tiles, false)) return launch_qmvs(b, a, tiles);
     // few tiles: cut every tile's K range over several waves, as far as the wave slots of the device and K allow
     const unsigned waves = QW_WAVES_GU, slots = (unsigned)b->g->ncu * waves;
     a->split = a->K % 256 == 0 ? pick_split(a->K / 256, tiles, slots) : 1;
@@ -1153,6 +1187,11 @@ static bool tr_qmv(qw_batch *b) { // src/engine.c:717-723: 0 W, 3 x, 4 y, 5 {N, 
         if (pk) F = QW_F_PACKED, a.W = pk, a.rowbytes = nblk * QW_SLAB_BYTES;
     }
     if (b->buf[0].h->released && F != QW_F_PACKED) return fail(b, "%s: the GGUF-order bytes of the weights were released and no tile-major copy serves this dispatch", b->k->name);
+    if (!p->valu) {
+        qwk_qmvm_args m = {.K = a.K, .xstride = a.xstride, .nb = a.nb, .yfloat = a.yfloat, .nmat = 1, .x = a.x, .W = {a.W}, .y = {a.y}, .N = {a.N}, .fmt = {(uint32_t)F},
+                           .rowbytes = {a.rowbytes}, .ystride = {a.ystride}, .ntiles = {a.ntiles}};
+        if (qmvs_fits(b->g, &m, a.ntiles, p->K > 2560)) return launch_qmvs(b, &m, a.ntiles);
+    }
     if (p->valu) { // the VALU GEMV, for measurement against the matrix-core form
         if (F != QW_F_PACKED || p->K % 512 || p->NB > 4) return fail(b, "qmv_gg: the VALU form needs packed IQ3_S weights, K a multiple of 512 and NB <= 4");
         fname_fmt(fn, sizeof fn, "qwk_qmv_valu_n%d", p->NB <= 1 ? 1 : p->NB <= 2 ? 2 : 4);
@@ -2052,7 +2091,7 @@ static size_t graph_key(const qw_batch *b, unsigned char *out) {
     size_t n = 0;
     for (int i = 0; i < b->nl; i++) {
         const qw_launch *l = &b->l[i];
-        const unsigned hdr[4] = {l->gx, l->bx, (unsigned)l->argsz, 0};
+        const unsigned hdr[4] = {l->gx, l->bx, (unsigned)l->argsz, l->lds};
         if (out) { memcpy(out + n, &l->f, sizeof l->f); memcpy(out + n + sizeof l->f, hdr, sizeof hdr); memcpy(out + n + sizeof l->f + sizeof hdr, l->args, l->argsz); }
         n += sizeof l->f + sizeof hdr + l->argsz;
     }
@@ -2091,7 +2130,7 @@ static int graph_run(qw_batch *b, hipStream_t st) {
     for (int i = 0; i < b->nl && ok; i++) {
         qw_launch *l = &b->l[i];
         void *params[] = {l->args};
-        ok = hipModuleLaunchKernel(l->f, l->gx, l->gy, l->gz, l->bx, 1, 1, 0, st, params, NULL) == hipSuccess;
+        ok = hipModuleLaunchKernel(l->f, l->gx, l->gy, l->gz, l->bx, 1, 1, l->lds, st, params, NULL) == hipSuccess;
     }
     if (hipStreamEndCapture(st, &graph) != hipSuccess || !ok || !graph || hipGraphInstantiate(&exec, graph, NULL, NULL, 0) != hipSuccess) {
         (void)hipGetLastError();
@@ -2271,7 +2310,7 @@ static bool submit_segment(qw_batch *b, bool last) {
         if (l->side && !b->prof) { // fork: the side stream starts from where the main stream stands now
             if (!side_open && !(side_open = side_link(g, st, side_of(g, b->stream)))) { b->failed = true; return false; }
             void *sparams[] = {l->args};
-            if (!HIPOK(g, hipModuleLaunchKernel(l->f, l->gx, l->gy, l->gz, l->bx, 1, 1, 0, g->side[b->stream], sparams, NULL))) { b->failed = true; return false; }
+            if (!HIPOK(g, hipModuleLaunchKernel(l->f, l->gx, l->gy, l->gz, l->bx, 1, 1, l->lds, g->side[b->stream], sparams, NULL))) { b->failed = true; return false; }
             continue;
         }
         if (l->join && side_open) { // join: the main stream goes on once the side stream has finished
@@ -2283,7 +2322,7 @@ static bool submit_segment(qw_batch *b, bool last) {
             if (!HIPOK(g, hipEventCreate(&b->pev[b->npev])) || !HIPOK(g, hipEventCreate(&b->pev[b->npev + 1])) || !HIPOK(g, hipEventRecord(b->pev[b->npev], st))) { b->failed = true; return false; }
         }
         void *params[] = {l->args}; // every kernel takes one record by value
-        if (!HIPOK(g, hipModuleLaunchKernel(l->f, l->gx, l->gy, l->gz, l->bx, 1, 1, 0, st, params, NULL))) { b->failed = true; return false; }
+        if (!HIPOK(g, hipModuleLaunchKernel(l->f, l->gx, l->gy, l->gz, l->bx, 1, 1, l->lds, st, params, NULL))) { b->failed = true; return false; }
         if (b->prof) {
             if (!HIPOK(g, hipEventRecord(b->pev[b->npev + 1], st))) { b->failed = true; return false; }
             b->npev += 2;
@@ -2464,7 +2503,7 @@ bool qw_hip_batch_launch_static(qw_batch *b, bool recorded) {
     for (int i = 0; ok && i < b->nl; i++) {
         qw_launch *l = &b->l[i];
         void *params[] = {l->args};
-        ok = HIPOK(g, hipModuleLaunchKernel(l->f, l->gx, l->gy, l->gz, l->bx, 1, 1, 0, st, params, NULL));
+        ok = HIPOK(g, hipModuleLaunchKernel(l->f, l->gx, l->gy, l->gz, l->bx, 1, 1, l->lds, st, params, NULL));
     }
     g->na_busy = false;
     return ok;

@@ -15,6 +15,7 @@
 
 /* Pre-signed IQ3_S table inside the lookup-table buffer the callers allocate (kernels/moe_gg.metal:89-95):
  * 8192 entries of four binary16 values at byte offset 49152; the whole buffer is 117760 bytes. */
+#define QW_TAB_IQ3C 0u /* (slot order only) the 512 codebook entries without signs, four binary16 each */
 #define QW_TAB_IQ3SS 49152u
 #define QW_TAB_IQ4 114688u
 #define QW_TAB_Q20 115712u
@@ -37,6 +38,7 @@ typedef struct { /* dense matvec, y[b][row] = W[row] . x[b] */
 
 /* Dense matvec over up to four matrices that share the activations (kernels/qmv_ggm.metal:232-262; one matrix:
  * kernels/qmv_gg.metal:17-39) for the formats 1, 12, 13, 14, 20, 23, 30. 16-row tiles of all matrices form one list. */
+#define QW_SMALL_TABU 264u /* qwk_qmvs: the IQ3_S table in LDS, units of 16 bytes (512 entries without signs, 16 sign masks; IQ4's fits in it) */
 #define QW_KQ_MAXK 4096u /* activations of up to 16 tokens staged in LDS: K * 32 bytes */
 typedef struct {
     const uint8_t *W[4];
@@ -49,6 +51,9 @@ typedef struct {
      * {2, 3, 5, 6}): nothing goes to y; H[t][topk][r] = silu(gate) * up as binary16 hi + lo planes, hplane halves apart */
     uint16_t *H;
     uint32_t topk, hplane;
+    /* qwk_qmvs: the backend's IQ3_S table without signs; 2^sh >= nb; 16-byte units of LDS kept for a table */
+    const void *ctab;
+    uint32_t sh, tabu;
 } qwk_qmvm_args;
 
 /* SwiGLU of the shared expert when its gate/up rows went through the multi-format matvec: g, u float [nb][I] ->

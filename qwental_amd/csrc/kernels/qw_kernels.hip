@@ -72,6 +72,7 @@ __shared__ uint32_t qw_sst[12 * 16];
 __device__ __forceinline__ uint32_t qw_wave() { return (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 __device__ __forceinline__ uint32_t qw_lane() { return threadIdx.x & 63; }
 #include "qw_grouped.hip.h"
+#include "qw_small.hip.h"
 constexpr bool qw_has_lut(int f) { return f == 21 || f == QW_F_PACKED || f == QW_F_ABLATE; } // formats decoded through the LDS table (the ablation copies it too)
 __device__ __forceinline__ uint32_t qw_all_tokens(uint32_t nbr) { return nbr >= 32 ? 0xffffffffu : (1u << nbr) - 1; }
 
@@ -144,7 +145,10 @@ extern "C" __global__ __launch_bounds__(64) void qwk_dq_test_kq(qwk_dq_args a) {
 #if QW_IN_PART(0)
 extern "C" __global__ void qwk_tab_init(qwk_tab_args a) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < QW_LUT_ENTRIES) ((u2 *)(a.tab + QW_TAB_IQ3SS))[a.slot_order ? qw_lut_slot(i) : i] = qw_lut_entry(i);
+    if (i >= QW_LUT_ENTRIES) return;
+    const uint32_t s = qw_lut_slot(i);
+    ((u2 *)(a.tab + QW_TAB_IQ3SS))[a.slot_order ? s : i] = qw_lut_entry(i);
+    if (a.slot_order && !(s & 15)) ((u2 *)(a.tab + QW_TAB_IQ3C))[s >> 5 | ((s >> 4) & 1) << 8] = qw_lut_entry(i);
 }
 #endif
 
@@ -290,6 +294,50 @@ template <int F, int CH, bool XLDS> __device__ __forceinline__ void qmv_body(con
 #if QW_IN_PART(0)
 QW_QMV(21, 2, true, _c2) QW_QMV(21, 1, true, _c1) QW_QMV(21, 1, false, _c1g)
 QW_QMV(121, 2, true, _c2) QW_QMV(121, 1, true, _c1) // packed IQ3_S: a.rowbytes = bytes of a 16-row tile
+#endif
+
+// Matrices that the device takes in one go, one to four a launch, any of the formats: qw_small.hip.h.
+#if QW_IN_PART(0)
+template <int XN> __device__ __forceinline__ void qmvs_body(const qwk_qmvm_args &a, u4 *dyn) { // dyn: table (tabu units), then a wave's activations, behind them in the same place its partial sums
+    const uint32_t lane = qw_lane(), wave = qw_wave(), nw = blockDim.x >> 6, own = a.sh ? 32u << a.sh : 64;
+    u2 *tab = (u2 *)dyn;
+    u4 *x = dyn + a.tabu + wave * own;
+    uint32_t j = 0, t = blockIdx.x;
+    while (j + 1 < a.nmat && t >= a.ntiles[j]) t -= a.ntiles[j++];
+    f4 acc = {0, 0, 0, 0};
+    switch (a.fmt[j]) {
+    case 8: acc = qmvs_part<8, XN>(a, j, t, tab, x); break;
+    case 12: acc = qmvs_part<12, XN>(a, j, t, tab, x); break;
+    case 13: acc = qmvs_part<13, XN>(a, j, t, tab, x); break;
+    case 14: acc = qmvs_part<14, XN>(a, j, t, tab, x); break;
+    case 20: acc = qmvs_part<20, XN>(a, j, t, tab, x); break;
+    case 21: acc = qmvs_part<21, XN>(a, j, t, tab, x); break;
+    case 23: acc = qmvs_part<23, XN>(a, j, t, tab, x); break;
+    case QW_F_PACKED: acc = qmvs_part<QW_F_PACKED, XN>(a, j, t, tab, x); break;
+    case 1: acc = qmvs_part<1, XN>(a, j, t, tab, x); break;
+    case 30: acc = qmvs_part<30, XN>(a, j, t, tab, x); break;
+    }
+    if (wave) ((f4 *)x)[lane] = acc;
+    __syncthreads();
+    if (wave) return;
+    for (uint32_t q = 1; q < nw; q++) acc += ((const f4 *)x)[q * own + lane];
+    const uint32_t r = 16 * t + (lane & 15), kg = lane >> 4;
+    if (r < a.N[j])
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            const uint32_t tok = 4 * kg + i;
+            if (tok < a.nb) {
+                if (a.yfloat) ((float *)a.y[j])[(size_t)tok * a.ystride[j] + r] = acc[i];
+                else ((uint16_t *)a.y[j])[(size_t)tok * a.ystride[j] + r] = qw_f2h(acc[i]);
+            }
+        }
+}
+#define QW_QMVS(XN)                                                                                  \
+    extern "C" __global__ __launch_bounds__(1024) void qwk_qmvs_x##XN(qwk_qmvm_args a) {              \
+        extern __shared__ u4 qw_dyn[];                                                                \
+        qmvs_body<XN>(a, qw_dyn);                                                                \
+    }
+QW_QMVS(1) QW_QMVS(2) QW_QMVS(4) QW_QMVS(8)
 #endif
 
 // ---- the other formats, one to four matrices a launch (kernels/qmv_ggm.metal:232-262).

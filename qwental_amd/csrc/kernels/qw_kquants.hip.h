@@ -277,7 +277,7 @@ __device__ __forceinline__ void qw_split_bf(h8 x, bf8 &hi, bf8 &lo) {
 }
 
 // One step of a block into the accumulator (tokens 4 kg .. 4 kg + 3 of row lane & 15).
-template <int F, int S> __device__ __forceinline__ void qw_kq_step(const qw_kq<F> &b, const uint32_t *tab, const qw_afrag_kq &af, uint32_t kb, uint32_t kg, f4 &acc) {
+template <int F, int S, class AFK> __device__ __forceinline__ void qw_kq_step(const qw_kq<F> &b, const uint32_t *tab, const AFK &af, uint32_t kb, uint32_t kg, f4 &acc) {
     typename qw_kq<F>::W w;
     float a, c;
     b.template dec<S>(tab, kg, w, a, c);
@@ -294,7 +294,7 @@ template <int F, int S> __device__ __forceinline__ void qw_kq_step(const qw_kq<F
     else acc += a * sub;
     if constexpr (qw_kq<F>::HAS_MIN) acc -= c * af.sum32(kb + 32 * S);
 }
-template <int F, int S = 0> __device__ __forceinline__ void qw_kq_block(const qw_kq<F> &b, const uint32_t *tab, const qw_afrag_kq &af, uint32_t kb, uint32_t kg, f4 &acc) {
+template <int F, int S = 0, class AFK> __device__ __forceinline__ void qw_kq_block(const qw_kq<F> &b, const uint32_t *tab, const AFK &af, uint32_t kb, uint32_t kg, f4 &acc) {
     if constexpr (S < (int)qw_kq<F>::STEPS) {
         qw_kq_step<F, S>(b, tab, af, kb, kg, acc);
         qw_kq_block<F, S + 1>(b, tab, af, kb, kg, acc);

@@ -1,0 +1,132 @@
+// The dense product for matrices that the device takes in one go (the projections of a decode step): one workgroup per tile
+// of 16 rows, one wave per 256 values of K. Such a launch is bound by latency, not by bytes (4096 x 2048 in IQ3_S is 14 KB a
+// compute unit), so everything a wave needs is asked for at its entry and in one round trip: its block of the sixteen rows,
+// its 256 values of every token, and for IQ3_S its share of a 4 KB table. Nothing is staged for the whole workgroup: a wave
+// puts its tokens into LDS for itself (coalesced loads, 512 bytes a token; read back in fragment order). The partial sums
+// of the waves meet in LDS and are added in the order of K.
+// The persistent kernels copy 64 KB of pre-signed table and all tokens' activations into every compute unit first
+// (2 to 3 us, behind it the weights' round trip). One launch of a chain of them, one token, 2048 values, us there -> here:
+// 2000 rows IQ3_S 6.0 -> 4.0, Q8_0 8.0 -> 4.9, Q4_K 8.2 -> 4.2, Q6_K 9.7 -> 5.1; 8192 rows 6.5 -> 5.8, 8.4 -> 6.5, 8.7 ->
+// 5.7, 10.2 -> 6.6; 4096 x 4096 9.6 -> 6.1, 20.2 -> 6.6, 12.4 -> 5.9, 16.6 -> 7.0 (16 tokens: 16.9 -> 7.5, 22 -> 8.1).
+#pragma once
+#include "qw_kquants.hip.h"
+
+// A wave's 256 values of up to 16 tokens in LDS: chunk c (8 values) of token m at (c << sh) + (m ^ (c & (2^sh - 1))), units of 16
+// bytes, 2^sh >= tokens: neither the writes (a token's chunks by 32 lanes) nor the reads (16 tokens of a chunk) meet in a bank.
+struct qw_afrag_small {
+    const u4 *x;
+    uint32_t m, sh; // m: lane & 15, taken modulo 2^sh (lanes without a token read another's; their results are not stored)
+    static constexpr bool has_lo = false;
+    __device__ __forceinline__ uint32_t unit(uint32_t c) const { return (c << sh) + (m ^ (c & ((1u << sh) - 1))); }
+    __device__ __forceinline__ h8 at8(uint32_t k) const { return __builtin_bit_cast(h8, x[unit(k >> 3)]); }
+    __device__ __forceinline__ h4 at4(uint32_t k) const { return __builtin_bit_cast(h4, ((const u2 *)x)[unit(k >> 3) * 2 + ((k >> 2) & 1)]); }
+    __device__ __forceinline__ h8 hi(uint32_t k) const { return at8(k); }
+    __device__ __forceinline__ h8 lo(uint32_t) const { return h8{}; }
+    __device__ __forceinline__ h4 hi4(uint32_t k) const { return at4(k); }
+    __device__ __forceinline__ h4 lo4(uint32_t) const { return h4{}; }
+};
+
+// Eight values of step J of an IQ3_S block from the 4 KB table: the magnitudes of two codebook entries, their signs put in by
+// masks (bit j of a nibble is the sign of value j), then the sub-block factor, as in qw_iq3_step.
+template <int J> __device__ __forceinline__ h8 qw_small_iq3(const qw_iq3_slice &s, const u2 *tab) {
+    constexpr int t = J / 4, j = J % 4;
+    const uint32_t q = s.qs[J / 2] >> (16 * (J % 2)), h = s.qh >> (8 * t + 2 * j), n = s.sg[t] >> (8 * j);
+    const u2 m0 = tab[(q & 255) | (h & 1) << 8], m1 = tab[((q >> 8) & 255) | (h & 2) << 7], s0 = tab[512 + (n & 15)], s1 = tab[512 + ((n >> 4) & 15)];
+    const h2 ff = qw_iq3_factor(s, t);
+    u4 raw = {m0.x ^ s0.x, m0.y ^ s0.y, m1.x ^ s1.x, m1.y ^ s1.y};
+#pragma unroll
+    for (int i = 0; i < 4; i++) raw[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, (uint32_t)raw[i]) * ff);
+    return __builtin_bit_cast(h8, raw);
+}
+template <int J> __device__ __forceinline__ void qw_small_iq3_steps(const qw_iq3_slice &s, const u2 *tab, const qw_afrag_small &af, uint32_t kg, f4 (&sub)[2]) {
+    if constexpr (J < 8) {
+        sub[J & 1] = qw_mfma(af.at8(64 * kg + 8 * J), qw_small_iq3<J>(s, tab), sub[J & 1]);
+        qw_small_iq3_steps<J + 1>(s, tab, af, kg, sub);
+    }
+}
+
+// 256 values of K of one tile as the wave loads and multiplies them.
+template <int F> struct qw_small_blk { // Q4_K, Q5_K, Q6_K, IQ4_XS; eight blocks of IQ4_NL, binary16, bfloat16
+    static constexpr int NB = qw_kq<F>::BLK_K == 256 ? 1 : 8;
+    typedef qw_chunk_kq<F, NB> C;
+    static constexpr uint32_t BYTES = NB * qw_kq<F>::BLK_B;
+    static __device__ __forceinline__ f4 mac(const C &c, const u2 *tab, const qw_afrag_small &af, uint32_t kg) {
+        f4 acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            if constexpr (qw_kq<F>::HAS_MIN) qw_kq_block_af<F>(c.b[i], (const uint32_t *)tab, af, qw_kq<F>::BLK_K * i, kg, acc);
+            else qw_kq_block<F>(c.b[i], (const uint32_t *)tab, af, qw_kq<F>::BLK_K * i, kg, acc);
+        }
+        return acc;
+    }
+};
+template <> struct qw_small_blk<8> {
+    typedef qw_chunk<8, 8> C;
+    static constexpr uint32_t BYTES = 8 * 34;
+    static __device__ __forceinline__ f4 mac(const C &c, const u2 *, const qw_afrag_small &af, uint32_t kg) {
+        f4 acc = {0, 0, 0, 0};
+        c.mac(nullptr, af, 0, kg, acc);
+        return acc;
+    }
+};
+template <> struct qw_small_blk<21> {
+    typedef qw_chunk<21, 1> C;
+    static constexpr uint32_t BYTES = 110;
+    static __device__ __forceinline__ f4 mac(const C &c, const u2 *tab, const qw_afrag_small &af, uint32_t kg) {
+        f4 sub[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+        qw_small_iq3_steps<0>(c.s[0], tab, af, kg, sub);
+        return c.s[0].d * (sub[0] + sub[1]);
+    }
+};
+template <> struct qw_small_blk<QW_F_PACKED> {
+    typedef qw_chunk<QW_F_PACKED, 1> C;
+    static constexpr uint32_t BYTES = QW_SLAB_BYTES;
+    static __device__ __forceinline__ f4 mac(const C &c, const u2 *tab, const qw_afrag_small &af, uint32_t kg) { return qw_small_blk<21>::mac(c, tab, af, kg); }
+};
+
+// The wave's part of tile t of matrix j: block `wave` of the rows. x: the wave's own LDS. XN: loads of two tokens, 2 XN >= nb.
+template <int F, int XN> __device__ __forceinline__ f4 qmvs_part(const qwk_qmvm_args &a, uint32_t j, uint32_t t, u2 *tab, u4 *x) {
+    typedef qw_small_blk<F> B;
+    constexpr bool iq3 = F == 21 || F == QW_F_PACKED, iq4 = F == 20 || F == 23;
+    const uint32_t lane = qw_lane(), wave = qw_wave(), n = lane & 15, kg = lane >> 4, row = 16 * t + (lane >> 2);
+    // the part of the 256 units of table that this thread puts into LDS: one from 256 threads on, else four (some by several threads)
+    u4 te[4];
+    const bool many = blockDim.x < 256;
+    if constexpr (iq3) {
+        te[0] = ((const u4 *)a.ctab)[threadIdx.x & 255];
+        if (many)
+#pragma unroll
+            for (uint32_t i = 1; i < 4; i++) te[i] = ((const u4 *)a.ctab)[(threadIdx.x + i * 64) & 255];
+    }
+    u4 xv[XN];
+    const uint16_t *xs = a.x + wave * 256 + 8 * (lane & 31);
+#pragma unroll
+    for (uint32_t i = 0; i < XN; i++) {
+        const uint32_t m = 2 * i + (lane >> 5);
+        xv[i] = *(const u4 *)(xs + (size_t)(m < a.nb ? m : a.nb - 1) * a.xstride);
+    }
+    typename B::C c;
+    if constexpr (F == QW_F_PACKED) c.load(a.W[j] + (size_t)t * a.rowbytes[j] + wave * B::BYTES, lane);
+    else c.load(a.W[j] + (size_t)(row < a.N[j] ? row : a.N[j] - 1) * a.rowbytes[j] + wave * B::BYTES, lane & 3);
+    if constexpr (iq3) {
+        ((u4 *)tab)[threadIdx.x & 255] = te[0];
+        if (many)
+#pragma unroll
+            for (uint32_t i = 1; i < 4; i++) ((u4 *)tab)[(threadIdx.x + i * 64) & 255] = te[i];
+        if (threadIdx.x < 16) {
+            const uint32_t s = threadIdx.x;
+            tab[512 + s] = u2{(s & 1) << 15 | (s & 2) << 30, (s & 4) << 13 | (s & 8) << 28};
+        }
+    }
+    if constexpr (iq4) qw_kq_tab_build((uint32_t *)tab);
+#pragma unroll
+    for (uint32_t i = 0; i < XN; i++) {
+        const uint32_t m = 2 * i + (lane >> 5), cc = lane & 31;
+        if (m < (1u << a.sh)) x[(cc << a.sh) + (m ^ (cc & ((1u << a.sh) - 1)))] = xv[i];
+    }
+    if constexpr (iq3 || iq4) __syncthreads();
+    else __builtin_amdgcn_wave_barrier(); // (a wave's LDS operations complete in order)
+    c.transpose();
+    const qw_afrag_small af = {x, n & ((1u << a.sh) - 1), a.sh};
+    return B::mac(c, tab, af, kg);
+}
