@@ -98,7 +98,7 @@ unsigned qw_hip_graph_launches(const qw_gpu *g);
  *   QW_HIP_PK_SPLIT           the packing sequence (p_zero, moe_count, moe_plan_t, moe_scatter, moe_pf_gg x 2, p_act2) one launch per
  *                             dispatch instead of one launch for the first four and SwiGLU inside the gate / up launch
  *   QW_HIP_SIDE=1             a shared expert's gate/up in the K-quant / IQ4 / plain formats runs on a side stream beside the router
- *   QW_HIP_DN_ANY             IQ4_NL down rows take the any-shape kernel instead of the range kernel
+ *   QW_HIP_DN_ANY             IQ4_NL, K-quant and IQ4_XS down rows take the any-shape kernel instead of the range kernel
  *   QW_HIP_NL_C4              IQ4_NL down rows from GGUF order in chunks of four blocks instead of ten
  *   QW_HIP_NO_SWIGLU_MATVEC   such a shared expert's gate/up as two launches (matvec, then SwiGLU) instead of one
  *   QW_HIP_KQ_OWN_LAUNCH      such a shared expert's gate/up as a launch of its own instead of on the workgroups behind the router's

@@ -1587,6 +1587,20 @@ static bool tr_dn_inner(qw_batch *b) {
     // A pair of types without a build of its own (Q4_K, Q5_K, Q6_K or IQ4_XS on either side; IQ4_NL beside IQ3_S): the
     // kernel that takes both types as arguments, rows in GGUF order.
     const bool kq_d = rt_ok(fd) && fd != 20, kq_s = rt_ok(fs) && fs != 20;
+    // The range kernel on GGUF rows (I is a multiple of the block, 256, and H rows fit in LDS up to 512; they are copied 16 bytes a lane)
+    if (kq_d && (fs == 0 || fs == fd || fs == 8) && p->I <= 512 && (uintptr_t)a.H % 16 == 0 && !rel && !b->sw.dn_any) {
+        char fn[48], tail[16] = "";
+        if (fs) fname_fmt(tail, sizeof tail, "_s%d_c%d", fs, fs == 8 ? 4 : 1);
+        fname_fmt(fn, sizeof fn, "qwk_dnr_f%d_c1%s", fd, tail);
+        const unsigned grid = persistent_grid(b->g, umax * (unsigned)(p->D / 16) + (unsigned)p->D / 16, QW_WAVES_DNR);
+        if (nbr > b->sw.dnc_nb) return add_launch(b, intern(fn), grid, 64 * QW_WAVES_DNR, &a, sizeof a);
+        char fu[48]; // a few tokens: wait for the combine, the two run as one launch
+        fname_fmt(fu, sizeof fu, "qwk_dnc_f%d_c1%s", fd, tail);
+        b->pend_dn.valid = true;
+        b->pend_dn.a = a;
+        b->pend_dn.fname = intern(fn), b->pend_dn.fused = intern(fu), b->pend_dn.kname = b->k->name, b->pend_dn.grid = grid, b->pend_dn.fused_grid = (unsigned)p->D / 16, b->pend_dn.quarters = false;
+        return true;
+    }
     if (kq_d || kq_s || ((fd == 20 || fs == 20) && (fd != 20 || (fs != 0 && fs != 20 && fs != 8)))) {
         if (rel) return fail(b, "%s: the GGUF-order bytes of the weights were released and no tile-major copy serves this dispatch", b->k->name);
         a.fd = (uint32_t)fd, a.fsd = (uint32_t)fs;

@@ -1454,6 +1454,7 @@ template <int F, int CH> __device__ __forceinline__ void shared_down_tiles(const
 // range of at most D / 16 tasks, which touches at most two experts: their H rows (both planes, only the tokens
 // that picked them) are copied into LDS once, in fragment order, and the waves then stream the range's tiles with operand A read
 // from LDS. The first weight loads are issued before the table copy, the row copy and the barrier.
+constexpr bool qw_has_tab(int F) { return F == 20 || F == 23 || F == QW_F_PACKED_NL; } // decoders that read the byte table of qw_kq_tab_build
 constexpr bool qw_tiled(int F) { return F == QW_F_PACKED || F == QW_F_PACKED_NL; } // weights come from a tile-major copy
 struct qw_dn_seg { // one expert's part of a workgroup's range (all fields wave-uniform)
     const uint8_t *W;  // the expert's matrix
@@ -1509,7 +1510,7 @@ template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_r
     auto div_tpe = [&](uint32_t x) { return tp2 ? x >> tsh : x / tpe; };
     qw_sel_load(*sc, a.sel, K, gnb); // one memory round trip for everything the ranges depend on
     if (qw_has_lut(F) || qw_has_lut(FSD)) qw_lut_copy_issue(lut, (const u2 *)a.glut); // lands in LDS meanwhile; awaited in ready()
-    if (F == 20 || FSD == 20 || F == QW_F_PACKED_NL || FSD == QW_F_PACKED_NL) qw_kq_tab_build((uint32_t *)lut); // the byte table of the 4-bit codebook instead
+    if (qw_has_tab(F) || qw_has_tab(FSD)) qw_kq_tab_build((uint32_t *)lut); // the byte table of the 4-bit codebook instead
     __syncthreads();
     const uint32_t *ue = sc->ue, *mask = sc->mask;
     const uint8_t *slot = sc->slot;
@@ -1596,7 +1597,7 @@ template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_r
 }
 #define QW_DN_RANGE(F, CH, FSD, CHSD, NAME)                                                       \
     extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) {                  \
-        __shared__ struct { u2 lut[(qw_has_lut(F) || qw_has_lut(FSD)) ? QW_LUT_ENTRIES : 1]; uint16_t arows[2 * 16 * 2 * 512]; qw_sel_cache sc; } L; \
+        __shared__ struct { u2 lut[(qw_has_lut(F) || qw_has_lut(FSD)) ? QW_LUT_ENTRIES : (qw_has_tab(F) || qw_has_tab(FSD)) ? QW_KQ_TAB / 2 : 1]; uint16_t arows[2 * 16 * 2 * 512]; qw_sel_cache sc; } L; \
         dn_range_body<F, CH, FSD, CHSD>(a, L.lut, L.arows, &L.sc);                                \
     }
 // IQ4_NL rows (the reference model's down projections: I = 640, five chunks of 4 blocks a row): no IQ3_S table in LDS,
@@ -1629,6 +1630,14 @@ QW_DN_RANGE(21, 1, 0, 1, qwk_dnr_f21_c1) QW_DN_RANGE(21, 1, 21, 1, qwk_dnr_f21_c
 QW_DN_RANGE(121, 2, 0, 1, qwk_dnr_f121_c2) QW_DN_RANGE(121, 2, 121, 2, qwk_dnr_f121_c2_s121_c2) QW_DN_RANGE(121, 2, 8, 4, qwk_dnr_f121_c2_s8_c4)
 QW_DN_RANGE(121, 1, 0, 1, qwk_dnr_f121_c1) QW_DN_RANGE(121, 1, 121, 1, qwk_dnr_f121_c1_s121_c1) QW_DN_RANGE(121, 1, 8, 4, qwk_dnr_f121_c1_s8_c4)
 QW_DN_RANGE(8, 4, 0, 1, qwk_dnr_f8_c4) QW_DN_RANGE(8, 4, 8, 4, qwk_dnr_f8_c4_s8_c4) QW_DN_RANGE(8, 4, 21, 2, qwk_dnr_f8_c4_s21_c2) QW_DN_RANGE(8, 4, 21, 1, qwk_dnr_f8_c4_s21_c1)
+#endif
+// Q4_K, Q5_K, Q6_K and IQ4_XS rows, I = 256 or 512, one block a chunk (three chunk buffers); the shared expert's rows of
+// the same type or Q8_0. These rows took the any-shape kernel (qwk_dn_rt): 8 waves, H rows read from memory by every wave
+// for every tile, one tile's loads at a time. Q6_K, 512 experts of 2048 x 512, four tokens: 44.2 -> 17.5 us a launch (34 MB).
+#define QW_DN_RANGE_KQ(F)                                                                         \
+    QW_DN_RANGE(F, 1, 0, 1, qwk_dnr_f##F##_c1) QW_DN_RANGE(F, 1, F, 1, qwk_dnr_f##F##_c1_s##F##_c1) QW_DN_RANGE(F, 1, 8, 4, qwk_dnr_f##F##_c1_s8_c4)
+#if QW_IN_PART(3)
+QW_DN_RANGE_KQ(12) QW_DN_RANGE_KQ(13) QW_DN_RANGE_KQ(14) QW_DN_RANGE_KQ(23)
 #endif
 
 // Down + combine in one launch for a few tokens (at most QW_DNC_MAXNB; kernels/moe_gg.metal:639-663 in one pass).
@@ -1673,7 +1682,7 @@ __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *p
     qw_sel_load(*sc, a.sel, K, gnb);
     const float *wg = (const float *)(a.sel + QW_SEL_OFF_W(gnb, K));
     for (uint32_t i = threadIdx.x; i < a.nbr * (K + 1); i += blockDim.x) wl[i] = wg[i];
-    if (F == QW_F_PACKED_NL || FSD == QW_F_PACKED_NL) qw_kq_tab_build((uint32_t *)lut); // the byte table of the 4-bit codebook instead
+    if (qw_has_tab(F) || qw_has_tab(FSD)) qw_kq_tab_build((uint32_t *)lut); // the byte table of the 4-bit codebook instead
     if constexpr (TAB) {
 #pragma unroll
         for (uint32_t it = 0; it < TPER; it++) ((u4 *)lut)[tat[it]] = tabv[it];
@@ -1730,7 +1739,7 @@ __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *p
 }
 #define QW_DNC(F, CH, FSD, CHSD, NAME)                                                              \
     extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) {                    \
-        __shared__ struct { u2 lut[(qw_has_lut(F) || qw_has_lut(FSD)) ? QW_LUT_ENTRIES : (F == QW_F_PACKED_NL || FSD == QW_F_PACKED_NL) ? QW_KQ_TAB / 2 : 1]; float part[QW_DNC_MAXNB * 17 * 16], wl[QW_DNC_MAXNB * 17]; qw_sel_cache sc; } L; \
+        __shared__ struct { u2 lut[(qw_has_lut(F) || qw_has_lut(FSD)) ? QW_LUT_ENTRIES : (qw_has_tab(F) || qw_has_tab(FSD)) ? QW_KQ_TAB / 2 : 1]; float part[QW_DNC_MAXNB * 17 * 16], wl[QW_DNC_MAXNB * 17]; qw_sel_cache sc; } L; \
         dnc_body<F, CH, FSD, CHSD>(a, L.lut, L.part, L.wl, &L.sc);                                  \
     }
 #if QW_IN_PART(4)
@@ -1738,6 +1747,8 @@ QW_DNC(121, 2, 0, 1, qwk_dnc_f121_c2) QW_DNC(121, 2, 121, 2, qwk_dnc_f121_c2_s12
 QW_DNC(121, 1, 0, 1, qwk_dnc_f121_c1) QW_DNC(121, 1, 121, 1, qwk_dnc_f121_c1_s121_c1) QW_DNC(121, 1, 8, 4, qwk_dnc_f121_c1_s8_c4)
 QW_DNC(8, 4, 0, 1, qwk_dnc_f8_c4) QW_DNC(8, 4, 8, 4, qwk_dnc_f8_c4_s8_c4)
 QW_DNC(120, 10, 0, 10, qwk_dnc_f120_c10) QW_DNC(120, 10, 120, 10, qwk_dnc_f120_c10_s120_c10) QW_DNC(120, 10, 8, 4, qwk_dnc_f120_c10_s8_c4) // tile-major IQ4_NL rows of 640
+#define QW_DNC_KQ(F) QW_DNC(F, 1, 0, 1, qwk_dnc_f##F##_c1) QW_DNC(F, 1, F, 1, qwk_dnc_f##F##_c1_s##F##_c1) QW_DNC(F, 1, 8, 4, qwk_dnc_f##F##_c1_s8_c4)
+QW_DNC_KQ(12) QW_DNC_KQ(13) QW_DNC_KQ(14) QW_DNC_KQ(23)
 #endif
 
 // Down + combine in one launch for 3 to 16 tokens. The range form above needs a second launch because the products
