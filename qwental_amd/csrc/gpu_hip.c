@@ -1350,8 +1350,8 @@ static bool shared_gu_kq(qw_batch *b, uint32_t nbr, const uint16_t *x, uint16_t 
     const int first = b->nl;
     // one launch when the K range splits so that a workgroup holds whole (gate tile, up tile) pairs; else matvec, then SwiGLU
     unsigned sw = 0;
-    for (unsigned s = 6; s > 1 && !sw; s--)
-        if (s != 4 && (unsigned)(p->D / 256) % s == 0 && !b->sw.no_swiglu_matvec) sw = s;
+    for (unsigned s = QW_WAVES_GU / 2; s > 1 && !sw; s--)
+        if ((unsigned)(p->D / 256) % s == 0 && !b->sw.no_swiglu_matvec) sw = s;
     if (sw) {
         m.split = sw, m.sums = 0, m.H = h, m.topk = (uint32_t)p->topk, m.hplane = sa.hplane;
         for (int j = 0; j < 2; j++) {

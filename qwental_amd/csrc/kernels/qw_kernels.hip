@@ -407,27 +407,37 @@ template <int F, int NB> __device__ __forceinline__ void qmvm_matrix_split(const
         __syncthreads();
     }
 }
-// One part of one tile: the product over chunks [part * cpp, (part + 1) * cpp) of the rows of tile t of matrix j.
-template <int F, int NB> __device__ __forceinline__ f4 qmvm_part(const qwk_qmvm_args &a, uint32_t j, const uint32_t *tab, const qw_afrag_kq &af, uint32_t t, uint32_t part) {
+// One part of one tile: the product over chunks [part * cpp, (part + 1) * cpp) of the rows of tile t of matrix j; ready() as in qw_task_pipeline.
+template <int F, int NB, class S> __device__ __forceinline__ f4 qmvm_part(const qwk_qmvm_args &a, uint32_t j, const uint32_t *tab, const qw_afrag_kq &af, uint32_t t, uint32_t part, S ready) {
     typedef qw_chunk_kq<F, NB> C;
     const qmvm_tile<F, NB> T = {a, j};
     const uint32_t lane = qw_lane(), kg = lane >> 4, cpp = a.K / (C::BLK_K * NB) / a.split;
     f4 acc = {0, 0, 0, 0};
     qw_task_pipeline<C>(1, 0, 1, cpp, NB * C::BLK_B, lane & 3, [&](uint32_t) { return T.rowp(t) + (size_t)part * cpp * NB * C::BLK_B; },
-                        [&](uint32_t, uint32_t ci, const C &c) { c.mac(tab, af, (part * cpp + ci) * NB * C::BLK_K, kg, acc); });
+                        [&](uint32_t, uint32_t ci, const C &c) { c.mac(tab, af, (part * cpp + ci) * NB * C::BLK_K, kg, acc); }, ready);
     return acc;
 }
 // The shared expert's gate/up in the other format family with SwiGLU in the same launch (kernels/moe_gg.metal:563-573):
 // matrix 0 holds the gate rows, matrix 1 the up rows, each of its own format. A workgroup takes 12 / split / 2 pairs of
-// tiles (gate tile t and up tile t side by side), split waves a tile as in qwk_qmvm; the partial sums meet in LDS, and
+// tiles (gate tile t and up tile t side by side), split waves a tile; the partial sums meet in LDS, and
 // the first wave of a gate tile adds up both tiles in part order, applies SwiGLU and stores H's two planes.
+// The work is a megabyte or two over a few dozen workgroups and bound by its round trips: the activations are asked for
+// first (straight into LDS), every wave asks for its blocks behind them (up to two, which all K up to 3072 come down to), and
+// only then the workgroup waits, once. (The weights asked for after the activations and their sums had arrived: four tokens, 512 columns of 2048 in Q4_K 13.7 us a front launch, now 9.0; eight tokens, 640 of 2560 in Q4_K and IQ4_XS 10.5, now 10.0.
+// Sixteen waves with a block each: 128 registers, which spill.)
 // bid of nblk: the workgroup's number among those that do this work (the front launch puts the router's workgroups first).
-struct qw_qmvm_lds { u4 xf[QW_KQ_MAXK * 2]; float xs[QW_KQ_MAXK / 2]; uint32_t tab[QW_KQ_TAB]; f4 red[QW_WG_QMVM]; };
-__device__ __forceinline__ void qmvm_swiglu_body(const qwk_qmvm_args &a, qw_qmvm_lds &L, uint32_t bid, uint32_t nblk) {
+struct qw_swiglu_lds { u4 xf[QW_KQ_MAXK * 2]; float xs[QW_KQ_MAXK / 2]; uint32_t tab[QW_KQ_TAB]; f4 red[QW_WG_QMVM]; };
+__device__ __forceinline__ void qmvm_swiglu_body(const qwk_qmvm_args &a, qw_swiglu_lds &L, uint32_t bid, uint32_t nblk) {
     qw_kq_tab_build(L.tab);
-    qw_stage_x(L.xf, a.x, a.xstride, a.K, a.nb);
-    __syncthreads();
-    if (a.sums) { // sums of 32 activations per token, in index order
+    qw_stage_x_issue(L.xf, a.x, a.xstride, a.K, a.nb);
+    bool staged = false;
+    auto ready = [&] { // once per wave, behind its first weight loads
+        if (staged) return;
+        staged = true;
+        qw_lds_arrive();
+        __syncthreads();
+        if (!a.sums) return;
+        // sums of 32 activations per token, in index order
         for (uint32_t i = threadIdx.x; i < (a.K >> 5) * 16; i += blockDim.x) {
             const uint32_t c = i >> 4, m = i & 15;
             float sum = 0;
@@ -440,7 +450,7 @@ __device__ __forceinline__ void qmvm_swiglu_body(const qwk_qmvm_args &a, qw_qmvm
             L.xs[i] = sum;
         }
         __syncthreads();
-    }
+    };
     const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave(), sp = a.split;
     const qw_afrag_kq af = {L.xf, L.xs, n, kg};
     const uint32_t pairs = (QW_WG_QMVM / 64) / sp / 2, slot = wave / sp, part = wave % sp, which = slot & 1, ntiles = a.ntiles[0];
@@ -450,15 +460,16 @@ __device__ __forceinline__ void qmvm_swiglu_body(const qwk_qmvm_args &a, qw_qmvm
         f4 acc = {0, 0, 0, 0};
         if (t < ntiles) {
             switch (a.fmt[which]) { // uniform in a wave
-            case 12: acc = qmvm_part<12, 1>(a, which, L.tab, af, t, part); break;
-            case 13: acc = qmvm_part<13, 1>(a, which, L.tab, af, t, part); break;
-            case 14: acc = qmvm_part<14, 1>(a, which, L.tab, af, t, part); break;
-            case 23: acc = qmvm_part<23, 1>(a, which, L.tab, af, t, part); break;
-            case 20: acc = qmvm_part<20, 8>(a, which, L.tab, af, t, part); break;
-            case 1: acc = qmvm_part<1, 8>(a, which, L.tab, af, t, part); break;
-            case 30: acc = qmvm_part<30, 8>(a, which, L.tab, af, t, part); break;
+            case 12: acc = qmvm_part<12, 1>(a, which, L.tab, af, t, part, ready); break;
+            case 13: acc = qmvm_part<13, 1>(a, which, L.tab, af, t, part, ready); break;
+            case 14: acc = qmvm_part<14, 1>(a, which, L.tab, af, t, part, ready); break;
+            case 23: acc = qmvm_part<23, 1>(a, which, L.tab, af, t, part, ready); break;
+            case 20: acc = qmvm_part<20, 8>(a, which, L.tab, af, t, part, ready); break;
+            case 1: acc = qmvm_part<1, 8>(a, which, L.tab, af, t, part, ready); break;
+            case 30: acc = qmvm_part<30, 8>(a, which, L.tab, af, t, part, ready); break;
+            default: ready(); // (no other format reaches this kernel; every wave meets the barriers all the same)
             }
-        }
+        } else ready();
         L.red[wave * 64 + lane] = acc;
         __syncthreads();
         if (part == 0 && which == 0 && t < ntiles) {
@@ -483,7 +494,7 @@ __device__ __forceinline__ void qmvm_swiglu_body(const qwk_qmvm_args &a, qw_qmvm
 }
 #if QW_IN_PART(0)
 extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_qmvm_swiglu(qwk_qmvm_args a) {
-    __shared__ qw_qmvm_lds L;
+    __shared__ qw_swiglu_lds L;
     qmvm_swiglu_body(a, L, blockIdx.x, gridDim.x);
 }
 #endif
@@ -1404,7 +1415,7 @@ QW_PRE(1, 121, 2, qwk_pre_w1_s121_c2) QW_PRE(30, 121, 2, qwk_pre_w30_s121_c2) QW
 // router on the first workgroups, the multi-format product with SwiGLU (qwk_qmvm_swiglu's work) on those after them.
 #if QW_IN_PART(2)
 extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_pre_w1_kq(qwk_prekq_args a) {
-    __shared__ qw_qmvm_lds L;
+    __shared__ qw_swiglu_lds L;
     if (blockIdx.x < a.nrouter) pre_router_mfma(a.r, L.xf, L.red);
     else qmvm_swiglu_body(a.m, L, blockIdx.x - a.nrouter, gridDim.x - a.nrouter);
 }

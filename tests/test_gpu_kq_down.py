@@ -1,4 +1,4 @@
-"""Down rows of the K-quant types and IQ4_XS through the range kernel (H rows staged in LDS, a contiguous range of tiles a
+"""K-quant and IQ4_XS rows in a layer. Down rows through the range kernel (H rows staged in LDS, a contiguous range of tiles a
 workgroup) and, for one or two tokens, through the launch that combines too: rows of one and two blocks, no, equal and Q8_0 shared
 rows, few experts (several rounds of ranges meet one expert) and many, and the line to the any-shape kernel."""
 import numpy as np
@@ -33,5 +33,22 @@ def test_kq_down_rows(gpu, oracle, fd, fshd, D, I, E, K, nb, want):
     with gpu.switches(dn_any="1"):  # the any-shape kernel: the same products in the same order, so the same bits
         other = run_moe(gpu, q.Path(gpu, D, I, E, K, 16), dl, x, nb)[0]
     assert np.array_equal(out.view(np.uint16), other.view(np.uint16))
+    dl.free()
+    path.close()
+
+
+@pytest.mark.parametrize("fsh,fshu,D,I,nb", [(12, 12, 1024, 256, 3), (12, 13, 2048, 512, 16), (14, 30, 2048, 384, 1), (20, 1, 2048, 640, 7), (23, 12, 1536, 512, 2), (13, 14, 2560, 640, 16),
+                                             (12, 12, 1792, 256, 5), (30, 20, 512, 512, 4)])
+def test_kq_shared_gate_up(gpu, oracle, fsh, fshu, D, I, nb):
+    """The shared expert's gate/up of the multi-format family in the front launch: K cut over two to six waves, one and two blocks each
+    (and 1792, which has no such cut)."""
+    rng = np.random.default_rng(fsh * 1000 + fshu * 10 + D + I + nb)
+    m = synth.moe_layer(rng, D, I, 16, fgu=21, fd=8, fsh=fsh, fshd=8, fshu=fshu)
+    m["topk"] = 4
+    x = synth.activations(rng, nb, D)
+    path = q.Path(gpu, D, I, 16, 4, 16)
+    dl = DeviceLayer(gpu, m, device_only=True)
+    out, lg, _, _ = run_moe(gpu, path, dl, x, nb)
+    assert maxrel(out, oracle.moe_layer_f64(m, lg, x)) <= TOL
     dl.free()
     path.close()
