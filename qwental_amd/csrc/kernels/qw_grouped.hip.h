@@ -124,7 +124,7 @@ template <> struct qw_pfg<QW_F_PACKED_NL> {
         for (int b = 0; b < 10; b++) {
             h8 w[QW_PFG_TW];
 #pragma unroll
-            for (uint32_t t = 0; t < QW_PFG_TW; t++) w[t] = qw_iq4_bytes((const uint32_t *)lut, c[t].q[b]);
+            for (uint32_t t = 0; t < QW_PFG_TW; t++) w[t] = qw_iq4_pairs((const uint32_t *)lut, c[t].q[b]);
 #pragma unroll
             for (int g = 0; g < NG; g++) {
                 const h8 a = qw_chunk<20, 1>::join(x.at4(g, 8 * b + x.kg), x.at4(g, 8 * b + 4 + x.kg));

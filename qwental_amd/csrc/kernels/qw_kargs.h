@@ -223,7 +223,8 @@ typedef struct { /* read-pattern ceiling of a decode layer (the reference's kern
 /* Tile-major copy of IQ4_NL rows (format code QW_F_PACKED_NL; qwk_pack_args with split = QW_F_PACKED_NL, nblk = chunks
  * of ten blocks per row, so the row length is a multiple of 320): every (tile of 16 rows, chunk) becomes
  * QW_NL_CHUNK_BYTES = 16 x 180 contiguous bytes in the lane order of the matrix instruction (lane = row & 15 | k-group
- * << 4; a lane owns bytes 4 kg .. 4 kg + 3 of qs of every block of its row):
+ * << 4; a lane owns bytes 4 kg .. 4 kg + 3 of qs of every block of its row, its eight nibbles in the order in which they are
+ * multiplied: the four low ones, then the four high ones, two a byte, so that a byte's table entry is a register of the operand):
  *   [0, 1024)    blocks 0..3: 16 bytes per lane      [1024, 2048)  blocks 4..7: 16 bytes per lane
  *   [2048, 2560) blocks 8..9:  8 bytes per lane      [2560, 2880)  d of the ten blocks, 20 bytes per row
  * A wave reads a chunk with three fully coalesced loads plus 20 bytes of scales per lane. */

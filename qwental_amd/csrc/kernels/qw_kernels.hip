@@ -206,7 +206,10 @@ extern "C" __global__ __launch_bounds__(256) void qwk_pack_nl(qwk_pack_args a) {
         uint8_t *dst = a.dst + ch * QW_NL_CHUNK_BYTES;
         uint32_t q[10];
 #pragma unroll
-        for (int b = 0; b < 10; b++) q[b] = *(const u1a2 *)(src + 18 * b + 2 + 4 * kg);
+        for (int b = 0; b < 10; b++) { // low nibbles of the four bytes, then the high ones, two a byte
+            const uint32_t v = *(const u1a2 *)(src + 18 * b + 2 + 4 * kg), l = v & 0x0f0f0f0fu, h = (v >> 4) & 0x0f0f0f0fu, lp = l | l >> 4, hp = h | h >> 4;
+            q[b] = (lp & 255) | ((lp >> 8) & 0xff00u) | (hp & 255) << 16 | ((hp >> 16) & 255) << 24;
+        }
         *(u4 *)(dst + 16 * lane) = u4{q[0], q[1], q[2], q[3]};
         *(u4 *)(dst + 1024 + 16 * lane) = u4{q[4], q[5], q[6], q[7]};
         *(u2 *)(dst + 2048 + 8 * lane) = u2{q[8], q[9]};

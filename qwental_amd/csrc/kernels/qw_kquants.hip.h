@@ -172,6 +172,10 @@ __device__ __forceinline__ h8 qw_iq4_bytes(const uint32_t *tab, uint32_t q) {
     raw[3] = __builtin_amdgcn_perm(t3, t2, 0x07060302u);
     return __builtin_bit_cast(h8, raw);
 }
+// The same eight values from a dword of the tile-major copy, whose bytes hold neighbours in that order.
+__device__ __forceinline__ h8 qw_iq4_pairs(const uint32_t *tab, uint32_t q) {
+    return __builtin_bit_cast(h8, u4{tab[q & 255], tab[(q >> 8) & 255], tab[(q >> 16) & 255], tab[q >> 24]});
+}
 template <class AFK> __device__ __forceinline__ h8 qw_iq4_xfrag(const AFK &af, uint32_t k32, uint32_t kg) { // x[4 kg .. + 4], x[16 + 4 kg .. + 4] of a 32-block
     const h4 a = af.at4(k32 + 4 * kg), b = af.at4(k32 + 16 + 4 * kg);
     return h8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
@@ -407,7 +411,7 @@ template <> struct qw_chunk<QW_F_PACKED_NL, 10> {
     template <class AF> __device__ __forceinline__ void mac(const u2 *lut, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const {
 #pragma unroll
         for (int b = 0; b < 10; b++) {
-            const h8 w = qw_iq4_bytes((const uint32_t *)lut, q[b]);
+            const h8 w = qw_iq4_pairs((const uint32_t *)lut, q[b]);
             const uint32_t kb = k0 + 32 * b + 4 * kg;
             f4 sub = {0, 0, 0, 0};
             sub = qw_mfma(qw_chunk<20, 1>::join(af.hi4(kb), af.hi4(kb + 16)), w, sub);
@@ -426,7 +430,7 @@ template <> struct qw_chunk<QW_F_PACKED_NL, 10> {
                 xh = qw_chunk<20, 1>::join(*(const h4 *)(af.rowhi + kb), *(const h4 *)(af.rowhi + kb + 16));
                 xl = qw_chunk<20, 1>::join(*(const h4 *)(af.rowlo + kb), *(const h4 *)(af.rowlo + kb + 16));
             }
-            const h8 w = qw_iq4_bytes((const uint32_t *)lut, q[b]);
+            const h8 w = qw_iq4_pairs((const uint32_t *)lut, q[b]);
             f4 sub = {0, 0, 0, 0};
             sub = qw_mfma(xh, w, sub);
             sub = qw_mfma(xl, w, sub);
