@@ -1593,8 +1593,11 @@ static bool tr_dn_inner(qw_batch *b) {
         if (fs) fname_fmt(tail, sizeof tail, "_s%d_c%d", fs, fs == 8 ? 4 : 1);
         fname_fmt(fn, sizeof fn, "qwk_dnr_f%d_c1%s", fd, tail);
         const unsigned grid = persistent_grid(b->g, umax * (unsigned)(p->D / 16) + (unsigned)p->D / 16, QW_WAVES_DNR);
-        if (nbr > b->sw.dnc_nb) return add_launch(b, intern(fn), grid, 64 * QW_WAVES_DNR, &a, sizeof a);
-        char fu[48]; // a few tokens: wait for the combine, the two run as one launch
+        // One token: wait for the combine, the two run as one launch (Q6_K rows of 256: 12.7 us against 12.4 + 6.1; of 512: 18.6
+        // against 13.2 + 6.2 and the gap between two launches). From two on its waves, which read H from memory step by
+        // step, take longer than both (31.4 against 13.6 + 6.4, rows of 256 20.0 against 12.4 + 6.2).
+        if (nbr > 1 || !b->sw.dnc_nb) return add_launch(b, intern(fn), grid, 64 * QW_WAVES_DNR, &a, sizeof a);
+        char fu[48];
         fname_fmt(fu, sizeof fu, "qwk_dnc_f%d_c1%s", fd, tail);
         b->pend_dn.valid = true;
         b->pend_dn.a = a;

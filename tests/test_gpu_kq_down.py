@@ -1,5 +1,5 @@
 """K-quant and IQ4_XS rows in a layer. Down rows through the range kernel (H rows staged in LDS, a contiguous range of tiles a
-workgroup) and, for one or two tokens, through the launch that combines too: rows of one and two blocks, no, equal and Q8_0 shared
+workgroup) and, for one token, through the launch that combines too: rows of one and two blocks, no, equal and Q8_0 shared
 rows, few experts (several rounds of ranges meet one expert) and many, and the line to the any-shape kernel."""
 import numpy as np
 import pytest
@@ -14,8 +14,8 @@ TOL = 2e-3  # binary16 results of a layer (half an ulp is 4.9e-4 of a value) aga
 
 @pytest.mark.parametrize("fd,fshd,D,I,E,K,nb,want", [
     (14, 14, 2048, 512, 64, 10, 4, "qwk_dnr_f14_c1_s14_c1"), (14, 8, 256, 256, 8, 2, 16, "qwk_dnr_f14_c1_s8_c4"), (14, 14, 1280, 512, 16, 4, 1, "qwk_dnc_f14_c1_s14_c1"),
-    (12, 12, 768, 256, 48, 6, 9, "qwk_dnr_f12_c1_s12_c1"), (12, 8, 2560, 512, 32, 10, 2, "qwk_dnc_f12_c1_s8_c4"), (13, 13, 1024, 512, 512, 10, 16, "qwk_dnr_f13_c1_s13_c1"),
-    (13, 13, 512, 256, 16, 16, 2, "qwk_dnc_f13_c1_s13_c1"), (23, 23, 2048, 256, 128, 8, 3, "qwk_dnr_f23_c1_s23_c1"), (23, 8, 1536, 512, 16, 1, 1, "qwk_dnc_f23_c1_s8_c4"),
+    (12, 12, 768, 256, 48, 6, 9, "qwk_dnr_f12_c1_s12_c1"), (12, 8, 2560, 512, 32, 10, 2, "qwk_dnr_f12_c1_s8_c4"), (13, 13, 1024, 512, 512, 10, 16, "qwk_dnr_f13_c1_s13_c1"),
+    (13, 13, 512, 256, 16, 16, 1, "qwk_dnc_f13_c1_s13_c1"), (12, 12, 1024, 256, 16, 4, 1, "qwk_dnc_f12_c1_s12_c1"), (23, 23, 2048, 256, 128, 8, 3, "qwk_dnr_f23_c1_s23_c1"), (23, 8, 1536, 512, 16, 1, 1, "qwk_dnc_f23_c1_s8_c4"),
     (14, 12, 1024, 512, 16, 4, 4, "qwk_dn_rt"), (12, 12, 1024, 768, 16, 4, 4, "qwk_dn_rt")])
 def test_kq_down_rows(gpu, oracle, fd, fshd, D, I, E, K, nb, want):
     rng = np.random.default_rng(fd * 1000 + fshd * 10 + D + I + nb)
