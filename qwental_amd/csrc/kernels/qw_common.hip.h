@@ -240,29 +240,29 @@ __device__ __forceinline__ bool qw_grid_barrier(uint32_t *sync, uint32_t gen0, u
 }
 
 // ---------------------------------------------------------------- activation fragment providers (operand A)
-// Fragment order in LDS: chunk c (8 consecutive k-values) of token m lives at xf[c * 16 + m], 16 bytes, so that the
-// 16 lanes of a k-group read 256 contiguous bytes. Tokens >= nb are stored as zeros.
 // Four values of token m, koff = a multiple of 8 plus 4 times the lane's k-group: byte offset of the half of a 16-byte unit.
 // (From the unit, ((koff >> 3) * 16 + m) * 16 + (koff & 4) * 2, the compiler made five instructions a read wherever the K range
 // of a chunk is no power of two; this is one shift of the chunk's base and constants that the reads carry.)
 __device__ __forceinline__ uint32_t qw_half_at(uint32_t koff, uint32_t m) { return (koff << 5) + (16 * m - 120 * ((threadIdx.x >> 4) & 1)); }
+// Eight bytes of LDS by an instruction of their own: the compiler pairs such reads (ds_read2st64_b64), and the two halves of
+// a pair, a multiple of 512 bytes apart, meet in the same banks. (IQ4_XS gate / up rows at 16 tokens 62 -> 53 us, the blocked
+// grouped product of IQ4_NL rows 213 -> 198 at 1000 rows, 70 -> 66 at 60. IQ4_NL down rows of the reference model at 8 and 16 tokens: as they were, unpaired with an address computed for each, 27.8 and 43.1 us;
+// with qw_half_at and paired 33.5 and 55.1; with qw_half_at and single 25.4 and 39.1. Q6_K rows 46.1 -> 45.4 at 16.)
+__device__ __forceinline__ u2 qw_half_read(const u4 *base, uint32_t at) {
+    return *(const volatile __attribute__((address_space(3))) u2 *)((const __attribute__((address_space(3))) char *)base + at);
+}
+// Fragment order in LDS: chunk c (8 consecutive k-values) of token m lives at xf[c * 16 + m], 16 bytes, so that the
+// 16 lanes of a k-group read 256 contiguous bytes. Tokens >= nb are stored as zeros.
 struct qw_afrag_lds {
     const u4 *xf;
     uint32_t m;
     static constexpr bool has_lo = false;
     __device__ __forceinline__ h8 hi(uint32_t koff) const { return __builtin_bit_cast(h8, xf[(koff >> 3) * 16 + m]); }
     __device__ __forceinline__ h8 lo(uint32_t) const { return h8{}; }
-    __device__ __forceinline__ h4 hi4(uint32_t koff) const { return __builtin_bit_cast(h4, *(const u2 *)((const char *)xf + qw_half_at(koff, m))); } // koff: qw_half_at
+    __device__ __forceinline__ h4 hi4(uint32_t koff) const { return __builtin_bit_cast(h4, qw_half_read(xf, qw_half_at(koff, m))); } // koff: qw_half_at
     __device__ __forceinline__ h4 lo4(uint32_t) const { return h4{}; }
 };
 
-// Eight bytes of LDS by an instruction of their own: the compiler pairs such reads (ds_read2st64_b64), and the two halves of
-// a pair, a multiple of 512 bytes apart, meet in the same banks. (IQ4_NL down
-// rows of the reference model at 8 and 16 tokens: as they were, unpaired with an address computed for each, 27.8 and 43.1 us;
-// with qw_half_at and paired 33.5 and 55.1; with qw_half_at and single 25.4 and 39.1. Q6_K rows 46.1 -> 45.4 at 16.)
-__device__ __forceinline__ u2 qw_half_read(const u4 *base, uint32_t at) {
-    return *(const volatile __attribute__((address_space(3))) u2 *)((const __attribute__((address_space(3))) char *)base + at);
-}
 // Two planes (hi + lo) staged the same way.
 struct qw_afrag_lds2 {
     const u4 *hi_, *lo_;

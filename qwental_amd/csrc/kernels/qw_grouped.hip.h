@@ -20,7 +20,7 @@
 // Measured (Zipf(1.1) routing over 512 experts, top-10, D = 2048, I = 512; gate / up and down product, us), against the
 // kernel before, in which a wave took 16 weight rows and up to 64 packed rows and read the activations from memory:
 // 2048 rows 1102 + 522 -> 255 + 140, 1000 rows 573 + 273 -> 195 + 101; reference model's layer, 1082 rows 840 + 627 ->
-// 268 + 212. What bounds it: at 2048 rows the loads alone (640 MB of slabs, 335 MB of rows that every block of tiles asks
+// 268 + 212 (1000 rows, down product: 213 -> 198 with operand reads that are not paired). What bounds it: at 2048 rows the loads alone (640 MB of slabs, 335 MB of rows that every block of tiles asks
 // for again) take 168 us, the arithmetic alone (vector ALU busy half of the time, LDS 53 %, matrix cores 21 %, at 1.75 GHz)
 // 209. Sixteen waves of one tile each, a barrier every step instead of every four, activations a step ahead or not, all
 // table values of a block at once: within 3 %.
@@ -42,7 +42,7 @@ template <uint32_t KS, int NG> struct qw_pfg_rows {
     static constexpr uint32_t GU = qw_pfg_subs(16 * NG) * KS / 32 * 64; // units of a group of rows in the buffer
     __device__ __forceinline__ uint32_t unit(uint32_t g, uint32_t c) const { return g * GU + (c >> 2) * 64 + 4 * n + ((c & 3) ^ ((n >> 2) & 3)); } // c: which 8 values of the step
     __device__ __forceinline__ h8 at8(uint32_t g, uint32_t c) const { return __builtin_bit_cast(h8, buf[unit(g, c)]); }
-    __device__ __forceinline__ h4 at4(uint32_t g, uint32_t c4) const { return __builtin_bit_cast(h4, ((const u2 *)buf)[unit(g, c4 >> 1) * 2 + (c4 & 1)]); } // c4: which 4 values
+    __device__ __forceinline__ h4 at4(uint32_t g, uint32_t c4) const { return __builtin_bit_cast(h4, qw_half_read(buf, unit(g, c4 >> 1) * 16 + (c4 & 1) * 8)); } // c4: which 4 values
 };
 
 // s_waitcnt for "at most n vector memory operations outstanding", the other counters not waited for (n < 64)
