@@ -3,8 +3,10 @@
  *
  * Host shadow rules (qw_buf.ptr is host memory, the kernels read HBM):
  *   - host -> device, when a batch is submitted, for every buffer a dispatch of the batch binds:
- *       a buffer of at most QW_HIP_SMALL_BYTES is copied every time (once its whole has been: the bytes that the batch's
- *       dispatches can touch; a copy out of HBM, or its address asked for, brings the rest into step first);
+ *       a buffer of at most QW_HIP_SMALL_BYTES is copied every time. Under qw_batch_end, once its whole has been copied and
+ *       while nobody has its device address, only the bytes that the batch's dispatches can touch: the rest stays the
+ *       host's until a copy out of HBM (qw_hip_buf_read, qw_hip_buf_download) or qw_hip_buf_devptr asks, which first
+ *       sends it up as the host side holds it then;
  *       a larger one is copied the first time it is bound and again only after qw_hip_buf_mark_dirty();
  *       qw_buf_wrap() buffers are copied once; device-only buffers never;
  *       not the bytes that the batch's kernels write whole before anything reads them (a product's result, say): what the

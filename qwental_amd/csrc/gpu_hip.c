@@ -66,6 +66,7 @@ typedef struct qw_hbuf {
     int pending_out; // submitted batches that bind it in an output role and have not been waited for: HBM is newer than the shadow
     uint64_t out_seq; // the last batch that counted itself in pending_out
     size_t plo, phi;  // the bytes that those batches' dispatches may write (the least range that holds them all)
+    bool addr;        // its device address was given out: uploads carry the whole buffer
     bool part;        // the last upload carried [slo, shi) only, the bytes its batch could touch: HBM may lack what the host wrote elsewhere
     size_t slo, shi;
     struct qw_gpu *g;
@@ -747,15 +748,21 @@ void qw_hip_set_repack(qw_gpu *g, bool on) { g->repack = on; }
 unsigned qw_hip_graph_launches(const qw_gpu *g) { return g->ngraph_launches; }
 void qw_hip_set_graphs(qw_gpu *g, bool on) { g->use_graphs = on; }
 size_t qw_hip_packed_bytes(const qw_gpu *g) { return g->pack_bytes; }
-// Before HBM is looked at from outside a batch: what the host wrote beyond the range of the last upload.
+// Before HBM is looked at from outside a batch: what the host wrote beyond the range of the last upload. (While outputs of h
+// are under way this has nothing to do: the batch that made them was submitted without a wait and took the whole buffer up.)
 static bool rest_up(qw_hbuf *h) {
-    if (!h || !h->part || h->pending_out || h->released || h->dirty || !h->host) return true;
+    if (!h || !h->part) return true;
     h->part = false;
     return (!h->slo || hipMemcpy(h->dptr, h->host, h->slo, hipMemcpyHostToDevice) == hipSuccess) &&
            (h->shi >= h->size || hipMemcpy((char *)h->dptr + h->shi, (char *)h->host + h->shi, h->size - h->shi, hipMemcpyHostToDevice) == hipSuccess);
 }
 static bool range_ok(const qw_hbuf *h, size_t off, size_t len) { return !h->released && off <= h->size && len <= h->size - off; } // a released buffer has no bytes to copy
-void *qw_hip_buf_devptr(const qw_buf *b) { return b && b->handle && !((qw_hbuf *)b->handle)->released && rest_up(b->handle) ? ((qw_hbuf *)b->handle)->dptr : NULL; }
+void *qw_hip_buf_devptr(const qw_buf *b) {
+    qw_hbuf *h = b ? b->handle : NULL;
+    if (!h || h->released || !rest_up(h)) return NULL;
+    h->addr = true; // the address may be kept: its holder sees every later submit's bytes
+    return h->dptr;
+}
 // Free the device bytes of a weight buffer and keep its tile-major copies (include/qw_hip_ext.h).
 // Bytes of h that some tile-major copy was made from: the union of the copies' source ranges inside the buffer.
 static size_t packed_source_bytes(const qw_hbuf *h) {
@@ -2276,13 +2283,17 @@ static bool submit_segment(qw_batch *b, bool last) {
         size_t lo, hi, tlo = 0, thi = h->size;
         whole_range(b, b->done_use, h, &lo, &hi);
         if (h->size > QW_HIP_BIG_OUT_BYTES) lo = hi = 0; // (its results are not carried back: the shadow must not be taken for them later)
-        if (!h->dirty) {
-            touched_range(b, i, h, false, &tlo, &thi);
+        if (h->pending_out > 0 && !h->dirty) {
             // A kernel of a batch that was submitted (or of an earlier segment of this one) and not yet waited for wrote
-            // this buffer: HBM holds the newer contents there, and the shadow must not overwrite them.
-            if (h->pending_out > 0) lo = h->plo, hi = h->phi;
+            // this buffer: HBM holds the newer contents there, and the shadow must not overwrite them. (The rest went up with that batch.)
+            touched_range(b, i, h, false, &tlo, &thi);
+            lo = h->plo, hi = h->phi;
+        } else {
+            // Only the bytes that the segment can touch where the caller waits for it at once, so that nobody looks at HBM
+            // before rest_up can; after a flush or qw_batch_submit the whole buffer is in step, whoever looks and when.
+            if (last && !h->dirty && !h->addr) touched_range(b, i, h, false, &tlo, &thi);
+            h->part = tlo > 0 || thi < h->size, h->slo = tlo, h->shi = thi;
         }
-        h->part = tlo > 0 || thi < h->size, h->slo = tlo, h->shi = thi;
         if (lo < tlo) lo = tlo;
         if (hi > thi) hi = thi;
         if (hi <= lo) lo = hi = thi;

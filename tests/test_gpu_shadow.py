@@ -99,3 +99,77 @@ def test_many_buffers_and_many_batches_in_flight(gpu, oracle, nbuf):
     for bb in [wb] + xb + yb:
         bb.free()
     path.close()
+
+
+def tail_setup(gpu, oracle, rng):
+    """A product whose result is the head of a 64 KB buffer that has been up and down once; (record a batch, buffer, tail, check of the head)."""
+    N, K, off = 64, 256, 32768
+    W, x = synth.matrix(rng, 8, N, K), synth.activations(rng, 1, K)
+    path = q.Path(gpu, 2048, 512, 512, 10, 16)
+    wb, xb, y = gpu.buf_from(W, device_only=True), gpu.buf_from(x), gpu.buf(65536)
+    ref = product(oracle, 8, W, N, K, x)[0]
+
+    def record():
+        b = gpu.batch()
+        path.qmv_gg(b, q.Tensor(wb, 8), N, K, xb, y, 1)
+        return b
+
+    def head_ok():
+        return np.abs(y.view(np.float32)[:N] - ref).max() <= 1e-5 * np.abs(ref).max()
+
+    def free():
+        for bb in (wb, xb, y):
+            bb.free()
+        path.close()
+
+    assert record().end() > 0
+    return record, y, off, head_ok, free
+
+
+@pytest.mark.parametrize("how", ["submit", "flush", "end", "dirty"])
+def test_hbm_looked_at_holds_what_the_host_wrote_elsewhere(gpu, oracle, how):
+    """The host writes the tail of a buffer whose head a batch computes. Read from HBM the tail holds those bytes, and a
+    download leaves them alone: between submit and wait, while a flushed part runs, after qw_batch_end, and where the buffer
+    was marked dirty in between."""
+    rng = np.random.default_rng(9)
+    record, y, off, head_ok, free = tail_setup(gpu, oracle, rng)
+    for _ in range(3):
+        mine = rng.integers(0, 256, y.size - off, dtype=np.uint8)
+        y.view()[off:] = mine
+        b = record()
+        if how == "submit":
+            gpu.L.qw_batch_submit(b.b)
+            while not gpu.L.qw_batch_poll(b.b):
+                pass
+        elif how == "flush":
+            b.flush()
+        else:
+            assert b.end() > 0
+            if how == "dirty":
+                gpu.L.qw_hip_buf_mark_dirty(y.ref())
+        if how == "flush":  # (the copy up is behind the flush on the stream: wait for it without waiting for the batch)
+            other = record()
+            assert other.end() > 0
+        assert np.array_equal(y.read(len(mine), off), mine)
+        assert gpu.L.qw_hip_buf_download(y.ref(), off, len(mine)) and np.array_equal(y.view()[off:], mine)
+        if how == "submit":
+            assert gpu.L.qw_batch_wait(b.b) > 0
+        elif how == "flush":
+            assert b.end() > 0
+        assert head_ok() and np.array_equal(y.view()[off:], mine)
+    free()
+
+
+def test_a_kept_device_address_sees_every_later_submit(gpu, oracle):
+    """Whoever asked for the address once reads the whole buffer as it was at the last submit, not the bytes of its batch only."""
+    rng = np.random.default_rng(10)
+    record, y, off, head_ok, free = tail_setup(gpu, oracle, rng)
+    addr = gpu.L.qw_hip_buf_devptr(y.ref())
+    got = np.empty(y.size - off, np.uint8)
+    for _ in range(3):
+        mine = rng.integers(0, 256, len(got), dtype=np.uint8)
+        y.view()[off:] = mine
+        assert record().end() > 0
+        assert gpu.L.hipMemcpy(C.c_void_p(got.ctypes.data), C.c_void_p(addr + off), C.c_size_t(len(got)), 2) == 0  # 2: device to host
+        assert np.array_equal(got, mine) and head_ok()
+    free()
