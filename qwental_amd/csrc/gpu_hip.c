@@ -1446,7 +1446,8 @@ static bool tr_gu(qw_batch *b) {
     if (!bind_ptr(b, 5, QW_SEL_BYTES((size_t)p->gnb, (size_t)p->topk), false, "selection", (void **)&a.sel)) return false;
     b->pend_sd.valid = false;
     b->pend_sd.rowbytes = (uint32_t)fmt_rb(p->fsd, p->I);
-    if (!bind_ptr(b, 2, (size_t)p->D * b->pend_sd.rowbytes, false, "shared down weights", (void **)&b->pend_sd.Wsd) || !bind_whole(b, 3, (size_t)nbr * p->D * 4, "Psh", (void **)&b->pend_sd.Psh)) return false;
+    if (!bind_ptr(b, 2, (size_t)p->D * b->pend_sd.rowbytes, false, "shared down weights", (void **)&b->pend_sd.Wsd) ||
+        !bind_ptr(b, 3, (size_t)nbr * p->D * 4, true, "Psh", (void **)&b->pend_sd.Psh)) return false; // (not bind_whole: only a moe_dn_gg of this batch writes it)
     b->pend_sd.valid = true;
     b->pend_sd.hd = b->buf[2].h;
     b->pend_sd.fmt = p->fsd;

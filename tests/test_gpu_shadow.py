@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import qwental_amd as q
+from helpers import DeviceLayer, run_moe
 from qwental_amd import synth
 
 pytestmark = pytest.mark.gpu
@@ -173,3 +174,33 @@ def test_a_kept_device_address_sees_every_later_submit(gpu, oracle):
         assert gpu.L.hipMemcpy(C.c_void_p(got.ctypes.data), C.c_void_p(addr + off), C.c_size_t(len(got)), 2) == 0  # 2: device to host
         assert np.array_equal(got, mine) and head_ok()
     free()
+
+
+def test_a_result_left_to_a_later_dispatch_keeps_the_hosts_bytes(gpu):
+    """moe_gu_gg binds the shared expert's down rows as a result, but the moe_dn_gg of the same batch writes them. A batch
+    that ends before it leaves them as the host had them."""
+    D, I, E, K, nb = 512, 256, 8, 2, 2
+    rng = np.random.default_rng(11)
+    m = synth.moe_layer(rng, D, I, E, 8, 8, 8)
+    x = synth.activations(rng, nb, D)
+    path = q.Path(gpu, D, I, E, K, 16)
+    dl = DeviceLayer(gpu, m)
+    sel = run_moe(gpu, path, dl, x, nb)[2]  # registers the kernels; its selection record
+    k = gpu.kernel("moe_gu_gg_8_8_g1_n2_e%dk%dd%di%d" % (E, K, D, I))
+    assert k
+    xb, sb, H, psh = gpu.buf_from(x), gpu.buf_from(sel), gpu.buf(2 * (K + 1) * I * 4), gpu.buf(nb * D * 4)
+    for _ in range(3):
+        mine = rng.standard_normal(nb * D).astype(np.float32)
+        psh.view(np.float32)[:] = mine
+        b = gpu.batch()
+        b.kernel(k)
+        for i, bb in ((0, dl.bufs["Wg"]), (1, dl.bufs["Wu"]), (2, dl.bufs["Wsd"]), (3, psh), (4, xb), (5, sb), (6, H)):
+            b.buf(i, bb)
+        b.bytes(12, np.array([nb], np.uint32))
+        b.dispatch(1)
+        assert b.end() > 0, gpu.last_error()
+        assert np.array_equal(psh.view(np.float32), mine) and np.array_equal(psh.read(dtype=np.float32), mine)
+    for bb in (xb, sb, H, psh):
+        bb.free()
+    dl.free()
+    path.close()
