@@ -45,11 +45,15 @@ template <uint32_t KS, int NG> struct qw_pfg_rows {
     __device__ __forceinline__ h4 at4(uint32_t g, uint32_t c4) const { return __builtin_bit_cast(h4, qw_half_read(buf, unit(g, c4 >> 1) * 16 + (c4 & 1) * 8)); } // c4: which 4 values
 };
 
-// s_waitcnt for "at most n vector memory operations outstanding", the other counters not waited for (n < 64)
-#define QW_VMCNT(n) ((((n) & 15) | ((n) >> 4) << 14) | 0x0f70)
 // A barrier of the workgroup behind its LDS operations only (__syncthreads also waits for every load and store in flight)
 __device__ __forceinline__ void qw_wg_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+}
+// The same once all but the wave's last N vector memory operations have completed. One piece, so that no load is moved
+// between the wait and the barrier.
+template <int N> __device__ __forceinline__ void qw_wg_barrier_but() {
+    static_assert(N > 0 && N < 64, "vmcnt");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
 }
 // Written as fused multiply-adds: left to the compiler, the first group of rows was multiplied and added in two roundings
 // (its addition merged over the four row counts) and the others in one, and a row's bits depended on where it lay.
@@ -57,9 +61,12 @@ __device__ __forceinline__ void pfg_fma(f4 &acc, float d, const f4 s) {
 #pragma unroll
     for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(d, s[i], acc[i]);
 }
+// LOADS: the fewest loads that bring a lane its part of one slab. The loop counts on no more than these behind the rows'
+// loads (more only make its wait stricter); qwental_amd/build.py counts them in the code object, on every path.
 template <int F> struct qw_pfg;
 template <> struct qw_pfg<QW_F_PACKED> {
-    static constexpr uint32_t KS = 256, BYTES = QW_SLAB_BYTES, LOADS = 3; // LOADS: of one slab, as the compiler issues them
+    static constexpr uint32_t KS = 256, BYTES = QW_SLAB_BYTES, LOADS = 3;
+    static_assert(BYTES == 64 * (16 + 8 + 4), "a lane's bytes lie in three places");
     typedef qw_chunk<QW_F_PACKED, 1> C;
     template <int J> static __device__ __forceinline__ void look(const C (&c)[QW_PFG_TW], const qw_iq3_keys (&k)[QW_PFG_TW], const u2 *lut, u2 (&w)[QW_PFG_TW][2]) {
 #pragma unroll
@@ -118,6 +125,7 @@ template <> struct qw_pfg<QW_F_PACKED> {
 };
 template <> struct qw_pfg<QW_F_PACKED_NL> {
     static constexpr uint32_t KS = 320, BYTES = QW_NL_CHUNK_BYTES, LOADS = 5;
+    static_assert(BYTES == 64 * (16 + 16 + 8) + 16 * 20, "a lane's bytes lie in four places, of which one is longer than the longest load");
     typedef qw_chunk<QW_F_PACKED_NL, 10> C;
     template <int NG> static __device__ __forceinline__ void mac(const C (&c)[QW_PFG_TW], const u2 *lut, const qw_pfg_rows<KS, NG> &x, f4 (&acc)[QW_PFG_TW][4]) {
 #pragma unroll
@@ -236,7 +244,7 @@ struct qw_pfg_cursor {
 // registers and stores to complete in any order, and would empty the queue at every turn). What it does not see makes
 // the hardware's count larger, so its own waits stay safe; the wait for the rows is the loop's.
 __device__ __forceinline__ void pfg_load_lds(const void *src_lane, uint32_t lds_wave) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src_lane), "s"(lds_wave) : "memory"); // (m0 too: nothing else of this kernel reads it after the first of these)
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src_lane), "s"(lds_wave) : "memory", "m0");
 }
 __device__ __forceinline__ void pfg_store16(void *p, u4 v) { asm volatile("global_store_dwordx4 %0, %1, off" : : "v"(p), "v"(v) : "memory"); }
 
@@ -289,8 +297,8 @@ template <int F> __device__ __forceinline__ void pfg_body(const qwk_pf_args &a, 
     auto phase = [&](auto B) -> bool {
         constexpr int b = decltype(B)::value;
         if (todo == 0) { // on to the rows that were asked for while the ones before were multiplied
-            __builtin_amdgcn_s_waitcnt(QW_VMCNT(QW_PFG_TW * P::LOADS)); // (the weights of the step after this one stay in flight)
-            qw_wg_barrier(); // everybody's rows; and everybody is done with the other buffer
+            // everybody's rows (the weights of the step after this one stay in flight: they were asked for behind the rows); and everybody is done with the other buffer
+            qw_wg_barrier_but<(int)(QW_PFG_TW * P::LOADS)>();
             const uint32_t subs = qw_pfg_subs(cur.rows);
             xb ^= 1, xk = cur.k, todo = nsteps - cur.k < subs ? nsteps - cur.k : subs;
             more = lx.next(S, subs, nsteps, nblocks, ntasks);
