@@ -1857,10 +1857,19 @@ static bool launch_pf(qw_batch *b, qwk_pf_args *a, int F, int E, qw_hbuf *hw, qw
     if (!wb) a->H = NULL, a->Y1 = NULL; // SwiGLU rides only in a launch that holds both matrices
     char fn[32];
     // The blocked kernel (qwk_pfg_*) wants its result rows 16-byte aligned. It takes IQ4_NL rows at any size (24 rows of the
-    // reference model's layer: down product 95 -> 51 us) and IQ3_S rows from entries of more than 16 rows on; with entries
-    // of 16 it passes the kernel that keeps an entry's rows in LDS once experts have several entries each (512 experts,
-    // top-10: 500 rows 154 + 83 against 151 + 83 us, 2048 rows 303 + 161 against 241 + 135, 250 rows 107 + 58 against 114 + 64).
+    // reference model's layer: down product 95 -> 51 us) and IQ3_S rows from entries of more than 16 rows on. With entries
+    // of 16 its gain over the kernel that keeps an entry's rows in LDS (qwk_pfr_*) is a weight decoded once for several of an
+    // expert's entries, and grows with the pairs that an expert has; its price is tasks of 64 rows x 256 columns, of which
+    // there have to be enough for the device, and shrinks with the pairs times the layer's inner width I. The two kernels
+    // are even where (M / E) * (M * I) is 2^26, within a fifth of M, for 16 to 512 experts with D x I from 1024 x 256 to 2560 x 640
+    // and to 1024 x 4096, even and Zipf(1.1) routing (down rows longer than D: a little later). Gate / up + down, us, qwk_pfr_* / qwk_pfg_*:
+    // 2048 x 512, 512 experts, 5120 pairs 146 + 79 / 163 + 87, 7680: 190 + 101 / 181 + 101, 15360: 295 + 159 / 226 + 121; 128
+    // experts, 2560 pairs 59 + 33 / 74 + 42, 5120: 88 + 49 / 84 + 47; 16 experts, 3200 pairs 54 + 31 / 38 + 25; 1024 x 256, 128
+    // experts, 5120 pairs 32 + 21 / 38 + 22, 10240: 52 + 32 / 40 + 28. Rows of more than 2560 values have no qwk_pfr_*, and
+    // the kernel left for them loses at nearly every size (4096 values, 64 experts, 320 pairs 54 / 40 us, 5120: 385 / 105).
     const bool blocked = ((uintptr_t)a->Y | (uintptr_t)a->Y1 | (uintptr_t)a->H) % 16 == 0;
+    const uint32_t inner = wb ? a->N : a->K;
+    const bool several = a->tm > 16 || a->K > 2560 || (uint64_t)a->M * a->M * inner >= (uint64_t)E << 26;
     if (F == 20 && a->K % 320 == 0 && blocked) {
         const uint32_t nch = a->K / 320;
         const uint8_t *pk = get_pack(b, hw, a->W, NULL, NULL, (uint64_t)E * (a->N / 16), nch, a->rowbytes, QW_F_PACKED_NL);
@@ -1875,7 +1884,7 @@ static bool launch_pf(qw_batch *b, qwk_pf_args *a, int F, int E, qw_hbuf *hw, qw
         const uint8_t *pk = get_pack(b, hw, a->W, wb ? hwb : NULL, wb, ntiles, nblk, a->rowbytes, split);
         if (pk) {
             a->W = pk, a->rowbytes = nblk * QW_SLAB_BYTES, a->split = split, a->ntn = a->N / split;
-            if (blocked && (a->tm > 16 || a->M > 5000)) return add_launch(b, "qwk_pfg_f121", (unsigned)b->g->ncu, 512, a, sizeof *a);
+            if (blocked && several) return add_launch(b, "qwk_pfg_f121", (unsigned)b->g->ncu, 512, a, sizeof *a);
             if (a->tm <= 16 && a->K <= 2560) { // entries of one group of rows: the rows are staged in LDS per workgroup range
                 fname_fmt(fn, sizeof fn, "qwk_pfr_f121_c%d", a->K % 512 == 0 ? 2 : 1);
                 return add_launch(b, intern(fn), umin((unsigned)b->g->ncu, a->max_tiles * a->ntn), 64 * QW_WAVES_GU, a, sizeof *a);

@@ -38,6 +38,39 @@ def test_entries_of_sixteen_rows_taken_together(gpu, oracle):
     run_case(gpu, oracle, T, ids, E, K, 256, 256, 21, 16, 33, device_only=True)
 
 
+@pytest.mark.parametrize("D,I,E,K,T,blocked", [(256, 256, 128, 10, 512, (False, False)), (256, 256, 128, 10, 600, (True, True)), (256, 256, 16, 4, 500, (False, False)),
+                                               (256, 256, 16, 4, 520, (True, True)), (256, 2816, 4, 1, 20, (False, True))])
+def test_which_kernel_takes_entries_of_sixteen_rows(gpu, oracle, D, I, E, K, T, blocked):
+    """The line between the two kernels, (pairs / experts) x (pairs x I) = 2^26, from both sides, with more and with less than
+    5000 pairs; rows of more than 2560 values have the blocked kernel alone. The two add up K in different orders, after which
+    gate, up, H and the down rows are rounded to binary16: four roundings of 2^-11, TOL."""
+    rng = np.random.default_rng(T)
+    assert I > 2560 or ((T * K) ** 2 * I >= E << 26) == blocked[0]
+    ids = synth.zipf_ids(rng, T, E, K)
+    m = synth.moe_layer(rng, D, I, E)
+    x = synth.activations(rng, T, D)
+    out = []
+    dl = DeviceLayer(gpu, m, device_only=True)
+    xb, ib = gpu.buf_from(x), gpu.buf_from(ids.ravel())
+    wb, ob = gpu.buf_from(np.full(T * K, 1.0 / K, np.float32)), gpu.buf(T * D * 2)
+    for tm in (16, 32):  # (from entries of 32 rows on it is always the blocked kernel)
+        path = q.Path(gpu, D, I, E, K, 16, device_scratch=True)
+        path.pf_reserve(T, tm)
+        gpu.profile(True)
+        b = gpu.batch()
+        path.pf_moe(b, dl.layer, T, xb, ib, wb, ob)
+        assert b.end() > 0
+        gpu.profile(False)
+        ran = [n.startswith("qwk_pfg") for n, _ in gpu.profile_entries() if n.startswith("qwk_pf")]
+        assert ran == list(blocked if tm == 16 else (True, True))
+        out.append(ob.view(np.float16).astype(np.float64))
+        path.close()
+    assert maxrel(out[0], out[1]) <= TOL
+    for bb in (xb, ib, wb, ob):
+        bb.free()
+    dl.free()
+
+
 @pytest.mark.parametrize("T,K", [(1024, 1), (1025, 1), (128, 8), (257, 5), (3000, 1), (513, 16)])
 def test_prepared_rows_by_pair_and_by_slice(gpu, oracle, T, K):
     """The preparation on both sides of its limit, with hot experts and experts without a row (values are the other tests')."""
