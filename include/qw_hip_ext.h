@@ -50,14 +50,18 @@ void *qw_hip_buf_devptr(const qw_buf *b);
 
 /* IQ3_S weight matrices of the MoE kernels are copied once, at their first use, into a tile-major layout that a wave
  * reads with fully coalesced loads (the copy costs 1792 / 1760 of the matrix's bytes of HBM; the GGUF bytes stay where
- * they are); IQ4_NL down matrices with rows of 640 values likewise (a copy of exactly their size). The copy is dropped when the source buffer is freed, marked dirty, uploaded, written, or bound as a
- * kernel's output. Buffers of at most QW_HIP_SMALL_BYTES with a host shadow are never copied. QW_HIP_REPACK=0 in the
+ * they are); so are, at exactly their size, IQ4_NL down matrices with rows of 320 or 640 values at their first moe_dn_gg, and
+ * IQ4_NL matrices whose rows are a multiple of 320 values, gate and up rows among them, at their first moe_pf_gg. The latter
+ * are resident twice where decode steps run beside the packing path: those read IQ4_NL gate and up rows in GGUF order (512
+ * experts of 640 x 2560: 944 MB more a layer for gate and up). A copy is dropped when the source buffer is freed, marked
+ * dirty, uploaded, written, or bound as a kernel's output. Without memory for one the dispatch reads the GGUF rows. Buffers of at most QW_HIP_SMALL_BYTES with a host shadow are never copied. QW_HIP_REPACK=0 in the
  * environment, or qw_hip_set_repack(g, false), turns the copies off (kernels then read the GGUF rows directly). */
 void qw_hip_set_repack(qw_gpu *g, bool on);
 size_t qw_hip_packed_bytes(const qw_gpu *g);
 /* Keep only the tile-major copies of a weight buffer: frees the buffer's device bytes (the GGUF-order rows) once the
  * copies that the kernels read have been made, i.e. after every matrix in it has been through a dispatch that makes one
- * (moe_gu_gg, moe_dn_gg, moe_pf_gg and qmv_gg over IQ3_S rows; moe_dn_gg over IQ4_NL rows of 320 or 640). Residency of
+ * (moe_gu_gg, moe_dn_gg, moe_pf_gg and qmv_gg over IQ3_S rows; moe_dn_gg over IQ4_NL rows of 320 or 640 - a copy of IQ4_NL
+ * rows that only moe_pf_gg has asked for does not count, decode steps may need the GGUF order). Residency of
  * such a matrix drops from 2.018 to 1.018 times its bytes. Afterwards the buffer may only be bound as those weights:
  * a dispatch that no existing copy serves (another shape or split, a matrix that was never dispatched, dq_test, any output
  * role) fails the batch with a message, the explicit copy calls return false, qw_hip_buf_devptr gives NULL, and the

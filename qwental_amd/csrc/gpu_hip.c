@@ -82,6 +82,7 @@ typedef struct {
     uint32_t nblk, split;
     void *dst;
     size_t bytes;
+    bool pf; // IQ4_NL rows that only moe_pf_gg has asked for: a decode dispatch may read them in GGUF order (gate / up rows)
 } qw_pack;
 
 typedef struct {
@@ -774,6 +775,7 @@ static size_t packed_source_bytes(const qw_hbuf *h) {
         const qw_pack *p = &g->packs[i];
         const bool nl = p->split == QW_F_PACKED_NL, q6 = p->split == QW_F_PACKED_Q6;
         const size_t rowb = (size_t)p->nblk * (nl ? 180u : q6 ? 210u : 110u), rows_a = nl || q6 ? 16 : p->split, rows_b = nl || q6 ? 0 : 16 - p->split;
+        if (p->pf) continue; // does not stand in for its source
         if (p->ha == h && p->A) lo[n] = (size_t)((const char *)p->A - (const char *)h->dptr), hi[n] = lo[n] + (size_t)p->ntiles * rows_a * rowb, n++;
         if (p->hb == h && p->B && rows_b) lo[n] = (size_t)((const char *)p->B - (const char *)h->dptr), hi[n] = lo[n] + (size_t)p->ntiles * rows_b * rowb, n++;
     }
@@ -1252,13 +1254,14 @@ static bool nbr_ok(qw_batch *b, uint32_t nbr) {
 static const uint8_t *get_pack(qw_batch *b, qw_hbuf *ha, const void *A, qw_hbuf *hb, const void *B, uint64_t ntiles, uint32_t nblk, uint32_t rowbytes, uint32_t split) {
     qw_gpu *g = b->g;
     if (!g->repack) return NULL;
+    const bool pf = split == QW_F_PACKED_NL && b->k->fam == FAM_PF;
     for (int i = 0; i < g->npacks; i++) {
-        const qw_pack *p = &g->packs[i];
+        qw_pack *p = &g->packs[i];
         if (p->A != A || p->B != B || p->ntiles != ntiles || p->nblk != nblk || p->split != split) continue;
         // The addresses are the key (a view of the same memory under another handle finds the copy too) — unless the
         // source was released: its address may since have been given to another allocation, so only its own handle matches.
         const bool gone = (p->ha && p->ha->released) || (p->hb && p->hb->released);
-        if (!gone || (p->ha == ha && p->hb == hb)) return p->dst;
+        if (!gone || (p->ha == ha && p->hb == hb)) return p->pf &= pf, p->dst;
     }
     if (b->noalloc) return NULL; // a copy that exists was found above; none is made here
     if ((ha && ha->released) || (hb && hb->released)) return NULL; // nothing left to copy from
@@ -1297,7 +1300,7 @@ static const uint8_t *get_pack(qw_batch *b, qw_hbuf *ha, const void *A, qw_hbuf 
         g->cappacks = g->cappacks ? 2 * g->cappacks : 64;
         g->packs = realloc(g->packs, sizeof *g->packs * (size_t)g->cappacks);
     }
-    g->packs[g->npacks++] = (qw_pack){.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .split = split, .dst = dst, .bytes = bytes};
+    g->packs[g->npacks++] = (qw_pack){.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .split = split, .dst = dst, .bytes = bytes, .pf = pf};
     g->pack_bytes += bytes;
     if (ha) ha->npack++;
     if (hb && hb != ha) hb->npack++;

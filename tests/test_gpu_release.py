@@ -97,3 +97,46 @@ def test_release_waits_until_every_matrix_of_the_buffer_has_a_copy(gpu, oracle):
     for bb in (wb, xb, ya, yb):
         bb.free()
     path.close()
+
+
+def test_release_refused_for_rows_that_only_the_packing_path_copied(gpu):
+    """IQ4_NL gate / up rows: moe_pf_gg makes a copy of them, but a decode step reads them in GGUF order, so their buffer is
+    not released. IQ4_NL down rows are, once a decode step has been through their copy, and both paths go on with it."""
+    import qwental_amd as q
+    from helpers import DeviceLayer
+    L = gpu.L
+    D, I, E, K, nb, T = 1280, 640, 8, 2, 3, 40
+    rng = np.random.default_rng(21)
+    m = synth.moe_layer(rng, D, I, E, fgu=20, fd=20, fsh=8)
+    path = q.Path(gpu, D, I, E, K, 16, device_scratch=True)
+    path.pf_reserve(T, 16)
+    dl = DeviceLayer(gpu, m, device_only=True)
+    ids, w = synth.zipf_ids(rng, T, E, K), np.full(T * K, 0.5, np.float32)
+    xb, ib, wb, ob = gpu.buf_from(synth.activations(rng, T, D)), gpu.buf_from(ids.ravel()), gpu.buf_from(w), gpu.buf(T * D * 2)
+    lg, sel, out = gpu.buf(path.logits_bytes(nb)), gpu.buf(path.sel_bytes(nb)), gpu.buf(nb * D * 2)
+
+    def packed():
+        b = gpu.batch()
+        path.pf_moe(b, dl.layer, T, xb, ib, wb, ob)
+        assert b.end() > 0, gpu.last_error()
+        return ob.view(np.uint16).copy()
+
+    def decoded():
+        b = gpu.batch()
+        path.gg_moe(b, dl.layer, nb, xb, lg, sel, out)
+        assert b.end() > 0, gpu.last_error()
+        return out.view(np.uint16).copy()
+
+    pk = packed()
+    for name in ("Wg", "Wu", "Wd"):
+        assert not L.qw_hip_buf_release_source(dl.bufs[name].ref()), name
+    dc = decoded()
+    for name in ("Wg", "Wu"):
+        assert not L.qw_hip_buf_release_source(dl.bufs[name].ref()), name
+    assert L.qw_hip_buf_release_source(dl.bufs["Wd"].ref()), gpu.last_error()
+    assert np.array_equal(packed(), pk) and np.array_equal(decoded(), dc)
+    assert not L.qw_hip_buf_release_source(dl.bufs["Wg"].ref())
+    for bb in (xb, ib, wb, ob, lg, sel, out):
+        bb.free()
+    dl.free()
+    path.close()
