@@ -101,8 +101,9 @@ typedef struct {
 typedef struct { qw_hbuf *b; bool out, whole; size_t lo, hi; } qw_use;
 
 // What the host and the device exchange about a batch in flight beside its data: pinned, one per batch at a time. t0 / t1:
-// the device clock at the start and the end of every submitted segment (0: not taken); done, copied: the batch's number
-// once its kernels have finished (where it was submitted without waiting) and once its outputs are in the shadows.
+// the device clock at the start and the end of every submitted segment (0: not taken); done, copied: 1 once its kernels
+// have finished (where it was submitted without waiting) and once its outputs are in the shadows. Cleared when a batch takes
+// the slot, which the batch before gave back after its last launch had ended.
 typedef struct { volatile uint64_t t0[9], t1[9]; volatile uint32_t done, copied; uint32_t pad[26]; } qw_ioslot;
 enum { QW_IO_SLOTS = 32 };
 
@@ -2223,7 +2224,7 @@ static bool io_wait(qw_batch *b, const volatile uint32_t *flag) {
     qw_gpu *g = b->g;
     for (double t0 = 0;;) {
         for (int i = 0; i < 512; i++) {
-            if (*flag == (uint32_t)b->seq) {
+            if (*flag) {
                 __atomic_thread_fence(__ATOMIC_ACQUIRE);
                 return true;
             }
@@ -2233,7 +2234,7 @@ static bool io_wait(qw_batch *b, const volatile uint32_t *flag) {
         else if (qw_now() - t0 > 20e-3) break;
     }
     if (!HIPOK(g, hipStreamSynchronize(g->stream[b->stream]))) return false;
-    if (*flag == (uint32_t)b->seq) return true;
+    if (*flag) return true;
     set_err(g, "a batch ended without its last launch");
     return false;
 }
@@ -2373,7 +2374,7 @@ static bool submit_segment(qw_batch *b, bool last) {
     if (b->events) {
         if (!HIPOK(g, hipEventRecord(ev[1], st))) { b->failed = true; return false; }
     } else if (!last) { // the segment's end, and for qw_batch_poll the batch's
-        qw_io end = {.a = {.t_enter = (uint64_t *)&b->io->t1[seg], .flag = b->submitted ? (uint32_t *)&b->io->done : NULL, .flagval = (uint32_t)b->seq}};
+        qw_io end = {.a = {.t_enter = (uint64_t *)&b->io->t1[seg], .flag = b->submitted ? (uint32_t *)&b->io->done : NULL, .flagval = 1}};
         if (!io_launch(b, &end)) return false;
     }
     b->done_l = b->nl;
@@ -2396,7 +2397,7 @@ void qw_batch_submit(qw_batch *b) {
 bool qw_batch_poll(qw_batch *b) {
     if (b->failed || !b->submitted) return true;
     if (b->events) return hipEventQuery(b->ev[2 * b->nseg - 1]) != hipErrorNotReady;
-    return b->io->done == (uint32_t)b->seq || hipStreamQuery(b->g->stream[b->stream]) != hipErrorNotReady; // (an error counts as done: the wait reports it)
+    return b->io->done || hipStreamQuery(b->g->stream[b->stream]) != hipErrorNotReady; // (an error counts as done: the wait reports it)
 }
 
 static void batch_free(qw_batch *b) {
@@ -2448,7 +2449,7 @@ static double batch_wait(qw_batch *b, bool ended) { // ended: submitted by qw_ba
         if (ended || down.a.n) {
             flag = &b->io->copied;
             if (ended) down.a.t_enter = (uint64_t *)&b->io->t1[b->nseg - 1];
-            down.a.flag = (uint32_t *)flag, down.a.flagval = (uint32_t)b->seq;
+            down.a.flag = (uint32_t *)flag, down.a.flagval = 1;
             ok = io_launch(b, &down);
         }
         ok = ok && (sync ? HIPOK(g, hipStreamSynchronize(st)) : io_wait(b, flag));
