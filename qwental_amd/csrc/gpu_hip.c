@@ -139,7 +139,7 @@ struct qw_batch {
     // expert's gate/up, and its gate/up dispatch the shared down; here they ride in the next launch, where they cost
     // almost nothing): set by moe_pre_gg / moe_gu_gg, consumed by moe_gu_gg / moe_dn_gg of the same batch.
     struct { bool valid; int fmt; const uint8_t *Wsg, *Wsu; qw_hbuf *hg, *hu; uint32_t rowbytes, nbr; } pend_sg;
-    struct { bool valid; int fmt; const uint8_t *Wsd; qw_hbuf *hd; float *Psh; uint32_t rowbytes, nbr; } pend_sd;
+    struct { bool valid; int fmt; const uint8_t *Wsd; qw_hbuf *hd; float *Psh; uint32_t rowbytes, nbr; int use; } pend_sd; // use: its binding of Psh
     struct { bool valid; qwk_select_args a; } pend_sel; // the selection moe_pre_gg owes: made inside the gate/up launch, or by a launch of its own
     // a grouped product over IQ3_S rows that waits for its twin (gate, then up over the same packed rows: one launch
     // over the tile-major copy that holds both); launched alone at the next other dispatch or at submit
@@ -1451,7 +1451,8 @@ static bool tr_gu(qw_batch *b) {
     b->pend_sd.valid = false;
     b->pend_sd.rowbytes = (uint32_t)fmt_rb(p->fsd, p->I);
     if (!bind_ptr(b, 2, (size_t)p->D * b->pend_sd.rowbytes, false, "shared down weights", (void **)&b->pend_sd.Wsd) ||
-        !bind_ptr(b, 3, (size_t)nbr * p->D * 4, true, "Psh", (void **)&b->pend_sd.Psh)) return false; // (not bind_whole: only a moe_dn_gg of this batch writes it)
+        !bind_ptr(b, 3, (size_t)nbr * p->D * 4, true, "Psh", (void **)&b->pend_sd.Psh)) return false; // (not bind_whole: it is written if a moe_dn_gg follows)
+    b->pend_sd.use = b->nuse - 1;
     b->pend_sd.valid = true;
     b->pend_sd.hd = b->buf[2].h;
     b->pend_sd.fmt = p->fsd;
@@ -1593,6 +1594,10 @@ static bool tr_dn_inner(qw_batch *b) {
         a.sd_rowbytes = b->pend_sd.rowbytes;
         a.snbr = b->pend_sd.nbr;
         b->pend_sd.valid = false;
+        qw_use *u = &b->use[b->pend_sd.use]; // Psh: written whole by this launch, unless something in between has read it
+        u->whole = true;
+        for (int i = b->pend_sd.use + 1; i < b->nuse; i++)
+            if (b->use[i].b == u->b && !b->use[i].out && b->use[i].lo < u->hi && b->use[i].hi > u->lo) u->whole = false;
     }
     const unsigned umax = umin((unsigned)p->E, nbr * (unsigned)p->topk);
     int fd = p->fd;
@@ -1719,6 +1724,7 @@ static bool tr_cmb(qw_batch *b) {
         if (same) {
             b->pend_dn.valid = false;
             d->nbr = nbr;
+            if (d->Wsd && d->snbr != nbr) b->use[b->pend_sd.use].whole = false; // the fused forms leave the rows of further tokens alone
             d->out = a.out;
             d->Psh = (float *)a.Psh;
             if (b->pend_gu.valid && b->pend_dn.quarters && b->pend_gu.a.nbr == nbr && (!d->Wsd || d->snbr == nbr)) { // gate/up, down and combine as one launch
@@ -1750,7 +1756,7 @@ static bool tr_cmb(qw_batch *b) {
 
 // ---------------------------------------------------------------- ragged packing (kernels/moe_prefill.metal; src/engine.c:4133-4224)
 // The sequence p_zero (the counters), moe_count, moe_plan(_t), moe_scatter of a step with at most QW_PREP_MAXP pairs runs as
-// one launch (qwk_moe_prep): each of the first three dispatches waits for the next one as long as it continues the
+// one launch (qwk_moe_prep, qwk_moe_prep_slices): each of the first three dispatches waits for the next one as long as it continues the
 // sequence on the same buffers; anything else launches what waits, one kernel per dispatch (QW_HIP_PK_SPLIT: always).
 static bool add_named(qw_batch *b, const char *kname, const char *fname, unsigned gx, unsigned bx, const void *args, size_t argsz) {
     const int first = b->nl;

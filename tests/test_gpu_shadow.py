@@ -200,7 +200,42 @@ def test_a_result_left_to_a_later_dispatch_keeps_the_hosts_bytes(gpu):
         b.dispatch(1)
         assert b.end() > 0, gpu.last_error()
         assert np.array_equal(psh.view(np.float32), mine) and np.array_equal(psh.read(dtype=np.float32), mine)
-    for bb in (xb, sb, H, psh):
+    # with moe_dn_gg and moe_cmb_gg behind it: written for the tokens of the combine, the rows of others computed or left alone
+    dn, cmb = (gpu.kernel("%s_8_s4_n2_e%dk%dd%di%d" % (n, E, K, D, I)) for n in ("moe_dn_gg", "moe_cmb_gg"))
+    pg, out = gpu.buf(nb * K * D * 4), gpu.buf(nb * D * 2)
+    got = {}
+    for tokens in (2, 1):
+        H.view(np.float16)[:] = np.random.default_rng(12).standard_normal(H.size // 2).astype(np.float16)  # (the shared expert's part is moe_pre_gg's)
+        mine = rng.standard_normal(nb * D).astype(np.float32)
+        psh.view(np.float32)[:] = mine
+        b = gpu.batch()
+        b.kernel(k)
+        for i, bb in ((0, dl.bufs["Wg"]), (1, dl.bufs["Wu"]), (2, dl.bufs["Wsd"]), (3, psh), (4, xb), (5, sb), (6, H)):
+            b.buf(i, bb)
+        b.bytes(12, np.array([nb], np.uint32))
+        b.dispatch(1)
+        b.kernel(dn)
+        for i, bb in ((0, dl.bufs["Wd"]), (2, H), (3, sb), (9, pg)):
+            b.buf(i, bb)
+        b.dispatch(1)
+        b.kernel(cmb)
+        for i, bb in ((1, psh), (3, sb), (4, out), (9, pg)):
+            b.buf(i, bb)
+        b.bytes(8, np.array([tokens], np.uint32))
+        b.dispatch(1)
+        assert b.end() > 0, gpu.last_error()
+        got[tokens] = psh.view(np.float32).copy()
+        psh.view(np.float32)[:] = rng.standard_normal(nb * D)  # other bytes in HBM before the next one
+        b = gpu.batch()
+        b.kernel(k)
+        for i, bb in ((0, dl.bufs["Wg"]), (1, dl.bufs["Wu"]), (2, dl.bufs["Wsd"]), (3, psh), (4, xb), (5, sb), (6, H)):
+            b.buf(i, bb)
+        b.bytes(12, np.array([nb], np.uint32))
+        b.dispatch(1)
+        assert b.end() > 0, gpu.last_error()
+    assert np.abs(got[2]).min() > 0 and np.array_equal(got[1][:D], got[2][:D])
+    assert np.array_equal(got[1][D:], mine[D:]) or np.array_equal(got[1][D:], got[2][D:])
+    for bb in (xb, sb, H, psh, pg, out):
         bb.free()
     dl.free()
     path.close()
