@@ -53,7 +53,9 @@ void *qw_hip_buf_devptr(const qw_buf *b);
  * they are); so are, at exactly their size, IQ4_NL down matrices with rows of 320 or 640 values at their first moe_dn_gg, and
  * IQ4_NL matrices whose rows are a multiple of 320 values, gate and up rows among them, at their first moe_pf_gg. The latter
  * are resident twice where decode steps run beside the packing path: those read IQ4_NL gate and up rows in GGUF order (512
- * experts of 640 x 2560: 944 MB more a layer for gate and up). A copy is dropped when the source buffer is freed, marked
+ * experts of 640 x 2560: 944 MB more a layer for gate and up); and, at exactly their size, Q8_0 and Q4_K gate / up matrices
+ * (D a multiple of 512) at their first moe_gu_gg and Q8_0 and (from 64 MB on) Q6_K down matrices (I 256 or 512) at their first
+ * moe_dn_gg, all of which stay resident twice. A copy is dropped when the source buffer is freed, marked
  * dirty, uploaded, written, or bound as a kernel's output. Without memory for one the dispatch reads the GGUF rows. Buffers of at most QW_HIP_SMALL_BYTES with a host shadow are never copied. QW_HIP_REPACK=0 in the
  * environment, or qw_hip_set_repack(g, false), turns the copies off (kernels then read the GGUF rows directly). */
 void qw_hip_set_repack(qw_gpu *g, bool on);
@@ -61,7 +63,8 @@ size_t qw_hip_packed_bytes(const qw_gpu *g);
 /* Keep only the tile-major copies of a weight buffer: frees the buffer's device bytes (the GGUF-order rows) once the
  * copies that the kernels read have been made, i.e. after every matrix in it has been through a dispatch that makes one
  * (moe_gu_gg, moe_dn_gg, moe_pf_gg and qmv_gg over IQ3_S rows; moe_dn_gg over IQ4_NL rows of 320 or 640 - a copy of IQ4_NL
- * rows that only moe_pf_gg has asked for does not count, decode steps may need the GGUF order). Residency of
+ * rows that only moe_pf_gg has asked for does not count, decode steps may need the GGUF order, nor do the copies of the MoE
+ * kernels' Q8_0, Q4_K and Q6_K rows). Residency of
  * such a matrix drops from 2.018 to 1.018 times its bytes. Afterwards the buffer may only be bound as those weights:
  * a dispatch that no existing copy serves (another shape or split, a matrix that was never dispatched, dq_test, any output
  * role) fails the batch with a message, the explicit copy calls return false, qw_hip_buf_devptr gives NULL, and the
@@ -99,12 +102,13 @@ unsigned qw_hip_graph_launches(const qw_gpu *g);
  *                             qw_hip_reload_switches() is called. All workgroups of such a launch must be resident at once:
  *                             it is used on stream 0 only and never by qw_path_gg_moe_noalloc (the caller's stream).
  *   QW_HIP_DNC_NB=n           token count up to which moe_dn_gg + moe_cmb_gg run as one launch (default 2, at most 4; 0: never)
- *   QW_HIP_DNQ_MIN=n          token count from which (up to 16) they run as the one launch by token shares, for tile-major IQ3_S
- *                             down rows (default 2; 0: never)
+ *   QW_HIP_DNQ_MIN=n          token count from which (up to 16) they run as the one launch by token shares, for tile-major IQ3_S,
+ *                             Q8_0 and Q6_K down rows (default 2; 0: never)
  *   QW_HIP_PK_SPLIT           the packing sequence (p_zero, moe_count, moe_plan_t, moe_scatter, moe_pf_gg x 2, p_act2) one launch per
  *                             dispatch instead of one launch for the first four and SwiGLU inside the gate / up launch
  *   QW_HIP_SIDE=1             a shared expert's gate/up in the K-quant / IQ4 / plain formats runs on a side stream beside the router
- *   QW_HIP_DN_ANY             IQ4_NL, K-quant and IQ4_XS down rows take the any-shape kernel instead of the range kernel
+ *   QW_HIP_DN_ANY             IQ4_NL, K-quant and IQ4_XS down rows take the any-shape kernel instead of the range kernel (and, like Q8_0 rows,
+ *                             no tile-major copy)
  *   QW_HIP_NL_C4              IQ4_NL down rows from GGUF order in chunks of four blocks instead of ten
  *   QW_HIP_NO_SWIGLU_MATVEC   such a shared expert's gate/up as two launches (matvec, then SwiGLU) instead of one
  *   QW_HIP_KQ_OWN_LAUNCH      such a shared expert's gate/up as a launch of its own instead of on the workgroups behind the router's

@@ -74,15 +74,15 @@ typedef struct qw_hbuf {
     bool released;   // the device bytes were freed (qw_hip_buf_release_source): dptr is only the key of its tile-major copies
 } qw_hbuf;
 
-// A tile-major copy of IQ3_S weight rows (layout: qwk_pack_args), made at the first use of a weight matrix.
+// A tile-major copy of weight rows (layouts: the QW_F_PACKED* of qw_kargs.h), made at the first use of a weight matrix.
 typedef struct {
     const void *A, *B;
     qw_hbuf *ha, *hb;
     uint64_t ntiles;
-    uint32_t nblk, split;
+    uint32_t nblk, fmt, split;
     void *dst;
     size_t bytes;
-    bool pf; // IQ4_NL rows that only moe_pf_gg has asked for: a decode dispatch may read them in GGUF order (gate / up rows)
+    bool pf; // IQ4_NL rows that only moe_pf_gg has asked for, Q6_K rows that only moe_dn_gg has: another dispatch may read them in GGUF order
 } qw_pack;
 
 typedef struct {
@@ -150,7 +150,8 @@ struct qw_batch {
     struct { int stage; qwk_zero_args z; qwk_count_args c; qwk_plan_args pl; const char *kn[3]; } pend_pk;
     // a down projection over a few tokens that waits for the combine of the same layer: both in one launch
     // (qwk_dnc_*); launched as it is at any other dispatch or at submit
-    struct { bool valid; qwk_dn_args a; const char *fname, *fused, *kname; unsigned grid, fused_grid; bool quarters; } pend_dn;
+    // plain: its arguments without the combine, where they are not those of the joint form (Wd NULL: they are)
+    struct { bool valid; qwk_dn_args a, plain; const char *fname, *fused, *kname; unsigned grid, fused_grid; bool quarters; } pend_dn;
     // a routed gate/up launch that waits for the down projection and the combine of the same layer: the three run as one
     // launch (qwk_gud_*) when the down dispatch qualifies for the form by token shares; launched as it is otherwise
     struct { bool valid; qwk_gu_args a; const char *fname, *kname; unsigned grid; } pend_gu;
@@ -765,6 +766,18 @@ void *qw_hip_buf_devptr(const qw_buf *b) {
     h->addr = true; // the address may be kept: its holder sees every later submit's bytes
     return h->dptr;
 }
+// The tile-major formats: bytes of a (tile, unit of K), source bytes of a row in it, the kernel that makes the copy, and whether
+// every dispatch that can bind such rows reads the copy (only then can the copy stand in for its source).
+typedef struct { uint32_t slab, row; const char *fname; bool stands_in; } qw_pack_fmt;
+static qw_pack_fmt pack_of(uint32_t fmt) {
+    switch (fmt) {
+    case QW_F_PACKED_NL: return (qw_pack_fmt){QW_NL_CHUNK_BYTES, 180, "qwk_pack_nl", true};
+    case QW_F_PACKED_Q6: return (qw_pack_fmt){QW_Q6_SLAB_BYTES, 210, "qwk_pack_q6", true};
+    case QW_F_PACKED_Q8: return (qw_pack_fmt){QW_Q8_SLAB_BYTES, 272, "qwk_pack_q8", false};
+    case QW_F_PACKED_Q4K: return (qw_pack_fmt){QW_Q4K_SLAB_BYTES, 144, "qwk_pack_q4k", false};
+    default: return (qw_pack_fmt){QW_SLAB_BYTES, 110, "qwk_pack_iq3", true};
+    }
+}
 // Free the device bytes of a weight buffer and keep its tile-major copies (include/qw_hip_ext.h).
 // Bytes of h that some tile-major copy was made from: the union of the copies' source ranges inside the buffer.
 static size_t packed_source_bytes(const qw_hbuf *h) {
@@ -774,9 +787,8 @@ static size_t packed_source_bytes(const qw_hbuf *h) {
     int n = 0;
     for (int i = 0; i < g->npacks && n + 2 <= MAXIV; i++) {
         const qw_pack *p = &g->packs[i];
-        const bool nl = p->split == QW_F_PACKED_NL, q6 = p->split == QW_F_PACKED_Q6;
-        const size_t rowb = (size_t)p->nblk * (nl ? 180u : q6 ? 210u : 110u), rows_a = nl || q6 ? 16 : p->split, rows_b = nl || q6 ? 0 : 16 - p->split;
-        if (p->pf) continue; // does not stand in for its source
+        const size_t rowb = (size_t)p->nblk * pack_of(p->fmt).row, rows_a = p->split, rows_b = 16 - p->split;
+        if (p->pf || !pack_of(p->fmt).stands_in) continue; // does not stand in for its source
         if (p->ha == h && p->A) lo[n] = (size_t)((const char *)p->A - (const char *)h->dptr), hi[n] = lo[n] + (size_t)p->ntiles * rows_a * rowb, n++;
         if (p->hb == h && p->B && rows_b) lo[n] = (size_t)((const char *)p->B - (const char *)h->dptr), hi[n] = lo[n] + (size_t)p->ntiles * rows_b * rowb, n++;
     }
@@ -1065,7 +1077,7 @@ static const void *glut(const qw_gpu *g) { return (const char *)g->tabs + QW_TAB
 // Blocks per prefetch chunk for a row of K values (the kernels are instantiated for these; 1 = any K).
 static int chunk_of(int F, int K) { return K % 512 == 0 ? (F == 21 ? 2 : 16) : 1; }
 
-static const uint8_t *get_pack(qw_batch *b, qw_hbuf *ha, const void *A, qw_hbuf *hb, const void *B, uint64_t ntiles, uint32_t nblk, uint32_t rowbytes, uint32_t split);
+static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const void *A, qw_hbuf *hb, const void *B, uint64_t ntiles, uint32_t nblk, uint32_t rowbytes);
 // One launch of the multi-format matvec over nmat matrices; W / y already bound into a.
 // Few tiles: the parts a tile's K range is cut into, one wave each — the largest divisor of the chunk count up to 6
 // that the wave slots of the device hold (a workgroup's waves beyond a whole number of tiles stay idle).
@@ -1117,7 +1129,7 @@ static bool launch_qmvm(qw_batch *b, qwk_qmvm_args *a, qw_hbuf *const *hw) {
         // its first use: five coalesced loads a block instead of seventeen 4-byte ones and seventeen cross-lane moves.
         if (hw && a->fmt[j] == 14 && a->K % 256 == 0 && a->N[j] % 16 == 0 && a->N[j] >= QW_Q6_PACK_MIN_ROWS) {
             const uint32_t nblk = a->K / 256;
-            const uint8_t *pk = get_pack(b, hw[j], a->W[j], NULL, NULL, a->N[j] / 16, nblk, a->rowbytes[j], QW_F_PACKED_Q6);
+            const uint8_t *pk = get_pack(b, QW_F_PACKED_Q6, hw[j], a->W[j], NULL, NULL, a->N[j] / 16, nblk, a->rowbytes[j]);
             if (pk) a->W[j] = pk, a->fmt[j] = QW_F_PACKED_Q6, a->rowbytes[j] = nblk * QW_Q6_SLAB_BYTES;
         }
         a->ntiles[j] = cdiv(a->N[j], 16);
@@ -1193,7 +1205,7 @@ static bool tr_qmv(qw_batch *b) { // src/engine.c:717-723: 0 W, 3 x, 4 y, 5 {N, 
     int F = p->F;
     if (F == 21 && p->K <= 2560 && a.N % 16 == 0) { // tile-major copy of the rows, made at first use
         const uint32_t nblk = (uint32_t)p->K / 256;
-        const uint8_t *pk = get_pack(b, b->buf[0].h, a.W, NULL, NULL, a.N / 16, nblk, a.rowbytes, 16);
+        const uint8_t *pk = get_pack(b, QW_F_PACKED, b->buf[0].h, a.W, NULL, NULL, a.N / 16, nblk, a.rowbytes);
         if (pk) F = QW_F_PACKED, a.W = pk, a.rowbytes = nblk * QW_SLAB_BYTES;
     }
     if (b->buf[0].h->released && F != QW_F_PACKED) return fail(b, "%s: the GGUF-order bytes of the weights were released and no tile-major copy serves this dispatch", b->k->name);
@@ -1247,18 +1259,19 @@ static bool nbr_ok(qw_batch *b, uint32_t nbr) {
 }
 
 // gate/up arguments. shared: one expert at (iWg, iWu), all tokens, slot topk.
-// The packed copy of IQ3_S rows: tiles of `split` rows of A and 16 - split rows of B (B = NULL, split 16: one matrix);
-// split = QW_F_PACKED_NL: the packed copy of one matrix of IQ4_NL rows, nblk chunks of ten blocks a row.
+// The packed copy (format fmt) of one matrix A in tiles of 16 rows, or of two, A and B, in tiles of eight rows of each; nblk: units of K
+// a row (256 values; IQ4_NL: chunks of ten blocks).
 // Made at the first request, on the batch's stream, and complete when this returns; NULL when packing is off, the
 // source may change without notice (a small buffer with a host shadow is copied at every submit) or memory is short:
 // the caller then reads the GGUF rows directly.
-static const uint8_t *get_pack(qw_batch *b, qw_hbuf *ha, const void *A, qw_hbuf *hb, const void *B, uint64_t ntiles, uint32_t nblk, uint32_t rowbytes, uint32_t split) {
+static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const void *A, qw_hbuf *hb, const void *B, uint64_t ntiles, uint32_t nblk, uint32_t rowbytes) {
     qw_gpu *g = b->g;
     if (!g->repack) return NULL;
-    const bool pf = split == QW_F_PACKED_NL && b->k->fam == FAM_PF;
+    const bool pf = (fmt == QW_F_PACKED_NL && b->k->fam == FAM_PF) || (fmt == QW_F_PACKED_Q6 && b->k->fam == FAM_DN);
+    const uint32_t split = B ? 8 : 16;
     for (int i = 0; i < g->npacks; i++) {
         qw_pack *p = &g->packs[i];
-        if (p->A != A || p->B != B || p->ntiles != ntiles || p->nblk != nblk || p->split != split) continue;
+        if (p->A != A || p->B != B || p->ntiles != ntiles || p->nblk != nblk || p->fmt != fmt) continue;
         // The addresses are the key (a view of the same memory under another handle finds the copy too) — unless the
         // source was released: its address may since have been given to another allocation, so only its own handle matches.
         const bool gone = (p->ha && p->ha->released) || (p->hb && p->hb->released);
@@ -1280,10 +1293,9 @@ static const uint8_t *get_pack(qw_batch *b, qw_hbuf *ha, const void *A, qw_hbuf 
             h->dirty = false;
         }
     }
-    const bool nl = split == QW_F_PACKED_NL, q6 = split == QW_F_PACKED_Q6; // IQ4_NL rows: nblk counts chunks of ten blocks; Q6_K rows: blocks
-    hipFunction_t f = get_func(g, nl ? "qwk_pack_nl" : q6 ? "qwk_pack_q6" : "qwk_pack_iq3");
+    hipFunction_t f = get_func(g, pack_of(fmt).fname);
     if (!f) return NULL;
-    const size_t bytes = (size_t)ntiles * nblk * (nl ? QW_NL_CHUNK_BYTES : q6 ? QW_Q6_SLAB_BYTES : QW_SLAB_BYTES);
+    const size_t bytes = (size_t)ntiles * nblk * pack_of(fmt).slab;
     void *dst;
     if (hipMalloc(&dst, bytes) != hipSuccess) {
         (void)hipGetLastError();
@@ -1301,7 +1313,7 @@ static const uint8_t *get_pack(qw_batch *b, qw_hbuf *ha, const void *A, qw_hbuf 
         g->cappacks = g->cappacks ? 2 * g->cappacks : 64;
         g->packs = realloc(g->packs, sizeof *g->packs * (size_t)g->cappacks);
     }
-    g->packs[g->npacks++] = (qw_pack){.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .split = split, .dst = dst, .bytes = bytes, .pf = pf};
+    g->packs[g->npacks++] = (qw_pack){.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .fmt = fmt, .split = split, .dst = dst, .bytes = bytes, .pf = pf};
     g->pack_bytes += bytes;
     if (ha) ha->npack++;
     if (hb && hb != ha) hb->npack++;
@@ -1419,7 +1431,7 @@ static bool tr_pre(qw_batch *b) {
     const unsigned cpr = (unsigned)p->D / 512;
     if (p->D % 512 == 0 && cpr <= 8 && !b->sw.shared_in_gu) {
         const uint32_t nblk = (uint32_t)p->D / 256;
-        const uint8_t *ps = p->fsg == 21 ? get_pack(b, b->pend_sg.hg, b->pend_sg.Wsg, b->pend_sg.hu, b->pend_sg.Wsu, (uint64_t)(p->I / 8), nblk, (uint32_t)rb, 8) : NULL;
+        const uint8_t *ps = p->fsg == 21 ? get_pack(b, QW_F_PACKED, b->pend_sg.hg, b->pend_sg.Wsg, b->pend_sg.hu, b->pend_sg.Wsu, (uint64_t)(p->I / 8), nblk, (uint32_t)rb) : NULL;
         if (p->fsg == 8 || ps) {
             a.g = (qwk_gu_args){.Wg = ps ? ps : b->pend_sg.Wsg, .Wu = ps ? NULL : b->pend_sg.Wsu, .x = a.r.x, .H = h, .D = (uint32_t)p->D, .I = (uint32_t)p->I,
                                 .rowbytes = ps ? nblk * QW_SLAB_BYTES : (uint32_t)rb, .nbr = nbr, .topk = (uint32_t)p->topk, .gnb = (uint32_t)p->gnb, .shared = 1,
@@ -1485,8 +1497,8 @@ static bool tr_gu(qw_batch *b) {
     }
     if (fgu == 21) { // tile-major copies of the IQ3_S rows, made at first use
         const uint32_t nblk = (uint32_t)p->D / 256, tileb = nblk * QW_SLAB_BYTES;
-        const uint8_t *pk = get_pack(b, b->buf[0].h, a.Wg, b->buf[1].h, a.Wu, (uint64_t)p->E * (uint64_t)(p->I / 8), nblk, a.rowbytes, 8);
-        const uint8_t *ps = pk && fs == 21 ? get_pack(b, hsg, a.Wsg, hsu, a.Wsu, (uint64_t)(p->I / 8), nblk, a.sg_rowbytes, 8) : NULL;
+        const uint8_t *pk = get_pack(b, QW_F_PACKED, b->buf[0].h, a.Wg, b->buf[1].h, a.Wu, (uint64_t)p->E * (uint64_t)(p->I / 8), nblk, a.rowbytes);
+        const uint8_t *ps = pk && fs == 21 ? get_pack(b, QW_F_PACKED, hsg, a.Wsg, hsu, a.Wsu, (uint64_t)(p->I / 8), nblk, a.sg_rowbytes) : NULL;
         if (pk && (fs != 21 || ps)) {
             fgu = QW_F_PACKED;
             a.Wg = pk, a.Wu = NULL, a.rowbytes = tileb;
@@ -1494,8 +1506,14 @@ static bool tr_gu(qw_batch *b) {
         }
     }
     if ((b->buf[0].h->released || b->buf[1].h->released) && fgu != QW_F_PACKED) return fail(b, "%s: the GGUF-order bytes of the weights were released and no tile-major copy serves this dispatch", b->k->name);
+    // Q8_0 and Q4_K rows: the same, where the shared expert's tiles are not in this launch
+    if ((fgu == 8 || fgu == 12) && !fs && p->D % 512 == 0 && b->buf[0].off % 16 == 0 && b->buf[1].off % 16 == 0) {
+        const uint32_t pf = fgu == 8 ? QW_F_PACKED_Q8 : QW_F_PACKED_Q4K, nblk = (uint32_t)p->D / 256;
+        const uint8_t *pk = get_pack(b, pf, b->buf[0].h, a.Wg, b->buf[1].h, a.Wu, (uint64_t)p->E * (uint64_t)(p->I / 8), nblk, a.rowbytes);
+        if (pk) fgu = (int)pf, cg = 2, a.Wg = pk, a.Wu = NULL, a.rowbytes = nblk * pack_of(pf).slab;
+    }
     char fn[64];
-    if (rt) {
+    if (rt && rt_ok(fgu)) {
         if (fs) fname_fmt(fn, sizeof fn, "qwk_gu_rt_s%d_c1", fs);
         else fname_fmt(fn, sizeof fn, "qwk_gu_rt");
     } else if (fs) fname_fmt(fn, sizeof fn, "qwk_gu_f%d_c%d_s%d_c%d", fgu, cg, fs, cs);
@@ -1538,7 +1556,8 @@ static bool flush_dn(qw_batch *b) {
     if (!b->pend_dn.valid) return true;
     b->pend_dn.valid = false;
     const int first = b->nl;
-    if (!add_launch(b, b->pend_dn.fname, b->pend_dn.grid, 64 * QW_WAVES_DNR, &b->pend_dn.a, sizeof b->pend_dn.a)) return false;
+    const qwk_dn_args *a = b->pend_dn.plain.Wd ? &b->pend_dn.plain : &b->pend_dn.a;
+    if (!add_launch(b, b->pend_dn.fname, b->pend_dn.grid, 64 * QW_WAVES_DNR, a, sizeof *a)) return false;
     if (b->nl > first) b->l[b->nl - 1].kname = b->pend_dn.kname, b->l[b->nl - 1].last_of_dispatch = true;
     return true;
 }
@@ -1571,6 +1590,7 @@ static bool tr_dn(qw_batch *b) {
     }
     return true;
 }
+#define QW_Q6_DOWN_PACK_MIN ((size_t)64 << 20)
 static bool tr_dn_inner(qw_batch *b) {
     const qw_kparams *p = &b->k->p;
     const uint32_t nbr = (uint32_t)p->NB;
@@ -1586,6 +1606,7 @@ static bool tr_dn_inner(qw_batch *b) {
         !bind_ptr(b, 3, QW_SEL_BYTES((size_t)p->gnb, (size_t)p->topk), false, "selection", (void **)&a.sel)) return false;
     int fs = 0;
     qw_hbuf *hsd = NULL;
+    b->pend_dn.plain.Wd = NULL;
     if (b->pend_sd.valid) {
         hsd = b->pend_sd.hd;
         fs = b->pend_sd.fmt;
@@ -1604,6 +1625,35 @@ static bool tr_dn_inner(qw_batch *b) {
     // A pair of types without a build of its own (Q4_K, Q5_K, Q6_K or IQ4_XS on either side; IQ4_NL beside IQ3_S): the
     // kernel that takes both types as arguments, rows in GGUF order.
     const bool kq_d = rt_ok(fd) && fd != 20, kq_s = rt_ok(fs) && fs != 20;
+    // Q8_0 and Q6_K rows from tile-major copies, down and combine in one launch: one token as qwk_dnc_*, two to sixteen as qwk_dnq_*.
+    // Everything that form asks of the shape, and a shared expert in the same format (or Q8_0 beside Q6_K, in GGUF order). Against
+    // the range kernel on GGUF rows and the combine behind it (512 experts of 2048 x 512, top-10, us): Q8_0 26.5 + 4.8 -> 14.2 at four
+    // tokens, 76.5 + 4.8 -> 35.4 at sixteen, one token (there one launch too) 11.1 -> 8.3; Q6_K 16.8 + 4.6 -> 15.3, 43.0 + 4.8 -> 33.1.
+    // Q6_K stacks of less than 64 MB stay with the range kernel.
+    if ((fd == 8 || fd == 14) && (fs == 0 || fs == fd || fs == 8) && p->I % 256 == 0 && p->I <= 512 && p->topk <= 10 && p->gnb * p->topk <= (int)QW_DNQ_MAXU && p->D % 256 == 0 &&
+        (fd == 8 || (size_t)p->E * (size_t)p->D * rb >= QW_Q6_DOWN_PACK_MIN) && b->buf[0].off % 2 == 0 && (uintptr_t)a.H % 16 == 0 && !rel && !b->sw.dn_any && (nbr == 1 ? b->sw.dnc_nb >= 1 : b->sw.dnq_min && nbr >= b->sw.dnq_min)) {
+        const uint32_t pf = fd == 8 ? QW_F_PACKED_Q8 : QW_F_PACKED_Q6, nblk = (uint32_t)p->I / 256, tileb = nblk * pack_of(pf).slab;
+        const uint8_t *pk = get_pack(b, pf, b->buf[0].h, a.Wd, NULL, NULL, (uint64_t)p->E * (uint64_t)(p->D / 16), nblk, a.rowbytes);
+        const uint8_t *ps = pk && fs == fd ? get_pack(b, pf, hsd, a.Wsd, NULL, NULL, (uint64_t)(p->D / 16), nblk, a.sd_rowbytes) : NULL;
+        if (pk && (fs != fd || ps)) {
+            char fn[48], fu[48], tail[16] = "";
+            if (fs) fname_fmt(tail, sizeof tail, fs == fd ? "_s%u_c1" : "_s8_c4", pf);
+            fname_fmt(fu, sizeof fu, "qwk_dn%c_f%u_c1%s", nbr == 1 ? 'c' : 'q', pf, tail);
+            b->pend_dn.valid = true;
+            b->pend_dn.plain = a; // without a combine behind it: the range kernel on the GGUF rows
+            if (fd == 8) fname_fmt(tail, sizeof tail, fs ? "_s8_c4" : "");
+            else if (fs) fname_fmt(tail, sizeof tail, fs == 14 ? "_s14_c1" : "_s8_c4");
+            fname_fmt(fn, sizeof fn, "qwk_dnr_f%d_c%d%s", fd, fd == 8 ? 4 : 1, tail);
+            a.Wd = pk, a.rowbytes = tileb;
+            if (ps) a.Wsd = ps, a.sd_rowbytes = tileb;
+            const unsigned nq = nbr == 1 ? 1 : dnq_quarters(nbr), tpw = nq > 2 ? 2 : 1;
+            a.nq = nq, a.tpw = tpw;
+            b->pend_dn.a = a;
+            b->pend_dn.fname = intern(fn), b->pend_dn.fused = intern(fu), b->pend_dn.kname = b->k->name, b->pend_dn.quarters = nbr > 1;
+            b->pend_dn.grid = persistent_grid(b->g, umax * (unsigned)(p->D / 16) + (unsigned)p->D / 16, QW_WAVES_DNR), b->pend_dn.fused_grid = (unsigned)p->D / 16 / tpw * nq;
+            return true;
+        }
+    }
     // The range kernel on GGUF rows (I is a multiple of the block, 256, and H rows fit in LDS up to 512; they are copied 16 bytes a lane)
     if (kq_d && (fs == 0 || fs == fd || fs == 8) && p->I <= 512 && (uintptr_t)a.H % 16 == 0 && !rel && !b->sw.dn_any) {
         char fn[48], tail[16] = "";
@@ -1628,8 +1678,8 @@ static bool tr_dn_inner(qw_batch *b) {
     }
     if (fd == 21 && p->I <= 512) {
         const uint32_t nblk = (uint32_t)p->I / 256, tileb = nblk * QW_SLAB_BYTES;
-        const uint8_t *pk = get_pack(b, b->buf[0].h, a.Wd, NULL, NULL, (uint64_t)p->E * (uint64_t)(p->D / 16), nblk, a.rowbytes, 16);
-        const uint8_t *ps = pk && fs == 21 ? get_pack(b, hsd, a.Wsd, NULL, NULL, (uint64_t)(p->D / 16), nblk, a.sd_rowbytes, 16) : NULL;
+        const uint8_t *pk = get_pack(b, QW_F_PACKED, b->buf[0].h, a.Wd, NULL, NULL, (uint64_t)p->E * (uint64_t)(p->D / 16), nblk, a.rowbytes);
+        const uint8_t *ps = pk && fs == 21 ? get_pack(b, QW_F_PACKED, hsd, a.Wsd, NULL, NULL, (uint64_t)(p->D / 16), nblk, a.sd_rowbytes) : NULL;
         if (pk && (fs != 21 || ps)) {
             fd = QW_F_PACKED;
             a.Wd = pk, a.rowbytes = tileb;
@@ -1643,8 +1693,8 @@ static bool tr_dn_inner(qw_batch *b) {
     if (fd == 20 && p->I <= 640 && !b->sw.dn_any) { // the range kernel with rows of up to 640 staged
         if (p->I % 320 == 0) { // tile-major copies, as for IQ3_S rows (the shared expert's only together with the routed ones)
             const uint32_t nch = (uint32_t)p->I / 320, tileb = nch * QW_NL_CHUNK_BYTES;
-            const uint8_t *pk = get_pack(b, b->buf[0].h, a.Wd, NULL, NULL, (uint64_t)p->E * (uint64_t)(p->D / 16), nch, a.rowbytes, QW_F_PACKED_NL);
-            const uint8_t *ps = pk && fs == 20 ? get_pack(b, hsd, a.Wsd, NULL, NULL, (uint64_t)(p->D / 16), nch, a.sd_rowbytes, QW_F_PACKED_NL) : NULL;
+            const uint8_t *pk = get_pack(b, QW_F_PACKED_NL, b->buf[0].h, a.Wd, NULL, NULL, (uint64_t)p->E * (uint64_t)(p->D / 16), nch, a.rowbytes);
+            const uint8_t *ps = pk && fs == 20 ? get_pack(b, QW_F_PACKED_NL, hsd, a.Wsd, NULL, NULL, (uint64_t)(p->D / 16), nch, a.sd_rowbytes) : NULL;
             if (pk && (fs != 20 || ps)) {
                 a.Wd = pk, a.rowbytes = tileb;
                 if (fs == 20) a.Wsd = ps, a.sd_rowbytes = tileb;
@@ -1727,7 +1777,7 @@ static bool tr_cmb(qw_batch *b) {
             if (d->Wsd && d->snbr != nbr) b->use[b->pend_sd.use].whole = false; // the fused forms leave the rows of further tokens alone
             d->out = a.out;
             d->Psh = (float *)a.Psh;
-            if (b->pend_gu.valid && b->pend_dn.quarters && b->pend_gu.a.nbr == nbr && (!d->Wsd || d->snbr == nbr)) { // gate/up, down and combine as one launch
+            if (b->pend_gu.valid && b->pend_dn.quarters && !b->pend_dn.plain.Wd && b->pend_gu.a.nbr == nbr && (!d->Wsd || d->snbr == nbr)) { // gate/up, down and combine as one launch
                 unsigned nq, tpw;
                 gud_shape(nbr, &nq, &tpw);
                 const unsigned grid = (unsigned)b->g->ncu, tpe = a.D / 16;
@@ -1882,7 +1932,7 @@ static bool launch_pf(qw_batch *b, qwk_pf_args *a, int F, int E, qw_hbuf *hw, qw
     const bool several = a->tm > 16 || a->K > 2560 || (uint64_t)a->M * a->M * inner >= (uint64_t)E << 26;
     if (F == 20 && a->K % 320 == 0 && blocked) {
         const uint32_t nch = a->K / 320;
-        const uint8_t *pk = get_pack(b, hw, a->W, NULL, NULL, (uint64_t)E * (a->N / 16), nch, a->rowbytes, QW_F_PACKED_NL);
+        const uint8_t *pk = get_pack(b, QW_F_PACKED_NL, hw, a->W, NULL, NULL, (uint64_t)E * (a->N / 16), nch, a->rowbytes);
         if (pk) {
             a->W = pk, a->rowbytes = nch * QW_NL_CHUNK_BYTES;
             return add_launch(b, "qwk_pfg_f120", (unsigned)b->g->ncu, 512, a, sizeof *a);
@@ -1891,7 +1941,7 @@ static bool launch_pf(qw_batch *b, qwk_pf_args *a, int F, int E, qw_hbuf *hw, qw
     if (F == 21 && a->K % 256 == 0) {
         const uint32_t nblk = a->K / 256, split = wb ? 8 : 16;
         const uint64_t ntiles = (uint64_t)E * (a->N / split);
-        const uint8_t *pk = get_pack(b, hw, a->W, wb ? hwb : NULL, wb, ntiles, nblk, a->rowbytes, split);
+        const uint8_t *pk = get_pack(b, QW_F_PACKED, hw, a->W, wb ? hwb : NULL, wb, ntiles, nblk, a->rowbytes);
         if (pk) {
             a->W = pk, a->rowbytes = nblk * QW_SLAB_BYTES, a->split = split, a->ntn = a->N / split;
             if (blocked && several) return add_launch(b, "qwk_pfg_f121", (unsigned)b->g->ncu, 512, a, sizeof *a);

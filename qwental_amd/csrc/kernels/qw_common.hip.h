@@ -240,6 +240,7 @@ __device__ __forceinline__ bool qw_grid_barrier(uint32_t *sync, uint32_t gen0, u
 }
 
 // ---------------------------------------------------------------- activation fragment providers (operand A)
+__device__ __forceinline__ h8 qw_join4(h4 a, h4 b) { return h8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
 // Four values of token m, koff = a multiple of 8 plus 4 times the lane's k-group: byte offset of the half of a 16-byte unit.
 // (From the unit, ((koff >> 3) * 16 + m) * 16 + (koff & 4) * 2, the compiler made five instructions a read wherever the K range
 // of a chunk is no power of two; this is one shift of the chunk's base and constants that the reads carry.)
@@ -261,6 +262,13 @@ struct qw_afrag_lds {
     __device__ __forceinline__ h8 lo(uint32_t) const { return h8{}; }
     __device__ __forceinline__ h4 hi4(uint32_t koff) const { return __builtin_bit_cast(h4, qw_half_read(xf, qw_half_at(koff, m))); } // koff: qw_half_at
     __device__ __forceinline__ h4 lo4(uint32_t) const { return h4{}; }
+};
+
+// The same with the sums of 32 activations beside them: xs[c * 16 + m] = values 32 c .. 32 c + 31 of token m.
+struct qw_afrag_lds_sums : qw_afrag_lds {
+    const float *xs;
+    static constexpr bool sums = true;
+    __device__ __forceinline__ float sum(uint32_t c) const { return xs[c * 16 + m]; }
 };
 
 // Two planes (hi + lo) staged the same way.
@@ -331,6 +339,16 @@ struct qw_afrag_gather {
             for (int i = 0; i < 4; i++) {
                 hi[i] = *(const h8 *)(rowhi + koff + i * kstep);
                 lo[i] = *(const h8 *)(rowlo + koff + i * kstep);
+            }
+        }
+    }
+    // Four values at koff, koff + 16, ... koff + 112 (koff a multiple of 4), two to a register group
+    __device__ __forceinline__ void fetch_quads(uint32_t koff) const {
+        if (on) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                hi[i] = qw_join4(*(const h4 *)(rowhi + koff + 32 * i), *(const h4 *)(rowhi + koff + 32 * i + 16));
+                lo[i] = qw_join4(*(const h4 *)(rowlo + koff + 32 * i), *(const h4 *)(rowlo + koff + 32 * i + 16));
             }
         }
     }
@@ -714,6 +732,57 @@ template <int NB> struct qw_chunk<8, NB> {
             if (AF::has_lo) sub = qw_mfma(af.lo(kb), w, sub);
             acc += qw_h2f(d[b]) * sub;
         }
+    }
+};
+
+// The same rows from their tile-major copy (QW_F_PACKED_Q8 in qw_kargs.h): NB groups of eight blocks, five coalesced loads each
+// in matrix-core lane order, nothing moved between lanes. The arithmetic, block by block, is that of the GGUF rows.
+template <int NB> struct qw_chunk<QW_F_PACKED_Q8, NB> {
+    static constexpr uint32_t BLK_K = 256, BLK_B = QW_Q8_SLAB_BYTES;
+    static constexpr int DEPTH = 2;
+    u4 q[NB][4], d[NB];
+    __device__ __forceinline__ void load(const uint8_t *p, uint32_t lane) {
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const uint8_t *sl = p + QW_Q8_SLAB_BYTES * b;
+#pragma unroll
+            for (int pl = 0; pl < 4; pl++) q[b][pl] = *(const u4 *)(sl + 1024 * pl + 16 * lane);
+            d[b] = *(const u4 *)(sl + 4096 + 16 * (lane & 15));
+        }
+    }
+    __device__ __forceinline__ void transpose() {}
+    __device__ __forceinline__ h8 weights(int b, int i) const { return qw_q8_cvt(i & 1 ? u2{q[b][i >> 1][2], q[b][i >> 1][3]} : u2{q[b][i >> 1][0], q[b][i >> 1][1]}); }
+    __device__ __forceinline__ float scale(int b, int i) const { return qw_h2f((uint16_t)(d[b][i >> 1] >> (16 * (i & 1)))); }
+    template <class AF> __device__ __forceinline__ void mac(const u2 *, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const {
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const h8 w = weights(b, i);
+                const uint32_t kb = k0 + 256 * b + 32 * i + 8 * kg;
+                f4 sub = {0, 0, 0, 0};
+                sub = qw_mfma(af.hi(kb), w, sub);
+                if (AF::has_lo) sub = qw_mfma(af.lo(kb), w, sub);
+                acc += scale(b, i) * sub;
+            }
+    }
+    template <class AF> __device__ __forceinline__ void mac_lean(const u2 *lut, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const { mac(lut, af, k0, kg, acc); }
+    template <class AF> __device__ __forceinline__ void mac_half(const u2 *lut, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const { mac(lut, af, k0, kg, acc); }
+    template <class AF> __device__ __forceinline__ void mac_gather(const u2 *, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const {
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int i4 = 0; i4 < 8; i4 += 4) {
+                af.fetch4(k0 + 256 * b + 32 * i4 + 8 * kg, 32);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const h8 w = weights(b, i4 + i);
+                    f4 sub = {0, 0, 0, 0};
+                    sub = qw_mfma(af.hi[i], w, sub);
+                    sub = qw_mfma(af.lo[i], w, sub);
+                    acc += scale(b, i4 + i) * sub;
+                }
+            }
     }
 };
 

@@ -220,7 +220,7 @@ typedef struct { /* read-pattern ceiling of a decode layer (the reference's kern
  * instructions left out - the loaded registers are merely folded into the result, which is therefore meaningless. Times
  * what the gate/up launch costs without its arithmetic (same selection, table and activation staging, loads, stores). */
 #define QW_F_ABLATE 122
-/* Tile-major copy of IQ4_NL rows (format code QW_F_PACKED_NL; qwk_pack_args with split = QW_F_PACKED_NL, nblk = chunks
+/* Tile-major copy of IQ4_NL rows (format code QW_F_PACKED_NL; nblk = chunks
  * of ten blocks per row, so the row length is a multiple of 320): every (tile of 16 rows, chunk) becomes
  * QW_NL_CHUNK_BYTES = 16 x 180 contiguous bytes in the lane order of the matrix instruction (lane = row & 15 | k-group
  * << 4; a lane owns bytes 4 kg .. 4 kg + 3 of qs of every block of its row, its eight nibbles in the order in which they are
@@ -232,18 +232,30 @@ typedef struct { /* read-pattern ceiling of a decode layer (the reference's kern
 /* Template argument of the kernels whose routed format is chosen when they run (qwk_gu_rt*: qwk_gu_args.fgu): not a format. */
 #define QW_F_RT 99
 #define QW_NL_CHUNK_BYTES 2880u
-/* Tile-major copy of Q6_K rows (format code QW_F_PACKED_Q6; qwk_pack_args with split = QW_F_PACKED_Q6, nblk = blocks a
+/* Tile-major copy of Q6_K rows (format code QW_F_PACKED_Q6; nblk = blocks a
  * row): per (tile of 16 rows, block of 256 values) QW_Q6_SLAB_BYTES = 16 x 210 contiguous bytes in the lane order of the
  * matrix instruction (lane = row & 15 | k-group << 4): [0, 3072) three planes of 16 bytes a lane holding the twelve
  * dwords of ql and qh that the lane decodes (the r[0..11] of the Q6_K decoder), [3072, 3328) the sixteen int8 scales of
  * every row (16 bytes a row, read by the row's four lanes), [3328, 3360) d of every row. Exactly the matrix's bytes. */
 #define QW_F_PACKED_Q6 114
 #define QW_Q6_SLAB_BYTES 3360u
+/* Tile-major copy of Q8_0 rows (QW_F_PACKED_Q8; nblk = groups of eight blocks a row, so the row length is a multiple of 256): per
+ * (tile of 16 rows, 256 values) QW_Q8_SLAB_BYTES = 16 x 8 x 34 contiguous bytes: [0, 4096) four planes of 16 bytes a lane, plane p
+ * the lane's eight bytes q[8 kg .. 8 kg + 8) of blocks 2 p and 2 p + 1; [4096, 4352) the eight d of every row, 16 bytes a row. */
+#define QW_F_PACKED_Q8 108
+#define QW_Q8_SLAB_BYTES 4352u
+/* Tile-major copy of Q4_K rows (QW_F_PACKED_Q4K): per (tile of 16 rows, block of 256 values) QW_Q4K_SLAB_BYTES = 16 x 144
+ * contiguous bytes: [0, 2048) two planes of 16 bytes a lane, dword s of the eight holding the lane's eight nibbles of
+ * sub-block s (values 32 s + 8 kg .. + 8, nibble 4 (i >> 1) + 16 (i & 1) bits up for value i, so that one mask takes a pair of
+ * binary16 significands out); [2048, 2304) the first 16 bytes of every row's block (d, dmin, the packed scales). */
+#define QW_F_PACKED_Q4K 112
+#define QW_Q4K_SLAB_BYTES 2304u
 typedef struct {
     const uint8_t *A, *B;
     uint8_t *dst;
     uint64_t ntiles;
-    uint32_t nblk, rowbytes, split, pad;
+    uint32_t nblk, rowbytes;
+    uint32_t split, pad; /* rows of a tile that come from A (the others from B): 16 or 8 */
 } qwk_pack_args;
 
 /* Ragged packing of (token, expert) pairs and the grouped product over the packed rows (kernels/moe_prefill.metal,

@@ -73,6 +73,8 @@ __device__ __forceinline__ uint32_t qw_wave() { return (uint32_t)__builtin_amdgc
 __device__ __forceinline__ uint32_t qw_lane() { return threadIdx.x & 63; }
 #include "qw_grouped.hip.h"
 #include "qw_small.hip.h"
+constexpr bool qw_tiled(int f) { return f == QW_F_PACKED || f == QW_F_ABLATE || f == QW_F_PACKED_NL || f == QW_F_PACKED_Q8 || f == QW_F_PACKED_Q4K || f == QW_F_PACKED_Q6; } // weights come from a tile-major copy
+constexpr bool qw_wants_sums(int f) { return f == QW_F_PACKED_Q4K; } // decoders that read the sums of 32 activations beside them
 constexpr bool qw_has_lut(int f) { return f == 21 || f == QW_F_PACKED || f == QW_F_ABLATE; } // formats decoded through the LDS table (the ablation copies it too)
 __device__ __forceinline__ uint32_t qw_all_tokens(uint32_t nbr) { return nbr >= 32 ? 0xffffffffu : (1u << nbr) - 1; }
 
@@ -154,6 +156,9 @@ extern "C" __global__ void qwk_tab_init(qwk_tab_args a) {
 
 // ================================================================ packing of IQ3_S rows (layout: qwk_pack_args)
 // One thread per (slab, lane), grid-stride over the slabs; run once per weight matrix, at its first use.
+__device__ __forceinline__ const uint8_t *pack_row(const qwk_pack_args &a, uint64_t tile, uint32_t n) { // row n of a tile
+    return n < a.split ? a.A + (tile * a.split + n) * a.rowbytes : a.B + (tile * (16 - a.split) + (n - a.split)) * a.rowbytes;
+}
 #if QW_IN_PART(0)
 extern "C" __global__ __launch_bounds__(256) void qwk_pack_iq3(qwk_pack_args a) {
     const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (blockDim.x >> 6);
@@ -161,8 +166,7 @@ extern "C" __global__ __launch_bounds__(256) void qwk_pack_iq3(qwk_pack_args a) 
     for (uint64_t sl = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
         const uint64_t tile = sl / a.nblk;
         const uint32_t blk = (uint32_t)(sl % a.nblk);
-        const uint8_t *row = n < a.split ? a.A + (tile * a.split + n) * a.rowbytes : a.B + (tile * (16 - a.split) + (n - a.split)) * a.rowbytes;
-        const uint8_t *src = row + 110 * blk;
+        const uint8_t *src = pack_row(a, tile, n) + 110 * blk;
         uint8_t *dst = a.dst + sl * QW_SLAB_BYTES;
         *(u4 *)(dst + 16 * lane) = *(const u4a2 *)(src + 2 + 16 * kg);
         *(u2 *)(dst + 1024 + 8 * lane) = *(const u2a2 *)(src + 74 + 8 * kg);
@@ -180,7 +184,7 @@ extern "C" __global__ __launch_bounds__(256) void qwk_pack_q6(qwk_pack_args a) {
     const uint32_t lane = threadIdx.x & 63, n = lane & 15, kg = lane >> 4;
     for (uint64_t sl = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
         const uint64_t tile = sl / a.nblk;
-        const uint8_t *src = a.A + (tile * 16 + n) * a.rowbytes + 210 * (sl % a.nblk);
+        const uint8_t *src = pack_row(a, tile, n) + 210 * (sl % a.nblk);
         uint8_t *dst = a.dst + sl * QW_Q6_SLAB_BYTES;
         uint32_t r[12];
 #pragma unroll
@@ -191,6 +195,45 @@ extern "C" __global__ __launch_bounds__(256) void qwk_pack_q6(qwk_pack_args a) {
         for (int pl = 0; pl < 3; pl++) *(u4 *)(dst + 1024 * pl + 16 * lane) = u4{r[4 * pl], r[4 * pl + 1], r[4 * pl + 2], r[4 * pl + 3]};
         *(uint32_t *)(dst + 3072 + 16 * n + 4 * kg) = *(const u1a2 *)(src + 192 + 4 * kg); // the row's four lanes write its sixteen scales
         if (kg == 0) *(uint16_t *)(dst + 3328 + 2 * n) = *(const uint16_t *)(src + 208);
+    }
+}
+#endif
+
+// The tile-major copies of Q8_0 and Q4_K rows (layouts: QW_F_PACKED_Q8, QW_F_PACKED_Q4K in qw_kargs.h); a wave per (tile, 256 values).
+#if QW_IN_PART(0)
+extern "C" __global__ __launch_bounds__(256) void qwk_pack_q8(qwk_pack_args a) {
+    const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (blockDim.x >> 6);
+    const uint32_t lane = threadIdx.x & 63, n = lane & 15, kg = lane >> 4;
+    for (uint64_t sl = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
+        const uint8_t *src = pack_row(a, sl / a.nblk, n) + 272 * (sl % a.nblk);
+        uint8_t *dst = a.dst + sl * QW_Q8_SLAB_BYTES;
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const u2 q0 = *(const u2a2 *)(src + 68 * p + 2 + 8 * kg), q1 = *(const u2a2 *)(src + 68 * p + 36 + 8 * kg);
+            *(u4 *)(dst + 1024 * p + 16 * lane) = u4{q0.x, q0.y, q1.x, q1.y};
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) *(uint16_t *)(dst + 4096 + 16 * n + 4 * kg + 2 * i) = *(const uint16_t *)(src + 34 * (2 * kg + i));
+    }
+}
+extern "C" __global__ __launch_bounds__(256) void qwk_pack_q4k(qwk_pack_args a) {
+    const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (blockDim.x >> 6);
+    const uint32_t lane = threadIdx.x & 63, n = lane & 15, kg = lane >> 4;
+    for (uint64_t sl = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
+        const uint8_t *src = pack_row(a, sl / a.nblk, n) + 144 * (sl % a.nblk);
+        uint8_t *dst = a.dst + sl * QW_Q4K_SLAB_BYTES;
+        uint32_t r[8];
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const u2 q = *(const u2a2 *)(src + 16 + 32 * (s >> 1) + 8 * kg);
+            uint32_t d = 0;
+#pragma unroll
+            for (int i = 0; i < 8; i++) d |= (((i < 4 ? q.x : q.y) >> (8 * (i & 3) + 4 * (s & 1))) & 15) << (4 * (i >> 1) + 16 * (i & 1));
+            r[s] = d;
+        }
+        *(u4 *)(dst + 16 * lane) = u4{r[0], r[1], r[2], r[3]};
+        *(u4 *)(dst + 1024 + 16 * lane) = u4{r[4], r[5], r[6], r[7]};
+        *(uint32_t *)(dst + 2048 + 16 * n + 4 * kg) = *(const u1a2 *)(src + 4 * kg);
     }
 }
 #endif
@@ -1067,6 +1110,20 @@ __device__ __forceinline__ void qw_sel_load(qw_sel_cache &c, const uint8_t *sel,
     if (threadIdx.x == 0) c.U = *(const uint32_t *)sel;
 }
 
+// The sums of 32 activations of every token from their fragments in LDS, in index order (all threads; a barrier before and after).
+__device__ __forceinline__ void qw_sum32(const u4 *xf, float *xs, uint32_t K) {
+    for (uint32_t i = threadIdx.x; i < (K >> 5) * 16; i += blockDim.x) {
+        const uint32_t c = i >> 4, m = i & 15;
+        float sum = 0;
+#pragma unroll
+        for (uint32_t f = 0; f < 4; f++) {
+            const h8 v = __builtin_bit_cast(h8, xf[(4 * c + f) * 16 + m]);
+#pragma unroll
+            for (int e = 0; e < 8; e++) sum += (float)v[e];
+        }
+        xs[i] = sum;
+    }
+}
 // Where the SwiGLU values of a tile go. The plain form: the two planes of H in global memory, for a later launch.
 struct qw_h_global {
     uint16_t *H;
@@ -1085,16 +1142,28 @@ struct qw_h_global {
 // the caller has set to the number of waves before a barrier (wave w starts with the w-th of them); else wave w0 of nw takes
 // tiles w0, w0 + nw, ...
 template <int F, int CH, bool QUEUE, class S, class HS>
-__device__ __forceinline__ void gu_tasks(const qwk_gu_args &a, const u2 *lut, const u4 *xf, qw_sel_cache *sc, uint32_t w0, uint32_t nw, S ready, HS &hs) {
+__device__ __forceinline__ void gu_tasks(const qwk_gu_args &a, const u2 *lut, const u4 *xf, float *xs, qw_sel_cache *sc, uint32_t w0, uint32_t nw, S ready0, HS &hs) {
     typedef qw_chunk<F, CH> C;
     const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, K = a.topk, gnb = a.gnb;
     const uint32_t U = a.shared ? 1 : sc->U, tpe = a.I / 8, ntasks = U * tpe;
     const uint32_t cpr = a.D / (C::BLK_K * CH);
-    const qw_afrag_lds af = {xf, n};
+    typename std::conditional<qw_wants_sums(F), qw_afrag_lds_sums, qw_afrag_lds>::type af;
+    af.xf = xf, af.m = n;
+    if constexpr (qw_wants_sums(F)) af.xs = xs;
+    bool summed = false;
+    auto ready = [&] { // once per wave, behind its first weight loads
+        ready0();
+        if constexpr (qw_wants_sums(F)) {
+            if (summed) return;
+            summed = true;
+            qw_sum32(xf, xs, a.D);
+            __syncthreads();
+        }
+    };
     const uint32_t nl = lane >> 2; // (row, k-group) this lane loads from GGUF rows: (lane >> 2, lane & 3)
     auto rowp = [&](uint32_t task) {
         const uint32_t u = task / tpe, e = a.shared ? 0 : (uint32_t)__builtin_amdgcn_readfirstlane((int)sc->ue[u]); // (wave-uniform: the row base stays in scalar registers)
-        if constexpr (F == QW_F_PACKED || F == QW_F_ABLATE) return a.Wg + ((size_t)e * tpe + task % tpe) * a.rowbytes; // the tile's slabs; rowbytes = bytes of a tile
+        if constexpr (qw_tiled(F)) return a.Wg + ((size_t)e * tpe + task % tpe) * a.rowbytes; // the tile's slabs; rowbytes = bytes of a tile
         else return (nl < 8 ? a.Wg : a.Wu) + ((size_t)e * a.I + 8 * (task % tpe) + (nl & 7)) * a.rowbytes;
     };
     f4 acc = {0, 0, 0, 0};
@@ -1118,8 +1187,8 @@ __device__ __forceinline__ void gu_tasks(const qwk_gu_args &a, const u2 *lut, co
         }
         acc = f4{0, 0, 0, 0};
     };
-    const uint32_t kl = F == QW_F_PACKED || F == QW_F_ABLATE ? lane : lane & 3;
-    const uint8_t *spare = qw_has_lut(F) ? (const uint8_t *)a.glut : nullptr;
+    const uint32_t kl = qw_tiled(F) ? lane : lane & 3;
+    const uint8_t *spare = qw_has_lut(F) || qw_tiled(F) ? (const uint8_t *)a.glut : nullptr;
     if constexpr (QUEUE) {
         auto next = [&]() -> uint32_t {
             uint32_t j = 0;
@@ -1140,7 +1209,7 @@ __device__ __forceinline__ void gu_tasks(const qwk_gu_args &a, const u2 *lut, co
 // weights in ss->w, not only the one that writes the record. selected(): called by every thread once the selection
 // cache *sc (and ss->w) is complete and published, before any tile is taken; ss may be reused after a barrier of its own.
 template <int FGU, int CHGU, int FSG, int CHSG, class HS, class SEL>
-__device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, qw_sel_cache *sc, qw_sel_scratch *ss, HS &hs, bool all_w, SEL selected) {
+__device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, float *xs, qw_sel_cache *sc, qw_sel_scratch *ss, HS &hs, bool all_w, SEL selected) {
     bool staged = false, tabled = false;
     if (threadIdx.x == 0) sc->qnext = blockDim.x >> 6; // (nothing below writes it; a barrier follows on every path)
     if (threadIdx.x == 0) QW_WSTAMP(12);
@@ -1201,21 +1270,21 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, q
             sa.Wu = a.Wsu;
             sa.rowbytes = a.sg_rowbytes;
             sa.shared = 1;
-            gu_tasks<FSG == 0 ? 8 : FSG, CHSG, false>(sa, lut, xf, nullptr, w0, nw, ready, hs);
+            gu_tasks<FSG == 0 ? 8 : FSG, CHSG, false>(sa, lut, xf, xs, nullptr, w0, nw, ready, hs);
         }
     }
     // the routed tiles: from the workgroup's queue (a wave that did a shared tile simply takes its next one later)
     if constexpr (FGU == QW_F_RT) { // the other GGUF types, one block a chunk; their byte table lies behind the IQ3_S table
         const u2 *tab = lut + (qw_has_lut(FSG) ? QW_LUT_ENTRIES : 0);
         switch (a.fgu) {
-        case 12: gu_tasks<12, 1, true>(a, tab, xf, sc, 0, 0, ready, hs); break;
-        case 13: gu_tasks<13, 1, true>(a, tab, xf, sc, 0, 0, ready, hs); break;
-        case 14: gu_tasks<14, 1, true>(a, tab, xf, sc, 0, 0, ready, hs); break;
-        case 20: gu_tasks<20, 8, true>(a, tab, xf, sc, 0, 0, ready, hs); break;
-        case 23: gu_tasks<23, 1, true>(a, tab, xf, sc, 0, 0, ready, hs); break;
+        case 12: gu_tasks<12, 1, true>(a, tab, xf, xs, sc, 0, 0, ready, hs); break;
+        case 13: gu_tasks<13, 1, true>(a, tab, xf, xs, sc, 0, 0, ready, hs); break;
+        case 14: gu_tasks<14, 1, true>(a, tab, xf, xs, sc, 0, 0, ready, hs); break;
+        case 20: gu_tasks<20, 8, true>(a, tab, xf, xs, sc, 0, 0, ready, hs); break;
+        case 23: gu_tasks<23, 1, true>(a, tab, xf, xs, sc, 0, 0, ready, hs); break;
         default: break; // (the host launches this kernel for these five only)
         }
-    } else gu_tasks<FGU, CHGU, true>(a, lut, xf, sc, 0, 0, ready, hs);
+    } else gu_tasks<FGU, CHGU, true>(a, lut, xf, xs, sc, 0, 0, ready, hs);
     QW_WSTAMP(qw_wave());
     QW_DSTAMP(2);
 }
@@ -1223,7 +1292,8 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, q
     extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_gu_args a) {                             \
         __shared__ struct { u2 lut[((qw_has_lut(FGU) || qw_has_lut(FSG)) ? QW_LUT_ENTRIES : 0) + (FGU == QW_F_RT ? QW_KQ_TAB / 2 : 1)]; u4 xf[QW_XF_MAXK * 2]; qw_sel_cache sc; qw_sel_scratch ss; } L; \
         qw_h_global hs = {a.H, a.hplane};                                                                      \
-        gu_body<FGU, CHGU, FSG, CHSG>(a, L.lut, L.xf, &L.sc, &L.ss, hs, false, [] {});                           \
+        static_assert(sizeof(qw_sel_scratch) >= QW_XF_MAXK / 2 * sizeof(float), "the sums of 32 activations take the place of the selection's scratch"); \
+        gu_body<FGU, CHGU, FSG, CHSG>(a, L.lut, L.xf, (float *)&L.ss, &L.sc, &L.ss, hs, false, [] {});                           \
         QW_WG_END_STAMP(10);                                                                                    \
         QW_SST_FLUSH();                                                                                         \
     }
@@ -1241,6 +1311,12 @@ QW_GU(8, 1, 8, 1, qwk_gu_f8_c1_s8_c1) QW_GU(8, 1, 21, 1, qwk_gu_f8_c1_s21_c1)
 QW_GU(121, 2, 0, 1, qwk_gu_f121_c2) QW_GU(121, 2, 121, 2, qwk_gu_f121_c2_s121_c2) QW_GU(121, 2, 8, 16, qwk_gu_f121_c2_s8_c16)
 QW_GU(QW_F_ABLATE, 2, 0, 1, qwk_gu_f122_c2) // measurement: the launch above without its arithmetic
 QW_GU(121, 1, 0, 1, qwk_gu_f121_c1) QW_GU(121, 1, 121, 1, qwk_gu_f121_c1_s121_c1) QW_GU(121, 1, 8, 1, qwk_gu_f121_c1_s8_c1)
+#endif
+// tile-major Q8_0 and Q4_K rows, D a multiple of 512; their shared expert is in the front launch. Measured (512 experts of 2048 x
+// 512, us a launch, GGUF rows -> these): Q8_0 14.3 -> 11.0 at one token, 32.9 -> 22.2 at four, 88.7 -> 63.2 at sixteen (310 MB: 4.9
+// TB/s); Q4_K (in qwk_gu_rt, with the arithmetic before qw_k45_steps) 21.5 -> 18.3 at four, 50.1 -> 40.5 at sixteen (164 MB).
+#if QW_IN_PART(1)
+QW_GU(108, 2, 0, 1, qwk_gu_f108_c2) QW_GU(112, 2, 0, 1, qwk_gu_f112_c2)
 #endif
 // routed rows of the other GGUF types (Q4_K, Q5_K, Q6_K, IQ4_NL, IQ4_XS: kernels/moe_gg.metal:336-395), the type an argument
 #if QW_IN_PART(1)
@@ -1469,7 +1545,6 @@ template <int F, int CH> __device__ __forceinline__ void shared_down_tiles(const
 // that picked them) are copied into LDS once, in fragment order, and the waves then stream the range's tiles with operand A read
 // from LDS. The first weight loads are issued before the table copy, the row copy and the barrier.
 constexpr bool qw_has_tab(int F) { return F == 20 || F == 23 || F == QW_F_PACKED_NL; } // decoders that read the byte table of qw_kq_tab_build
-constexpr bool qw_tiled(int F) { return F == QW_F_PACKED || F == QW_F_PACKED_NL; } // weights come from a tile-major copy
 struct qw_dn_seg { // one expert's part of a workgroup's range (all fields wave-uniform)
     const uint8_t *W;  // the expert's matrix
     float *P;          // Pg or Psh
@@ -1759,6 +1834,8 @@ __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *p
 #if QW_IN_PART(4)
 QW_DNC(121, 2, 0, 1, qwk_dnc_f121_c2) QW_DNC(121, 2, 121, 2, qwk_dnc_f121_c2_s121_c2) QW_DNC(121, 2, 8, 4, qwk_dnc_f121_c2_s8_c4)
 QW_DNC(121, 1, 0, 1, qwk_dnc_f121_c1) QW_DNC(121, 1, 121, 1, qwk_dnc_f121_c1_s121_c1) QW_DNC(121, 1, 8, 4, qwk_dnc_f121_c1_s8_c4)
+QW_DNC(108, 1, 0, 1, qwk_dnc_f108_c1) QW_DNC(108, 1, 108, 1, qwk_dnc_f108_c1_s108_c1)
+QW_DNC(114, 1, 0, 1, qwk_dnc_f114_c1) QW_DNC(114, 1, 114, 1, qwk_dnc_f114_c1_s114_c1) QW_DNC(114, 1, 8, 4, qwk_dnc_f114_c1_s8_c4)
 QW_DNC(8, 4, 0, 1, qwk_dnc_f8_c4) QW_DNC(8, 4, 8, 4, qwk_dnc_f8_c4_s8_c4)
 QW_DNC(120, 10, 0, 10, qwk_dnc_f120_c10) QW_DNC(120, 10, 120, 10, qwk_dnc_f120_c10_s120_c10) QW_DNC(120, 10, 8, 4, qwk_dnc_f120_c10_s8_c4) // tile-major IQ4_NL rows of 640
 #define QW_DNC_KQ(F) QW_DNC(F, 1, 0, 1, qwk_dnc_f##F##_c1) QW_DNC(F, 1, F, 1, qwk_dnc_f##F##_c1_s##F##_c1) QW_DNC(F, 1, 8, 4, qwk_dnc_f##F##_c1_s8_c4)
@@ -1800,6 +1877,16 @@ template <uint32_t ROWS> struct qw_afrag_rows {
             for (int i = 0; i < 4; i++) {
                 hi[i] = __builtin_bit_cast(h8, hi_[((koff + i * kstep) >> 3) * ROWS]);
                 lo[i] = __builtin_bit_cast(h8, lo_[((koff + i * kstep) >> 3) * ROWS]);
+            }
+        }
+    }
+    __device__ __forceinline__ void fetch_quads(uint32_t koff) const { // (as qw_afrag_gather)
+        if (on) {
+            const uint32_t at = (koff >> 3) * ROWS * 16 + (koff & 4) * 2;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                hi[i] = qw_join4(__builtin_bit_cast(h4, qw_half_read(hi_, at + 4 * i * ROWS * 16)), __builtin_bit_cast(h4, qw_half_read(hi_, at + (4 * i + 2) * ROWS * 16)));
+                lo[i] = qw_join4(__builtin_bit_cast(h4, qw_half_read(lo_, at + 4 * i * ROWS * 16)), __builtin_bit_cast(h4, qw_half_read(lo_, at + (4 * i + 2) * ROWS * 16)));
             }
         }
     }
@@ -1886,7 +1973,7 @@ __device__ __forceinline__ void dnq_run(const qwk_dn_args &a, const u2 *lut, con
             }
             acc = f4{0, 0, 0, 0};
         },
-        ready, qw_has_lut(F) ? (const uint8_t *)a.glut : nullptr);
+        ready, qw_has_lut(F) || qw_tiled(F) ? (const uint8_t *)a.glut : nullptr);
 }
 template <int F, int CH, int FSD, int CHSD>
 __device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_lds &L) {
@@ -2009,11 +2096,14 @@ __device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_l
 }
 #define QW_DNQ(F, CH, FSD, CHSD, NAME)                                                              \
     extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) {                    \
-        __shared__ struct { u2 lut[QW_LUT_ENTRIES]; qw_dnq_lds d; } L;                               \
+        __shared__ struct { u2 lut[qw_has_lut(F) || qw_has_lut(FSD) ? QW_LUT_ENTRIES : 1]; qw_dnq_lds d; } L; \
         dnq_body<F, CH, FSD, CHSD>(a, L.lut, L.d);                                                  \
     }
 #if QW_IN_PART(4)
 QW_DNQ(121, 2, 0, 1, qwk_dnq_f121_c2) QW_DNQ(121, 2, 121, 2, qwk_dnq_f121_c2_s121_c2) QW_DNQ(121, 2, 8, 4, qwk_dnq_f121_c2_s8_c4)
+// tile-major Q8_0 and Q6_K rows
+QW_DNQ(108, 1, 0, 1, qwk_dnq_f108_c1) QW_DNQ(108, 1, 108, 1, qwk_dnq_f108_c1_s108_c1)
+QW_DNQ(114, 1, 0, 1, qwk_dnq_f114_c1) QW_DNQ(114, 1, 114, 1, qwk_dnq_f114_c1_s114_c1) QW_DNQ(114, 1, 8, 4, qwk_dnq_f114_c1_s8_c4)
 QW_DNQ(121, 1, 0, 1, qwk_dnq_f121_c1) QW_DNQ(121, 1, 121, 1, qwk_dnq_f121_c1_s121_c1) QW_DNQ(121, 1, 8, 4, qwk_dnq_f121_c1_s8_c4)
 #endif
 
@@ -2085,7 +2175,7 @@ template <int FSD, int CHSD> __device__ __forceinline__ void gud_body(const qwk_
     if (nt > QW_GUD_SHARE) nt = QW_GUD_SHARE; // (the host keeps the shares that small)
     uint32_t nv = 0;
     qw_h_lds hs = {&L.hcount, L.u.hb.off, L.u.hb.val, a.H, a.hplane, 0};
-    gu_body<F, CH, 0, 1>(a, L.lut, L.big.xf, &L.sc, &L.u.ss, hs, true, [&] {
+    gu_body<F, CH, 0, 1>(a, L.lut, L.big.xf, nullptr, &L.sc, &L.u.ss, hs, true, [&] {
         // the down phase's lists, made while everything they come from is in LDS: gating weights of the share's tokens,
         // experts, masks, the share's slot bytes, and the unique experts its tokens picked in record order (every wave
         // makes the whole list: all write the same values)

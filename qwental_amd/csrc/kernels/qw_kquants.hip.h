@@ -68,6 +68,17 @@ template <int J> __device__ __forceinline__ void qw_k4_scale_min(const uint32_t 
 
 template <int F> struct qw_kq;
 
+// All eight scales and minima of those 12 bytes (s[0 .. 2]), four bytes a dword.
+__device__ __forceinline__ void qw_k4_scales(const uint32_t *s, uint32_t (&sc)[2], uint32_t (&mn)[2]) {
+    sc[0] = s[0] & 0x3f3f3f3fu, sc[1] = (s[2] & 0x0f0f0f0fu) | ((s[0] >> 2) & 0x30303030u);
+    mn[0] = s[1] & 0x3f3f3f3fu, mn[1] = ((s[2] >> 4) & 0x0f0f0f0fu) | ((s[1] >> 2) & 0x30303030u);
+}
+// Byte J of a dword (< 1024 as an integer) as binary16 in both halves.
+template <int J> __device__ __forceinline__ h2 qw_byte_h2(uint32_t v) {
+    const h2 bias = {(_Float16)1024.0f, (_Float16)1024.0f};
+    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, v, 0x04000400u | J | J << 16)) - bias;
+}
+
 // ---------------------------------------------------------------- Q4_K: 144 bytes, d @0, dmin @2, scales[12] @4, qs[128] @16
 // Step S = sub-block S (32 values): lane group kg supplies values 32 S + 8 kg .. + 8 = the low (S even) or high
 // (S odd) nibbles of qs[32 (S / 2) + 8 kg .. + 8].
@@ -344,7 +355,7 @@ template <int NB> struct qw_chunk<20, NB> {
             d[b] = (uint16_t)qw_pull(d[b], src4);
         }
     }
-    static __device__ __forceinline__ h8 join(h4 a, h4 b) { return h8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
+    static __device__ __forceinline__ h8 join(h4 a, h4 b) { return qw_join4(a, b); }
     template <class AF> __device__ __forceinline__ void mac(const u2 *lut, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const {
 #pragma unroll
         for (int b = 0; b < NB; b++) {
@@ -549,6 +560,89 @@ template <int F, int NB> struct qw_chunk_kqa : qw_chunk_kq<F, NB> {
     template <class AF> __device__ __forceinline__ void mac_gather(const u2 *lut, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const {
         const qw_afrag_glb<true> g = {af.on ? af.rowhi : nullptr, af.on ? af.rowlo : nullptr};
         mac(lut, g, k0, kg, acc);
+    }
+};
+// Q6_K from the tile-major copy: the loads of qw_chunk_kq<QW_F_PACKED_Q6>, the arithmetic of qw_kq<14>.
+template <int NB> struct qw_chunk<QW_F_PACKED_Q6, NB> : qw_chunk_kq<QW_F_PACKED_Q6, NB> {
+    template <class AF> __device__ __forceinline__ void mac(const u2 *lut, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const {
+#pragma unroll
+        for (int i = 0; i < NB; i++) qw_kq_block_af<14>(this->b[i], (const uint32_t *)lut, af, k0 + 256 * i, kg, acc);
+    }
+    template <class AF> __device__ __forceinline__ void mac_lean(const u2 *lut, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const { mac(lut, af, k0, kg, acc); }
+    template <class AF> __device__ __forceinline__ void mac_half(const u2 *lut, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const { mac(lut, af, k0, kg, acc); }
+    // step G of a block with its operand A in registers: quads G & 7 of a fetch
+    template <int G, class AF> __device__ __forceinline__ void gather_steps(const qw_kq<14> &b, const AF &af, uint32_t kb, uint32_t kg, f4 &acc) const {
+        if constexpr (G < 16) {
+            if constexpr (G % 8 == 0) af.fetch_quads(kb + 16 * G + 4 * kg);
+            h4 w;
+            float a, c;
+            b.template dec<G>(nullptr, kg, w, a, c);
+            constexpr int r = (G & 7) >> 1, e = 4 * (G & 1);
+            f4 sub = {0, 0, 0, 0};
+            sub = qw_mfma16(h4{af.hi[r][e], af.hi[r][e + 1], af.hi[r][e + 2], af.hi[r][e + 3]}, w, sub);
+            sub = qw_mfma16(h4{af.lo[r][e], af.lo[r][e + 1], af.lo[r][e + 2], af.lo[r][e + 3]}, w, sub);
+            acc += a * sub;
+            gather_steps<G + 1>(b, af, kb, kg, acc);
+        }
+    }
+    template <class AF> __device__ __forceinline__ void mac_gather(const u2 *, const AF &af, uint32_t k0, uint32_t kg, f4 &acc) const {
+#pragma unroll
+        for (int i = 0; i < NB; i++) gather_steps<0>(this->b[i], af, k0 + 256 * i, kg, acc);
+    }
+};
+// Q4_K from the tile-major copy (QW_F_PACKED_Q4K in qw_kargs.h), three coalesced loads a block, for gate / up rows (an operand A with
+// the sums of 32 activations beside it: qw_afrag_lds_sums). A weight is d sc q - dmin m; written as d (q - 8) sc + (8 d sc - dmin m), its
+// first part has small integers, |(q - 8) sc| <= 504, exact in binary16 and made from the nibble by one mask (16 + q: the
+// nibble under the exponent of 16) and one fused multiply-add, (16 + q) sc - 24 sc; the eight steps of a block share an accumulator,
+// which d multiplies once. The second part is constant over a sub-block: two binary32 matrix instructions a block add its products
+// with the 32 activations' sums, four sub-blocks each, a lane bringing one sub-block's constant and one token's sum.
+// Against scale and minimum applied to each step's binary32 result (twelve vector instructions a step, and one more matrix instruction
+// for the sums): SwiGLU values 1.7e-7 to 2.8e-7 from float64 (512 to 2560 values, 1 to 16 tokens) where those are 1.9e-7 to 3.6e-7 (2-norm);
+// with q instead of q - 8 a dense product was 1.3e-7 off instead of 1.0e-7. Times: at qwk_gu_f112_c2.
+struct qw_q4_blk {
+    uint32_t h[4], q[8]; // d, dmin and the packed scales; q[S]: the lane's eight nibbles of sub-block S
+    template <int S> __device__ __forceinline__ void steps(const qw_afrag_lds_sums &af, uint32_t kb, uint32_t kg, const uint32_t (&sc)[2], f4 &sub) const {
+        if constexpr (S < 8) {
+            const h2 f = qw_byte_h2<(S & 3)>(sc[S >> 2]), m24 = {(_Float16)-24.0f, (_Float16)-24.0f}, z = f * m24;
+            const uint32_t v = q[S];
+            u4 w = {v << 6, v << 2, v >> 2, v >> 6};
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, (uint32_t)((w[i] & 0x03c003c0u) | 0x4c004c00u)), f, z));
+            sub = qw_mfma(af.hi(kb + 32 * S + 8 * kg), __builtin_bit_cast(h8, w), sub);
+            steps<S + 1>(af, kb, kg, sc, sub);
+        }
+    }
+};
+template <int NB> struct qw_chunk<QW_F_PACKED_Q4K, NB> {
+    static constexpr uint32_t BLK_K = 256, BLK_B = QW_Q4K_SLAB_BYTES;
+    static constexpr int DEPTH = 2;
+    qw_q4_blk b[NB];
+    __device__ __forceinline__ void load(const uint8_t *p, uint32_t lane) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const uint8_t *sl = p + QW_Q4K_SLAB_BYTES * i;
+            const u4 q0 = *(const u4 *)(sl + 16 * lane), q1 = *(const u4 *)(sl + 1024 + 16 * lane), h = *(const u4 *)(sl + 2048 + 16 * (lane & 15));
+#pragma unroll
+            for (int j = 0; j < 4; j++) b[i].h[j] = h[j], b[i].q[j] = q0[j], b[i].q[4 + j] = q1[j];
+        }
+    }
+    __device__ __forceinline__ void transpose() {}
+    __device__ __forceinline__ void mac_lean(const u2 *, const qw_afrag_lds_sums &af, uint32_t k0, uint32_t kg, f4 &acc) const {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            uint32_t sc[2], mn[2];
+            qw_k4_scales(b[i].h + 1, sc, mn);
+            f4 sub = {0, 0, 0, 0};
+            b[i].template steps<0>(af, k0 + 256 * i, kg, sc, sub);
+            const float d = qw_h2f((uint16_t)b[i].h[0]), dm = qw_h2f((uint16_t)(b[i].h[0] >> 16));
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[j] = __builtin_fmaf(d, sub[j], acc[j]);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const float c = __builtin_fmaf(8.0f * d, (float)((sc[j] >> (8 * kg)) & 255), -dm * (float)((mn[j] >> (8 * kg)) & 255));
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af.sum((k0 + 256 * i) / 32 + 4 * j + kg), c, acc, 0, 0, 0);
+            }
+        }
     }
 };
 template <int NB> struct qw_chunk<12, NB> : qw_chunk_kqa<12, NB> {};
