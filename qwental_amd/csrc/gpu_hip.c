@@ -1005,7 +1005,6 @@ static bool bind_bytes(qw_batch *b, unsigned index, void *dst, size_t len, const
     return true;
 }
 
-_Static_assert(sizeof(qwk_prekq_args) <= QW_MAX_ARGS, "argument record");
 _Static_assert(sizeof(qwk_pre_args) <= QW_MAX_ARGS && sizeof(qwk_gu_args) <= QW_MAX_ARGS && sizeof(qwk_dn_args) <= QW_MAX_ARGS && sizeof(qwk_qmv_args) <= QW_MAX_ARGS,
                "a kernel argument record is larger than the launch record's copy of it");
 
@@ -1119,7 +1118,7 @@ static bool launch_qmvs(qw_batch *b, qwk_qmvm_args *a, unsigned tiles) {
     b->l[b->nl - 1].lds = qmvs_lds(a);
     return true;
 }
-// hw: the buffers the matrices lie in (NULL, a shared expert's rows of one chunk: the persistent kernel, no tile-major copies)
+// hw: the buffers the matrices lie in (NULL, a shared expert's rows: the persistent kernel, no tile-major copies)
 #define QW_Q6_PACK_MIN_ROWS 16384u
 static bool launch_qmvm(qw_batch *b, qwk_qmvm_args *a, qw_hbuf *const *hw) {
     unsigned tiles = 0;
@@ -1350,46 +1349,44 @@ static bool tr_sel(qw_batch *b) { // src/engine.c:609-614: 0 logits, 1 sel, 2 nb
     return bind_bytes(b, 2, &nbr, 4, "nbr") && nbr_ok(b, nbr) && launch_select(b, 0, 1, nbr);
 }
 
+// The front launch's grid: the router's workgroups, then the shared expert's; a wave per 256 values of K.
+static bool launch_pre(qw_batch *b, const char *fname, qwk_pre_args *a, unsigned shared) {
+    a->ctab = (const char *)b->g->tabs + QW_TAB_IQ3C;
+    for (a->sh = 0; 1u << a->sh < a->r.nb; a->sh++) {}
+    return add_launch(b, fname, a->nrouter + shared, a->r.D / 4, a, sizeof *a);
+}
 // A shared expert whose gate and up rows are in the other format family (Q4_K gate and IQ4_XS up in the reference's
-// model, bench/moe_bw.c:19-20): the multi-format matvec over the two matrices, then SwiGLU into H.
+// model, bench/moe_bw.c:19-20): behind the router's workgroups (front: the launch to come, *rode: it was sent off here), or a launch
+// of its own when the logits are given; or the matvec over the two matrices, then SwiGLU into H (QW_HIP_NO_SWIGLU_MATVEC).
 #define QW_SHGU_MAXI 4096
-// front: the router's arguments when the caller is the front launch, which then takes this work onto the workgroups
-// after the router's (one launch, qwk_pre_w1_kq) when it can; *rode tells whether it did.
 static bool shared_gu_kq(qw_batch *b, uint32_t nbr, const uint16_t *x, uint16_t *h, const qwk_pre_args *front, bool *rode) {
     const qw_kparams *p = &b->k->p;
     if (rode) *rode = false;
     if (p->I > QW_SHGU_MAXI) return fail(b, "moe_pre_gg: I %d too wide for shared gate/up types %d/%d", p->I, p->fsg, p->fsu);
     if (b->buf[2].off % 16 || b->buf[6].off % 16 || b->buf[7].off % 16) return fail(b, "moe_pre_gg: x and shared gate/up offsets must be 16-byte aligned for types %d/%d", p->fsg, p->fsu);
-    float *gy = b->g->shgu + (size_t)b->stream * 2 * 16 * QW_SHGU_MAXI, *uy = gy + (size_t)16 * p->I;
-    qwk_qmvm_args m = {.K = (uint32_t)p->D, .xstride = (uint32_t)p->D, .nb = nbr, .yfloat = 1, .nmat = 2, .x = x,
-                       .W = {b->pend_sg.Wsg, b->pend_sg.Wsu}, .y = {gy, uy}, .N = {(uint32_t)p->I, (uint32_t)p->I}, .fmt = {(uint32_t)p->fsg, (uint32_t)p->fsu},
-                       .rowbytes = {(uint32_t)fmt_rb(p->fsg, p->D), (uint32_t)fmt_rb(p->fsu, p->D)}, .ystride = {(uint32_t)p->I, (uint32_t)p->I}};
-    qwk_shact_args sa = {.g = gy, .u = uy, .H = h, .I = (uint32_t)p->I, .nb = nbr, .topk = (uint32_t)p->topk, .hplane = (uint32_t)p->NB * (uint32_t)(p->topk + 1) * (uint32_t)p->I};
+    const uint32_t hplane = (uint32_t)p->NB * (uint32_t)(p->topk + 1) * (uint32_t)p->I;
+    qwk_pre_args f = {.r = {.x = x, .D = (uint32_t)p->D, .nb = nbr}};
+    if (front) f = *front;
+    f.Wg = b->pend_sg.Wsg, f.Wu = b->pend_sg.Wsu, f.H = h, f.fg = (uint32_t)p->fsg, f.fu = (uint32_t)p->fsu;
+    f.rbg = (uint32_t)fmt_rb(p->fsg, p->D), f.rbu = (uint32_t)fmt_rb(p->fsu, p->D), f.I = (uint32_t)p->I, f.topk = (uint32_t)p->topk, f.hplane = hplane;
     b->pend_sg.valid = false; // done here
-    // This work depends on x alone, so it may run beside the router and the routed gate/up on the side stream
-    // (QW_HIP_SIDE=1). Off by default: with the matvec and SwiGLU as two launches it paid with one or two tokens (48
-    // layers of the reference model's shape: 2.89 -> 2.70 ms a token) and cost with more (6.81 -> 6.93 ms at 16); as
-    // the one launch it is now, the fork and join cost as much as the overlap gives at every token count.
+    // This work depends on x alone, so it may run beside the router and the routed gate/up on the side stream (QW_HIP_SIDE=1; off
+    // by default: the fork and join cost what the overlap gives at every token count).
     const int first = b->nl;
-    // one launch when the K range splits so that a workgroup holds whole (gate tile, up tile) pairs; else matvec, then SwiGLU
-    unsigned sw = 0;
-    for (unsigned s = QW_WAVES_GU / 2; s > 1 && !sw; s--)
-        if ((unsigned)(p->D / 256) % s == 0 && !b->sw.no_swiglu_matvec) sw = s;
-    if (sw) {
-        m.split = sw, m.sums = 0, m.H = h, m.topk = (uint32_t)p->topk, m.hplane = sa.hplane;
-        for (int j = 0; j < 2; j++) {
-            m.ntiles[j] = cdiv((unsigned)p->I, 16);
-            if (m.fmt[j] == 12 || m.fmt[j] == 13) m.sums = 1;
-        }
-        const unsigned wgs = umin((unsigned)b->g->ncu, cdiv(m.ntiles[0], QW_WAVES_GU / sw / 2));
-        if (front && p->rwf == 1 && b->sw.side != 1 && !b->sw.kq_own) { // binary16 router: its workgroups first, then these
-            qwk_prekq_args f = {.r = front->r, .nrouter = front->nrouter, .m = m};
-            if (!add_launch(b, "qwk_pre_w1_kq", f.nrouter + wgs, 64 * QW_WAVES_GU, &f, sizeof f)) return false;
+    if (!b->sw.no_swiglu_matvec) {
+        if (front && b->sw.side != 1 && !b->sw.kq_own) {
             *rode = true;
-            return true;
+            return launch_pre(b, p->rwf == 30 ? "qwk_pre_w30_kq" : "qwk_pre_w1_kq", &f, (unsigned)p->I / (p->fsg == p->fsu ? 8 : 16));
         }
-        if (!add_launch(b, "qwk_qmvm_swiglu", wgs, 64 * QW_WAVES_GU, &m, sizeof m)) return false;
-    } else if (!launch_qmvm(b, &m, NULL) || !add_launch(b, "qwk_sh_act", cdiv(nbr * (unsigned)p->I, 256), 256, &sa, sizeof sa)) return false;
+        f.nrouter = 0;
+        if (!launch_pre(b, "qwk_qmvm_swiglu", &f, (unsigned)p->I / (p->fsg == p->fsu ? 8 : 16))) return false;
+    } else {
+        float *gy = b->g->shgu + (size_t)b->stream * 2 * 16 * QW_SHGU_MAXI, *uy = gy + (size_t)16 * p->I;
+        qwk_qmvm_args m = {.K = (uint32_t)p->D, .xstride = (uint32_t)p->D, .nb = nbr, .yfloat = 1, .nmat = 2, .x = x, .W = {f.Wg, f.Wu}, .y = {gy, uy}, .N = {f.I, f.I},
+                           .fmt = {f.fg, f.fu}, .rowbytes = {f.rbg, f.rbu}, .ystride = {f.I, f.I}};
+        qwk_shact_args sa = {.g = gy, .u = uy, .H = h, .I = f.I, .nb = nbr, .topk = f.topk, .hplane = hplane};
+        if (!launch_qmvm(b, &m, NULL) || !add_launch(b, "qwk_sh_act", cdiv(nbr * (unsigned)p->I, 256), 256, &sa, sizeof sa)) return false;
+    }
     if (b->sw.side == 1)
         for (int i = first; i < b->nl; i++) b->l[i].side = true;
     return true;
@@ -1417,34 +1414,31 @@ static bool tr_pre(qw_batch *b) {
         const uint16_t *x;
         return !kq_ok(p->fsg) || (bind_ptr(b, 2, (size_t)nbr * p->D * 2, false, "x", (void **)&x) && shared_gu_kq(b, nbr, x, h, NULL, NULL));
     }
-    // router rows per workgroup: 16 on the matrix cores (binary16 router), 8 on the vector units (bf16 router)
-    qwk_pre_args a = {.nrouter = cdiv((unsigned)p->E + 1, p->rwf == 1 ? 16 : 8)};
+    // router rows per workgroup: 16 (binary16), or one a wave and eight tokens at most (bfloat16)
+    qwk_pre_args a = {.nrouter = p->rwf == 1 ? cdiv((unsigned)p->E + 1, 16) : cdiv((unsigned)p->E + 1, (unsigned)p->D / 256) * cdiv(nbr, 8)};
     if (!fill_router(b, &a.r, 0, 1, 2, 3, nbr)) return false;
     if (b->buf[2].off % 16) return fail(b, "moe_pre_gg: x offset %zu is not 16-byte aligned", b->buf[2].off);
     if (p->rwf == 1 && (b->buf[0].off % 16 || b->buf[1].off % 16)) return fail(b, "moe_pre_gg: router weight offsets must be 16-byte aligned");
-    // The shared expert's gate/up runs on the workgroups after the router's when a tile row splits into at most 8
-    // chunks (D a multiple of 512, at most 4096) and the weights are Q8_0 or packed IQ3_S; otherwise it is left for
-    // the gate/up launch (pend_sg).
+    // The shared expert's gate/up runs on the workgroups after the router's when D is a multiple of 512 and the weights are
+    // Q8_0 or packed IQ3_S, and in the formats of the other family at any D; otherwise it is left for the gate/up launch (pend_sg).
     char fn[48];
     fname_fmt(fn, sizeof fn, "qwk_pre_w%d", p->rwf == 30 ? 30 : 1);
-    unsigned grid = a.nrouter;
-    const unsigned cpr = (unsigned)p->D / 512;
-    if (p->D % 512 == 0 && cpr <= 8 && !b->sw.shared_in_gu) {
+    unsigned shared = 0;
+    if (p->D % 512 == 0 && !b->sw.shared_in_gu) {
         const uint32_t nblk = (uint32_t)p->D / 256;
         const uint8_t *ps = p->fsg == 21 ? get_pack(b, QW_F_PACKED, b->pend_sg.hg, b->pend_sg.Wsg, b->pend_sg.hu, b->pend_sg.Wsu, (uint64_t)(p->I / 8), nblk, (uint32_t)rb) : NULL;
         if (p->fsg == 8 || ps) {
-            a.g = (qwk_gu_args){.Wg = ps ? ps : b->pend_sg.Wsg, .Wu = ps ? NULL : b->pend_sg.Wsu, .x = a.r.x, .H = h, .D = (uint32_t)p->D, .I = (uint32_t)p->I,
-                                .rowbytes = ps ? nblk * QW_SLAB_BYTES : (uint32_t)rb, .nbr = nbr, .topk = (uint32_t)p->topk, .gnb = (uint32_t)p->gnb, .shared = 1,
-                                .hplane = (uint32_t)p->NB * (uint32_t)(p->topk + 1) * (uint32_t)p->I, .glut = glut(b->g)};
-            fname_fmt(fn, sizeof fn, "qwk_pre_w%d_s%d_c%d", p->rwf == 30 ? 30 : 1, ps ? QW_F_PACKED : 8, ps ? 2 : 16);
-            grid += cdiv((unsigned)p->I / 8, 8 / cpr);
+            a.Wg = ps ? ps : b->pend_sg.Wsg, a.Wu = ps ? NULL : b->pend_sg.Wsu, a.rbg = ps ? nblk * QW_SLAB_BYTES : (uint32_t)rb;
+            a.H = h, a.I = (uint32_t)p->I, a.topk = (uint32_t)p->topk, a.hplane = (uint32_t)p->NB * (uint32_t)(p->topk + 1) * (uint32_t)p->I;
+            fname_fmt(fn, sizeof fn, "qwk_pre_w%d_s%d", p->rwf == 30 ? 30 : 1, ps ? QW_F_PACKED : 8);
+            shared = (unsigned)p->I / 8;
             b->pend_sg.valid = false; // done here
         }
     }
     // the counter buffer of the reference's hand-over (index 4) is not used
     bool rode = false;
     if (kq_ok(p->fsg) && !shared_gu_kq(b, nbr, a.r.x, h, &a, &rode)) return false; // first: side launches fork where they stand in the batch
-    if (!rode && !add_launch(b, intern(fn), grid, 512, &a, sizeof a)) return false;
+    if (!rode && !launch_pre(b, intern(fn), &a, shared)) return false;
     if (!fill_select(b, &b->pend_sel.a, 3, 5, nbr)) return false;
     b->pend_sel.valid = true; // made by the gate/up launch if one follows for the same record, else by its own launch
     return true;

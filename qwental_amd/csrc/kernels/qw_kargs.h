@@ -47,10 +47,6 @@ typedef struct {
     uint32_t N[4], fmt[4], rowbytes[4], ystride[4], ntiles[4];
     uint32_t K, xstride, nb, yfloat, nmat, sums; /* sums: some matrix is Q4_K / Q5_K (needs the 32-value sums of x) */
     uint32_t split, pad;                         /* waves a tile's K range is cut over (1 .. 6; > 1 needs K % (256 * split) == 0) */
-    /* qwk_qmvm_swiglu (matrix 0 = gate rows, matrix 1 = up rows of a shared expert, N[0] = N[1] = I, split in
-     * {2, 3, 4, 5, 6}): nothing goes to y; H[t][topk][r] = silu(gate) * up as binary16 hi + lo planes, hplane halves apart */
-    uint16_t *H;
-    uint32_t topk, hplane;
     /* qwk_qmvs: the backend's IQ3_S table without signs; 2^sh >= nb; 16-byte units of LDS kept for a table */
     const void *ctab;
     uint32_t sh, tabu;
@@ -148,20 +144,17 @@ typedef struct {
     uint32_t spin_limit, pad; /* polls of the generation word after which a waiting workgroup gives up */
 } qwk_gud_args;
 
-/* front part of a layer: router rows on the first nrouter workgroups; when g.Wsg != NULL the shared expert's gate/up
- * on the workgroups after them (g: its arguments, shared = 1), one chunk of a tile per wave, summed through LDS. */
+/* front part of a layer: router rows on the first nrouter workgroups, the shared expert's gate/up with SwiGLU on those after them (x,
+ * nb and D: r's): H[t][topk][j] = silu(gate) * up as binary16 hi + lo planes, hplane halves apart. A workgroup has D / 256 waves. */
+#define QW_PRE_WAVES 10u
 typedef struct {
     qwk_router_args r;
-    uint32_t nrouter, pad;
-    qwk_gu_args g;
+    uint32_t nrouter, sh;    /* 2^sh >= nb */
+    const uint8_t *Wg, *Wu;  /* tile-major IQ3_S: one copy of both at Wg, rbg bytes a tile */
+    uint16_t *H;
+    const void *ctab;        /* the backend's IQ3_S table without signs */
+    uint32_t fg, fu, rbg, rbu, I, topk, hplane, pad;
 } qwk_pre_args;
-/* the front launch when the shared expert's gate/up rows are in the K-quant / IQ4 / plain family (qwk_pre_w1_kq):
- * m as for qwk_qmvm_swiglu, on the workgroups after the router's */
-typedef struct {
-    qwk_router_args r;
-    uint32_t nrouter, pad;
-    qwk_qmvm_args m;
-} qwk_prekq_args;
 
 typedef struct { /* out[t][row] = half(sum_s w[t][s] * Pg[t][s][row] + w[t][topk] * Psh[t][row]) */
     const float *Pg, *Psh;

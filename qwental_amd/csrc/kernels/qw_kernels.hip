@@ -43,13 +43,6 @@ __shared__ uint32_t qw_sst[12 * 16];
 #define QW_SDEP(v) do {} while (0)
 #define QW_SST_FLUSH() do {} while (0)
 #endif
-#if defined(QW_STAMPS) && QW_STAMPS == 4 // steps of the front launch only
-#undef QW_DSTAMP
-#define QW_DSTAMP(k) do {} while (0)
-#define QW_PSTAMP(k) do { if (threadIdx.x == 0 && qw_stamp_ptr) qw_stamp_ptr[512 + 16 * blockIdx.x + (k)] = (uint32_t)__builtin_amdgcn_s_memrealtime(); } while (0)
-#else
-#define QW_PSTAMP(k) do {} while (0)
-#endif
 #if defined(QW_STAMPS) && QW_STAMPS == 5 // steps of the hyper-connection's launches (workgroups 0 .. 255 of each)
 #undef QW_DSTAMP
 #define QW_DSTAMP(k) do {} while (0)
@@ -453,98 +446,6 @@ template <int F, int NB> __device__ __forceinline__ void qmvm_matrix_split(const
         __syncthreads();
     }
 }
-// One part of one tile: the product over chunks [part * cpp, (part + 1) * cpp) of the rows of tile t of matrix j; ready() as in qw_task_pipeline.
-template <int F, int NB, class S> __device__ __forceinline__ f4 qmvm_part(const qwk_qmvm_args &a, uint32_t j, const uint32_t *tab, const qw_afrag_kq &af, uint32_t t, uint32_t part, S ready) {
-    typedef qw_chunk_kq<F, NB> C;
-    const qmvm_tile<F, NB> T = {a, j};
-    const uint32_t lane = qw_lane(), kg = lane >> 4, cpp = a.K / (C::BLK_K * NB) / a.split;
-    f4 acc = {0, 0, 0, 0};
-    qw_task_pipeline<C>(1, 0, 1, cpp, NB * C::BLK_B, lane & 3, [&](uint32_t) { return T.rowp(t) + (size_t)part * cpp * NB * C::BLK_B; },
-                        [&](uint32_t, uint32_t ci, const C &c) { c.mac(tab, af, (part * cpp + ci) * NB * C::BLK_K, kg, acc); }, ready);
-    return acc;
-}
-// The shared expert's gate/up in the other format family with SwiGLU in the same launch (kernels/moe_gg.metal:563-573):
-// matrix 0 holds the gate rows, matrix 1 the up rows, each of its own format. A workgroup takes 12 / split / 2 pairs of
-// tiles (gate tile t and up tile t side by side), split waves a tile; the partial sums meet in LDS, and
-// the first wave of a gate tile adds up both tiles in part order, applies SwiGLU and stores H's two planes.
-// The work is a megabyte or two over a few dozen workgroups and bound by its round trips: the activations are asked for
-// first (straight into LDS), every wave asks for its blocks behind them (up to two, which all K up to 3072 come down to), and
-// only then the workgroup waits, once. (The weights asked for after the activations and their sums had arrived: four tokens, 512 columns of 2048 in Q4_K 13.7 us a front launch, now 9.0; eight tokens, 640 of 2560 in Q4_K and IQ4_XS 10.5, now 10.0.
-// Sixteen waves with a block each: 128 registers, which spill.)
-// bid of nblk: the workgroup's number among those that do this work (the front launch puts the router's workgroups first).
-struct qw_swiglu_lds { u4 xf[QW_KQ_MAXK * 2]; float xs[QW_KQ_MAXK / 2]; uint32_t tab[QW_KQ_TAB]; f4 red[QW_WG_QMVM]; };
-__device__ __forceinline__ void qmvm_swiglu_body(const qwk_qmvm_args &a, qw_swiglu_lds &L, uint32_t bid, uint32_t nblk) {
-    qw_kq_tab_build(L.tab);
-    qw_stage_x_issue(L.xf, a.x, a.xstride, a.K, a.nb);
-    bool staged = false;
-    auto ready = [&] { // once per wave, behind its first weight loads
-        if (staged) return;
-        staged = true;
-        qw_lds_arrive();
-        __syncthreads();
-        if (!a.sums) return;
-        // sums of 32 activations per token, in index order
-        for (uint32_t i = threadIdx.x; i < (a.K >> 5) * 16; i += blockDim.x) {
-            const uint32_t c = i >> 4, m = i & 15;
-            float sum = 0;
-#pragma unroll
-            for (uint32_t f = 0; f < 4; f++) {
-                const h8 v = __builtin_bit_cast(h8, L.xf[(4 * c + f) * 16 + m]);
-#pragma unroll
-                for (int e = 0; e < 8; e++) sum += (float)v[e];
-            }
-            L.xs[i] = sum;
-        }
-        __syncthreads();
-    };
-    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave(), sp = a.split;
-    const qw_afrag_kq af = {L.xf, L.xs, n, kg};
-    const uint32_t pairs = (QW_WG_QMVM / 64) / sp / 2, slot = wave / sp, part = wave % sp, which = slot & 1, ntiles = a.ntiles[0];
-    const uint32_t ngroups = (ntiles + pairs - 1) / pairs;
-    for (uint32_t g = bid; g < ngroups; g += nblk) {
-        const uint32_t t = slot < 2 * pairs ? g * pairs + slot / 2 : ntiles; // waves past a whole number of pairs: none
-        f4 acc = {0, 0, 0, 0};
-        if (t < ntiles) {
-            switch (a.fmt[which]) { // uniform in a wave
-            case 12: acc = qmvm_part<12, 1>(a, which, L.tab, af, t, part, ready); break;
-            case 13: acc = qmvm_part<13, 1>(a, which, L.tab, af, t, part, ready); break;
-            case 14: acc = qmvm_part<14, 1>(a, which, L.tab, af, t, part, ready); break;
-            case 23: acc = qmvm_part<23, 1>(a, which, L.tab, af, t, part, ready); break;
-            case 20: acc = qmvm_part<20, 8>(a, which, L.tab, af, t, part, ready); break;
-            case 1: acc = qmvm_part<1, 8>(a, which, L.tab, af, t, part, ready); break;
-            case 30: acc = qmvm_part<30, 8>(a, which, L.tab, af, t, part, ready); break;
-            default: ready(); // (no other format reaches this kernel; every wave meets the barriers all the same)
-            }
-        } else ready();
-        L.red[wave * 64 + lane] = acc;
-        __syncthreads();
-        if (part == 0 && which == 0 && t < ntiles) {
-            f4 gate = L.red[wave * 64 + lane], up = L.red[(wave + sp) * 64 + lane];
-            for (uint32_t q = 1; q < sp; q++) gate += L.red[(wave + q) * 64 + lane], up += L.red[(wave + sp + q) * 64 + lane];
-            const uint32_t r = 16 * t + n;
-            if (r < a.N[0])
-#pragma unroll
-                for (uint32_t j = 0; j < 4; j++) {
-                    const uint32_t tok = 4 * kg + j;
-                    if (tok < a.nb) {
-                        const float gv = gate[j], h = gv / (1.0f + __expf(-gv)) * up[j];
-                        const _Float16 hi = (_Float16)h, lo = (_Float16)(h - (float)hi);
-                        const size_t o = ((size_t)tok * (a.topk + 1) + a.topk) * a.N[0] + r;
-                        a.H[o] = __builtin_bit_cast(uint16_t, hi);
-                        a.H[o + a.hplane] = __builtin_bit_cast(uint16_t, lo);
-                    }
-                }
-        }
-        __syncthreads();
-    }
-}
-#if QW_IN_PART(0)
-extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_qmvm_swiglu(qwk_qmvm_args a) {
-    __shared__ qw_swiglu_lds L;
-    qmvm_swiglu_body(a, L, blockIdx.x, gridDim.x);
-}
-#endif
-
 #if QW_IN_PART(0)
 extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_qmvm(qwk_qmvm_args a) {
     __shared__ struct { u4 xf[QW_KQ_MAXK * 2]; float xs[QW_KQ_MAXK / 2]; uint32_t tab[QW_KQ_TAB]; f4 red[QW_WG_QMVM]; } L;
@@ -676,44 +577,6 @@ template <int WF, int NB> __device__ __forceinline__ void router_row(const qwk_r
         if (lane == 0 && (uint32_t)t < a.nb) a.logits[(size_t)t * (a.E + 1) + r] = v;
     }
 }
-// The same arithmetic with the activations read from LDS (xs: binary16 [nb][D], copied there by the workgroup).
-template <int WF, int NB> __device__ __forceinline__ void router_row_lds(const qwk_router_args &a, const uint16_t *xs, uint32_t r, uint32_t lane) {
-    const uint16_t *w = r < a.E ? a.Wr + (size_t)r * a.D : a.Wsg;
-    float acc[NB];
-#pragma unroll
-    for (int t = 0; t < NB; t++) acc[t] = 0;
-    for (uint32_t c = lane; c < a.D / 8; c += 64) {
-        const u4 wv = *(const u4 *)(w + 8 * c);
-        float wf[8];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            wf[2 * i] = WF == 30 ? qw_bf2f((uint16_t)wv[i]) : qw_h2f((uint16_t)wv[i]);
-            wf[2 * i + 1] = WF == 30 ? qw_bf2f((uint16_t)(wv[i] >> 16)) : qw_h2f((uint16_t)(wv[i] >> 16));
-        }
-#pragma unroll
-        for (int t = 0; t < NB; t++) {
-            const h8 xv = *(const h8 *)(xs + (size_t)((uint32_t)t < a.nb ? t : a.nb - 1) * a.D + 8 * c);
-#pragma unroll
-            for (int i = 0; i < 8; i++) acc[t] = __builtin_fmaf(wf[i], (float)xv[i], acc[t]);
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < NB; t++) {
-        float v = acc[t];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-        if (lane == 0 && (uint32_t)t < a.nb) a.logits[(size_t)t * (a.E + 1) + r] = v;
-    }
-}
-template <int WF> __device__ __forceinline__ void router_rows_lds(const qwk_router_args &a, const uint16_t *xs, uint32_t r, uint32_t lane) {
-    if (r > a.E) return;
-    if (a.nb <= 1) router_row_lds<WF, 1>(a, xs, r, lane);
-    else if (a.nb <= 2) router_row_lds<WF, 2>(a, xs, r, lane);
-    else if (a.nb <= 4) router_row_lds<WF, 4>(a, xs, r, lane);
-    else if (a.nb <= 8) router_row_lds<WF, 8>(a, xs, r, lane);
-    else router_row_lds<WF, 16>(a, xs, r, lane);
-}
-
 template <int WF> __device__ __forceinline__ void router_rows(const qwk_router_args &a, uint32_t r, uint32_t lane) {
     if (r > a.E) return;
     if (a.nb <= 1) router_row<WF, 1>(a, r, lane);
@@ -1324,179 +1187,355 @@ QW_GU(QW_F_RT, 1, 0, 1, qwk_gu_rt) QW_GU(QW_F_RT, 1, 21, 1, qwk_gu_rt_s21_c1) QW
 #endif
 
 // ================================================================ front part of a layer (kernels/moe_gg.metal:534-590)
-// Router rows with the activations copied into LDS once per workgroup (8 rows per workgroup) on the first
-// a.nrouter workgroups. The workgroups after them do the shared expert's gate/up (the reference computes it in the
-// same dispatch, kernels/moe_gg.metal:563-573): a tile of 8 gate + 8 up rows is split by chunk over consecutive
-// waves of one workgroup (a chunk each, so that the whole expert takes one memory round trip), the partial sums meet
-// in LDS and the wave of chunk 0 adds them in chunk order, applies SwiGLU and stores H[t][topk].
+// Router rows, sixteen a workgroup, on the first a.nrouter workgroups; on those after them the shared expert's gate/up with SwiGLU
+// (the reference computes it in the same dispatch, kernels/moe_gg.metal:563-573), a tile of 8 gate + 8 up rows a workgroup
+// (IQ3_S, Q8_0), or a gate tile and an up tile of 16 rows, each in its own format (the K-quant / IQ4 / plain family).
+// A few megabytes over a hundred workgroups, bound by latency, built as the dense products of qw_small.hip.h are: a wave takes 256
+// values of K and asks for everything it needs at entry - its block of the sixteen (or twice sixteen) rows, its 256 values of
+// every token, for IQ3_S its share of the 4 KB table -, puts its tokens into LDS for itself, and the partial sums meet in LDS and are
+// added in the order of K. The router's rows are asked for four lanes to 64 contiguous bytes and moved to the lanes of the
+// matrix instruction afterwards (in that instruction's own order every lane asks for a row of its own, 64 requests a load, which
+// the address unit serves one by one: 1.6 us for the eight waves).
+// Measured (512 router rows of 2048, shared 512 x 2048, us a launch; before: the table of 64 KB and all tokens staged in every workgroup, a
+// wave 512 values): IQ3_S 6.2 -> 4.4 at one token, 6.8 -> 5.1 at four, 7.9 -> 6.0 at sixteen; Q8_0 7.2 -> 5.8, 9.2 -> 6.0, 10.3 -> 7.1; Q4_K
+// 8.1 -> 4.6, 8.9 -> 6.0, 9.0 -> 7.1; Q4_K and IQ4_XS at 640 x 2560 9.5 -> 7.7, 9.8 -> 9.2 (eight), 10.7 -> 10.6; a bfloat16 router beside
+// IQ3_S 6.3 -> 4.2 at two, 11.6 -> 7.8 at sixteen. The order of every sum is that of the kernels before, except where both shared
+// matrices have one format of the K-quant family.
 // The selection is not made here: handing it to the last router workgroup through a device-wide counter was measured
 // slower than a kernel boundary.
-template <int WF> __device__ __forceinline__ void pre_router(const qwk_pre_args &a, u4 *lds) {
-    const uint32_t nx = a.r.nb * a.r.D / 8; // 16-byte units of x
-    for (uint32_t i = threadIdx.x; i < nx; i += blockDim.x) lds[i] = ((const u4 *)a.r.x)[i];
-    __syncthreads();
-    router_rows_lds<WF>(a.r, (const uint16_t *)lds, blockIdx.x * (blockDim.x >> 6) + qw_wave(), qw_lane());
-}
-// Binary16 router on the matrix cores: a workgroup takes 16 router rows (row E is the shared-expert gate vector), its
-// waves split K among themselves (256 values = 8 matrix instructions a wave per pass), the partial sums meet in LDS
-// and wave 0 adds them in wave order. A token's logits do not depend on the other token columns.
-// Eight waves take part whatever the workgroup's size: the split of K and the order of the final sum, hence the bits
-// of the logits, are the same in every kernel that holds this router.
-// Up to this many tokens the front launch reads operand A straight from memory instead of staging all of x in LDS: a
-// wave then reads only the K range it multiplies (8 KB of 64 at sixteen tokens) and no barrier stands before the first
-// product — but every lane of an operand reads its own token's row, 64 requests an instruction, which the address unit
-// serialises: with 8 or 16 tokens the staged form is 1 to 2 us faster, with one or two the direct one (24 layers at one
-// token: 0.638 -> 0.618 ms).
-#define QW_PRE_DIRECT_NB 2u
-__device__ __forceinline__ void pre_router_mfma(const qwk_router_args &a, u4 *xf, f4 *part) {
-    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave(), nwv = QW_WG / 64;
-    const uint32_t row = 16 * blockIdx.x + n;
-    const uint16_t *wrow = row < a.E ? (const uint16_t *)a.Wr + (size_t)row * a.D : (const uint16_t *)a.Wsg; // rows past E repeat the gate vector; not stored
-    f4 acc = {0, 0, 0, 0};
-    u4 w[8];
-    uint32_t k0 = wave < nwv ? 256 * wave : a.D; // (waves past the eighth: nothing)
-    if (a.nb <= QW_PRE_DIRECT_NB) {
-        // lane (n, kg) supplies eight activations of token n per step; token columns past the batch read token 0's row,
-        // their results are never stored
-        const uint16_t *xrow = a.x + (size_t)(n < a.nb ? n : 0) * a.D;
-        u4 xa[8];
-        if (k0 < a.D)
-#pragma unroll
-            for (int j = 0; j < 8; j++) w[j] = *(const u4 *)(wrow + k0 + 32 * j + 8 * kg), xa[j] = *(const u4 *)(xrow + k0 + 32 * j + 8 * kg);
-        for (; k0 < a.D; k0 += 256 * nwv) {
-#pragma unroll
-            for (int j = 0; j < 8; j++) acc = qw_mfma(__builtin_bit_cast(h8, xa[j]), __builtin_bit_cast(h8, w[j]), acc);
-            if (k0 + 256 * nwv < a.D)
-#pragma unroll
-                for (int j = 0; j < 8; j++) w[j] = *(const u4 *)(wrow + k0 + 256 * nwv + 32 * j + 8 * kg), xa[j] = *(const u4 *)(xrow + k0 + 256 * nwv + 32 * j + 8 * kg);
-        }
-    } else {
-        // the first pass's weights are in flight while x is staged
-        if (k0 < a.D)
-#pragma unroll
-            for (int j = 0; j < 8; j++) w[j] = *(const u4 *)(wrow + k0 + 32 * j + 8 * kg);
-        qw_stage_x(xf, a.x, a.D, a.D, a.nb);
-        __syncthreads();
-        for (; k0 < a.D; k0 += 256 * nwv) {
-#pragma unroll
-            for (int j = 0; j < 8; j++) acc = qw_mfma(__builtin_bit_cast(h8, xf[((k0 + 32 * j + 8 * kg) >> 3) * 16 + n]), __builtin_bit_cast(h8, w[j]), acc);
-            if (k0 + 256 * nwv < a.D)
-#pragma unroll
-                for (int j = 0; j < 8; j++) w[j] = *(const u4 *)(wrow + k0 + 256 * nwv + 32 * j + 8 * kg);
-        }
+// A token's logits do not depend on the other token columns. Eight waves at most take part in a router row, wave w with
+// blocks w and w + 8, so that the order of its sum is the same whatever D.
+struct qw_pre_lds { u2 tab[QW_SMALL_TABU * 2]; u4 x[QW_PRE_WAVES * 512]; float xs[QW_PRE_WAVES][256]; }; // table; a wave's activations (32 << sh units a block), later in the same place its partial sums; its sums of 32 activations
+// The wave's 256 values of K from k0 on of every token, two tokens a load; lds: where they go (layout: qw_afrag_small)
+struct qw_pre_x {
+    u4 v[8];
+    __device__ __forceinline__ void load(const qwk_router_args &r, uint32_t k0) {
+        const uint16_t *p = r.x + k0 + 8 * (threadIdx.x & 31);
+        auto get = [&](uint32_t i) {
+            const uint32_t m = 2 * i + ((threadIdx.x >> 5) & 1);
+            v[i] = *(const u4 *)(p + (size_t)(m < r.nb ? m : r.nb - 1) * r.D);
+        };
+        get(0);
+        if (r.nb > 2) get(1);
+        if (r.nb > 4) get(2), get(3);
+        if (r.nb > 8) get(4), get(5), get(6), get(7);
     }
-    part[wave * 64 + lane] = acc;
+    __device__ __forceinline__ void store(u4 *lds, uint32_t nb, uint32_t sh) const {
+        auto put = [&](uint32_t i) {
+            const uint32_t m = 2 * i + ((threadIdx.x >> 5) & 1), c = threadIdx.x & 31;
+            if (m < (1u << sh)) lds[(c << sh) + (m ^ (c & ((1u << sh) - 1)))] = v[i];
+        };
+        put(0);
+        if (nb > 2) put(1);
+        if (nb > 4) put(2), put(3);
+        if (nb > 8) put(4), put(5), put(6), put(7);
+    }
+};
+// Binary16 rows, sixteen a workgroup.
+__device__ __forceinline__ void pre_router(const qwk_pre_args &a, qw_pre_lds &L) {
+    const qwk_router_args &r = a.r;
+    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave(), nwv = (blockDim.x >> 6) < 8 ? blockDim.x >> 6 : 8;
+    u4 *const x = L.x + wave * 512;
+    f4 acc = {0, 0, 0, 0};
+    if (wave < nwv) {
+        const uint32_t lrow = 16 * blockIdx.x + (lane >> 2);
+        const uint16_t *w = (lrow < r.E ? (const uint16_t *)r.Wr + (size_t)lrow * r.D : (const uint16_t *)r.Wsg) + 256 * wave + 8 * (lane & 3); // rows past E repeat the gate vector; not stored
+        const bool two = 256 * (wave + 8) < r.D;
+        u4 w0[8], w1[8];
+        qw_pre_x x0, x1;
+#pragma unroll
+        for (int j = 0; j < 8; j++) w0[j] = *(const u4 *)(w + 32 * j);
+        if (two)
+#pragma unroll
+            for (int j = 0; j < 8; j++) w1[j] = *(const u4 *)(w + 2048 + 32 * j);
+        x0.load(r, 256 * wave);
+        if (two) x1.load(r, 256 * (wave + 8));
+        const uint32_t src4 = qw_pull_addr();
+        auto block = [&](u4 (&wv)[8], const qw_pre_x &xv, u4 *lds) {
+            xv.store(lds, r.nb, a.sh);
+            __builtin_amdgcn_wave_barrier(); // (a wave's LDS operations complete in order)
+            const qw_afrag_small af = {lds, n & ((1u << a.sh) - 1), a.sh};
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) wv[j][i] = qw_pull(wv[j][i], src4);
+#pragma unroll
+            for (int j = 0; j < 8; j++) acc = qw_mfma(af.at8(32 * j + 8 * kg), __builtin_bit_cast(h8, wv[j]), acc);
+        };
+        block(w0, x0, x);
+        if (two) block(w1, x1, x + 8 * 512); // (waves 8 and 9, whose place this is, have nothing to do here)
+        if (wave) ((f4 *)x)[lane] = acc;
+    }
     __syncthreads();
-    if (wave != 0) return;
-    for (uint32_t i = 1; i < nwv; i++) acc += part[i * 64 + lane];
-    if (row <= a.E)
+    if (wave) return;
+    for (uint32_t q = 1; q < nwv; q++) acc += ((const f4 *)L.x)[q * 512 + lane];
+    const uint32_t row = 16 * blockIdx.x + n;
+    if (row <= r.E)
 #pragma unroll
         for (uint32_t j = 0; j < 4; j++)
-            if (4 * kg + j < a.nb) a.logits[(size_t)(4 * kg + j) * (a.E + 1) + row] = acc[j];
+            if (4 * kg + j < r.nb) r.logits[(size_t)(4 * kg + j) * (r.E + 1) + row] = acc[j];
 }
-// Operand A of one chunk held in registers: the fragments a lane needs for its chunk, asked for together with the chunk's
-// weights (read by position: qw_af_hi). BLK_K = 256: a lane's slice of a block is 64 values, eight steps of 8; BLK_K = 32:
-// one step a block.
-template <int BLK_K, int NB> struct qw_afrag_regs {
-    static constexpr int NX = BLK_K == 256 ? 8 * NB : NB;
-    static constexpr bool indexed = true, has_lo = false;
-    h8 x[NX];
-    __device__ __forceinline__ void load(const uint16_t *row, uint32_t k0, uint32_t kg) { // row: this lane's token
+// Bfloat16 rows, one a wave (the arithmetic of router_row, so its bits: multiply-adds in index order per lane, then the sums over lanes 32,
+// 16, ... 1 apart), and eight tokens at most: the token groups of a row block lie nrb workgroups apart. Weights and activations are asked
+// for together; the sums of up to eight tokens go through the exchange side by side, every step halving what a lane holds.
+template <int NB> __device__ __forceinline__ void pre_router_bf(const qwk_pre_args &a, qw_pre_lds &L, uint32_t r0, uint32_t t0, uint32_t nt) {
+    const qwk_router_args &r = a.r;
+    const uint32_t lane = qw_lane(), row = r0 + qw_wave(), units = r.D / 8, nx = nt * units;
+    const uint16_t *w = row < r.E ? (const uint16_t *)r.Wr + (size_t)row * r.D : (const uint16_t *)r.Wsg;
+    u4 wv[5], xv[4];
 #pragma unroll
-        for (int i = 0; i < NX; i++) x[i] = *(const h8 *)(row + k0 + (BLK_K == 256 ? 64 * kg + 256 * (i >> 3) + 8 * (i & 7) : 8 * kg + 32 * i));
+    for (uint32_t k = 0; k < 5; k++)
+        if (64 * k < units) wv[k] = *(const u4 *)(w + 8 * (lane + 64 * k < units ? lane + 64 * k : 0));
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) // (two tokens to a round of the workgroup's threads)
+        if (k * blockDim.x < nx) xv[k] = ((const u4 *)(r.x + (size_t)t0 * r.D))[threadIdx.x + k * blockDim.x < nx ? threadIdx.x + k * blockDim.x : 0];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++)
+        if (threadIdx.x + k * blockDim.x < nx) L.x[threadIdx.x + k * blockDim.x] = xv[k];
+    __syncthreads();
+    float acc[NB];
+#pragma unroll
+    for (int t = 0; t < NB; t++) acc[t] = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 5; k++) {
+        const uint32_t c = lane + 64 * k;
+        if (c < units)
+#pragma unroll
+            for (int t = 0; t < NB; t++) {
+                const h8 v = __builtin_bit_cast(h8, L.x[((uint32_t)t < nt ? t : nt - 1) * units + c]);
+#pragma unroll
+                for (int i = 0; i < 8; i++) acc[t] = __builtin_fmaf(qw_bf2f((uint16_t)(wv[k][i >> 1] >> (16 * (i & 1)))), (float)v[i], acc[t]);
+            }
     }
-    __device__ __forceinline__ h8 hi(uint32_t) const { return h8{}; } // (not used: the provider is indexed)
-    __device__ __forceinline__ h8 lo(uint32_t) const { return h8{}; }
-};
-template <int F, int CH> __device__ __forceinline__ void pre_shared(const qwk_pre_args &pa, u2 *lut, u4 *xf, f4 *part) {
-    typedef qw_chunk<F, CH> C;
-    const qwk_gu_args &a = pa.g;
-    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, K = a.topk, wave = qw_wave(), nwv = blockDim.x >> 6;
-    const uint32_t cpr = a.D / (C::BLK_K * CH), tpw = nwv / cpr; // tiles per workgroup (the host checks cpr <= waves)
-    const uint32_t tile = (blockIdx.x - pa.nrouter) * tpw + wave / cpr, ci = wave % cpr;
-    const bool on = wave < tpw * cpr && tile < a.I / 8;
-    QW_PSTAMP(1);
-    C c;
-    if (on) {
-        if constexpr (F == QW_F_PACKED) c.load(a.Wg + (size_t)tile * a.rowbytes + (size_t)ci * CH * C::BLK_B, lane);
-        else c.load(((lane >> 2) < 8 ? a.Wg : a.Wu) + ((size_t)8 * tile + ((lane >> 2) & 7)) * a.rowbytes + (size_t)ci * CH * C::BLK_B, lane & 3);
+    // lane bits 5, 4, 3 pick the token as the exchange goes on: token bit 2, 1, 0 of eight (bit 5 alone of two)
+#pragma unroll
+    for (int h = NB / 2, o = 32; o; o >>= 1, h >>= 1) {
+        if (h) {
+            const bool up = lane & o;
+#pragma unroll
+            for (int t = 0; t < (h ? h : 1); t++) acc[t] = (up ? acc[t + h] : acc[t]) + __shfl_xor(up ? acc[t] : acc[t + h], o);
+        } else acc[0] += __shfl_xor(acc[0], o);
     }
-    f4 acc = {0, 0, 0, 0};
-    if (a.nbr <= QW_PRE_DIRECT_NB) {
-        // one or two tokens: the chunk's activations straight into registers, the table behind the weights; all awaited
-        // once. Token columns past the batch read token 0's row; their results are never stored.
-        qw_afrag_regs<C::BLK_K, CH> af;
-        if (on) af.load(a.x + (size_t)(n < a.nbr ? n : 0) * a.D, ci * CH * C::BLK_K, kg);
-        if (qw_has_lut(F)) {
-            qw_lut_copy_issue(lut, (const u2 *)a.glut);
-            qw_lds_arrive();
-            __syncthreads();
-        }
-        if (on) {
+    constexpr uint32_t lg = NB == 8 ? 3 : NB == 4 ? 2 : NB == 2 ? 1 : 0;
+    const uint32_t t = lane >> (6 - lg);
+    if ((lane & ((64u >> lg) - 1)) == 0 && t < nt && row <= r.E) r.logits[(size_t)(t0 + t) * (r.E + 1) + row] = acc[0];
+}
+template <int WF> __device__ __forceinline__ void pre_router_any(const qwk_pre_args &a, qw_pre_lds &L) {
+    if constexpr (WF == 1) pre_router(a, L);
+    else {
+        const uint32_t nwv = blockDim.x >> 6, nrb = (a.r.E + nwv) / nwv, t0 = 8 * (blockIdx.x / nrb), r0 = blockIdx.x % nrb * nwv, nt = a.r.nb - t0 < 8 ? a.r.nb - t0 : 8;
+        if (nt == 1) pre_router_bf<1>(a, L, r0, t0, nt);
+        else if (nt == 2) pre_router_bf<2>(a, L, r0, t0, nt);
+        else if (nt <= 4) pre_router_bf<4>(a, L, r0, t0, nt);
+        else pre_router_bf<8>(a, L, r0, t0, nt);
+    }
+}
+__device__ __forceinline__ void pre_swiglu(const qwk_pre_args &a, float g, float up, uint32_t tok, uint32_t col) {
+    const float s = g / (1.0f + __expf(-g)), h = s * up;
+    const _Float16 hi = (_Float16)h, lo = (_Float16)__builtin_fmaf(s, up, -(float)hi); // (written out: left to the compiler, some of a lane's four tokens were rounded once and others twice)
+    const size_t o = ((size_t)tok * (a.topk + 1) + a.topk) * a.I + col;
+    a.H[o] = __builtin_bit_cast(uint16_t, hi);
+    a.H[o + a.hplane] = __builtin_bit_cast(uint16_t, lo);
+}
+// A block of a format of that family as raw registers, so that the blocks of two formats can be on their way at once
+template <int F> __device__ __forceinline__ void pre_load(const uint8_t *p, uint32_t (&r)[32]) {
+    typename qw_small_blk<F>::C c;
+    c.load(p, qw_lane() & 3);
+    __builtin_memcpy(r, &c, sizeof c);
+}
+template <int F> __device__ __forceinline__ f4 pre_mac(const uint32_t (&r)[32], const u2 *tab, const qw_afrag_small &af, uint32_t kg) {
+    typename qw_small_blk<F>::C c;
+    __builtin_memcpy(&c, r, sizeof c);
+    c.transpose();
+    return qw_small_blk<F>::mac(c, tab, af, kg);
+}
+#define QW_PRE_FORMATS(DO) case 12: DO(12); break; case 13: DO(13); break; case 14: DO(14); break; case 23: DO(23); break; case 20: DO(20); break; case 1: DO(1); break; case 30: DO(30); break;
+// A tile of 8 gate + 8 up rows, a wave 256 values of K (Q8_0: 512). SH: QW_F_PACKED (tile-major IQ3_S), or 8, 12, 13, 14, 20, 23, 1, 30 (GGUF rows).
+// IQ3_S and Q8_0 sums are added as a wave with 512 values adds them (two blocks of IQ3_S, sixteen of Q8_0, one after the other), then in the order of K.
+template <int SH> __device__ __forceinline__ void pre_shared(const qwk_pre_args &a, uint32_t t, qw_pre_lds &L) {
+    const qwk_router_args &r = a.r;
+    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave();
+    const uint32_t nwv = SH == 8 ? r.D / 512 : blockDim.x >> 6; // the waves that take part
+    u4 *const x = L.x + wave * (SH == 8 ? 1024 : 512);
+    const qw_afrag_small af = {x, n & ((1u << a.sh) - 1), a.sh};
+    f4 g = {0, 0, 0, 0};
+    if constexpr (SH == 8) {
+        if (wave < nwv) {
+            qw_chunk<8, 16> c;
+            qw_pre_x x0, x1;
+            c.load((lane < 32 ? a.Wg : a.Wu) + ((size_t)8 * t + ((lane >> 2) & 7)) * a.rbg + wave * (16 * 34), lane & 3);
+            x0.load(r, 512 * wave);
+            x1.load(r, 512 * wave + 256);
+            x0.store(x, r.nb, a.sh);
+            x1.store(x + (32 << a.sh), r.nb, a.sh);
+            __builtin_amdgcn_wave_barrier(); // (a wave's LDS operations complete in order)
             c.transpose();
-            c.mac_lean(lut, af, ci * CH * C::BLK_K, kg, acc);
-            part[wave * 64 + lane] = acc;
+            c.mac(nullptr, af, 0, kg, g);
+            if (wave) ((f4 *)x)[lane] = g;
         }
     } else {
-        // the table and the activations behind the weights, all awaited once: one memory round trip before the barrier
-        QW_PSTAMP(2);
-        if (qw_has_lut(F)) qw_lut_copy_issue(lut, (const u2 *)a.glut);
-        qw_stage_x_issue(xf, a.x, a.D, a.D, a.nbr);
-        QW_PSTAMP(3);
-        qw_lds_arrive();
-        QW_PSTAMP(4);
-        __syncthreads();
-        QW_PSTAMP(5);
-        if (on) {
-            c.transpose();
-            const qw_afrag_lds af = {xf, n};
-            c.mac_lean(lut, af, ci * CH * C::BLK_K, kg, acc);
-            part[wave * 64 + lane] = acc;
+        qw_pre_x xv;
+        typename qw_small_blk<SH>::C c;
+        if constexpr (SH == QW_F_PACKED) c.load(a.Wg + (size_t)t * a.rbg + wave * qw_small_blk<SH>::BYTES, lane);
+        else c.load((lane < 32 ? a.Wg : a.Wu) + ((size_t)8 * t + ((lane >> 2) & 7)) * a.rbg + wave * qw_small_blk<SH>::BYTES, lane & 3);
+        xv.load(r, 256 * wave);
+        if constexpr (SH == QW_F_PACKED) { // the table, a unit a thread or four (a few by several threads)
+            const uint32_t few = blockDim.x < 256 ? 4 : 1;
+            for (uint32_t i = 0; i < few; i++) ((u4 *)L.tab)[(threadIdx.x + 64 * i) & 255] = ((const u4 *)a.ctab)[(threadIdx.x + 64 * i) & 255];
+            if (threadIdx.x < 16) qw_small_signs(L.tab, threadIdx.x);
         }
-        QW_PSTAMP(6);
+        if constexpr (SH == 20 || SH == 23) qw_kq_tab_build((uint32_t *)L.tab);
+        xv.store(x, r.nb, a.sh);
+        if constexpr (SH == QW_F_PACKED || SH == 20 || SH == 23) __syncthreads();
+        else __builtin_amdgcn_wave_barrier();
+        c.transpose();
+        if constexpr (SH == QW_F_PACKED) {
+            f4 sub[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+            qw_small_iq3_steps<0>(c.s[0], L.tab, af, kg, sub);
+            ((f4 *)x)[lane] = sub[0] + sub[1];
+            ((float *)x)[256 + lane] = c.s[0].d;
+        } else {
+            g = qw_small_blk<SH>::mac(c, L.tab, af, kg);
+            if (wave) ((f4 *)x)[lane] = g;
+        }
     }
     __syncthreads();
-    QW_PSTAMP(7);
-    if (!on || ci != 0) return;
-    acc = part[wave * 64 + lane];
-    for (uint32_t i = 1; i < cpr; i++) acc += part[(wave + i) * 64 + lane]; // chunk order
+    if (wave) return;
+    if constexpr (SH == QW_F_PACKED) { // (nwv is even: D is a multiple of 512)
+        for (uint32_t q = 0; q < nwv; q += 2) {
+            const f4 *p0 = (const f4 *)L.x + q * 512, *p1 = p0 + 512;
+            const f4 s0 = p0[lane], s1 = p1[lane];
+            const float d0 = ((const float *)p0)[256 + lane], d1 = ((const float *)p1)[256 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float p = __builtin_fmaf(d1, s1[i], d0 * s0[i]);
+                g[i] = q ? g[i] + p : p;
+            }
+        }
+    } else
+        for (uint32_t q = 1; q < nwv; q++) g += ((const f4 *)L.x)[q * (SH == 8 ? 1024 : 512) + lane];
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++) {
-        const float up = __shfl_xor(acc[j], 8), g = acc[j];
         const uint32_t tok = 4 * kg + j;
-        if (n < 8 && tok < a.nbr) {
-            const float h = g / (1.0f + __expf(-g)) * up;
-            const _Float16 hi = (_Float16)h, lo = (_Float16)(h - (float)hi);
-            const size_t o = ((size_t)tok * (K + 1) + K) * a.I + 8 * tile + n;
-            a.H[o] = __builtin_bit_cast(uint16_t, hi);
-            a.H[o + a.hplane] = __builtin_bit_cast(uint16_t, lo);
-        }
+        const float up = __shfl_xor(g[j], 8); // (rows 8 .. 15 are the up rows)
+        if (tok < r.nb && n < 8) pre_swiglu(a, g[j], up, tok, 8 * t + n);
     }
-    QW_PSTAMP(8);
 }
-#define QW_PRE(WF, F, CH, NAME)                                                                          \
-    extern "C" __global__ __launch_bounds__(QW_WG) void NAME(qwk_pre_args a) {                           \
-        __shared__ struct { u2 lut[qw_has_lut(F) ? QW_LUT_ENTRIES : 1]; u4 xf[QW_XF_MAXK * 2]; f4 part[(QW_WG / 64) * 64]; } L; \
-        QW_DSTAMP(3);                                                                                   \
-        QW_PSTAMP(0);                                                                                   \
-        if (blockIdx.x < a.nrouter) {                                                                   \
-            if (WF == 1) pre_router_mfma(a.r, L.xf, L.part);                                            \
-            else pre_router<WF>(a, L.xf);                                                               \
-            QW_DSTAMP(4);                                                                               \
-        }                                                                                               \
-        else if (F != 0) { pre_shared<F ? F : 8, CH>(a, L.lut, L.xf, L.part); QW_DSTAMP(5); }            \
+// Two formats of that family: a gate tile and an up tile of 16 rows. D a multiple of 512: the waves of the first half take the gate rows, 512
+// values of K each, those of the second half the up rows; a wave reads one format. Otherwise a wave takes 256 values of both.
+struct qw_afrag_pre : qw_afrag_small {
+    const float *xs;
+    uint32_t kg;
+    __device__ __forceinline__ f4 sum32(uint32_t k) const { return *(const f4 *)(xs + (k >> 5) * 16 + 4 * kg); }
+};
+// The wave's part in one format: blocks 2 part and 2 part + 1 of its rows (p: where they start) times x, which the part's two waves share
+// and of which each brings one block.
+template <int F> __device__ __forceinline__ f4 pre_part(const qwk_pre_args &a, const uint8_t *p, uint32_t part, uint32_t up, u4 *x, float *xs, qw_pre_lds &L) {
+    typedef qw_small_blk<F> B;
+    const uint32_t lane = qw_lane(), kg = lane >> 4, live = 1u << a.sh;
+    typename B::C c[2];
+    qw_pre_x xv;
+#pragma unroll
+    for (int h = 0; h < 2; h++) c[h].load(p + h * B::BYTES, lane & 3);
+    xv.load(a.r, 512 * part + 256 * up);
+    if constexpr (F == 20 || F == 23) qw_kq_tab_build((uint32_t *)L.tab, lane, 64); // (every wave of such a format all of it: the others may not)
+    xv.store(x + (up ? 32 << a.sh : 0), a.r.nb, a.sh);
+    __syncthreads();
+    qw_afrag_pre af;
+    af.x = x, af.m = lane & 15 & (live - 1), af.sh = a.sh, af.xs = xs, af.kg = kg;
+    if constexpr (qw_kq<F>::HAS_MIN) { // sums of 32 activations, in index order
+        for (uint32_t i = lane; i < 16 * live; i += 64) {
+            const uint32_t ch = i >> a.sh, m = i & (live - 1);
+            const qw_afrag_small one = {x, m, a.sh};
+            float sum = 0;
+#pragma unroll
+            for (uint32_t f = 0; f < 4; f++) {
+                const h8 v = one.at8(32 * ch + 8 * f);
+#pragma unroll
+                for (int e = 0; e < 8; e++) sum += (float)v[e];
+            }
+            xs[ch * 16 + m] = sum;
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    f4 acc = {0, 0, 0, 0};
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        c[h].transpose();
+#pragma unroll
+        for (int i = 0; i < B::NB; i++) qw_kq_block<F>(c[h].b[i], (const uint32_t *)L.tab, af, 256 * h + qw_kq<F>::BLK_K * i, kg, acc);
+    }
+    return acc;
+}
+__device__ __forceinline__ void pre_pair(const qwk_pre_args &a, uint32_t t, qw_pre_lds &L) {
+    const qwk_router_args &r = a.r;
+    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave();
+    f4 g = {0, 0, 0, 0}, u = {0, 0, 0, 0};
+    const uint32_t row = 16 * t + (lane >> 2);
+    if (r.D % 512 == 0) {
+        const uint32_t np = r.D / 512, up = wave >= np, part = up ? wave - np : wave, f = up ? a.fu : a.fg;
+        const uint8_t *p = (up ? a.Wu : a.Wg) + (size_t)row * (up ? a.rbu : a.rbg);
+#define QW_DO(F) g = pre_part<F>(a, p + 2 * part * qw_small_blk<F>::BYTES, part, up, L.x + part * 1024, L.xs[wave], L)
+        switch (f) { QW_PRE_FORMATS(QW_DO) }
+#undef QW_DO
+        __syncthreads(); // (the part's other wave may still read the activations)
+        ((f4 *)L.x)[wave * 64 + lane] = g;
+        __syncthreads();
+        if (wave) return;
+        u = ((const f4 *)L.x)[np * 64 + lane];
+        for (uint32_t q = 1; q < np; q++) g += ((const f4 *)L.x)[q * 64 + lane], u += ((const f4 *)L.x)[(np + q) * 64 + lane];
+    } else {
+        u4 *const x = L.x + wave * 512;
+        const qw_afrag_small af = {x, n & ((1u << a.sh) - 1), a.sh};
+        qw_pre_x xv;
+        uint32_t rg[32], ru[32];
+#define QW_DO(F) pre_load<F>(a.Wg + (size_t)row * a.rbg + wave * qw_small_blk<F>::BYTES, rg)
+        switch (a.fg) { QW_PRE_FORMATS(QW_DO) }
+#undef QW_DO
+#define QW_DO(F) pre_load<F>(a.Wu + (size_t)row * a.rbu + wave * qw_small_blk<F>::BYTES, ru)
+        switch (a.fu) { QW_PRE_FORMATS(QW_DO) }
+#undef QW_DO
+        xv.load(r, 256 * wave);
+        qw_kq_tab_build((uint32_t *)L.tab);
+        xv.store(x, r.nb, a.sh);
+        __syncthreads();
+#define QW_DO(F) g = pre_mac<F>(rg, L.tab, af, kg)
+        switch (a.fg) { QW_PRE_FORMATS(QW_DO) }
+#undef QW_DO
+#define QW_DO(F) u = pre_mac<F>(ru, L.tab, af, kg)
+        switch (a.fu) { QW_PRE_FORMATS(QW_DO) }
+#undef QW_DO
+        if (wave) ((f4 *)x)[lane] = g, ((f4 *)x)[64 + lane] = u;
+        __syncthreads();
+        if (wave) return;
+        for (uint32_t q = 1; q < blockDim.x >> 6; q++) g += ((const f4 *)L.x)[q * 512 + lane], u += ((const f4 *)L.x)[q * 512 + 64 + lane];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++)
+        if (4 * kg + j < r.nb) pre_swiglu(a, g[j], u[j], 4 * kg + j, 16 * t + n);
+}
+template <int SH> __device__ __forceinline__ void pre_shared_any(const qwk_pre_args &a, uint32_t t, qw_pre_lds &L) {
+    if constexpr (SH == QW_F_RT) { // formats a.fg and a.fu, one of 1, 12, 13, 14, 20, 23, 30 each
+        if (a.fg == a.fu) {
+#define QW_DO(F) pre_shared<F>(a, t, L)
+            switch (a.fg) { QW_PRE_FORMATS(QW_DO) }
+#undef QW_DO
+        } else pre_pair(a, t, L);
+    } else if constexpr (SH != 0) pre_shared<SH>(a, t, L);
+}
+#define QW_PRE(WF, SH, NAME)                                                                             \
+    extern "C" __global__ __launch_bounds__(64 * QW_PRE_WAVES) void NAME(qwk_pre_args a) {               \
+        __shared__ qw_pre_lds L;                                                                         \
+        if (blockIdx.x < a.nrouter) pre_router_any<WF>(a, L);                                            \
+        else pre_shared_any<SH>(a, blockIdx.x - a.nrouter, L);                                           \
     }
 #if QW_IN_PART(2)
-QW_PRE(1, 0, 1, qwk_pre_w1) QW_PRE(30, 0, 1, qwk_pre_w30)
-QW_PRE(1, 121, 2, qwk_pre_w1_s121_c2) QW_PRE(30, 121, 2, qwk_pre_w30_s121_c2) QW_PRE(1, 8, 16, qwk_pre_w1_s8_c16) QW_PRE(30, 8, 16, qwk_pre_w30_s8_c16)
-#endif
-// The same front launch for a shared expert whose gate/up rows are in the K-quant / IQ4 / plain family: the binary16
-// router on the first workgroups, the multi-format product with SwiGLU (qwk_qmvm_swiglu's work) on those after them.
-#if QW_IN_PART(2)
-extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_pre_w1_kq(qwk_prekq_args a) {
-    __shared__ qw_swiglu_lds L;
-    if (blockIdx.x < a.nrouter) pre_router_mfma(a.r, L.xf, L.red);
-    else qmvm_swiglu_body(a.m, L, blockIdx.x - a.nrouter, gridDim.x - a.nrouter);
+QW_PRE(1, 0, qwk_pre_w1) QW_PRE(1, QW_F_PACKED, qwk_pre_w1_s121) QW_PRE(1, 8, qwk_pre_w1_s8) QW_PRE(1, QW_F_RT, qwk_pre_w1_kq)
+QW_PRE(30, 0, qwk_pre_w30) QW_PRE(30, QW_F_PACKED, qwk_pre_w30_s121) QW_PRE(30, 8, qwk_pre_w30_s8) QW_PRE(30, QW_F_RT, qwk_pre_w30_kq)
+// the shared expert's part alone (the logits given by the caller, or beside the router on another stream)
+extern "C" __global__ __launch_bounds__(64 * QW_PRE_WAVES) void qwk_qmvm_swiglu(qwk_pre_args a) {
+    __shared__ qw_pre_lds L;
+    pre_shared_any<QW_F_RT>(a, blockIdx.x, L);
 }
 #endif
 

@@ -33,13 +33,18 @@ struct qw_afrag_kq {
     __device__ __forceinline__ f4 sum32(uint32_t k) const { return *(const f4 *)(xs + (k >> 5) * 16 + 4 * kg); } // tokens 4 kg .. 4 kg + 3
 };
 
-__constant__ const int8_t qw_iq4nl_values[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
-__device__ __forceinline__ void qw_kq_tab_build(uint32_t *tab) {
-    for (uint32_t i = threadIdx.x; i < QW_KQ_TAB; i += blockDim.x) {
-        const _Float16 lo = (_Float16)(float)qw_iq4nl_values[i & 15], hi = (_Float16)(float)qw_iq4nl_values[i >> 4];
+// -127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113, from literals (an array would be a load)
+__device__ __forceinline__ float qw_iq4nl_value(uint32_t i) {
+    const uint32_t lo = __builtin_amdgcn_perm(0xf6eaddcfu, 0xbfad9881u, i & 7), hi = __builtin_amdgcn_perm(0x71594535u, 0x26190d01u, i & 7);
+    return (float)(int8_t)(i & 8 ? hi : lo);
+}
+__device__ __forceinline__ void qw_kq_tab_build(uint32_t *tab, uint32_t first, uint32_t step) {
+    for (uint32_t i = first; i < QW_KQ_TAB; i += step) {
+        const _Float16 lo = (_Float16)qw_iq4nl_value(i & 15), hi = (_Float16)qw_iq4nl_value(i >> 4);
         tab[i] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | (uint32_t)__builtin_bit_cast(uint16_t, hi) << 16;
     }
 }
+__device__ __forceinline__ void qw_kq_tab_build(uint32_t *tab) { qw_kq_tab_build(tab, threadIdx.x, blockDim.x); } // by the workgroup
 
 // Four bytes (each < 256) to four binary16 integers minus bias: bytes b0 b1 -> first pair, b2 b3 -> second pair.
 __device__ __forceinline__ u2 qw_bytes_h4(uint32_t v, float bias) {

@@ -26,6 +26,8 @@ struct qw_afrag_small {
     __device__ __forceinline__ h4 lo4(uint32_t) const { return h4{}; }
 };
 
+// The sign masks behind the table: nibble s (bit j = the sign of value j)
+__device__ __forceinline__ void qw_small_signs(u2 *tab, uint32_t s) { tab[512 + s] = u2{(s & 1) << 15 | (s & 2) << 30, (s & 4) << 13 | (s & 8) << 28}; }
 // Eight values of step J of an IQ3_S block from the 4 KB table: the magnitudes of two codebook entries, their signs put in by
 // masks (bit j of a nibble is the sign of value j), then the sub-block factor, as in qw_iq3_step.
 template <int J> __device__ __forceinline__ h8 qw_small_iq3(const qw_iq3_slice &s, const u2 *tab) {
@@ -45,6 +47,48 @@ template <int J> __device__ __forceinline__ void qw_small_iq3_steps(const qw_iq3
     }
 }
 
+// A block of Q4_K or Q5_K with the factors as integers, as in qw_chunk<QW_F_PACKED_Q4K>: d (q - C) sc + (C d sc - dmin m), C half of
+// the range of q, (q - C) sc exact in binary16. The sums of 32 activations are made by the lane that brings them to the binary32
+// matrix instruction. (Scale and minimum applied to each step's binary32 result, the sums by a matrix instruction a step, take twice
+// the vector instructions. Two steps an accumulator: errors to float64 as there, Q4_K 1.07e-7 and 1.07e-7 of a product of 2048 values,
+// Q5_K 0.96e-7 and 0.99e-7; all eight in one: 1.14e-7 and 1.05e-7.)
+template <int F, int S> __device__ __forceinline__ void qw_small_k45_steps(const qw_kq<F> &b, const qw_afrag_small &af, uint32_t kg, const uint32_t (&sc)[2], f4 (&sub)[4]) {
+    if constexpr (S < 8) {
+        constexpr int sh = 4 * (S & 1), q0 = F == 13 ? 6 : 4;
+        uint32_t lo = (b.r[q0 + 2 * (S >> 1)] >> sh) & 0x0f0f0f0fu, hi = (b.r[q0 + 1 + 2 * (S >> 1)] >> sh) & 0x0f0f0f0fu;
+        if constexpr (F == 13) lo |= ((b.r[4] >> S) & 0x01010101u) << 4, hi |= ((b.r[5] >> S) & 0x01010101u) << 4;
+        const h2 f = qw_byte_h2<(S & 3)>(sc[S >> 2]);
+        const h8 q = qw_bytes_h8(lo, hi, F == 13 ? 16.0f : 8.0f);
+        u4 w = __builtin_bit_cast(u4, q);
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, (uint32_t)w[i]) * f);
+        sub[S & 3] = qw_mfma(af.at8(32 * S + 8 * kg), __builtin_bit_cast(h8, w), sub[S & 3]);
+        qw_small_k45_steps<F, S + 1>(b, af, kg, sc, sub);
+    }
+}
+template <int F> __device__ __forceinline__ void qw_small_k45(const qw_kq<F> &b, const qw_afrag_small &af, uint32_t kg, f4 &acc) {
+    uint32_t sc[2], mn[2];
+    qw_k4_scales(b.r + 1, sc, mn);
+    f4 sub[4] = {};
+    qw_small_k45_steps<F, 0>(b, af, kg, sc, sub);
+    const float d = qw_h2f((uint16_t)b.r[0]), dm = qw_h2f((uint16_t)(b.r[0] >> 16));
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(d, (sub[0][i] + sub[1][i]) + (sub[2][i] + sub[3][i]), acc[i]);
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        float xs = 0;
+        const h2 one = {(_Float16)1.0f, (_Float16)1.0f};
+#pragma unroll
+        for (int f = 0; f < 4; f++) {
+            const u4 v = __builtin_bit_cast(u4, af.at8(32 * (4 * j + kg) + 8 * f));
+#pragma unroll
+            for (int i = 0; i < 4; i++) xs = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, (uint32_t)v[i]), one, xs, false);
+        }
+        const float c = __builtin_fmaf((F == 13 ? 16.0f : 8.0f) * d, (float)((sc[j] >> (8 * kg)) & 255), -dm * (float)((mn[j] >> (8 * kg)) & 255));
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xs, c, acc, 0, 0, 0);
+    }
+}
+
 // 256 values of K of one tile as the wave loads and multiplies them.
 template <int F> struct qw_small_blk { // Q4_K, Q5_K, Q6_K, IQ4_XS; eight blocks of IQ4_NL, binary16, bfloat16
     static constexpr int NB = qw_kq<F>::BLK_K == 256 ? 1 : 8;
@@ -54,7 +98,7 @@ template <int F> struct qw_small_blk { // Q4_K, Q5_K, Q6_K, IQ4_XS; eight blocks
         f4 acc = {0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < NB; i++) {
-            if constexpr (qw_kq<F>::HAS_MIN) qw_kq_block_af<F>(c.b[i], (const uint32_t *)tab, af, qw_kq<F>::BLK_K * i, kg, acc);
+            if constexpr (qw_kq<F>::HAS_MIN) qw_small_k45<F>(c.b[i], af, kg, acc);
             else qw_kq_block<F>(c.b[i], (const uint32_t *)tab, af, qw_kq<F>::BLK_K * i, kg, acc);
         }
         return acc;
@@ -113,10 +157,7 @@ template <int F, int XN> __device__ __forceinline__ f4 qmvs_part(const qwk_qmvm_
         if (many)
 #pragma unroll
             for (uint32_t i = 1; i < 4; i++) ((u4 *)tab)[(threadIdx.x + i * 64) & 255] = te[i];
-        if (threadIdx.x < 16) {
-            const uint32_t s = threadIdx.x;
-            tab[512 + s] = u2{(s & 1) << 15 | (s & 2) << 30, (s & 4) << 13 | (s & 8) << 28};
-        }
+        if (threadIdx.x < 16) qw_small_signs(tab, threadIdx.x);
     }
     if constexpr (iq4) qw_kq_tab_build((uint32_t *)tab);
 #pragma unroll

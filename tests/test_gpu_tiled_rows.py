@@ -14,7 +14,7 @@ TOL = 2e-3  # binary16 results of a layer (half an ulp is 4.9e-4 of a value) aga
 
 @pytest.mark.parametrize("nb", [1, 2, 3, 5, 8, 9, 16])
 @pytest.mark.parametrize("fgu,fd,fsh,fshd,D,I,E,K", [
-    (8, 8, 8, 8, 2048, 512, 16, 10), (8, 8, 21, 21, 512, 256, 4, 2), (8, 21, 8, 8, 2560, 512, 8, 4), (12, 8, 12, 8, 1024, 256, 33, 8),
+    (8, 8, 8, 8, 2048, 512, 16, 10), (8, 8, 8, 21, 512, 256, 4, 2), (8, 21, 8, 8, 2560, 512, 8, 4), (12, 8, 12, 8, 1024, 256, 33, 8),
     (12, 14, 12, 14, 2048, 512, 80, 10), (12, 14, 8, 8, 1536, 256, 208, 6), (12, 12, 12, 12, 512, 256, 8, 8)])
 def test_tiled_rows_equal_gguf_rows(gpu, oracle, nb, fgu, fd, fsh, fshd, D, I, E, K):
     rng = np.random.default_rng(fgu * 100 + fd * 10 + D + nb)
