@@ -16,6 +16,7 @@
 #include <hip/hip_runtime_api.h>
 #include <pthread.h>
 #include <stdarg.h>
+#include <stddef.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -95,10 +96,15 @@ typedef struct {
     bool last_of_dispatch;
     bool side; // independent of the launches before it in the batch: runs on the side stream, beside them
     bool join; // needs the side stream's results: the main stream waits for them first
+    // Outputs that the kernel can also write to a shadow: their uses, and where in the record the second pointers and the
+    // qwk_fin lie (host_outputs)
+    int ndirect, direct_use[4];
+    unsigned short direct_at[4], fin_at;
 } qw_launch;
 
 // A buffer as a dispatch binds it, and the bytes it may touch. whole: every byte of [lo, hi) is written, whatever they held.
-typedef struct { qw_hbuf *b; bool out, whole; size_t lo, hi; } qw_use;
+// direct: the kernel writes the shadow too.
+typedef struct { qw_hbuf *b; bool out, whole, direct; size_t lo, hi; } qw_use;
 
 // What the host and the device exchange about a batch in flight beside its data: pinned, one per batch at a time. t0 / t1:
 // the device clock at the start and the end of every submitted segment (0: not taken); done, copied: 1 once its kernels
@@ -133,6 +139,7 @@ struct qw_batch {
     int io_idx;
     hipEvent_t ev[2 * 9]; // profiled batches, and those for which no slot was free: start/stop per submitted segment (end + at most 8 flushes)
     bool events;
+    bool fin;            // the last launch raises the flag itself
     hipEvent_t *pev;      // profiling: 2 events per launch
     int npev;
     // Work deferred from one dispatch of a layer to the next (the reference's front part also computes the shared
@@ -990,7 +997,7 @@ static bool bind_ptr(qw_batch *b, unsigned index, size_t need, bool out, const c
         b->capuse = b->capuse ? 2 * b->capuse : 64;
         b->use = realloc(b->use, sizeof *b->use * (size_t)b->capuse);
     }
-    b->use[b->nuse++] = (qw_use){h, out, false, off, off + need};
+    b->use[b->nuse++] = (qw_use){.b = h, .out = out, .lo = off, .hi = off + need};
     return true;
 }
 // The same for an output of which the dispatch writes every byte of the range: what the range held before does not matter.
@@ -1005,7 +1012,7 @@ static bool bind_bytes(qw_batch *b, unsigned index, void *dst, size_t len, const
     return true;
 }
 
-_Static_assert(sizeof(qwk_pre_args) <= QW_MAX_ARGS && sizeof(qwk_gu_args) <= QW_MAX_ARGS && sizeof(qwk_dn_args) <= QW_MAX_ARGS && sizeof(qwk_qmv_args) <= QW_MAX_ARGS,
+_Static_assert(sizeof(qwk_pre_args) <= QW_MAX_ARGS && sizeof(qwk_gu_args) <= QW_MAX_ARGS && sizeof(qwk_dn_args) <= QW_MAX_ARGS && sizeof(qwk_qmv_args) <= QW_MAX_ARGS && sizeof(qwk_qmvm_args) <= QW_MAX_ARGS,
                "a kernel argument record is larger than the launch record's copy of it");
 
 static bool add_launch(qw_batch *b, const char *fname, unsigned gx, unsigned bx, const void *args, size_t argsz) {
@@ -1118,6 +1125,14 @@ static bool launch_qmvs(qw_batch *b, qwk_qmvm_args *a, unsigned tiles) {
     b->l[b->nl - 1].lds = qmvs_lds(a);
     return true;
 }
+// The launch just added writes its results as float to n buffers, bound as uses[]; where a copy of them may go.
+static bool direct_slots(qw_batch *b, int n, const int *uses, size_t yh_at, size_t fin_at) {
+    qw_launch *l = &b->l[b->nl - 1];
+    l->ndirect = n;
+    l->fin_at = (unsigned short)fin_at;
+    for (int j = 0; j < n; j++) l->direct_use[j] = uses[j], l->direct_at[j] = (unsigned short)(yh_at + (size_t)j * sizeof(void *));
+    return true;
+}
 // hw: the buffers the matrices lie in (NULL, a shared expert's rows: the persistent kernel, no tile-major copies)
 #define QW_Q6_PACK_MIN_ROWS 16384u
 static bool launch_qmvm(qw_batch *b, qwk_qmvm_args *a, qw_hbuf *const *hw) {
@@ -1157,6 +1172,7 @@ static bool tr_qmvm(qw_batch *b) { // src/engine.c:752-771: 0..3 W, 4 x, 5..8 y,
     if (b->buf[4].h && b->buf[4].off % 16) return fail(b, "qmv_ggm: x offset %zu is not 16-byte aligned", b->buf[4].off);
     if (!bind_ptr(b, 4, ((size_t)(a.nb - 1) * a.xstride + a.K) * 2, false, "x", (void **)&a.x)) return false;
     uint32_t total = 0;
+    int uses[4];
     for (int j = 0; j < p->nmat; j++) {
         a.N[j] = in.N[j], a.fmt[j] = (uint32_t)p->gf[j], a.rowbytes[j] = (uint32_t)fmt_rb(p->gf[j], p->K), a.ystride[j] = in.N[j];
         if (in.off[j] != total) return fail(b, "qmv_ggm: off[%d] = %u, expected %u (rows of the matrices before it)", j, in.off[j], total);
@@ -1165,10 +1181,11 @@ static bool tr_qmvm(qw_batch *b) { // src/engine.c:752-771: 0..3 W, 4 x, 5..8 y,
         if (b->buf[j].h && b->buf[j].off % 16) return fail(b, "qmv_ggm: offset %zu of matrix %d is not 16-byte aligned", b->buf[j].off, j);
         if (!bind_ptr(b, (unsigned)j, (size_t)a.N[j] * a.rowbytes[j], false, "W", (void **)&a.W[j]) ||
             !bind_whole(b, 5u + (unsigned)j, (size_t)a.nb * a.N[j] * (a.yfloat ? 4 : 2), "y", &a.y[j])) return false;
+        uses[j] = b->nuse - 1;
     }
     if (in.total != total) return fail(b, "qmv_ggm: total %u, the matrices have %u rows", in.total, total);
     qw_hbuf *hm[4] = {b->buf[0].h, b->buf[1].h, b->buf[2].h, b->buf[3].h};
-    return launch_qmvm(b, &a, hm);
+    return launch_qmvm(b, &a, hm) && (!a.yfloat || direct_slots(b, p->nmat, uses, offsetof(qwk_qmvm_args, yh), offsetof(qwk_qmvm_args, fin)));
 }
 
 static bool tr_qmv(qw_batch *b) { // src/engine.c:717-723: 0 W, 3 x, 4 y, 5 {N, xstride, ystride, pad}
@@ -1184,9 +1201,10 @@ static bool tr_qmv(qw_batch *b) { // src/engine.c:717-723: 0 W, 3 x, 4 y, 5 {N, 
         if (!bind_ptr(b, 0, (size_t)m.N[0] * m.rowbytes[0], false, "W", (void **)&m.W[0]) ||
             !bind_ptr(b, 3, ((size_t)(m.nb - 1) * m.xstride + m.K) * 2, false, "x", (void **)&m.x) ||
             !bind_ptr(b, 4, ((size_t)(m.nb - 1) * m.ystride[0] + m.N[0]) * (m.yfloat ? 4 : 2), true, "y", &m.y[0])) return false;
-        b->use[b->nuse - 1].whole = m.nb == 1 || m.ystride[0] == m.N[0];
+        const int use = b->nuse - 1;
+        b->use[use].whole = m.nb == 1 || m.ystride[0] == m.N[0];
         qw_hbuf *hm[4] = {b->buf[0].h};
-        return launch_qmvm(b, &m, hm);
+        return launch_qmvm(b, &m, hm) && (!m.yfloat || !b->use[use].whole || direct_slots(b, 1, &use, offsetof(qwk_qmvm_args, yh), offsetof(qwk_qmvm_args, fin)));
     }
     qwk_qmv_args a = {.N = a4[0], .K = (uint32_t)p->K, .rowbytes = (uint32_t)p->RB, .xstride = a4[1], .ystride = a4[2], .nb = (uint32_t)p->NB, .yfloat = (uint32_t)p->yfloat,
                       .glut = glut(b->g)};
@@ -1199,7 +1217,8 @@ static bool tr_qmv(qw_batch *b) { // src/engine.c:717-723: 0 W, 3 x, 4 y, 5 {N, 
     b->allow_released = false;
     if (!bound || !bind_ptr(b, 3, ((size_t)(a.nb - 1) * a.xstride + a.K) * 2, false, "x", (void **)&a.x) ||
         !bind_ptr(b, 4, ((size_t)(a.nb - 1) * a.ystride + a.N) * (a.yfloat ? 4 : 2), true, "y", &a.y)) return false;
-    b->use[b->nuse - 1].whole = a.nb == 1 || a.ystride == a.N;
+    const int use = b->nuse - 1;
+    const bool direct = (b->use[use].whole = a.nb == 1 || a.ystride == a.N) && a.yfloat;
     char fn[48];
     int F = p->F;
     if (F == 21 && p->K <= 2560 && a.N % 16 == 0) { // tile-major copy of the rows, made at first use
@@ -1211,7 +1230,8 @@ static bool tr_qmv(qw_batch *b) { // src/engine.c:717-723: 0 W, 3 x, 4 y, 5 {N, 
     if (!p->valu) {
         qwk_qmvm_args m = {.K = a.K, .xstride = a.xstride, .nb = a.nb, .yfloat = a.yfloat, .nmat = 1, .x = a.x, .W = {a.W}, .y = {a.y}, .N = {a.N}, .fmt = {(uint32_t)F},
                            .rowbytes = {a.rowbytes}, .ystride = {a.ystride}, .ntiles = {a.ntiles}};
-        if (qmvs_fits(b->g, &m, a.ntiles, p->K > 2560)) return launch_qmvs(b, &m, a.ntiles);
+        if (qmvs_fits(b->g, &m, a.ntiles, p->K > 2560))
+            return launch_qmvs(b, &m, a.ntiles) && (!direct || direct_slots(b, 1, &use, offsetof(qwk_qmvm_args, yh), offsetof(qwk_qmvm_args, fin)));
     }
     if (p->valu) { // the VALU GEMV, for measurement against the matrix-core form
         if (F != QW_F_PACKED || p->K % 512 || p->NB > 4) return fail(b, "qmv_gg: the VALU form needs packed IQ3_S weights, K a multiple of 512 and NB <= 4");
@@ -1223,10 +1243,13 @@ static bool tr_qmv(qw_batch *b) { // src/engine.c:717-723: 0 W, 3 x, 4 y, 5 {N, 
         // few tiles: cut every tile's chunks over several waves, as far as the wave slots of the device allow
         const unsigned cpr = (unsigned)p->K / ((unsigned)fmt_qb(base) * (unsigned)ch), slots = (unsigned)b->g->ncu * QW_WAVES_GU;
         a.split = pick_split(cpr, a.ntiles, slots);
-        if (a.split > 1) return add_launch(b, intern(fn), umin((unsigned)b->g->ncu, cdiv(a.ntiles, QW_WAVES_GU / a.split)), 64 * QW_WAVES_GU, &a, sizeof a);
+        if (a.split > 1)
+            return add_launch(b, intern(fn), umin((unsigned)b->g->ncu, cdiv(a.ntiles, QW_WAVES_GU / a.split)), 64 * QW_WAVES_GU, &a, sizeof a) &&
+                   (!direct || direct_slots(b, 1, &use, offsetof(qwk_qmv_args, yh), offsetof(qwk_qmv_args, fin)));
     }
     a.split = 1;
-    return add_launch(b, intern(fn), persistent_grid(b->g, a.ntiles, QW_WAVES_GU), 64 * QW_WAVES_GU, &a, sizeof a);
+    return add_launch(b, intern(fn), persistent_grid(b->g, a.ntiles, QW_WAVES_GU), 64 * QW_WAVES_GU, &a, sizeof a) &&
+           (!direct || p->valu || direct_slots(b, 1, &use, offsetof(qwk_qmv_args, yh), offsetof(qwk_qmv_args, fin)));
 }
 
 static bool fill_router(qw_batch *b, qwk_router_args *a, unsigned iWr, unsigned iWsg, unsigned ix, unsigned ilg, uint32_t nbr) {
@@ -2325,6 +2348,35 @@ static void touched_range(const qw_batch *b, int first, const qw_hbuf *h, bool o
     if (*hi < *lo) *hi = *lo;
 }
 
+static bool carried_back(const qw_use *u) { return u->out && !u->b->device_only && u->b->host && !u->b->wrapped && u->b->size <= QW_HIP_BIG_OUT_BYTES; }
+// Before the last launches of a batch that the caller waits for: those whose kernels can write a shadow themselves do so
+// where nothing else of the batch writes that buffer, and if that leaves nothing to carry back, the last one raises the flag.
+static void host_outputs(qw_batch *b) {
+    if (!b->io || b->uses_sync) return;
+    for (int i = b->done_l; i < b->nl; i++) {
+        qw_launch *l = &b->l[i];
+        for (int d = 0; d < l->ndirect; d++) {
+            qw_use *u = &b->use[l->direct_use[d]];
+            if (!carried_back(u) || !u->b->pinned) continue;
+            int writers = 0;
+            for (int j = 0; j < b->nuse; j++) writers += b->use[j].out && b->use[j].b == u->b;
+            if (writers != 1) continue;
+            float *host = (float *)((char *)u->b->host + u->lo);
+            memcpy(l->args + l->direct_at[d], &host, sizeof host);
+            u->direct = true;
+        }
+    }
+    qw_launch *l = b->nl > b->done_l ? &b->l[b->nl - 1] : NULL;
+    if (!l || !l->ndirect) return;
+    for (int i = b->done_l; i < b->nl; i++)
+        if (b->l[i].side) return;
+    for (int j = 0; j < b->nuse; j++)
+        if (carried_back(&b->use[j]) && !b->use[j].direct) return;
+    const qwk_fin fin = {.t_done = (uint64_t *)&b->io->t1[b->nseg - 1], .flag = (uint32_t *)&b->io->copied, .count = b->g->io_count + b->io_idx};
+    memcpy(l->args + l->fin_at, &fin, sizeof fin);
+    b->fin = true;
+}
+
 // last: the caller waits for the batch at once, and its last launch also carries the outputs back (qw_batch_wait).
 static bool submit_segment(qw_batch *b, bool last) {
     qw_gpu *g = b->g;
@@ -2394,6 +2446,7 @@ static bool submit_segment(qw_batch *b, bool last) {
         up.a.t_done = (uint64_t *)&b->io->t0[seg];
         if (!io_launch(b, &up)) return false;
     }
+    if (last) host_outputs(b); // (the segment is counted above: its stamp is t1[seg])
     const int as_graph = graph_run(b, st);
     if (as_graph < 0) { b->failed = true; return false; }
     bool side_open = false;
@@ -2483,7 +2536,7 @@ static double batch_wait(qw_batch *b, bool ended) { // ended: submitted by qw_ba
         qw_hbuf *h = b->use[i].b;
         if (!b->use[i].out || h->mark == mark) continue;
         h->mark = mark;
-        if (h->device_only || !h->host || h->wrapped || h->size > QW_HIP_BIG_OUT_BYTES) continue;
+        if (!carried_back(&b->use[i]) || b->use[i].direct) continue;
         size_t lo, hi; // only what its dispatches may have written: the rest of the shadow is the host's own
         touched_range(b, i, h, true, &lo, &hi);
         if (hi <= lo) continue;
@@ -2495,8 +2548,8 @@ static double batch_wait(qw_batch *b, bool ended) { // ended: submitted by qw_ba
         else ok = HIPOK(g, hipMemcpyAsync(g->sync_host, g->sync + QW_SYNC_ERR_WORD, 4, hipMemcpyDeviceToHost, st));
     }
     if (ok && b->io) {
-        const volatile uint32_t *flag = &b->io->done;
-        if (ended || down.a.n) {
+        const volatile uint32_t *flag = b->fin ? &b->io->copied : &b->io->done;
+        if ((ended && !b->fin) || down.a.n) {
             flag = &b->io->copied;
             if (ended) down.a.t_enter = (uint64_t *)&b->io->t1[b->nseg - 1];
             down.a.flag = (uint32_t *)flag, down.a.flagval = 1;

@@ -27,6 +27,14 @@ typedef struct { /* dq_test: rows x K values to float */
     uint32_t K, rowbytes, rows, fmt; /* fmt: used by the kernel that serves the formats 1, 12, 13, 14, 20, 23, 30 */
 } qwk_dq_args;
 
+/* What the last launch of a batch does for the host when its own outputs are all that the host waits for (flag NULL: not
+ * asked for): the last workgroup to end writes the device clock and raises the flag. */
+typedef struct {
+    uint64_t *t_done; /* host */
+    uint32_t *flag;   /* host, set to 1 */
+    uint32_t *count;  /* device word, zero before and after the launch: workgroups that are done */
+} qwk_fin;
+
 typedef struct { /* dense matvec, y[b][row] = W[row] . x[b] */
     const uint8_t *W;
     const uint16_t *x; /* binary16 [nb][xstride] */
@@ -34,6 +42,8 @@ typedef struct { /* dense matvec, y[b][row] = W[row] . x[b] */
     uint32_t N, K, rowbytes, xstride, ystride, nb, yfloat, ntiles;
     const void *glut; /* the backend's pre-signed IQ3_S table in global memory (64 KB) */
     uint32_t split, pad; /* waves a tile's chunks are cut over (1 .. 6; the chunk count of a row is a multiple of it) */
+    float *yh;           /* host, may be NULL (always for binary16 results): a second place for y */
+    qwk_fin fin;
 } qwk_qmv_args;
 
 /* Dense matvec over up to four matrices that share the activations (kernels/qmv_ggm.metal:232-262; one matrix:
@@ -50,6 +60,8 @@ typedef struct {
     /* qwk_qmvs: the backend's IQ3_S table without signs; 2^sh >= nb; 16-byte units of LDS kept for a table */
     const void *ctab;
     uint32_t sh, tabu;
+    float *yh[4]; /* host, may be NULL (always for binary16 results): a second place for y[j] */
+    qwk_fin fin;
 } qwk_qmvm_args;
 
 /* SwiGLU of the shared expert when its gate/up rows went through the multi-format matvec: g, u float [nb][I] ->

@@ -257,6 +257,40 @@ extern "C" __global__ __launch_bounds__(256) void qwk_pack_nl(qwk_pack_args a) {
 #endif
 
 // ================================================================ dense matvec (kernels/qmv_gg.metal:17-39)
+// A result and its copy on the host. Stores of system scope go through the caches of the device to their memory, and have
+// arrived there when they are acknowledged. The results used to follow in a launch of their own (qwk_io), behind the product
+// instead of beside it; for a batch of one product that launch and its copy are a fifth of the whole. Measured, start of the
+// batch to its end on the host: 4096 x 2048 IQ3_S for one token 21.9 -> 20.8 us, 5127 x 2560 Q8_0 for seven 29.4 -> 24.8,
+// 131072 x 2048 Q6_K for four (2 MB back) at the end of 24 others 351 -> 340: 64 bytes a row of tile and token cross PCIe at
+// 35 GB/s where whole KBs (qwk_io) have 45, but while the product runs.
+__device__ __forceinline__ void qw_store_y(void *y, float *yh, bool f32, const qwk_fin &f, size_t i, float v) {
+    if (!f32) {
+        ((uint16_t *)y)[i] = qw_f2h(v);
+        return;
+    }
+    if (f.flag) __hip_atomic_store((float *)y + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    else ((float *)y)[i] = v;
+    if (yh) __hip_atomic_store(yh + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// The end of a workgroup in the last launch of a batch, by the wave that stored its results (qw_fin_wave) or by all of its
+// waves. What a launch with a flag stores it stores by qw_store_y, so that a wait for the stores is all that has to come
+// before the flag (a release would write the whole L2 back, once a workgroup: 1 us more at 256 of them).
+__device__ __forceinline__ void qw_fin_wave(const qwk_fin &f) {
+    if (!f.flag) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (qw_lane() == 0 && __hip_atomic_fetch_add(f.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+        __hip_atomic_store(f.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); // for the next batch
+        __hip_atomic_store(f.t_done, __builtin_amdgcn_s_memrealtime(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __hip_atomic_store(f.flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+__device__ __forceinline__ void qw_fin_wg(const qwk_fin &f) {
+    if (!f.flag) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this wave's stores,
+    __syncthreads();                                 // and everybody's
+    if (threadIdx.x < 64) qw_fin_wave(f);
+}
 // y[b][row] = sum_k W[row][k] x[b][k] for up to 16 activations; the weights are streamed once for all of them.
 // Tiles of 16 rows are dealt round-robin to the waves of a persistent grid; a row is CPR chunks of CH blocks.
 template <int F, int CH, bool XLDS> __device__ __forceinline__ void qmv_body(const qwk_qmv_args &a, u2 *lut, u4 *xf, f4 *red) {
@@ -278,10 +312,7 @@ template <int F, int CH, bool XLDS> __device__ __forceinline__ void qmv_body(con
 #pragma unroll
             for (uint32_t j = 0; j < 4; j++) {
                 const uint32_t tok = 4 * kg + j;
-                if (tok < a.nb) {
-                    if (a.yfloat) ((float *)a.y)[(size_t)tok * a.ystride + r] = acc[j];
-                    else ((uint16_t *)a.y)[(size_t)tok * a.ystride + r] = qw_f2h(acc[j]);
-                }
+                if (tok < a.nb) qw_store_y(a.y, a.yh, a.yfloat, a.fin, (size_t)tok * a.ystride + r, acc[j]);
             }
     };
     if (qw_has_lut(F)) qw_lut_copy_issue(lut, (const u2 *)a.glut);
@@ -329,6 +360,7 @@ template <int F, int CH, bool XLDS> __device__ __forceinline__ void qmv_body(con
     extern "C" __global__ __launch_bounds__(QW_WG_GU) void qwk_qmv_f##F##SFX(qwk_qmv_args a) {             \
         __shared__ struct { u2 lut[qw_has_lut(F) ? QW_LUT_ENTRIES : 1]; u4 xf[XLDS ? QW_XF_MAXK * 2 : 1]; f4 red[QW_WG_GU]; } L; /* table first: LDS address 0 */ \
         qmv_body<F, CH, XLDS>(a, L.lut, L.xf, L.red);                                                   \
+        qw_fin_wg(a.fin);                                                                               \
     }
 #if QW_IN_PART(0)
 QW_QMV(21, 2, true, _c2) QW_QMV(21, 1, true, _c1) QW_QMV(21, 1, false, _c1g)
@@ -365,11 +397,9 @@ template <int XN> __device__ __forceinline__ void qmvs_body(const qwk_qmvm_args 
 #pragma unroll
         for (uint32_t i = 0; i < 4; i++) {
             const uint32_t tok = 4 * kg + i;
-            if (tok < a.nb) {
-                if (a.yfloat) ((float *)a.y[j])[(size_t)tok * a.ystride[j] + r] = acc[i];
-                else ((uint16_t *)a.y[j])[(size_t)tok * a.ystride[j] + r] = qw_f2h(acc[i]);
-            }
+            if (tok < a.nb) qw_store_y(a.y[j], a.yh[j], a.yfloat, a.fin, (size_t)tok * a.ystride[j] + r, acc[i]);
         }
+    qw_fin_wave(a.fin);
 }
 #define QW_QMVS(XN)                                                                                  \
     extern "C" __global__ __launch_bounds__(1024) void qwk_qmvs_x##XN(qwk_qmvm_args a) {              \
@@ -403,10 +433,7 @@ template <int F, int NB> struct qmvm_tile {
 #pragma unroll
         for (uint32_t i = 0; i < 4; i++) {
             const uint32_t tok = 4 * kg + i;
-            if (tok < a.nb) {
-                if (a.yfloat) ((float *)a.y[j])[(size_t)tok * a.ystride[j] + r] = acc[i];
-                else ((uint16_t *)a.y[j])[(size_t)tok * a.ystride[j] + r] = qw_f2h(acc[i]);
-            }
+            if (tok < a.nb) qw_store_y(a.y[j], a.yh[j], a.yfloat, a.fin, (size_t)tok * a.ystride[j] + r, acc[i]);
         }
     }
 };
@@ -499,6 +526,7 @@ extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_qmvm(qwk_qmvm_args 
         }
         toff += a.ntiles[j];
     }
+    qw_fin_wg(a.fin);
 }
 #endif
 

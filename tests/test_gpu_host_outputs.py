@@ -1,0 +1,118 @@
+"""Results of a dense product that its kernel writes to the shadow itself (and, as the last launch of a batch, ends the batch
+with): after every batch the shadow holds the bytes that HBM holds, over each kernel that does so, and where the rule sends
+the results back by a launch of their own instead."""
+import numpy as np
+import pytest
+import torch
+
+import qwental_amd as q
+from qwental_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def env():
+    g = q.Gpu()
+    p = q.Path(g, 1024, 256, 64, 4, 16, device_scratch=True)
+    yield g, p
+    p.close()
+    g.close()
+
+
+def weights(g, rng, fmt, N, K):
+    raw = synth.matrix(rng, fmt, N, K)
+    buf = q.Buf(g, raw.nbytes, device_only=True)
+    buf.fill(raw)
+    return buf, q.Tensor(buf, fmt)
+
+
+def same(y):
+    """Shadow and HBM, bit for bit."""
+    return np.array_equal(y.view(np.uint32), y.read(dtype=np.uint32))
+
+
+# (type, rows, K, tokens): a workgroup a tile with one and several waves; the persistent kernels over whole and cut rows;
+# rows that do not fill a tile; IQ3_S beside the tile-major copy and past the staged K
+SHAPES = [(8, 17, 256, 1), (8, 5127, 2560, 7), (12, 100, 4096, 16), (14, 20000, 1024, 4), (14, 40000, 512, 3), (1, 9, 512, 5), (30, 30000, 768, 2),
+          (20, 24000, 1024, 16), (21, 4096, 2048, 1), (21, 100, 1024, 3), (21, 33000, 512, 2), (21, 20000, 2816, 16)]
+
+
+@pytest.mark.parametrize("fmt,N,K,nb", SHAPES)
+def test_shadow_is_hbm(env, fmt, N, K, nb):
+    g, p = env
+    rng = np.random.default_rng(N + K)
+    wb, W = weights(g, rng, fmt, N, K)
+    x, y = q.Buf(g, nb * K * 2), q.Buf(g, nb * N * 4)
+    seen = []
+    for step in range(3):  # other activations each time: nothing of the step before may be left
+        x.fill(synth.activations(rng, nb, K))
+        y.view()[:] = 0xEE
+        b = g.batch()
+        p.qmv_gg(b, W, N, K, x, y, nb)
+        assert b.end() > 0
+        assert same(y)
+        seen.append(y.view(np.float32).copy())
+    assert all(np.isfinite(v).all() for v in seen) and not np.array_equal(seen[0], seen[1])
+    for o in (wb, x, y):
+        o.free()
+
+
+@pytest.mark.parametrize("form", ["two writers", "chain", "flush", "submit", "binary16", "device output", "graph"])
+def test_rules(env, form):
+    """What else may surround such a launch in a batch."""
+    g, p = env
+    rng = np.random.default_rng(5)
+    K = N = 1024
+    wb, W = weights(g, rng, 8, N, K)
+    vb, V = weights(g, rng, 12, N, K)
+    x, y, z, dev = q.Buf(g, 2 * K * 2), q.Buf(g, 4 * N * 4), q.Buf(g, 2 * N * 4), q.Buf(g, 2 * N * 4, device_only=True)
+    g.L.qw_hip_set_graphs(g.g, form == "graph")
+    try:
+        for step in range(4):
+            x.fill(synth.activations(rng, 2, K))
+            y.view()[:] = 0xEE
+            b = g.batch()
+            if form == "two writers":  # one buffer, two ranges
+                p.qmv_gg(b, W, N, K, x, y, 2)
+                p.qmv_gg(b, V, N, K, x, y, 2, yoff=2 * N * 4)
+            elif form == "binary16":
+                p.qmv_gg(b, W, N, K, x, y, 2, fout=False)
+            elif form == "device output":  # nothing at all is carried back; the reader takes HBM
+                p.qmv_gg(b, W, N, K, x, dev, 2)
+            else:
+                for _ in range(10 if form == "graph" else 1):
+                    p.qmv_gg(b, W, N, K, x, y, 2)
+                    p.qmv_gg(b, V, N, K, x, dev, 2)
+                    if form == "flush":
+                        b.flush()
+                p.qmv_gg(b, V, N, K, x, z, 2)
+            if form == "submit":
+                g.L.qw_batch_submit(b.b)
+                assert g.L.qw_batch_wait(b.b) > 0
+            else:
+                assert b.end() > 0
+            ref = q.Buf(g, 4 * N * 4, device_only=True)  # the same products, results read from HBM
+            c = g.batch()
+            p.qmv_gg(c, W, N, K, x, ref, 2, fout=form != "binary16")
+            p.qmv_gg(c, V, N, K, x, ref, 2, yoff=2 * N * 4)
+            assert c.end() > 0
+            r = ref.read(dtype=np.uint32)
+            first, second = r[:2 * N] if form != "binary16" else r[:N], r[2 * N:]
+            if form == "device output":
+                assert np.array_equal(dev.read(dtype=np.uint32), first)
+            else:
+                got = y.view(np.uint32)
+                assert np.array_equal(got[:first.size], first)
+                if form == "two writers":
+                    assert np.array_equal(got[2 * N:], second)
+                else:
+                    assert (got[first.size:] == 0xEEEEEEEE).all()
+                    if form != "binary16":
+                        assert np.array_equal(z.view(np.uint32), second) and same(z) and np.array_equal(dev.read(dtype=np.uint32), second)
+            ref.free()
+    finally:
+        g.L.qw_hip_set_graphs(g.g, False)
+        torch.cuda.synchronize()
+        for o in (wb, vb, x, y, z, dev):
+            o.free()
