@@ -28,7 +28,7 @@ static const unsigned char qw_code_object[] = {
 };
 
 #define QW_DNQ_MIN_DEFAULT 2u // token count from which down + combine run as one launch of token quarters (qwk_dnq_*)
-enum { QW_MAX_ARGS = 288, QW_MAX_KERNELS = 4096, QW_MAX_BIND = 32, QW_MAX_BYTES = 256, QW_PROF_MAX = 8192, QW_MAX_FUNCS = 256 };
+enum { QW_MAX_ARGS = 448, QW_MAX_KERNELS = 4096, QW_MAX_BIND = 32, QW_MAX_BYTES = 256, QW_PROF_MAX = 8192, QW_MAX_FUNCS = 256 };
 
 // ---------------------------------------------------------------- records
 typedef enum {
@@ -96,10 +96,10 @@ typedef struct {
     bool last_of_dispatch;
     bool side; // independent of the launches before it in the batch: runs on the side stream, beside them
     bool join; // needs the side stream's results: the main stream waits for them first
-    // Outputs that the kernel can also write to a shadow: their uses, and where in the record the second pointers and the
-    // qwk_fin lie (host_outputs)
+    // Outputs that the kernel can also write to a shadow: their uses, and where in the record the second pointers, the
+    // qwk_fin and, if the kernel copies what others left (0: it does not), the qwk_back lie (host_outputs)
     int ndirect, direct_use[4];
-    unsigned short direct_at[4], fin_at;
+    unsigned short direct_at[4], fin_at, back_at;
 } qw_launch;
 
 // A buffer as a dispatch binds it, and the bytes it may touch. whole: every byte of [lo, hi) is written, whatever they held.
@@ -147,6 +147,9 @@ struct qw_batch {
     // almost nothing): set by moe_pre_gg / moe_gu_gg, consumed by moe_gu_gg / moe_dn_gg of the same batch.
     struct { bool valid; int fmt; const uint8_t *Wsg, *Wsu; qw_hbuf *hg, *hu; uint32_t rowbytes, nbr; } pend_sg;
     struct { bool valid; int fmt; const uint8_t *Wsd; qw_hbuf *hd; float *Psh; uint32_t rowbytes, nbr; int use; } pend_sd; // use: its binding of Psh
+    // The selection that a moe_pre_gg dispatch of this batch stands for, made by this backend: topk different experts for each of
+    // its nbr tokens, so that the gate/up and down dispatches that follow on the same record write every row of H and Pg.
+    struct { bool valid, gu; qwk_select_args a; const uint16_t *h; int seg, use_h, use_sel; } made;
     struct { bool valid; qwk_select_args a; } pend_sel; // the selection moe_pre_gg owes: made inside the gate/up launch, or by a launch of its own
     // a grouped product over IQ3_S rows that waits for its twin (gate, then up over the same packed rows: one launch
     // over the tile-major copy that holds both); launched alone at the next other dispatch or at submit
@@ -158,7 +161,7 @@ struct qw_batch {
     // a down projection over a few tokens that waits for the combine of the same layer: both in one launch
     // (qwk_dnc_*); launched as it is at any other dispatch or at submit
     // plain: its arguments without the combine, where they are not those of the joint form (Wd NULL: they are)
-    struct { bool valid; qwk_dn_args a, plain; const char *fname, *fused, *kname; unsigned grid, fused_grid; bool quarters; } pend_dn;
+    struct { bool valid; qwk_dn_args a, plain; const char *fname, *fused, *kname; unsigned grid, fused_grid; bool quarters; int use_p; /* its binding of Pg */ uint32_t rows; /* tokens of which it writes every row (0: not known) */ } pend_dn;
     // a routed gate/up launch that waits for the down projection and the combine of the same layer: the three run as one
     // launch (qwk_gud_*) when the down dispatch qualifies for the form by token shares; launched as it is otherwise
     struct { bool valid; qwk_gu_args a; const char *fname, *kname; unsigned grid; } pend_gu;
@@ -1012,7 +1015,7 @@ static bool bind_bytes(qw_batch *b, unsigned index, void *dst, size_t len, const
     return true;
 }
 
-_Static_assert(sizeof(qwk_pre_args) <= QW_MAX_ARGS && sizeof(qwk_gu_args) <= QW_MAX_ARGS && sizeof(qwk_dn_args) <= QW_MAX_ARGS && sizeof(qwk_qmv_args) <= QW_MAX_ARGS && sizeof(qwk_qmvm_args) <= QW_MAX_ARGS,
+_Static_assert(sizeof(qwk_pre_args) <= QW_MAX_ARGS && sizeof(qwk_gu_args) <= QW_MAX_ARGS && sizeof(qwk_dn_args) <= QW_MAX_ARGS && sizeof(qwk_qmv_args) <= QW_MAX_ARGS && sizeof(qwk_qmvm_args) <= QW_MAX_ARGS && sizeof(qwk_gud_args) <= QW_MAX_ARGS,
                "a kernel argument record is larger than the launch record's copy of it");
 
 static bool add_launch(qw_batch *b, const char *fname, unsigned gx, unsigned bx, const void *args, size_t argsz) {
@@ -1427,6 +1430,8 @@ static bool tr_pre(qw_batch *b) {
     b->pend_sg.valid = false;
     if (!bind_ptr(b, 6, (size_t)p->I * rb, false, "shared gate weights", (void **)&b->pend_sg.Wsg) || !bind_ptr(b, 7, (size_t)p->I * fmt_rb(p->fsu, p->D), false, "shared up weights", (void **)&b->pend_sg.Wsu) ||
         !bind_ptr(b, 8, (size_t)p->NB * (p->topk + 1) * p->I * 4, true, "H", (void **)&h)) return false;
+    const int use_h = b->nuse - 1;
+    b->made.valid = false;
     b->pend_sg.valid = true;
     b->pend_sg.hg = b->buf[6].h;
     b->pend_sg.hu = b->buf[7].h;
@@ -1464,6 +1469,23 @@ static bool tr_pre(qw_batch *b) {
     if (!rode && !launch_pre(b, intern(fn), &a, shared)) return false;
     if (!fill_select(b, &b->pend_sel.a, 3, 5, nbr)) return false;
     b->pend_sel.valid = true; // made by the gate/up launch if one follows for the same record, else by its own launch
+    b->use[b->nuse - 1].whole = true; // (the record is written in one piece)
+    const bool distinct = p->E == 64 || p->E == 128 || p->E == 256 || p->E == 512 || p->E == 1024; // (the other form may pick an expert twice where logits are -inf)
+    b->made.valid = distinct && !b->sw.ablate, b->made.gu = false, b->made.a = b->pend_sel.a, b->made.h = h, b->made.seg = b->nseg, b->made.use_h = use_h, b->made.use_sel = b->nuse - 1;
+    return true;
+}
+// A dispatch on record `sel` of its kernel's shape comes in the same segment as the front part that stands for the selection, and no
+// other dispatch has written the record or the H rows in between.
+static bool made_for(const qw_batch *b, const uint8_t *sel, const uint16_t *h) {
+    const qw_kparams *p = &b->k->p;
+    const qwk_select_args *m = &b->made.a;
+    if (!b->made.valid || b->made.seg != b->nseg || m->sel != sel || b->made.h != h || m->E != (uint32_t)p->E || m->topk != (uint32_t)p->topk || m->gnb != (uint32_t)p->gnb) return false;
+    const qw_use *us = &b->use[b->made.use_sel], *uh = &b->use[b->made.use_h];
+    for (int i = b->made.use_h + 1; i < b->nuse; i++) {
+        const qw_use *u = &b->use[i];
+        if (u->out && i > b->made.use_sel && u->b == us->b && u->lo < us->hi && u->hi > us->lo) return false;
+        if (!b->made.gu && u->b == uh->b && !(u->lo == uh->lo && u->hi == uh->hi && u->out) && u->lo < uh->hi && u->hi > uh->lo) return false; // H: read or written by anything but a gate/up dispatch
+    }
     return true;
 }
 
@@ -1476,6 +1498,11 @@ static bool tr_gu(qw_batch *b) {
     if (!bind_bytes(b, 12, &nbr, 4, "nbr") || !nbr_ok(b, nbr)) return false;
     qwk_gu_args a;
     if (!fill_gu(b, &a, p->fgu, 0, 1, 4, 6, nbr, false)) return false;
+    if (b->made.valid && !b->made.gu) { // the front part has written the shared expert's rows of H, or this launch does; it writes the others
+        b->made.valid = b->made.a.nbr == nbr && made_for(b, b->buf[5].h ? (const uint8_t *)b->buf[5].h->dptr + b->buf[5].off : NULL, a.H);
+        b->made.gu = true;
+        if (b->made.valid && nbr == (uint32_t)p->NB) b->use[b->made.use_h].whole = b->use[b->nuse - 1].whole = true;
+    } else b->made.valid = false;
     if (!bind_ptr(b, 5, QW_SEL_BYTES((size_t)p->gnb, (size_t)p->topk), false, "selection", (void **)&a.sel)) return false;
     b->pend_sd.valid = false;
     b->pend_sd.rowbytes = (uint32_t)fmt_rb(p->fsd, p->I);
@@ -1621,6 +1648,12 @@ static bool tr_dn_inner(qw_batch *b) {
     if (!bound || !bind_ptr(b, 2, (size_t)a.hplane * 4, false, "H", (void **)&a.H) ||
         !bind_ptr(b, 9, (size_t)nbr * p->topk * p->D * 4, true, "Pg", (void **)&a.P) ||
         !bind_ptr(b, 3, QW_SEL_BYTES((size_t)p->gnb, (size_t)p->topk), false, "selection", (void **)&a.sel)) return false;
+    b->pend_dn.use_p = b->nuse - 2, b->pend_dn.rows = 0;
+    if (b->made.gu && made_for(b, a.sel, a.H)) { // (Pg: the rows of the selection's tokens, all of them)
+        qw_use *u = &b->use[b->pend_dn.use_p];
+        u->hi = u->lo + (size_t)b->made.a.nbr * p->topk * p->D * 4, u->whole = true;
+        b->pend_dn.rows = b->made.a.nbr;
+    }
     int fs = 0;
     qw_hbuf *hsd = NULL;
     b->pend_dn.plain.Wd = NULL;
@@ -1791,6 +1824,7 @@ static bool tr_cmb(qw_batch *b) {
         if (same) {
             b->pend_dn.valid = false;
             d->nbr = nbr;
+            if (nbr < b->pend_dn.rows) b->use[b->pend_dn.use_p].whole = false;
             if (d->Wsd && d->snbr != nbr) b->use[b->pend_sd.use].whole = false; // the fused forms leave the rows of further tokens alone
             d->out = a.out;
             d->Psh = (float *)a.Psh;
@@ -1813,7 +1847,14 @@ static bool tr_cmb(qw_batch *b) {
                 d->nq = dnq_quarters(nbr), d->tpw = d->nq > 2 ? 2 : 1;
                 b->pend_dn.fused_grid = a.D / 16 / d->tpw * d->nq;
             }
-            return add_launch(b, b->pend_dn.fused, b->pend_dn.fused_grid, 64 * QW_WAVES_DNR, d, sizeof *d);
+            if (!add_launch(b, b->pend_dn.fused, b->pend_dn.fused_grid, 64 * QW_WAVES_DNR, d, sizeof *d)) return false;
+            qw_launch *l = &b->l[b->nl - 1];
+            const int uses[3] = {b->pend_dn.use_p, b->nuse - 1, b->pend_sd.use};
+            const size_t at[3] = {offsetof(qwk_dn_args, Ph), offsetof(qwk_dn_args, outh), offsetof(qwk_dn_args, Pshh)};
+            l->ndirect = d->Wsd ? 3 : 2; // (without a shared expert Psh is only read)
+            for (int j = 0; j < l->ndirect; j++) l->direct_use[j] = uses[j], l->direct_at[j] = (unsigned short)at[j];
+            l->fin_at = offsetof(qwk_dn_args, fin), l->back_at = offsetof(qwk_dn_args, back);
+            return true;
         }
         if (!flush_gu(b) || !flush_dn(b)) return false;
     }
@@ -2349,31 +2390,60 @@ static void touched_range(const qw_batch *b, int first, const qw_hbuf *h, bool o
 }
 
 static bool carried_back(const qw_use *u) { return u->out && !u->b->device_only && u->b->host && !u->b->wrapped && u->b->size <= QW_HIP_BIG_OUT_BYTES; }
-// Before the last launches of a batch that the caller waits for: those whose kernels can write a shadow themselves do so
-// where nothing else of the batch writes that buffer, and if that leaves nothing to carry back, the last one raises the flag.
+// After u's launch (last: the last one of b) the range of u's buffer that b carries back may be written to the shadow by
+// that launch alone: no other dispatch of b writes the buffer, or u comes last and writes all that they do; and what it
+// leaves alone of [u->lo, u->hi) is the same in the shadow and in HBM, because it went up with this segment.
+static bool direct_ok(const qw_batch *b, const qw_use *u, bool last) {
+    if (!carried_back(u) || !u->b->pinned) return false;
+    for (int j = 0; j < b->nuse; j++) {
+        const qw_use *o = &b->use[j];
+        if (o->out && o->b == u->b && o != u && !(last && u->whole && o->lo >= u->lo && o->hi <= u->hi)) return false;
+    }
+    return u->whole || (u->b->size <= QW_HIP_SMALL_BYTES && u->b->pending_out == 1);
+}
+static void direct_set(qw_batch *b, qw_launch *l, int d) {
+    qw_use *u = &b->use[l->direct_use[d]];
+    const char *host = (const char *)u->b->host + u->lo;
+    memcpy(l->args + l->direct_at[d], &host, sizeof host);
+    u->direct = true;
+}
+// Before the last launches of a batch that the caller waits for: a dense product writes the shadows of its results itself;
+// and where the last launch can see to all that is to be carried back (its own results and, if it is a layer's down
+// projection and combine, up to QW_BACK_MAX buffers of the launches before), it does, raises the flag, and no launch
+// follows it.
 static void host_outputs(qw_batch *b) {
     if (!b->io || b->uses_sync) return;
+    bool side = false;
     for (int i = b->done_l; i < b->nl; i++) {
         qw_launch *l = &b->l[i];
-        for (int d = 0; d < l->ndirect; d++) {
-            qw_use *u = &b->use[l->direct_use[d]];
-            if (!carried_back(u) || !u->b->pinned) continue;
-            int writers = 0;
-            for (int j = 0; j < b->nuse; j++) writers += b->use[j].out && b->use[j].b == u->b;
-            if (writers != 1) continue;
-            float *host = (float *)((char *)u->b->host + u->lo);
-            memcpy(l->args + l->direct_at[d], &host, sizeof host);
-            u->direct = true;
-        }
+        side = side || l->side;
+        for (int d = 0; d < l->ndirect && !l->back_at; d++)
+            if (direct_ok(b, &b->use[l->direct_use[d]], false)) direct_set(b, l, d);
     }
     qw_launch *l = b->nl > b->done_l ? &b->l[b->nl - 1] : NULL;
-    if (!l || !l->ndirect) return;
-    for (int i = b->done_l; i < b->nl; i++)
-        if (b->l[i].side) return;
-    for (int j = 0; j < b->nuse; j++)
-        if (carried_back(&b->use[j]) && !b->use[j].direct) return;
+    if (!l || !l->ndirect || side) return;
+    const unsigned mark = ++b->g->mark; // buffers that are seen to
+    for (int d = 0; d < l->ndirect; d++) {
+        const qw_use *u = &b->use[l->direct_use[d]];
+        if (carried_back(u) && !direct_ok(b, u, true)) return;
+        u->b->mark = mark;
+    }
+    qwk_back back = {0};
+    for (int j = 0; j < b->nuse; j++) {
+        const qw_use *u = &b->use[j];
+        if (!carried_back(u) || u->direct || u->b->mark == mark) continue;
+        if (!l->back_at || back.n == QW_BACK_MAX || !u->b->pinned) return;
+        u->b->mark = mark;
+        size_t lo, hi;
+        touched_range(b, j, u->b, true, &lo, &hi);
+        if (hi - lo > UINT32_MAX) return;
+        back.src[back.n] = (const char *)u->b->dptr + lo, back.dst[back.n] = (char *)u->b->host + lo, back.bytes[back.n++] = (uint32_t)(hi - lo);
+    }
     const qwk_fin fin = {.t_done = (uint64_t *)&b->io->t1[b->nseg - 1], .flag = (uint32_t *)&b->io->copied, .count = b->g->io_count + b->io_idx};
     memcpy(l->args + l->fin_at, &fin, sizeof fin);
+    if (l->back_at) memcpy(l->args + l->back_at, &back, sizeof back);
+    for (int d = 0; d < l->ndirect; d++)
+        if (carried_back(&b->use[l->direct_use[d]])) direct_set(b, l, d);
     b->fin = true;
 }
 
@@ -2532,7 +2602,7 @@ static double batch_wait(qw_batch *b, bool ended) { // ended: submitted by qw_ba
     const unsigned mark = ++g->mark;
     bool ok = true, sync = b->events;
     qw_io down = {.a = {.to_host = 1}};
-    for (int i = 0; i < b->nuse && ok; i++) {
+    for (int i = 0; i < b->nuse && ok && !b->fin; i++) {
         qw_hbuf *h = b->use[i].b;
         if (!b->use[i].out || h->mark == mark) continue;
         h->mark = mark;

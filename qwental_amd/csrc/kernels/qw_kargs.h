@@ -34,6 +34,13 @@ typedef struct {
     uint32_t *flag;   /* host, set to 1 */
     uint32_t *count;  /* device word, zero before and after the launch: workgroups that are done */
 } qwk_fin;
+/* What launches before it left for the host: pieces that the last launch copies beside its own work. */
+#define QW_BACK_MAX 4u
+typedef struct {
+    const void *src[QW_BACK_MAX]; /* device, 16-byte aligned */
+    void *dst[QW_BACK_MAX];       /* host */
+    uint32_t bytes[QW_BACK_MAX], n, pad;
+} qwk_back;
 
 typedef struct { /* dense matvec, y[b][row] = W[row] . x[b] */
     const uint8_t *W;
@@ -130,6 +137,12 @@ typedef struct {
     /* qwk_dn_rt: the ggml types of the routed and of the shared down rows (0: no shared expert in this launch),
      * chosen when the kernel runs */
     uint32_t fd, fsd;
+    /* qwk_dnc_*, qwk_dnq_* as the last launch of a batch over host-visible buffers (fin.flag NULL: not): second places for
+     * P, Psh (NULL where the launch does not make it) and out, and what the launches before left */
+    float *Ph, *Pshh;
+    uint16_t *outh;
+    qwk_fin fin;
+    qwk_back back;
 } qwk_dn_args;
 /* Down + combine with a quarter of the tokens per workgroup (qwk_dnq_*): limits of the staged H rows */
 #define QW_DNQ_ROWS 44u /* 4 tokens x (topk + 1) rows, topk <= 10 */

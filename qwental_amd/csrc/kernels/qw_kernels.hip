@@ -291,6 +291,26 @@ __device__ __forceinline__ void qw_fin_wg(const qwk_fin &f) {
     __syncthreads();                                 // and everybody's
     if (threadIdx.x < 64) qw_fin_wave(f);
 }
+// The same for a launch that stores in the ordinary way and also carries back what the launches before it left: every
+// workgroup its share, once its own work is done (what it waits for then overlaps with the others' work), and a release.
+// For a layer over host-visible buffers (down + combine, qwk_dnq_* and qwk_dnc_*): 250 KB at two tokens, 1.8 MB at sixteen go
+// back, of which Pg leaves as it is made, beside the weights. Against a qwk_io launch behind the layer, and with H, Pg and the
+// record, which the layer writes whole, no longer carried up first: layer of 512 experts, 2048 x 512 IQ3_S, one token 45.2 ->
+// 39.0 us, two 52.3 -> 46.6, eight 97.3 -> 79.2, sixteen 153 -> 102 (Pg from the sums in LDS at the end of the workgroup: 115).
+__device__ __forceinline__ void qw_back_fin(const qwk_back &k, const qwk_fin &f) {
+    if (!f.flag) return;
+    const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    for (uint32_t p = 0; p < k.n; p++) {
+        const uint32_t n16 = k.bytes[p] / 16;
+        for (uint32_t i = i0; i < n16; i += step) ((u4 *)k.dst[p])[i] = ((const u4 *)k.src[p])[i];
+        if (i0 < k.bytes[p] % 16) ((uint8_t *)k.dst[p])[n16 * 16 + i0] = ((const uint8_t *)k.src[p])[n16 * 16 + i0];
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    qw_fin_wave(f);
+}
 // y[b][row] = sum_k W[row][k] x[b][k] for up to 16 activations; the weights are streamed once for all of them.
 // Tiles of 16 rows are dealt round-robin to the waves of a persistent grid; a row is CPR chunks of CH blocks.
 template <int F, int CH, bool XLDS> __device__ __forceinline__ void qmv_body(const qwk_qmv_args &a, u2 *lut, u4 *xf, f4 *red) {
@@ -648,7 +668,7 @@ __device__ __forceinline__ void select_tokens(const float *logits, uint32_t E, u
         on[t] = tok < nbr;
         const float *lg = logits + (size_t)(on[t] ? tok : tok0) * (E + 1);
 #pragma unroll
-        for (int j = 0; j < PER; j++) k[t][j] = qw_fkey(lg[lane * PER + j]);
+        for (int j = 0; j < PER; j++) k[t][j] = max(qw_fkey(lg[lane * PER + j]), 1u); // 0 is left for what has been picked
         pk[t] = 0;
     }
     auto local_max = [&](int t) { // among equals the lower position wins
@@ -670,7 +690,7 @@ __device__ __forceinline__ void select_tokens(const float *logits, uint32_t E, u
             if (lane == L) {
 #pragma unroll
                 for (int jj = 0; jj < PER; jj++)
-                    if ((uint32_t)jj == j) k[t][jj] = 0; // below every key, -inf included
+                    if ((uint32_t)jj == j) k[t][jj] = 0; // below every key: with K experts or more no pick comes twice
                 local_max(t);
             }
         }
@@ -1877,8 +1897,9 @@ __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *p
             if (tok < QW_DNC_MAXNB && ((mask >> tok) & 1)) {
                 const uint32_t s = sh ? K : sc->slot[u * gnb + tok];
                 part[(tok * (K + 1) + s) * 16 + n] = acc[j];
-                if (sh) a.Psh[(size_t)tok * a.D + r] = acc[j];
-                else a.P[((size_t)tok * K + s) * a.D + r] = acc[j];
+                const size_t o = sh ? (size_t)tok * a.D + r : ((size_t)tok * K + s) * a.D + r;
+                (sh ? a.Psh : a.P)[o] = acc[j];
+                if (sh ? a.Pshh : a.Ph) (sh ? a.Pshh : a.Ph)[o] = acc[j];
             }
         }
     }
@@ -1891,7 +1912,9 @@ __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *p
         for (uint32_t s = 0; s < K; s++) o = __builtin_fmaf(w[s], p[s * 16], o);
         o = __builtin_fmaf(w[K], nsh ? p[K * 16] : a.Psh[(size_t)t * a.D + r], o);
         a.out[(size_t)t * a.D + r] = qw_f2h(o);
+        if (a.outh) a.outh[(size_t)t * a.D + r] = qw_f2h(o);
     }
+    qw_back_fin(a.back, a.fin);
 }
 #define QW_DNC(F, CH, FSD, CHSD, NAME)                                                              \
     extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) {                    \
@@ -2034,7 +2057,9 @@ __device__ __forceinline__ void dnq_run(const qwk_dn_args &a, const u2 *lut, con
                         const uint32_t s = SHARED ? K : (L.slot4[u] >> (8 * j)) & 255;
                         L.part[(j * (K + 1) + s) * rw + col] = acc[j];
                         // (untracked store: the combine below reads L.part, never Pg or Psh of this launch from memory)
-                        qw_store_f32(SHARED ? a.Psh + (size_t)(t0 + j) * a.D + r : a.P + ((size_t)(t0 + j) * K + s) * a.D + r, acc[j]);
+                        const size_t o = SHARED ? (size_t)(t0 + j) * a.D + r : ((size_t)(t0 + j) * K + s) * a.D + r;
+                        qw_store_f32((SHARED ? a.Psh : a.P) + o, acc[j]);
+                        if (SHARED ? a.Pshh : a.Ph) qw_store_f32((SHARED ? a.Pshh : a.Ph) + o, acc[j]);
                     }
                 }
             }
@@ -2158,8 +2183,10 @@ __device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_l
         else sh = a.Psh[(size_t)(t0 + t) * a.D + r]; // the caller's own shared product
         o = __builtin_fmaf(w[K], sh, o);
         a.out[(size_t)(t0 + t) * a.D + r] = qw_f2h(o);
+        if (a.outh) a.outh[(size_t)(t0 + t) * a.D + r] = qw_f2h(o);
     }
     QW_DSTAMP(14);
+    qw_back_fin(a.back, a.fin);
 }
 #define QW_DNQ(F, CH, FSD, CHSD, NAME)                                                              \
     extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) {                    \

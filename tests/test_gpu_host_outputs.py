@@ -7,6 +7,7 @@ import torch
 
 import qwental_amd as q
 from qwental_amd import synth
+from helpers import DeviceLayer
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +117,48 @@ def test_rules(env, form):
         torch.cuda.synchronize()
         for o in (wb, vb, x, y, z, dev):
             o.free()
+
+
+@pytest.mark.parametrize("recipe,D,I,E,topk,nb", [((21, 21, 21, 21, 21), 1024, 256, 64, 4, 1), ((21, 21, 8, 8, 8), 2048, 512, 128, 10, 3), ((8, 8, 8, 8, 8), 1024, 512, 64, 8, 16),
+                                                  ((21, 20, 12, 23, 20), 2560, 640, 64, 4, 1), ((21, 20, 12, 23, 20), 2560, 640, 64, 4, 5), ((12, 14, 12, 12, 14), 1024, 256, 64, 6, 2)])
+@pytest.mark.parametrize("scratch", [False, True])
+def test_layer(env, recipe, D, I, E, topk, nb, scratch):
+    """One MoE layer over host-visible buffers: every shadow (its scratch buffers too, where they are host-visible) holds what
+    HBM holds, the output what a batch ended by a launch of its own (submit, then wait) leaves."""
+    g, _ = env
+    rng = np.random.default_rng(D + nb)
+    p = q.Path(g, D, I, E, topk, 16, device_scratch=scratch)
+    layer = DeviceLayer(g, synth.moe_layer(rng, D, I, E, fgu=recipe[0], fd=recipe[1], fsh=recipe[2], fshd=recipe[4], fshu=recipe[3]), device_only=True)
+    x, lg, sel, out = q.Buf(g, nb * D * 2), q.Buf(g, p.logits_bytes(nb)), q.Buf(g, p.sel_bytes(nb)), q.Buf(g, nb * D * 2)
+    for step in range(3):
+        x.fill(synth.activations(rng, nb, D))
+        got = []
+        for ended in (False, True):
+            out.view()[:] = lg.view()[:] = sel.view()[:] = 0xEE
+            if not scratch:  # what the layer overwrites need not go up: garbage in it changes nothing
+                for i, lo, n in ((1, 0, nb * (topk + 1) * I * 2), (3, 0, nb * topk * D * 4)):
+                    c = g.L.qw_path_scratch(p.p, i).contents
+                    np.ctypeslib.as_array((q.gpu.C.c_uint8 * c.size).from_address(c.ptr))[lo:lo + n] = 0x7F
+            b = g.batch()
+            p.gg_moe(b, layer.layer, nb, x, lg, sel, out)
+            if ended:
+                assert b.end() > 0
+            else:
+                g.L.qw_batch_submit(b.b)
+                assert g.L.qw_batch_wait(b.b) > 0
+            for buf in (lg, sel, out):
+                assert np.array_equal(buf.view(), buf.read())
+            got.append([buf.view().copy() for buf in (out, lg, sel)])
+            if not scratch:
+                for i in (1, 2, 3):  # H, Psh, Pg
+                    c = g.L.qw_path_scratch(p.p, i).contents
+                    raw = np.ctypeslib.as_array((q.gpu.C.c_uint8 * c.size).from_address(c.ptr)).copy()
+                    hbm = np.empty(c.size, np.uint8)
+                    assert g.L.qw_hip_buf_read(q.gpu.C.byref(c), 0, hbm.ctypes.data, c.size) and np.array_equal(raw, hbm)
+                    got[-1].append(raw)
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+        assert np.isfinite(out.view(np.float16)).all()
+    p.close()
+    layer.free()
+    for o in (x, lg, sel, out):
+        o.free()
