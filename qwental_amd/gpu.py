@@ -5,6 +5,7 @@ method per C function."""
 import contextlib
 import ctypes as C
 import os
+import struct
 
 import numpy as np
 
@@ -127,6 +128,11 @@ def load_lib():
         f = getattr(L, name)  # AttributeError if the library lacks a declared symbol
         f.restype = res
         f.argtypes = args
+    # A prototype that takes the tensor as packed bytes (ctypes makes an object for every structure, pointer and array: 11 us
+    # a call of Path.qmv_ggm with four matrices, 2 packed).
+    if hasattr(L, "qw_path_qmv_gg"):
+        L.qmv_gg_packed = L["qw_path_qmv_gg"]
+        L.qmv_gg_packed.restype, L.qmv_gg_packed.argtypes = _b, [_vp, _vp, _vp, _i, _i, _pb, _sz, _pb, _sz, _i, _b]
     _lib = L
     return L
 
@@ -207,12 +213,20 @@ class SelRecord:
         self.w = raw[o:o + 4 * gnb * (topk + 1)].view(np.float32).reshape(gnb, topk + 1)
 
 
+_TENSOR = struct.Struct("PNixxxx")  # a QwTensor
+assert _TENSOR.size == C.sizeof(QwTensor)
+
+
 class Tensor:
     def __init__(self, buf, ftype, offset=0):
         self.buf, self.ftype, self.offset = buf, ftype, offset
 
     def c(self):
         return QwTensor(C.pointer(self.buf.c), self.offset, self.ftype)
+
+    def fields(self):
+        """The values of c() for _TENSOR."""
+        return C.addressof(self.buf.c), self.offset, self.ftype
 
 
 class MoeLayer:
@@ -362,16 +376,15 @@ class Path:
         return self.L.qw_path_logits_bytes(self.p, nb)
 
     def qmv_gg(self, batch, W, N, K, x, y, nb, fout=True, xoff=0, yoff=0):
-        t = W.c()
-        if not self.L.qw_path_qmv_gg(self.p, batch.b, C.byref(t), N, K, x.ref(), xoff, y.ref(), yoff, nb, fout):
+        if not self.L.qmv_gg_packed(self.p, batch.b, _TENSOR.pack(*W.fields()), N, K, x.ref(), xoff, y.ref(), yoff, nb, fout):
             raise RuntimeError("qw_path_qmv_gg failed")
 
     def qmv_ggm(self, batch, Ws, Ns, K, x, ys, nb, fout=True):
         """Up to four matrices (Tensor list) over the same x in one launch; ys: one output buffer per matrix."""
         n = len(Ws)
-        wt = (QwTensor * n)(*[w.c() for w in Ws])
-        na = (C.c_int * n)(*Ns)
-        ya = (C.POINTER(QwBuf) * n)(*[C.pointer(y.c) for y in ys])
+        wt = b"".join([_TENSOR.pack(*w.fields()) for w in Ws])
+        na = struct.pack("%di" % n, *Ns)
+        ya = struct.pack("%dP" % n, *[C.addressof(y.c) for y in ys])
         if not self.L.qw_path_qmv_ggm(self.p, batch.b, wt, na, n, K, x.ref(), ya, nb, fout):
             raise RuntimeError("qw_path_qmv_ggm failed")
 
