@@ -224,9 +224,13 @@ class Tensor:
     def c(self):
         return QwTensor(C.pointer(self.buf.c), self.offset, self.ftype)
 
-    def fields(self):
-        """The values of c() for _TENSOR."""
-        return C.addressof(self.buf.c), self.offset, self.ftype
+
+def _packed(w, keep):
+    """w.c() as bytes; what another class's c() made is kept alive in keep."""
+    if type(w) is Tensor:
+        return _TENSOR.pack(C.addressof(w.buf.c), w.offset, w.ftype)
+    keep.append(w.c())
+    return bytes(keep[-1])
 
 
 class MoeLayer:
@@ -376,13 +380,15 @@ class Path:
         return self.L.qw_path_logits_bytes(self.p, nb)
 
     def qmv_gg(self, batch, W, N, K, x, y, nb, fout=True, xoff=0, yoff=0):
-        if not self.L.qmv_gg_packed(self.p, batch.b, _TENSOR.pack(*W.fields()), N, K, x.ref(), xoff, y.ref(), yoff, nb, fout):
+        keep = []
+        if not self.L.qmv_gg_packed(self.p, batch.b, _packed(W, keep), N, K, x.ref(), xoff, y.ref(), yoff, nb, fout):
             raise RuntimeError("qw_path_qmv_gg failed")
 
     def qmv_ggm(self, batch, Ws, Ns, K, x, ys, nb, fout=True):
         """Up to four matrices (Tensor list) over the same x in one launch; ys: one output buffer per matrix."""
         n = len(Ws)
-        wt = b"".join([_TENSOR.pack(*w.fields()) for w in Ws])
+        keep = []
+        wt = b"".join([_packed(w, keep) for w in Ws])
         na = struct.pack("%di" % n, *Ns)
         ya = struct.pack("%dP" % n, *[C.addressof(y.c) for y in ys])
         if not self.L.qw_path_qmv_ggm(self.p, batch.b, wt, na, n, K, x.ref(), ya, nb, fout):

@@ -15,4 +15,12 @@ class Holder:  # a buffer's C record, without a device
 def test_packed_tensor():
     for ftype, offset in ((1, 0), (30, 16), (21, 2**33 + 110), (np.int64(14), np.int64(4096))):
         t = q.Tensor(Holder(), ftype, offset)
-        assert gpu._TENSOR.pack(*t.fields()) == bytes(gpu.QwTensor(C.pointer(t.buf.c), int(offset), int(ftype)))
+        want = gpu.QwTensor(C.pointer(t.buf.c), int(offset), int(ftype))
+        assert gpu._packed(t, []) == bytes(want)
+
+        class Other:  # anything with a c() of its own
+            def c(self):
+                return want
+
+        keep = []
+        assert gpu._packed(Other(), keep) == bytes(want) and keep == [want]
