@@ -991,6 +991,52 @@ __device__ __forceinline__ void qw_task_pipeline(uint32_t ntasks, uint32_t w0, u
     qw_task_pipeline<C>(ntasks, w0, nw, cpr, cstride, kl, rowp, use, [] {});
 }
 
+// ---------------------------------------------------------------- sums over lanes
+// A value plus that of lane l ^ o, or the latter alone, in the vector ALU: data-parallel primitives within a row of sixteen
+// lanes, the row and half swaps of gfx950 beyond. (__shfl_xor is an LDS round trip; the same additions, the same bits.)
+template <int CTRL> __device__ __forceinline__ float qw_dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 15, 15, false));
+}
+template <int O> __device__ __forceinline__ float qw_plus_xor(float v) {
+    static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "one bit");
+    if constexpr (O == 1) return v + qw_dpp<0xb1>(v);
+    else if constexpr (O == 2) return v + qw_dpp<0x4e>(v);
+    else if constexpr (O == 4) return v + qw_dpp<0x1b>(qw_dpp<0x141>(v)); // l ^ 7, then ^ 3
+    else if constexpr (O == 8) return v + qw_dpp<0x128>(v);               // row rotated by eight
+    else { // both rows (halves) of a pair in every lane of the pair
+        const uint32_t u = __builtin_bit_cast(uint32_t, v);
+        uint32_t x, y;
+        if constexpr (O == 16) {
+            const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+            x = r[0], y = r[1];
+        } else {
+            const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+            x = r[0], y = r[1];
+        }
+        return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+    }
+}
+__device__ __forceinline__ float qw_wave_sum(float v) {
+    return qw_plus_xor<1>(qw_plus_xor<2>(qw_plus_xor<4>(qw_plus_xor<8>(qw_plus_xor<16>(qw_plus_xor<32>(v))))));
+}
+__device__ __forceinline__ float qw_xor_lane(float v, int o) { // o: a power of two that the compiler knows
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    switch (o) {
+    case 1: return qw_dpp<0xb1>(v);
+    case 2: return qw_dpp<0x4e>(v);
+    case 4: return qw_dpp<0x1b>(qw_dpp<0x141>(v));
+    case 8: return qw_dpp<0x128>(v);
+    case 16: {
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        return __builtin_bit_cast(float, threadIdx.x & 16 ? r[0] : r[1]);
+    }
+    default: {
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return __builtin_bit_cast(float, threadIdx.x & 32 ? r[0] : r[1]);
+    }
+    }
+}
+
 // ---------------------------------------------------------------- wave-wide maximum of an unsigned key
 // DPP row shifts inside each row of 16 lanes, then the two row broadcasts of the gfx9 family; every lane receives
 // the result through a read of lane 63.

@@ -619,9 +619,7 @@ template <int WF, int NB> __device__ __forceinline__ void router_row(const qwk_r
     }
 #pragma unroll
     for (int t = 0; t < NB; t++) {
-        float v = acc[t];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+        const float v = qw_wave_sum(acc[t]);
         if (lane == 0 && (uint32_t)t < a.nb) a.logits[(size_t)t * (a.E + 1) + r] = v;
     }
 }
@@ -1086,7 +1084,7 @@ __device__ __forceinline__ void gu_tasks(const qwk_gu_args &a, const u2 *lut, co
         hs.tile(m);
 #pragma unroll
         for (uint32_t j = 0; j < 4; j++) {
-            const float up = __shfl_xor(acc[j], 8), g = acc[j];
+            const float up = __shfl_xor(acc[j], 8), g = acc[j]; // (in the vector ALU, qw_dpp<0x128>, the sixteen-token stack is 0.7 % slower)
             const uint32_t tok = 4 * kg + j;
             if (n < 8 && ((m >> tok) & 1)) {
                 const uint32_t s = a.shared ? K : sc->slot[u * gnb + tok];
@@ -1361,8 +1359,8 @@ template <int NB> __device__ __forceinline__ void pre_router_bf(const qwk_pre_ar
         if (h) {
             const bool up = lane & o;
 #pragma unroll
-            for (int t = 0; t < (h ? h : 1); t++) acc[t] = (up ? acc[t + h] : acc[t]) + __shfl_xor(up ? acc[t] : acc[t + h], o);
-        } else acc[0] += __shfl_xor(acc[0], o);
+            for (int t = 0; t < (h ? h : 1); t++) acc[t] = (up ? acc[t + h] : acc[t]) + qw_xor_lane(up ? acc[t] : acc[t + h], o);
+        } else acc[0] += qw_xor_lane(acc[0], o);
     }
     constexpr uint32_t lg = NB == 8 ? 3 : NB == 4 ? 2 : NB == 2 ? 1 : 0;
     const uint32_t t = lane >> (6 - lg);
@@ -1465,7 +1463,7 @@ template <int SH> __device__ __forceinline__ void pre_shared(const qwk_pre_args 
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++) {
         const uint32_t tok = 4 * kg + j;
-        const float up = __shfl_xor(g[j], 8); // (rows 8 .. 15 are the up rows)
+        const float up = qw_dpp<0x128>(g[j]); // (rows 8 .. 15 are the up rows)
         if (tok < r.nb && n < 8) pre_swiglu(a, g[j], up, tok, 8 * t + n);
     }
 }
@@ -2930,11 +2928,6 @@ extern "C" __global__ __launch_bounds__(256) void qwk_bw_read(qwk_mem_args a) {
 // ================================================================ hyper-connection, GGUF profile (kernels/hyper_gg.metal:94-233)
 // Everything in binary32, as there. Two launches a hyper-connection whatever the token count: a launch boundary costs
 // more here than recomputing nb x 320 activations per workgroup, which is what the reference's third kernel avoids.
-__device__ __forceinline__ float qw_wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
 // 2 sigmoid(sum over the streams of their inject sums for stream s / HC) (kernels/hyper_gg.metal:47-51)
 __device__ __forceinline__ float hc_coef(const float *injp, uint32_t s) {
     float t = 0;
@@ -2944,13 +2937,13 @@ __device__ __forceinline__ float hc_coef(const float *injp, uint32_t s) {
 }
 // Four sums at once over the lanes of a wave (W = 64) or of each half (W = 32): two exchange steps leave every lane with
 // one of the four values summed over a quad of lanes, the remaining steps add the quads. Lane l ends with the whole sum
-// of value number 2 (l & 1) + ((l >> 1) & 1). Seven (six) shuffles instead of four times six (five).
+// of value number 2 (l & 1) + ((l >> 1) & 1). Seven (six) exchanges instead of four times six (five).
 template <int W> __device__ __forceinline__ float qw_sum4(float d0, float d1, float d2, float d3, uint32_t lane) {
     const bool b0 = lane & 1, b1 = lane & 2;
-    const float e0 = (b0 ? d2 : d0) + __shfl_xor(b0 ? d0 : d2, 1), e1 = (b0 ? d3 : d1) + __shfl_xor(b0 ? d1 : d3, 1);
-    float f = (b1 ? e1 : e0) + __shfl_xor(b1 ? e0 : e1, 2);
-#pragma unroll
-    for (int o = 4; o < W; o <<= 1) f += __shfl_xor(f, o);
+    const float e0 = (b0 ? d2 : d0) + qw_dpp<0xb1>(b0 ? d0 : d2), e1 = (b0 ? d3 : d1) + qw_dpp<0xb1>(b0 ? d1 : d3);
+    float f = (b1 ? e1 : e0) + qw_dpp<0x4e>(b1 ? e0 : e1);
+    f = qw_plus_xor<16>(qw_plus_xor<8>(qw_plus_xor<4>(f)));
+    if constexpr (W == 64) f = qw_plus_xor<32>(f);
     return f;
 }
 // Down: residual, sums of squares and the un-normalised mix_down / inject sums (kernels/hyper_gg.metal:94-137).
@@ -2959,9 +2952,13 @@ template <int W> __device__ __forceinline__ float qw_sum4(float d0, float d1, fl
 // asked for before anything is used, so the kernel is one memory round trip whatever the token count. Per token: the
 // lane's eight h' w products, R dot products of eight and the squares, summed over the wave, then over the waves in
 // order. R = 4 fills the machine at a few tokens; R = 16 re-reads h and out four times less often at many.
+// Thirteen sums over lanes a token and four rows follow one another; as LDS round trips (__shfl_xor) they were 1 us of the
+// launch. In the vector ALU, and with five tokens as groups of three and two instead of four and one: down 7.1 -> 5.9 us at five
+// tokens, 10.0 -> 8.9 at sixteen, up 6.0 -> 5.0 and 8.5 -> 8.0 (D = 2048), with the same bits.
 template <uint32_t R> __device__ __forceinline__ void hc_down_body(const qwk_hc_args &a, float (*part)[QW_HC_TG][17]) {
-    const uint32_t rb = blockIdx.x, s = blockIdx.y, t0 = blockIdx.z * QW_HC_TG, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, nwv = blockDim.x >> 6;
-    const uint32_t nt = a.nb - t0 < QW_HC_TG ? a.nb - t0 : QW_HC_TG;
+    const uint32_t tg = (a.nb + gridDim.z - 1) / gridDim.z; // tokens of a group: as even as can be (five tokens: three and two)
+    const uint32_t rb = blockIdx.x, s = blockIdx.y, t0 = blockIdx.z * tg, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, nwv = blockDim.x >> 6;
+    const uint32_t nt = a.nb - t0 < tg ? a.nb - t0 : tg;
     QW_HSTAMP(0);
     const bool is_inj = rb == QW_HC_LR / R;
     const uint32_t nrow = is_inj ? QW_HC : R; // rows of this block (uniform)
@@ -3092,8 +3089,8 @@ extern "C" __global__ __launch_bounds__(320) void qwk_hc_mid(qwk_hc_args a) {
 // four mix_up rows s D + i (20 bytes each). GIVEN: sx and rs come from qwk_hc_mid instead of being made here.
 template <bool GIVEN> __device__ __forceinline__ void hc_up_body(const qwk_hc_args &a) {
     __shared__ float sx[QW_HC_TG][QW_HC_LR], rs[QW_HC_TG][QW_HC], js[QW_HC_TG][QW_HC];
-    const uint32_t tid = threadIdx.x, l32 = tid & 31, i = blockIdx.x * 8 + (tid >> 5), t0 = blockIdx.y * QW_HC_TG;
-    const uint32_t nt = a.nb - t0 < QW_HC_TG ? a.nb - t0 : QW_HC_TG;
+    const uint32_t tid = threadIdx.x, l32 = tid & 31, tg = (a.nb + gridDim.y - 1) / gridDim.y, i = blockIdx.x * 8 + (tid >> 5), t0 = blockIdx.y * tg;
+    const uint32_t nt = a.nb - t0 < tg ? a.nb - t0 : tg;
     const size_t HCD = (size_t)QW_HC * a.D;
     QW_HSTAMP(8);
     // Everything a thread will read is asked for here and without conditions (a lane without a token or a thread without
@@ -3206,8 +3203,7 @@ template <bool GIVEN> __device__ __forceinline__ void hc_up_body(const qwk_hc_ar
         }
         m = (hq * rs[ts][sq]) * wn / (1.0f + __expf(-uv));
     }
-    m += __shfl_xor(m, 1);
-    m += __shfl_xor(m, 2);
+    m = qw_plus_xor<2>(qw_plus_xor<1>(m));
     if (mine && sq == 0) a.x[(size_t)(t0 + ts) * a.D + i] = qw_f2h(m / QW_HC);
     QW_HSTAMP(13);
 }
