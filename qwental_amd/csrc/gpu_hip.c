@@ -112,6 +112,7 @@ typedef struct { qw_hbuf *b; bool out, whole, direct; size_t lo, hi; } qw_use;
 // the slot, which the batch before gave back after its last launch had ended.
 typedef struct { volatile uint64_t t0[9], t1[9]; volatile uint32_t done, copied; uint32_t pad[26]; } qw_ioslot;
 enum { QW_IO_SLOTS = 32 };
+_Static_assert(QW_IO_SLOTS % QW_FIN_LINE == 0, "the counters behind the words begin a line");
 
 // measurement switches: read from the environment by qw_gpu_open (and again by qw_hip_reload_switches), never per batch
 typedef struct { unsigned dnc_nb, dnq_min, spin_limit, hc_rows; int side, load_threads; bool dn_any, nl_c4, no_swiglu_matvec, shared_in_gu, split_select, pk_split, kq_own, no_fuse, ablate, verbose, quiet; } qw_switches;
@@ -218,7 +219,7 @@ struct qw_gpu {
     float *shgu;         // [2 streams][2][16][QW_SHGU_MAXI] gate and up results of a shared expert in the K-quant format family
     qw_ioslot *io;       // QW_IO_SLOTS of them, pinned; io_used: bit per slot taken by a batch
     uint32_t io_used;
-    uint32_t *io_count;  // device: a zero word per slot for qwk_io
+    uint32_t *io_count;  // device, zero: a word per slot for qwk_io, behind them QW_FIN_BYTES per slot for the launches that end a batch themselves
     hipFunction_t io_func;
     double tick;         // seconds of the device clock's unit
     bool repack;         // make packed copies (QW_HIP_REPACK=0 in the environment or qw_hip_set_repack turn it off)
@@ -326,7 +327,7 @@ qw_gpu *qw_gpu_open(void) {
             hipMalloc((void **)&g->sync, QW_SYNC_ALLOC) != hipSuccess || hipMemset(g->sync, 0, QW_SYNC_ALLOC) != hipSuccess ||
             hipHostMalloc((void **)&g->sync_host, 64, hipHostMallocCoherent) != hipSuccess ||
             hipHostMalloc((void **)&g->io, sizeof(qw_ioslot) * QW_IO_SLOTS, hipHostMallocCoherent) != hipSuccess ||
-            hipMalloc((void **)&g->io_count, QW_IO_SLOTS * 4) != hipSuccess || hipMemset(g->io_count, 0, QW_IO_SLOTS * 4) != hipSuccess ||
+            hipMalloc((void **)&g->io_count, QW_IO_SLOTS * (4 + QW_FIN_BYTES)) != hipSuccess || hipMemset(g->io_count, 0, QW_IO_SLOTS * (4 + QW_FIN_BYTES)) != hipSuccess ||
             !(g->io_func = find_func(g, "qwk_io")) || !(f = find_func(g, "qwk_tab_init"))) { free(g->kernels); free(g); return NULL; }
         ta = (qwk_tab_args){.tab = g->tabs, .slot_order = 1};
         if (hipDeviceSynchronize() != hipSuccess || hipModuleLaunchKernel(f, 32, 1, 1, 256, 1, 1, 0, g->stream[0], params, NULL) != hipSuccess ||
@@ -2439,7 +2440,7 @@ static void host_outputs(qw_batch *b) {
         if (hi - lo > UINT32_MAX) return;
         back.src[back.n] = (const char *)u->b->dptr + lo, back.dst[back.n] = (char *)u->b->host + lo, back.bytes[back.n++] = (uint32_t)(hi - lo);
     }
-    const qwk_fin fin = {.t_done = (uint64_t *)&b->io->t1[b->nseg - 1], .flag = (uint32_t *)&b->io->copied, .count = b->g->io_count + b->io_idx};
+    const qwk_fin fin = {.t_done = (uint64_t *)&b->io->t1[b->nseg - 1], .flag = (uint32_t *)&b->io->copied, .count = b->g->io_count + QW_IO_SLOTS + (size_t)b->io_idx * (QW_FIN_BYTES / 4)};
     memcpy(l->args + l->fin_at, &fin, sizeof fin);
     if (l->back_at) memcpy(l->args + l->back_at, &back, sizeof back);
     for (int d = 0; d < l->ndirect; d++)

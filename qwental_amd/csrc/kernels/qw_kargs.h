@@ -32,8 +32,12 @@ typedef struct { /* dq_test: rows x K values to float */
 typedef struct {
     uint64_t *t_done; /* host */
     uint32_t *flag;   /* host, set to 1 */
-    uint32_t *count;  /* device word, zero before and after the launch: workgroups that are done */
+    uint32_t *count;  /* device, QW_FIN_BYTES, zero before and after the launch: workgroups that are done */
 } qwk_fin;
+/* A word for all, and sixteen that every sixteenth workgroup of a larger launch counts in first, each in a line of its own: */
+#define QW_FIN_SUBS 16u
+#define QW_FIN_LINE 32u /* words */
+#define QW_FIN_BYTES (4u * QW_FIN_LINE * (1u + QW_FIN_SUBS))
 /* What launches before it left for the host: pieces that the last launch copies beside its own work. */
 #define QW_BACK_MAX 4u
 typedef struct {

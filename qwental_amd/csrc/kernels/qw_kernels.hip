@@ -260,7 +260,7 @@ extern "C" __global__ __launch_bounds__(256) void qwk_pack_nl(qwk_pack_args a) {
 // A result and its copy on the host. Stores of system scope go through the caches of the device to their memory, and have
 // arrived there when they are acknowledged. The results used to follow in a launch of their own (qwk_io), behind the product
 // instead of beside it; for a batch of one product that launch and its copy are a fifth of the whole. Measured, start of the
-// batch to its end on the host: 4096 x 2048 IQ3_S for one token 21.9 -> 20.8 us, 5127 x 2560 Q8_0 for seven 29.4 -> 24.8,
+// batch to its end on the host: 4096 x 2048 IQ3_S for one token 21.4 -> 18.6 us, 5127 x 2560 Q8_0 for seven 29.4 -> 24.7, 20000 x 512 Q8_0 for one 22.8 -> 19.7,
 // 131072 x 2048 Q6_K for four (2 MB back) at the end of 24 others 351 -> 340: 64 bytes a row of tile and token cross PCIe at
 // 35 GB/s where whole KBs (qwk_io) have 45, but while the product runs.
 __device__ __forceinline__ void qw_store_y(void *y, float *yh, bool f32, const qwk_fin &f, size_t i, float v) {
@@ -278,12 +278,21 @@ __device__ __forceinline__ void qw_store_y(void *y, float *yh, bool f32, const q
 __device__ __forceinline__ void qw_fin_wave(const qwk_fin &f) {
     if (!f.flag) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (qw_lane() == 0 && __hip_atomic_fetch_add(f.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
-        __hip_atomic_store(f.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); // for the next batch
-        __hip_atomic_store(f.t_done, __builtin_amdgcn_s_memrealtime(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __hip_atomic_store(f.flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    if (qw_lane()) return;
+    auto last = [](uint32_t *c, uint32_t n) { // the n-th to come, which clears the word for the next batch
+        if (__hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != n - 1) return false;
+        __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (the next batch may come on another stream, as soon as the flag is up)
+        return true;
+    };
+    // An atomic on one word takes 6 ns, one after the other: 1250 workgroups of a short product (20000 x 512) ended 8 us late
+    // (31.4 us for the batch; with the sixteen words 19.7, and 4096 x 2048, 256 workgroups, 20.8 -> 18.6).
+    const uint32_t subs = gridDim.x < 128 ? 1 : QW_FIN_SUBS, sub = blockIdx.x % subs;
+    if (subs > 1 && !last(f.count + QW_FIN_LINE * (1 + sub), (gridDim.x - sub + subs - 1) / subs)) return;
+    if (!last(f.count, subs > 1 ? subs : gridDim.x)) return;
+    __hip_atomic_store(f.t_done, __builtin_amdgcn_s_memrealtime(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(f.flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 __device__ __forceinline__ void qw_fin_wg(const qwk_fin &f) {
     if (!f.flag) return;

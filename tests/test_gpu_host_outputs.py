@@ -36,7 +36,8 @@ def same(y):
 # (type, rows, K, tokens): a workgroup a tile with one and several waves; the persistent kernels over whole and cut rows;
 # rows that do not fill a tile; IQ3_S beside the tile-major copy and past the staged K
 SHAPES = [(8, 17, 256, 1), (8, 5127, 2560, 7), (12, 100, 4096, 16), (14, 20000, 1024, 4), (14, 40000, 512, 3), (1, 9, 512, 5), (30, 30000, 768, 2),
-          (20, 24000, 1024, 16), (21, 4096, 2048, 1), (21, 100, 1024, 3), (21, 33000, 512, 2), (21, 20000, 2816, 16)]
+          (20, 24000, 1024, 16), (21, 4096, 2048, 1), (21, 100, 1024, 3), (21, 33000, 512, 2), (21, 20000, 2816, 16),
+          (8, 8191, 256, 2), (8, 20000, 512, 1), (12, 32000, 512, 3), (14, 2047, 256, 1)]  # up to 2000 workgroups; 128 and more count in sixteen words first
 
 
 @pytest.mark.parametrize("fmt,N,K,nb", SHAPES)
