@@ -2608,7 +2608,9 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_prep(qwk_prep_args a) 
 // The same for more pairs: a workgroup takes a slice of them, two workgroups a compute unit, so that the counting is not
 // repeated for every pair (a workgroup per pair reads all ids P times: 13.0 us at 2500 pairs). Bound by latency (ids,
 // atomics, scan: about 8 us) and then by the rows' copy. Measured: 2500 pairs of 4 KB rows 13.0 -> 10.3 us; 20480 pairs
-// 72.5 (the four launches) -> 30.3, of which the copy's 168 MB are 32 us at the rate of a large copy.
+// 72.5 (the four launches) -> 30.3. A token's row is read once for all of its pairs in the slice, at the kernel's entry, so that
+// only stores follow the scan (read for every pair, five loads one after the other a wave): 28.5 -> 24.6 at 20480 pairs, whose 84 MB
+// of stores are 16 at the rate of a large copy.
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(512) void qwk_moe_prep_slices(qwk_prep_args a) {
     __shared__ uint32_t cnt[1024], at[1024], wr[8], wt[8], id[QW_PREP_SLICE], pos[QW_PREP_SLICE];
@@ -2616,6 +2618,14 @@ extern "C" __global__ __launch_bounds__(512) void qwk_moe_prep_slices(qwk_prep_a
     const uint32_t p0 = blockIdx.x * a.slice < a.P ? blockIdx.x * a.slice : a.P, p1 = p0 + a.slice < a.P ? p0 + a.slice : a.P, np = p1 - p0;
     for (uint32_t e = tid; e < 1024; e += nth) cnt[e] = 0;
     if (tid < np) id[tid] = a.ids[p0 + tid];
+    // The slice's rows, asked for now and written when the places are known: an item is 16 bytes of a token's row, which up
+    // to topk of the slice's pairs take
+    const uint32_t units = a.KD / 8, tk0 = p0 / a.topk, items = np ? ((p1 - 1) / a.topk + 1 - tk0) * units : 0;
+    const u4 *src = (const u4 *)a.X + (size_t)tk0 * units;
+    u4 v[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++)
+        if (tid + k * nth < items) v[k] = src[tid + k * nth];
     __syncthreads();
     auto count = [&](uint32_t from, uint32_t to) {
         for (uint32_t q = from + tid; q < to; q += 8 * nth) { // eight ids under way at a time
@@ -2672,20 +2682,20 @@ extern "C" __global__ __launch_bounds__(512) void qwk_moe_prep_slices(qwk_prep_a
     __syncthreads();
     if (tid < np) a.pos_of[p0 + tid] = pos[tid] = mine < a.E ? at[mine] + rank : 0xffffffffu; // an expert id outside the table: the pair is dropped
     __syncthreads();
-    const uint32_t units = a.KD / 8; // a wave takes rows, four units of 16 bytes a lane under way at a time
-    for (uint32_t r = wave; r < np; r += nwv) {
-        const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)pos[r]);
-        if (to >= a.P) continue;
-        const u4 *src = (const u4 *)(a.X + (size_t)((p0 + r) / a.topk) * a.KD);
-        u4 *dst = (u4 *)(a.Xs + (size_t)to * a.KD);
-        for (uint32_t i = lane; i < units; i += 256) {
-            u4 v[4];
+    for (uint32_t i0 = tid; i0 < items; i0 += 4 * nth) {
+        if (i0 != tid) // more than four items a thread
 #pragma unroll
             for (uint32_t k = 0; k < 4; k++)
-                if (i + 64 * k < units) v[k] = src[i + 64 * k];
+                if (i0 + k * nth < items) v[k] = src[i0 + k * nth];
 #pragma unroll
-            for (uint32_t k = 0; k < 4; k++)
-                if (i + 64 * k < units) dst[i + 64 * k] = v[k];
+        for (uint32_t k = 0; k < 4; k++) {
+            const uint32_t i = i0 + k * nth;
+            if (i >= items) break;
+            const uint32_t t = i / units, c = i - t * units, first = (tk0 + t) * a.topk;
+            for (uint32_t q = first > p0 ? first : p0; q < first + a.topk && q < p1; q++) {
+                const uint32_t to = pos[q - p0];
+                if (to < a.P) ((u4 *)a.Xs)[(size_t)to * units + c] = v[k];
+            }
         }
     }
 }
