@@ -152,13 +152,17 @@ template <int F> struct qw_pfg_lds {
     u4 x[2][QW_PFG_ROWS * qw_pfg<F>::KS / 8 > QW_PFG_ROWS * QW_PFG_OS / 8 ? QW_PFG_ROWS * qw_pfg<F>::KS / 8 : QW_PFG_ROWS * QW_PFG_OS / 8];
     uint32_t m0[2048];   // the groups of rows: the first row,
     uint16_t er[2048];   // expert | rows - 1 << 10
-    uint32_t last[QW_PFG_WAVES], sum[QW_PFG_WAVES];
+    uint32_t last[QW_PFG_WAVES], sum[2][QW_PFG_WAVES];
 };
 
 // Entry f carries on where entry e of the table ends: the same expert, the next rows, and e is full.
 __device__ __forceinline__ bool pfg_follows(const u4 e, const u4 f, uint32_t tm) { return f.z > f.y && f.x == e.x && f.y == e.z && e.z - e.y == tm; }
-// The table's entries (tm rows each, an expert's one after the other) taken together to groups of up to 64 rows: head[i] =
-// first entry of group i. Four entries a thread, two scans (first entry of each run, number of groups before).
+// The table's entries (tm rows each, an expert's one after the other) taken together to groups of up to 64 rows, listed by size:
+// those of more than 48 rows first, then of more than 32, of more than 16, the others (in the table's order within each). Four
+// entries a thread, two scans (first entry of each run, groups of each size before). Why by size: a task takes 6 to 12 us
+// (64 rows cost almost twice what 16 do) and a workgroup's are every 256th of the list. In the table's order some
+// workgroups had many long ones and the launch waited for them: 2048 rows 406.7 -> 379.4 us for the whole path, 1000 rows 286.5 ->
+// 268.7, 400 rows 233.5 -> 219.9, the reference model's layer at 1000 rows 487 -> 430.
 template <class L> __device__ __forceinline__ uint32_t pfg_groups(const qwk_pf_args &a, L &S, uint32_t per) {
     const uint32_t lane = qw_lane(), wave = threadIdx.x >> 6, i0 = 4 * threadIdx.x; // (threads past entry 2047 have none)
     u4 e[5]; // e[0]: the entry before the thread's first
@@ -186,40 +190,53 @@ template <class L> __device__ __forceinline__ uint32_t pfg_groups(const qwk_pf_a
     if (lane == 0) before = 0;
     __syncthreads();
     for (uint32_t w = 0; w < wave; w++) before = S.last[w] > before ? S.last[w] : before;
-    uint32_t heads = 0, cnt = 0;
+    uint32_t rows[4], cnt[2] = {0, 0}; // rows: of the group that begins here, or 0; cnt: groups of one and two, of three and four times sixteen rows (16 bits each)
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++) {
         const uint32_t f = first[j] > before ? first[j] : before;
-        if ((used >> j & 1) && (i0 + j + 1 - f) % per == 0) heads |= 1u << j, cnt++;
-    }
-    uint32_t s = cnt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t u = __shfl_up(s, o);
-        if (lane >= (uint32_t)o) s += u;
-    }
-    if (lane == 63) S.sum[wave] = s;
-    __syncthreads();
-    uint32_t at = s - cnt, total = 0;
-    for (uint32_t w = 0; w < QW_PFG_WAVES; w++) {
-        if (w < wave) at += S.sum[w];
-        total += S.sum[w];
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < 4; j++)
-        if (heads >> j & 1) {
+        rows[j] = 0;
+        if ((used >> j & 1) && (i0 + j + 1 - f) % per == 0) {
             u4 l = e[j + 1]; // the group's last entry
             for (uint32_t i = 1; i < per && i0 + j + i < a.max_tiles; i++) {
-                const u4 f = *(const u4 *)(a.tiles + 4 * (i0 + j + i));
-                if (!pfg_follows(l, f, a.tm)) break;
-                l = f;
+                const u4 g = *(const u4 *)(a.tiles + 4 * (i0 + j + i));
+                if (!pfg_follows(l, g, a.tm)) break;
+                l = g;
             }
-            const uint32_t rows = l.z - e[j + 1].y;
-            S.m0[at] = e[j + 1].y;
-            S.er[at++] = (uint16_t)(e[j + 1].x | ((rows < QW_PFG_ROWS ? rows : QW_PFG_ROWS) - 1) << 10);
+            rows[j] = l.z - e[j + 1].y < QW_PFG_ROWS ? l.z - e[j + 1].y : QW_PFG_ROWS;
+            const uint32_t c = (rows[j] - 1) / 16, one = 1u << (c & 1) * 16;
+            if (c < 2) cnt[0] += one;
+            else cnt[1] += one;
+        }
+    }
+    uint32_t at[2] = {cnt[0], cnt[1]}, total[2] = {0, 0};
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u0 = __shfl_up(at[0], o), u1 = __shfl_up(at[1], o);
+        if (lane >= (uint32_t)o) at[0] += u0, at[1] += u1;
+    }
+    if (lane == 63) S.sum[0][wave] = at[0], S.sum[1][wave] = at[1];
+    __syncthreads();
+    for (uint32_t h = 0; h < 2; h++) {
+        at[h] -= cnt[h];
+        for (uint32_t w = 0; w < QW_PFG_WAVES; w++) {
+            if (w < wave) at[h] += S.sum[h][w];
+            total[h] += S.sum[h][w];
+        }
+    }
+    // the largest class first, the table's order within a class
+    const uint32_t n4 = total[1] >> 16, n3 = total[1] & 0xffff, n2 = total[0] >> 16, n1 = total[0] & 0xffff;
+    at[1] += n4, at[0] += (n4 + n3) << 16, at[0] += n4 + n3 + n2;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++)
+        if (rows[j]) {
+            const uint32_t c = (rows[j] - 1) / 16, sh = (c & 1) * 16, i = (c < 2 ? at[0] : at[1]) >> sh & 0xffff;
+            if (c < 2) at[0] += 1u << sh;
+            else at[1] += 1u << sh;
+            S.m0[i] = e[j + 1].y;
+            S.er[i] = (uint16_t)(e[j + 1].x | (rows[j] - 1) << 10);
         }
     __syncthreads();
-    return total;
+    return n4 + n3 + n2 + n1;
 }
 
 // Where a workgroup is in its sequence of steps: task (group of rows, block of tiles) and step of K.
