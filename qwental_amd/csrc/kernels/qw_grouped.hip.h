@@ -19,7 +19,7 @@
 //
 // Measured (Zipf(1.1) routing over 512 experts, top-10, D = 2048, I = 512; gate / up and down product, us), against the
 // kernel before, in which a wave took 16 weight rows and up to 64 packed rows and read the activations from memory:
-// 2048 rows 1102 + 522 -> 255 + 140, 1000 rows 573 + 273 -> 195 + 101; reference model's layer, 1082 rows 840 + 627 ->
+// 2048 rows 1102 + 522 -> 255 + 140 (219 + 127 with the groups listed by size), 1000 rows 573 + 273 -> 195 + 101; reference model's layer, 1082 rows 840 + 627 ->
 // 268 + 212 (1000 rows, down product: 213 -> 198 with operand reads that are not paired). What bounds it: at 2048 rows the loads alone (640 MB of slabs, 335 MB of rows that every block of tiles asks
 // for again) take 168 us, the arithmetic alone (vector ALU busy half of the time, LDS 53 %, matrix cores 21 %, at 1.75 GHz)
 // 209. Sixteen waves of one tile each, a barrier every step instead of every four, activations a step ahead or not, all
@@ -160,9 +160,11 @@ __device__ __forceinline__ bool pfg_follows(const u4 e, const u4 f, uint32_t tm)
 // The table's entries (tm rows each, an expert's one after the other) taken together to groups of up to 64 rows, listed by size:
 // those of more than 48 rows first, then of more than 32, of more than 16, the others (in the table's order within each). Four
 // entries a thread, two scans (first entry of each run, groups of each size before). Why by size: a task takes 6 to 12 us
-// (64 rows cost almost twice what 16 do) and a workgroup's are every 256th of the list. In the table's order some
+// (64 rows cost almost twice what 16 do) and a workgroup has one in 256 of the list. In the table's order some
 // workgroups had many long ones and the launch waited for them: 2048 rows 406.7 -> 379.4 us for the whole path, 1000 rows 286.5 ->
-// 268.7, 400 rows 233.5 -> 219.9, the reference model's layer at 1000 rows 487 -> 430.
+// 268.7, 400 rows 233.5 -> 219.9, the reference model's layer at 1000 rows 487 -> 430. Dealt there and back instead of in rounds
+// from the same end (where two rounds are not full, whoever had the longest task got a second one): 386.8 -> 380.4, 275.4 -> 269.3,
+// 227.0 -> 224.7, 436 -> 427; 272 rows of a layer of 256 experts of 256 x 1024 68.5 -> 62.0.
 template <class L> __device__ __forceinline__ uint32_t pfg_groups(const qwk_pf_args &a, L &S, uint32_t per) {
     const uint32_t lane = qw_lane(), wave = threadIdx.x >> 6, i0 = 4 * threadIdx.x; // (threads past entry 2047 have none)
     u4 e[5]; // e[0]: the entry before the thread's first
@@ -241,7 +243,7 @@ template <class L> __device__ __forceinline__ uint32_t pfg_groups(const qwk_pf_a
 
 // Where a workgroup is in its sequence of steps: task (group of rows, block of tiles) and step of K.
 struct qw_pfg_cursor {
-    uint32_t task, k, expert, m0, rows, tile0;
+    uint32_t task, k, expert, m0, rows, tile0, step; // step: to the next task; the list goes to the workgroups in turn, there and back (who had the longest of a round has the shortest of the next)
     template <class L> __device__ __forceinline__ void look(const L &S, uint32_t nblocks) {
         const uint32_t g = task / nblocks, er = (uint32_t)__builtin_amdgcn_readfirstlane(S.er[g]);
         m0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)S.m0[g]);
@@ -250,8 +252,8 @@ struct qw_pfg_cursor {
     // n steps on. False: there is no further one (the cursor stays, so that what it points at can still be read)
     template <class L> __device__ __forceinline__ bool next(const L &S, uint32_t n, uint32_t nsteps, uint32_t nblocks, uint32_t ntasks) {
         if (k + n < nsteps) return k += n, true;
-        if (task + gridDim.x >= ntasks) return false;
-        task += gridDim.x, k = 0;
+        if (task + step >= ntasks) return false;
+        task += step, step = 2 * gridDim.x - step, k = 0;
         look(S, nblocks);
         return true;
     }
@@ -275,7 +277,7 @@ template <int F> __device__ __forceinline__ void pfg_body(const qwk_pf_args &a, 
     const uint32_t per = a.tm < QW_PFG_ROWS ? QW_PFG_ROWS / a.tm : 1;
     const uint32_t ngroups = pfg_groups(a, S, per), nblocks = (a.ntn + QW_PFG_TB - 1) / QW_PFG_TB, ntasks = ngroups * nblocks, nsteps = a.K / KS;
     qw_pfg_cursor cur; // the step being multiplied; lx, lw: the ones whose rows (one ahead) and weights (two ahead) are asked for
-    cur.task = blockIdx.x, cur.k = 0;
+    cur.task = blockIdx.x, cur.k = 0, cur.step = 2 * (gridDim.x - blockIdx.x) - 1;
     qw_lds_arrive();
     __syncthreads(); // the table
     if (cur.task >= ntasks) return;
