@@ -67,7 +67,7 @@ __device__ __forceinline__ uint32_t qw_lane() { return threadIdx.x & 63; }
 #include "qw_grouped.hip.h"
 #include "qw_small.hip.h"
 constexpr bool qw_tiled(int f) { return f == QW_F_PACKED || f == QW_F_ABLATE || f == QW_F_PACKED_NL || f == QW_F_PACKED_Q8 || f == QW_F_PACKED_Q4K || f == QW_F_PACKED_Q6; } // weights come from a tile-major copy
-constexpr bool qw_wants_sums(int f) { return f == QW_F_PACKED_Q4K; } // decoders that read the sums of 32 activations beside them
+constexpr bool qw_wants_sums(int f) { return f == QW_F_PACKED_Q4K || f == 12; } // gate / up decoders that read the sums of 32 activations beside them
 constexpr bool qw_has_lut(int f) { return f == 21 || f == QW_F_PACKED || f == QW_F_ABLATE; } // formats decoded through the LDS table (the ablation copies it too)
 __device__ __forceinline__ uint32_t qw_all_tokens(uint32_t nbr) { return nbr >= 32 ? 0xffffffffu : (1u << nbr) - 1; }
 
@@ -1232,7 +1232,7 @@ QW_GU(121, 1, 0, 1, qwk_gu_f121_c1) QW_GU(121, 1, 121, 1, qwk_gu_f121_c1_s121_c1
 #endif
 // tile-major Q8_0 and Q4_K rows, D a multiple of 512; their shared expert is in the front launch. Measured (512 experts of 2048 x
 // 512, us a launch, GGUF rows -> these): Q8_0 14.3 -> 11.0 at one token, 32.9 -> 22.2 at four, 88.7 -> 63.2 at sixteen (310 MB: 4.9
-// TB/s); Q4_K (in qwk_gu_rt, with the arithmetic before qw_k45_steps) 21.5 -> 18.3 at four, 50.1 -> 40.5 at sixteen (164 MB).
+// TB/s); Q4_K 21.5 -> 18.3 at four, 50.1 -> 40.5 at sixteen (164 MB; qwk_gu_rt with scale and minimum applied to each step's result).
 #if QW_IN_PART(1)
 QW_GU(108, 2, 0, 1, qwk_gu_f108_c2) QW_GU(112, 2, 0, 1, qwk_gu_f112_c2)
 #endif

@@ -595,27 +595,48 @@ template <int NB> struct qw_chunk<QW_F_PACKED_Q6, NB> : qw_chunk_kq<QW_F_PACKED_
         for (int i = 0; i < NB; i++) gather_steps<0>(this->b[i], af, k0 + 256 * i, kg, acc);
     }
 };
-// Q4_K from the tile-major copy (QW_F_PACKED_Q4K in qw_kargs.h), three coalesced loads a block, for gate / up rows (an operand A with
-// the sums of 32 activations beside it: qw_afrag_lds_sums). A weight is d sc q - dmin m; written as d (q - 8) sc + (8 d sc - dmin m), its
-// first part has small integers, |(q - 8) sc| <= 504, exact in binary16 and made from the nibble by one mask (16 + q: the
-// nibble under the exponent of 16) and one fused multiply-add, (16 + q) sc - 24 sc; the eight steps of a block share an accumulator,
-// which d multiplies once. The second part is constant over a sub-block: two binary32 matrix instructions a block add its products
-// with the 32 activations' sums, four sub-blocks each, a lane bringing one sub-block's constant and one token's sum.
+// Q4_K gate / up rows (an operand A with the sums of 32 activations beside it: qw_afrag_lds_sums). A weight is d sc q - dmin m; written
+// as d (q - 8) sc + (8 d sc - dmin m), its first part has small integers, |(q - 8) sc| <= 504, exact in binary16; the eight steps of a
+// block share an accumulator, which d multiplies once. The second part is constant over a sub-block: two binary32 matrix
+// instructions a block add its products with the 32 activations' sums, four sub-blocks each, a lane bringing one sub-block's constant
+// and one token's sum. Rows in GGUF order and their tile-major copy go through this one block, whose integers are exact however they
+// are made, so a layer's bits do not depend on whether a copy could be made.
 // Against scale and minimum applied to each step's binary32 result (twelve vector instructions a step, and one more matrix instruction
 // for the sums): SwiGLU values 1.7e-7 to 2.8e-7 from float64 (512 to 2560 values, 1 to 16 tokens) where those are 1.9e-7 to 3.6e-7 (2-norm);
-// with q instead of q - 8 a dense product was 1.3e-7 off instead of 1.0e-7. Times: at qwk_gu_f112_c2.
+// with q instead of q - 8 a dense product was 1.3e-7 off instead of 1.0e-7. Times: at qwk_gu_f112_c2 and qwk_gu_rt.
+// b.template weight<S>(f): the eight (q - 8) sc of step S, sc in both halves of f.
+template <int S, class B> __device__ __forceinline__ void qw_q4_steps(const B &b, const qw_afrag_lds_sums &af, uint32_t kb, uint32_t kg, const uint32_t (&sc)[2], f4 &sub) {
+    if constexpr (S < 8) {
+        sub = qw_mfma(af.hi(kb + 32 * S + 8 * kg), b.template weight<S>(qw_byte_h2<(S & 3)>(sc[S >> 2])), sub);
+        qw_q4_steps<S + 1>(b, af, kb, kg, sc, sub);
+    }
+}
+// h: d, dmin and the packed scales
+template <class B> __device__ __forceinline__ void qw_q4_block(const B &b, const uint32_t *h, const qw_afrag_lds_sums &af, uint32_t kb, uint32_t kg, f4 &acc) {
+    uint32_t sc[2], mn[2];
+    qw_k4_scales(h + 1, sc, mn);
+    f4 sub = {0, 0, 0, 0};
+    qw_q4_steps<0>(b, af, kb, kg, sc, sub);
+    const float d = qw_h2f((uint16_t)h[0]), dm = qw_h2f((uint16_t)(h[0] >> 16));
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc[j] = __builtin_fmaf(d, sub[j], acc[j]);
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const float c = __builtin_fmaf(8.0f * d, (float)((sc[j] >> (8 * kg)) & 255), -dm * (float)((mn[j] >> (8 * kg)) & 255));
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af.sum(kb / 32 + 4 * j + kg), c, acc, 0, 0, 0);
+    }
+}
+// The block from the tile-major copy (QW_F_PACKED_Q4K in qw_kargs.h), three coalesced loads. A weight is made from the nibble by one mask
+// (16 + q: the nibble under the exponent of 16) and one fused multiply-add, (16 + q) sc - 24 sc.
 struct qw_q4_blk {
     uint32_t h[4], q[8]; // d, dmin and the packed scales; q[S]: the lane's eight nibbles of sub-block S
-    template <int S> __device__ __forceinline__ void steps(const qw_afrag_lds_sums &af, uint32_t kb, uint32_t kg, const uint32_t (&sc)[2], f4 &sub) const {
-        if constexpr (S < 8) {
-            const h2 f = qw_byte_h2<(S & 3)>(sc[S >> 2]), m24 = {(_Float16)-24.0f, (_Float16)-24.0f}, z = f * m24;
-            const uint32_t v = q[S];
-            u4 w = {v << 6, v << 2, v >> 2, v >> 6};
+    template <int S> __device__ __forceinline__ h8 weight(h2 f) const {
+        const h2 m24 = {(_Float16)-24.0f, (_Float16)-24.0f}, z = f * m24;
+        const uint32_t v = q[S];
+        u4 w = {v << 6, v << 2, v >> 2, v >> 6};
 #pragma unroll
-            for (int i = 0; i < 4; i++) w[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, (uint32_t)((w[i] & 0x03c003c0u) | 0x4c004c00u)), f, z));
-            sub = qw_mfma(af.hi(kb + 32 * S + 8 * kg), __builtin_bit_cast(h8, w), sub);
-            steps<S + 1>(af, kb, kg, sc, sub);
-        }
+        for (int i = 0; i < 4; i++) w[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, (uint32_t)((w[i] & 0x03c003c0u) | 0x4c004c00u)), f, z));
+        return __builtin_bit_cast(h8, w);
     }
 };
 template <int NB> struct qw_chunk<QW_F_PACKED_Q4K, NB> {
@@ -634,23 +655,27 @@ template <int NB> struct qw_chunk<QW_F_PACKED_Q4K, NB> {
     __device__ __forceinline__ void transpose() {}
     __device__ __forceinline__ void mac_lean(const u2 *, const qw_afrag_lds_sums &af, uint32_t k0, uint32_t kg, f4 &acc) const {
 #pragma unroll
-        for (int i = 0; i < NB; i++) {
-            uint32_t sc[2], mn[2];
-            qw_k4_scales(b[i].h + 1, sc, mn);
-            f4 sub = {0, 0, 0, 0};
-            b[i].template steps<0>(af, k0 + 256 * i, kg, sc, sub);
-            const float d = qw_h2f((uint16_t)b[i].h[0]), dm = qw_h2f((uint16_t)(b[i].h[0] >> 16));
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc[j] = __builtin_fmaf(d, sub[j], acc[j]);
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const float c = __builtin_fmaf(8.0f * d, (float)((sc[j] >> (8 * kg)) & 255), -dm * (float)((mn[j] >> (8 * kg)) & 255));
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af.sum((k0 + 256 * i) / 32 + 4 * j + kg), c, acc, 0, 0, 0);
-            }
-        }
+        for (int i = 0; i < NB; i++) qw_q4_block(b[i], b[i].h, af, k0 + 256 * i, kg, acc);
     }
 };
-template <int NB> struct qw_chunk<12, NB> : qw_chunk_kqa<12, NB> {};
+// The block in GGUF order, as the decoder of the format holds it (value order: the sub-block's bytes one after the other)
+struct qw_q4_row {
+    const qw_kq<12> &b;
+    template <int S> __device__ __forceinline__ h8 weight(h2 f) const {
+        constexpr int sh = 4 * (S & 1);
+        u4 w = __builtin_bit_cast(u4, qw_bytes_h8((b.r[4 + 2 * (S >> 1)] >> sh) & 0x0f0f0f0fu, (b.r[5 + 2 * (S >> 1)] >> sh) & 0x0f0f0f0fu, 8.0f));
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, (uint32_t)w[i]) * f);
+        return __builtin_bit_cast(h8, w);
+    }
+};
+template <int NB> struct qw_chunk<12, NB> : qw_chunk_kqa<12, NB> {
+    using qw_chunk_kqa<12, NB>::mac_lean;
+    __device__ __forceinline__ void mac_lean(const u2 *, const qw_afrag_lds_sums &af, uint32_t k0, uint32_t kg, f4 &acc) const {
+#pragma unroll
+        for (int i = 0; i < NB; i++) qw_q4_block(qw_q4_row{this->b[i]}, this->b[i].r, af, k0 + 256 * i, kg, acc);
+    }
+};
 template <int NB> struct qw_chunk<13, NB> : qw_chunk_kqa<13, NB> {};
 template <int NB> struct qw_chunk<14, NB> : qw_chunk_kqa<14, NB> {};
 template <int NB> struct qw_chunk<23, NB> : qw_chunk_kqa<23, NB> {};
