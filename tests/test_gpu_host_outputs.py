@@ -163,3 +163,42 @@ def test_layer(env, recipe, D, I, E, topk, nb, scratch):
     layer.free()
     for o in (x, lg, sel, out):
         o.free()
+
+
+def test_slot_passes_between_streams(env):
+    """A batch that ends itself gives its slot and the counters in it back as it found them: the next batch, on the other stream, takes the
+    same slot and ends itself too. Few and many workgroups (which count in sixteen words first), the persistent kernel, a layer."""
+    g, _ = env
+    rng = np.random.default_rng(9)
+    p = q.Path(g, 1024, 256, 64, 4, 16, device_scratch=True)
+    layer = DeviceLayer(g, synth.moe_layer(rng, 1024, 256, 64), device_only=True)
+    x, lg, sel, out = q.Buf(g, 3 * 1024 * 2), g.buf(p.logits_bytes(3)), g.buf(p.sel_bytes(3)), q.Buf(g, 3 * 1024 * 2)
+    shapes = [(8, 8000, 1024), (8, 64, 1024), (14, 40000, 512), (12, 2064, 256)]
+    ws = [weights(g, rng, *s) for s in shapes]
+    ys = [q.Buf(g, 3 * N * 4) for _, N, _ in shapes]
+    want = None
+    x.fill(synth.activations(rng, 3, 1024))
+    try:
+        for step in range(8):
+            g.L.qw_gpu_set_stream(g.g, step % 2)
+            got = []
+            for (_, N, K), (_, W), y in zip(shapes, ws, ys):
+                y.view()[:] = 0xEE
+                b = g.batch()
+                p.qmv_gg(b, W, N, K, x, y, 3)
+                assert b.end() > 0 and same(y)
+                got.append(y.view().copy())
+                g.L.qw_gpu_set_stream(g.g, (step + len(got)) % 2)
+            out.view()[:] = 0xEE
+            b = g.batch()
+            p.gg_moe(b, layer.layer, 3, x, lg, sel, out)
+            assert b.end() > 0 and np.array_equal(out.view(), out.read())
+            got.append(out.view().copy())
+            want = want or got
+            assert all(np.array_equal(a, c) for a, c in zip(got, want))
+    finally:
+        g.L.qw_gpu_set_stream(g.g, 0)
+        p.close()
+        layer.free()
+        for o in [x, lg, sel, out] + ys + [w for w, _ in ws]:
+            o.free()
