@@ -54,11 +54,18 @@ void *qw_hip_buf_devptr(const qw_buf *b);
  * IQ4_NL matrices whose rows are a multiple of 320 values, gate and up rows among them, at their first moe_pf_gg. The latter
  * are resident twice where decode steps run beside the packing path: those read IQ4_NL gate and up rows in GGUF order (512
  * experts of 640 x 2560: 944 MB more a layer for gate and up); and, at exactly their size, Q8_0 and Q4_K gate / up matrices
- * (D a multiple of 512) at their first moe_gu_gg and Q8_0 and (from 64 MB on) Q6_K down matrices (I 256 or 512) at their first
- * moe_dn_gg, all of which stay resident twice. A copy is dropped when the source buffer is freed, marked
+ * (D a multiple of 512) by moe_gu_gg and Q8_0 and (from 64 MB on) Q6_K down matrices (I 256 or 512) by moe_dn_gg, all of which
+ * stay resident twice (when: qw_hip_set_copy_uses). A copy is dropped when the source buffer is freed, marked
  * dirty, uploaded, written, or bound as a kernel's output. Without memory for one the dispatch reads the GGUF rows. Buffers of at most QW_HIP_SMALL_BYTES with a host shadow are never copied. QW_HIP_REPACK=0 in the
  * environment, or qw_hip_set_repack(g, false), turns the copies off (kernels then read the GGUF rows directly). */
 void qw_hip_set_repack(qw_gpu *g, bool on);
+/* The copies of Q8_0, Q4_K and Q6_K matrices that stay beside their source are worth their cost only for weights that come
+ * often: one of up to 96 MB is made at the matrix's first dispatch, a larger one at the uses-th dispatch that would read it (with the
+ * host waiting, as for every copy: some tenths of a millisecond each, once). Until then the dispatches read the GGUF rows; results are
+ * the same bits. uses 0 or 1: at the first dispatch, whatever the size - for a program that is about to use qw_path_gg_moe_noalloc,
+ * which makes no copies, or that would rather wait at its start. */
+#define QW_HIP_COPY_USES 32u
+void qw_hip_set_copy_uses(qw_gpu *g, unsigned uses);
 size_t qw_hip_packed_bytes(const qw_gpu *g);
 /* Keep only the tile-major copies of a weight buffer: frees the buffer's device bytes (the GGUF-order rows) once the
  * copies that the kernels read have been made, i.e. after every matrix in it has been through a dispatch that makes one

@@ -71,7 +71,7 @@ typedef struct qw_hbuf {
     bool part;        // the last upload carried [slo, shi) only, the bytes its batch could touch: HBM may lack what the host wrote elsewhere
     size_t slo, shi;
     struct qw_gpu *g;
-    int npack;       // packed copies made from this buffer (dropped when its contents change)
+    int npack, nwant; // packed copies made from this buffer (dropped when its contents change), and copies that are not due yet
     bool released;   // the device bytes were freed (qw_hip_buf_release_source): dptr is only the key of its tile-major copies
 } qw_hbuf;
 
@@ -85,6 +85,13 @@ typedef struct {
     size_t bytes;
     bool pf; // IQ4_NL rows that only moe_pf_gg has asked for, Q6_K rows that only moe_dn_gg has: another dispatch may read them in GGUF order
 } qw_pack;
+// A copy that would stay beside its source and is not due yet: the key of the copy, and how often a dispatch would have read it.
+typedef struct {
+    const void *A, *B;
+    qw_hbuf *ha, *hb;
+    uint64_t ntiles;
+    uint32_t nblk, fmt, uses;
+} qw_want;
 
 typedef struct {
     hipFunction_t f;
@@ -194,6 +201,9 @@ struct qw_gpu {
     uint64_t batch_seq;
     qw_pack *packs;
     int npacks, cappacks;
+    qw_want *wants;
+    int nwants, capwants;
+    uint32_t copy_uses; // qw_hip_set_copy_uses
     struct qw_ldlane { void *pin[2]; hipStream_t st; hipEvent_t ev[2]; } ld[QW_LD_MAX]; // staging of qw_hip_buf_write_fd, made at first use
     int nld;
     hipStream_t side[2]; // one beside each stream: launches of a batch that do not depend on the ones before them (made at first use)
@@ -311,6 +321,7 @@ qw_gpu *qw_gpu_open(void) {
     for (int i = 0; i < 2; i++)
         if (hipStreamCreateWithFlags(&g->stream[i], hipStreamNonBlocking) != hipSuccess) { free(g); return NULL; }
     g->kernels = calloc(QW_MAX_KERNELS, sizeof *g->kernels);
+    g->copy_uses = QW_HIP_COPY_USES;
     read_switches(g);
     {
         const char *e = getenv("QW_HIP_REPACK"); // these two have setters of their own; the environment gives the start value
@@ -380,7 +391,12 @@ void qw_gpu_close(qw_gpu *g) {
         if (g->packs[i].ha) g->packs[i].ha->npack = 0;
         if (g->packs[i].hb) g->packs[i].hb->npack = 0;
     }
+    for (int i = 0; i < g->nwants; i++) {
+        if (g->wants[i].ha) g->wants[i].ha->nwant = 0;
+        if (g->wants[i].hb) g->wants[i].hb->nwant = 0;
+    }
     free(g->packs);
+    free(g->wants);
     (void)hipFree(g->tabs);
     for (int i = 0; i < 8; i++) {
         if (g->graphs[i].exec) (void)hipGraphExecDestroy(g->graphs[i].exec);
@@ -713,10 +729,19 @@ bool qw_buf_wrap(qw_gpu *g, void *ptr, size_t len, qw_buf *out) {
     return true;
 }
 
-// The packed copies made from h are stale (its contents changed or it goes away): free them.
+static void want_drop(qw_gpu *g, int i) {
+    const qw_want *w = &g->wants[i];
+    if (w->ha) w->ha->nwant--;
+    if (w->hb && w->hb != w->ha) w->hb->nwant--;
+    g->wants[i] = g->wants[--g->nwants];
+}
+// The packed copies made from h are stale (its contents changed or it goes away): free them. Those not made yet are counted anew.
 static void packs_drop(qw_hbuf *h) {
-    if (!h || !h->npack) return;
+    if (!h) return;
     qw_gpu *g = h->g;
+    for (int i = g->nwants - 1; i >= 0 && h->nwant; i--)
+        if (g->wants[i].ha == h || g->wants[i].hb == h) want_drop(g, i);
+    if (!h->npack) return;
     (void)hipDeviceSynchronize(); // a batch in flight may still read them
     int n = 0;
     for (int i = 0; i < g->npacks; i++) {
@@ -759,6 +784,7 @@ void qw_hip_buf_mark_dirty(qw_buf *b) {
     packs_drop(b->handle);
 }
 void qw_hip_set_repack(qw_gpu *g, bool on) { g->repack = on; }
+void qw_hip_set_copy_uses(qw_gpu *g, unsigned uses) { g->copy_uses = uses; }
 unsigned qw_hip_graph_launches(const qw_gpu *g) { return g->ngraph_launches; }
 void qw_hip_set_graphs(qw_gpu *g, bool on) { g->use_graphs = on; }
 size_t qw_hip_packed_bytes(const qw_gpu *g) { return g->pack_bytes; }
@@ -1284,16 +1310,44 @@ static bool nbr_ok(qw_batch *b, uint32_t nbr) {
     return true;
 }
 
-// gate/up arguments. shared: one expert at (iWg, iWu), all tokens, slot topk.
+// Whether a copy of `bytes` that stays beside its source is made at this dispatch. Its cost is paid once and comes back as a few
+// microseconds a pass, so a matrix that is dispatched once or twice only loses by it, and a first pass over new weights takes up to
+// fifteen times as long (four layers of 512 experts of 2048 x 512, us a pass without copies, the pass that makes them, a pass with
+// them: Q4_K and Q6_K 205, 2550, 172 at four tokens, 426, 2750, 349 at sixteen; Q8_0 300, 5000, 191 and 717, 5280, 439: paid back
+// after 70, 29, 43 and 16 passes). So copies of more than QW_COPY_AT_ONCE wait until the matrix has come QW_HIP_COPY_USES times, in
+// the middle of these: whoever stops before has paid nothing, whoever stops right after it at most about twice what the passes took. Smaller
+// ones cost 70 to 100 us each, most of it the allocation and the wait, and are made at once (a layer of 16 to 80 such experts, four tokens,
+// us without copies, first pass, later ones: Q8_0 55, 213, 38 to 74, 371, 51; Q4_K 45, 122, 44 to 53, 250, 47). The bits of a layer are the
+// same either way.
+#define QW_COPY_AT_ONCE ((size_t)96 << 20)
+static bool copy_due(qw_gpu *g, const qw_want *key, size_t bytes) {
+    int i = 0;
+    while (i < g->nwants && !(g->wants[i].A == key->A && g->wants[i].B == key->B && g->wants[i].ntiles == key->ntiles && g->wants[i].nblk == key->nblk && g->wants[i].fmt == key->fmt)) i++;
+    if (i == g->nwants) {
+        if (bytes <= QW_COPY_AT_ONCE || g->copy_uses <= 1) return true;
+        if (g->nwants == g->capwants) {
+            g->capwants = g->capwants ? 2 * g->capwants : 64;
+            g->wants = realloc(g->wants, sizeof *g->wants * (size_t)g->capwants);
+        }
+        g->wants[g->nwants++] = *key;
+        if (key->ha) key->ha->nwant++;
+        if (key->hb && key->hb != key->ha) key->hb->nwant++;
+    }
+    if (++g->wants[i].uses < g->copy_uses) return false;
+    want_drop(g, i);
+    return true;
+}
+
 // The packed copy (format fmt) of one matrix A in tiles of 16 rows, or of two, A and B, in tiles of eight rows of each; nblk: units of K
 // a row (256 values; IQ4_NL: chunks of ten blocks).
-// Made at the first request, on the batch's stream, and complete when this returns; NULL when packing is off, the
-// source may change without notice (a small buffer with a host shadow is copied at every submit) or memory is short:
-// the caller then reads the GGUF rows directly.
+// Made at the first request (one that stays beside its source: when copy_due says so), on the batch's stream, and complete
+// when this returns; NULL until then, and when packing is off, the source may change without notice (a small buffer with a host shadow
+// is copied at every submit) or memory is short: the caller then reads the GGUF rows directly.
 static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const void *A, qw_hbuf *hb, const void *B, uint64_t ntiles, uint32_t nblk, uint32_t rowbytes) {
     qw_gpu *g = b->g;
     if (!g->repack) return NULL;
     const bool pf = (fmt == QW_F_PACKED_NL && b->k->fam == FAM_PF) || (fmt == QW_F_PACKED_Q6 && b->k->fam == FAM_DN);
+    const bool beside = fmt == QW_F_PACKED_Q8 || fmt == QW_F_PACKED_Q4K || (fmt == QW_F_PACKED_Q6 && b->k->fam == FAM_DN); // GGUF-order rows that the tuned kernels of a layer read too
     const uint32_t split = B ? 8 : 16;
     for (int i = 0; i < g->npacks; i++) {
         qw_pack *p = &g->packs[i];
@@ -1314,14 +1368,16 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
         // the submit): a copy made now would hold the old bytes.
         for (int u = b->done_use; u < b->nuse; u++)
             if (b->use[u].b == h && b->use[u].out) return NULL;
-        if (h->dirty && h->host) { // what the next submit would do for this buffer
-            if (hipMemcpyAsync(h->dptr, h->host, h->size, hipMemcpyHostToDevice, g->stream[b->stream]) != hipSuccess) return NULL;
-            h->dirty = false;
-        }
     }
+    const size_t bytes = (size_t)ntiles * nblk * pack_of(fmt).slab;
+    if (beside && !copy_due(g, &(qw_want){.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .fmt = fmt}, bytes)) return NULL;
+    for (int i = 0; i < 2; i++)
+        if (hs[i] && hs[i]->dirty && hs[i]->host) { // what the next submit would do for this buffer
+            if (hipMemcpyAsync(hs[i]->dptr, hs[i]->host, hs[i]->size, hipMemcpyHostToDevice, g->stream[b->stream]) != hipSuccess) return NULL;
+            hs[i]->dirty = false;
+        }
     hipFunction_t f = get_func(g, pack_of(fmt).fname);
     if (!f) return NULL;
-    const size_t bytes = (size_t)ntiles * nblk * pack_of(fmt).slab;
     void *dst;
     if (hipMalloc(&dst, bytes) != hipSuccess) {
         (void)hipGetLastError();
@@ -1346,6 +1402,7 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
     return dst;
 }
 
+// gate/up arguments. shared: one expert at (iWg, iWu), all tokens, slot topk.
 static bool fill_gu(qw_batch *b, qwk_gu_args *a, int F, unsigned iWg, unsigned iWu, unsigned ix, unsigned iH, uint32_t nbr, bool shared) {
     const qw_kparams *p = &b->k->p;
     const size_t rb = fmt_rb(F, p->D), ne = shared ? 1 : (size_t)p->E;
