@@ -66,6 +66,11 @@ void qw_hip_set_repack(qw_gpu *g, bool on);
  * which makes no copies, or that would rather wait at its start. */
 #define QW_HIP_COPY_USES 32u
 void qw_hip_set_copy_uses(qw_gpu *g, unsigned uses);
+/* The bytes that those copies may take together (at first a third of the device's memory; besides, none is made that would leave less
+ * than an eighth of it free). A matrix without room for its copy is read in GGUF order, and asked for again every
+ * QW_HIP_COPY_USES dispatches and at the first one after this call; copies that exist stay. The second gives the budget and what is taken of it. */
+void qw_hip_set_copy_budget(qw_gpu *g, size_t bytes);
+size_t qw_hip_copy_budget(const qw_gpu *g, size_t *used);
 size_t qw_hip_packed_bytes(const qw_gpu *g);
 /* Keep only the tile-major copies of a weight buffer: frees the buffer's device bytes (the GGUF-order rows) once the
  * copies that the kernels read have been made, i.e. after every matrix in it has been through a dispatch that makes one

@@ -83,14 +83,17 @@ typedef struct {
     uint32_t nblk, fmt, split;
     void *dst;
     size_t bytes;
+    bool beside; // counts into qw_gpu.beside_bytes
     bool pf; // IQ4_NL rows that only moe_pf_gg has asked for, Q6_K rows that only moe_dn_gg has: another dispatch may read them in GGUF order
 } qw_pack;
-// A copy that would stay beside its source and is not due yet: the key of the copy, and how often a dispatch would have read it.
+// A copy that would stay beside its source and is not due yet: the key of the copy, and how often a dispatch would have read it
+// (refused: since there was no room for it).
 typedef struct {
     const void *A, *B;
     qw_hbuf *ha, *hb;
     uint64_t ntiles;
     uint32_t nblk, fmt, uses;
+    bool refused;
 } qw_want;
 
 typedef struct {
@@ -204,6 +207,7 @@ struct qw_gpu {
     qw_want *wants;
     int nwants, capwants;
     uint32_t copy_uses; // qw_hip_set_copy_uses
+    size_t copy_budget, beside_bytes; // qw_hip_set_copy_budget, and what it bounds
     struct qw_ldlane { void *pin[2]; hipStream_t st; hipEvent_t ev[2]; } ld[QW_LD_MAX]; // staging of qw_hip_buf_write_fd, made at first use
     int nld;
     hipStream_t side[2]; // one beside each stream: launches of a batch that do not depend on the ones before them (made at first use)
@@ -322,6 +326,7 @@ qw_gpu *qw_gpu_open(void) {
         if (hipStreamCreateWithFlags(&g->stream[i], hipStreamNonBlocking) != hipSuccess) { free(g); return NULL; }
     g->kernels = calloc(QW_MAX_KERNELS, sizeof *g->kernels);
     g->copy_uses = QW_HIP_COPY_USES;
+    g->copy_budget = g->total_mem / 3;
     read_switches(g);
     {
         const char *e = getenv("QW_HIP_REPACK"); // these two have setters of their own; the environment gives the start value
@@ -752,6 +757,7 @@ static void packs_drop(qw_hbuf *h) {
                 fprintf(stderr, "qw_hip: a tile-major copy is dropped whose other source buffer was released: that buffer's matrix can no longer be dispatched\n");
             (void)hipFree(p->dst);
             g->pack_bytes -= p->bytes;
+            if (p->beside) g->beside_bytes -= p->bytes;
             if (p->ha && p->ha != h) p->ha->npack--;
             if (p->hb && p->hb != h && p->hb != p->ha) p->hb->npack--;
         } else g->packs[n++] = *p;
@@ -785,6 +791,15 @@ void qw_hip_buf_mark_dirty(qw_buf *b) {
 }
 void qw_hip_set_repack(qw_gpu *g, bool on) { g->repack = on; }
 void qw_hip_set_copy_uses(qw_gpu *g, unsigned uses) { g->copy_uses = uses; }
+void qw_hip_set_copy_budget(qw_gpu *g, size_t bytes) {
+    g->copy_budget = bytes;
+    for (int i = 0; i < g->nwants; i++)
+        if (g->wants[i].refused) g->wants[i].uses = QW_HIP_COPY_USES;
+}
+size_t qw_hip_copy_budget(const qw_gpu *g, size_t *used) {
+    if (used) *used = g->beside_bytes;
+    return g->copy_budget;
+}
 unsigned qw_hip_graph_launches(const qw_gpu *g) { return g->ngraph_launches; }
 void qw_hip_set_graphs(qw_gpu *g, bool on) { g->use_graphs = on; }
 size_t qw_hip_packed_bytes(const qw_gpu *g) { return g->pack_bytes; }
@@ -1319,23 +1334,40 @@ static bool nbr_ok(qw_batch *b, uint32_t nbr) {
 // ones cost 70 to 100 us each, most of it the allocation and the wait, and are made at once (a layer of 16 to 80 such experts, four tokens,
 // us without copies, first pass, later ones: Q8_0 55, 213, 38 to 74, 371, 51; Q4_K 45, 122, 44 to 53, 250, 47). The bits of a layer are the
 // same either way.
+// They double the memory of their weights, so they stop at a budget of their own (a third of the device unless
+// qw_hip_set_copy_budget says otherwise: 48 layers of the largest of these, Q8_0 experts of 512 x 2048 x 512, take 82 of 103 GB) and where an
+// eighth of the device would not stay free for others; a copy without room is asked for again after QW_HIP_COPY_USES dispatches.
 #define QW_COPY_AT_ONCE ((size_t)96 << 20)
-static bool copy_due(qw_gpu *g, const qw_want *key, size_t bytes) {
-    int i = 0;
-    while (i < g->nwants && !(g->wants[i].A == key->A && g->wants[i].B == key->B && g->wants[i].ntiles == key->ntiles && g->wants[i].nblk == key->nblk && g->wants[i].fmt == key->fmt)) i++;
-    if (i == g->nwants) {
-        if (bytes <= QW_COPY_AT_ONCE || g->copy_uses <= 1) return true;
-        if (g->nwants == g->capwants) {
-            g->capwants = g->capwants ? 2 * g->capwants : 64;
-            g->wants = realloc(g->wants, sizeof *g->wants * (size_t)g->capwants);
-        }
-        g->wants[g->nwants++] = *key;
-        if (key->ha) key->ha->nwant++;
-        if (key->hb && key->hb != key->ha) key->hb->nwant++;
+static int want_find(const qw_gpu *g, const qw_want *key) {
+    for (int i = 0; i < g->nwants; i++) {
+        const qw_want *w = &g->wants[i];
+        if (w->A == key->A && w->B == key->B && w->ntiles == key->ntiles && w->nblk == key->nblk && w->fmt == key->fmt) return i;
     }
-    if (++g->wants[i].uses < g->copy_uses) return false;
-    want_drop(g, i);
-    return true;
+    return -1;
+}
+static int want_add(qw_gpu *g, const qw_want *key) {
+    if (g->nwants == g->capwants) {
+        g->capwants = g->capwants ? 2 * g->capwants : 64;
+        g->wants = realloc(g->wants, sizeof *g->wants * (size_t)g->capwants);
+    }
+    g->wants[g->nwants] = *key;
+    if (key->ha) key->ha->nwant++;
+    if (key->hb && key->hb != key->ha) key->hb->nwant++;
+    return g->nwants++;
+}
+static void copy_refused(qw_gpu *g, const qw_want *key) {
+    int i = want_find(g, key);
+    if (i < 0) i = want_add(g, key);
+    g->wants[i].uses = 0, g->wants[i].refused = true;
+}
+static bool copy_due(qw_gpu *g, const qw_want *key, size_t bytes) {
+    int i = want_find(g, key);
+    if (i < 0 && bytes > QW_COPY_AT_ONCE && g->copy_uses > 1) i = want_add(g, key);
+    if (i >= 0 && ++g->wants[i].uses < (g->wants[i].refused ? QW_HIP_COPY_USES : g->copy_uses)) return false;
+    size_t avail, total;
+    if (bytes <= g->copy_budget && g->beside_bytes <= g->copy_budget - bytes && hipMemGetInfo(&avail, &total) == hipSuccess && avail >= total / 8 && avail - total / 8 >= bytes) return true;
+    copy_refused(g, key);
+    return false;
 }
 
 // The packed copy (format fmt) of one matrix A in tiles of 16 rows, or of two, A and B, in tiles of eight rows of each; nblk: units of K
@@ -1370,7 +1402,8 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
             if (b->use[u].b == h && b->use[u].out) return NULL;
     }
     const size_t bytes = (size_t)ntiles * nblk * pack_of(fmt).slab;
-    if (beside && !copy_due(g, &(qw_want){.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .fmt = fmt}, bytes)) return NULL;
+    const qw_want key = {.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .fmt = fmt};
+    if (beside && !copy_due(g, &key, bytes)) return NULL;
     for (int i = 0; i < 2; i++)
         if (hs[i] && hs[i]->dirty && hs[i]->host) { // what the next submit would do for this buffer
             if (hipMemcpyAsync(hs[i]->dptr, hs[i]->host, hs[i]->size, hipMemcpyHostToDevice, g->stream[b->stream]) != hipSuccess) return NULL;
@@ -1381,6 +1414,7 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
     void *dst;
     if (hipMalloc(&dst, bytes) != hipSuccess) {
         (void)hipGetLastError();
+        if (beside) copy_refused(g, &key);
         return NULL;
     }
     qwk_pack_args pa = {.A = A, .B = B, .dst = dst, .ntiles = ntiles, .nblk = nblk, .rowbytes = rowbytes, .split = split};
@@ -1395,8 +1429,13 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
         g->cappacks = g->cappacks ? 2 * g->cappacks : 64;
         g->packs = realloc(g->packs, sizeof *g->packs * (size_t)g->cappacks);
     }
-    g->packs[g->npacks++] = (qw_pack){.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .fmt = fmt, .split = split, .dst = dst, .bytes = bytes, .pf = pf};
+    g->packs[g->npacks++] = (qw_pack){.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .fmt = fmt, .split = split, .dst = dst, .bytes = bytes, .beside = beside, .pf = pf};
     g->pack_bytes += bytes;
+    if (beside) {
+        g->beside_bytes += bytes;
+        const int i = want_find(g, &key);
+        if (i >= 0) want_drop(g, i);
+    }
     if (ha) ha->npack++;
     if (hb && hb != ha) hb->npack++;
     return dst;

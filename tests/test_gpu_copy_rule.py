@@ -62,3 +62,25 @@ def test_a_large_matrix_is_copied_when_it_has_come_often():
     L.g.L.qw_hip_set_copy_uses(L.g.g, 1)  # a caller that wants them now
     assert np.array_equal(L.step(), first) and L.copied() == experts_bytes(E) + one
     L.close()
+
+
+def test_copies_stop_at_their_budget():
+    E = 16  # gate and up 36 MB, down 18 MB
+    L = Layer(E)
+    one = D * I // 32 * 34
+    budget = L.g.L.qw_hip_copy_budget(L.g.g, None)
+    assert budget == L.g.L.qw_gpu_max_working_set(L.g.g) // 3
+    L.g.L.qw_hip_set_copy_budget(L.g.g, experts_bytes(E) - 1)  # all but one byte of the layer
+    first = L.step()
+    used = q.gpu.C.c_size_t()
+    assert L.copied() == experts_bytes(E) - experts_bytes(E, True)
+    assert L.g.L.qw_hip_copy_budget(L.g.g, q.gpu.C.byref(used)) == experts_bytes(E) - 1 and used.value == L.copied()
+    for _ in range(40):
+        assert np.array_equal(L.step(), first)
+    assert L.copied() == experts_bytes(E) - experts_bytes(E, True)
+    L.g.L.qw_hip_set_copy_budget(L.g.g, budget)
+    assert np.array_equal(L.step(), first) and L.copied() == experts_bytes(E) + one
+    L.dl.bufs["Wd"].fill(L.dl.bufs["Wd"].read())  # the room of a copy that is dropped is given back
+    L.g.L.qw_hip_copy_budget(L.g.g, q.gpu.C.byref(used))
+    assert used.value == L.copied() == experts_bytes(E) - experts_bytes(E, True) + one
+    L.close()
