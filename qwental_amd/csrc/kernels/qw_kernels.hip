@@ -1395,6 +1395,7 @@ __device__ __forceinline__ void pre_swiglu(const qwk_pre_args &a, float g, float
 // A block of a format of that family as raw registers, so that the blocks of two formats can be on their way at once
 template <int F> __device__ __forceinline__ void pre_load(const uint8_t *p, uint32_t (&r)[32]) {
     typename qw_small_blk<F>::C c;
+    static_assert(sizeof c <= sizeof r, "a block of every format fits the registers");
     c.load(p, qw_lane() & 3);
     __builtin_memcpy(r, &c, sizeof c);
 }
@@ -1483,44 +1484,33 @@ struct qw_afrag_pre : qw_afrag_small {
     uint32_t kg;
     __device__ __forceinline__ f4 sum32(uint32_t k) const { return *(const f4 *)(xs + (k >> 5) * 16 + 4 * kg); }
 };
-// The wave's part in one format: blocks 2 part and 2 part + 1 of its rows (p: where they start) times x, which the part's two waves share
-// and of which each brings one block.
-template <int F> __device__ __forceinline__ f4 pre_part(const qwk_pre_args &a, const uint8_t *p, uint32_t part, uint32_t up, u4 *x, float *xs, qw_pre_lds &L) {
-    typedef qw_small_blk<F> B;
-    const uint32_t lane = qw_lane(), kg = lane >> 4, live = 1u << a.sh;
-    typename B::C c[2];
-    qw_pre_x xv;
+// Sums of 32 activations of a part's 512 values, in index order (by one wave; xs: its own).
+__device__ __forceinline__ void pre_sums(const qw_afrag_pre &af, float *xs) {
+    for (uint32_t i = qw_lane(); i < 16u << af.sh; i += 64) {
+        const uint32_t ch = i >> af.sh, m = i & ((1u << af.sh) - 1);
+        const qw_afrag_small one = {af.x, m, af.sh};
+        float sum = 0;
 #pragma unroll
-    for (int h = 0; h < 2; h++) c[h].load(p + h * B::BYTES, lane & 3);
-    xv.load(a.r, 512 * part + 256 * up);
-    if constexpr (F == 20 || F == 23) qw_kq_tab_build((uint32_t *)L.tab, lane, 64); // (every wave of such a format all of it: the others may not)
-    xv.store(x + (up ? 32 << a.sh : 0), a.r.nb, a.sh);
-    __syncthreads();
-    qw_afrag_pre af;
-    af.x = x, af.m = lane & 15 & (live - 1), af.sh = a.sh, af.xs = xs, af.kg = kg;
-    if constexpr (qw_kq<F>::HAS_MIN) { // sums of 32 activations, in index order
-        for (uint32_t i = lane; i < 16 * live; i += 64) {
-            const uint32_t ch = i >> a.sh, m = i & (live - 1);
-            const qw_afrag_small one = {x, m, a.sh};
-            float sum = 0;
+        for (uint32_t f = 0; f < 4; f++) {
+            const h8 v = one.at8(32 * ch + 8 * f);
 #pragma unroll
-            for (uint32_t f = 0; f < 4; f++) {
-                const h8 v = one.at8(32 * ch + 8 * f);
-#pragma unroll
-                for (int e = 0; e < 8; e++) sum += (float)v[e];
-            }
-            xs[ch * 16 + m] = sum;
+            for (int e = 0; e < 8; e++) sum += (float)v[e];
         }
-        __builtin_amdgcn_wave_barrier();
+        xs[ch * 16 + m] = sum;
     }
-    f4 acc = {0, 0, 0, 0};
+    __builtin_amdgcn_wave_barrier();
+}
+// The part's two blocks times its activations
+template <int F> __device__ __forceinline__ void pre_part(const uint32_t (&r0)[32], const uint32_t (&r1)[32], const qw_afrag_pre &af, const u2 *tab, f4 &acc) {
+    typename qw_small_blk<F>::C c[2];
+    __builtin_memcpy(&c[0], r0, sizeof c[0]);
+    __builtin_memcpy(&c[1], r1, sizeof c[1]);
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         c[h].transpose();
 #pragma unroll
-        for (int i = 0; i < B::NB; i++) qw_kq_block<F>(c[h].b[i], (const uint32_t *)L.tab, af, 256 * h + qw_kq<F>::BLK_K * i, kg, acc);
+        for (int i = 0; i < qw_small_blk<F>::NB; i++) qw_kq_block<F>(c[h].b[i], (const uint32_t *)tab, af, 256 * h + qw_kq<F>::BLK_K * i, af.kg, acc);
     }
-    return acc;
 }
 __device__ __forceinline__ void pre_pair(const qwk_pre_args &a, uint32_t t, qw_pre_lds &L) {
     const qwk_router_args &r = a.r;
@@ -1530,7 +1520,20 @@ __device__ __forceinline__ void pre_pair(const qwk_pre_args &a, uint32_t t, qw_p
     if (r.D % 512 == 0) {
         const uint32_t np = r.D / 512, up = wave >= np, part = up ? wave - np : wave, f = up ? a.fu : a.fg;
         const uint8_t *p = (up ? a.Wu : a.Wg) + (size_t)row * (up ? a.rbu : a.rbg);
-#define QW_DO(F) g = pre_part<F>(a, p + 2 * part * qw_small_blk<F>::BYTES, part, up, L.x + part * 1024, L.xs[wave], L)
+        u4 *const x = L.x + part * 1024;
+        uint32_t r0[32], r1[32]; // blocks 2 part and 2 part + 1 of the rows
+#define QW_DO(F) pre_load<F>(p + 2 * part * qw_small_blk<F>::BYTES, r0), pre_load<F>(p + (2 * part + 1) * qw_small_blk<F>::BYTES, r1)
+        switch (f) { QW_PRE_FORMATS(QW_DO) }
+#undef QW_DO
+        qw_pre_x xv; // the part's two waves share its activations, of which each brings one block
+        xv.load(r, 512 * part + 256 * up);
+        if (f == 20 || f == 23) qw_kq_tab_build((uint32_t *)L.tab, lane, 64); // (every wave of such a format all of it: the others may not)
+        xv.store(x + (up ? 32 << a.sh : 0), r.nb, a.sh);
+        __syncthreads(); // (waves of this workgroup may be in two formats: no barrier may stand in what the switches call)
+        qw_afrag_pre af;
+        af.x = x, af.m = n & ((1u << a.sh) - 1), af.sh = a.sh, af.xs = L.xs[wave], af.kg = kg;
+        if (f == 12 || f == 13) pre_sums(af, L.xs[wave]);
+#define QW_DO(F) pre_part<F>(r0, r1, af, L.tab, g)
         switch (f) { QW_PRE_FORMATS(QW_DO) }
 #undef QW_DO
         __syncthreads(); // (the part's other wave may still read the activations)

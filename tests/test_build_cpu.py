@@ -28,3 +28,20 @@ def test_counted_waits_have_their_loads_behind_them(kernel):
     assert refused(set(loads)) and any(refused({i}) for i in loads)
     with pytest.raises(RuntimeError):
         build.check_counted_waits(text.replace("s_barrier", "s_nop"))
+
+
+def test_waves_in_two_formats_meet_at_one_barrier():
+    """pre_pair: the waves of one workgroup may be in two formats, so nothing that its switches over the format call holds a barrier."""
+    with open(os.path.join(build.CSRC, "kernels", "qw_kernels.hip")) as f:
+        src = f.read()
+
+    def body(name):
+        m = re.search(r"^(?:template <int F> )?__device__ __forceinline__ \w+ %s\(.*?^\}" % name, src, re.S | re.M)
+        assert m, name
+        return m[0]
+
+    pair = body("pre_pair")
+    called = set(re.findall(r"#define QW_DO\(F\) (?:\w+ = )?(\w+)<F>", pair))
+    assert called and "__syncthreads" in pair
+    for name in called:
+        assert "__syncthreads" not in body(name) and "s_barrier" not in body(name), name
