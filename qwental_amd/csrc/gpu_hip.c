@@ -1776,7 +1776,10 @@ static bool tr_dn_inner(qw_batch *b) {
     // Everything that form asks of the shape, and a shared expert in the same format (or Q8_0 beside Q6_K, in GGUF order). Against
     // the range kernel on GGUF rows and the combine behind it (512 experts of 2048 x 512, top-10, us): Q8_0 26.5 + 4.8 -> 14.2 at four
     // tokens, 76.5 + 4.8 -> 35.4 at sixteen, one token (there one launch too) 11.1 -> 8.3; Q6_K 16.8 + 4.6 -> 15.3, 43.0 + 4.8 -> 33.1.
-    // Q6_K stacks of less than 64 MB stay with the range kernel.
+    // Q6_K stacks of less than 64 MB stay with the range kernel, for the sake of sixteen tokens: there a layer (Q4_K gate / up, 2048 x 512 down
+    // rows, us, range kernel -> this form) goes 51.9 -> 52.5 at 13 MB of down rows, 58.3 -> 62.7 at 26, 67.7 -> 70.8 at 39, 59.4 -> 60.7 at 52,
+    // 78.6 -> 79.0 at 59, 81.3 -> 81.0 at 66, 85.0 -> 83.5 at 79, 78.3 -> 75.0 at 105, 94.9 -> 86.5 at 210: with few experts every one is
+    // picked by several tokens, and each share decodes its rows again. One to eight tokens gain 3 to 6 us at every one of these sizes.
     if ((fd == 8 || fd == 14) && (fs == 0 || fs == fd || fs == 8) && p->I % 256 == 0 && p->I <= 512 && p->topk <= 10 && p->gnb * p->topk <= (int)QW_DNQ_MAXU && p->D % 256 == 0 &&
         (fd == 8 || (size_t)p->E * (size_t)p->D * rb >= QW_Q6_DOWN_PACK_MIN) && b->buf[0].off % 2 == 0 && (uintptr_t)a.H % 16 == 0 && !rel && !b->sw.dn_any && (nbr == 1 ? b->sw.dnc_nb >= 1 : b->sw.dnq_min && nbr >= b->sw.dnq_min)) {
         const uint32_t pf = fd == 8 ? QW_F_PACKED_Q8 : QW_F_PACKED_Q6, nblk = (uint32_t)p->I / 256, tileb = nblk * pack_of(pf).slab;
