@@ -742,7 +742,7 @@ static void want_drop(qw_gpu *g, int i) {
 }
 // The packed copies made from h are stale (its contents changed or it goes away): free them. Those not made yet are counted anew.
 static void packs_drop(qw_hbuf *h) {
-    if (!h) return;
+    if (!h || (!h->npack && !h->nwant)) return; // (a buffer may outlive its device: without either, the device is not looked at)
     qw_gpu *g = h->g;
     for (int i = g->nwants - 1; i >= 0 && h->nwant; i--)
         if (g->wants[i].ha == h || g->wants[i].hb == h) want_drop(g, i);

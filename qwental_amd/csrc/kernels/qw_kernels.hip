@@ -1232,11 +1232,13 @@ QW_GU(121, 1, 0, 1, qwk_gu_f121_c1) QW_GU(121, 1, 121, 1, qwk_gu_f121_c1_s121_c1
 #endif
 // tile-major Q8_0 and Q4_K rows, D a multiple of 512; their shared expert is in the front launch. Measured (512 experts of 2048 x
 // 512, us a launch, GGUF rows -> these): Q8_0 14.3 -> 11.0 at one token, 32.9 -> 22.2 at four, 88.7 -> 63.2 at sixteen (310 MB: 4.9
-// TB/s); Q4_K 21.5 -> 18.3 at four, 50.1 -> 40.5 at sixteen (164 MB; qwk_gu_rt with scale and minimum applied to each step's result).
+// TB/s); Q4_K 12.1 -> 11.6, 20.2 -> 18.3, 45.9 -> 42.0 (164 MB).
 #if QW_IN_PART(1)
 QW_GU(108, 2, 0, 1, qwk_gu_f108_c2) QW_GU(112, 2, 0, 1, qwk_gu_f112_c2)
 #endif
-// routed rows of the other GGUF types (Q4_K, Q5_K, Q6_K, IQ4_NL, IQ4_XS: kernels/moe_gg.metal:336-395), the type an argument
+// routed rows of the other GGUF types (Q4_K, Q5_K, Q6_K, IQ4_NL, IQ4_XS: kernels/moe_gg.metal:336-395), the type an argument. Q4_K with
+// scale and minimum applied to each step's result, as the other two still are, against the block that its tile-major rows
+// take (same shape, us): 12.8 -> 12.3 at one token, 21.4 -> 19.7 at four, 50.1 -> 45.6 at sixteen.
 #if QW_IN_PART(1)
 QW_GU(QW_F_RT, 1, 0, 1, qwk_gu_rt) QW_GU(QW_F_RT, 1, 21, 1, qwk_gu_rt_s21_c1) QW_GU(QW_F_RT, 1, 8, 1, qwk_gu_rt_s8_c1)
 #endif

@@ -50,8 +50,9 @@ template <int J> __device__ __forceinline__ void qw_small_iq3_steps(const qw_iq3
 // A block of Q4_K or Q5_K with the factors as integers, as in qw_chunk<QW_F_PACKED_Q4K>: d (q - C) sc + (C d sc - dmin m), C half of
 // the range of q, (q - C) sc exact in binary16. The sums of 32 activations are made by the lane that brings them to the binary32
 // matrix instruction. (Scale and minimum applied to each step's binary32 result, the sums by a matrix instruction a step, take twice
-// the vector instructions. Two steps an accumulator: errors to float64 as there, Q4_K 1.07e-7 and 1.07e-7 of a product of 2048 values,
-// Q5_K 0.96e-7 and 0.99e-7; all eight in one: 1.14e-7 and 1.05e-7.)
+// the vector instructions. Errors to float64, 2-norm, 1024 to 4096 values, one to sixteen tokens, that form -> this one with two
+// steps an accumulator: Q4_K 8.2e-8 to 1.04e-7 -> 8.1e-8 to 1.04e-7, Q5_K 8.4e-8 to 1.16e-7 -> 8.0e-8 to 1.11e-7. All eight steps in one
+// accumulator lose: at 2048 values Q4_K 1.14e-7, Q5_K 1.05e-7, where both forms are at 0.8e-7 to 0.97e-7.)
 template <int F, int S> __device__ __forceinline__ void qw_small_k45_steps(const qw_kq<F> &b, const qw_afrag_small &af, uint32_t kg, const uint32_t (&sc)[2], f4 (&sub)[4]) {
     if constexpr (S < 8) {
         constexpr int sh = 4 * (S & 1), q0 = F == 13 ? 6 : 4;

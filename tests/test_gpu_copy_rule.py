@@ -84,3 +84,14 @@ def test_copies_stop_at_their_budget():
     L.g.L.qw_hip_copy_budget(L.g.g, q.gpu.C.byref(used))
     assert used.value == L.copied() == experts_bytes(E) - experts_bytes(E, True) + one
     L.close()
+
+
+def test_buffers_may_outlive_the_device():
+    """Weights that were counted, and weights that were copied: the device goes first."""
+    L = Layer(64)
+    L.step()
+    L.path.close()
+    L.g.close()
+    for o in (L.x, L.lg, L.sel, L.out):
+        o.free()
+    L.dl.free()
