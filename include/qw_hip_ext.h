@@ -99,7 +99,8 @@ unsigned qw_hip_graph_launches(const qw_gpu *g);
 /* Measurement switches, read from the environment ONCE, by qw_gpu_open(); a batch takes the device's switches as they
  * are when it begins, and nothing reads the environment afterwards. A program that changes a variable while it holds
  * a device (the tests and the benchmark do, to time two forms on one shape) calls qw_hip_reload_switches() to have
- * them read again. Each switch routes a layer through kernels that other shapes or formats reach by themselves;
+ * them read again. Each switch but two (QW_HIP_ABLATE, and QW_HIP_NO_SWIGLU_MATVEC, whose second launch
+ * runs under it alone) routes a layer through kernels that other shapes or formats reach by themselves;
  * results do not change (tests/test_gpu_path.py runs a layer with each of them set).
  *   QW_HIP_FUSE=1             routed gate/up, down and combine of a layer run as one launch whose workgroups meet at a barrier
  *                             (qwk_gud_*: tile-major IQ3_S rows with D <= 2048, I = 512, top-k <= 10, on stream 0). Off by
