@@ -127,6 +127,7 @@ unsigned qw_hip_graph_launches(const qw_gpu *g);
  *   QW_HIP_KQ_OWN_LAUNCH      such a shared expert's gate/up as a launch of its own instead of on the workgroups behind the router's
  *   QW_HIP_SHARED_IN_GU       an IQ3_S / Q8_0 shared expert's gate/up inside the gate/up launch instead of the front launch
  *   QW_HIP_SPLIT_SELECT       the selection as a launch of its own instead of inside the gate/up launch
+ *   QW_HIP_NO_HOST_UP         small uploads always by a launch, never by stores of the host through the PCIe window
  * Read at the same two places: QW_HIP_LOAD_THREADS (threads of qw_hip_buf_write_fd), QW_HIP_VERBOSE (every error text
  * goes to stderr as it is set) and QW_HIP_QUIET (qw_batch_wait prints none). QW_HIP_REPACK=0 and QW_HIP_GRAPH=1 are
  * read by qw_gpu_open() only (see above); afterwards qw_hip_set_repack / qw_hip_set_graphs change them. */

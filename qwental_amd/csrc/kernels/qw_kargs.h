@@ -27,6 +27,9 @@ typedef struct { /* dq_test: rows x K values to float */
     uint32_t K, rowbytes, rows, fmt; /* fmt: used by the kernel that serves the formats 1, 12, 13, 14, 20, 23, 30 */
 } qwk_dq_args;
 
+/* t_start, in the records of launches that can be the first of a batch: host, may be NULL; where the launch writes the device clock
+ * as it starts (a batch that has nothing for qwk_io to carry up then needs no launch of that before its first). */
+
 /* What the last launch of a batch does for the host when its own outputs are all that the host waits for (flag NULL: not
  * asked for): the last workgroup to end writes the device clock and raises the flag. */
 typedef struct {
@@ -55,6 +58,7 @@ typedef struct { /* dense matvec, y[b][row] = W[row] . x[b] */
     uint32_t split, pad; /* waves a tile's chunks are cut over (1 .. 6; the chunk count of a row is a multiple of it) */
     float *yh;           /* host, may be NULL (always for binary16 results): a second place for y */
     qwk_fin fin;
+    uint64_t *t_start;
 } qwk_qmv_args;
 
 /* Dense matvec over up to four matrices that share the activations (kernels/qmv_ggm.metal:232-262; one matrix:
@@ -73,6 +77,7 @@ typedef struct {
     uint32_t sh, tabu;
     float *yh[4]; /* host, may be NULL (always for binary16 results): a second place for y[j] */
     qwk_fin fin;
+    uint64_t *t_start;
 } qwk_qmvm_args;
 
 /* SwiGLU of the shared expert when its gate/up rows went through the multi-format matvec: g, u float [nb][I] ->
@@ -183,6 +188,7 @@ typedef struct {
     uint16_t *H;
     const void *ctab;        /* the backend's IQ3_S table without signs */
     uint32_t fg, fu, rbg, rbu, I, topk, hplane, pad;
+    uint64_t *t_start;
 } qwk_pre_args;
 
 typedef struct { /* out[t][row] = half(sum_s w[t][s] * Pg[t][s][row] + w[t][topk] * Psh[t][row]) */
@@ -341,6 +347,7 @@ typedef struct {
     const uint16_t *X;
     uint16_t *Xs;
     uint32_t P, E, topk, KD, tm, max_tiles, slice, pad;
+    uint64_t *t_start;
 } qwk_prep_args;
 
 typedef struct { /* synthetic weights: nblocks GGUF blocks of one type, scale d = binary16(|N(0, sigma)|), the rest uniform */

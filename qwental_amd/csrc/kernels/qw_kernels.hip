@@ -272,6 +272,12 @@ __device__ __forceinline__ void qw_store_y(void *y, float *yh, bool f32, const q
     else ((float *)y)[i] = v;
     if (yh) __hip_atomic_store(yh + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+// The start of the first launch of a batch, at the entry of its kernel. qwk_io used to be that launch, for its stamp alone where
+// nothing goes up (2.4 us and a gap). Not in the hyper-connection's kernels: the look at the pointer, in the last line of their
+// arguments, comes before their first loads and takes them 0.6 us in every launch (5.9 -> 6.4).
+__device__ __forceinline__ void qw_started(uint64_t *t) {
+    if (t && blockIdx.x + blockIdx.y + blockIdx.z == 0 && threadIdx.x == 0) __hip_atomic_store(t, __builtin_amdgcn_s_memrealtime(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // The end of a workgroup in the last launch of a batch, by the wave that stored its results (qw_fin_wave) or by all of its
 // waves. What a launch with a flag stores it stores by qw_store_y, so that a wait for the stores is all that has to come
 // before the flag (a release would write the whole L2 back, once a workgroup: 1 us more at 256 of them).
@@ -388,6 +394,7 @@ template <int F, int CH, bool XLDS> __device__ __forceinline__ void qmv_body(con
 #define QW_QMV(F, CH, XLDS, SFX)                                                                        \
     extern "C" __global__ __launch_bounds__(QW_WG_GU) void qwk_qmv_f##F##SFX(qwk_qmv_args a) {             \
         __shared__ struct { u2 lut[qw_has_lut(F) ? QW_LUT_ENTRIES : 1]; u4 xf[XLDS ? QW_XF_MAXK * 2 : 1]; f4 red[QW_WG_GU]; } L; /* table first: LDS address 0 */ \
+        qw_started(a.t_start);                                                                          \
         qmv_body<F, CH, XLDS>(a, L.lut, L.xf, L.red);                                                   \
         qw_fin_wg(a.fin);                                                                               \
     }
@@ -433,6 +440,7 @@ template <int XN> __device__ __forceinline__ void qmvs_body(const qwk_qmvm_args 
 #define QW_QMVS(XN)                                                                                  \
     extern "C" __global__ __launch_bounds__(1024) void qwk_qmvs_x##XN(qwk_qmvm_args a) {              \
         extern __shared__ u4 qw_dyn[];                                                                \
+        qw_started(a.t_start);                                                                   \
         qmvs_body<XN>(a, qw_dyn);                                                                \
     }
 QW_QMVS(1) QW_QMVS(2) QW_QMVS(4) QW_QMVS(8)
@@ -505,6 +513,7 @@ template <int F, int NB> __device__ __forceinline__ void qmvm_matrix_split(const
 #if QW_IN_PART(0)
 extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_qmvm(qwk_qmvm_args a) {
     __shared__ struct { u4 xf[QW_KQ_MAXK * 2]; float xs[QW_KQ_MAXK / 2]; uint32_t tab[QW_KQ_TAB]; f4 red[QW_WG_QMVM]; } L;
+    qw_started(a.t_start);
     qw_kq_tab_build(L.tab);
     qw_stage_x(L.xf, a.x, a.xstride, a.K, a.nb);
     __syncthreads();
@@ -1586,6 +1595,7 @@ template <int SH> __device__ __forceinline__ void pre_shared_any(const qwk_pre_a
 #define QW_PRE(WF, SH, NAME)                                                                             \
     extern "C" __global__ __launch_bounds__(64 * QW_PRE_WAVES) void NAME(qwk_pre_args a) {               \
         __shared__ qw_pre_lds L;                                                                         \
+        qw_started(a.t_start);                                                                           \
         if (blockIdx.x < a.nrouter) pre_router_any<WF>(a, L);                                            \
         else pre_shared_any<SH>(a, blockIdx.x - a.nrouter, L);                                           \
     }
@@ -1595,6 +1605,7 @@ QW_PRE(30, 0, qwk_pre_w30) QW_PRE(30, QW_F_PACKED, qwk_pre_w30_s121) QW_PRE(30, 
 // the shared expert's part alone (the logits given by the caller, or beside the router on another stream)
 extern "C" __global__ __launch_bounds__(64 * QW_PRE_WAVES) void qwk_qmvm_swiglu(qwk_pre_args a) {
     __shared__ qw_pre_lds L;
+    qw_started(a.t_start);
     pre_shared_any<QW_F_RT>(a, blockIdx.x, L);
 }
 #endif
@@ -2549,6 +2560,7 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_scatter(qwk_scatter_ar
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(256) void qwk_moe_prep(qwk_prep_args a) {
     __shared__ uint32_t cnt[1024], red[4], wr[4], wt[4];
+    qw_started(a.t_start);
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, p = blockIdx.x;
     const uint32_t ep = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.ids[p]);
     for (uint32_t e = tid; e < a.E; e += 256) cnt[e] = 0;
@@ -2619,6 +2631,7 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_prep(qwk_prep_args a) 
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(512) void qwk_moe_prep_slices(qwk_prep_args a) {
     __shared__ uint32_t cnt[1024], at[1024], wr[8], wt[8], id[QW_PREP_SLICE], pos[QW_PREP_SLICE];
+    qw_started(a.t_start);
     const uint32_t tid = threadIdx.x, nth = blockDim.x, lane = tid & 63, wave = tid >> 6, nwv = nth >> 6;
     const uint32_t p0 = blockIdx.x * a.slice < a.P ? blockIdx.x * a.slice : a.P, p1 = p0 + a.slice < a.P ? p0 + a.slice : a.P, np = p1 - p0;
     for (uint32_t e = tid; e < 1024; e += nth) cnt[e] = 0;
