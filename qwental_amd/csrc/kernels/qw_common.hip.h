@@ -34,6 +34,11 @@ typedef u2 __attribute__((aligned(2))) u2a2;
 #define QW_LUT_ENTRIES 8192
 #define QW_LUT_BYTES (QW_LUT_ENTRIES * 8)
 
+// Threads of the workgroup. (blockDim.x allows for a last workgroup of another size: the compiler reads one of two 16-bit fields, chosen by
+// comparing the workgroup's index with their number, through the vector memory - a round trip that most kernels waited for before
+// they asked for anything else. No launch here has such a workgroup; this is a scalar load beside the arguments'.)
+__device__ __forceinline__ uint32_t qw_threads() { return __builtin_amdgcn_workgroup_size_x(); }
+
 __device__ __forceinline__ float qw_h2f(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
 __device__ __forceinline__ uint16_t qw_f2h(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
 __device__ __forceinline__ float qw_bf2f(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
@@ -63,7 +68,7 @@ __device__ __forceinline__ uint32_t qw_lut_slot(uint32_t i) { return ((i & 255) 
 
 // Fill the 64 KB table in LDS; every thread of the workgroup takes part. Caller synchronises afterwards.
 __device__ __forceinline__ void qw_lut_build(u2 *lut) {
-    for (uint32_t i = threadIdx.x; i < QW_LUT_ENTRIES; i += blockDim.x) lut[qw_lut_slot(i)] = qw_lut_entry(i);
+    for (uint32_t i = threadIdx.x; i < QW_LUT_ENTRIES; i += qw_threads()) lut[qw_lut_slot(i)] = qw_lut_entry(i);
 }
 
 __device__ __forceinline__ f4 qw_mfma(h8 a, h8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
@@ -292,7 +297,7 @@ __device__ __forceinline__ void qw_lds_arrive();
 // part, nparts: the calling wave is number `part` of the `nparts` waves that do the copy (default: all of the workgroup).
 __device__ __forceinline__ void qw_stage_x_issue(u4 *xf, const uint16_t *x, uint32_t xstride, uint32_t K, uint32_t nb, uint32_t part = ~0u, uint32_t nparts = 0) {
     const uint32_t n = (K >> 3) * 16, rot = (blockIdx.x * 320u) % n, lane = threadIdx.x & 63; // n and rot are multiples of 64
-    if (part == ~0u) part = threadIdx.x >> 6, nparts = blockDim.x >> 6;
+    if (part == ~0u) part = threadIdx.x >> 6, nparts = qw_threads() >> 6;
     for (uint32_t i0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)part) * 64; i0 < n; i0 += 64 * nparts) {
         const uint32_t base = i0 + rot < n ? i0 + rot : i0 + rot - n, i = base + lane, c = i >> 4, m = i & 15;
         if (m < nb) qw_load_to_lds((const u4 *)(x + (size_t)m * xstride + 8 * c), xf + base);
@@ -975,7 +980,7 @@ __device__ __forceinline__ void qw_lut_copy_issue(u2 *lut, const u2 *glut, uint3
     u4 *dst = (u4 *)lut;
     constexpr uint32_t N = QW_LUT_BYTES / 16;
     const uint32_t rot = blockIdx.x * 320u, lane = threadIdx.x & 63;
-    if (part == ~0u) part = threadIdx.x >> 6, nparts = blockDim.x >> 6;
+    if (part == ~0u) part = threadIdx.x >> 6, nparts = qw_threads() >> 6;
     for (uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)part) * 64; i < N; i += 64 * nparts) {
         const uint32_t j = (i + rot) & (N - 1); // a multiple of 64, the same in every lane
         qw_load_to_lds(src + j + lane, dst + j);

@@ -77,7 +77,7 @@ template <int F> __device__ __forceinline__ void dq_test_body(const qwk_dq_args 
     const uint8_t *row = a.W + (size_t)blockIdx.x * a.rowbytes;
     float *y = a.y + (size_t)blockIdx.x * a.K;
     if (F == 21) {
-        for (uint32_t i = threadIdx.x; i < a.K / 64; i += blockDim.x) {
+        for (uint32_t i = threadIdx.x; i < a.K / 64; i += qw_threads()) {
             const uint32_t blk = i >> 2, kg = i & 3;
             const qw_iq3_slice s = qw_iq3_load(row + 110 * blk, kg);
             h8 v[8] = {qw_iq3_step<0>(s, lut), qw_iq3_step<1>(s, lut), qw_iq3_step<2>(s, lut), qw_iq3_step<3>(s, lut),
@@ -86,7 +86,7 @@ template <int F> __device__ __forceinline__ void dq_test_body(const qwk_dq_args 
                 for (int e = 0; e < 8; e++) y[256 * blk + 64 * kg + 8 * j + e] = s.d * (float)v[j][e];
         }
     } else {
-        for (uint32_t i = threadIdx.x; i < a.K / 8; i += blockDim.x) {
+        for (uint32_t i = threadIdx.x; i < a.K / 8; i += qw_threads()) {
             const uint32_t blk = i >> 2, kg = i & 3;
             const uint8_t *b = row + 34 * blk;
             const h8 v = qw_q8_cvt(*(const u2a2 *)(b + 2 + 8 * kg));
@@ -111,7 +111,7 @@ extern "C" __global__ __launch_bounds__(64) void qwk_dq_test_f8(qwk_dq_args a) {
 template <int F> __device__ __forceinline__ void dq_test_kq(const qwk_dq_args &a, const uint32_t *tab) {
     const uint8_t *row = a.W + (size_t)blockIdx.x * a.rowbytes;
     float *y = a.y + (size_t)blockIdx.x * a.K;
-    for (uint32_t i = threadIdx.x; i < a.K / qw_kq<F>::BLK_K * 4; i += blockDim.x) {
+    for (uint32_t i = threadIdx.x; i < a.K / qw_kq<F>::BLK_K * 4; i += qw_threads()) {
         const uint32_t blk = i >> 2, kg = i & 3;
         qw_kq<F> b;
         b.load(row + (size_t)qw_kq<F>::BLK_B * blk, kg);
@@ -139,7 +139,7 @@ extern "C" __global__ __launch_bounds__(64) void qwk_dq_test_kq(qwk_dq_args a) {
 // Only the IQ3_S section is produced; the sections of formats without a gfx950 build stay zero. Grid: 32 x 256.
 #if QW_IN_PART(0)
 extern "C" __global__ void qwk_tab_init(qwk_tab_args a) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = blockIdx.x * qw_threads() + threadIdx.x;
     if (i >= QW_LUT_ENTRIES) return;
     const uint32_t s = qw_lut_slot(i);
     ((u2 *)(a.tab + QW_TAB_IQ3SS))[a.slot_order ? s : i] = qw_lut_entry(i);
@@ -154,9 +154,9 @@ __device__ __forceinline__ const uint8_t *pack_row(const qwk_pack_args &a, uint6
 }
 #if QW_IN_PART(0)
 extern "C" __global__ __launch_bounds__(256) void qwk_pack_iq3(qwk_pack_args a) {
-    const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (blockDim.x >> 6);
+    const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (qw_threads() >> 6);
     const uint32_t lane = threadIdx.x & 63, n = lane & 15, kg = lane >> 4;
-    for (uint64_t sl = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
+    for (uint64_t sl = (uint64_t)blockIdx.x * (qw_threads() >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
         const uint64_t tile = sl / a.nblk;
         const uint32_t blk = (uint32_t)(sl % a.nblk);
         const uint8_t *src = pack_row(a, tile, n) + 110 * blk;
@@ -173,9 +173,9 @@ extern "C" __global__ __launch_bounds__(256) void qwk_pack_iq3(qwk_pack_args a) 
 // lane takes are the ones qw_kq<14>::load reads for that lane's row and k-group.
 #if QW_IN_PART(0)
 extern "C" __global__ __launch_bounds__(256) void qwk_pack_q6(qwk_pack_args a) {
-    const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (blockDim.x >> 6);
+    const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (qw_threads() >> 6);
     const uint32_t lane = threadIdx.x & 63, n = lane & 15, kg = lane >> 4;
-    for (uint64_t sl = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
+    for (uint64_t sl = (uint64_t)blockIdx.x * (qw_threads() >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
         const uint64_t tile = sl / a.nblk;
         const uint8_t *src = pack_row(a, tile, n) + 210 * (sl % a.nblk);
         uint8_t *dst = a.dst + sl * QW_Q6_SLAB_BYTES;
@@ -195,9 +195,9 @@ extern "C" __global__ __launch_bounds__(256) void qwk_pack_q6(qwk_pack_args a) {
 // The tile-major copies of Q8_0 and Q4_K rows (layouts: QW_F_PACKED_Q8, QW_F_PACKED_Q4K in qw_kargs.h); a wave per (tile, 256 values).
 #if QW_IN_PART(0)
 extern "C" __global__ __launch_bounds__(256) void qwk_pack_q8(qwk_pack_args a) {
-    const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (blockDim.x >> 6);
+    const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (qw_threads() >> 6);
     const uint32_t lane = threadIdx.x & 63, n = lane & 15, kg = lane >> 4;
-    for (uint64_t sl = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
+    for (uint64_t sl = (uint64_t)blockIdx.x * (qw_threads() >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
         const uint8_t *src = pack_row(a, sl / a.nblk, n) + 272 * (sl % a.nblk);
         uint8_t *dst = a.dst + sl * QW_Q8_SLAB_BYTES;
 #pragma unroll
@@ -210,9 +210,9 @@ extern "C" __global__ __launch_bounds__(256) void qwk_pack_q8(qwk_pack_args a) {
     }
 }
 extern "C" __global__ __launch_bounds__(256) void qwk_pack_q4k(qwk_pack_args a) {
-    const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (blockDim.x >> 6);
+    const uint64_t nslab = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (qw_threads() >> 6);
     const uint32_t lane = threadIdx.x & 63, n = lane & 15, kg = lane >> 4;
-    for (uint64_t sl = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
+    for (uint64_t sl = (uint64_t)blockIdx.x * (qw_threads() >> 6) + (threadIdx.x >> 6); sl < nslab; sl += step) {
         const uint8_t *src = pack_row(a, sl / a.nblk, n) + 144 * (sl % a.nblk);
         uint8_t *dst = a.dst + sl * QW_Q4K_SLAB_BYTES;
         uint32_t r[8];
@@ -234,9 +234,9 @@ extern "C" __global__ __launch_bounds__(256) void qwk_pack_q4k(qwk_pack_args a) 
 // The tile-major copy of IQ4_NL rows (layout: QW_F_PACKED_NL in qw_kargs.h); a wave per (tile, chunk of ten blocks).
 #if QW_IN_PART(0)
 extern "C" __global__ __launch_bounds__(256) void qwk_pack_nl(qwk_pack_args a) {
-    const uint64_t nchunk = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (blockDim.x >> 6);
+    const uint64_t nchunk = a.ntiles * a.nblk, step = (uint64_t)gridDim.x * (qw_threads() >> 6);
     const uint32_t lane = threadIdx.x & 63, n = lane & 15, kg = lane >> 4;
-    for (uint64_t ch = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); ch < nchunk; ch += step) {
+    for (uint64_t ch = (uint64_t)blockIdx.x * (qw_threads() >> 6) + (threadIdx.x >> 6); ch < nchunk; ch += step) {
         const uint64_t tile = ch / a.nblk;
         const uint8_t *src = a.A + (tile * 16 + n) * a.rowbytes + 180 * (ch % a.nblk);
         uint8_t *dst = a.dst + ch * QW_NL_CHUNK_BYTES;
@@ -314,7 +314,7 @@ __device__ __forceinline__ void qw_fin_wg(const qwk_fin &f) {
 // 39.0 us, two 52.3 -> 46.6, eight 97.3 -> 79.2, sixteen 153 -> 102 (Pg from the sums in LDS at the end of the workgroup: 115).
 __device__ __forceinline__ void qw_back_fin(const qwk_back &k, const qwk_fin &f) {
     if (!f.flag) return;
-    const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    const uint32_t i0 = blockIdx.x * qw_threads() + threadIdx.x, step = gridDim.x * qw_threads();
     for (uint32_t p = 0; p < k.n; p++) {
         const uint32_t n16 = k.bytes[p] / 16;
         for (uint32_t i = i0; i < n16; i += step) ((u4 *)k.dst[p])[i] = ((const u4 *)k.src[p])[i];
@@ -331,7 +331,7 @@ __device__ __forceinline__ void qw_back_fin(const qwk_back &k, const qwk_fin &f)
 template <int F, int CH, bool XLDS> __device__ __forceinline__ void qmv_body(const qwk_qmv_args &a, u2 *lut, u4 *xf, f4 *red) {
     typedef qw_chunk<F, CH> C;
     const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4;
-    const uint32_t nw = gridDim.x * (blockDim.x >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x /* wave-major: see gu_body */;
+    const uint32_t nw = gridDim.x * (qw_threads() >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x /* wave-major: see gu_body */;
     const uint32_t cpr = a.K / (C::BLK_K * CH);
     const uint32_t nl = lane >> 2, kl = lane & 3; // (row, k-group) this lane loads
     auto rowp = [&](uint32_t t) {
@@ -406,7 +406,7 @@ QW_QMV(121, 2, true, _c2) QW_QMV(121, 1, true, _c1) // packed IQ3_S: a.rowbytes 
 // Matrices that the device takes in one go, one to four a launch, any of the formats: qw_small.hip.h.
 #if QW_IN_PART(0)
 template <int XN> __device__ __forceinline__ void qmvs_body(const qwk_qmvm_args &a, u4 *dyn) { // dyn: table (tabu units), then a wave's activations, behind them in the same place its partial sums
-    const uint32_t lane = qw_lane(), wave = qw_wave(), nw = blockDim.x >> 6, own = a.sh ? 32u << a.sh : 64;
+    const uint32_t lane = qw_lane(), wave = qw_wave(), nw = qw_threads() >> 6, own = a.sh ? 32u << a.sh : 64;
     u2 *tab = (u2 *)dyn;
     u4 *x = dyn + a.tabu + wave * own;
     uint32_t j = 0, t = blockIdx.x;
@@ -518,7 +518,7 @@ extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_qmvm(qwk_qmvm_args 
     qw_stage_x(L.xf, a.x, a.xstride, a.K, a.nb);
     __syncthreads();
     if (a.sums) { // sums of 32 activations per token, in index order
-        for (uint32_t i = threadIdx.x; i < (a.K >> 5) * 16; i += blockDim.x) {
+        for (uint32_t i = threadIdx.x; i < (a.K >> 5) * 16; i += qw_threads()) {
             const uint32_t c = i >> 4, m = i & 15;
             float sum = 0;
 #pragma unroll
@@ -531,7 +531,7 @@ extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_qmvm(qwk_qmvm_args 
         }
         __syncthreads();
     }
-    const uint32_t lane = qw_lane(), nw = gridDim.x * (blockDim.x >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x /* wave-major: see gu_body */;
+    const uint32_t lane = qw_lane(), nw = gridDim.x * (qw_threads() >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x /* wave-major: see gu_body */;
     const qw_afrag_kq af = {L.xf, L.xs, lane & 15, lane >> 4};
     const bool k256 = a.K % 256 == 0;
     uint32_t toff = 0; // tiles (split == 1) or tile groups (split > 1) of the matrices before j
@@ -574,7 +574,7 @@ extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_qmvm(qwk_qmvm_args 
 template <int NT> __device__ __forceinline__ void qmv_valu_body(const qwk_qmv_args &a, u2 *lut, u4 *xf) {
     typedef qw_chunk<QW_F_PACKED, 2> C;
     const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4;
-    const uint32_t nw = gridDim.x * (blockDim.x >> 6), w0 = blockIdx.x * (blockDim.x >> 6) + qw_wave(), cpr = a.K / 512;
+    const uint32_t nw = gridDim.x * (qw_threads() >> 6), w0 = blockIdx.x * (qw_threads() >> 6) + qw_wave(), cpr = a.K / 512;
     float acc[NT];
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[t] = 0;
@@ -894,7 +894,7 @@ __device__ __forceinline__ bool qw_select_fast_e(uint32_t E) { return E == 64 ||
 template <uint32_t NSTAGE = 0, class H>
 __device__ __forceinline__ void select_all(const qwk_select_args &a, qw_sel_scratch &s, qw_sel_cache &c, float *lgs, bool store, H stage, bool need_w = false) {
     need_w = need_w || store;
-    const uint32_t tid = threadIdx.x, nth = blockDim.x, wave = qw_wave(), lane = qw_lane(), nwv = nth >> 6;
+    const uint32_t tid = threadIdx.x, nth = qw_threads(), wave = qw_wave(), lane = qw_lane(), nwv = nth >> 6;
     const uint32_t E = a.E, K = a.topk, gnb = a.gnb, GU = gnb * K, UM = a.nbr * K;
     const bool fast = qw_select_fast_e(E);
     const uint32_t tw = nwv - NSTAGE; // the waves that take tokens
@@ -1032,14 +1032,14 @@ __device__ __forceinline__ void qw_sel_load(qw_sel_cache &c, const uint8_t *sel,
     const uint32_t GU = gnb * K;
     const uint32_t *ue = (const uint32_t *)(sel + QW_SEL_OFF_UE(gnb, K)), *mask = (const uint32_t *)(sel + QW_SEL_OFF_MASK(gnb, K));
     const uint32_t *slot = (const uint32_t *)(sel + QW_SEL_OFF_SLOT(gnb, K));
-    for (uint32_t i = threadIdx.x; i < GU; i += blockDim.x) c.ue[i] = ue[i], c.mask[i] = mask[i];
-    for (uint32_t i = threadIdx.x; i < GU * gnb / 4; i += blockDim.x) ((uint32_t *)c.slot)[i] = slot[i];
+    for (uint32_t i = threadIdx.x; i < GU; i += qw_threads()) c.ue[i] = ue[i], c.mask[i] = mask[i];
+    for (uint32_t i = threadIdx.x; i < GU * gnb / 4; i += qw_threads()) ((uint32_t *)c.slot)[i] = slot[i];
     if (threadIdx.x == 0) c.U = *(const uint32_t *)sel;
 }
 
 // The sums of 32 activations of every token from their fragments in LDS, in index order (all threads; a barrier before and after).
 __device__ __forceinline__ void qw_sum32(const u4 *xf, float *xs, uint32_t K) {
-    for (uint32_t i = threadIdx.x; i < (K >> 5) * 16; i += blockDim.x) {
+    for (uint32_t i = threadIdx.x; i < (K >> 5) * 16; i += qw_threads()) {
         const uint32_t c = i >> 4, m = i & 15;
         float sum = 0;
 #pragma unroll
@@ -1138,7 +1138,7 @@ __device__ __forceinline__ void gu_tasks(const qwk_gu_args &a, const u2 *lut, co
 template <int FGU, int CHGU, int FSG, int CHSG, class HS, class SEL>
 __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, float *xs, qw_sel_cache *sc, qw_sel_scratch *ss, HS &hs, bool all_w, SEL selected) {
     bool staged = false, tabled = false;
-    if (threadIdx.x == 0) sc->qnext = blockDim.x >> 6; // (nothing below writes it; a barrier follows on every path)
+    if (threadIdx.x == 0) sc->qnext = qw_threads() >> 6; // (nothing below writes it; a barrier follows on every path)
     if (threadIdx.x == 0) QW_WSTAMP(12);
     QW_DSTAMP(0);
     QW_SSTAMP(0);
@@ -1164,7 +1164,7 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, f
             qw_sel_scratch &so = *(qw_sel_scratch *)xf;
             select_all(sa, so, *sc, (float *)(xf + (sizeof(qw_sel_scratch) + 15) / 16), blockIdx.x == 0, [](uint32_t, uint32_t) {}, all_w);
             if (all_w) { // (the caller reads the weights from ss)
-                for (uint32_t i = threadIdx.x; i < a.gnb * (a.topk + 1); i += blockDim.x) ss->w[i] = so.w[i];
+                for (uint32_t i = threadIdx.x; i < a.gnb * (a.topk + 1); i += qw_threads()) ss->w[i] = so.w[i];
                 __syncthreads();
             }
         }
@@ -1172,7 +1172,7 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, f
         if (!a.shared) qw_sel_load(*sc, a.sel, a.topk, a.gnb);
         if (all_w) {
             const float *wg = (const float *)(a.sel + QW_SEL_OFF_W(a.gnb, a.topk));
-            for (uint32_t i = threadIdx.x; i < a.gnb * (a.topk + 1); i += blockDim.x) ss->w[i] = wg[i];
+            for (uint32_t i = threadIdx.x; i < a.gnb * (a.topk + 1); i += qw_threads()) ss->w[i] = wg[i];
         }
         __syncthreads();
     }
@@ -1189,7 +1189,7 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, f
     };
     // Waves are numbered wave-major (wave w of workgroup b is number w * gridDim.x + b), so that when the tiles do not
     // divide evenly the waves with one tile more are spread over all compute units instead of filling the first ones.
-    const uint32_t nw = gridDim.x * (blockDim.x >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x;
+    const uint32_t nw = gridDim.x * (qw_threads() >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x;
     if (FSG != 0) {
         if (a.Wsg) { // the shared expert's tiles go to the first waves
             qwk_gu_args sa = a;
@@ -1300,7 +1300,7 @@ struct qw_pre_x {
 // Binary16 rows, sixteen a workgroup.
 __device__ __forceinline__ void pre_router(const qwk_pre_args &a, qw_pre_lds &L) {
     const qwk_router_args &r = a.r;
-    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave(), nwv = (blockDim.x >> 6) < 8 ? blockDim.x >> 6 : 8;
+    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave(), nwv = (qw_threads() >> 6) < 8 ? qw_threads() >> 6 : 8;
     u4 *const x = L.x + wave * 512;
     f4 acc = {0, 0, 0, 0};
     if (wave < nwv) {
@@ -1354,10 +1354,10 @@ template <int NB> __device__ __forceinline__ void pre_router_bf(const qwk_pre_ar
         if (64 * k < units) wv[k] = *(const u4 *)(w + 8 * (lane + 64 * k < units ? lane + 64 * k : 0));
 #pragma unroll
     for (uint32_t k = 0; k < 4; k++) // (two tokens to a round of the workgroup's threads)
-        if (k * blockDim.x < nx) xv[k] = ((const u4 *)(r.x + (size_t)t0 * r.D))[threadIdx.x + k * blockDim.x < nx ? threadIdx.x + k * blockDim.x : 0];
+        if (k * qw_threads() < nx) xv[k] = ((const u4 *)(r.x + (size_t)t0 * r.D))[threadIdx.x + k * qw_threads() < nx ? threadIdx.x + k * qw_threads() : 0];
 #pragma unroll
     for (uint32_t k = 0; k < 4; k++)
-        if (threadIdx.x + k * blockDim.x < nx) L.x[threadIdx.x + k * blockDim.x] = xv[k];
+        if (threadIdx.x + k * qw_threads() < nx) L.x[threadIdx.x + k * qw_threads()] = xv[k];
     __syncthreads();
     float acc[NB];
 #pragma unroll
@@ -1389,7 +1389,7 @@ template <int NB> __device__ __forceinline__ void pre_router_bf(const qwk_pre_ar
 template <int WF> __device__ __forceinline__ void pre_router_any(const qwk_pre_args &a, qw_pre_lds &L) {
     if constexpr (WF == 1) pre_router(a, L);
     else {
-        const uint32_t nwv = blockDim.x >> 6, nrb = (a.r.E + nwv) / nwv, t0 = 8 * (blockIdx.x / nrb), r0 = blockIdx.x % nrb * nwv, nt = a.r.nb - t0 < 8 ? a.r.nb - t0 : 8;
+        const uint32_t nwv = qw_threads() >> 6, nrb = (a.r.E + nwv) / nwv, t0 = 8 * (blockIdx.x / nrb), r0 = blockIdx.x % nrb * nwv, nt = a.r.nb - t0 < 8 ? a.r.nb - t0 : 8;
         if (nt == 1) pre_router_bf<1>(a, L, r0, t0, nt);
         else if (nt == 2) pre_router_bf<2>(a, L, r0, t0, nt);
         else if (nt <= 4) pre_router_bf<4>(a, L, r0, t0, nt);
@@ -1422,7 +1422,7 @@ template <int F> __device__ __forceinline__ f4 pre_mac(const uint32_t (&r)[32], 
 template <int SH> __device__ __forceinline__ void pre_shared(const qwk_pre_args &a, uint32_t t, qw_pre_lds &L) {
     const qwk_router_args &r = a.r;
     const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave();
-    const uint32_t nwv = SH == 8 ? r.D / 512 : blockDim.x >> 6; // the waves that take part
+    const uint32_t nwv = SH == 8 ? r.D / 512 : qw_threads() >> 6; // the waves that take part
     u4 *const x = L.x + wave * (SH == 8 ? 1024 : 512);
     const qw_afrag_small af = {x, n & ((1u << a.sh) - 1), a.sh};
     f4 g = {0, 0, 0, 0};
@@ -1447,7 +1447,7 @@ template <int SH> __device__ __forceinline__ void pre_shared(const qwk_pre_args 
         else c.load((lane < 32 ? a.Wg : a.Wu) + ((size_t)8 * t + ((lane >> 2) & 7)) * a.rbg + wave * qw_small_blk<SH>::BYTES, lane & 3);
         xv.load(r, 256 * wave);
         if constexpr (SH == QW_F_PACKED) { // the table, a unit a thread or four (a few by several threads)
-            const uint32_t few = blockDim.x < 256 ? 4 : 1;
+            const uint32_t few = qw_threads() < 256 ? 4 : 1;
             for (uint32_t i = 0; i < few; i++) ((u4 *)L.tab)[(threadIdx.x + 64 * i) & 255] = ((const u4 *)a.ctab)[(threadIdx.x + 64 * i) & 255];
             if (threadIdx.x < 16) qw_small_signs(L.tab, threadIdx.x);
         }
@@ -1577,7 +1577,7 @@ __device__ __forceinline__ void pre_pair(const qwk_pre_args &a, uint32_t t, qw_p
         if (wave) ((f4 *)x)[lane] = g, ((f4 *)x)[64 + lane] = u;
         __syncthreads();
         if (wave) return;
-        for (uint32_t q = 1; q < blockDim.x >> 6; q++) g += ((const f4 *)L.x)[q * 512 + lane], u += ((const f4 *)L.x)[q * 512 + 64 + lane];
+        for (uint32_t q = 1; q < qw_threads() >> 6; q++) g += ((const f4 *)L.x)[q * 512 + lane], u += ((const f4 *)L.x)[q * 512 + 64 + lane];
     }
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++)
@@ -1614,7 +1614,7 @@ extern "C" __global__ __launch_bounds__(64 * QW_PRE_WAVES) void qwk_qmvm_swiglu(
 // family: the arithmetic and the two-plane store of pre_shared. One thread per (token, column).
 #if QW_IN_PART(2)
 extern "C" __global__ __launch_bounds__(256) void qwk_sh_act(qwk_shact_args a) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = blockIdx.x * qw_threads() + threadIdx.x;
     if (i >= a.nb * a.I) return;
     const uint32_t t = i / a.I, j = i % a.I;
     const float g = a.g[i], up = a.u[i], h = g / (1.0f + __expf(-g)) * up;
@@ -1664,7 +1664,7 @@ struct qw_dn_seg { // one expert's part of a workgroup's range (all fields wave-
 template <int F, int CH, class S> __device__ __forceinline__ void dn_range_run(const qwk_dn_args &a, const u2 *lut, const uint16_t *arows, const qw_dn_seg &g0, const qw_dn_seg &g1,
                                                                                  bool both, const uint8_t *slots0, const uint8_t *slots1, S ready) {
     typedef qw_chunk<F, CH> C;
-    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, K = a.topk, nwv = blockDim.x >> 6, nl = lane >> 2;
+    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, K = a.topk, nwv = qw_threads() >> 6, nl = lane >> 2;
     const uint32_t ntask = g0.ntile + (both ? g1.ntile : 0), cpr = a.I / (C::BLK_K * CH);
     // per lane: where the results of tokens 4 kg .. 4 kg + 3 go in either segment, as float offsets of row 0
     // (token * topk + slot for a routed expert, token for the shared one; 32 bits hold them), ~0 = not picked
@@ -1758,7 +1758,7 @@ template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_r
             staged = true;
             const uint32_t upr = a.I / 8, ncb = upr / 4, ninst = (both ? 2 : 1) * 2 * ncb; // 16-byte units per plane row; instructions
             const uint32_t lane = qw_lane(), t = lane & 15, rows = g0.mask | (both ? g1.mask << 16 : 0), nrows = (uint32_t)__builtin_popcount(rows);
-            if (nrows * 2 * upr <= blockDim.x) {
+            if (nrows * 2 * upr <= qw_threads()) {
                 // few rows (a token or two per expert): one 16-byte unit per thread through a register, the waves
                 // of a row finding its bit in the mask by a (mostly scalar) walk
                 // (a row of both planes is 2 upr threads: whole waves when I is a multiple of 256, else a wave may span two rows)
@@ -1772,7 +1772,7 @@ template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_r
                 }
             } else {
                 const uint32_t s0 = g0.sh ? K : slot[g0.u * gnb + t], s1 = !both ? 0 : g1.sh ? K : slot[g1.u * gnb + t]; // result slot of token t
-                for (uint32_t q = qw_wave(); q < ninst; q += blockDim.x >> 6) {
+                for (uint32_t q = qw_wave(); q < ninst; q += qw_threads() >> 6) {
                     const uint32_t sg = q / (2 * ncb), r = q % (2 * ncb), pl = r / ncb, cb = r % ncb;
                     const uint32_t m = sg ? g1.mask : g0.mask, sl = sg ? s1 : s0, c = 4 * cb + (lane >> 4);
                     if ((m >> t) & 1)
@@ -1861,7 +1861,7 @@ __device__ __forceinline__ f4 dnc_tile(const qwk_dn_args &a, const u2 *lut, cons
 }
 template <int F, int CH, int FSD, int CHSD>
 __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *part /* [QW_DNC_MAXNB][topk + 1][16] */, float *wl /* [QW_DNC_MAXNB][topk + 1] */, qw_sel_cache *sc) {
-    const uint32_t K = a.topk, gnb = a.gnb, tpe = a.D / 16, tile = blockIdx.x, lane = qw_lane(), n = lane & 15, kg = lane >> 4, nwv = blockDim.x >> 6;
+    const uint32_t K = a.topk, gnb = a.gnb, tpe = a.D / 16, tile = blockIdx.x, lane = qw_lane(), n = lane & 15, kg = lane >> 4, nwv = qw_threads() >> 6;
     // The table through registers, asked for first and stored behind the record (published by the barrier of ready()): a
     // copy straight into LDS kept every wave in the issue of its loads for more than a microsecond, between the record and
     // the first weights (which need the record).
@@ -1880,7 +1880,7 @@ __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *p
     }
     qw_sel_load(*sc, a.sel, K, gnb);
     const float *wg = (const float *)(a.sel + QW_SEL_OFF_W(gnb, K));
-    for (uint32_t i = threadIdx.x; i < a.nbr * (K + 1); i += blockDim.x) wl[i] = wg[i];
+    for (uint32_t i = threadIdx.x; i < a.nbr * (K + 1); i += qw_threads()) wl[i] = wg[i];
     if (qw_has_tab(F) || qw_has_tab(FSD)) qw_kq_tab_build((uint32_t *)lut); // the byte table of the 4-bit codebook instead
     if constexpr (TAB) {
 #pragma unroll
@@ -2152,7 +2152,7 @@ __device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_l
             L.ue[tid] = r_ue, L.mask[tid] = (uint16_t)r_mk, L.slot4[tid] = s4;
         }
         if (hasw) L.wl[tid] = r_w;
-        if (tid == 0) L.U = r_U, L.q[0] = blockDim.x >> 6, L.q[1] = 0;
+        if (tid == 0) L.U = r_U, L.q[0] = qw_threads() >> 6, L.q[1] = 0;
     }
     __syncthreads();
     QW_DSTAMP(7);
@@ -2196,7 +2196,7 @@ __device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_l
     }
     QW_DSTAMP(9);
     __syncthreads();
-    for (uint32_t j = tid; j < nt * rw; j += blockDim.x) { // rank order, then the shared expert (qwk_cmb's arithmetic)
+    for (uint32_t j = tid; j < nt * rw; j += qw_threads()) { // rank order, then the shared expert (qwk_cmb's arithmetic)
         const uint32_t t = j >> (4 + __builtin_ctz(tpw)), i = j & (rw - 1), r = g * rw + i;
         const float *w = L.wl + t * (K + 1), *p = L.part + t * (K + 1) * rw + i;
         float o = 0;
@@ -2298,13 +2298,13 @@ template <int FSD, int CHSD> __device__ __forceinline__ void gud_body(const qwk_
         // makes the whole list: all write the same values)
         uint32_t GU = gnb * K;
         if (GU > QW_DNQ_MAXU) GU = QW_DNQ_MAXU;
-        for (uint32_t i = tid; i < nt * (K + 1); i += blockDim.x) L.wl[i] = L.u.ss.w[t0 * (K + 1) + i];
-        for (uint32_t i = tid; i < GU; i += blockDim.x) {
+        for (uint32_t i = tid; i < nt * (K + 1); i += qw_threads()) L.wl[i] = L.u.ss.w[t0 * (K + 1) + i];
+        for (uint32_t i = tid; i < GU; i += qw_threads()) {
             uint32_t s4 = 0;
             for (uint32_t j = 0; j < nt; j++) s4 |= (uint32_t)L.sc.slot[i * gnb + t0 + j] << (8 * j);
             L.ue[i] = L.sc.ue[i], L.mask[i] = (uint16_t)L.sc.mask[i], L.slot4[i] = s4;
         }
-        if (tid == 0) L.hcount = 0, L.bail = 0, L.dq[0] = blockDim.x >> 6, L.dq[1] = 0;
+        if (tid == 0) L.hcount = 0, L.bail = 0, L.dq[0] = qw_threads() >> 6, L.dq[1] = 0;
         uint32_t U = L.sc.U;
         if (U > GU) U = GU;
         const uint32_t want = (1u << nt) - 1;
@@ -2330,7 +2330,7 @@ template <int FSD, int CHSD> __device__ __forceinline__ void gud_body(const qwk_
         QW_STAMP(4);
         uint32_t cnt = L.hcount;
         if (cnt > QW_GUD_HCAP) cnt = QW_GUD_HCAP;
-        for (uint32_t i = tid; i < cnt * 4; i += blockDim.x) { // two columns a thread, a dword a plane
+        for (uint32_t i = tid; i < cnt * 4; i += qw_threads()) { // two columns a thread, a dword a plane
             const uint32_t e = i >> 2, c = 2 * (i & 3), v0 = L.u.hb.val[e * 8 + c], v1 = L.u.hb.val[e * 8 + c + 1];
             uint32_t *p = (uint32_t *)(a.H + L.u.hb.off[e] + c);
             qw_st_coh(p, (v0 & 0xffffu) | (v1 << 16));
@@ -2381,7 +2381,7 @@ template <int FSD, int CHSD> __device__ __forceinline__ void gud_body(const qwk_
     __syncthreads();
     QW_STAMP(9);
     if (L.bail) return;
-    for (uint32_t j = tid; j < nt * rw; j += blockDim.x) { // rank order, then the shared expert (qwk_cmb's arithmetic)
+    for (uint32_t j = tid; j < nt * rw; j += qw_threads()) { // rank order, then the shared expert (qwk_cmb's arithmetic)
         const uint32_t t = j >> (4 + __builtin_ctz(tpw)), i = j & (rw - 1), r = g * rw + i;
         const float *w = L.wl + t * (K + 1), *p = L.u.part + t * (K + 1) * rw + i;
         float o = 0;
@@ -2430,7 +2430,7 @@ template <int F, int FSD> __device__ __forceinline__ void dn_any_body(const qwk_
     if (F == 20 || FSD == 20) qw_kq_tab_build((uint32_t *)lut); // the byte table of the 4-bit codebook (IQ3_S never meets it here)
     qw_sel_load(*sc, a.sel, a.topk, a.gnb);
     __syncthreads();
-    const uint32_t nw = gridDim.x * (blockDim.x >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x /* wave-major: see gu_body */;
+    const uint32_t nw = gridDim.x * (qw_threads() >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x /* wave-major: see gu_body */;
     if (FSD != 0) {
         if (a.Wsd) shared_down_tiles<FSD == 0 ? 8 : FSD, 1>(a, lut, w0, nw);
     }
@@ -2445,7 +2445,7 @@ __device__ __forceinline__ void dn_rt_body(const qwk_dn_args &a, u2 *lut, qw_sel
     qw_kq_tab_build((uint32_t *)tab);
     qw_sel_load(*sc, a.sel, a.topk, a.gnb);
     __syncthreads();
-    const uint32_t nw = gridDim.x * (blockDim.x >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x;
+    const uint32_t nw = gridDim.x * (qw_threads() >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x;
     if (a.Wsd) switch (a.fsd) {
         case 8: shared_down_tiles<8, 1>(a, lut, w0, nw); break;
         case 21: shared_down_tiles<21, 1>(a, lut, w0, nw); break;
@@ -2494,11 +2494,11 @@ QW_DN_ANY(20, 0, qwk_dn_f20_any) QW_DN_ANY(20, 20, qwk_dn_f20_any_s20) QW_DN_ANY
 // the packing sequence several times, and all of it is recorded before any of it runs.
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(256) void qwk_zero(qwk_zero_args a) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = blockIdx.x * qw_threads() + threadIdx.x;
     if (i < a.n) a.x[i] = 0;
 }
 extern "C" __global__ __launch_bounds__(256) void qwk_moe_count(qwk_count_args a) {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t p = blockIdx.x * qw_threads() + threadIdx.x;
     if (p < a.P && a.ids[p] < a.E) atomicAdd(&a.counts[a.ids[p]], 1u);
 }
 #endif
@@ -2531,7 +2531,7 @@ extern "C" __global__ __launch_bounds__(1024) void qwk_moe_plan(qwk_plan_args a)
             if (tile0 + t < a.max_tiles) *(u4 *)(a.tiles + 4 * (tile0 + t)) = u4{tid, r, r + a.tm < row0 + c ? r + a.tm : row0 + c, 0};
         }
     }
-    for (uint32_t t = total_t + tid; t < a.max_tiles; t += blockDim.x) *(u4 *)(a.tiles + 4 * t) = u4{0, 0, 0, 0}; // unused entries
+    for (uint32_t t = total_t + tid; t < a.max_tiles; t += qw_threads()) *(u4 *)(a.tiles + 4 * t) = u4{0, 0, 0, 0}; // unused entries
 }
 #endif
 // One workgroup per pair: take the next row of the pair's expert, remember it, copy the token's row there.
@@ -2548,7 +2548,7 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_scatter(qwk_scatter_ar
     if (pos >= a.P) return; // an expert id outside the table: the pair is dropped
     const u4 *src = (const u4 *)(a.X + (size_t)(p / a.topk) * a.KD);
     u4 *dst = (u4 *)(a.Xs + (size_t)pos * a.KD);
-    for (uint32_t i = threadIdx.x; i < a.KD / 8; i += blockDim.x) dst[i] = src[i];
+    for (uint32_t i = threadIdx.x; i < a.KD / 8; i += qw_threads()) dst[i] = src[i];
 }
 #endif
 // The four launches above as one, for a step of about a thousand pairs at most: a workgroup per pair, and every workgroup
@@ -2632,7 +2632,7 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_prep(qwk_prep_args a) 
 extern "C" __global__ __launch_bounds__(512) void qwk_moe_prep_slices(qwk_prep_args a) {
     __shared__ uint32_t cnt[1024], at[1024], wr[8], wt[8], id[QW_PREP_SLICE], pos[QW_PREP_SLICE];
     qw_started(a.t_start);
-    const uint32_t tid = threadIdx.x, nth = blockDim.x, lane = tid & 63, wave = tid >> 6, nwv = nth >> 6;
+    const uint32_t tid = threadIdx.x, nth = qw_threads(), lane = tid & 63, wave = tid >> 6, nwv = nth >> 6;
     const uint32_t p0 = blockIdx.x * a.slice < a.P ? blockIdx.x * a.slice : a.P, p1 = p0 + a.slice < a.P ? p0 + a.slice : a.P, np = p1 - p0;
     for (uint32_t e = tid; e < 1024; e += nth) cnt[e] = 0;
     if (tid < np) id[tid] = a.ids[p0 + tid];
@@ -2721,7 +2721,7 @@ extern "C" __global__ __launch_bounds__(512) void qwk_moe_prep_slices(qwk_prep_a
 // H = SiLU(gate) * up, binary16 in and out, the product rounded once (kernels/moe_prefill.metal:95-103, kernels/prefill.metal:485-488)
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(256) void qwk_moe_act(qwk_act_args a) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = blockIdx.x * qw_threads() + threadIdx.x;
     if (i >= a.n) return;
     float g, u;
     if (a.U) g = qw_h2f(a.G[i]), u = qw_h2f(a.U[i]);
@@ -2781,7 +2781,7 @@ template <int F, int CH> __device__ __forceinline__ void pf_body(const qwk_pf_ar
     if (F == 20) qw_kq_tab_build((uint32_t *)lut); // the byte table of the 4-bit codebook
     __syncthreads();
     uint32_t mine = 0;
-    for (uint32_t t = threadIdx.x; t < a.max_tiles; t += blockDim.x) {
+    for (uint32_t t = threadIdx.x; t < a.max_tiles; t += qw_threads()) {
         const u4 e = *(const u4 *)(a.tiles + 4 * t);
         tl[t] = e;
         mine += e.z > e.y;
@@ -2789,7 +2789,7 @@ template <int F, int CH> __device__ __forceinline__ void pf_body(const qwk_pf_ar
     if (mine) atomicAdd(cnt, mine);
     __syncthreads();
     const uint32_t used = *cnt, ntn = a.ntn, ntasks = used * ntn, cpr = a.K / (C::BLK_K * CH);
-    const uint32_t nw = gridDim.x * (blockDim.x >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x /* wave-major: see gu_body */;
+    const uint32_t nw = gridDim.x * (qw_threads() >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x /* wave-major: see gu_body */;
     f4 acc[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
     qw_task_pipeline<C>(ntasks, w0, nw, cpr, CH * C::BLK_B, F == QW_F_PACKED ? lane : lane & 3,
         [&](uint32_t task) {
@@ -2867,12 +2867,12 @@ extern "C" __global__ __launch_bounds__(64 * QW_PFG_WAVES) void qwk_pfg_f120(qwk
 // issued) and its waves walk the tiles with the activations read from LDS.
 template <int CH> __device__ __forceinline__ void pf_range_body(const qwk_pf_args &a, u2 *lut, u4 *xf, uint32_t *cnt) {
     typedef qw_chunk<QW_F_PACKED, CH> C;
-    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, nwv = blockDim.x >> 6;
+    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, nwv = qw_threads() >> 6;
     if (threadIdx.x == 0) *cnt = 0;
     qw_lut_copy_issue(lut, (const u2 *)a.glut); // lands while the table of entries is read: one memory round trip for both
     __syncthreads();
     uint32_t mine = 0; // the non-empty entries are the first ones of the table
-    for (uint32_t t = threadIdx.x; t < a.max_tiles; t += blockDim.x) {
+    for (uint32_t t = threadIdx.x; t < a.max_tiles; t += qw_threads()) {
         const u4 e = *(const u4 *)(a.tiles + 4 * t);
         mine += e.z > e.y;
     }
@@ -2929,7 +2929,7 @@ QW_PFR(2, qwk_pfr_f121_c2) QW_PFR(1, qwk_pfr_f121_c1)
 // Rank order, then the shared expert. One thread per (token, row).
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(256) void qwk_cmb(qwk_cmb_args a) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = blockIdx.x * qw_threads() + threadIdx.x;
     if (i >= a.nbr * a.D) return;
     const uint32_t t = i / a.D, row = i % a.D, K = a.topk;
     const float *w = (const float *)(a.sel + QW_SEL_OFF_W(a.gnb, K)) + t * (K + 1);
@@ -2952,8 +2952,8 @@ extern "C" __global__ __launch_bounds__(256) void qwk_cmb(qwk_cmb_args a) {
 extern "C" __global__ __launch_bounds__(256) void qwk_bw_read(qwk_mem_args a) {
     const u4 *p = (const u4 *)a.src;
     u4 s = {0, 0, 0, 0};
-    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t step = (uint64_t)gridDim.x * qw_threads();
+    uint64_t i = (uint64_t)blockIdx.x * qw_threads() + threadIdx.x;
     for (; i + 3 * step < a.n; i += 4 * step) {
         const u4 v0 = p[i], v1 = p[i + step], v2 = p[i + 2 * step], v3 = p[i + 3 * step];
         s ^= v0 ^ v1 ^ v2 ^ v3;
@@ -2994,7 +2994,7 @@ template <int W> __device__ __forceinline__ float qw_sum4(float d0, float d1, fl
 // tokens, 10.0 -> 8.9 at sixteen, up 6.0 -> 5.0 and 8.5 -> 8.0 (D = 2048), with the same bits.
 template <uint32_t R> __device__ __forceinline__ void hc_down_body(const qwk_hc_args &a, float (*part)[QW_HC_TG][17]) {
     const uint32_t tg = (a.nb + gridDim.z - 1) / gridDim.z; // tokens of a group: as even as can be (five tokens: three and two)
-    const uint32_t rb = blockIdx.x, s = blockIdx.y, t0 = blockIdx.z * tg, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, nwv = blockDim.x >> 6;
+    const uint32_t rb = blockIdx.x, s = blockIdx.y, t0 = blockIdx.z * tg, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, nwv = qw_threads() >> 6;
     const uint32_t nt = a.nb - t0 < tg ? a.nb - t0 : tg;
     QW_HSTAMP(0);
     const bool is_inj = rb == QW_HC_LR / R;
@@ -3053,7 +3053,7 @@ template <uint32_t R> __device__ __forceinline__ void hc_down_body(const qwk_hc_
     QW_HSTAMP(3);
     __syncthreads();
     QW_HSTAMP(4);
-    for (uint32_t j = tid; j < nt * 17; j += blockDim.x) {
+    for (uint32_t j = tid; j < nt * 17; j += qw_threads()) {
         const uint32_t tt = j / 17, r = j % 17;
         if (r < 16 && r >= nrow) continue;
         float sum = 0;
@@ -3083,19 +3083,19 @@ extern "C" __global__ __launch_bounds__(512) void qwk_hc_down_r16(qwk_hc_args a)
 // (kernels/hyper_gg.metal:165-181, 312-340). rs [nt][HC] and sx [nt][LR] are in LDS; ends with a barrier.
 __device__ __forceinline__ void hc_mid(const qwk_hc_args &a, uint32_t t0, uint32_t nt, float *rs, float *sx, float *injo) {
     const float *pd = a.pd + (size_t)t0 * QW_HC * QW_HC_PDS;
-    for (uint32_t j = threadIdx.x; j < nt * QW_HC; j += blockDim.x) rs[j] = rsqrtf(pd[j * QW_HC_PDS + QW_HC_LR + QW_HC] / (float)a.D + 1e-6f);
+    for (uint32_t j = threadIdx.x; j < nt * QW_HC; j += qw_threads()) rs[j] = rsqrtf(pd[j * QW_HC_PDS + QW_HC_LR + QW_HC] / (float)a.D + 1e-6f);
     __syncthreads();
-    for (uint32_t j0 = threadIdx.x; j0 < nt * QW_HC_LR; j0 += 4 * blockDim.x) { // four elements a round: their sixteen loads go out together
+    for (uint32_t j0 = threadIdx.x; j0 < nt * QW_HC_LR; j0 += 4 * qw_threads()) { // four elements a round: their sixteen loads go out together
         float p[4][QW_HC];
 #pragma unroll
         for (uint32_t e = 0; e < 4; e++) {
-            const uint32_t j = j0 + e * blockDim.x, t = j / QW_HC_LR, r = j % QW_HC_LR;
+            const uint32_t j = j0 + e * qw_threads(), t = j / QW_HC_LR, r = j % QW_HC_LR;
 #pragma unroll
             for (uint32_t q = 0; q < QW_HC; q++) p[e][q] = j < nt * QW_HC_LR ? pd[(t * QW_HC + q) * QW_HC_PDS + r] : 0.0f;
         }
 #pragma unroll
         for (uint32_t e = 0; e < 4; e++) {
-            const uint32_t j = j0 + e * blockDim.x, t = j / QW_HC_LR;
+            const uint32_t j = j0 + e * qw_threads(), t = j / QW_HC_LR;
             if (j >= nt * QW_HC_LR) break;
             float d = 0;
 #pragma unroll
@@ -3105,7 +3105,7 @@ __device__ __forceinline__ void hc_mid(const qwk_hc_args &a, uint32_t t0, uint32
         }
     }
     if (injo)
-        for (uint32_t j = threadIdx.x; j < nt * QW_HC * QW_HC; j += blockDim.x) // j = (t, s, q)
+        for (uint32_t j = threadIdx.x; j < nt * QW_HC * QW_HC; j += qw_threads()) // j = (t, s, q)
             injo[t0 * QW_HC * QW_HC + j] = rs[j / QW_HC] * pd[(j / QW_HC) * QW_HC_PDS + QW_HC_LR + j % QW_HC];
     __syncthreads();
 }
@@ -3115,7 +3115,7 @@ extern "C" __global__ __launch_bounds__(320) void qwk_hc_mid(qwk_hc_args a) {
     __shared__ float rs[QW_HC], sx[QW_HC_LR];
     const uint32_t t = blockIdx.x;
     hc_mid(a, t, 1, rs, sx, a.want_inj ? a.injo : nullptr);
-    for (uint32_t r = threadIdx.x; r < QW_HC_LR; r += blockDim.x) a.sx[t * QW_HC_LR + r] = sx[r];
+    for (uint32_t r = threadIdx.x; r < QW_HC_LR; r += qw_threads()) a.sx[t * QW_HC_LR + r] = sx[r];
     if (threadIdx.x < QW_HC) a.rs[t * QW_HC + threadIdx.x] = rs[threadIdx.x];
 }
 #endif
@@ -3178,13 +3178,13 @@ template <bool GIVEN> __device__ __forceinline__ void hc_up_body(const qwk_hc_ar
         js[tid / QW_HC][tid % QW_HC] = a.apply ? 2.0f / (1.0f + expf(-t / QW_HC)) : 0.0f; // hc_coef
     }
     if (GIVEN) {
-        for (uint32_t j0 = tid; j0 < nt * QW_HC_LR; j0 += 8 * blockDim.x) { // eight loads in flight a thread
+        for (uint32_t j0 = tid; j0 < nt * QW_HC_LR; j0 += 8 * qw_threads()) { // eight loads in flight a thread
             float v[8];
 #pragma unroll
-            for (uint32_t e = 0; e < 8; e++) v[e] = j0 + e * blockDim.x < nt * QW_HC_LR ? a.sx[t0 * QW_HC_LR + j0 + e * blockDim.x] : 0.0f;
+            for (uint32_t e = 0; e < 8; e++) v[e] = j0 + e * qw_threads() < nt * QW_HC_LR ? a.sx[t0 * QW_HC_LR + j0 + e * qw_threads()] : 0.0f;
 #pragma unroll
             for (uint32_t e = 0; e < 8; e++)
-                if (j0 + e * blockDim.x < nt * QW_HC_LR) (&sx[0][0])[j0 + e * blockDim.x] = v[e];
+                if (j0 + e * qw_threads() < nt * QW_HC_LR) (&sx[0][0])[j0 + e * qw_threads()] = v[e];
         }
         if (tid < nt * QW_HC) rs[tid / QW_HC][tid % QW_HC] = a.rs[t0 * QW_HC + tid];
     } else { // hc_mid for the workgroup's tokens, on the values read above
@@ -3252,7 +3252,7 @@ extern "C" __global__ __launch_bounds__(256) void qwk_hc_upv(qwk_hc_args a) { hc
 // Read pattern of a decode layer without the decoding (kernels/moe_bw.metal:7-26): workgroup (x, c) reads slice x
 // (SL 16-byte units) of chunk c, every thread LD independent loads a round, folded into an XOR sink.
 template <int LD> __device__ __forceinline__ void bw_chunks_body(const qwk_bwpat_args &a) {
-    const uint32_t nt = blockDim.x, tid = threadIdx.x;
+    const uint32_t nt = qw_threads(), tid = threadIdx.x;
     const uint64_t start = a.chunks[2 * blockIdx.y];
     uint64_t len = a.chunks[2 * blockIdx.y + 1];
     if (start >= a.src_n) return;
@@ -3305,8 +3305,8 @@ extern "C" __global__ __launch_bounds__(256) void qwk_bw_rows(qwk_bwpat_args a) 
 extern "C" __global__ __launch_bounds__(256) void qwk_copy(qwk_mem_args a) {
     const u4 *p = (const u4 *)a.src;
     u4 *q = (u4 *)a.dst;
-    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += step) q[i] = p[i];
+    const uint64_t step = (uint64_t)gridDim.x * qw_threads();
+    for (uint64_t i = (uint64_t)blockIdx.x * qw_threads() + threadIdx.x; i < a.n; i += step) q[i] = p[i];
 }
 #endif
 #if QW_IN_PART(5)
@@ -3355,8 +3355,8 @@ __device__ __forceinline__ uint32_t qw_mix(uint64_t x) {
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(256) void qwk_fill_random(qwk_mem_args a) {
     u4 *q = (u4 *)a.dst;
-    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += step) {
+    const uint64_t step = (uint64_t)gridDim.x * qw_threads();
+    for (uint64_t i = (uint64_t)blockIdx.x * qw_threads() + threadIdx.x; i < a.n; i += step) {
         const uint64_t c = a.seed + 4 * i;
         q[i] = u4{qw_mix(c), qw_mix(c + 1), qw_mix(c + 2), qw_mix(c + 3)};
     }
@@ -3367,9 +3367,9 @@ extern "C" __global__ __launch_bounds__(256) void qwk_fill_random(qwk_mem_args a
 // every other byte uniform (IQ3_S, IQ4_NL), or int8 uniform in [-127, 127] (Q8_0). Blocks are 2-byte aligned: 16-bit stores.
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(256) void qwk_fill_blocks(qwk_fill_args a) {
-    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
+    const uint64_t step = (uint64_t)gridDim.x * qw_threads();
     const uint32_t bb = a.type == 21 ? 110 : a.type == 20 ? 18 : 34; // IQ4_NL: d and sixteen uniform bytes
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.nblocks; i += step) {
+    for (uint64_t i = (uint64_t)blockIdx.x * qw_threads() + threadIdx.x; i < a.nblocks; i += step) {
         uint16_t *p = (uint16_t *)(a.dst + i * bb);
         const uint64_t c = a.seed + i * 64;
         const float u1 = ((float)(qw_mix(c) >> 8) + 1.0f) * (1.0f / 16777216.0f), u2 = (float)(qw_mix(c + 1) >> 8) * (1.0f / 16777216.0f);

@@ -44,7 +44,7 @@ __device__ __forceinline__ void qw_kq_tab_build(uint32_t *tab, uint32_t first, u
         tab[i] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | (uint32_t)__builtin_bit_cast(uint16_t, hi) << 16;
     }
 }
-__device__ __forceinline__ void qw_kq_tab_build(uint32_t *tab) { qw_kq_tab_build(tab, threadIdx.x, blockDim.x); } // by the workgroup
+__device__ __forceinline__ void qw_kq_tab_build(uint32_t *tab) { qw_kq_tab_build(tab, threadIdx.x, qw_threads()); } // by the workgroup
 
 // Four bytes (each < 256) to four binary16 integers minus bias: bytes b0 b1 -> first pair, b2 b3 -> second pair.
 __device__ __forceinline__ u2 qw_bytes_h4(uint32_t v, float bias) {
