@@ -1489,7 +1489,7 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
 static bool fill_gu(qw_batch *b, qwk_gu_args *a, int F, unsigned iWg, unsigned iWu, unsigned ix, unsigned iH, uint32_t nbr, bool shared) {
     const qw_kparams *p = &b->k->p;
     const size_t rb = fmt_rb(F, p->D), ne = shared ? 1 : (size_t)p->E;
-    *a = (qwk_gu_args){.D = (uint32_t)p->D, .I = (uint32_t)p->I, .rowbytes = (uint32_t)rb, .nbr = nbr, .topk = (uint32_t)p->topk, .gnb = (uint32_t)p->gnb, .shared = shared,
+    *a = (qwk_gu_args){.tpe_mul = QW_DIV_MUL((uint32_t)p->I / 8), .D = (uint32_t)p->D, .I = (uint32_t)p->I, .rowbytes = (uint32_t)rb, .nbr = nbr, .topk = (uint32_t)p->topk, .gnb = (uint32_t)p->gnb, .shared = shared,
                        .hplane = (uint32_t)p->NB * (uint32_t)(p->topk + 1) * (uint32_t)p->I, .glut = glut(b->g)};
     b->allow_released = !shared; // the routed matrices may be buffers of which only the tile-major copy is left (the caller checks that one serves)
     const bool bound = bind_ptr(b, iWg, ne * p->I * rb, false, "gate weights", (void **)&a->Wg) && bind_ptr(b, iWu, ne * p->I * rb, false, "up weights", (void **)&a->Wu);
@@ -1780,7 +1780,7 @@ static bool tr_dn_inner(qw_batch *b) {
     const qw_kparams *p = &b->k->p;
     const uint32_t nbr = (uint32_t)p->NB;
     const size_t rb = fmt_rb(p->fd, p->I);
-    qwk_dn_args a = {.D = (uint32_t)p->D, .I = (uint32_t)p->I, .rowbytes = (uint32_t)rb, .nbr = nbr, .topk = (uint32_t)p->topk, .gnb = (uint32_t)p->gnb, .shared = 0,
+    qwk_dn_args a = {.tpe_mul = QW_DIV_MUL((uint32_t)p->D / 16), .upr_mul = QW_DIV_MUL((uint32_t)p->I / 8), .D = (uint32_t)p->D, .I = (uint32_t)p->I, .rowbytes = (uint32_t)rb, .nbr = nbr, .topk = (uint32_t)p->topk, .gnb = (uint32_t)p->gnb, .shared = 0,
                      .hplane = (uint32_t)p->NB * (uint32_t)(p->topk + 1) * (uint32_t)p->I, .glut = glut(b->g)};
     b->allow_released = true; // Wd may be a buffer of which only the tile-major copy is left
     const bool bound = bind_ptr(b, 0, (size_t)p->E * p->D * rb, false, "down weights", (void **)&a.Wd);

@@ -39,6 +39,10 @@ typedef u2 __attribute__((aligned(2))) u2a2;
 // they asked for anything else. No launch here has such a workgroup; this is a scalar load beside the arguments'.)
 __device__ __forceinline__ uint32_t qw_threads() { return __builtin_amdgcn_workgroup_size_x(); }
 
+// x / d with mul = 2^32 / d + 1 from the host (QW_DIV_MUL), exact for x * d < 2^32, d >= 2: one instruction, where a division by an argument
+// is a chain of some thirty - and the address of a launch's first load often waits for several of them.
+__device__ __forceinline__ uint32_t qw_div(uint32_t x, uint32_t mul) { return __umulhi(x, mul); }
+
 __device__ __forceinline__ float qw_h2f(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
 __device__ __forceinline__ uint16_t qw_f2h(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
 __device__ __forceinline__ float qw_bf2f(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
@@ -296,7 +300,7 @@ __device__ __forceinline__ void qw_load_to_lds(const u4 *src_lane, u4 *dst_wave)
 __device__ __forceinline__ void qw_lds_arrive();
 // part, nparts: the calling wave is number `part` of the `nparts` waves that do the copy (default: all of the workgroup).
 __device__ __forceinline__ void qw_stage_x_issue(u4 *xf, const uint16_t *x, uint32_t xstride, uint32_t K, uint32_t nb, uint32_t part = ~0u, uint32_t nparts = 0) {
-    const uint32_t n = (K >> 3) * 16, rot = (blockIdx.x * 320u) % n, lane = threadIdx.x & 63; // n and rot are multiples of 64
+    const uint32_t n = (K >> 3) * 16, rot = ((blockIdx.x & 63) * (n >> 6)) & ~63u, lane = threadIdx.x & 63; // n and rot are multiples of 64
     if (part == ~0u) part = threadIdx.x >> 6, nparts = qw_threads() >> 6;
     for (uint32_t i0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)part) * 64; i0 < n; i0 += 64 * nparts) {
         const uint32_t base = i0 + rot < n ? i0 + rot : i0 + rot - n, i = base + lane, c = i >> 4, m = i & 15;

@@ -123,8 +123,11 @@ typedef struct {
      * itself and workgroup 0 also writes the record to sel (the later kernels of the layer read it from there) */
     const float *logits;
     /* qwk_gu_rt*: the routed rows' ggml type (12, 13, 14, 20 or 23), chosen when the kernel runs */
-    uint32_t fgu, pad_fgu;
+    uint32_t fgu;
+    uint32_t tpe_mul; /* QW_DIV_MUL(I / 8) */
 } qwk_gu_args;
+/* For qw_div: x / d = x * QW_DIV_MUL(d) >> 32, d >= 2, x * d < 2^32 */
+#define QW_DIV_MUL(d) ((uint32_t)((((uint64_t)1) << 32) / (d) + 1))
 
 /* down projection. routed: Pg[t][slot][row] for the tokens in mask[u]; shared != 0: Psh[t][row] from slot topk. */
 typedef struct {
@@ -146,6 +149,7 @@ typedef struct {
     /* qwk_dn_rt: the ggml types of the routed and of the shared down rows (0: no shared expert in this launch),
      * chosen when the kernel runs */
     uint32_t fd, fsd;
+    uint32_t tpe_mul, upr_mul; /* QW_DIV_MUL of D / 16 and of I / 8 */
     /* qwk_dnc_*, qwk_dnq_* as the last launch of a batch over host-visible buffers (fin.flag NULL: not): second places for
      * P, Psh (NULL where the launch does not make it) and out, and what the launches before left */
     float *Ph, *Pshh;

@@ -917,7 +917,7 @@ __device__ __forceinline__ void select_all(const qwk_select_args &a, qw_sel_scra
         clear();
     } else if (fast) { // a wave takes one token, or two when there are more tokens than such waves (lgs gives a wave 288 dwords)
         uint32_t *ws = (uint32_t *)lgs + 288 * wave;
-        const uint32_t trot = a.nbr ? blockIdx.x % a.nbr : 0; // the workgroups of a launch read the tokens' logits in different orders
+        const uint32_t trot = ((blockIdx.x & 15) * a.nbr) >> 4; // the workgroups of a launch read the tokens' logits in different orders
         auto rot = [&](uint32_t tt) { return tt + trot < a.nbr ? tt + trot : tt + trot - a.nbr; };
         const bool pairs = E <= 512; // sixteen keys a lane: one token at a time (registers)
         auto slow = [&](uint32_t tok) { // the repeated maximum
@@ -1089,15 +1089,15 @@ __device__ __forceinline__ void gu_tasks(const qwk_gu_args &a, const u2 *lut, co
     };
     const uint32_t nl = lane >> 2; // (row, k-group) this lane loads from GGUF rows: (lane >> 2, lane & 3)
     auto rowp = [&](uint32_t task) {
-        const uint32_t u = task / tpe, e = a.shared ? 0 : (uint32_t)__builtin_amdgcn_readfirstlane((int)sc->ue[u]); // (wave-uniform: the row base stays in scalar registers)
-        if constexpr (qw_tiled(F)) return a.Wg + ((size_t)e * tpe + task % tpe) * a.rowbytes; // the tile's slabs; rowbytes = bytes of a tile
-        else return (nl < 8 ? a.Wg : a.Wu) + ((size_t)e * a.I + 8 * (task % tpe) + (nl & 7)) * a.rowbytes;
+        const uint32_t u = qw_div(task, a.tpe_mul), t = task - u * tpe, e = a.shared ? 0 : (uint32_t)__builtin_amdgcn_readfirstlane((int)sc->ue[u]); // (wave-uniform: the row base stays in scalar registers)
+        if constexpr (qw_tiled(F)) return a.Wg + ((size_t)e * tpe + t) * a.rowbytes; // the tile's slabs; rowbytes = bytes of a tile
+        else return (nl < 8 ? a.Wg : a.Wu) + ((size_t)e * a.I + 8 * t + (nl & 7)) * a.rowbytes;
     };
     f4 acc = {0, 0, 0, 0};
     auto use = [&](uint32_t task, uint32_t ci, const C &c) {
         c.mac_lean(lut, af, ci * CH * C::BLK_K, kg, acc);
         if (ci + 1 != cpr) return;
-        const uint32_t u = task / tpe, j0 = 8 * (task % tpe);
+        const uint32_t u = qw_div(task, a.tpe_mul), j0 = 8 * (task - u * tpe);
         const uint32_t m = (a.shared ? 0xffffffffu : sc->mask[u]) & qw_all_tokens(a.nbr);
         hs.tile(m);
 #pragma unroll
@@ -1704,9 +1704,7 @@ template <int F, int CH, class S> __device__ __forceinline__ void dn_range_run(c
 }
 template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_range_body(const qwk_dn_args &a, u2 *lut, uint16_t *arows /* [2][16][2][I] */, qw_sel_cache *sc) {
     const uint32_t K = a.topk, gnb = a.gnb, GU = gnb * K, tpe = a.D / 16;
-    const bool tp2 = (tpe & (tpe - 1)) == 0; // D = 1024, 2048: shifts instead of divisions
-    const uint32_t tsh = (uint32_t)__builtin_ctz(tpe);
-    auto div_tpe = [&](uint32_t x) { return tp2 ? x >> tsh : x / tpe; };
+    auto div_tpe = [&](uint32_t x) { return qw_div(x, a.tpe_mul); };
     qw_sel_load(*sc, a.sel, K, gnb); // one memory round trip for everything the ranges depend on
     if (qw_has_lut(F) || qw_has_lut(FSD)) qw_lut_copy_issue(lut, (const u2 *)a.glut); // lands in LDS meanwhile; awaited in ready()
     if (qw_has_tab(F) || qw_has_tab(FSD)) qw_kq_tab_build((uint32_t *)lut); // the byte table of the 4-bit codebook instead
@@ -1717,7 +1715,7 @@ template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_r
     if (U > GU) U = GU;
     // a shared-expert tile of a wider format counts as several tasks, so that ranges hold about the same bytes
     const uint32_t tb = qw_tiled(F) ? a.rowbytes : 16 * a.rowbytes, stb = qw_tiled(FSD) ? a.sd_rowbytes : 16 * a.sd_rowbytes; // bytes of a tile
-    const uint32_t nsh = (FSD != 0 && a.Wsd) ? 1 : 0, shw = nsh ? (stb + tb - 1) / tb : 1, vsh = nsh * shw * tpe;
+    const uint32_t nsh = (FSD != 0 && a.Wsd) ? 1 : 0, shw = FSD != F && nsh ? (stb + tb - 1) / tb : 1, vsh = nsh * shw * tpe;
     const uint32_t V = vsh + U * tpe;
     uint32_t per = (V + gridDim.x - 1) / gridDim.x;
     if (per > tpe) per = tpe;
@@ -1762,7 +1760,7 @@ template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_r
                 // few rows (a token or two per expert): one 16-byte unit per thread through a register, the waves
                 // of a row finding its bit in the mask by a (mostly scalar) walk
                 // (a row of both planes is 2 upr threads: whole waves when I is a multiple of 256, else a wave may span two rows)
-                const uint32_t i = threadIdx.x, kl = i / (2 * upr), k = (2 * upr) % 64 == 0 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)kl) : kl, r = i % (2 * upr), pl = r / upr, c = r % upr;
+                const uint32_t i = threadIdx.x, row = qw_div(i, a.upr_mul), kl = row >> 1, k = (2 * upr) % 64 == 0 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)kl) : kl, pl = row & 1, c = i - row * upr;
                 if (k < nrows) {
                     uint32_t m = rows;
                     for (uint32_t j = 0; j < k; j++) m &= m - 1;
@@ -1773,7 +1771,7 @@ template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_r
             } else {
                 const uint32_t s0 = g0.sh ? K : slot[g0.u * gnb + t], s1 = !both ? 0 : g1.sh ? K : slot[g1.u * gnb + t]; // result slot of token t
                 for (uint32_t q = qw_wave(); q < ninst; q += qw_threads() >> 6) {
-                    const uint32_t sg = q / (2 * ncb), r = q % (2 * ncb), pl = r / ncb, cb = r % ncb;
+                    const uint32_t part = qw_div(4 * q, a.upr_mul) /* q / ncb */, sg = part >> 1, pl = part & 1, cb = q - part * ncb;
                     const uint32_t m = sg ? g1.mask : g0.mask, sl = sg ? s1 : s0, c = 4 * cb + (lane >> 4);
                     if ((m >> t) & 1)
                         qw_load_to_lds((const u4 *)(a.H + pl * (size_t)a.hplane + ((size_t)t * (K + 1) + sl) * a.I + 8 * c), (u4 *)arows + ((sg * 2 + pl) * upr + 4 * cb) * 16);
@@ -2097,8 +2095,8 @@ __device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_l
     if (GU > QW_DNQ_MAXU) GU = QW_DNQ_MAXU; // (the host admits topk <= 10: 160 at most)
     // workgroup -> (tile group g, quarter q): the quarters of a group are eight workgroups apart, which puts them on one XCD.
     // The nq quarters (2 or 4) share the tokens evenly: sizes differ by one at most, four at most each.
-    const uint32_t hi8 = blockIdx.x >> 3, g = (hi8 / nq) * 8 + (blockIdx.x & 7), q = hi8 % nq;
-    const uint32_t base = a.nbr / nq, rem = a.nbr % nq, t0 = q * base + (q < rem ? q : rem);
+    const uint32_t nqs = (uint32_t)__builtin_ctz(nq), hi8 = blockIdx.x >> 3, g = (hi8 >> nqs) * 8 + (blockIdx.x & 7), q = hi8 & (nq - 1); // (nq is 1, 2 or 4)
+    const uint32_t base = a.nbr >> nqs, rem = a.nbr & (nq - 1), t0 = q * base + (q < rem ? q : rem);
     uint32_t nt = base + (q < rem ? 1 : 0);
     if (nt > 4) nt = 4; // (the host admits 16 tokens in four quarters, 8 in two)
     QW_DSTAMP(6);
@@ -2128,7 +2126,8 @@ __device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_l
         const uint32_t upr = a.I / 8, cbs = upr / 8, used = nt * (K + 1), nrb = (used + 7) / 8, nunits = 2 * nrb * cbs, wv = qw_wave();
 #pragma unroll
         for (uint32_t it = 0; it < RPER; it++) {
-            const uint32_t unit = wv + it * NW, cb = unit % cbs, rest = unit / cbs, rb = rest % nrb, pl = rest / nrb;
+            // (I is 256 or 512, so cbs 4 or 8; a unit in use has rest < 2 nrb. By divisions this was a microsecond in front of the loads.)
+            const uint32_t unit = wv + it * NW, cb = unit & (cbs - 1), rest = unit >> __builtin_ctz(cbs), pl = rest >= nrb, rb = rest - (pl ? nrb : 0);
             const uint32_t r = 8 * rb + ((lane >> 2) & 7), c = 8 * cb + 4 * (lane >> 5) + (lane & 3);
             const bool on = unit < nunits && r < used;
             at[it] = on ? (pl * upr + c) * QW_DNQ_ROWS + r : ~0u;
@@ -2353,7 +2352,8 @@ template <int FSD, int CHSD> __device__ __forceinline__ void gud_body(const qwk_
         uint32_t at[PER];
 #pragma unroll
         for (uint32_t it = 0; it < PER; it++) {
-            const uint32_t unit = wv + it * NW, cb = unit % cbs, rest = unit / cbs, rb = rest % nrb, pl = rest / nrb;
+            // (I is 256 or 512, so cbs 4 or 8; a unit in use has rest < 2 nrb. By divisions this was a microsecond in front of the loads.)
+            const uint32_t unit = wv + it * NW, cb = unit & (cbs - 1), rest = unit >> __builtin_ctz(cbs), pl = rest >= nrb, rb = rest - (pl ? nrb : 0);
             const uint32_t r = 8 * rb + ((lane >> 2) & 7), c = 8 * cb + 4 * (lane >> 5) + (lane & 3);
             const bool on = unit < nunits && r < used;
             at[it] = on ? (pl * upr + c) * QW_GUD_ROWS + r : ~0u;
