@@ -121,7 +121,9 @@ typedef struct { qw_hbuf *b; bool out, whole, direct; size_t lo, hi; } qw_use;
 // the device clock at the start and the end of every submitted segment (0: not taken); done, copied: 1 once its kernels
 // have finished (where it was submitted without waiting) and once its outputs are in the shadows. Cleared when a batch takes
 // the slot, which the batch before gave back after its last launch had ended.
-typedef struct { volatile uint64_t t0[9], t1[9]; volatile uint32_t done, copied; uint32_t pad[26]; } qw_ioslot;
+// part[k]: the clock at the start of part k of a batch that is recorded in parts (0: not taken).
+enum { QW_PARTS_MAX = 64 };
+typedef struct { volatile uint64_t t0[9], t1[9]; volatile uint32_t done, copied; uint32_t pad[26]; volatile uint64_t part[QW_PARTS_MAX]; } qw_ioslot;
 enum { QW_IO_SLOTS = 32 };
 _Static_assert(QW_IO_SLOTS % QW_FIN_LINE == 0, "the counters behind the words begin a line");
 
@@ -152,6 +154,8 @@ struct qw_batch {
     hipEvent_t ev[2 * 9]; // profiled batches, and those for which no slot was free: start/stop per submitted segment (end + at most 8 flushes)
     bool events;
     bool fin;            // the last launch raises the flag itself
+    int nparts, part_l[QW_PARTS_MAX]; // qw_hip_batch_part: the first launch of every part
+    double *part_s;      // where the seconds of the parts go (qw_hip_batch_end_parts)
     hipEvent_t *pev;      // profiling: 2 events per launch
     int npev;
     // Work deferred from one dispatch of a layer to the next (the reference's front part also computes the shared
@@ -2545,6 +2549,21 @@ static bool direct_ok(const qw_batch *b, const qw_use *u, bool last) {
     }
     return u->whole || (u->b->size <= QW_HIP_SMALL_BYTES && u->b->pending_out == 1);
 }
+// The dispatches of b that write h write disjoint ranges of it whole, and every one can write the shadow too: then all do.
+static bool split_ok(const qw_batch *b, const qw_hbuf *h) {
+    int uses = 0, slots = 0;
+    for (int j = 0; j < b->nuse; j++) {
+        const qw_use *u = &b->use[j];
+        if (!u->out || u->b != h) continue;
+        if (!u->whole || !carried_back(u) || !h->pinned) return false;
+        for (int k = 0; k < j; k++)
+            if (b->use[k].out && b->use[k].b == h && b->use[k].lo < u->hi && b->use[k].hi > u->lo) return false;
+        uses++;
+    }
+    for (int i = b->done_l; i < b->nl; i++)
+        for (int d = 0; d < b->l[i].ndirect; d++) slots += b->use[b->l[i].direct_use[d]].b == h && !b->l[i].side;
+    return uses > 1 && uses == slots;
+}
 static void direct_set(qw_batch *b, qw_launch *l, int d) {
     qw_use *u = &b->use[l->direct_use[d]];
     const char *host = (const char *)u->b->host + u->lo;
@@ -2561,15 +2580,17 @@ static void host_outputs(qw_batch *b) {
     for (int i = b->done_l; i < b->nl; i++) {
         qw_launch *l = &b->l[i];
         side = side || l->side;
-        for (int d = 0; d < l->ndirect && !l->back_at; d++)
-            if (direct_ok(b, &b->use[l->direct_use[d]], false)) direct_set(b, l, d);
+        for (int d = 0; d < l->ndirect; d++) {
+            const qw_use *u = &b->use[l->direct_use[d]];
+            if ((!l->back_at && direct_ok(b, u, false)) || (u->out && split_ok(b, u->b))) direct_set(b, l, d);
+        }
     }
     qw_launch *l = b->nl > b->done_l ? &b->l[b->nl - 1] : NULL;
     if (!l || !l->ndirect || side) return;
     const unsigned mark = ++b->g->mark; // buffers that are seen to
     for (int d = 0; d < l->ndirect; d++) {
         const qw_use *u = &b->use[l->direct_use[d]];
-        if (carried_back(u) && !direct_ok(b, u, true)) return;
+        if (carried_back(u) && !u->direct && !direct_ok(b, u, true)) return;
         u->b->mark = mark;
     }
     qwk_back back = {0};
@@ -2673,6 +2694,11 @@ static bool submit_segment(qw_batch *b, bool last) {
         (void)*back;
     }
     if (!b->nseg) g->in_flight++;
+    for (int k = 1; k < b->nparts && b->io && !b->nseg; k++) { // (part 0 starts with the batch)
+        qw_launch *l = b->part_l[k] < b->nl ? &b->l[b->part_l[k]] : NULL;
+        const volatile uint64_t *t = &b->io->part[k];
+        if (l && !l->side && start_of(l->fname)) memcpy(l->args + start_of(l->fname), &t, sizeof t);
+    }
     const int seg = b->nseg++;
     hipEvent_t *ev = &b->ev[2 * seg];
     if (b->events) {
@@ -2817,6 +2843,12 @@ static double batch_wait(qw_batch *b, bool ended) { // ended: submitted by qw_ba
             secs += (double)ms * 1e-3;
         }
     }
+    if (b->part_s) { // from one part's start to the next one's; 0 where a stamp is missing
+        for (int k = 0; k < b->nparts; k++) {
+            const uint64_t t0 = !ok || !b->io ? 0 : k ? b->io->part[k] : b->io->t0[0], t1 = !ok || !b->io ? 0 : k + 1 < b->nparts ? b->io->part[k + 1] : b->io->t1[0];
+            b->part_s[k] = t0 && t1 > t0 ? (double)(t1 - t0) * g->tick : 0;
+        }
+    }
     if (ok && b->prof) {
         g->nprof = 0;
         for (int i = 0; i < b->nl && g->nprof < QW_PROF_MAX && 2 * i + 1 < b->npev; i++) {
@@ -2840,6 +2872,16 @@ double qw_batch_wait(qw_batch *b) {
     return qw_batch_end(b);
 }
 
+// A batch recorded in parts (csrc/qw_internal.h)
+bool qw_hip_parts_ok(const qw_gpu *g) { return !g->prof && g->io_used != ~0u; }
+void qw_hip_batch_part(qw_batch *b) {
+    if (b->nparts < QW_PARTS_MAX) b->part_l[b->nparts++] = b->nl;
+}
+double qw_hip_batch_end_parts(qw_batch *b, double *secs) {
+    for (int k = 0; k < b->nparts; k++) secs[k] = 0;
+    b->part_s = secs;
+    return qw_batch_end(b);
+}
 double qw_batch_end(qw_batch *b) {
     if (b->submitted) return batch_wait(b, false);
     b->submitted = true;

@@ -272,6 +272,8 @@ __device__ __forceinline__ void qw_store_y(void *y, float *yh, bool f32, const q
     else ((float *)y)[i] = v;
     if (yh) __hip_atomic_store(yh + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+// A value for the host alone: past the caches, so that the end of the launch is all that has to come before the host looks.
+__device__ __forceinline__ void qw_store_host(uint16_t *p, uint16_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 // The start of the first launch of a batch, at the entry of its kernel. qwk_io used to be that launch, for its stamp alone where
 // nothing goes up (2.4 us and a gap). Not in the hyper-connection's kernels: the look at the pointer, in the last line of their
 // arguments, comes before their first loads and takes them 0.6 us in every launch (5.9 -> 6.4).
@@ -1933,7 +1935,7 @@ __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *p
         for (uint32_t s = 0; s < K; s++) o = __builtin_fmaf(w[s], p[s * 16], o);
         o = __builtin_fmaf(w[K], nsh ? p[K * 16] : a.Psh[(size_t)t * a.D + r], o);
         a.out[(size_t)t * a.D + r] = qw_f2h(o);
-        if (a.outh) a.outh[(size_t)t * a.D + r] = qw_f2h(o);
+        if (a.outh) qw_store_host(a.outh + (size_t)t * a.D + r, qw_f2h(o));
     }
     qw_back_fin(a.back, a.fin);
 }
@@ -2205,7 +2207,7 @@ __device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_l
         else sh = a.Psh[(size_t)(t0 + t) * a.D + r]; // the caller's own shared product
         o = __builtin_fmaf(w[K], sh, o);
         a.out[(size_t)(t0 + t) * a.D + r] = qw_f2h(o);
-        if (a.outh) a.outh[(size_t)(t0 + t) * a.D + r] = qw_f2h(o);
+        if (a.outh) qw_store_host(a.outh + (size_t)(t0 + t) * a.D + r, qw_f2h(o));
     }
     QW_DSTAMP(14);
     qw_back_fin(a.back, a.fin);

@@ -31,6 +31,12 @@ QW_INTERNAL qw_batch *qw_hip_batch_begin_static(qw_gpu *g, void *stream);
  * refused, nothing is launched. false + qw_hip_last_error in those cases and when a launch failed. */
 QW_INTERNAL bool qw_hip_batch_launch_static(qw_batch *b, bool recorded);
 
+/* A batch in parts: qw_hip_batch_part before the dispatches of each part (up to 64), qw_hip_batch_end_parts instead of qw_batch_end;
+ * secs[k]: device time of part k (0: its first launch takes no stamp). Only while qw_hip_parts_ok: profiled batches have no stamps. */
+QW_INTERNAL bool qw_hip_parts_ok(const qw_gpu *g);
+QW_INTERNAL void qw_hip_batch_part(qw_batch *b);
+QW_INTERNAL double qw_hip_batch_end_parts(qw_batch *b, double *secs);
+
 #ifdef __cplusplus
 }
 #endif

@@ -412,9 +412,9 @@ bool qw_path_hyper_moe_stack(qw_path *p, qw_batch *b, const qw_hyper_w *H, const
 
 // ---------------------------------------------------------------- a ragged step (src/engine.c:8783-8814, :9138-9161, :9037)
 // Slot i brings n[i] rows; its first row is r0[i] = n[0] + ... + n[i - 1] (src/engine.c:9150-9161). The R rows are cut
-// into groups by the measured table (qw_par_split: the reference's par_split with groups of up to 16 rows), every
-// group is one batch through the layer (the reference's par_step runs its groups one after the other, each reading
-// the weights once, src/engine.c:8805-8812), and each group's wall time goes back into the table (src/engine.c:9037).
+// into groups by the measured table (qw_par_split: the reference's par_split with groups of up to 16 rows), the
+// groups go through the layer one after the other (the reference's par_step, src/engine.c:8805-8812, each reading
+// the weights once), and each group's time goes back into the table (src/engine.c:9037).
 bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int *n, int B, const qw_buf *x, const qw_buf *out, qw_vstep_info *info) {
     if (!p || !par || !M || !n || !x || !out || B < 1 || B > QW_PAR_MAX) return false;
     int R = 0, r0[QW_PAR_MAX];
@@ -438,6 +438,29 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
         memcpy(info->groups, grp, sizeof(int) * (size_t)ng);
     }
     double gpu = 0, wall = 0;
+    if (qw_hip_parts_ok(p->g)) {
+        // All groups in one batch: one upload, one wait, the rows written to the host by each group's last launch. A group's time is
+        // the device's from its first launch to the next group's, and its share of what the host adds once. (A batch a group, each waited for:
+        // 251 us for sixteen slots and 45 rows of the benchmark's layer, this 205.)
+        double part[QW_PAR_MAX], sum = 0;
+        const double t0 = qw_now();
+        qw_batch *b = qw_batch_begin(p->g, false);
+        if (!b) return false;
+        bool rec = true;
+        for (int gi = 0, c = 0; gi < ng && rec; c += grp[gi++]) {
+            qw_hip_batch_part(b);
+            rec = gg_moe_at(p, b, M, grp[gi], x, (size_t)c * (size_t)p->D * 2, &p->vlg, &p->vsel, out, (size_t)c * (size_t)p->D * 2, false);
+        }
+        const double t = qw_hip_batch_end_parts(b, part);
+        if (!rec || t < 0) return false;
+        gpu = t * 1e3, wall = (qw_now() - t0) * 1e3;
+        bool stamped = true;
+        for (int gi = 0; gi < ng; gi++) stamped = stamped && part[gi] > 0;
+        for (int gi = 0; gi < ng; gi++) sum += part[gi] = stamped ? part[gi] * 1e3 : gpu * grp[gi] / R; // (a front launch without a stamp: by rows)
+        for (int gi = 0; gi < ng; gi++) qw_par_observe(par, grp[gi], part[gi] + (wall > sum ? wall - sum : 0) / ng);
+        if (info) info->gpu_ms = gpu, info->wall_ms = wall;
+        return true;
+    }
     for (int gi = 0, c = 0; gi < ng; c += grp[gi++]) {
         const double t0 = qw_now();
         qw_batch *b = qw_batch_begin(p->g, false);
