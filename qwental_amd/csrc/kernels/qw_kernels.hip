@@ -411,31 +411,31 @@ template <int XN> __device__ __forceinline__ void qmvs_body(const qwk_qmvm_args 
     const uint32_t lane = qw_lane(), wave = qw_wave(), nw = qw_threads() >> 6, own = a.sh ? 32u << a.sh : 64;
     u2 *tab = (u2 *)dyn;
     u4 *x = dyn + a.tabu + wave * own;
-    uint32_t j = 0, t = blockIdx.x;
-    while (j + 1 < a.nmat && t >= a.ntiles[j]) t -= a.ntiles[j++];
+    uint32_t t = blockIdx.x;
+    const qmvs_mat M = qmvs_pick(a, t);
     f4 acc = {0, 0, 0, 0};
-    switch (a.fmt[j]) {
-    case 8: acc = qmvs_part<8, XN>(a, j, t, tab, x); break;
-    case 12: acc = qmvs_part<12, XN>(a, j, t, tab, x); break;
-    case 13: acc = qmvs_part<13, XN>(a, j, t, tab, x); break;
-    case 14: acc = qmvs_part<14, XN>(a, j, t, tab, x); break;
-    case 20: acc = qmvs_part<20, XN>(a, j, t, tab, x); break;
-    case 21: acc = qmvs_part<21, XN>(a, j, t, tab, x); break;
-    case 23: acc = qmvs_part<23, XN>(a, j, t, tab, x); break;
-    case QW_F_PACKED: acc = qmvs_part<QW_F_PACKED, XN>(a, j, t, tab, x); break;
-    case 1: acc = qmvs_part<1, XN>(a, j, t, tab, x); break;
-    case 30: acc = qmvs_part<30, XN>(a, j, t, tab, x); break;
+    switch (M.fmt) {
+    case 8: acc = qmvs_part<8, XN>(a, M, t, tab, x); break;
+    case 12: acc = qmvs_part<12, XN>(a, M, t, tab, x); break;
+    case 13: acc = qmvs_part<13, XN>(a, M, t, tab, x); break;
+    case 14: acc = qmvs_part<14, XN>(a, M, t, tab, x); break;
+    case 20: acc = qmvs_part<20, XN>(a, M, t, tab, x); break;
+    case 21: acc = qmvs_part<21, XN>(a, M, t, tab, x); break;
+    case 23: acc = qmvs_part<23, XN>(a, M, t, tab, x); break;
+    case QW_F_PACKED: acc = qmvs_part<QW_F_PACKED, XN>(a, M, t, tab, x); break;
+    case 1: acc = qmvs_part<1, XN>(a, M, t, tab, x); break;
+    case 30: acc = qmvs_part<30, XN>(a, M, t, tab, x); break;
     }
     if (wave) ((f4 *)x)[lane] = acc;
     __syncthreads();
     if (wave) return;
     for (uint32_t q = 1; q < nw; q++) acc += ((const f4 *)x)[q * own + lane];
     const uint32_t r = 16 * t + (lane & 15), kg = lane >> 4;
-    if (r < a.N[j])
+    if (r < M.N)
 #pragma unroll
         for (uint32_t i = 0; i < 4; i++) {
             const uint32_t tok = 4 * kg + i;
-            if (tok < a.nb) qw_store_y(a.y[j], a.yh[j], a.yfloat, a.fin, (size_t)tok * a.ystride[j] + r, acc[i]);
+            if (tok < a.nb) qw_store_y(M.y, M.yh, a.yfloat, a.fin, (size_t)tok * M.ystride + r, acc[i]);
         }
     qw_fin_wave(a.fin);
 }

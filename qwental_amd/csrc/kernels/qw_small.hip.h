@@ -129,8 +129,26 @@ template <> struct qw_small_blk<QW_F_PACKED> {
     static __device__ __forceinline__ f4 mac(const C &c, const u2 *tab, const qw_afrag_small &af, uint32_t kg) { return qw_small_blk<21>::mac(c, tab, af, kg); }
 };
 
-// The wave's part of tile t of matrix j: block `wave` of the rows. x: the wave's own LDS. XN: loads of two tokens, 2 XN >= nb.
-template <int F, int XN> __device__ __forceinline__ f4 qmvs_part(const qwk_qmvm_args &a, uint32_t j, uint32_t t, u2 *tab, u4 *x) {
+// The workgroup's matrix, chosen by value from arguments that all come in one read. (Chosen by index they were read one after the
+// other, the tile counts up to the workgroup's own, then the format, then the rest: three and more scalar round trips in front of the weights.)
+struct qmvs_mat {
+    const uint8_t *W;
+    void *y;
+    float *yh;
+    uint32_t N, fmt, rowbytes, ystride;
+};
+template <class T> __device__ __forceinline__ T qw_pick4(uint32_t j, T a, T b, T c, T d) { return j == 0 ? a : j == 1 ? b : j == 2 ? c : d; }
+__device__ __forceinline__ qmvs_mat qmvs_pick(const qwk_qmvm_args &a, uint32_t &t) { // t: tile among all of them -> of the matrix
+    const uint32_t e0 = a.ntiles[0], e1 = e0 + a.ntiles[1], e2 = e1 + a.ntiles[2], n = a.nmat - 1;
+    uint32_t j = (t >= e0) + (t >= e1) + (t >= e2);
+    j = j < n ? j : n; // (what lies behind the last matrix in the record is not looked at)
+    t -= qw_pick4(j, 0u, e0, e1, e2);
+#define QW_P(v) qw_pick4(j, a.v[0], a.v[1], a.v[2], a.v[3])
+    return {QW_P(W), QW_P(y), QW_P(yh), QW_P(N), QW_P(fmt), QW_P(rowbytes), QW_P(ystride)};
+#undef QW_P
+}
+// The wave's part of tile t of a matrix: block `wave` of the rows. x: the wave's own LDS. XN: loads of two tokens, 2 XN >= nb.
+template <int F, int XN> __device__ __forceinline__ f4 qmvs_part(const qwk_qmvm_args &a, const qmvs_mat &M, uint32_t t, u2 *tab, u4 *x) {
     typedef qw_small_blk<F> B;
     constexpr bool iq3 = F == 21 || F == QW_F_PACKED, iq4 = F == 20 || F == 23;
     const uint32_t lane = qw_lane(), wave = qw_wave(), n = lane & 15, kg = lane >> 4, row = 16 * t + (lane >> 2);
@@ -151,8 +169,8 @@ template <int F, int XN> __device__ __forceinline__ f4 qmvs_part(const qwk_qmvm_
         xv[i] = *(const u4 *)(xs + (size_t)(m < a.nb ? m : a.nb - 1) * a.xstride);
     }
     typename B::C c;
-    if constexpr (F == QW_F_PACKED) c.load(a.W[j] + (size_t)t * a.rowbytes[j] + wave * B::BYTES, lane);
-    else c.load(a.W[j] + (size_t)(row < a.N[j] ? row : a.N[j] - 1) * a.rowbytes[j] + wave * B::BYTES, lane & 3);
+    if constexpr (F == QW_F_PACKED) c.load(M.W + (size_t)t * M.rowbytes + wave * B::BYTES, lane);
+    else c.load(M.W + (size_t)(row < M.N ? row : M.N - 1) * M.rowbytes + wave * B::BYTES, lane & 3);
     if constexpr (iq3) {
         ((u4 *)tab)[threadIdx.x & 255] = te[0];
         if (many)

@@ -99,9 +99,12 @@ bool qw_path_qmv_gg(qw_path *p, qw_batch *b, const qw_tensor *W, int N, int K, c
     char name[96], defs[512];
     const int f = W->type;
     snprintf(name, sizeof name, "qmv_gg_f%d_k%d_n%d%s", f, K, nb, fout ? "_f" : "");
-    snprintf(defs, sizeof defs, "#define IQ_DQ_ONLY 1\n#define qmv_gg %s\n#define GF %d\n#define KD %d\n#define RB %d\n#define NB %d\n%s", name, f, K,
-             row_bytes(f, K), nb, fout ? "#define YT float\n" : "");
-    qw_kernel *k = compile_get(p, name, defs);
+    qw_kernel *k = qw_kernel_get(p->g, name);
+    if (!k) { // (the text is only made for a kernel that is new)
+        snprintf(defs, sizeof defs, "#define IQ_DQ_ONLY 1\n#define qmv_gg %s\n#define GF %d\n#define KD %d\n#define RB %d\n#define NB %d\n%s", name, f, K,
+                 row_bytes(f, K), nb, fout ? "#define YT float\n" : "");
+        k = compile_get(p, name, defs);
+    }
     if (!k) return false;
     struct { uint32_t N, xs, ys, pad; } a = {(uint32_t)N, (uint32_t)K, (uint32_t)N, 0};
     qw_batch_kernel(b, k);
@@ -124,9 +127,12 @@ bool qw_path_qmv_ggm(qw_path *p, qw_batch *b, const qw_tensor *W, const int *N, 
     for (int i = 0; i < 4; i++) f[i] = W[i < n ? i : 0].type;
     snprintf(base, sizeof base, "qmv_ggm_k%d_m%d_%d_%d_%d_%d%s", K, n, f[0], f[1], f[2], f[3], fout ? "_f" : "");
     snprintf(name, sizeof name, "%s_b%d", base, nb);
-    snprintf(defs, sizeof defs, "#define IQ_DQ_ONLY 1\n#define qmv_ggm %s\n#define KD %d\n#define NB 0\n#define NMAT %d\n#define GF0 %d\n#define GF1 %d\n#define GF2 %d\n#define GF3 %d\n%s",
-             base, K, n, f[0], f[1], f[2], f[3], fout ? "#define YT float\n" : "");
-    qw_kernel *k = compile_get(p, name, defs);
+    qw_kernel *k = qw_kernel_get(p->g, name);
+    if (!k) {
+        snprintf(defs, sizeof defs, "#define IQ_DQ_ONLY 1\n#define qmv_ggm %s\n#define KD %d\n#define NB 0\n#define NMAT %d\n#define GF0 %d\n#define GF1 %d\n#define GF2 %d\n#define GF3 %d\n%s",
+                 base, K, n, f[0], f[1], f[2], f[3], fout ? "#define YT float\n" : "");
+        k = compile_get(p, name, defs);
+    }
     if (!k) return false;
     struct { uint32_t N[4], off[4], total, xstride; } a = {{0}, {0}, 0, (uint32_t)K};
     qw_batch_kernel(b, k);
