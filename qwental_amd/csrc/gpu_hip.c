@@ -2007,7 +2007,9 @@ static bool tr_cmb(qw_batch *b) {
         if (!flush_gu(b) || !flush_dn(b)) return false;
     }
     if (!flush_gu(b)) return false;
-    return add_launch(b, "qwk_cmb", cdiv(nbr * (unsigned)p->D, 256), 256, &a, sizeof a);
+    if (!add_launch(b, "qwk_cmb", cdiv((unsigned)p->D, 256), 256, &a, sizeof a)) return false;
+    b->l[b->nl - 1].gy = nbr;
+    return true;
 }
 
 // ---------------------------------------------------------------- ragged packing (kernels/moe_prefill.metal; src/engine.c:4133-4224)

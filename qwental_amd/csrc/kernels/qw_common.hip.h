@@ -39,6 +39,8 @@ typedef u2 __attribute__((aligned(2))) u2a2;
 // they asked for anything else. No launch here has such a workgroup; this is a scalar load beside the arguments'.)
 __device__ __forceinline__ uint32_t qw_threads() { return __builtin_amdgcn_workgroup_size_x(); }
 
+// Loads above it are issued above it. (The scheduler saves registers in a short kernel by moving each load to its use: a round trip each.)
+__device__ __forceinline__ void qw_asked() { __builtin_amdgcn_sched_barrier(0); }
 // x / d with mul = 2^32 / d + 1 from the host (QW_DIV_MUL), exact for x * d < 2^32, d >= 2: one instruction, where a division by an argument
 // is a chain of some thirty - and the address of a launch's first load often waits for several of them.
 __device__ __forceinline__ uint32_t qw_div(uint32_t x, uint32_t mul) { return __umulhi(x, mul); }

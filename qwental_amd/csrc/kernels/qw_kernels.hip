@@ -671,6 +671,10 @@ struct qw_sel_scratch {
     float w[16 * 17];
 };
 
+// What hardly ever comes is marked so: its code then lies behind the rest. (Between the steps that always come it cost a jump over it to
+// instructions that no cache holds at the start of a launch: 0.4 us between a token's last pick and the barrier behind it.)
+#define QW_SELDOM(c) __builtin_expect(!!(c), 0)
+
 // PER = E / 64 values per lane, lane l holding experts l * PER .. l * PER + PER - 1 (lowest lane = lowest index).
 // T tokens at once (tok0, tok0 + tstep, ...; those >= nbr are skipped): a round is a chain of dependent instructions,
 // so two tokens in flight cost about the time of one. Every lane keeps the maximum of its PER keys and the position
@@ -788,10 +792,10 @@ __device__ __forceinline__ uint32_t select_tokens_ranked(const float *logits, ui
         gather(t);
         if (c[t] > 64) more |= 1u << t;
     }
-    if (more) refine(more, 15, 0);
+    if (QW_SELDOM(more)) refine(more, 15, 0);
 #pragma unroll
     for (int t = 0; t < T; t++) {
-        if ((more >> t) & 1) gather(t);
+        if (QW_SELDOM((more >> t) & 1)) gather(t);
         if (c[t] > 64 || !on[t]) fail |= 1u << t;
     }
     QW_SDEP(pos[T - 1][PER - 1]);
@@ -884,7 +888,7 @@ __device__ __forceinline__ void select_token_any(const float *lg, float *v, uint
     if (lane == K) w[tok * (K + 1) + K] = 1.0f / (1.0f + __expf(-lg[E]));
 }
 
-__device__ __forceinline__ bool qw_select_fast_e(uint32_t E) { return E == 64 || E == 128 || E == 256 || E == 512 || E == 1024; }
+__device__ __forceinline__ bool qw_select_fast_e(uint32_t E) { return (E & (E - 1)) == 0 && E >= 64 && E <= 1024; }
 
 // The whole selection by one workgroup (a multiple of 64 threads, at least nbr * topk of them). lgs: LDS scratch, 1024
 // floats per wave (288 are used when E is 64 * {1, 2, 4, 8, 16}). c is complete for every thread on return.
@@ -917,7 +921,7 @@ __device__ __forceinline__ void select_all(const qwk_select_args &a, qw_sel_scra
         stage(wave - tw, NSTAGE);
         QW_SSTAMP(4);
         clear();
-    } else if (fast) { // a wave takes one token, or two when there are more tokens than such waves (lgs gives a wave 288 dwords)
+    } else if (__builtin_expect(fast, 1)) { // a wave takes one token, or two when there are more tokens than such waves (lgs gives a wave 288 dwords)
         uint32_t *ws = (uint32_t *)lgs + 288 * wave;
         const uint32_t trot = ((blockIdx.x & 15) * a.nbr) >> 4; // the workgroups of a launch read the tokens' logits in different orders
         auto rot = [&](uint32_t tt) { return tt + trot < a.nbr ? tt + trot : tt + trot - a.nbr; };
@@ -946,10 +950,10 @@ __device__ __forceinline__ void select_all(const qwk_select_args &a, qw_sel_scra
             default: fail = select_tokens_ranked<16, 1>(a.logits, E, K, t1, on1, s.w, s.ids, ws, lane, need_w, clear); break;
             }
             for (uint32_t i = 0; i < 2; i++) // more than 64 keys tie at the bound
-                if (((fail >> i) & 1) && (i == 0 || two)) slow(tk[i]);
+                if (QW_SELDOM(((fail >> i) & 1) && (i == 0 || two))) slow(tk[i]);
         } else clear();
         // tokens that the first pass does not reach (more than such waves when a lane holds sixteen keys, more than twice as many otherwise)
-        for (uint32_t tt = wave + (pairs ? 2 : 1) * tw; tt < a.nbr; tt += tw) {
+        for (uint32_t tt = wave + (pairs ? 2 : 1) * tw; QW_SELDOM(tt < a.nbr); tt += tw) {
             const uint32_t t1[1] = {rot(tt)};
             const bool on1[1] = {true};
             if (pairs || select_tokens_ranked<16, 1>(a.logits, E, K, t1, on1, s.w, s.ids, ws, lane, need_w, [] {})) slow(t1[0]);
@@ -1030,13 +1034,29 @@ extern "C" __global__ __launch_bounds__(1024) void qwk_select(qwk_select_args a)
 // ================================================================ gate/up + SwiGLU (kernels/moe_gg.metal:428-447, 563-573, 600-631)
 // A tile holds gate rows j0..j0+7 (n < 8) and up rows j0..j0+7 (n >= 8) of one expert; the up results move over by
 // 8 lanes, and H = g / (1 + exp(-g)) * up is stored as binary16 hi + lo planes for the tokens that picked the expert.
+// All of it in one round trip: a thread takes an expert, a mask and up to two dwords of slots (at most 256 and 1024; workgroups of
+// 512 threads and more), the first ones again where there are fewer. (In loops it was three.)
+struct qw_sel_read {
+    uint32_t ue, mask, s0, s1, U;
+    __device__ __forceinline__ void ask(const uint8_t *sel, uint32_t K, uint32_t gnb) {
+        const uint32_t GU = gnb * K, ns = GU * gnb / 4, i = threadIdx.x, j = i + qw_threads();
+        const uint32_t *slot = (const uint32_t *)(sel + QW_SEL_OFF_SLOT(gnb, K));
+        ue = ((const uint32_t *)(sel + QW_SEL_OFF_UE(gnb, K)))[i < GU ? i : 0], mask = ((const uint32_t *)(sel + QW_SEL_OFF_MASK(gnb, K)))[i < GU ? i : 0];
+        s0 = slot[i < ns ? i : 0], s1 = slot[j < ns ? j : 0], U = ((const uint32_t *)sel)[i >> 10]; // (0, but not for the compiler: a scalar load would wait for its use)
+    }
+    __device__ __forceinline__ void put(qw_sel_cache &c, uint32_t K, uint32_t gnb) const {
+        const uint32_t GU = gnb * K, ns = GU * gnb / 4, i = threadIdx.x, j = i + qw_threads();
+        if (i < GU) c.ue[i] = ue, c.mask[i] = mask;
+        if (i < ns) ((uint32_t *)c.slot)[i] = s0;
+        if (j < ns) ((uint32_t *)c.slot)[j] = s1;
+        if (i == 0) c.U = U;
+    }
+};
 __device__ __forceinline__ void qw_sel_load(qw_sel_cache &c, const uint8_t *sel, uint32_t K, uint32_t gnb) {
-    const uint32_t GU = gnb * K;
-    const uint32_t *ue = (const uint32_t *)(sel + QW_SEL_OFF_UE(gnb, K)), *mask = (const uint32_t *)(sel + QW_SEL_OFF_MASK(gnb, K));
-    const uint32_t *slot = (const uint32_t *)(sel + QW_SEL_OFF_SLOT(gnb, K));
-    for (uint32_t i = threadIdx.x; i < GU; i += qw_threads()) c.ue[i] = ue[i], c.mask[i] = mask[i];
-    for (uint32_t i = threadIdx.x; i < GU * gnb / 4; i += qw_threads()) ((uint32_t *)c.slot)[i] = slot[i];
-    if (threadIdx.x == 0) c.U = *(const uint32_t *)sel;
+    qw_sel_read r;
+    r.ask(sel, K, gnb);
+    qw_asked();
+    r.put(c, K, gnb);
 }
 
 // The sums of 32 activations of every token from their fragments in LDS, in index order (all threads; a barrier before and after).
@@ -1147,7 +1167,7 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, f
     if constexpr (FGU == QW_F_RT) qw_kq_tab_build((uint32_t *)(lut + (qw_has_lut(FSG) ? QW_LUT_ENTRIES : 0))); // (published by the barriers below)
     if (a.logits) { // the selection, made here by every workgroup
         const qwk_select_args sa = {a.logits, const_cast<uint8_t *>(a.sel), a.nbr, a.E, a.topk, a.gnb};
-        if (qw_select_fast_e(a.E)) {
+        if (__builtin_expect(qw_select_fast_e(a.E), 1)) {
             // The selection's scratch lies behind the staged activations when D leaves room there (D <= 2048), else in
             // their place (they follow in ready()).
             constexpr bool lutp = qw_has_lut(FGU) || qw_has_lut(FSG);
@@ -1869,6 +1889,10 @@ __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *p
     constexpr uint32_t TPER = TAB ? (QW_LUT_BYTES / 16 + QW_WG_DN - 1) / QW_WG_DN : 0;
     u4 tabv[TPER ? TPER : 1];
     uint32_t tat[TPER ? TPER : 1];
+    qw_sel_read rec;
+    rec.ask(a.sel, K, gnb);
+    const uint32_t nwt = a.nbr * (K + 1); // (at most QW_DNC_MAXNB tokens: fewer than there are threads)
+    const float rw = ((const float *)(a.sel + QW_SEL_OFF_W(gnb, K)))[threadIdx.x < nwt ? threadIdx.x : 0];
     if constexpr (TAB) { // (every workgroup starts at another place of the table; the last piece of some threads repeats an earlier one)
 #pragma unroll
         for (uint32_t it = 0; it < TPER; it++) {
@@ -1878,9 +1902,9 @@ __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *p
             tabv[it] = ((const u4 *)a.glut)[tat[it]];
         }
     }
-    qw_sel_load(*sc, a.sel, K, gnb);
-    const float *wg = (const float *)(a.sel + QW_SEL_OFF_W(gnb, K));
-    for (uint32_t i = threadIdx.x; i < a.nbr * (K + 1); i += qw_threads()) wl[i] = wg[i];
+    qw_asked();
+    rec.put(*sc, K, gnb);
+    if (threadIdx.x < nwt) wl[threadIdx.x] = rw;
     if (qw_has_tab(F) || qw_has_tab(FSD)) qw_kq_tab_build((uint32_t *)lut); // the byte table of the 4-bit codebook instead
     if constexpr (TAB) {
 #pragma unroll
@@ -2930,19 +2954,25 @@ QW_PFR(2, qwk_pfr_f121_c2) QW_PFR(1, qwk_pfr_f121_c1)
 // ================================================================ combine (kernels/moe_gg.metal:655-663)
 // Rank order, then the shared expert. One thread per (token, row).
 #if QW_IN_PART(5)
-extern "C" __global__ __launch_bounds__(256) void qwk_cmb(qwk_cmb_args a) {
-    const uint32_t i = blockIdx.x * qw_threads() + threadIdx.x;
-    if (i >= a.nbr * a.D) return;
-    const uint32_t t = i / a.D, row = i % a.D, K = a.topk;
+extern "C" __global__ __launch_bounds__(256) void qwk_cmb(qwk_cmb_args a) { // grid: 256 rows, tokens
+    const uint32_t t = blockIdx.y, row = blockIdx.x * 256 + threadIdx.x, K = a.topk;
+    if (row >= a.D) return;
     const float *w = (const float *)(a.sel + QW_SEL_OFF_W(a.gnb, K)) + t * (K + 1);
-    float pg[16];
+    // Everything in one round trip, without conditions (past topk the last one again): the weights by scalar loads - a workgroup has one token.
+    // (With a condition a load, or moved to their uses, they were up to sixteen round trips. IQ4_NL layers at eight tokens 778 -> 748 us over twelve.)
+    float pg[16], wv[16];
+    const float wk = w[K], ps = a.Psh[(size_t)t * a.D + row];
 #pragma unroll
-    for (uint32_t s = 0; s < 16; s++) pg[s] = s < K ? a.Pg[((size_t)t * K + s) * a.D + row] : 0.0f; // loads first
+    for (uint32_t s = 0; s < 16; s++) {
+        const uint32_t c = s < K ? s : K - 1;
+        pg[s] = a.Pg[((size_t)t * K + c) * a.D + row], wv[s] = w[c];
+    }
+    qw_asked();
     float o = 0;
 #pragma unroll
     for (uint32_t s = 0; s < 16; s++)
-        if (s < K) o = __builtin_fmaf(w[s], pg[s], o);
-    o = __builtin_fmaf(w[K], a.Psh[(size_t)t * a.D + row], o);
+        if (s < K) o = __builtin_fmaf(wv[s], pg[s], o);
+    o = __builtin_fmaf(wk, ps, o);
     a.out[(size_t)t * a.D + row] = qw_f2h(o);
 }
 #endif
