@@ -2150,15 +2150,17 @@ __device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_l
         for (uint32_t j = 0; j < 4; j++) r_sl[j] = sl[ri * gnb + t0 + (j < nt ? j : 0)];
         const float r_w = wg[hasw ? tid : 0];
         const uint32_t upr = a.I / 8, cbs = upr / 8, used = nt * (K + 1), nrb = (used + 7) / 8, nunits = 2 * nrb * cbs, wv = qw_wave();
+        // (I is 256 or 512, so cbs 4 or 8; a unit in use has rest < 2 nrb. A unit's part of the addresses is scalar, a lane's the same in all of
+        // them, and an offset of 32 bits goes with the load: thirty instructions and a branch a load otherwise, before the table is asked for.)
+        const uint32_t lr = (lane >> 2) & 7, lc = 4 * (lane >> 5) + (lane & 3), loff = 2 * (lr * a.I + 8 * lc), lat = lc * QW_DNQ_ROWS + lr;
 #pragma unroll
         for (uint32_t it = 0; it < RPER; it++) {
-            // (I is 256 or 512, so cbs 4 or 8; a unit in use has rest < 2 nrb. By divisions this was a microsecond in front of the loads.)
             const uint32_t unit = wv + it * NW, cb = unit & (cbs - 1), rest = unit >> __builtin_ctz(cbs), pl = rest >= nrb, rb = rest - (pl ? nrb : 0);
-            const uint32_t r = 8 * rb + ((lane >> 2) & 7), c = 8 * cb + 4 * (lane >> 5) + (lane & 3);
-            const bool on = unit < nunits && r < used;
-            at[it] = on ? (pl * upr + c) * QW_DNQ_ROWS + r : ~0u;
+            const uint32_t off = lr < (unit < nunits ? used - 8 * rb : 0) ? 0 : ~0u;
+            const uint32_t sat = (pl * upr + 8 * cb) * QW_DNQ_ROWS + 8 * rb, soff = 2 * ((pl ? a.hplane : 0) + (t0 * (K + 1) + 8 * rb) * a.I + 64 * cb);
+            at[it] = ((uint32_t)__builtin_amdgcn_readfirstlane((int)sat) + lat) | off; // (masks: a choice became a branch)
             // (a unit that is off reads the first bytes of H: a load under a condition made the compiler keep the whole array in scratch memory)
-            rowv[it] = *(const u4 *)(on ? a.H + pl * (size_t)a.hplane + ((size_t)t0 * (K + 1) + r) * a.I + 8 * c : a.H);
+            rowv[it] = *(const u4 *)((const char *)a.H + (((uint32_t)__builtin_amdgcn_readfirstlane((int)soff) + loff) & ~off));
         }
         if constexpr (TAB) { // every workgroup starts at another place of the table (as qw_lut_copy_issue); the last piece of some threads repeats an earlier one
 #pragma unroll
@@ -3047,16 +3049,19 @@ template <uint32_t R> __device__ __forceinline__ void hc_down_body(const qwk_hc_
         }
     }
     QW_HSTAMP(1);
+    float jv[QW_HC_TG]; // (here, while the loads above are under way: in the loop below each token's waited for scalar loads of its own)
+    if (a.apply)
+#pragma unroll
+        for (uint32_t tt = 0; tt < QW_HC_TG; tt++) jv[tt] = hc_coef(a.inj + (t0 + (tt < nt ? tt : 0)) * QW_HC * QW_HC, s);
 #pragma unroll
     for (uint32_t tt = 0; tt < QW_HC_TG; tt++) {
         if (tt >= nt) break;
         float v[8] = {hv[tt][0][0], hv[tt][0][1], hv[tt][0][2], hv[tt][0][3], hv[tt][1][0], hv[tt][1][1], hv[tt][1][2], hv[tt][1][3]};
         if (a.apply) {
-            const float js = hc_coef(a.inj + (t0 + tt) * QW_HC * QW_HC, s);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                v[2 * k] = fmaf(qw_h2f((uint16_t)ou[tt][k]), js, v[2 * k]);
-                v[2 * k + 1] = fmaf(qw_h2f((uint16_t)(ou[tt][k] >> 16)), js, v[2 * k + 1]);
+                v[2 * k] = fmaf(qw_h2f((uint16_t)ou[tt][k]), jv[tt], v[2 * k]);
+                v[2 * k + 1] = fmaf(qw_h2f((uint16_t)(ou[tt][k] >> 16)), jv[tt], v[2 * k + 1]);
             }
         }
         float ss = 0, x[8];
