@@ -394,7 +394,7 @@ template <int F, int CH, bool XLDS> __device__ __forceinline__ void qmv_body(con
     });
 }
 #define QW_QMV(F, CH, XLDS, SFX)                                                                        \
-    extern "C" __global__ __launch_bounds__(QW_WG_GU) void qwk_qmv_f##F##SFX(qwk_qmv_args a) {             \
+    extern "C" __global__ __launch_bounds__(QW_WG_GU) void qwk_qmv_f##F##SFX(qwk_qmv_args a) { QW_THREADS(QW_WG_GU); \
         __shared__ struct { u2 lut[qw_has_lut(F) ? QW_LUT_ENTRIES : 1]; u4 xf[XLDS ? QW_XF_MAXK * 2 : 1]; f4 red[QW_WG_GU]; } L; /* table first: LDS address 0 */ \
         qw_started(a.t_start);                                                                          \
         qmv_body<F, CH, XLDS>(a, L.lut, L.xf, L.red);                                                   \
@@ -408,7 +408,7 @@ QW_QMV(121, 2, true, _c2) QW_QMV(121, 1, true, _c1) // packed IQ3_S: a.rowbytes 
 // Matrices that the device takes in one go, one to four a launch, any of the formats: qw_small.hip.h.
 #if QW_IN_PART(0)
 template <int XN> __device__ __forceinline__ void qmvs_body(const qwk_qmvm_args &a, u4 *dyn) { // dyn: table (tabu units), then a wave's activations, behind them in the same place its partial sums
-    const uint32_t lane = qw_lane(), wave = qw_wave(), nw = qw_threads() >> 6, own = a.sh ? 32u << a.sh : 64;
+    const uint32_t lane = qw_lane(), wave = qw_wave(), nw = a.K >> 8 /* a wave per 256 values */, own = a.sh ? 32u << a.sh : 64;
     u2 *tab = (u2 *)dyn;
     u4 *x = dyn + a.tabu + wave * own;
     uint32_t t = blockIdx.x;
@@ -514,6 +514,7 @@ template <int F, int NB> __device__ __forceinline__ void qmvm_matrix_split(const
 }
 #if QW_IN_PART(0)
 extern "C" __global__ __launch_bounds__(QW_WG_QMVM) void qwk_qmvm(qwk_qmvm_args a) {
+    QW_THREADS(QW_WG_QMVM);
     __shared__ struct { u4 xf[QW_KQ_MAXK * 2]; float xs[QW_KQ_MAXK / 2]; uint32_t tab[QW_KQ_TAB]; f4 red[QW_WG_QMVM]; } L;
     qw_started(a.t_start);
     qw_kq_tab_build(L.tab);
@@ -604,7 +605,7 @@ template <int NT> __device__ __forceinline__ void qmv_valu_body(const qwk_qmv_ar
         });
 }
 #define QW_QMV_VALU(NT)                                                                                  \
-    extern "C" __global__ __launch_bounds__(QW_WG_GU) void qwk_qmv_valu_n##NT(qwk_qmv_args a) {          \
+    extern "C" __global__ __launch_bounds__(QW_WG_GU) void qwk_qmv_valu_n##NT(qwk_qmv_args a) { QW_THREADS(QW_WG_GU); \
         __shared__ struct { u2 lut[QW_LUT_ENTRIES]; u4 xf[QW_XF_MAXK * 2]; } L;                          \
         qmv_valu_body<NT>(a, L.lut, L.xf);                                                               \
     }
@@ -1024,6 +1025,7 @@ __device__ __forceinline__ void select_all(const qwk_select_args &a, qw_sel_scra
 
 #if QW_IN_PART(0)
 extern "C" __global__ __launch_bounds__(1024) void qwk_select(qwk_select_args a) {
+    QW_THREADS(1024);
     __shared__ qw_sel_scratch s;
     __shared__ qw_sel_cache c;
     __shared__ float lgs[16 * 1024];
@@ -1238,7 +1240,7 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, f
     QW_DSTAMP(2);
 }
 #define QW_GU(FGU, CHGU, FSG, CHSG, NAME)                                                                 \
-    extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_gu_args a) {                             \
+    extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_gu_args a) { QW_THREADS(QW_WG_GU); \
         __shared__ struct { u2 lut[((qw_has_lut(FGU) || qw_has_lut(FSG)) ? QW_LUT_ENTRIES : 0) + (FGU == QW_F_RT ? QW_KQ_TAB / 2 : 1)]; u4 xf[QW_XF_MAXK * 2]; qw_sel_cache sc; qw_sel_scratch ss; } L; \
         qw_h_global hs = {a.H, a.hplane};                                                                      \
         static_assert(sizeof(qw_sel_scratch) >= QW_XF_MAXK / 2 * sizeof(float), "the sums of 32 activations take the place of the selection's scratch"); \
@@ -1322,7 +1324,7 @@ struct qw_pre_x {
 // Binary16 rows, sixteen a workgroup.
 __device__ __forceinline__ void pre_router(const qwk_pre_args &a, qw_pre_lds &L) {
     const qwk_router_args &r = a.r;
-    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave(), nwv = (qw_threads() >> 6) < 8 ? qw_threads() >> 6 : 8;
+    const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave(), nwv = ((r.D >> 2) >> 6) < 8 ? (r.D >> 2) >> 6 : 8;
     u4 *const x = L.x + wave * 512;
     f4 acc = {0, 0, 0, 0};
     if (wave < nwv) {
@@ -1376,10 +1378,10 @@ template <int NB> __device__ __forceinline__ void pre_router_bf(const qwk_pre_ar
         if (64 * k < units) wv[k] = *(const u4 *)(w + 8 * (lane + 64 * k < units ? lane + 64 * k : 0));
 #pragma unroll
     for (uint32_t k = 0; k < 4; k++) // (two tokens to a round of the workgroup's threads)
-        if (k * qw_threads() < nx) xv[k] = ((const u4 *)(r.x + (size_t)t0 * r.D))[threadIdx.x + k * qw_threads() < nx ? threadIdx.x + k * qw_threads() : 0];
+        if (k * (r.D >> 2) < nx) xv[k] = ((const u4 *)(r.x + (size_t)t0 * r.D))[threadIdx.x + k * (r.D >> 2) < nx ? threadIdx.x + k * (r.D >> 2) : 0];
 #pragma unroll
     for (uint32_t k = 0; k < 4; k++)
-        if (threadIdx.x + k * qw_threads() < nx) L.x[threadIdx.x + k * qw_threads()] = xv[k];
+        if (threadIdx.x + k * (r.D >> 2) < nx) L.x[threadIdx.x + k * (r.D >> 2)] = xv[k];
     __syncthreads();
     float acc[NB];
 #pragma unroll
@@ -1411,7 +1413,7 @@ template <int NB> __device__ __forceinline__ void pre_router_bf(const qwk_pre_ar
 template <int WF> __device__ __forceinline__ void pre_router_any(const qwk_pre_args &a, qw_pre_lds &L) {
     if constexpr (WF == 1) pre_router(a, L);
     else {
-        const uint32_t nwv = qw_threads() >> 6, nrb = (a.r.E + nwv) / nwv, t0 = 8 * (blockIdx.x / nrb), r0 = blockIdx.x % nrb * nwv, nt = a.r.nb - t0 < 8 ? a.r.nb - t0 : 8;
+        const uint32_t nwv = (a.r.D >> 2) >> 6, nrb = (a.r.E + nwv) / nwv, t0 = 8 * (blockIdx.x / nrb), r0 = blockIdx.x % nrb * nwv, nt = a.r.nb - t0 < 8 ? a.r.nb - t0 : 8;
         if (nt == 1) pre_router_bf<1>(a, L, r0, t0, nt);
         else if (nt == 2) pre_router_bf<2>(a, L, r0, t0, nt);
         else if (nt <= 4) pre_router_bf<4>(a, L, r0, t0, nt);
@@ -1444,7 +1446,7 @@ template <int F> __device__ __forceinline__ f4 pre_mac(const uint32_t (&r)[32], 
 template <int SH> __device__ __forceinline__ void pre_shared(const qwk_pre_args &a, uint32_t t, qw_pre_lds &L) {
     const qwk_router_args &r = a.r;
     const uint32_t lane = qw_lane(), n = lane & 15, kg = lane >> 4, wave = qw_wave();
-    const uint32_t nwv = SH == 8 ? r.D / 512 : qw_threads() >> 6; // the waves that take part
+    const uint32_t nwv = SH == 8 ? r.D / 512 : (r.D >> 2) >> 6; // the waves that take part
     u4 *const x = L.x + wave * (SH == 8 ? 1024 : 512);
     const qw_afrag_small af = {x, n & ((1u << a.sh) - 1), a.sh};
     f4 g = {0, 0, 0, 0};
@@ -1469,7 +1471,7 @@ template <int SH> __device__ __forceinline__ void pre_shared(const qwk_pre_args 
         else c.load((lane < 32 ? a.Wg : a.Wu) + ((size_t)8 * t + ((lane >> 2) & 7)) * a.rbg + wave * qw_small_blk<SH>::BYTES, lane & 3);
         xv.load(r, 256 * wave);
         if constexpr (SH == QW_F_PACKED) { // the table, a unit a thread or four (a few by several threads)
-            const uint32_t few = qw_threads() < 256 ? 4 : 1;
+            const uint32_t few = (r.D >> 2) < 256 ? 4 : 1;
             for (uint32_t i = 0; i < few; i++) ((u4 *)L.tab)[(threadIdx.x + 64 * i) & 255] = ((const u4 *)a.ctab)[(threadIdx.x + 64 * i) & 255];
             if (threadIdx.x < 16) qw_small_signs(L.tab, threadIdx.x);
         }
@@ -1599,7 +1601,7 @@ __device__ __forceinline__ void pre_pair(const qwk_pre_args &a, uint32_t t, qw_p
         if (wave) ((f4 *)x)[lane] = g, ((f4 *)x)[64 + lane] = u;
         __syncthreads();
         if (wave) return;
-        for (uint32_t q = 1; q < qw_threads() >> 6; q++) g += ((const f4 *)L.x)[q * 512 + lane], u += ((const f4 *)L.x)[q * 512 + 64 + lane];
+        for (uint32_t q = 1; q < (r.D >> 2) >> 6; q++) g += ((const f4 *)L.x)[q * 512 + lane], u += ((const f4 *)L.x)[q * 512 + 64 + lane];
     }
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++)
@@ -1815,14 +1817,14 @@ template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_r
     }
 }
 #define QW_DN_RANGE(F, CH, FSD, CHSD, NAME)                                                       \
-    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) {                  \
+    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) { QW_THREADS(QW_WG_DN); \
         __shared__ struct { u2 lut[(qw_has_lut(F) || qw_has_lut(FSD)) ? QW_LUT_ENTRIES : (qw_has_tab(F) || qw_has_tab(FSD)) ? QW_KQ_TAB / 2 : 1]; uint16_t arows[2 * 16 * 2 * 512]; qw_sel_cache sc; } L; \
         dn_range_body<F, CH, FSD, CHSD>(a, L.lut, L.arows, &L.sc);                                \
     }
 // IQ4_NL rows (the reference model's down projections: I = 640, five chunks of 4 blocks a row): no IQ3_S table in LDS,
 // so the staged H rows may be 640 wide
 #define QW_DN_RANGE_NL(CH, FSD, CHSD, NAME)                                                       \
-    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) {                  \
+    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) { QW_THREADS(QW_WG_DN); \
         __shared__ struct { u2 lut[QW_KQ_TAB / 2]; uint16_t arows[2 * 16 * 2 * 640]; qw_sel_cache sc; } L; \
         dn_range_body<20, CH, FSD, CHSD>(a, L.lut, L.arows, &L.sc);                               \
     }
@@ -1830,7 +1832,7 @@ template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_r
 QW_DN_RANGE_NL(4, 0, 1, qwk_dnr_f20_c4) QW_DN_RANGE_NL(4, 20, 4, qwk_dnr_f20_c4_s20_c4) QW_DN_RANGE_NL(4, 8, 4, qwk_dnr_f20_c4_s8_c4)
 #endif
 #define QW_DN_RANGE_NLP(FSD, CHSD, NAME)                                                          \
-    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) {                  \
+    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) { QW_THREADS(QW_WG_DN); \
         __shared__ struct { u2 lut[QW_KQ_TAB / 2]; uint16_t arows[2 * 16 * 2 * 640]; qw_sel_cache sc; } L; \
         dn_range_body<QW_F_PACKED_NL, 10, FSD, CHSD>(a, L.lut, L.arows, &L.sc);                   \
     }
@@ -1964,7 +1966,7 @@ __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *p
     qw_back_fin(a.back, a.fin);
 }
 #define QW_DNC(F, CH, FSD, CHSD, NAME)                                                              \
-    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) {                    \
+    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) { QW_THREADS(QW_WG_DN); \
         __shared__ struct { u2 lut[(qw_has_lut(F) || qw_has_lut(FSD)) ? QW_LUT_ENTRIES : (qw_has_tab(F) || qw_has_tab(FSD)) ? QW_KQ_TAB / 2 : 1]; float part[QW_DNC_MAXNB * 17 * 16], wl[QW_DNC_MAXNB * 17]; qw_sel_cache sc; } L; \
         dnc_body<F, CH, FSD, CHSD>(a, L.lut, L.part, L.wl, &L.sc);                                  \
     }
@@ -2239,7 +2241,7 @@ __device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_l
     qw_back_fin(a.back, a.fin);
 }
 #define QW_DNQ(F, CH, FSD, CHSD, NAME)                                                              \
-    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) {                    \
+    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) { QW_THREADS(QW_WG_DN); \
         __shared__ struct { u2 lut[qw_has_lut(F) || qw_has_lut(FSD) ? QW_LUT_ENTRIES : 1]; qw_dnq_lds d; } L; \
         dnq_body<F, CH, FSD, CHSD>(a, L.lut, L.d);                                                  \
     }
@@ -2422,7 +2424,7 @@ template <int FSD, int CHSD> __device__ __forceinline__ void gud_body(const qwk_
     }
 }
 #define QW_GUD(FSD, CHSD, NAME)                                                                     \
-    extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_gud_args a) {                   \
+    extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_gud_args a) { QW_THREADS(QW_WG_GU); \
         __shared__ qw_gud_lds L;                                                                    \
         gud_body<FSD, CHSD>(a, L);                                                                  \
     }
@@ -2497,12 +2499,13 @@ __device__ __forceinline__ void dn_rt_body(const qwk_dn_args &a, u2 *lut, qw_sel
 }
 #if QW_IN_PART(2)
 extern "C" __global__ __launch_bounds__(QW_WG) void qwk_dn_rt(qwk_dn_args a) {
+    QW_THREADS(QW_WG);
     __shared__ struct { u2 lut[QW_LUT_ENTRIES + QW_KQ_TAB / 2]; qw_sel_cache sc; } L;
     dn_rt_body(a, L.lut, &L.sc);
 }
 #endif
 #define QW_DN_ANY(F, FSD, NAME)                                                       \
-    extern "C" __global__ __launch_bounds__(QW_WG) void NAME(qwk_dn_args a) {         \
+    extern "C" __global__ __launch_bounds__(QW_WG) void NAME(qwk_dn_args a) { QW_THREADS(QW_WG); \
         __shared__ struct { u2 lut[(F == 21 || FSD == 21) ? QW_LUT_ENTRIES : (F == 20 || FSD == 20) ? QW_KQ_TAB / 2 : 1]; qw_sel_cache sc; } L; \
         dn_any_body<F, FSD>(a, L.lut, &L.sc);                                         \
     }
@@ -2658,6 +2661,7 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_prep(qwk_prep_args a) 
 // of stores are 16 at the rate of a large copy.
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(512) void qwk_moe_prep_slices(qwk_prep_args a) {
+    QW_THREADS(512);
     __shared__ uint32_t cnt[1024], at[1024], wr[8], wt[8], id[QW_PREP_SLICE], pos[QW_PREP_SLICE];
     qw_started(a.t_start);
     const uint32_t tid = threadIdx.x, nth = qw_threads(), lane = tid & 63, wave = tid >> 6, nwv = nth >> 6;
@@ -2868,7 +2872,7 @@ template <int F, int CH> __device__ __forceinline__ void pf_body(const qwk_pf_ar
         });
 }
 #define QW_PF(F, CH, NAME)                                                                       \
-    extern "C" __global__ __launch_bounds__(QW_WG) void NAME(qwk_pf_args a) {                    \
+    extern "C" __global__ __launch_bounds__(QW_WG) void NAME(qwk_pf_args a) { QW_THREADS(QW_WG); \
         __shared__ struct { u2 lut[qw_has_lut(F) ? QW_LUT_ENTRIES : F == 20 ? QW_KQ_TAB / 2 : 1]; u4 tl[2048]; uint32_t cnt; } L; \
         pf_body<F, CH>(a, L.lut, L.tl, &L.cnt);                                                  \
     }
@@ -2880,10 +2884,12 @@ QW_PF(121, 2, qwk_pf_f121_c2) QW_PF(121, 1, qwk_pf_f121_c1) // tile-major IQ3_S:
 
 #if QW_IN_PART(5)
 extern "C" __global__ __launch_bounds__(64 * QW_PFG_WAVES) void qwk_pfg_f121(qwk_pf_args a) {
+    QW_THREADS(64 * QW_PFG_WAVES);
     __shared__ qw_pfg_lds<QW_F_PACKED> L;
     pfg_body<QW_F_PACKED>(a, L);
 }
 extern "C" __global__ __launch_bounds__(64 * QW_PFG_WAVES) void qwk_pfg_f120(qwk_pf_args a) {
+    QW_THREADS(64 * QW_PFG_WAVES);
     __shared__ qw_pfg_lds<QW_F_PACKED_NL> L;
     pfg_body<QW_F_PACKED_NL>(a, L);
 }
@@ -2945,7 +2951,7 @@ template <int CH> __device__ __forceinline__ void pf_range_body(const qwk_pf_arg
     }
 }
 #define QW_PFR(CH, NAME)                                                                          \
-    extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_pf_args a) {                 \
+    extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_pf_args a) { QW_THREADS(QW_WG_GU); \
         __shared__ struct { u2 lut[QW_LUT_ENTRIES]; u4 xf[QW_XF_MAXK * 2]; uint32_t cnt; } L;     \
         pf_range_body<CH>(a, L.lut, L.xf, &L.cnt);                                                \
     }
@@ -3028,7 +3034,7 @@ template <int W> __device__ __forceinline__ float qw_sum4(float d0, float d1, fl
 // tokens, 10.0 -> 8.9 at sixteen, up 6.0 -> 5.0 and 8.5 -> 8.0 (D = 2048), with the same bits.
 template <uint32_t R> __device__ __forceinline__ void hc_down_body(const qwk_hc_args &a, float (*part)[QW_HC_TG][17]) {
     const uint32_t tg = (a.nb + gridDim.z - 1) / gridDim.z; // tokens of a group: as even as can be (five tokens: three and two)
-    const uint32_t rb = blockIdx.x, s = blockIdx.y, t0 = blockIdx.z * tg, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, nwv = qw_threads() >> 6;
+    const uint32_t rb = blockIdx.x, s = blockIdx.y, t0 = blockIdx.z * tg, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, nth = a.D >> 3 /* its threads */, nwv = nth >> 6;
     const uint32_t nt = a.nb - t0 < tg ? a.nb - t0 : tg;
     QW_HSTAMP(0);
     const bool is_inj = rb == QW_HC_LR / R;
@@ -3090,7 +3096,7 @@ template <uint32_t R> __device__ __forceinline__ void hc_down_body(const qwk_hc_
     QW_HSTAMP(3);
     __syncthreads();
     QW_HSTAMP(4);
-    for (uint32_t j = tid; j < nt * 17; j += qw_threads()) {
+    for (uint32_t j = tid; j < nt * 17; j += nth) {
         const uint32_t tt = j / 17, r = j % 17;
         if (r < 16 && r >= nrow) continue;
         float sum = 0;
@@ -3282,8 +3288,8 @@ template <bool GIVEN> __device__ __forceinline__ void hc_up_body(const qwk_hc_ar
     QW_HSTAMP(13);
 }
 #if QW_IN_PART(5)
-extern "C" __global__ __launch_bounds__(256) void qwk_hc_up(qwk_hc_args a) { hc_up_body<false>(a); }
-extern "C" __global__ __launch_bounds__(256) void qwk_hc_upv(qwk_hc_args a) { hc_up_body<true>(a); }
+extern "C" __global__ __launch_bounds__(256) void qwk_hc_up(qwk_hc_args a) { QW_THREADS(256); hc_up_body<false>(a); }
+extern "C" __global__ __launch_bounds__(256) void qwk_hc_upv(qwk_hc_args a) { QW_THREADS(256); hc_up_body<true>(a); }
 #endif
 
 // Read pattern of a decode layer without the decoding (kernels/moe_bw.metal:7-26): workgroup (x, c) reads slice x

@@ -154,7 +154,7 @@ template <int F, int XN> __device__ __forceinline__ f4 qmvs_part(const qwk_qmvm_
     const uint32_t lane = qw_lane(), wave = qw_wave(), n = lane & 15, kg = lane >> 4, row = 16 * t + (lane >> 2);
     // the part of the 256 units of table that this thread puts into LDS: one from 256 threads on, else four (some by several threads)
     u4 te[4];
-    const bool many = qw_threads() < 256;
+    const bool many = a.K < 1024; // (K / 4 threads)
     if constexpr (iq3) {
         te[0] = ((const u4 *)a.ctab)[threadIdx.x & 255];
         if (many)
