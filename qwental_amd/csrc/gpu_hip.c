@@ -209,6 +209,7 @@ struct qw_gpu {
     uint64_t batch_seq;
     qw_pack *packs;
     int npacks, cappacks;
+    unsigned pack_hint[512]; // where a copy was found last, by its source's address: looked at before all of them are
     qw_want *wants;
     int nwants, capwants;
     uint32_t copy_uses; // qw_hip_set_copy_uses
@@ -1429,13 +1430,18 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
     const bool pf = (fmt == QW_F_PACKED_NL && b->k->fam == FAM_PF) || (fmt == QW_F_PACKED_Q6 && b->k->fam == FAM_DN);
     const bool beside = fmt == QW_F_PACKED_Q8 || fmt == QW_F_PACKED_Q4K || (fmt == QW_F_PACKED_Q6 && b->k->fam == FAM_DN); // GGUF-order rows that the tuned kernels of a layer read too
     const uint32_t split = B ? 8 : 16;
+    unsigned *hint = &g->pack_hint[((uint64_t)(uintptr_t)A * 0x9e3779b97f4a7c15u ^ (uint64_t)fmt << 57) >> 55];
+    if (*hint < (unsigned)g->npacks) { // its own handles only: where the address of a released source was given out again, two copies have the same key
+        qw_pack *p = &g->packs[*hint];
+        if (p->A == A && p->B == B && p->ntiles == ntiles && p->nblk == nblk && p->fmt == fmt && p->ha == ha && p->hb == hb) return p->pf &= pf, p->dst;
+    }
     for (int i = 0; i < g->npacks; i++) {
         qw_pack *p = &g->packs[i];
         if (p->A != A || p->B != B || p->ntiles != ntiles || p->nblk != nblk || p->fmt != fmt) continue;
         // The addresses are the key (a view of the same memory under another handle finds the copy too) — unless the
         // source was released: its address may since have been given to another allocation, so only its own handle matches.
         const bool gone = (p->ha && p->ha->released) || (p->hb && p->hb->released);
-        if (!gone || (p->ha == ha && p->hb == hb)) return p->pf &= pf, p->dst;
+        if (!gone || (p->ha == ha && p->hb == hb)) return *hint = (unsigned)i, p->pf &= pf, p->dst;
     }
     if (b->noalloc) return NULL; // a copy that exists was found above; none is made here
     if ((ha && ha->released) || (hb && hb->released)) return NULL; // nothing left to copy from

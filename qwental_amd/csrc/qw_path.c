@@ -9,6 +9,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+enum { QW_MEMO = 64, QW_MEMO_WAYS = 8, QW_MEMO_KEY = 8 };
 struct qw_path {
     qw_gpu *g;
     int D, I, E, topk, nbmax;
@@ -22,6 +23,10 @@ struct qw_path {
     unsigned pf_max_tiles;
     uint64_t flush_mask; // bit l: submit what is recorded after layer l of a stack (src/engine.c:142, :5997 vb_flush)
     qw_buf vlg, vsel;    // logits and selection record of one group of a ragged step (qw_path_par_vstep), made at first use
+    // Kernels by what their names are made of (kernel_memo): the names are text, and three of them printed and looked up a
+    // dispatch were most of what recording a layer cost (24 layers, 72 launches: 108 us with the names and a search of all
+    // tile-major copies, 30 without; all of a batch is recorded before its first launch goes out)
+    struct { const char *base; int key[QW_MEMO_KEY]; qw_kernel *k; } memo[QW_MEMO];
 };
 
 static int blk_values(int type) { // src/gguf.c:15-25
@@ -80,6 +85,21 @@ void qw_path_close(qw_path *p) {
 
 const qw_buf *qw_path_scratch(const qw_path *p, int which) { return which == 0 ? &p->tab : which == 1 ? &p->H : which == 2 ? &p->psh : which == 3 ? &p->pd : NULL; }
 
+// Where the kernel of (base, key) is kept, and whether it is there; base by its address. A kernel stays where it is as long as its device is open.
+static qw_kernel **kernel_memo(qw_path *p, const char *base, const int *key, bool *hit) {
+    uint32_t h = (uint32_t)((uintptr_t)base >> 2);
+    for (int i = 0; i < QW_MEMO_KEY; i++) h = (h ^ (uint32_t)key[i]) * 0x9e3779b1u;
+    uint32_t at = h >> 26;
+    for (uint32_t i = 0; i < QW_MEMO_WAYS; i++) { // (any of a few places, so that two kernels of a layer do not keep putting each other out)
+        const uint32_t j = (at + i) % QW_MEMO;
+        if (p->memo[j].k && p->memo[j].base == base && !memcmp(p->memo[j].key, key, sizeof p->memo[j].key)) return *hit = true, &p->memo[j].k;
+    }
+    for (uint32_t i = 0; i < QW_MEMO_WAYS && p->memo[at].k; i++) at = (at + 1) % QW_MEMO; // all taken: the one behind them goes
+    p->memo[at].base = base, p->memo[at].k = NULL;
+    memcpy(p->memo[at].key, key, sizeof p->memo[at].key);
+    return *hit = false, &p->memo[at].k;
+}
+
 static qw_kernel *compile_get(qw_path *p, const char *name, const char *defs) {
     char err[2048];
     qw_kernel *k = qw_kernel_get(p->g, name);
@@ -98,12 +118,13 @@ bool qw_path_qmv_gg(qw_path *p, qw_batch *b, const qw_tensor *W, int N, int K, c
                     size_t yoff, int nb, bool fout) {
     char name[96], defs[512];
     const int f = W->type;
-    snprintf(name, sizeof name, "qmv_gg_f%d_k%d_n%d%s", f, K, nb, fout ? "_f" : "");
-    qw_kernel *k = qw_kernel_get(p->g, name);
-    if (!k) { // (the text is only made for a kernel that is new)
+    bool hit;
+    qw_kernel **memo = kernel_memo(p, "qmv_gg", (const int[QW_MEMO_KEY]){f, K, nb, fout}, &hit), *k = *memo;
+    if (!hit) {
+        snprintf(name, sizeof name, "qmv_gg_f%d_k%d_n%d%s", f, K, nb, fout ? "_f" : "");
         snprintf(defs, sizeof defs, "#define IQ_DQ_ONLY 1\n#define qmv_gg %s\n#define GF %d\n#define KD %d\n#define RB %d\n#define NB %d\n%s", name, f, K,
                  row_bytes(f, K), nb, fout ? "#define YT float\n" : "");
-        k = compile_get(p, name, defs);
+        *memo = k = compile_get(p, name, defs);
     }
     if (!k) return false;
     struct { uint32_t N, xs, ys, pad; } a = {(uint32_t)N, (uint32_t)K, (uint32_t)N, 0};
@@ -125,13 +146,14 @@ bool qw_path_qmv_ggm(qw_path *p, qw_batch *b, const qw_tensor *W, const int *N, 
     char base[128], name[140], defs[512];
     int f[4];
     for (int i = 0; i < 4; i++) f[i] = W[i < n ? i : 0].type;
-    snprintf(base, sizeof base, "qmv_ggm_k%d_m%d_%d_%d_%d_%d%s", K, n, f[0], f[1], f[2], f[3], fout ? "_f" : "");
-    snprintf(name, sizeof name, "%s_b%d", base, nb);
-    qw_kernel *k = qw_kernel_get(p->g, name);
-    if (!k) {
+    bool hit;
+    qw_kernel **memo = kernel_memo(p, "qmv_ggm", (const int[QW_MEMO_KEY]){K, n, f[0], f[1], f[2], f[3], fout, nb}, &hit), *k = *memo;
+    if (!hit) {
+        snprintf(base, sizeof base, "qmv_ggm_k%d_m%d_%d_%d_%d_%d%s", K, n, f[0], f[1], f[2], f[3], fout ? "_f" : "");
+        snprintf(name, sizeof name, "%s_b%d", base, nb);
         snprintf(defs, sizeof defs, "#define IQ_DQ_ONLY 1\n#define qmv_ggm %s\n#define KD %d\n#define NB 0\n#define NMAT %d\n#define GF0 %d\n#define GF1 %d\n#define GF2 %d\n#define GF3 %d\n%s",
                  base, K, n, f[0], f[1], f[2], f[3], fout ? "#define YT float\n" : "");
-        k = compile_get(p, name, defs);
+        *memo = k = compile_get(p, name, defs);
     }
     if (!k) return false;
     struct { uint32_t N[4], off[4], total, xstride; } a = {{0}, {0}, 0, (uint32_t)K};
@@ -151,7 +173,14 @@ bool qw_path_qmv_ggm(qw_path *p, qw_batch *b, const qw_tensor *W, const int *N, 
 }
 
 // ---------------------------------------------------------------- MoE kernels by part (src/engine.c:460-517)
+static qw_kernel *gg_kernel_new(qw_path *p, const char *base, const qw_moe_layer *M, int nb);
 static qw_kernel *gg_kernel(qw_path *p, const char *base, const qw_moe_layer *M, int nb) {
+    const int key[QW_MEMO_KEY] = {nb, M->router.type, M->gate.type, M->down.type, M->sh_gate.type, M->sh_up.type, M->sh_down.type, p->rbf};
+    bool hit;
+    qw_kernel **k = kernel_memo(p, base, key, &hit);
+    return hit ? *k : (*k = gg_kernel_new(p, base, M, nb));
+}
+static qw_kernel *gg_kernel_new(qw_path *p, const char *base, const qw_moe_layer *M, int nb) {
     const int part = !strcmp(base, "moe_sel_gg") || !strcmp(base, "gg_tab_init") ? 0 : !strcmp(base, "moe_pre_gg") ? 1 : !strcmp(base, "moe_gu_gg") ? 2
                      : !strcmp(base, "moe_dn_gg") || !strcmp(base, "moe_cmb_gg") ? 3 : 4;
     const int nbv = part == 4 ? nb : qw_path_nbv(nb);
@@ -204,15 +233,17 @@ static void bind_t(qw_batch *b, unsigned index, const qw_tensor *t) { qw_batch_b
 // defaults for its own kernels (src/engine.c:1295-1312) and mean nothing to this backend.
 static qw_kernel *gh_kernel(qw_path *p, const char *base, int nb) {
     char name[64], defs[768];
+    bool hit;
+    qw_kernel **k = kernel_memo(p, base, (const int[QW_MEMO_KEY]){nb}, &hit);
+    if (hit) return *k;
     snprintf(name, sizeof name, "%s_n%d_d%d", base, nb, p->D);
-    qw_kernel *k = qw_kernel_get(p->g, name);
-    if (k) return k;
+    if ((*k = qw_kernel_get(p->g, name))) return *k;
     snprintf(defs, sizeof defs,
              "#define ghc_down ghc_down_n%d_d%d\n#define ghc_up ghc_up_n%d_d%d\n#define ghc_dsk ghc_dsk_n%d_d%d\n#define ghc_mid ghc_mid_n%d_d%d\n"
              "#define ghc_upv ghc_upv_n%d_d%d\n#define D %d\n#define HC %d\n#define NB %d\n"
              "#define GH_R %d\n#define GH_G %d\n#define GU_SG %d\n#define GV_SG %d\n#define GV_RP %d\n#define GK %d\n",
              nb, p->D, nb, p->D, nb, p->D, nb, p->D, nb, p->D, p->D, QW_PATH_HC, nb, nb <= 4 ? 16 : 32, nb <= 2 ? 16 : 8, 8, 8, 10, 10);
-    return compile_get(p, name, defs);
+    return *k = compile_get(p, name, defs);
 }
 size_t qw_path_hyper_pd_bytes(int nb) { return (size_t)nb * (QW_PATH_HC * (QW_PATH_HC_LR + 2 * QW_PATH_HC) + QW_PATH_HC_LR + QW_PATH_HC) * 4; }
 
