@@ -1884,7 +1884,7 @@ __device__ __forceinline__ f4 dnc_tile(const qwk_dn_args &a, const u2 *lut, cons
 template <int F, int CH, int FSD, int CHSD>
 __device__ __forceinline__ void dnc_body(const qwk_dn_args &a, u2 *lut, float *part /* [QW_DNC_MAXNB][topk + 1][16] */, float *wl /* [QW_DNC_MAXNB][topk + 1] */, qw_sel_cache *sc) {
     const uint32_t K = a.topk, gnb = a.gnb, tpe = a.D / 16, tile = blockIdx.x, lane = qw_lane(), n = lane & 15, kg = lane >> 4, nwv = qw_threads() >> 6;
-    // The table through registers, asked for first and stored behind the record (published by the barrier of ready()): a
+    // The table through registers, asked for right behind the record and stored once that is there (published by the barrier of ready()): a
     // copy straight into LDS kept every wave in the issue of its loads for more than a microsecond, between the record and
     // the first weights (which need the record).
     constexpr bool TAB = qw_has_lut(F) || qw_has_lut(FSD);

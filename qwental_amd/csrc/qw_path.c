@@ -478,7 +478,7 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
     if (qw_hip_parts_ok(p->g)) {
         // All groups in one batch: one upload, one wait, the rows written to the host by each group's last launch. A group's time is
         // the device's from its first launch to the next group's, and its share of what the host adds once. (A batch a group, each waited for:
-        // 251 us for sixteen slots and 45 rows of the benchmark's layer, this 205.)
+        // 248 us for sixteen slots and 45 rows of the benchmark's layer, this 200.)
         double part[QW_PAR_MAX], sum = 0;
         const double t0 = qw_now();
         qw_batch *b = qw_batch_begin(p->g, false);
