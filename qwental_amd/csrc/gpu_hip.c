@@ -73,6 +73,8 @@ typedef struct qw_hbuf {
     struct qw_gpu *g;
     int npack, nwant; // packed copies made from this buffer (dropped when its contents change), and copies that are not due yet
     bool written;    // some dispatch has bound it in an output role
+    unsigned nwriters, nslots; // dispatches of the batch being submitted that write it, and launches that can write the shadow for them (count_writers)
+    bool apart;      // those several dispatches may all write the shadow themselves
     bool released;   // the device bytes were freed (qw_hip_buf_release_source): dptr is only the key of its tile-major copies
 } qw_hbuf;
 
@@ -2546,31 +2548,52 @@ static void touched_range(const qw_batch *b, int first, const qw_hbuf *h, bool o
 }
 
 static bool carried_back(const qw_use *u) { return u->out && !u->b->device_only && u->b->host && !u->b->wrapped && u->b->size <= QW_HIP_BIG_OUT_BYTES; }
-// After u's launch (last: the last one of b) the range of u's buffer that b carries back may be written to the shadow by
-// that launch alone: no other dispatch of b writes the buffer, or u comes last and writes all that they do; and what it
-// leaves alone of [u->lo, u->hi) is the same in the shadow and in HBM, because it went up with this segment.
-static bool direct_ok(const qw_batch *b, const qw_use *u, bool last) {
-    if (!carried_back(u) || !u->b->pinned) return false;
+// What u's launch leaves alone of [u->lo, u->hi) is the same in the shadow and in HBM: nothing, or it went up with this segment.
+static bool direct_ok(const qw_use *u) { return carried_back(u) && u->b->pinned && (u->whole || (u->b->size <= QW_HIP_SMALL_BYTES && u->b->pending_out == 1)); }
+// After u's launch, the last one of b, the range of u's buffer that b carries back may be written to the shadow by that launch alone:
+// it writes all that the other dispatches of b write there.
+static bool last_ok(const qw_batch *b, const qw_use *u) {
+    if (!direct_ok(u)) return false;
     for (int j = 0; j < b->nuse; j++) {
         const qw_use *o = &b->use[j];
-        if (o->out && o->b == u->b && o != u && !(last && u->whole && o->lo >= u->lo && o->hi <= u->hi)) return false;
+        if (o->out && o->b == u->b && o != u && !(u->whole && o->lo >= u->lo && o->hi <= u->hi)) return false;
     }
-    return u->whole || (u->b->size <= QW_HIP_SMALL_BYTES && u->b->pending_out == 1);
+    return true;
 }
-// The dispatches of b that write h write disjoint ranges of it whole, and every one can write the shadow too: then all do.
-static bool split_ok(const qw_batch *b, const qw_hbuf *h) {
-    int uses = 0, slots = 0;
+static int by_range(const void *x, const void *y) {
+    const qw_use *u = *(const qw_use *const *)x, *v = *(const qw_use *const *)y;
+    if (u->b != v->b) return (uintptr_t)u->b < (uintptr_t)v->b ? -1 : 1;
+    return u->lo < v->lo ? -1 : u->lo > v->lo;
+}
+// How many dispatches of b write each buffer, and where there are several, whether all of them may write the shadow (apart): they write
+// disjoint ranges of the buffer whole, by launches of this segment that can. Decided for all buffers at once by a sort: a look at every pair
+// of writers for every launch took the host 130 ms over 512 products into one buffer.
+static void count_writers(qw_batch *b) {
+    const unsigned mark = ++b->g->mark;
+    bool several = false;
     for (int j = 0; j < b->nuse; j++) {
         const qw_use *u = &b->use[j];
-        if (!u->out || u->b != h) continue;
-        if (!u->whole || !carried_back(u) || !h->pinned) return false;
-        for (int k = 0; k < j; k++)
-            if (b->use[k].out && b->use[k].b == h && b->use[k].lo < u->hi && b->use[k].hi > u->lo) return false;
-        uses++;
+        qw_hbuf *h = u->b;
+        if (!u->out) continue;
+        if (h->mark != mark) h->mark = mark, h->nwriters = h->nslots = 0, h->apart = true;
+        several |= ++h->nwriters > 1;
+        if (!u->whole || !carried_back(u) || !h->pinned) h->apart = false;
     }
+    if (!several) return;
     for (int i = b->done_l; i < b->nl; i++)
-        for (int d = 0; d < b->l[i].ndirect; d++) slots += b->use[b->l[i].direct_use[d]].b == h && !b->l[i].side;
-    return uses > 1 && uses == slots;
+        for (int d = 0; d < b->l[i].ndirect; d++) b->use[b->l[i].direct_use[d]].b->nslots += !b->l[i].side;
+    const qw_use **w = malloc(sizeof *w * (size_t)b->nuse);
+    int n = 0;
+    for (int j = 0; j < b->nuse; j++) {
+        const qw_use *u = &b->use[j];
+        if (!u->out || u->b->nwriters < 2 || !u->b->apart) continue;
+        if (!w || u->b->nslots != u->b->nwriters) u->b->apart = false;
+        else w[n++] = u;
+    }
+    if (n) qsort(w, (size_t)n, sizeof *w, by_range);
+    for (int i = 1; i < n; i++)
+        if (w[i]->b == w[i - 1]->b && w[i]->lo < w[i - 1]->hi) w[i]->b->apart = false;
+    free(w);
 }
 static void direct_set(qw_batch *b, qw_launch *l, int d) {
     qw_use *u = &b->use[l->direct_use[d]];
@@ -2585,12 +2608,13 @@ static void direct_set(qw_batch *b, qw_launch *l, int d) {
 static void host_outputs(qw_batch *b) {
     if (!b->io || b->uses_sync) return;
     bool side = false;
+    count_writers(b);
     for (int i = b->done_l; i < b->nl; i++) {
         qw_launch *l = &b->l[i];
         side = side || l->side;
         for (int d = 0; d < l->ndirect; d++) {
             const qw_use *u = &b->use[l->direct_use[d]];
-            if ((!l->back_at && direct_ok(b, u, false)) || (u->out && split_ok(b, u->b))) direct_set(b, l, d);
+            if (u->b->nwriters > 1 ? u->b->apart : !l->back_at && direct_ok(u)) direct_set(b, l, d);
         }
     }
     qw_launch *l = b->nl > b->done_l ? &b->l[b->nl - 1] : NULL;
@@ -2598,7 +2622,7 @@ static void host_outputs(qw_batch *b) {
     const unsigned mark = ++b->g->mark; // buffers that are seen to
     for (int d = 0; d < l->ndirect; d++) {
         const qw_use *u = &b->use[l->direct_use[d]];
-        if (carried_back(u) && !u->direct && !direct_ok(b, u, true)) return;
+        if (carried_back(u) && !u->direct && !last_ok(b, u)) return;
         u->b->mark = mark;
     }
     qwk_back back = {0};
