@@ -113,6 +113,7 @@ typedef struct {
     // qwk_fin and, if the kernel copies what others left (0: it does not), the qwk_back lie (host_outputs)
     int ndirect, direct_use[4];
     unsigned short direct_at[4], fin_at, back_at;
+    unsigned past; // bit d: the kernel stores the second place of output d past the caches, so that the launch need not be the one that ends the batch
 } qw_launch;
 
 // A buffer as a dispatch binds it, and the bytes it may touch. whole: every byte of [lo, hi) is written, whatever they held.
@@ -1225,6 +1226,7 @@ static bool launch_qmvs(qw_batch *b, qwk_qmvm_args *a, unsigned tiles) {
 static bool direct_slots(qw_batch *b, int n, const int *uses, size_t yh_at, size_t fin_at) {
     qw_launch *l = &b->l[b->nl - 1];
     l->ndirect = n;
+    l->past = ~0u; // (qw_store_y)
     l->fin_at = (unsigned short)fin_at;
     for (int j = 0; j < n; j++) l->direct_use[j] = uses[j], l->direct_at[j] = (unsigned short)(yh_at + (size_t)j * sizeof(void *));
     return true;
@@ -2009,6 +2011,7 @@ static bool tr_cmb(qw_batch *b) {
             const size_t at[3] = {offsetof(qwk_dn_args, Ph), offsetof(qwk_dn_args, outh), offsetof(qwk_dn_args, Pshh)};
             l->ndirect = d->Wsd ? 3 : 2; // (without a shared expert Psh is only read)
             for (int j = 0; j < l->ndirect; j++) l->direct_use[j] = uses[j], l->direct_at[j] = (unsigned short)at[j];
+            l->past = 1u << 1; // out alone (qw_store_host): Ph and Pshh are stored in the ordinary way, for the release at the end of the batch's last launch (qw_back_fin)
             l->fin_at = offsetof(qwk_dn_args, fin), l->back_at = offsetof(qwk_dn_args, back);
             return true;
         }
@@ -2566,7 +2569,7 @@ static int by_range(const void *x, const void *y) {
     return u->lo < v->lo ? -1 : u->lo > v->lo;
 }
 // How many dispatches of b write each buffer, and where there are several, whether all of them may write the shadow (apart): they write
-// disjoint ranges of the buffer whole, by launches of this segment that can. Decided for all buffers at once by a sort: a look at every pair
+// disjoint ranges of the buffer whole, by launches of this segment that can without ending the batch. Decided for all buffers at once by a sort: a look at every pair
 // of writers for every launch took the host 130 ms over 512 products into one buffer.
 static void count_writers(qw_batch *b) {
     const unsigned mark = ++b->g->mark;
@@ -2581,7 +2584,7 @@ static void count_writers(qw_batch *b) {
     }
     if (!several) return;
     for (int i = b->done_l; i < b->nl; i++)
-        for (int d = 0; d < b->l[i].ndirect; d++) b->use[b->l[i].direct_use[d]].b->nslots += !b->l[i].side;
+        for (int d = 0; d < b->l[i].ndirect; d++) b->use[b->l[i].direct_use[d]].b->nslots += !b->l[i].side && (b->l[i].past >> d & 1);
     const qw_use **w = malloc(sizeof *w * (size_t)b->nuse);
     int n = 0;
     for (int j = 0; j < b->nuse; j++) {

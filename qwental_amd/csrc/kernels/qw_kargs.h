@@ -150,8 +150,9 @@ typedef struct {
      * chosen when the kernel runs */
     uint32_t fd, fsd;
     uint32_t tpe_mul, upr_mul; /* QW_DIV_MUL of D / 16 and of I / 8 */
-    /* qwk_dnc_*, qwk_dnq_* as the last launch of a batch over host-visible buffers (fin.flag NULL: not): second places for
-     * P, Psh (NULL where the launch does not make it) and out, and what the launches before left */
+    /* qwk_dnc_*, qwk_dnq_* as the last launch of a batch over host-visible buffers (fin.flag NULL: not): second places for P and Psh
+     * (NULL where the launch does not make it), and what the launches before left. They are stored in the ordinary way, for the
+     * release in front of the flag. outh, the second place of out, is stored past the caches and may be given in any launch. */
     float *Ph, *Pshh;
     uint16_t *outh;
     qwk_fin fin;
