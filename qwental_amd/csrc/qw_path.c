@@ -27,6 +27,7 @@ struct qw_path {
     // dispatch were most of what recording a layer cost (24 layers, 72 launches: 108 us with the names and a search of all
     // tile-major copies, 30 without; all of a batch is recorded before its first launch goes out)
     struct { const char *base; int key[QW_MEMO_KEY]; qw_kernel *k; } memo[QW_MEMO];
+    unsigned memo_out; // which of its places a kernel takes where all are taken: each in turn
 };
 
 static int blk_values(int type) { // src/gguf.c:15-25
@@ -89,12 +90,15 @@ const qw_buf *qw_path_scratch(const qw_path *p, int which) { return which == 0 ?
 static qw_kernel **kernel_memo(qw_path *p, const char *base, const int *key, bool *hit) {
     uint32_t h = (uint32_t)((uintptr_t)base >> 2);
     for (int i = 0; i < QW_MEMO_KEY; i++) h = (h ^ (uint32_t)key[i]) * 0x9e3779b1u;
-    uint32_t at = h >> 26;
+    _Static_assert(QW_MEMO == 64, "the upper six bits of the hash");
+    const uint32_t first = h >> 26;
+    uint32_t at = QW_MEMO;
     for (uint32_t i = 0; i < QW_MEMO_WAYS; i++) { // (any of a few places, so that two kernels of a layer do not keep putting each other out)
-        const uint32_t j = (at + i) % QW_MEMO;
+        const uint32_t j = (first + i) % QW_MEMO;
         if (p->memo[j].k && p->memo[j].base == base && !memcmp(p->memo[j].key, key, sizeof p->memo[j].key)) return *hit = true, &p->memo[j].k;
+        if (!p->memo[j].k && at == QW_MEMO) at = j;
     }
-    for (uint32_t i = 0; i < QW_MEMO_WAYS && p->memo[at].k; i++) at = (at + 1) % QW_MEMO; // all taken: the one behind them goes
+    if (at == QW_MEMO) at = (first + p->memo_out++ % QW_MEMO_WAYS) % QW_MEMO; // (one of those that are looked at)
     p->memo[at].base = base, p->memo[at].k = NULL;
     memcpy(p->memo[at].key, key, sizeof p->memo[at].key);
     return *hit = false, &p->memo[at].k;
@@ -345,6 +349,7 @@ static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, co
         return false;
     }
     qw_kernel *k;
+    const int nbv = qw_path_nbv(nb); // what these kernels are built for: one of five counts, and one place each in the table of kernels
     if (!p->tab_ready) { // first use: build the lookup tables in the same batch, before they are needed
         if (!(k = gg_kernel(p, "gg_tab_init", M, 1))) return false;
         qw_batch_kernel(b, k);
@@ -355,14 +360,14 @@ static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, co
     const uint32_t nbr = (uint32_t)nb;
     const unsigned E = (unsigned)p->E, I = (unsigned)p->I, D = (unsigned)p->D, K = (unsigned)p->topk;
     if (given) { // the selection from the caller's logits (src/engine.c:609-614)
-        if (!(k = gg_kernel(p, "moe_sel_gg", M, nb))) return false;
+        if (!(k = gg_kernel(p, "moe_sel_gg", M, nbv))) return false;
         qw_batch_kernel(b, k);
         qw_batch_buf(b, 0, lg, 0);
         qw_batch_buf(b, 1, sel, 0);
         qw_batch_bytes(b, 2, &nbr, 4);
         qw_batch_dispatch(b, 1, 1, 1, 1024, 1, 1);
     }
-    if (!(k = gg_kernel(p, "moe_pre_gg", M, nb))) return false;
+    if (!(k = gg_kernel(p, "moe_pre_gg", M, nbv))) return false;
     qw_batch_kernel(b, k);
     bind_t(b, 0, &M->router);
     bind_t(b, 1, &M->sh_gate_w);
@@ -381,7 +386,7 @@ static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, co
     qw_batch_bytes(b, 14, &nbr, 4);
     qw_batch_dispatch(b, (E + 1 + 7) / 8 + I / 8, 1, 1, 256, 1, 1);
 
-    if (!(k = gg_kernel(p, "moe_gu_gg", M, nb))) return false;
+    if (!(k = gg_kernel(p, "moe_gu_gg", M, nbv))) return false;
     qw_batch_kernel(b, k);
     bind_t(b, 0, &M->gate);
     bind_t(b, 1, &M->up);
@@ -399,7 +404,7 @@ static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, co
         qw_batch_dispatch(b, a > c ? a : c, nbr * K + 1, 1, 256, 1, 1);
     }
 
-    if (!(k = gg_kernel(p, "moe_dn_gg", M, nb))) return false;
+    if (!(k = gg_kernel(p, "moe_dn_gg", M, nbv))) return false;
     qw_batch_kernel(b, k);
     bind_t(b, 0, &M->down);
     qw_batch_buf(b, 2, &p->H, 0);
@@ -408,7 +413,7 @@ static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, co
     qw_batch_buf(b, 9, &p->pd, 0);
     qw_batch_dispatch(b, D / 16, nbr * K, 1, 128, 1, 1);
 
-    if (!(k = gg_kernel(p, "moe_cmb_gg", M, nb))) return false;
+    if (!(k = gg_kernel(p, "moe_cmb_gg", M, nbv))) return false;
     qw_batch_kernel(b, k);
     qw_batch_buf(b, 1, &p->psh, 0);
     qw_batch_buf(b, 3, sel, 0);
