@@ -32,6 +32,12 @@ void qw_par_free(qw_par *p);
 void qw_par_observe(qw_par *p, int b, double ms);
 /* The table entry of size b: the running average, 0 when not measured yet. */
 double qw_par_group_cost(const qw_par *p, int b);
+/* What a step took beside its groups, whose times are then the device's alone: upload, recording, submission and wait come once
+ * a step, however many groups it has. Averaged as the groups' times are, and added once to the estimate of a step; the cut does not
+ * depend on it. For whoever runs the groups of a step in one batch (qw_path_par_vstep); never called, it is 0: a group's
+ * time holds all that the group brought. */
+void qw_par_observe_step(qw_par *p, double ms);
+double qw_par_step_cost(const qw_par *p);
 /* Estimated ms of a step of B rows (B above QW_PAR_MAX counts as QW_PAR_MAX); 0 when nothing was measured or B < 1. */
 double qw_par_cost(const qw_par *p, int B);
 /* Group sizes for B rows (1 .. QW_PAR_MAX) into groups[], from the back as the reference emits them; returns their

@@ -7,6 +7,8 @@
 struct qw_par {
     double cost[QW_PAR_VBMAX + 1];
     int seen[QW_PAR_VBMAX + 1];
+    double step; // once a step, whatever its groups
+    int step_seen;
     double pcost[NBUCKET + 1]; // bucket k: rows 16 (k - 1) + 1 .. 16 k
     int pseen[NBUCKET + 1];
 };
@@ -21,6 +23,10 @@ static void observe(double *cost, int *seen, double ms) {
 void qw_par_observe(qw_par *p, int b, double ms) {
     if (b >= 1 && b <= QW_PAR_VBMAX && ms > 0) observe(&p->cost[b], &p->seen[b], ms);
 }
+void qw_par_observe_step(qw_par *p, double ms) {
+    if (ms > 0) observe(&p->step, &p->step_seen, ms);
+}
+double qw_par_step_cost(const qw_par *p) { return p->step; }
 double qw_par_group_cost(const qw_par *p, int b) { return b >= 1 && b <= QW_PAR_VBMAX ? p->cost[b] : 0; }
 
 // Sizes never measured, filled in on the line through the smallest and the largest measured size (one size: flat).
@@ -70,7 +76,7 @@ double qw_par_cost(const qw_par *p, int B) { // the estimate: sizes never measur
     if (!fill_line(p->cost, QW_PAR_VBMAX, c)) return 0;
     if (B > QW_PAR_MAX) B = QW_PAR_MAX;
     cover(c, B, cheapest, last);
-    return cheapest[B];
+    return cheapest[B] + p->step;
 }
 
 int qw_par_split(const qw_par *p, int B, int *g) { // the cut: a size never measured costs 0, so that it gets tried

@@ -456,7 +456,8 @@ bool qw_path_hyper_moe_stack(qw_path *p, qw_batch *b, const qw_hyper_w *H, const
 // Slot i brings n[i] rows; its first row is r0[i] = n[0] + ... + n[i - 1] (src/engine.c:9150-9161). The R rows are cut
 // into groups by the measured table (qw_par_split: the reference's par_split with groups of up to 16 rows), the
 // groups go through the layer one after the other (the reference's par_step, src/engine.c:8805-8812, each reading
-// the weights once), and each group's time goes back into the table (src/engine.c:9037).
+// the weights once), and each group's time goes back into the table (src/engine.c:9037): the device's alone, which does not depend on how many
+// groups the step has. What the host adds comes once a step, and goes back as that.
 bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int *n, int B, const qw_buf *x, const qw_buf *out, qw_vstep_info *info) {
     if (!p || !par || !M || !n || !x || !out || B < 1 || B > QW_PAR_MAX) return false;
     int R = 0, r0[QW_PAR_MAX];
@@ -482,7 +483,7 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
     double gpu = 0, wall = 0;
     if (qw_hip_parts_ok(p->g)) {
         // All groups in one batch: one upload, one wait, the rows written to the host by each group's last launch. A group's time is
-        // the device's from its first launch to the next group's, and its share of what the host adds once. (A batch a group, each waited for:
+        // the device's from its first launch to the next group's. (A batch a group, each waited for:
         // 248 us for sixteen slots and 45 rows of the benchmark's layer, this 200.)
         double part[QW_PAR_MAX], sum = 0;
         const double t0 = qw_now();
@@ -499,7 +500,8 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
         bool stamped = true;
         for (int gi = 0; gi < ng; gi++) stamped = stamped && part[gi] > 0;
         for (int gi = 0; gi < ng; gi++) sum += part[gi] = stamped ? part[gi] * 1e3 : gpu * grp[gi] / R; // (a front launch without a stamp: by rows)
-        for (int gi = 0; gi < ng; gi++) qw_par_observe(par, grp[gi], part[gi] + (wall > sum ? wall - sum : 0) / ng);
+        for (int gi = 0; gi < ng; gi++) qw_par_observe(par, grp[gi], part[gi]);
+        qw_par_observe_step(par, wall - sum);
         if (info) info->gpu_ms = gpu, info->wall_ms = wall;
         return true;
     }
@@ -510,10 +512,10 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
         const bool rec = gg_moe_at(p, b, M, grp[gi], x, (size_t)c * (size_t)p->D * 2, &p->vlg, &p->vsel, out, (size_t)c * (size_t)p->D * 2, false);
         const double t = qw_batch_end(b);
         if (!rec || t < 0) return false;
-        const double ms = (qw_now() - t0) * 1e3;
-        qw_par_observe(par, grp[gi], ms);
-        gpu += t * 1e3, wall += ms;
+        qw_par_observe(par, grp[gi], t * 1e3);
+        gpu += t * 1e3, wall += (qw_now() - t0) * 1e3;
     }
+    qw_par_observe_step(par, wall - gpu);
     if (info) info->gpu_ms = gpu, info->wall_ms = wall;
     return true;
 }

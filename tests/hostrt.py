@@ -11,13 +11,26 @@ PRELUDE = r"""
 #include "gpu_hip.c"
 #include "qw_path.c"
 static qw_ioslot io_slots[QW_IO_SLOTS];
+static uint64_t device_clock = 1; // ten ticks a launch
 static uint32_t io_counts[QW_IO_SLOTS * (4 + QW_FIN_BYTES) / 4];
 static void on_launch(const char *fname, unsigned gx, unsigned bx, const void *args);
 hipError_t hipModuleGetFunction(hipFunction_t *f, hipModule_t m, const char *name) { return (void)m, *f = (hipFunction_t)strdup(name), hipSuccess; }
 hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned by, unsigned bz, unsigned lds, hipStream_t st, void **params, void **extra) {
     (void)gy, (void)gz, (void)by, (void)bz, (void)lds, (void)st, (void)extra;
     on_launch((const char *)f, gx, bx, params[0]);
-    for (int i = 0; i < QW_IO_SLOTS; i++) io_slots[i].t0[0] = 1, io_slots[i].t1[0] = 2, io_slots[i].done = io_slots[i].copied = 1;
+    const bool io = !strcmp((const char *)f, "qwk_io");
+    const qwk_io_args *a = params[0];
+    const size_t at = start_of((const char *)f);
+    uint64_t *started = NULL;
+    if (at) memcpy(&started, (const char *)params[0] + at, sizeof started);
+    if (io) started = a->t_enter;
+    if (started) *started = device_clock;
+    device_clock += 10;
+    if (io && a->t_done) *a->t_done = device_clock;
+    for (int i = 0; i < QW_IO_SLOTS; i++) {
+        io_slots[i].done = io_slots[i].copied = 1;
+        if (!io) io_slots[i].t1[0] = device_clock;
+    }
     return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t st) { return (void)st, hipSuccess; }
@@ -36,7 +49,7 @@ static qw_gpu *device(void) { // what qw_gpu_open sets up, without tile-major co
     static char tabs[QW_TAB_BYTES];
     qw_gpu *g = calloc(1, sizeof *g);
     g->kernels = calloc(QW_MAX_KERNELS, sizeof *g->kernels);
-    g->ncu = 256, g->tick = 1, g->tabs = tabs, g->io = io_slots, g->io_count = io_counts, g->total_mem = (size_t)1 << 38;
+    g->ncu = 256, g->tick = 1e-9, g->tabs = tabs, g->io = io_slots, g->io_count = io_counts, g->total_mem = (size_t)1 << 38;
     g->io_func = find_func(g, "qwk_io");
     read_switches(g);
     return g;

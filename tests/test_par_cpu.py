@@ -7,6 +7,7 @@ import itertools
 import numpy as np
 import pytest
 
+import hostrt
 import qwental_amd as q
 
 
@@ -139,6 +140,26 @@ def test_groups_or_packing_path():
     p.free()
 
 
+def test_what_comes_once_a_step():
+    """It is averaged as the groups are, comes once to a step's estimate whatever its groups, and leaves the cut alone."""
+    p = q.Par()
+    for b in range(1, 17):
+        feed(p, b, [36 + 2.6 * b])
+    feed(p, 40, [220.0], packed=True)
+    before, cuts = {B: p.cost(B) for B in range(1, 65)}, {B: p.split(B) for B in range(1, 65)}
+    assert p.step_cost() == 0 and before[40] == pytest.approx(212.0) and p.choose(40)[0] is False
+    p.observe_step(1e6)                  # the first sample is dropped
+    p.observe_step(-1.0)
+    assert p.step_cost() == 0 and p.cost(40) == before[40]
+    p.observe_step(20.0)
+    p.observe_step(30.0)
+    assert p.step_cost() == pytest.approx(0.9 * 20.0 + 0.1 * 30.0)
+    for B in before:
+        assert p.cost(B) == pytest.approx(before[B] + 21.0) and p.split(B) == cuts[B]
+    assert p.group_cost(16) == 36 + 2.6 * 16 and p.choose(40)[0]  # 233 against 220
+    p.free()
+
+
 def test_time_slices_or_a_joint_step():
     """qw_par_want_slice, the rule of the reference's tools/serve.c:1715-1729: the trivial counts, the figures it falls
     back on, and the five per cent either way before the mode changes."""
@@ -170,3 +191,36 @@ def test_time_slices_or_a_joint_step():
     assert p.want_slice(2, True, sliced_rate=191.0) and not p.want_slice(2, True, sliced_rate=189.0)
     assert p.want_slice(3, False, sliced_rate=3e3 / p.cost(3) * 1.06) and not p.want_slice(3, False, sliced_rate=3e3 / p.cost(3) * 1.04)
     p.free()
+
+
+# A step of 16 rows as one group, two and four, on a device clock of ten nanoseconds a launch
+VSTEP = r"""
+static void on_launch(const char *fname, unsigned gx, unsigned bx, const void *args) { (void)fname, (void)gx, (void)bx, (void)args; }
+int main(void) {
+    qw_gpu *g = device();
+    qw_path *p = qw_path_open(g, 1024, 256, 64, 4, 16, true);
+    qw_buf w, x, out;
+    if (!qw_hip_buf_new_device(g, (size_t)64 * 1024 * 256 * 2, &w) || !qw_buf_new(g, 64 * 2048, &x) || !qw_buf_new(g, 64 * 2048, &out)) return printf("no buffers\n"), 1;
+    const qw_tensor W = {.buf = &w, .type = 8}, R = {.buf = &w, .type = 1};
+    const qw_moe_layer M = {.router = R, .sh_gate_w = R, .gate = W, .up = W, .down = W, .sh_gate = W, .sh_up = W, .sh_down = W};
+    qw_vstep_info info;
+    const int n = 16;
+    for (int size = 16; size >= 4; size /= 2) {
+        qw_par *par = qw_par_new();
+        for (int b = 1; b <= 16; b++) // a table whose cheapest cut is into groups of that size, and the first sample of none is to come
+            for (int i = 0; i < 2; i++) qw_par_observe(par, b, b == size ? 1e-9 : 50);
+        for (int step = 0; step < 400; step++) // what the table began with has gone after 400 samples
+            if (!qw_path_par_vstep(p, par, &M, &n, 1, &x, &out, &info) || info.ngroups != n / size) return printf("%d groups: %s\n", info.ngroups, g->err), 1;
+        printf("%.6g %.6g %.6g\n", qw_par_group_cost(par, size), qw_par_step_cost(par), info.wall_ms);
+        qw_par_free(par);
+    }
+    return 0;
+}
+"""
+
+
+def test_a_groups_time_does_not_depend_on_how_many_groups_its_step_has(tmp_path):
+    rows = [list(map(float, line.split())) for line in hostrt.run(tmp_path, VSTEP).splitlines()]
+    launches = {16: 4, 8: 4, 4: 4}  # front, gate/up, down and combine: 40 ns a group
+    for (cost, step, wall), n in zip(rows, launches.values()):
+        assert cost == pytest.approx(n * 1e-5, rel=1e-3) and 0 < step < 100 * wall
