@@ -188,6 +188,39 @@ struct qw_batch {
     qw_switches sw; // the device's switches when the batch began (no_fuse also set for what must not wait for its workgroups)
 };
 
+// Threads of a workgroup that the kernels whose names begin with `name` are compiled for, or take from a number in their argument record
+// (at `at`, divided by div; both 0: any size). The first rule that fits counts; a kernel without one reads its size.
+typedef struct { const char *name; unsigned threads; unsigned short at, div; } qw_wg_rule;
+static const qw_wg_rule wg_rules[] = {
+    {"qwk_qmvs_", 0, offsetof(qwk_qmvm_args, K), 4}, // a wave per 256 values
+    {"qwk_qmvm_swiglu", 0, offsetof(qwk_pre_args, r.D), 4},
+    {"qwk_pre_", 0, offsetof(qwk_pre_args, r.D), 4},
+    {"qwk_hc_down_", 0, offsetof(qwk_hc_args, D), 8}, // a thread per eight columns
+    {"qwk_qmvm", QW_WG_QMVM, 0, 0},
+    {"qwk_qmv_", QW_WG_GU, 0, 0},
+    {"qwk_gu_", QW_WG_GU, 0, 0},
+    {"qwk_gud_", QW_WG_GU, 0, 0},
+    {"qwk_pfr_", QW_WG_GU, 0, 0},
+    {"qwk_dnr_", QW_WG_DN, 0, 0},
+    {"qwk_dnc_", QW_WG_DN, 0, 0},
+    {"qwk_dnq_", QW_WG_DN, 0, 0},
+    {"qwk_dn_", QW_WG, 0, 0},
+    {"qwk_pf_", QW_WG, 0, 0},
+    {"qwk_pfg_", QW_WG_PFG, 0, 0},
+    {"qwk_select", QW_WG_SELECT, 0, 0},
+    {"qwk_cmb", QW_WG_CMB, 0, 0},
+    {"qwk_moe_prep_slices", QW_WG_PREP_SLICES, 0, 0},
+    {"qwk_moe_prep", QW_WG_PREP, 0, 0},
+    {"qwk_hc_up", QW_WG_HC_UP, 0, 0},
+};
+static const qw_wg_rule *wg_rule(const char *fname) {
+    static const qw_wg_rule any = {"", 0, 0, 0};
+    for (size_t i = 0; i < sizeof wg_rules / sizeof *wg_rules; i++)
+        if (!strncmp(fname, wg_rules[i].name, strlen(wg_rules[i].name))) return &wg_rules[i];
+    return &any;
+}
+typedef struct { char name[48]; hipFunction_t f; const qw_wg_rule *wg; } qw_func;
+
 #define QW_LD_MAX 16
 struct qw_gpu {
     int dev;
@@ -200,7 +233,7 @@ struct qw_gpu {
     int cur_stream;
     struct qw_kernel *kernels;
     int nkernels;
-    struct { char name[48]; hipFunction_t f; } funcs[QW_MAX_FUNCS];
+    qw_func funcs[QW_MAX_FUNCS];
     int nfuncs;
     char err[1024];
     bool prof;
@@ -464,15 +497,16 @@ const char *qw_hip_last_error(const qw_gpu *g) { return g->err; }
 int qw_hip_cu_count(const qw_gpu *g) { return g->ncu; }
 const char *qw_hip_arch(void) { return "gfx950"; }
 
-static hipFunction_t get_func(qw_gpu *g, const char *fname) {
+static const qw_func *get_func(qw_gpu *g, const char *fname) {
     for (int i = 0; i < g->nfuncs; i++)
-        if (!strcmp(g->funcs[i].name, fname)) return g->funcs[i].f;
+        if (!strcmp(g->funcs[i].name, fname)) return &g->funcs[i];
     if (g->nfuncs >= QW_MAX_FUNCS) return NULL;
     hipFunction_t f = find_func(g, fname);
     if (!f) { set_err(g, "no entry point %s in the code objects", fname); return NULL; }
     snprintf(g->funcs[g->nfuncs].name, sizeof g->funcs[0].name, "%s", fname);
     g->funcs[g->nfuncs].f = f;
-    return g->funcs[g->nfuncs++].f;
+    g->funcs[g->nfuncs].wg = wg_rule(fname);
+    return &g->funcs[g->nfuncs++];
 }
 
 // ---------------------------------------------------------------- define block -> kernels
@@ -1114,9 +1148,12 @@ static size_t start_of(const char *fname) {
 
 static bool add_launch(qw_batch *b, const char *fname, unsigned gx, unsigned bx, const void *args, size_t argsz) {
     if (argsz > QW_MAX_ARGS) return fail(b, "%s: argument record of %zu bytes", fname, argsz);
-    hipFunction_t f = get_func(b->g, fname);
+    const qw_func *f = get_func(b->g, fname);
     if (!f) return fail(b, "%s: entry point %s missing from the code object", b->k->name, fname);
     if (gx == 0) return true; // nothing to do
+    uint32_t threads = f->wg->threads;
+    if (f->wg->div) memcpy(&threads, (const char *)args + f->wg->at, sizeof threads), threads /= f->wg->div;
+    if (threads && threads != bx) return fail(b, "%s: %s launched with %u threads a workgroup, made for %u", b->k->name, fname, bx, threads);
     if (b->nl == b->capl) {
         if (b->noalloc) return fail(b, "%s: more than %d launches in the fixed recorder", b->k->name, b->capl);
         b->capl = b->capl ? 2 * b->capl : 64;
@@ -1124,7 +1161,7 @@ static bool add_launch(qw_batch *b, const char *fname, unsigned gx, unsigned bx,
     }
     qw_launch *l = &b->l[b->nl++];
     memset(l, 0, sizeof *l);
-    l->f = f;
+    l->f = f->f;
     l->fname = fname;
     l->gx = gx; l->gy = 1; l->gz = 1; l->bx = bx;
     memcpy(l->args, args, argsz);
@@ -1140,7 +1177,7 @@ static unsigned cdiv(unsigned a, unsigned b) { return (a + b - 1) / b; }
 // work is smaller. tasks are per-wave units; 8 waves per workgroup.
 static unsigned persistent_grid(const qw_gpu *g, unsigned wave_tasks, unsigned waves) { return umin((unsigned)g->ncu, cdiv(wave_tasks, waves)); }
 // waves per workgroup: gate/up + matvec kernels, front / any-shape down kernels, down range kernels
-enum { QW_WAVES_GU = 12, QW_WAVES_DN = 8, QW_WAVES_DNR = 12 }; // (the routed gate/up launch with 8 or 10 waves a workgroup: 2 % slower at 16 tokens)
+enum { QW_WAVES_GU = QW_WG_GU / 64, QW_WAVES_DN = QW_WG / 64, QW_WAVES_DNR = QW_WG_DN / 64 }; // (the routed gate/up launch with 8 or 10 waves a workgroup: 2 % slower at 16 tokens)
 
 static const char *fname_fmt(char *buf, size_t n, const char *fmt, ...) {
     va_list ap;
@@ -1251,7 +1288,7 @@ static bool launch_qmvm(qw_batch *b, qwk_qmvm_args *a, qw_hbuf *const *hw) {
     if (!tiles) return true;
     if (hw && qmvs_fits(b->g, a, tiles, false)) return launch_qmvs(b, a, tiles);
     // few tiles: cut every tile's K range over several waves, as far as the wave slots of the device and K allow
-    const unsigned waves = QW_WAVES_GU, slots = (unsigned)b->g->ncu * waves;
+    const unsigned waves = QW_WG_QMVM / 64, slots = (unsigned)b->g->ncu * waves;
     a->split = a->K % 256 == 0 ? pick_split(a->K / 256, tiles, slots) : 1;
     if (a->split > 1) {
         unsigned groups = 0;
@@ -1342,11 +1379,11 @@ static bool tr_qmv(qw_batch *b) { // src/engine.c:717-723: 0 W, 3 x, 4 y, 5 {N, 
         const unsigned cpr = (unsigned)p->K / ((unsigned)fmt_qb(base) * (unsigned)ch), slots = (unsigned)b->g->ncu * QW_WAVES_GU;
         a.split = pick_split(cpr, a.ntiles, slots);
         if (a.split > 1)
-            return add_launch(b, intern(fn), umin((unsigned)b->g->ncu, cdiv(a.ntiles, QW_WAVES_GU / a.split)), 64 * QW_WAVES_GU, &a, sizeof a) &&
+            return add_launch(b, intern(fn), umin((unsigned)b->g->ncu, cdiv(a.ntiles, QW_WAVES_GU / a.split)), QW_WG_GU, &a, sizeof a) &&
                    (!direct || direct_slots(b, 1, &use, offsetof(qwk_qmv_args, yh), offsetof(qwk_qmv_args, fin)));
     }
     a.split = 1;
-    return add_launch(b, intern(fn), persistent_grid(b->g, a.ntiles, QW_WAVES_GU), 64 * QW_WAVES_GU, &a, sizeof a) &&
+    return add_launch(b, intern(fn), persistent_grid(b->g, a.ntiles, QW_WAVES_GU), QW_WG_GU, &a, sizeof a) &&
            (!direct || p->valu || direct_slots(b, 1, &use, offsetof(qwk_qmv_args, yh), offsetof(qwk_qmv_args, fin)));
 }
 
@@ -1364,13 +1401,13 @@ static bool fill_select(qw_batch *b, qwk_select_args *a, unsigned ilg, unsigned 
 }
 static bool launch_select(qw_batch *b, unsigned ilg, unsigned isel, uint32_t nbr) {
     qwk_select_args a;
-    return fill_select(b, &a, ilg, isel, nbr) && add_launch(b, "qwk_select", 1, 1024, &a, sizeof a);
+    return fill_select(b, &a, ilg, isel, nbr) && add_launch(b, "qwk_select", 1, QW_WG_SELECT, &a, sizeof a);
 }
 // The selection that a moe_pre_gg dispatch left pending and no gate/up dispatch took over: a launch of its own.
 static bool flush_select(qw_batch *b) {
     if (!b->pend_sel.valid) return true;
     b->pend_sel.valid = false;
-    return add_launch(b, "qwk_select", 1, 1024, &b->pend_sel.a, sizeof b->pend_sel.a);
+    return add_launch(b, "qwk_select", 1, QW_WG_SELECT, &b->pend_sel.a, sizeof b->pend_sel.a);
 }
 
 static bool nbr_ok(qw_batch *b, uint32_t nbr) {
@@ -1467,7 +1504,7 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
             if (hipMemcpyAsync(hs[i]->dptr, hs[i]->host, hs[i]->size, hipMemcpyHostToDevice, g->stream[b->stream]) != hipSuccess) return NULL;
             hs[i]->dirty = false;
         }
-    hipFunction_t f = get_func(g, pack_of(fmt).fname);
+    const qw_func *f = get_func(g, pack_of(fmt).fname);
     if (!f) return NULL;
     void *dst;
     if (hipMalloc(&dst, bytes) != hipSuccess) {
@@ -1479,7 +1516,7 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
     void *params[] = {&pa};
     const uint64_t nslab = ntiles * nblk;
     const unsigned gx = (unsigned)(nslab / 4 < 65536 ? (nslab + 3) / 4 : 65536);
-    if (hipModuleLaunchKernel(f, gx, 1, 1, 256, 1, 1, 0, g->stream[b->stream], params, NULL) != hipSuccess || hipStreamSynchronize(g->stream[b->stream]) != hipSuccess) {
+    if (hipModuleLaunchKernel(f->f, gx, 1, 1, 256, 1, 1, 0, g->stream[b->stream], params, NULL) != hipSuccess || hipStreamSynchronize(g->stream[b->stream]) != hipSuccess) {
         (void)hipFree(dst);
         return NULL;
     }
@@ -1731,7 +1768,7 @@ static bool tr_gu(qw_batch *b) {
         b->pend_gu.fname = intern(fn), b->pend_gu.kname = b->k->name, b->pend_gu.grid = grid;
         return true;
     }
-    return add_launch(b, intern(fn), grid, 64 * QW_WAVES_GU, &a, sizeof a);
+    return add_launch(b, intern(fn), grid, QW_WG_GU, &a, sizeof a);
 }
 
 // The gate/up launch that waited for a down dispatch to join it, on its own after all.
@@ -1739,7 +1776,7 @@ static bool flush_gu(qw_batch *b) {
     if (!b->pend_gu.valid) return true;
     b->pend_gu.valid = false;
     const int first = b->nl;
-    if (!add_launch(b, b->pend_gu.fname, b->pend_gu.grid, 64 * QW_WAVES_GU, &b->pend_gu.a, sizeof b->pend_gu.a)) return false;
+    if (!add_launch(b, b->pend_gu.fname, b->pend_gu.grid, QW_WG_GU, &b->pend_gu.a, sizeof b->pend_gu.a)) return false;
     if (b->nl > first) b->l[b->nl - 1].kname = b->pend_gu.kname, b->l[b->nl - 1].last_of_dispatch = true;
     return true;
 }
@@ -1756,7 +1793,7 @@ static bool flush_dn(qw_batch *b) {
     b->pend_dn.valid = false;
     const int first = b->nl;
     const qwk_dn_args *a = b->pend_dn.plain.Wd ? &b->pend_dn.plain : &b->pend_dn.a;
-    if (!add_launch(b, b->pend_dn.fname, b->pend_dn.grid, 64 * QW_WAVES_DNR, a, sizeof *a)) return false;
+    if (!add_launch(b, b->pend_dn.fname, b->pend_dn.grid, QW_WG_DN, a, sizeof *a)) return false;
     if (b->nl > first) b->l[b->nl - 1].kname = b->pend_dn.kname, b->l[b->nl - 1].last_of_dispatch = true;
     return true;
 }
@@ -1871,7 +1908,7 @@ static bool tr_dn_inner(qw_batch *b) {
         // One token: wait for the combine, the two run as one launch (Q6_K rows of 256: 12.7 us against 12.4 + 6.1; of 512: 18.6
         // against 13.2 + 6.2 and the gap between two launches). From two on its waves, which read H from memory step by
         // step, take longer than both (31.4 against 13.6 + 6.4, rows of 256 20.0 against 12.4 + 6.2).
-        if (nbr > 1 || !b->sw.dnc_nb) return add_launch(b, intern(fn), grid, 64 * QW_WAVES_DNR, &a, sizeof a);
+        if (nbr > 1 || !b->sw.dnc_nb) return add_launch(b, intern(fn), grid, QW_WG_DN, &a, sizeof a);
         char fu[48];
         fname_fmt(fu, sizeof fu, "qwk_dnc_f%d_c1%s", fd, tail);
         b->pend_dn.valid = true;
@@ -1882,7 +1919,7 @@ static bool tr_dn_inner(qw_batch *b) {
     if (kq_d || kq_s || ((fd == 20 || fs == 20) && (fd != 20 || (fs != 0 && fs != 20 && fs != 8)))) {
         if (rel) return fail(b, "%s: the GGUF-order bytes of the weights were released and no tile-major copy serves this dispatch", b->k->name);
         a.fd = (uint32_t)fd, a.fsd = (uint32_t)fs;
-        return add_launch(b, "qwk_dn_rt", persistent_grid(b->g, umax * (unsigned)(p->D / 16) + (unsigned)p->D / 16, QW_WAVES_DN), 64 * QW_WAVES_DN, &a, sizeof a);
+        return add_launch(b, "qwk_dn_rt", persistent_grid(b->g, umax * (unsigned)(p->D / 16) + (unsigned)p->D / 16, QW_WAVES_DN), QW_WG, &a, sizeof a);
     }
     if (fd == 21 && p->I <= 512) {
         const uint32_t nblk = (uint32_t)p->I / 256, tileb = nblk * QW_SLAB_BYTES;
@@ -1918,14 +1955,14 @@ static bool tr_dn_inner(qw_batch *b) {
                     b->pend_dn.fname = intern(fn), b->pend_dn.fused = intern(fu), b->pend_dn.kname = b->k->name, b->pend_dn.grid = grid, b->pend_dn.fused_grid = (unsigned)p->D / 16, b->pend_dn.quarters = false;
                     return true;
                 }
-                return add_launch(b, intern(fn), grid, 64 * QW_WAVES_DNR, &a, sizeof a);
+                return add_launch(b, intern(fn), grid, QW_WG_DN, &a, sizeof a);
             }
         }
         if (rel) return fail(b, "%s: the GGUF-order bytes of the weights were released and no tile-major copy serves this dispatch", b->k->name);
         const int ch = p->I % 320 == 0 && !b->sw.nl_c4 ? 10 : 4; // blocks per chunk
         if (fs) fname_fmt(fn, sizeof fn, "qwk_dnr_f20_c%d_s%d_c%d", ch, fs, fs == 20 ? ch : 4);
         else fname_fmt(fn, sizeof fn, "qwk_dnr_f20_c%d", ch);
-        return add_launch(b, intern(fn), persistent_grid(b->g, umax * (unsigned)(p->D / 16) + (unsigned)p->D / 16, QW_WAVES_DNR), 64 * QW_WAVES_DNR, &a, sizeof a);
+        return add_launch(b, intern(fn), persistent_grid(b->g, umax * (unsigned)(p->D / 16) + (unsigned)p->D / 16, QW_WAVES_DNR), QW_WG_DN, &a, sizeof a);
     }
     if (fd != 20 && p->I <= 512 && p->I % 256 == 0) { // contiguous task ranges per workgroup, operand A staged in LDS
         const int ch = fd == 8 ? 4 : p->I / 256;
@@ -1959,12 +1996,12 @@ static bool tr_dn_inner(qw_batch *b) {
             b->pend_dn.fname = intern(fn), b->pend_dn.fused = intern(fu), b->pend_dn.kname = b->k->name, b->pend_dn.grid = grid, b->pend_dn.fused_grid = tpe / tpw * nq, b->pend_dn.quarters = true;
             return true;
         }
-        return add_launch(b, intern(fn), grid, 64 * QW_WAVES_DNR, &a, sizeof a);
+        return add_launch(b, intern(fn), grid, QW_WG_DN, &a, sizeof a);
     }
     // wider rows: one tile at a time, operand A from global memory
     fname_fmt(fn, sizeof fn, "qwk_dn_f%d_any%s", p->fd, sfx);
     if (rel && fd != QW_F_PACKED) return fail(b, "%s: the GGUF-order bytes of the weights were released and no tile-major copy serves this dispatch", b->k->name);
-    return add_launch(b, intern(fn), persistent_grid(b->g, umax * (unsigned)(p->D / 16) + (unsigned)p->D / 16, QW_WAVES_DN), 64 * QW_WAVES_DN, &a, sizeof a);
+    return add_launch(b, intern(fn), persistent_grid(b->g, umax * (unsigned)(p->D / 16) + (unsigned)p->D / 16, QW_WAVES_DN), QW_WG, &a, sizeof a);
 }
 
 // src/engine.c:640-646: 1 Psh, 3 sel, 4 out, 8 nbr, 9 Pg
@@ -1997,7 +2034,7 @@ static bool tr_cmb(qw_batch *b) {
                     char fu[48];
                     fname_fmt(fu, sizeof fu, "qwk_gud%s", b->pend_dn.fused + 7); // the same formats as the qwk_dnq_* launch
                     b->uses_sync = true;
-                    return add_launch(b, intern(fu), grid, 64 * QW_WAVES_GU, &f, sizeof f);
+                    return add_launch(b, intern(fu), grid, QW_WG_GU, &f, sizeof f);
                 }
             }
             if (!flush_gu(b)) return false;
@@ -2005,7 +2042,7 @@ static bool tr_cmb(qw_batch *b) {
                 d->nq = dnq_quarters(nbr), d->tpw = d->nq > 2 ? 2 : 1;
                 b->pend_dn.fused_grid = a.D / 16 / d->tpw * d->nq;
             }
-            if (!add_launch(b, b->pend_dn.fused, b->pend_dn.fused_grid, 64 * QW_WAVES_DNR, d, sizeof *d)) return false;
+            if (!add_launch(b, b->pend_dn.fused, b->pend_dn.fused_grid, QW_WG_DN, d, sizeof *d)) return false;
             qw_launch *l = &b->l[b->nl - 1];
             const int uses[3] = {b->pend_dn.use_p, b->nuse - 1, b->pend_sd.use};
             const size_t at[3] = {offsetof(qwk_dn_args, Ph), offsetof(qwk_dn_args, outh), offsetof(qwk_dn_args, Pshh)};
@@ -2018,7 +2055,7 @@ static bool tr_cmb(qw_batch *b) {
         if (!flush_gu(b) || !flush_dn(b)) return false;
     }
     if (!flush_gu(b)) return false;
-    if (!add_launch(b, "qwk_cmb", cdiv((unsigned)p->D, 256), 256, &a, sizeof a)) return false;
+    if (!add_launch(b, "qwk_cmb", cdiv((unsigned)p->D, QW_WG_CMB), QW_WG_CMB, &a, sizeof a)) return false;
     b->l[b->nl - 1].gy = nbr;
     return true;
 }
@@ -2090,9 +2127,9 @@ static bool tr_pk_scatter(qw_batch *b, unsigned gx) { // 0 X, 1 ids, 2 cursor, 3
                                  .P = a.P, .E = a.E, .topk = a.topk, .KD = a.KD, .tm = pl->tm, .max_tiles = pl->max_tiles,
                                  .slice = 1};
         b->pend_pk.stage = 0;
-        if (a.P <= QW_PREP_ONE) return add_launch(b, "qwk_moe_prep", a.P, 256, &f, sizeof f);
+        if (a.P <= QW_PREP_ONE) return add_launch(b, "qwk_moe_prep", a.P, QW_WG_PREP, &f, sizeof f);
         f.slice = umin(cdiv(a.P, 2 * (unsigned)b->g->ncu), QW_PREP_SLICE);
-        return add_launch(b, "qwk_moe_prep_slices", cdiv(a.P, f.slice), 512, &f, sizeof f);
+        return add_launch(b, "qwk_moe_prep_slices", cdiv(a.P, f.slice), QW_WG_PREP_SLICES, &f, sizeof f);
     }
     if (!flush_pk(b)) return false;
     return add_launch(b, "qwk_moe_scatter", gx, 256, &a, sizeof a);
@@ -2154,7 +2191,7 @@ static bool launch_pf(qw_batch *b, qwk_pf_args *a, int F, int E, qw_hbuf *hw, qw
         const uint8_t *pk = get_pack(b, QW_F_PACKED_NL, hw, a->W, NULL, NULL, (uint64_t)E * (a->N / 16), nch, a->rowbytes);
         if (pk) {
             a->W = pk, a->rowbytes = nch * QW_NL_CHUNK_BYTES;
-            return add_launch(b, "qwk_pfg_f120", (unsigned)b->g->ncu, 512, a, sizeof *a);
+            return add_launch(b, "qwk_pfg_f120", (unsigned)b->g->ncu, QW_WG_PFG, a, sizeof *a);
         }
     }
     if (F == 21 && a->K % 256 == 0) {
@@ -2163,13 +2200,13 @@ static bool launch_pf(qw_batch *b, qwk_pf_args *a, int F, int E, qw_hbuf *hw, qw
         const uint8_t *pk = get_pack(b, QW_F_PACKED, hw, a->W, wb ? hwb : NULL, wb, ntiles, nblk, a->rowbytes);
         if (pk) {
             a->W = pk, a->rowbytes = nblk * QW_SLAB_BYTES, a->split = split, a->ntn = a->N / split;
-            if (blocked && several) return add_launch(b, "qwk_pfg_f121", (unsigned)b->g->ncu, 512, a, sizeof *a);
+            if (blocked && several) return add_launch(b, "qwk_pfg_f121", (unsigned)b->g->ncu, QW_WG_PFG, a, sizeof *a);
             if (a->tm <= 16 && a->K <= 2560) { // entries of one group of rows: the rows are staged in LDS per workgroup range
                 fname_fmt(fn, sizeof fn, "qwk_pfr_f121_c%d", a->K % 512 == 0 ? 2 : 1);
-                return add_launch(b, intern(fn), umin((unsigned)b->g->ncu, a->max_tiles * a->ntn), 64 * QW_WAVES_GU, a, sizeof *a);
+                return add_launch(b, intern(fn), umin((unsigned)b->g->ncu, a->max_tiles * a->ntn), QW_WG_GU, a, sizeof *a);
             }
             fname_fmt(fn, sizeof fn, "qwk_pf_f121_c%d", a->K % 512 == 0 ? 2 : 1);
-            return add_launch(b, intern(fn), persistent_grid(b->g, a->max_tiles * a->ntn, 8), 512, a, sizeof *a);
+            return add_launch(b, intern(fn), persistent_grid(b->g, a->max_tiles * a->ntn, QW_WAVES_DN), QW_WG, a, sizeof *a);
         }
         if (wb) return false; // the caller launches the two matrices one by one
     }
@@ -2177,7 +2214,7 @@ static bool launch_pf(qw_batch *b, qwk_pf_args *a, int F, int E, qw_hbuf *hw, qw
     if (F == 21) fname_fmt(fn, sizeof fn, "qwk_pf_f21_c%d", a->K % 512 == 0 ? 2 : 1);
     else fname_fmt(fn, sizeof fn, "qwk_pf_f%d_c4", F == 20 ? 20 : 8);
     // every entry can hold a tile: the grid covers the whole table, the kernel counts the entries in use
-    return add_launch(b, intern(fn), persistent_grid(b->g, a->max_tiles * a->ntn, 8), 512, a, sizeof *a);
+    return add_launch(b, intern(fn), persistent_grid(b->g, a->max_tiles * a->ntn, QW_WAVES_DN), QW_WG, a, sizeof *a);
 }
 
 static bool flush_pf(qw_batch *b) {
@@ -2303,7 +2340,7 @@ static bool tr_hc(qw_batch *b) {
         if (a.want_inj && !bind_whole(b, 7, nb * QW_HC * QW_HC * 4, "new inject sums", (void **)&a.injo)) return false;
     } else if (!bind_ptr(b, 5, nb * QW_HC_LR * 4, false, "sx", (void **)&a.sx) || !bind_ptr(b, 6, nb * QW_HC * 4, false, "rs", (void **)&a.rs) ||
                !bind_whole(b, 7, nb * D * 2, "x", (void **)&a.x)) return false;
-    if (!add_launch(b, f == FAM_HC_UP ? "qwk_hc_up" : "qwk_hc_upv", (unsigned)(D / 8), 256, &a, sizeof a)) return false;
+    if (!add_launch(b, f == FAM_HC_UP ? "qwk_hc_up" : "qwk_hc_upv", (unsigned)(D / 8), QW_WG_HC_UP, &a, sizeof a)) return false;
     b->l[b->nl - 1].gy = (unsigned)(nb + QW_HC_TG - 1) / QW_HC_TG; // tokens four at a time
     return true;
 }

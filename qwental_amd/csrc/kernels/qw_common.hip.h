@@ -38,8 +38,8 @@ typedef u2 __attribute__((aligned(2))) u2a2;
 // comparing the workgroup's index with their number, through the vector memory - a round trip that most kernels waited for before
 // they asked for anything else. No launch here has such a workgroup; this is a scalar load beside the arguments'.)
 __device__ __forceinline__ uint32_t qw_threads() { return __builtin_amdgcn_workgroup_size_x(); }
-// The same known when the kernel is compiled (the host launches it with n threads): no load at all. It lies behind the
-// arguments, in a line of memory of its own that nothing else of the launch has touched yet.
+// The same known when the kernel is compiled (the host launches it with n threads and refuses to record another size, wg_rules): no load at
+// all. It lies behind the arguments, in a line of memory of its own that nothing else of the launch has touched yet.
 #define QW_THREADS(n) __builtin_assume(__builtin_amdgcn_workgroup_size_x() == (n))
 
 // Loads above it are issued above it. (The scheduler saves registers in a short kernel by moving each load to its use: a round trip each.)

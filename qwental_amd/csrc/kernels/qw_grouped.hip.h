@@ -28,7 +28,7 @@
 #include "qw_kquants.hip.h"
 
 #define QW_PFG_TW 2u            /* weight tiles of a wave */
-#define QW_PFG_WAVES 8u
+#define QW_PFG_WAVES (QW_WG_PFG / 64)
 #define QW_PFG_TB (QW_PFG_TW * QW_PFG_WAVES) /* tiles of a task */
 #define QW_PFG_ROWS 64u
 #define QW_PFG_OS 264u          /* halves between rows of the result tile in LDS (256 + 8: rows start at different banks) */

@@ -3,6 +3,18 @@
 #pragma once
 #include <stdint.h>
 
+/* Threads of a workgroup, where a kernel is compiled for one size and the host has to launch it with that (wg_rules in gpu_hip.c) */
+#define QW_WG 512u             /* any-shape down, grouped products in GGUF order: 8 waves */
+#define QW_WG_DN 768u          /* down range kernels, down + combine: 12 waves */
+#define QW_WG_GU 768u          /* gate/up and dense matvec: 12 waves, three per SIMD (a wave issues at most one instruction in ~6 cycles) */
+#define QW_WG_QMVM 768u        /* 12 waves: a tile's K range is cut over 1, 2 or 4 of them */
+#define QW_WG_SELECT 1024u
+#define QW_WG_PREP 256u
+#define QW_WG_PREP_SLICES 512u
+#define QW_WG_PFG 512u         /* blocked grouped product: 8 waves */
+#define QW_WG_HC_UP 256u       /* eight output columns, 32 lanes each */
+#define QW_WG_CMB 256u
+
 /* Selection record written by the select kernel and read by gate/up, down and combine. For gnb == 8 and
  * topk == 10 this is byte for byte the reference's struct gg_sel (kernels/moe_gg.metal:110-116), 1636 bytes;
  * gnb == 16 is the wide layout for up to 16 token columns (4548 bytes with topk == 10). GU = gnb * topk.

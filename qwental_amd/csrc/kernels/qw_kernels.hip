@@ -56,9 +56,6 @@ __shared__ uint32_t qw_sst[12 * 16];
 #define QW_WG_END_STAMP(k) do {} while (0)
 #endif
 
-#define QW_WG 512          // threads per workgroup of the down and front kernels (8 waves)
-#define QW_WG_DN 768       // down range kernels: 12 waves
-#define QW_WG_GU 768       // gate/up and dense matvec: 12 waves, three per SIMD (a wave issues at most one instruction in ~6 cycles)
 #define QW_XF_MAXK 2560    // largest K whose activations are staged in LDS in fragment order (K * 32 bytes)
 
 // wave index in the workgroup, as a scalar (so that task indices and row bases stay in scalar registers)
@@ -454,7 +451,6 @@ QW_QMVS(1) QW_QMVS(2) QW_QMVS(4) QW_QMVS(8)
 // split > 1 (few tiles: the projections of one decode step): the K range of a tile is cut into split parts, one per
 // wave, so that a row is one memory round trip instead of a chain of them; the waves of a tile sit in one workgroup
 // and their partial sums are added in part order through LDS (the same order whatever else the launch holds).
-#define QW_WG_QMVM 768 // 12 waves: a tile's K range is cut over 1, 2 or 4 of them
 template <int F, int NB> struct qmvm_tile {
     typedef qw_chunk_kq<F, NB> C;
     const qwk_qmvm_args &a;
@@ -1024,8 +1020,8 @@ __device__ __forceinline__ void select_all(const qwk_select_args &a, qw_sel_scra
 }
 
 #if QW_IN_PART(0)
-extern "C" __global__ __launch_bounds__(1024) void qwk_select(qwk_select_args a) {
-    QW_THREADS(1024);
+extern "C" __global__ __launch_bounds__(QW_WG_SELECT) void qwk_select(qwk_select_args a) {
+    QW_THREADS(QW_WG_SELECT);
     __shared__ qw_sel_scratch s;
     __shared__ qw_sel_cache c;
     __shared__ float lgs[16 * 1024];
@@ -2589,7 +2585,8 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_scatter(qwk_scatter_ar
 // product and the combine do not care about). Workgroup 0 also leaves counts, offsets, cursors (where the scatter
 // would have left them) and the tile table.
 #if QW_IN_PART(5)
-extern "C" __global__ __launch_bounds__(256) void qwk_moe_prep(qwk_prep_args a) {
+extern "C" __global__ __launch_bounds__(QW_WG_PREP) void qwk_moe_prep(qwk_prep_args a) {
+    QW_THREADS(QW_WG_PREP);
     __shared__ uint32_t cnt[1024], red[4], wr[4], wt[4];
     qw_started(a.t_start);
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, p = blockIdx.x;
@@ -2660,8 +2657,8 @@ extern "C" __global__ __launch_bounds__(256) void qwk_moe_prep(qwk_prep_args a) 
 // only stores follow the scan (read for every pair, five loads one after the other a wave): 28.5 -> 24.6 at 20480 pairs, whose 84 MB
 // of stores are 16 at the rate of a large copy.
 #if QW_IN_PART(5)
-extern "C" __global__ __launch_bounds__(512) void qwk_moe_prep_slices(qwk_prep_args a) {
-    QW_THREADS(512);
+extern "C" __global__ __launch_bounds__(QW_WG_PREP_SLICES) void qwk_moe_prep_slices(qwk_prep_args a) {
+    QW_THREADS(QW_WG_PREP_SLICES);
     __shared__ uint32_t cnt[1024], at[1024], wr[8], wt[8], id[QW_PREP_SLICE], pos[QW_PREP_SLICE];
     qw_started(a.t_start);
     const uint32_t tid = threadIdx.x, nth = qw_threads(), lane = tid & 63, wave = tid >> 6, nwv = nth >> 6;
@@ -2883,13 +2880,13 @@ QW_PF(121, 2, qwk_pf_f121_c2) QW_PF(121, 1, qwk_pf_f121_c1) // tile-major IQ3_S:
 #endif
 
 #if QW_IN_PART(5)
-extern "C" __global__ __launch_bounds__(64 * QW_PFG_WAVES) void qwk_pfg_f121(qwk_pf_args a) {
-    QW_THREADS(64 * QW_PFG_WAVES);
+extern "C" __global__ __launch_bounds__(QW_WG_PFG) void qwk_pfg_f121(qwk_pf_args a) {
+    QW_THREADS(QW_WG_PFG);
     __shared__ qw_pfg_lds<QW_F_PACKED> L;
     pfg_body<QW_F_PACKED>(a, L);
 }
-extern "C" __global__ __launch_bounds__(64 * QW_PFG_WAVES) void qwk_pfg_f120(qwk_pf_args a) {
-    QW_THREADS(64 * QW_PFG_WAVES);
+extern "C" __global__ __launch_bounds__(QW_WG_PFG) void qwk_pfg_f120(qwk_pf_args a) {
+    QW_THREADS(QW_WG_PFG);
     __shared__ qw_pfg_lds<QW_F_PACKED_NL> L;
     pfg_body<QW_F_PACKED_NL>(a, L);
 }
@@ -2962,8 +2959,9 @@ QW_PFR(2, qwk_pfr_f121_c2) QW_PFR(1, qwk_pfr_f121_c1)
 // ================================================================ combine (kernels/moe_gg.metal:655-663)
 // Rank order, then the shared expert. One thread per (token, row).
 #if QW_IN_PART(5)
-extern "C" __global__ __launch_bounds__(256) void qwk_cmb(qwk_cmb_args a) { // grid: 256 rows, tokens
-    const uint32_t t = blockIdx.y, row = blockIdx.x * 256 + threadIdx.x, K = a.topk;
+extern "C" __global__ __launch_bounds__(QW_WG_CMB) void qwk_cmb(qwk_cmb_args a) { // grid: 256 rows, tokens
+    QW_THREADS(QW_WG_CMB);
+    const uint32_t t = blockIdx.y, row = blockIdx.x * QW_WG_CMB + threadIdx.x, K = a.topk;
     if (row >= a.D) return;
     const float *w = (const float *)(a.sel + QW_SEL_OFF_W(a.gnb, K)) + t * (K + 1);
     // Everything in one round trip, without conditions (past topk the last one again): the weights by scalar loads - a workgroup has one token.
@@ -3299,8 +3297,8 @@ template <bool GIVEN> __device__ __forceinline__ void hc_up_body(const qwk_hc_ar
     QW_HSTAMP(13);
 }
 #if QW_IN_PART(5)
-extern "C" __global__ __launch_bounds__(256) void qwk_hc_up(qwk_hc_args a) { QW_THREADS(256); hc_up_body<false>(a); }
-extern "C" __global__ __launch_bounds__(256) void qwk_hc_upv(qwk_hc_args a) { QW_THREADS(256); hc_up_body<true>(a); }
+extern "C" __global__ __launch_bounds__(QW_WG_HC_UP) void qwk_hc_up(qwk_hc_args a) { QW_THREADS(QW_WG_HC_UP); hc_up_body<false>(a); }
+extern "C" __global__ __launch_bounds__(QW_WG_HC_UP) void qwk_hc_upv(qwk_hc_args a) { QW_THREADS(QW_WG_HC_UP); hc_up_body<true>(a); }
 #endif
 
 // Read pattern of a decode layer without the decoding (kernels/moe_bw.metal:7-26): workgroup (x, c) reads slice x
