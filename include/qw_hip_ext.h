@@ -132,6 +132,8 @@ unsigned qw_hip_graph_launches(const qw_gpu *g);
  * goes to stderr as it is set) and QW_HIP_QUIET (qw_batch_wait prints none). QW_HIP_REPACK=0 and QW_HIP_GRAPH=1 are
  * read by qw_gpu_open() only (see above); afterwards qw_hip_set_repack / qw_hip_set_graphs change them. */
 void qw_hip_reload_switches(qw_gpu *g);
+/* Whether the host can write the device's memory itself (small uploads then need no launch), and how many bytes it has uploaded so. */
+bool qw_hip_host_uploads(const qw_gpu *g, size_t *bytes);
 /* The device's synchronisation words (the first 384 are the barrier's: all zero between launches except word 0, the
  * generation; word 352 is the error word), copied to dst after a device synchronisation. For tests. */
 bool qw_hip_sync_words(qw_gpu *g, uint32_t *dst, size_t nwords);

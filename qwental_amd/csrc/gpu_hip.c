@@ -278,6 +278,7 @@ struct qw_gpu {
     uint32_t *io_count;  // device, zero: a word per slot for qwk_io, behind them QW_FIN_BYTES per slot for the launches that end a batch themselves
     hipFunction_t io_func;
     bool host_up;        // the host can write HBM itself (the whole of it lies in the PCIe window): host_write
+    size_t host_up_bytes;
     int in_flight;       // batches that have launched something and have not been waited for
     double tick;         // seconds of the device clock's unit
     bool repack;         // make packed copies (QW_HIP_REPACK=0 in the environment or qw_hip_set_repack turn it off)
@@ -875,6 +876,7 @@ size_t qw_hip_copy_budget(const qw_gpu *g, size_t *used) {
     return g->copy_budget;
 }
 unsigned qw_hip_graph_launches(const qw_gpu *g) { return g->ngraph_launches; }
+bool qw_hip_host_uploads(const qw_gpu *g, size_t *bytes) { return *bytes = g->host_up_bytes, g->host_up; }
 void qw_hip_set_graphs(qw_gpu *g, bool on) { g->use_graphs = on; }
 size_t qw_hip_packed_bytes(const qw_gpu *g) { return g->pack_bytes; }
 // Before HBM is looked at from outside a batch: what the host wrote beyond the range of the last upload. (While outputs of h
@@ -2764,6 +2766,7 @@ static bool submit_segment(qw_batch *b, bool last) {
     if (back) {
         __builtin_ia32_sfence();
         (void)*back;
+        g->host_up_bytes += written;
     }
     if (!b->nseg) g->in_flight++;
     for (int k = 1; k < b->nparts && b->io && !b->nseg; k++) { // (part 0 starts with the batch)
