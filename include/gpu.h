@@ -68,8 +68,10 @@ bool qw_buf_wrap(qw_gpu *g, void *ptr, size_t len, qw_buf *out);
  * Bindings are sticky across dispatches, indices 0..31; inline bytes are limited to 256 per index.
  * dispatch takes the grid in threadgroups, as the reference does. barrier is a no-op on an in-order stream.
  * flush submits what is recorded so far and keeps recording. end = submit + wait. wait returns the GPU execution
- * time in seconds (HIP events around the batch's kernels; host<->device copies are outside it), negative on any
- * failure (unknown kernel, missing or undersized binding, HIP error), and frees the batch. */
+ * time in seconds, negative on any failure (unknown kernel, missing or undersized binding, HIP error), and frees the
+ * batch. The time is the device clock's, from the start of the batch's first kernel to the end of its last: uploads
+ * before and copies to the host behind them are outside it, results that the last kernels store to the host themselves
+ * are inside. Profiled batches, and those beyond 32 at once, take HIP events around their kernels instead. */
 qw_batch *qw_batch_begin(qw_gpu *g, bool concurrent);
 void qw_batch_kernel(qw_batch *b, qw_kernel *k);
 void qw_batch_buf(qw_batch *b, unsigned index, const qw_buf *buf, size_t offset);

@@ -2965,7 +2965,8 @@ extern "C" __global__ __launch_bounds__(QW_WG_CMB) void qwk_cmb(qwk_cmb_args a) 
     if (row >= a.D) return;
     const float *w = (const float *)(a.sel + QW_SEL_OFF_W(a.gnb, K)) + t * (K + 1);
     // Everything in one round trip, without conditions (past topk the last one again): the weights by scalar loads - a workgroup has one token.
-    // (With a condition a load, or moved to their uses, they were up to sixteen round trips. IQ4_NL layers at eight tokens 778 -> 748 us over twelve.)
+    // (With a condition a load, or moved to their uses, they were up to sixteen round trips; of D = 2560 rows at eight tokens a launch takes
+    // 4.7 us with its gap either way, which is the launch.)
     float pg[16], wv[16];
     const float wk = w[K], ps = a.Psh[(size_t)t * a.D + row];
 #pragma unroll
