@@ -484,7 +484,7 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
     if (qw_hip_parts_ok(p->g)) {
         // All groups in one batch: one upload, one wait, the rows written to the host by each group's last launch. A group's time is
         // the device's from its first launch to the next group's. (A batch a group, each waited for:
-        // 248 us for sixteen slots and 45 rows of the benchmark's layer, this 200.)
+        // 232.9 us for sixteen slots and 45 rows of the benchmark's layer, this 207.9.)
         double part[QW_PAR_MAX], sum = 0;
         const double t0 = qw_now();
         qw_batch *b = qw_batch_begin(p->g, false);
