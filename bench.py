@@ -3,7 +3,7 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--layers 48] [--nb 16]
 
-Workload (BASELINE.json configs[4]): the 48-layer MoE FFN stack decode step at B = 16 — hidden 2048, 512 experts of
+Workload: the 48-layer MoE FFN stack decode step at B = 16 — hidden 2048, 512 experts of
 gate/up 2 x (512 x 2048) and down 2048 x 512 in IQ3_S plus one shared expert per layer, top-10 routing by each
 layer's own binary16 router on x ~ N(0, 1), every 4th layer's shared-expert projections in Q8_0; about 33 GB of
 weights resident in HBM, generated on the device (seeded). One step = one pass of the stack over one batch of 16
@@ -67,7 +67,7 @@ def model_shape_leg(gpu, layers, steps, warmup, cpu_check):
         per.setdefault(name, []).append(us)
     res["kernel_us_mean"] = {k: float(np.mean(v)) for k, v in per.items()}
     if cpu_check:
-        from oracle import oracle as o  # the checker of the CPU baseline leg
+        from oracle import oracle as o  # what the CPU baseline leg compares with
         # one 16-token step of the first layer alone: `out` is the last layer's otherwise
         stack.step(x, 16, nlayers=1)
         lg = stack.lg[0].read(dtype=np.float32)[:16 * (stack.E + 1)].reshape(16, stack.E + 1).copy()
@@ -228,7 +228,7 @@ def hyper_ffn_leg(gpu, stack, steps, warmup):
 
 
 def ragged_steps(gpu, stack, reps=5):
-    """a continuous-batching step of one layer (layer 0 of the stack): 16 slots with seeded
+    """A continuous-batching step of one layer (layer 0 of the stack): 16 slots with seeded
     uniform row counts in 1..16 redrawn until the total is near the target, Zipf(1.1) routing forced through the
     logits. Timed two ways on the same rows: the decode path in groups of at most 16 rows (one batch), and the packing
     path (count -> prefix sums -> scatter -> grouped product -> combine) in one pass. Routed experts' bytes are read
@@ -299,7 +299,7 @@ def ragged_steps(gpu, stack, reps=5):
 
 
 def qmv_table(gpu, reps=5, nmat=64):
-    """BASELINE.json configs[0..1]: y = W x for a 4096 x 2048 matrix, IQ3_S and Q8_0, 1..16 activations. nmat matrices
+    """y = W x for a 4096 x 2048 matrix, IQ3_S and Q8_0, 1..16 activations. nmat matrices
     at different addresses go into one batch so that no cache holds the weights (the method of bench/moe_bw.c:50-89);
     the figure is GPU time per matrix. For IQ3_S and up to 4 activations the VALU GEMV form is timed beside the
     matrix-core form."""
@@ -573,9 +573,9 @@ def main():
             "launches": n_l, "mean_launch_us": mean_s * 1e6, "algorithmic_bytes_per_launch": gu_bytes}
     line = {"metric": "batched IQ3_S MoE decode tokens/s at B=16 (48-layer FFN stack); achieved HBM GB/s", "value": res[nb]["tokens_per_s"], "unit": "tokens/s",
             "n_gpus": 1, "steps": a.steps, "warmup": a.warmup, "ms_per_step": res[nb]["ms_per_step"], "higher_is_better": True, "scaling": "weak",
-            "vs_baseline": None, "dtype": "u8 blocks -> f16 matrix-core operands, f32 accumulate", "data": "synthetic (seeded, generated on device); block scales d drawn as BASELINE states them times %g (synth.MOE_D_SCALE: the stated |N(0, 0.02)| "
-                    "overflows the binary16 layer output; bytes and work are unchanged)" % synth.MOE_D_SCALE,
-            "config": {"workload": "configs[4]: %d-layer MoE FFN stack decode, B=%d, D=2048 I=512 E=512 top-10, IQ3_S experts, shared expert Q8_0 every 4th layer; "
+            "vs_baseline": None, "dtype": "u8 blocks -> f16 matrix-core operands, f32 accumulate", "data": "synthetic (seeded, generated on device); block scales d drawn as |N(0, 0.02)| times %g (synth.MOE_D_SCALE: without it a layer "
+                    "overflows its binary16 output; bytes and work are unchanged)" % synth.MOE_D_SCALE,
+            "config": {"workload": "%d-layer MoE FFN stack decode, B=%d, D=2048 I=512 E=512 top-10, IQ3_S experts, shared expert Q8_0 every 4th layer; "
                                    "every layer reads the same x and overwrites one out, launched in order on one stream (a bandwidth bench: no overlap between layers is used)" % (stack.L, nb),
                        "resident_weight_bytes": int(stack.weight_bytes), "packed_copy_bytes": int(gpu.L.qw_hip_packed_bytes(gpu.g)), "released_source_bytes": released, "device": gpu.name()},
             "roofline": roof,

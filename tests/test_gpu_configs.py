@@ -32,7 +32,7 @@ def layer_logits(stack, l, nb):
 
 
 def test_config2_one_layer_eight_tokens(gpu, oracle, stack8):
-    """one MoE decode layer, B = 8, 512 experts, binary16 router, top-10 softmax gating, SwiGLU."""
+    """One MoE decode layer, B = 8, 512 experts, binary16 router, top-10 softmax gating, SwiGLU."""
     nb = 8
     xh = synth.activations(np.random.default_rng(8), nb, D)
     x = gpu.buf_from(xh, device_only=True)
@@ -56,7 +56,7 @@ def test_config2_one_layer_eight_tokens(gpu, oracle, stack8):
 
 
 def test_config4_every_layer_of_the_mixed_stack(gpu, oracle, stack8):
-    """BASELINE configs[4] over 8 consecutive layers at B = 16 (layers 3 and 7 carry their shared expert in Q8_0):
+    """The stack over 8 consecutive layers at B = 16 (layers 3 and 7 carry their shared expert in Q8_0):
     the stack call with l + 1 layers leaves layer l's output, which is compared with the oracle for every l; the top-k
     of every layer is the oracle's."""
     nb = 16
@@ -81,7 +81,7 @@ def test_config4_every_layer_of_the_mixed_stack(gpu, oracle, stack8):
 
 
 def test_config4_all_48_layers_at_full_size(gpu, oracle):
-    """BASELINE configs[4] at its full size: the 48-layer stack (about 33 GB resident, every fourth layer's shared expert in
+    """The 48-layer stack (about 33 GB resident, every fourth layer's shared expert in
     Q8_0) at B = 16, every one of the 48 layers against the float32 oracle on the layer's own resident bytes, top-k
     identical everywhere. (The benchmark's CPU leg makes the same comparison on the layers its time budget reaches.)"""
     from qwental_amd.stack import MoeStack
@@ -107,7 +107,7 @@ def test_config4_all_48_layers_at_full_size(gpu, oracle):
 
 
 def test_config3_continuous_batching_step(gpu, oracle, stack8):
-    """BASELINE configs[3]: 16 slots with seeded row counts in 1..16 (64 rows), Zipf(1.1) routing forced through the
+    """16 slots with seeded row counts in 1..16 (64 rows), Zipf(1.1) routing forced through the
     logits. The rows go through the decode path in groups of 16 (every group against the float64 layer) and through
     the packing path in one pass: counts, offsets, tile table and packed positions bit-exact against the oracle, the
     routed sums against a float64 recompute per row."""

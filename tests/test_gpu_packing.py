@@ -118,7 +118,7 @@ def test_packing_all_pairs_one_expert(gpu, oracle):
 
 
 def test_ragged_step_decode_groups_equal_packing_path(gpu, oracle):
-    """A continuous-batching step in small (BASELINE configs[3] shape: 16 slots, n[i] ~ U{1..16} rows each, Zipf(1.1)
+    """A continuous-batching step in small (16 slots, n[i] ~ U{1..16} rows each, Zipf(1.1)
     routing forced through the logits): the decode path in groups of at most 16 rows and the packing path in one pass
     give the same routed sums. The shared expert's block scales are zero here, so that the decode path's output is
     the routed part alone."""
