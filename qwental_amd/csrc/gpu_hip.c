@@ -113,6 +113,10 @@ typedef struct {
     // qwk_fin and, if the kernel copies what others left (0: it does not), the qwk_back lie (host_outputs)
     int ndirect, direct_use[4];
     unsigned short direct_at[4], fin_at, back_at;
+    // Launches of one kernel in neighbouring parts of a batch that go out as one (join_parts): the first holds how many and which, the others are
+    // launched with it.
+    int nj, jl[QW_JOIN_MAX];
+    bool joined;
     unsigned past; // bit d: the kernel stores the second place of output d past the caches, so that the launch need not be the one that ends the batch
 } qw_launch;
 
@@ -158,6 +162,7 @@ struct qw_batch {
     bool events;
     bool fin;            // the last launch raises the flag itself
     int nparts, part_l[QW_PARTS_MAX]; // qw_hip_batch_part: the first launch of every part
+    int part_join;       // parts that come in sets of so many whose parts touch nothing of each other's (0: not known)
     double *part_s;      // where the seconds of the parts go (qw_hip_batch_end_parts)
     hipEvent_t *pev;      // profiling: 2 events per launch
     int npev;
@@ -497,6 +502,19 @@ size_t qw_gpu_max_working_set(const qw_gpu *g) { return g->total_mem; }
 const char *qw_hip_last_error(const qw_gpu *g) { return g->err; }
 int qw_hip_cu_count(const qw_gpu *g) { return g->ncu; }
 const char *qw_hip_arch(void) { return "gfx950"; }
+
+// Kernels that have a form for several launches in one (name + "_j"): what the layers of a ragged step are made of
+static const char *const joinable[] = {
+    "qwk_pre_w1_s121", "qwk_pre_w1_s8", "qwk_pre_w1_kq", "qwk_pre_w30_s121", "qwk_pre_w30_s8", "qwk_pre_w30_kq",
+    "qwk_gu_f121_c2", "qwk_gu_f8_c16", "qwk_gu_f108_c2", "qwk_gu_f112_c2", "qwk_gu_rt",
+    "qwk_dnq_f121_c2_s121_c2", "qwk_dnq_f121_c2_s8_c4", "qwk_dnq_f121_c1_s121_c1", "qwk_dnq_f121_c1_s8_c4", "qwk_dnq_f108_c1_s108_c1", "qwk_dnq_f114_c1_s114_c1",
+    "qwk_dnr_f120_c10_s120_c10", "qwk_cmb",
+};
+static bool can_join(const char *fname) {
+    for (size_t i = 0; i < sizeof joinable / sizeof *joinable; i++)
+        if (!strcmp(fname, joinable[i])) return true;
+    return false;
+}
 
 static const qw_func *get_func(qw_gpu *g, const char *fname) {
     for (int i = 0; i < g->nfuncs; i++)
@@ -1134,6 +1152,8 @@ static bool bind_bytes(qw_batch *b, unsigned index, void *dst, size_t len, const
     return true;
 }
 
+_Static_assert(sizeof(qwk_gu_join) == QW_JOIN_MAX * (sizeof(qwk_gu_args) + 4) && sizeof(qwk_dn_join) == QW_JOIN_MAX * (sizeof(qwk_dn_args) + 4) && sizeof(qwk_pre_join) == QW_JOIN_MAX * (sizeof(qwk_pre_args) + 4) &&
+               sizeof(qwk_cmb_join) == QW_JOIN_MAX * (sizeof(qwk_cmb_args) + 4), "records, then grids");
 _Static_assert(sizeof(qwk_pre_args) <= QW_MAX_ARGS && sizeof(qwk_gu_args) <= QW_MAX_ARGS && sizeof(qwk_dn_args) <= QW_MAX_ARGS && sizeof(qwk_qmv_args) <= QW_MAX_ARGS && sizeof(qwk_qmvm_args) <= QW_MAX_ARGS && sizeof(qwk_gud_args) <= QW_MAX_ARGS,
                "a kernel argument record is larger than the launch record's copy of it");
 
@@ -2453,7 +2473,7 @@ static int graph_run(qw_batch *b, hipStream_t st) {
     qw_gpu *g = b->g;
     if (!g->use_graphs || b->prof || b->done_l != 0 || b->nl < 8) return 0;
     for (int i = 0; i < b->nl; i++)
-        if (b->l[i].side) return 0;
+        if (b->l[i].side || b->l[i].joined) return 0;
     const size_t bytes = graph_key(b, NULL);
     unsigned char *key = malloc(bytes);
     if (!key) return 0;
@@ -2661,6 +2681,11 @@ static void host_outputs(qw_batch *b) {
     }
     qw_launch *l = b->nl > b->done_l ? &b->l[b->nl - 1] : NULL;
     if (!l || !l->ndirect || side) return;
+    const qw_launch *head = NULL; // l goes out with this one, which ends the batch if nothing is launched between the two
+    for (int i = b->nl - 1; l->joined && !head; i--) {
+        if (b->l[i].nj) head = &b->l[i];
+        else if (i < b->done_l || !b->l[i].joined) return;
+    }
     const unsigned mark = ++b->g->mark; // buffers that are seen to
     for (int d = 0; d < l->ndirect; d++) {
         const qw_use *u = &b->use[l->direct_use[d]];
@@ -2681,6 +2706,10 @@ static void host_outputs(qw_batch *b) {
     const qwk_fin fin = {.t_done = (uint64_t *)&b->io->t1[b->nseg - 1], .flag = (uint32_t *)&b->io->copied, .count = b->g->io_count + QW_IO_SLOTS + (size_t)b->io_idx * (QW_FIN_BYTES / 4)};
     memcpy(l->args + l->fin_at, &fin, sizeof fin);
     if (l->back_at) memcpy(l->args + l->back_at, &back, sizeof back);
+    for (int k = 0; head && k < head->nj; k++) { // (every workgroup of the joint launch counts and copies)
+        memcpy(b->l[head->jl[k]].args + l->fin_at, &fin, sizeof fin);
+        if (l->back_at) memcpy(b->l[head->jl[k]].args + l->back_at, &back, sizeof back);
+    }
     for (int d = 0; d < l->ndirect; d++)
         if (carried_back(&b->use[l->direct_use[d]])) direct_set(b, l, d);
     b->fin = true;
@@ -2696,12 +2725,65 @@ static void host_outputs(qw_batch *b) {
 #define QW_HOST_UP_MAX ((size_t)256 << 10)
 static bool host_write_ok(const qw_batch *b, const qw_hbuf *h, bool last) { return last && b->g->host_up && !b->sw.no_host_up && b->nseg == 0 && b->g->in_flight == 0 && !h->written && !h->addr && h->pinned; }
 
+// Neighbouring parts of a batch that touch nothing of each other's (qw_hip_batch_join): where they are the same kernels launch for launch, and
+// all of these have a form for several launches in one, the k-th launches of up to part_join parts go out as one, at the place of the first
+// part's. All or none: a part of which only some launches ran with another part's would have no time of its own for what it could not share.
+// Three groups of 15 tokens (benchmark's layer, IQ3_S, us): front 3 x 5.3 -> 10.4, gate/up 3 x 32.4 -> 73.7, down + combine 3 x 26.9 -> 72.3.
+// Grids: those that follow from the shape stay; gate/up and down by ranges deal their tiles over whatever grid they get, and get the compute
+// units shared out evenly.
+static bool same_launch(const qw_launch *l, const qw_launch *f) {
+    return !l->side && l->gz == 1 && !l->lds && l->fname == f->fname && l->bx == f->bx && l->argsz == f->argsz && (l->gy == 1 || !strcmp(l->fname, "qwk_cmb"));
+}
+static void join_parts(qw_batch *b) {
+    for (int s = 0, m; s < b->nparts; s += m) {
+        const int first = b->part_l[s], n = (s + 1 < b->nparts ? b->part_l[s + 1] : b->nl) - first;
+        bool ok = n > 0;
+        for (int k = 0; ok && k < n; k++) ok = same_launch(&b->l[first + k], &b->l[first + k]) && can_join(b->l[first + k].fname);
+        for (m = 1; ok && m < b->part_join && s + m < b->nparts; m++) {
+            const int at = b->part_l[s + m];
+            bool same = (s + m + 1 < b->nparts ? b->part_l[s + m + 1] : b->nl) - at == n;
+            for (int k = 0; same && k < n; k++) same = same_launch(&b->l[at + k], &b->l[first + k]);
+            if (!same) break;
+        }
+        for (int k = 0; m > 1 && k < n; k++) {
+            qw_launch *f = &b->l[first + k];
+            const bool dealt = !strncmp(f->fname, "qwk_gu_", 7) || !strncmp(f->fname, "qwk_dnr_", 8);
+            unsigned gx = (unsigned)b->g->ncu / (unsigned)m;
+            for (int j = 0; j < m; j++) gx = umin(gx, b->l[b->part_l[s + j] + k].gx);
+            f->nj = m;
+            for (int j = 0; j < m; j++) {
+                qw_launch *l = &b->l[f->jl[j] = b->part_l[s + j] + k];
+                l->joined = true;
+                if (dealt) l->gx = gx;
+            }
+        }
+    }
+}
+// The launches f->jl as one: their records side by side, then their grids (qwk_*_join)
+static bool launch_joined(qw_batch *b, const qw_launch *f, hipStream_t st) {
+    _Alignas(16) unsigned char rec[QW_JOIN_MAX * QW_MAX_ARGS + 4 * QW_JOIN_MAX] = {0};
+    char name[sizeof((qw_func *)0)->name];
+    snprintf(name, sizeof name, "%s_j", f->fname);
+    const qw_func *fn = get_func(b->g, name);
+    uint32_t *gx = (uint32_t *)(rec + QW_JOIN_MAX * f->argsz), most = 0, gy = 1;
+    for (int j = 0; j < f->nj; j++) {
+        const qw_launch *l = &b->l[f->jl[j]];
+        memcpy(rec + (size_t)j * f->argsz, l->args, f->argsz);
+        gx[j] = l->gx;
+        if (l->gx > most) most = l->gx;
+        if (l->gy > gy) gy = l->gy;
+    }
+    void *params[] = {rec};
+    return fn && HIPOK(b->g, hipModuleLaunchKernel(fn->f, most, gy, strncmp(f->fname, "qwk_dnq_", 8) ? (unsigned)f->nj : 1, f->bx, 1, 1, 0, st, params, NULL));
+}
+
 // last: the caller waits for the batch at once, and its last launch also carries the outputs back (qw_batch_wait).
 static bool submit_segment(qw_batch *b, bool last) {
     qw_gpu *g = b->g;
     hipStream_t st = g->stream[b->stream];
     if (b->failed || !flush_select(b) || !flush_tw(b, NULL, NULL) || !flush_pf(b) || !flush_gu(b) || !flush_dn(b) || !flush_pk(b)) return false;
     if (b->nseg >= 9) return fail(b, "too many flushes in one batch");
+    if (b->part_join > 1 && last && !b->prof && b->nseg == 0) join_parts(b);
     io_take(b);
     // host -> device for what this segment binds
     const unsigned mark = ++g->mark;
@@ -2795,6 +2877,10 @@ static bool submit_segment(qw_batch *b, bool last) {
             if (!side_open && !(side_open = side_link(g, st, side_of(g, b->stream)))) { b->failed = true; return false; }
             void *sparams[] = {l->args};
             if (!HIPOK(g, hipModuleLaunchKernel(l->f, l->gx, l->gy, l->gz, l->bx, 1, 1, l->lds, g->side[b->stream], sparams, NULL))) { b->failed = true; return false; }
+            continue;
+        }
+        if (l->joined) {
+            if (l->nj && !launch_joined(b, l, st)) { b->failed = true; return false; }
             continue;
         }
         if (l->join && side_open) { // join: the main stream goes on once the side stream has finished
@@ -2952,6 +3038,7 @@ bool qw_hip_parts_ok(const qw_gpu *g) { return !g->prof && g->io_used != ~0u; }
 void qw_hip_batch_part(qw_batch *b) {
     if (b->nparts < QW_PARTS_MAX) b->part_l[b->nparts++] = b->nl;
 }
+void qw_hip_batch_join(qw_batch *b, int n) { b->part_join = n < (int)QW_JOIN_MAX ? n : (int)QW_JOIN_MAX; }
 double qw_hip_batch_end_parts(qw_batch *b, double *secs) {
     for (int k = 0; k < b->nparts; k++) secs[k] = 0;
     b->part_s = secs;

@@ -215,6 +215,14 @@ typedef struct { /* out[t][row] = half(sum_s w[t][s] * Pg[t][s][row] + w[t][topk
     uint32_t D, nbr, topk, gnb;
 } qwk_cmb_args;
 
+/* Several launches of one kernel as one (the _j entry points): launch z has record g[z] and gx[z] workgroups (0: there is none).
+ * z is the grid's z, but in down + combine by token shares, whose workgroups go through the launches one after the other. */
+#define QW_JOIN_MAX 4u
+typedef struct { qwk_pre_args g[QW_JOIN_MAX]; uint32_t gx[QW_JOIN_MAX]; } qwk_pre_join;
+typedef struct { qwk_gu_args g[QW_JOIN_MAX]; uint32_t gx[QW_JOIN_MAX]; } qwk_gu_join;
+typedef struct { qwk_dn_args g[QW_JOIN_MAX]; uint32_t gx[QW_JOIN_MAX]; } qwk_dn_join;
+typedef struct { qwk_cmb_args g[QW_JOIN_MAX]; uint32_t gx[QW_JOIN_MAX]; } qwk_cmb_join;
+
 typedef struct { /* pure-read ceiling and fill helpers */
     const void *src;
     void *dst;

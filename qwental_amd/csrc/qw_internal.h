@@ -35,6 +35,9 @@ QW_INTERNAL bool qw_hip_batch_launch_static(qw_batch *b, bool recorded);
  * secs[k]: device time of part k (0: its first launch takes no stamp). Only while qw_hip_parts_ok: profiled batches have no stamps. */
 QW_INTERNAL bool qw_hip_parts_ok(const qw_gpu *g);
 QW_INTERNAL void qw_hip_batch_part(qw_batch *b);
+/* Of n neighbouring parts (0 .. n - 1, n .. 2 n - 1, ...; at most QW_JOIN_MAX) none touches what another writes: their launches may go out together. Those that
+ * did have no stamps of their own. */
+QW_INTERNAL void qw_hip_batch_join(qw_batch *b, int n);
 QW_INTERNAL double qw_hip_batch_end_parts(qw_batch *b, double *secs);
 
 #ifdef __cplusplus

@@ -23,6 +23,7 @@ struct qw_path {
     unsigned pf_max_tiles;
     uint64_t flush_mask; // bit l: submit what is recorded after layer l of a stack (src/engine.c:142, :5997 vb_flush)
     qw_buf vlg, vsel;    // logits and selection record of one group of a ragged step (qw_path_par_vstep), made at first use
+    qw_buf vset;         // and all that a group needs, for each of the others that go through the layer together
     // Kernels by what their names are made of (kernel_memo): the names are text, and three of them printed and looked up a
     // dispatch were most of what recording a layer cost (24 layers, 72 launches: 108 us with the names and a search of all
     // tile-major copies, 30 without; all of a batch is recorded before its first launch goes out)
@@ -78,7 +79,7 @@ qw_path *qw_path_open(qw_gpu *g, int D, int I, int E, int topk, int nbmax, bool 
 void qw_path_close(qw_path *p) {
     if (!p) return;
     qw_buf_free(&p->tab); qw_buf_free(&p->H); qw_buf_free(&p->psh); qw_buf_free(&p->pd); qw_buf_free(&p->cnt);
-    qw_buf_free(&p->vlg); qw_buf_free(&p->vsel);
+    qw_buf_free(&p->vlg); qw_buf_free(&p->vsel); qw_buf_free(&p->vset);
     qw_buf *pf[] = {&p->pcnt, &p->poffs, &p->pcur, &p->ptiles, &p->ppos, &p->pXs, &p->pGg, &p->pGu, &p->pH, &p->pDm};
     for (size_t i = 0; i < sizeof pf / sizeof *pf; i++) qw_buf_free(pf[i]);
     free(p);
@@ -327,10 +328,11 @@ bool qw_path_gg_router(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, c
 }
 
 // src/engine.c:568-647: front part (router + shared gate/up + selection) -> routed gate/up + shared down -> routed down -> combine
-static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, const qw_buf *x, size_t xoff, const qw_buf *lg, const qw_buf *sel, const qw_buf *out, size_t outoff,
-                      bool given);
+// What the four dispatches of a layer hand each other: buffers and byte offsets
+typedef struct { const qw_buf *lg, *sel, *H, *psh, *pd; size_t lg_at, sel_at, H_at, psh_at, pd_at; } moe_scratch;
+static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, const qw_buf *x, size_t xoff, const moe_scratch *s, const qw_buf *out, size_t outoff, bool given);
 static bool gg_moe(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, const qw_buf *x, const qw_buf *lg, const qw_buf *sel, const qw_buf *out, bool given) {
-    return gg_moe_at(p, b, M, nb, x, 0, lg, sel, out, 0, given);
+    return gg_moe_at(p, b, M, nb, x, 0, &(moe_scratch){.lg = lg, .sel = sel, .H = &p->H, .psh = &p->psh, .pd = &p->pd}, out, 0, given);
 }
 bool qw_path_gg_moe(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, const qw_buf *x, const qw_buf *lg, const qw_buf *sel,
                     const qw_buf *out) {
@@ -341,8 +343,7 @@ bool qw_path_gg_moe_lg(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, c
     return gg_moe(p, b, M, nb, x, lg, sel, out, true);
 }
 // x and out may be rows of larger buffers (byte offsets): the rows of one group of a step
-static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, const qw_buf *x, size_t xoff, const qw_buf *lg, const qw_buf *sel, const qw_buf *out, size_t outoff,
-                      bool given) {
+static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, const qw_buf *x, size_t xoff, const moe_scratch *s, const qw_buf *out, size_t outoff, bool given) {
     p->rbf = given ? 0 : 1;
     if (nb < 1 || nb > p->nbmax) {
         fprintf(stderr, "gg_moe: %d tokens, scratch was sized for %d\n", nb, p->nbmax);
@@ -362,8 +363,8 @@ static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, co
     if (given) { // the selection from the caller's logits (src/engine.c:609-614)
         if (!(k = gg_kernel(p, "moe_sel_gg", M, nbv))) return false;
         qw_batch_kernel(b, k);
-        qw_batch_buf(b, 0, lg, 0);
-        qw_batch_buf(b, 1, sel, 0);
+        qw_batch_buf(b, 0, s->lg, s->lg_at);
+        qw_batch_buf(b, 1, s->sel, s->sel_at);
         qw_batch_bytes(b, 2, &nbr, 4);
         qw_batch_dispatch(b, 1, 1, 1, 1024, 1, 1);
     }
@@ -372,12 +373,12 @@ static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, co
     bind_t(b, 0, &M->router);
     bind_t(b, 1, &M->sh_gate_w);
     qw_batch_buf(b, 2, x, xoff);
-    qw_batch_buf(b, 3, lg, 0);
+    qw_batch_buf(b, 3, s->lg, s->lg_at);
     qw_batch_buf(b, 4, &p->cnt, 0);
-    qw_batch_buf(b, 5, sel, 0);
+    qw_batch_buf(b, 5, s->sel, s->sel_at);
     bind_t(b, 6, &M->sh_gate);
     bind_t(b, 7, &M->sh_up);
-    qw_batch_buf(b, 8, &p->H, 0);
+    qw_batch_buf(b, 8, s->H, s->H_at);
     for (unsigned i = 0; i < 2; i++) { // scale / bias slots of the MLX formats: bound to the weights as placeholders
         bind_t(b, 9 + 2 * i, i ? &M->sh_up : &M->sh_gate);
         bind_t(b, 10 + 2 * i, i ? &M->sh_up : &M->sh_gate);
@@ -391,10 +392,10 @@ static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, co
     bind_t(b, 0, &M->gate);
     bind_t(b, 1, &M->up);
     bind_t(b, 2, &M->sh_down);
-    qw_batch_buf(b, 3, &p->psh, 0);
+    qw_batch_buf(b, 3, s->psh, s->psh_at);
     qw_batch_buf(b, 4, x, xoff);
-    qw_batch_buf(b, 5, sel, 0);
-    qw_batch_buf(b, 6, &p->H, 0);
+    qw_batch_buf(b, 5, s->sel, s->sel_at);
+    qw_batch_buf(b, 6, s->H, s->H_at);
     bind_t(b, 7, &M->sh_down);
     bind_t(b, 8, &M->sh_down);
     qw_batch_buf(b, 11, &p->tab, 0);
@@ -407,19 +408,19 @@ static bool gg_moe_at(qw_path *p, qw_batch *b, const qw_moe_layer *M, int nb, co
     if (!(k = gg_kernel(p, "moe_dn_gg", M, nbv))) return false;
     qw_batch_kernel(b, k);
     bind_t(b, 0, &M->down);
-    qw_batch_buf(b, 2, &p->H, 0);
-    qw_batch_buf(b, 3, sel, 0);
+    qw_batch_buf(b, 2, s->H, s->H_at);
+    qw_batch_buf(b, 3, s->sel, s->sel_at);
     qw_batch_buf(b, 7, &p->tab, 0);
-    qw_batch_buf(b, 9, &p->pd, 0);
+    qw_batch_buf(b, 9, s->pd, s->pd_at);
     qw_batch_dispatch(b, D / 16, nbr * K, 1, 128, 1, 1);
 
     if (!(k = gg_kernel(p, "moe_cmb_gg", M, nbv))) return false;
     qw_batch_kernel(b, k);
-    qw_batch_buf(b, 1, &p->psh, 0);
-    qw_batch_buf(b, 3, sel, 0);
+    qw_batch_buf(b, 1, s->psh, s->psh_at);
+    qw_batch_buf(b, 3, s->sel, s->sel_at);
     qw_batch_buf(b, 4, out, outoff);
     qw_batch_bytes(b, 8, &nbr, 4);
-    qw_batch_buf(b, 9, &p->pd, 0);
+    qw_batch_buf(b, 9, s->pd, s->pd_at);
     qw_batch_dispatch(b, D / 256, 1, 1, 256, 1, 1);
     return true;
 }
@@ -482,34 +483,47 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
     }
     double gpu = 0, wall = 0;
     if (qw_hip_parts_ok(p->g)) {
-        // All groups in one batch: one upload, one wait, the rows written to the host by each group's last launch. A group's time is
-        // the device's from its first launch to the next group's. (A batch a group, each waited for:
-        // 232.9 us for sixteen slots and 45 rows of the benchmark's layer, this 207.9.)
+        // All groups in one batch: one upload, one wait, the rows written to the host by the last launches. Up to QW_JOIN_MAX groups go through the
+        // layer side by side, each in a scratch set of its own (the last one in the path's own), three launches for all of them.
+        // (A batch a group, each waited for: 232.9 us for sixteen slots and 45 rows of the benchmark's layer; one batch, one group after the other
+        // 207.9, and on another box 198.2 against 174.2 side by side.)
         double part[QW_PAR_MAX], sum = 0;
+        const size_t sz[5] = {qw_path_logits_bytes(p, QW_PAR_VBMAX), qw_path_sel_bytes(p, QW_PAR_VBMAX), p->H.size, p->psh.size, p->pd.size};
+        size_t at[5], set = 0;
+        for (int i = 0; i < 5; i++) at[i] = set, set += (sz[i] + 255) & ~(size_t)255;
+        bool sets = ng > 1 && p->device_scratch;
+        if (sets && !p->vset.handle) sets = qw_hip_buf_new_device(p->g, (QW_JOIN_MAX - 1) * set, &p->vset); // (no memory for it: one after the other)
         const double t0 = qw_now();
         qw_batch *b = qw_batch_begin(p->g, false);
         if (!b) return false;
         bool rec = true;
         for (int gi = 0, c = 0; gi < ng && rec; c += grp[gi++]) {
+            const size_t k = sets ? (size_t)(ng - 1 - gi) % QW_JOIN_MAX : 0, o = k ? (k - 1) * set : 0;
+            const qw_buf *v = &p->vset;
+            const moe_scratch s = k ? (moe_scratch){v, v, v, v, v, o + at[0], o + at[1], o + at[2], o + at[3], o + at[4]} : (moe_scratch){.lg = &p->vlg, .sel = &p->vsel, .H = &p->H, .psh = &p->psh, .pd = &p->pd};
             qw_hip_batch_part(b);
-            rec = gg_moe_at(p, b, M, grp[gi], x, (size_t)c * (size_t)p->D * 2, &p->vlg, &p->vsel, out, (size_t)c * (size_t)p->D * 2, false);
+            rec = gg_moe_at(p, b, M, grp[gi], x, (size_t)c * (size_t)p->D * 2, &s, out, (size_t)c * (size_t)p->D * 2, false);
         }
+        if (sets) qw_hip_batch_join(b, QW_JOIN_MAX);
         const double t = qw_hip_batch_end_parts(b, part);
         if (!rec || t < 0) return false;
         gpu = t * 1e3, wall = (qw_now() - t0) * 1e3;
         bool stamped = true;
         for (int gi = 0; gi < ng; gi++) stamped = stamped && part[gi] > 0;
-        for (int gi = 0; gi < ng; gi++) sum += part[gi] = stamped ? part[gi] * 1e3 : gpu * grp[gi] / R; // (a front launch without a stamp: by rows)
+        // Without stamps of their own (groups that ran together, a front launch that takes none) the groups share the batch's time, a share being what
+        // a group takes by itself to first order: a part that does not depend on its rows, as long as eight rows' reads take, and one that does.
+        for (int gi = 0; gi < ng; gi++) sum += part[gi] = stamped ? part[gi] * 1e3 : gpu * (8 + grp[gi]) / (8 * ng + R);
         for (int gi = 0; gi < ng; gi++) qw_par_observe(par, grp[gi], part[gi]);
         qw_par_observe_step(par, wall - sum);
         if (info) info->gpu_ms = gpu, info->wall_ms = wall;
         return true;
     }
+    const moe_scratch s = {.lg = &p->vlg, .sel = &p->vsel, .H = &p->H, .psh = &p->psh, .pd = &p->pd};
     for (int gi = 0, c = 0; gi < ng; c += grp[gi++]) {
         const double t0 = qw_now();
         qw_batch *b = qw_batch_begin(p->g, false);
         if (!b) return false;
-        const bool rec = gg_moe_at(p, b, M, grp[gi], x, (size_t)c * (size_t)p->D * 2, &p->vlg, &p->vsel, out, (size_t)c * (size_t)p->D * 2, false);
+        const bool rec = gg_moe_at(p, b, M, grp[gi], x, (size_t)c * (size_t)p->D * 2, &s, out, (size_t)c * (size_t)p->D * 2, false);
         const double t = qw_batch_end(b);
         if (!rec || t < 0) return false;
         qw_par_observe(par, grp[gi], t * 1e3);
