@@ -1315,10 +1315,6 @@ QW_GU(108, 2, 0, 1, qwk_gu_f108_c2) QW_GU(112, 2, 0, 1, qwk_gu_f112_c2)
 QW_GU(QW_F_RT, 1, 0, 1, qwk_gu_rt) QW_GU(QW_F_RT, 1, 21, 1, qwk_gu_rt_s21_c1) QW_GU(QW_F_RT, 1, 8, 1, qwk_gu_rt_s8_c1)
 #endif
 
-#if QW_IN_PART(1)
-QW_GU_J(121, 2, 0, 1, qwk_gu_f121_c2_j) QW_GU_J(8, 16, 0, 1, qwk_gu_f8_c16_j) QW_GU_J(108, 2, 0, 1, qwk_gu_f108_c2_j) QW_GU_J(112, 2, 0, 1, qwk_gu_f112_c2_j) QW_GU_J(QW_F_RT, 1, 0, 1, qwk_gu_rt_j)
-#endif
-
 // ================================================================ front part of a layer (kernels/moe_gg.metal:534-590)
 // Router rows, sixteen a workgroup, on the first a.nrouter workgroups; on those after them the shared expert's gate/up with SwiGLU
 // (the reference computes it in the same dispatch, kernels/moe_gg.metal:563-573), a tile of 8 gate + 8 up rows a workgroup
@@ -1677,8 +1673,6 @@ template <int SH> __device__ __forceinline__ void pre_shared_any(const qwk_pre_a
 #if QW_IN_PART(2)
 QW_PRE(1, 0, qwk_pre_w1) QW_PRE(1, QW_F_PACKED, qwk_pre_w1_s121) QW_PRE(1, 8, qwk_pre_w1_s8) QW_PRE(1, QW_F_RT, qwk_pre_w1_kq)
 QW_PRE(30, 0, qwk_pre_w30) QW_PRE(30, QW_F_PACKED, qwk_pre_w30_s121) QW_PRE(30, 8, qwk_pre_w30_s8) QW_PRE(30, QW_F_RT, qwk_pre_w30_kq)
-QW_PRE_J(1, QW_F_PACKED, qwk_pre_w1_s121_j) QW_PRE_J(1, 8, qwk_pre_w1_s8_j) QW_PRE_J(1, QW_F_RT, qwk_pre_w1_kq_j)
-QW_PRE_J(30, QW_F_PACKED, qwk_pre_w30_s121_j) QW_PRE_J(30, 8, qwk_pre_w30_s8_j) QW_PRE_J(30, QW_F_RT, qwk_pre_w30_kq_j)
 // the shared expert's part alone (the logits given by the caller, or beside the router on another stream)
 extern "C" __global__ __launch_bounds__(64 * QW_PRE_WAVES) void qwk_qmvm_swiglu(qwk_pre_args a) {
     __shared__ qw_pre_lds L;
@@ -1899,7 +1893,6 @@ QW_DN_RANGE_NL(4, 0, 1, qwk_dnr_f20_c4) QW_DN_RANGE_NL(4, 20, 4, qwk_dnr_f20_c4_
 // the tile-major copy: rows of 320 or 640
 #if QW_IN_PART(3)
 QW_DN_RANGE_NLP(0, 10, qwk_dnr_f120_c10) QW_DN_RANGE_NLP(QW_F_PACKED_NL, 10, qwk_dnr_f120_c10_s120_c10) QW_DN_RANGE_NLP(8, 4, qwk_dnr_f120_c10_s8_c4)
-QW_DN_RANGE_NLP_J(QW_F_PACKED_NL, 10, qwk_dnr_f120_c10_s120_c10_j)
 #endif
 // rows of 320 or 640: chunks of ten blocks (a row of 640 in two), 5760 bytes a tile in flight per wave
 #if QW_IN_PART(3)
@@ -2358,8 +2351,6 @@ QW_DNQ(121, 2, 0, 1, qwk_dnq_f121_c2) QW_DNQ(121, 2, 121, 2, qwk_dnq_f121_c2_s12
 QW_DNQ(108, 1, 0, 1, qwk_dnq_f108_c1) QW_DNQ(108, 1, 108, 1, qwk_dnq_f108_c1_s108_c1)
 QW_DNQ(114, 1, 0, 1, qwk_dnq_f114_c1) QW_DNQ(114, 1, 114, 1, qwk_dnq_f114_c1_s114_c1) QW_DNQ(114, 1, 8, 4, qwk_dnq_f114_c1_s8_c4)
 QW_DNQ(121, 1, 0, 1, qwk_dnq_f121_c1) QW_DNQ(121, 1, 121, 1, qwk_dnq_f121_c1_s121_c1) QW_DNQ(121, 1, 8, 4, qwk_dnq_f121_c1_s8_c4)
-QW_DNQ_J(121, 2, 121, 2, qwk_dnq_f121_c2_s121_c2_j) QW_DNQ_J(121, 2, 8, 4, qwk_dnq_f121_c2_s8_c4_j) QW_DNQ_J(121, 1, 121, 1, qwk_dnq_f121_c1_s121_c1_j) QW_DNQ_J(121, 1, 8, 4, qwk_dnq_f121_c1_s8_c4_j)
-QW_DNQ_J(108, 1, 108, 1, qwk_dnq_f108_c1_s108_c1_j) QW_DNQ_J(114, 1, 114, 1, qwk_dnq_f114_c1_s114_c1_j)
 #endif
 
 // ================================================================ routed gate/up, down and combine as one launch
@@ -3098,13 +3089,6 @@ extern "C" __global__ __launch_bounds__(QW_WG_CMB) void qwk_cmb(qwk_cmb_args a) 
     QW_THREADS(QW_WG_CMB);
     cmb_body(a);
 }
-extern "C" __global__ __launch_bounds__(QW_WG_CMB) void qwk_cmb_j(qwk_cmb_join a) {
-    QW_THREADS(QW_WG_CMB);
-    {
-        QW_JOIN(cmb);
-        if (!idle && blockIdx.y < a.nbr) cmb_body(a);
-    }
-}
 #endif
 
 // ================================================================ memory helpers
@@ -3559,6 +3543,25 @@ extern "C" __global__ __launch_bounds__(256) void qwk_fill_blocks(qwk_fill_args 
             }
             p[w] = (uint16_t)r;
         }
+    }
+}
+#endif
+
+// ================================================================ several groups of a ragged step in one launch (QW_JOIN)
+// (At the end of the file, so that the kernels before lie beside each other as they did.)
+#if QW_IN_PART(6)
+QW_GU_J(121, 2, 0, 1, qwk_gu_f121_c2_j) QW_GU_J(8, 16, 0, 1, qwk_gu_f8_c16_j)
+QW_GU_J(108, 2, 0, 1, qwk_gu_f108_c2_j) QW_GU_J(112, 2, 0, 1, qwk_gu_f112_c2_j) QW_GU_J(QW_F_RT, 1, 0, 1, qwk_gu_rt_j)
+QW_PRE_J(1, QW_F_PACKED, qwk_pre_w1_s121_j) QW_PRE_J(1, 8, qwk_pre_w1_s8_j) QW_PRE_J(1, QW_F_RT, qwk_pre_w1_kq_j)
+QW_PRE_J(30, QW_F_PACKED, qwk_pre_w30_s121_j) QW_PRE_J(30, 8, qwk_pre_w30_s8_j) QW_PRE_J(30, QW_F_RT, qwk_pre_w30_kq_j)
+QW_DN_RANGE_NLP_J(QW_F_PACKED_NL, 10, qwk_dnr_f120_c10_s120_c10_j)
+QW_DNQ_J(121, 2, 121, 2, qwk_dnq_f121_c2_s121_c2_j) QW_DNQ_J(121, 2, 8, 4, qwk_dnq_f121_c2_s8_c4_j) QW_DNQ_J(121, 1, 121, 1, qwk_dnq_f121_c1_s121_c1_j) QW_DNQ_J(121, 1, 8, 4, qwk_dnq_f121_c1_s8_c4_j)
+QW_DNQ_J(108, 1, 108, 1, qwk_dnq_f108_c1_s108_c1_j) QW_DNQ_J(114, 1, 114, 1, qwk_dnq_f114_c1_s114_c1_j)
+extern "C" __global__ __launch_bounds__(QW_WG_CMB) void qwk_cmb_j(qwk_cmb_join a) {
+    QW_THREADS(QW_WG_CMB);
+    {
+        QW_JOIN(cmb);
+        if (!idle && blockIdx.y < a.nbr) cmb_body(a);
     }
 }
 #endif
