@@ -4,10 +4,12 @@
 
 Three steps, all cross-compile without a GPU:
   1. hipcc --genco: csrc/kernels/qw_kernels.hip -> csrc/qw_kernels_gfx950.hsaco (one code object: the same kernels spread over
-     several measured 3 % slower on the 48-layer step), and a look at the waits in it that count loads (check_counted_waits)
+     several measured 3 % slower on the 48-layer step), and a look at the waits in it that count loads (check_counted_waits);
+     beside it the kernels for several launches in one -> csrc/qw_joined_gfx950.hsaco (kernels/qw_joined.hip.h says why they lie apart)
   2. hipcc -c: csrc/qw_noalloc.hip (host + device: the per-device scratch array of the entry point that allocates nothing) -> csrc/qw_noalloc.o
-  3. clang -std=c23: csrc/gpu_hip.c (embeds the code object) + csrc/qw_path.c + csrc/qw_gguf.c + csrc/qw_par.c + qw_noalloc.o -> qwental_amd/libqwgpu_hip.so
+  3. clang -std=c23: csrc/gpu_hip.c and csrc/qw_joined.c (embed the code objects) + csrc/qw_path.c + csrc/qw_gguf.c + csrc/qw_par.c + qw_noalloc.o -> qwental_amd/libqwgpu_hip.so
 """
+import concurrent.futures
 import heapq
 import os
 import re
@@ -23,13 +25,15 @@ CLANG = os.path.join(ROCM, "llvm", "bin", "clang")
 LIB = os.path.join(HERE, "libqwgpu_hip.so")
 # Experiments: QW_BUILD_TAG=<tag> makes a second build beside the product's, libqwgpu_hip_<tag>.so with its objects in
 # csrc/_<tag>/ (QW_HIP_LIB selects it at run time); QW_BUILD_DEFS adds compiler flags, e.g. -DQW_PARTS=0x37 for a code
-# object that holds only some groups of kernels (a short compile).
+# object that holds only some groups of kernels (a short compile; the joined forms are compiled all the same).
 TAG = os.environ.get("QW_BUILD_TAG", "")
 OBJDIR = os.path.join(CSRC, "_" + TAG) if TAG else CSRC
 if TAG:
     os.makedirs(OBJDIR, exist_ok=True)
     LIB = os.path.join(HERE, "libqwgpu_hip_%s.so" % TAG)
 HSACO = os.path.join(OBJDIR, "qw_kernels_gfx950.hsaco")
+JOINED = os.path.join(OBJDIR, "qw_joined_gfx950.hsaco")
+PARTS, JOINED_PARTS = 0x3f, 0x40  # of qw_kernels.hip, groups of kernels in either code object
 # -packed-fp32-ops: packed FP32 instructions are kept out of every kernel of this library
 HIPFLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"] + os.environ.get("QW_BUILD_DEFS", "").split()
 
@@ -109,10 +113,13 @@ def check_counted_waits(text):
 
 def build(verbose=False, kernels=True):
     """kernels=False keeps the code object of the last build (host-side iterations: `python -m qwental_amd.build --host-only`)."""
-    if kernels or not os.path.exists(HSACO):
-        out = _run([HIPCC] + HIPFLAGS + ["--genco", "-I", os.path.join(CSRC, "kernels"), "-o", HSACO, os.path.join(CSRC, "kernels", "qw_kernels.hip")])
-        if verbose and out.strip():
-            print(out)
+    if kernels or not (os.path.exists(HSACO) and os.path.exists(JOINED)):
+        genco = lambda out, parts: _run([HIPCC] + HIPFLAGS + parts + ["--genco", "-I", os.path.join(CSRC, "kernels"), "-o", out, os.path.join(CSRC, "kernels", "qw_kernels.hip")])
+        some = any(f.startswith("-DQW_PARTS=") for f in HIPFLAGS)
+        with concurrent.futures.ThreadPoolExecutor(2) as two:
+            for out in two.map(genco, (HSACO, JOINED), ([] if some else ["-DQW_PARTS=%d" % PARTS], ["-UQW_PARTS", "-DQW_PARTS=%d" % JOINED_PARTS])):
+                if verbose and out.strip():
+                    print(out)
         for k in COUNTING:
             text = listing(k)
             if text.strip() or not TAG:  # (a working build may hold some groups of kernels only)
@@ -120,7 +127,7 @@ def build(verbose=False, kernels=True):
     noalloc_o = os.path.join(OBJDIR, "qw_noalloc.o")
     _run([HIPCC] + HIPFLAGS + ["-fPIC", "-I", CSRC, "-I", os.path.join(ROOT, "include"), "-c", os.path.join(CSRC, "qw_noalloc.hip"), "-o", noalloc_o])
     out = _run([CLANG, "-std=c23", "-O2", "-Wall", "-Wextra", "-fPIC", "-shared", "--embed-dir=" + OBJDIR] + [f for f in os.environ.get("QW_BUILD_DEFS", "").split() if f.startswith("-D")] + ["-I", os.path.join(ROOT, "include"), "-I", CSRC,
-                "-I", os.path.join(ROCM, "include"), os.path.join(CSRC, "gpu_hip.c"), os.path.join(CSRC, "qw_path.c"), os.path.join(CSRC, "qw_gguf.c"), os.path.join(CSRC, "qw_par.c"), noalloc_o, "-pthread", "-o", LIB,
+                "-I", os.path.join(ROCM, "include"), os.path.join(CSRC, "gpu_hip.c"), os.path.join(CSRC, "qw_joined.c"), os.path.join(CSRC, "qw_path.c"), os.path.join(CSRC, "qw_gguf.c"), os.path.join(CSRC, "qw_par.c"), noalloc_o, "-pthread", "-o", LIB,
                 "-L", os.path.join(ROCM, "lib"), "-lamdhip64", "-Wl,-rpath," + os.path.join(ROCM, "lib")])
     if verbose and out.strip():
         print(out)

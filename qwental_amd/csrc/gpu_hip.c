@@ -26,6 +26,7 @@
 static const unsigned char qw_code_object[] = {
 #embed <qw_kernels_gfx950.hsaco>
 };
+extern const unsigned char qw_joined_object[]; // (qw_joined.c)
 
 #define QW_DNQ_MIN_DEFAULT 2u // token count from which down + combine run as one launch of token quarters (qwk_dnq_*)
 enum { QW_MAX_ARGS = 448, QW_MAX_KERNELS = 4096, QW_MAX_BIND = 32, QW_MAX_BYTES = 256, QW_PROF_MAX = 8192, QW_MAX_FUNCS = 256 };
@@ -100,7 +101,7 @@ typedef struct {
 } qw_want;
 
 typedef struct {
-    hipFunction_t f;
+    hipFunction_t f, fj; // (qw_func)
     const char *fname;
     unsigned gx, gy, gz, bx, lds; // lds: bytes of dynamic LDS
     unsigned char args[QW_MAX_ARGS];
@@ -224,7 +225,7 @@ static const qw_wg_rule *wg_rule(const char *fname) {
         if (!strncmp(fname, wg_rules[i].name, strlen(wg_rules[i].name))) return &wg_rules[i];
     return &any;
 }
-typedef struct { char name[48]; hipFunction_t f; const qw_wg_rule *wg; } qw_func;
+typedef struct { char name[48]; hipFunction_t f, fj; const qw_wg_rule *wg; } qw_func; // fj: the form for several launches in one (joinable; else NULL)
 
 #define QW_LD_MAX 16
 struct qw_gpu {
@@ -232,7 +233,7 @@ struct qw_gpu {
     char name[256];
     size_t total_mem;
     int ncu;
-    hipModule_t mod;
+    hipModule_t mod, joined; // the kernels, and the forms of some of them for several launches in one
     void *tabs;   // this backend's own lookup tables in HBM (QW_TAB_BYTES); the pre-signed IQ3_S table sits at QW_TAB_IQ3SS
     hipStream_t stream[2];
     int cur_stream;
@@ -345,12 +346,13 @@ void qw_hip_reload_switches(qw_gpu *g) {
     g->fuse_broken = false; // fused launches are tried again
 }
 
-static hipFunction_t find_func(qw_gpu *g, const char *fname) {
+static hipFunction_t find_func_in(hipModule_t mod, const char *fname) {
     hipFunction_t f;
-    if (hipModuleGetFunction(&f, g->mod, fname) == hipSuccess) return f;
+    if (hipModuleGetFunction(&f, mod, fname) == hipSuccess) return f;
     (void)hipGetLastError();
     return NULL;
 }
+static hipFunction_t find_func(qw_gpu *g, const char *fname) { return find_func_in(g->mod, fname); }
 
 // ---------------------------------------------------------------- device
 // n bytes into HBM by stores of the host; returns a word whose reading back says that they have arrived.
@@ -395,8 +397,8 @@ qw_gpu *qw_gpu_open(void) {
         free(g);
         return NULL;
     }
-    if (hipModuleLoadData(&g->mod, qw_code_object) != hipSuccess) {
-        fprintf(stderr, "qw_gpu_open: the embedded gfx950 code object does not load\n");
+    if (hipModuleLoadData(&g->mod, qw_code_object) != hipSuccess || hipModuleLoadData(&g->joined, qw_joined_object) != hipSuccess) {
+        fprintf(stderr, "qw_gpu_open: the embedded gfx950 code objects do not load\n");
         free(g);
         return NULL;
     }
@@ -443,8 +445,10 @@ qw_gpu *qw_gpu_open(void) {
     {
         hipDeviceptr_t p;
         size_t sz;
-        if (hipModuleGetGlobal(&p, &sz, g->mod, "qw_stamp_ptr") == hipSuccess) (void)hipMemcpy((void *)p, &g->sync, sizeof g->sync, hipMemcpyHostToDevice);
-        else (void)hipGetLastError();
+        const hipModule_t mods[] = {g->mod, g->joined};
+        for (int i = 0; i < 2; i++)
+            if (hipModuleGetGlobal(&p, &sz, mods[i], "qw_stamp_ptr") == hipSuccess) (void)hipMemcpy((void *)p, &g->sync, sizeof g->sync, hipMemcpyHostToDevice);
+            else (void)hipGetLastError();
     }
 #endif
     g->na_batch = calloc(1, sizeof *g->na_batch);
@@ -493,6 +497,7 @@ void qw_gpu_close(qw_gpu *g) {
     (void)hipFree(g->io_count);
     if (g->na_batch) { free(g->na_batch->l); free(g->na_batch->use); free(g->na_batch); }
     (void)hipModuleUnload(g->mod);
+    (void)hipModuleUnload(g->joined);
     free(g->kernels);
     free(g);
 }
@@ -521,9 +526,15 @@ static const qw_func *get_func(qw_gpu *g, const char *fname) {
         if (!strcmp(g->funcs[i].name, fname)) return &g->funcs[i];
     if (g->nfuncs >= QW_MAX_FUNCS) return NULL;
     hipFunction_t f = find_func(g, fname);
+    hipFunction_t fj = NULL;
+    if (f && can_join(fname)) { // (looked for once a kernel, not once a launch)
+        char name[sizeof g->funcs[0].name + 2];
+        snprintf(name, sizeof name, "%s_j", fname);
+        if (!(fj = find_func_in(g->joined, name))) f = NULL;
+    }
     if (!f) { set_err(g, "no entry point %s in the code objects", fname); return NULL; }
     snprintf(g->funcs[g->nfuncs].name, sizeof g->funcs[0].name, "%s", fname);
-    g->funcs[g->nfuncs].f = f;
+    g->funcs[g->nfuncs].f = f, g->funcs[g->nfuncs].fj = fj;
     g->funcs[g->nfuncs].wg = wg_rule(fname);
     return &g->funcs[g->nfuncs++];
 }
@@ -1183,7 +1194,7 @@ static bool add_launch(qw_batch *b, const char *fname, unsigned gx, unsigned bx,
     }
     qw_launch *l = &b->l[b->nl++];
     memset(l, 0, sizeof *l);
-    l->f = f->f;
+    l->f = f->f, l->fj = f->fj;
     l->fname = fname;
     l->gx = gx; l->gy = 1; l->gz = 1; l->bx = bx;
     memcpy(l->args, args, argsz);
@@ -2738,7 +2749,7 @@ static void join_parts(qw_batch *b) {
     for (int s = 0, m; s < b->nparts; s += m) {
         const int first = b->part_l[s], n = (s + 1 < b->nparts ? b->part_l[s + 1] : b->nl) - first;
         bool ok = n > 0;
-        for (int k = 0; ok && k < n; k++) ok = same_launch(&b->l[first + k], &b->l[first + k]) && can_join(b->l[first + k].fname);
+        for (int k = 0; ok && k < n; k++) ok = b->l[first + k].fj && same_launch(&b->l[first + k], &b->l[first + k]);
         for (m = 1; ok && m < b->part_join && s + m < b->nparts; m++) {
             const int at = b->part_l[s + m];
             bool same = (s + m + 1 < b->nparts ? b->part_l[s + m + 1] : b->nl) - at == n;
@@ -2762,9 +2773,6 @@ static void join_parts(qw_batch *b) {
 // The launches f->jl as one: their records side by side, then their grids (qwk_*_join)
 static bool launch_joined(qw_batch *b, const qw_launch *f, hipStream_t st) {
     _Alignas(16) unsigned char rec[QW_JOIN_MAX * QW_MAX_ARGS + 4 * QW_JOIN_MAX] = {0};
-    char name[sizeof((qw_func *)0)->name];
-    snprintf(name, sizeof name, "%s_j", f->fname);
-    const qw_func *fn = get_func(b->g, name);
     uint32_t *gx = (uint32_t *)(rec + QW_JOIN_MAX * f->argsz), most = 0, gy = 1;
     for (int j = 0; j < f->nj; j++) {
         const qw_launch *l = &b->l[f->jl[j]];
@@ -2774,7 +2782,7 @@ static bool launch_joined(qw_batch *b, const qw_launch *f, hipStream_t st) {
         if (l->gy > gy) gy = l->gy;
     }
     void *params[] = {rec};
-    return fn && HIPOK(b->g, hipModuleLaunchKernel(fn->f, most, gy, strncmp(f->fname, "qwk_dnq_", 8) ? (unsigned)f->nj : 1, f->bx, 1, 1, 0, st, params, NULL));
+    return HIPOK(b->g, hipModuleLaunchKernel(f->fj, most, gy, strncmp(f->fname, "qwk_dnq_", 8) ? (unsigned)f->nj : 1, f->bx, 1, 1, 0, st, params, NULL));
 }
 
 // last: the caller waits for the batch at once, and its last launch also carries the outputs back (qw_batch_wait).

@@ -10,8 +10,9 @@
 #include "qw_kquants.hip.h"
 
 // The entry points come in groups, QW_IN_PART(k) around each: a build with -DQW_PARTS=<bit mask> holds only the groups
-// whose bit is set (experiments that need a few kernels and a short compile); the product build holds all of them, in
-// one code object (the same kernels spread over several code objects measured 3 % slower on the 48-layer step).
+// whose bit is set (experiments that need a few kernels and a short compile); the product build holds groups 0 to 5 in
+// one code object (the same kernels spread over several code objects measured 3 % slower on the 48-layer step) and group 6 in another
+// (qw_joined.hip.h).
 #ifdef QW_PARTS
 #define QW_IN_PART(k) ((QW_PARTS >> (k)) & 1)
 #else
@@ -325,14 +326,6 @@ __device__ __forceinline__ void qw_back_fin(const qwk_back &k, const qwk_fin &f)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
     qw_fin_wave(f);
 }
-// The launches of up to QW_JOIN_MAX groups of a ragged step as one (entry points ..._j). Every group has its own rows of x, H, record, Pg and
-// out, so nothing orders them, and one after the other each pays its own start: the launch, the selection, the first round trips, the last
-// tiles. z picks the record, of which a workgroup reads what it needs by scalar loads, as from a record of its own (through the
-// kernel's argument segment: a copy of it, indexed by z, went to scratch memory where its arrays are walked).
-#define QW_JOINED(T) (*(const qwk_##T##_join *)(const void *)__builtin_amdgcn_kernarg_segment_ptr())
-#define QW_JOIN(T)                                                                                         \
-    const qwk_##T##_args &a = QW_JOINED(T).g[blockIdx.z];                                                   \
-    const bool idle = blockIdx.x >= QW_JOINED(T).gx[blockIdx.z]
 // y[b][row] = sum_k W[row][k] x[b][k] for up to 16 activations; the weights are streamed once for all of them.
 // Tiles of 16 rows are dealt round-robin to the waves of a persistent grid; a row is CPR chunks of CH blocks.
 template <int F, int CH, bool XLDS> __device__ __forceinline__ void qmv_body(const qwk_qmv_args &a, u2 *lut, u4 *xf, f4 *red) {
@@ -1243,50 +1236,15 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, f
     QW_WSTAMP(qw_wave());
     QW_DSTAMP(2);
 }
-// The experts of the selection in the order of their numbers instead of that of the record, which has gone to memory as it is (all
-// threads; sc is complete before and after; results go by token and slot, so their places and bits do not depend on it). Groups that run beside
-// each other then come by an expert that several of them picked at about the same time, and all but the first find it in the last-level cache.
-__device__ __forceinline__ void qw_sel_by_expert(qw_sel_cache &sc, uint32_t gnb) {
-    const uint32_t U = sc.U, i = threadIdx.x, ns = gnb / 4; // (U <= 256 < threads; gnb is 8 or 16)
-    uint32_t e = 0, m = 0, at = 0, sl[4] = {};
-    if (i < U) {
-        e = sc.ue[i], m = sc.mask[i];
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++)
-            if (j < ns) sl[j] = ((const uint32_t *)sc.slot)[i * ns + j];
-#pragma unroll 8
-        for (uint32_t v = 0; v < U; v++) at += sc.ue[v] < e || (sc.ue[v] == e && v < i);
-    }
-    __syncthreads();
-    if (i < U) {
-        sc.ue[at] = e, sc.mask[at] = m;
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++)
-            if (j < ns) ((uint32_t *)sc.slot)[at * ns + j] = sl[j];
-    }
-    __syncthreads();
-}
-#define QW_GU_BODY(FGU, CHGU, FSG, CHSG, SELECTED)                                                       \
+#define QW_GU(FGU, CHGU, FSG, CHSG, NAME)                                                                 \
+    extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_gu_args a) { QW_THREADS(QW_WG_GU); \
         __shared__ struct { u2 lut[((qw_has_lut(FGU) || qw_has_lut(FSG)) ? QW_LUT_ENTRIES : 0) + (FGU == QW_F_RT ? QW_KQ_TAB / 2 : 1)]; u4 xf[QW_XF_MAXK * 2]; qw_sel_cache sc; qw_sel_scratch ss; } L; \
         qw_h_global hs = {a.H, a.hplane};                                                                      \
         static_assert(sizeof(qw_sel_scratch) >= QW_XF_MAXK / 2 * sizeof(float), "the sums of 32 activations take the place of the selection's scratch"); \
-        gu_body<FGU, CHGU, FSG, CHSG>(a, L.lut, L.xf, (float *)&L.ss, &L.sc, &L.ss, hs, false, SELECTED);                        \
+        gu_body<FGU, CHGU, FSG, CHSG>(a, L.lut, L.xf, (float *)&L.ss, &L.sc, &L.ss, hs, false, [] {});                           \
         QW_WG_END_STAMP(10);                                                                                    \
-        QW_SST_FLUSH();
-#define QW_GU(FGU, CHGU, FSG, CHSG, NAME)                                                                 \
-    extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_gu_args a) { QW_THREADS(QW_WG_GU); \
-        QW_GU_BODY(FGU, CHGU, FSG, CHSG, [] {})                                                          \
+        QW_SST_FLUSH();                                                                                         \
     }
-// Several groups' gate/up: the compute units are shared out evenly among the groups, so that one start and one end serve all of them. Three groups
-// of 15 tokens (512 experts of 2048 x 512, IQ3_S): 3 x 32.4 us one after the other, 76.6 like this, 73.7 with the experts in order (350 MB). What
-// bounds it is the stream of a compute unit's twelve waves: 80 workgroups a group instead of 85, so that an expert's tile meets the
-// same XCD's L2 in every group, took 76.2.
-#define QW_GU_J(FGU, CHGU, FSG, CHSG, NAME)                                                               \
-    extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_gu_join a) { QW_THREADS(QW_WG_GU); \
-        { QW_JOIN(gu);                                                                                   \
-        if (idle) return;                                                                                 \
-        QW_GU_BODY(FGU, CHGU, FSG, CHSG, ([&] { qw_sel_by_expert(L.sc, a.gnb); }))                       \
-    } }
 // K = D a multiple of 512: 2 IQ3_S blocks or 16 Q8_0 blocks a chunk; any other K: 1.
 #if QW_IN_PART(1)
 QW_GU(21, 2, 0, 1, qwk_gu_f21_c2) QW_GU(21, 1, 0, 1, qwk_gu_f21_c1)
@@ -1655,21 +1613,13 @@ template <int SH> __device__ __forceinline__ void pre_shared_any(const qwk_pre_a
         } else pre_pair(a, t, L);
     } else if constexpr (SH != 0) pre_shared<SH>(a, t, L);
 }
-#define QW_PRE_BODY(WF, SH)                                                                              \
+#define QW_PRE(WF, SH, NAME)                                                                             \
+    extern "C" __global__ __launch_bounds__(64 * QW_PRE_WAVES) void NAME(qwk_pre_args a) {               \
         __shared__ qw_pre_lds L;                                                                         \
         qw_started(a.t_start);                                                                           \
         if (blockIdx.x < a.nrouter) pre_router_any<WF>(a, L);                                            \
-        else pre_shared_any<SH>(a, blockIdx.x - a.nrouter, L);
-#define QW_PRE(WF, SH, NAME)                                                                             \
-    extern "C" __global__ __launch_bounds__(64 * QW_PRE_WAVES) void NAME(qwk_pre_args a) {               \
-        QW_PRE_BODY(WF, SH)                                                                              \
+        else pre_shared_any<SH>(a, blockIdx.x - a.nrouter, L);                                           \
     }
-#define QW_PRE_J(WF, SH, NAME)                                                                           \
-    extern "C" __global__ __launch_bounds__(64 * QW_PRE_WAVES) void NAME(qwk_pre_join a) {               \
-        { QW_JOIN(pre);                                                                                 \
-        if (idle) return;                                                                                \
-        QW_PRE_BODY(WF, SH)                                                                              \
-    } }
 #if QW_IN_PART(2)
 QW_PRE(1, 0, qwk_pre_w1) QW_PRE(1, QW_F_PACKED, qwk_pre_w1_s121) QW_PRE(1, 8, qwk_pre_w1_s8) QW_PRE(1, QW_F_RT, qwk_pre_w1_kq)
 QW_PRE(30, 0, qwk_pre_w30) QW_PRE(30, QW_F_PACKED, qwk_pre_w30_s121) QW_PRE(30, 8, qwk_pre_w30_s8) QW_PRE(30, QW_F_RT, qwk_pre_w30_kq)
@@ -1883,13 +1833,6 @@ QW_DN_RANGE_NL(4, 0, 1, qwk_dnr_f20_c4) QW_DN_RANGE_NL(4, 20, 4, qwk_dnr_f20_c4_
         __shared__ struct { u2 lut[QW_KQ_TAB / 2]; uint16_t arows[2 * 16 * 2 * 640]; qw_sel_cache sc; } L; \
         dn_range_body<QW_F_PACKED_NL, 10, FSD, CHSD>(a, L.lut, L.arows, &L.sc);                   \
     }
-#define QW_DN_RANGE_NLP_J(FSD, CHSD, NAME)                                                        \
-    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_join a) { QW_THREADS(QW_WG_DN); \
-        __shared__ struct { u2 lut[QW_KQ_TAB / 2]; uint16_t arows[2 * 16 * 2 * 640]; qw_sel_cache sc; } L; \
-        { QW_JOIN(dn);                                                                           \
-        if (idle) return;                                                                         \
-        dn_range_body<QW_F_PACKED_NL, 10, FSD, CHSD>(a, L.lut, L.arows, &L.sc);                   \
-    } }
 // the tile-major copy: rows of 320 or 640
 #if QW_IN_PART(3)
 QW_DN_RANGE_NLP(0, 10, qwk_dnr_f120_c10) QW_DN_RANGE_NLP(QW_F_PACKED_NL, 10, qwk_dnr_f120_c10_s120_c10) QW_DN_RANGE_NLP(8, 4, qwk_dnr_f120_c10_s8_c4)
@@ -2170,7 +2113,7 @@ __device__ __forceinline__ void dnq_run(const qwk_dn_args &a, const u2 *lut, con
         },
         ready, qw_has_lut(F) || qw_tiled(F) ? (const uint8_t *)a.glut : nullptr);
 }
-// What a workgroup has to do for a launch's record (qw_dnq_work), and what it asks for at first, on its way (qw_dnq_asked)
+// What a workgroup has to do for a launch's record
 struct qw_dnq_work { uint32_t g, t0, nt, GU; };
 __device__ __forceinline__ qw_dnq_work dnq_work(const qwk_dn_args &a) {
     const uint32_t nq = a.nq;
@@ -2184,166 +2127,128 @@ __device__ __forceinline__ qw_dnq_work dnq_work(const qwk_dn_args &a) {
     if (nt > 4) nt = 4; // (the host admits 16 tokens in four quarters, 8 in two)
     return {g, t0, nt, GU};
 }
-constexpr uint32_t QW_DNQ_NW = QW_WG_DN / 64, QW_DNQ_RPER = (2 * 6 * 8 + QW_DNQ_NW - 1) / QW_DNQ_NW; // 2 planes x 6 row blocks x 8 column blocks at most
-struct qw_dnq_asked {
-    u4 rowv[QW_DNQ_RPER];
-    uint32_t at[QW_DNQ_RPER], ue, mk, U, sl[4];
-    float w;
-};
+template <int F, int CH, int FSD, int CHSD>
+__device__ __forceinline__ void dnq_body(const qwk_dn_args &a, u2 *lut, qw_dnq_lds &L) {
+    const uint32_t K = a.topk, gnb = a.gnb, tid = threadIdx.x, lane = qw_lane(), tpw = a.tpw, rw = 16 * tpw;
+    const qw_dnq_work k = dnq_work(a);
+    const uint32_t g = k.g, t0 = k.t0, nt = k.nt, GU = k.GU;
+    QW_DSTAMP(6);
     // Everything is asked for at once, in the order in which it is wanted: the record (U, experts, masks, this quarter's slot
     // bytes and gating weights), every H row of the quarter's tokens (which rows they are does not depend on the record)
     // and the table - all through registers, so that the waits are exact (with loads straight into LDS in flight the
     // compiler waits for everything outstanding). The record goes to LDS as soon as it is there, the waves list the
     // experts and ask for their first tiles; rows and table follow into LDS while those tiles are on their way (ready()).
     // A wave's row load takes 8 rows x 128 bytes (whole cache lines), lanes 0 .. 31 the first 64 bytes of a row, 32 .. 63 the rest.
-__device__ __forceinline__ void dnq_ask(const qwk_dn_args &a, const qw_dnq_work &k, qw_dnq_asked &r) {
-    const uint32_t K = a.topk, gnb = a.gnb, tid = threadIdx.x, lane = qw_lane(), t0 = k.t0, nt = k.nt, GU = k.GU;
-    const uint32_t *ue = (const uint32_t *)(a.sel + QW_SEL_OFF_UE(gnb, K)), *mk = (const uint32_t *)(a.sel + QW_SEL_OFF_MASK(gnb, K));
-    const uint8_t *sl = a.sel + QW_SEL_OFF_SLOT(gnb, K);
-    const float *wg = (const float *)(a.sel + QW_SEL_OFF_W(gnb, K)) + t0 * (K + 1);
-    // (GU <= 160 and nt * (K + 1) <= 44: one element a thread; a thread without one reads element 0)
-    const bool rec = tid < GU, hasw = tid < nt * (K + 1);
-    const uint32_t ri = rec ? tid : 0;
-    r.ue = ue[ri], r.mk = mk[ri], r.U = *(const uint32_t *)a.sel;
-#pragma unroll
-    for (uint32_t j = 0; j < 4; j++) r.sl[j] = sl[ri * gnb + t0 + (j < nt ? j : 0)];
-    r.w = wg[hasw ? tid : 0];
-    const uint32_t upr = a.I / 8, cbs = upr / 8, used = nt * (K + 1), nrb = (used + 7) / 8, nunits = 2 * nrb * cbs, wv = qw_wave();
-    // (I is 256 or 512, so cbs 4 or 8; a unit in use has rest < 2 nrb. A unit's part of the addresses is scalar, a lane's the same in all of
-    // them, and an offset of 32 bits goes with the load: thirty instructions and a branch a load otherwise, before the table is asked for.)
-    const uint32_t lr = (lane >> 2) & 7, lc = 4 * (lane >> 5) + (lane & 3), loff = 2 * (lr * a.I + 8 * lc), lat = lc * QW_DNQ_ROWS + lr;
-#pragma unroll
-    for (uint32_t it = 0; it < QW_DNQ_RPER; it++) {
-        const uint32_t unit = wv + it * QW_DNQ_NW, cb = unit & (cbs - 1), rest = unit >> __builtin_ctz(cbs), pl = rest >= nrb, rb = rest - (pl ? nrb : 0);
-        const uint32_t off = lr < (unit < nunits ? used - 8 * rb : 0) ? 0 : ~0u;
-        const uint32_t sat = (pl * upr + 8 * cb) * QW_DNQ_ROWS + 8 * rb, soff = 2 * ((pl ? a.hplane : 0) + (t0 * (K + 1) + 8 * rb) * a.I + 64 * cb);
-        r.at[it] = ((uint32_t)__builtin_amdgcn_readfirstlane((int)sat) + lat) | off; // (masks: a choice became a branch)
-        // (a unit that is off reads the first bytes of H: a load under a condition made the compiler keep the whole array in scratch memory)
-        r.rowv[it] = *(const u4 *)((const char *)a.H + (((uint32_t)__builtin_amdgcn_readfirstlane((int)soff) + loff) & ~off));
-    }
-}
-// JOINED: several launches as one (QW_JOINED), of which a workgroup does its part one after the other: the table is in LDS once and for all, and what
-// it needs for the next one is asked for behind this one's first weights. gx: their grids. Three groups of 15 tokens (512 experts, 2048 x 512 IQ3_S
-// down rows): 3 x 26.9 us as launches of their own, 80.7 with the workgroups of the three behind one another in one grid, 72.3 like this.
-template <int F, int CH, int FSD, int CHSD, bool JOINED = false>
-__device__ __forceinline__ void dnq_body(const qwk_dn_args &a0, u2 *lut, qw_dnq_lds &L, const uint32_t *gx = nullptr) {
-    const uint32_t tid = threadIdx.x, lane = qw_lane();
-    QW_DSTAMP(6);
+    constexpr uint32_t NW = QW_WG_DN / 64, RPER = (2 * 6 * 8 + NW - 1) / NW; // 2 planes x 6 row blocks x 8 column blocks at most
     constexpr bool TAB = qw_has_lut(F) || qw_has_lut(FSD);
-    constexpr bool AHEAD = F == QW_F_PACKED && FSD == F; // (the other decoders leave no registers for it: they ask when their turn comes)
     constexpr uint32_t TPER = TAB ? (QW_LUT_BYTES / 16 + QW_WG_DN - 1) / QW_WG_DN : 0;
-    u4 tabv[TPER ? TPER : 1];
-    uint32_t tat[TPER ? TPER : 1];
-    qw_dnq_asked r;
-    auto from = [&](uint32_t z) { // the next launch that this workgroup has a part in
-        while (z < QW_JOIN_MAX && blockIdx.x >= gx[z]) z++;
-        return z;
+    u4 rowv[RPER], tabv[TPER ? TPER : 1];
+    uint32_t at[RPER], tat[TPER ? TPER : 1];
+    {
+        const uint32_t *ue = (const uint32_t *)(a.sel + QW_SEL_OFF_UE(gnb, K)), *mk = (const uint32_t *)(a.sel + QW_SEL_OFF_MASK(gnb, K));
+        const uint8_t *sl = a.sel + QW_SEL_OFF_SLOT(gnb, K);
+        const float *wg = (const float *)(a.sel + QW_SEL_OFF_W(gnb, K)) + t0 * (K + 1);
+        // (GU <= 160 and nt * (K + 1) <= 44: one element a thread; a thread without one reads element 0)
+        const bool rec = tid < GU, hasw = tid < nt * (K + 1);
+        const uint32_t ri = rec ? tid : 0;
+        const uint32_t r_ue = ue[ri], r_mk = mk[ri], r_U = *(const uint32_t *)a.sel;
+        uint32_t r_sl[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) r_sl[j] = sl[ri * gnb + t0 + (j < nt ? j : 0)];
+        const float r_w = wg[hasw ? tid : 0];
+        const uint32_t upr = a.I / 8, cbs = upr / 8, used = nt * (K + 1), nrb = (used + 7) / 8, nunits = 2 * nrb * cbs, wv = qw_wave();
+        // (I is 256 or 512, so cbs 4 or 8; a unit in use has rest < 2 nrb. A unit's part of the addresses is scalar, a lane's the same in all of
+        // them, and an offset of 32 bits goes with the load: thirty instructions and a branch a load otherwise, before the table is asked for.)
+        const uint32_t lr = (lane >> 2) & 7, lc = 4 * (lane >> 5) + (lane & 3), loff = 2 * (lr * a.I + 8 * lc), lat = lc * QW_DNQ_ROWS + lr;
+#pragma unroll
+        for (uint32_t it = 0; it < RPER; it++) {
+            const uint32_t unit = wv + it * NW, cb = unit & (cbs - 1), rest = unit >> __builtin_ctz(cbs), pl = rest >= nrb, rb = rest - (pl ? nrb : 0);
+            const uint32_t off = lr < (unit < nunits ? used - 8 * rb : 0) ? 0 : ~0u;
+            const uint32_t sat = (pl * upr + 8 * cb) * QW_DNQ_ROWS + 8 * rb, soff = 2 * ((pl ? a.hplane : 0) + (t0 * (K + 1) + 8 * rb) * a.I + 64 * cb);
+            at[it] = ((uint32_t)__builtin_amdgcn_readfirstlane((int)sat) + lat) | off; // (masks: a choice became a branch)
+            // (a unit that is off reads the first bytes of H: a load under a condition made the compiler keep the whole array in scratch memory)
+            rowv[it] = *(const u4 *)((const char *)a.H + (((uint32_t)__builtin_amdgcn_readfirstlane((int)soff) + loff) & ~off));
+        }
+        if constexpr (TAB) { // every workgroup starts at another place of the table (as qw_lut_copy_issue); the last piece of some threads repeats an earlier one
+#pragma unroll
+            for (uint32_t it = 0; it < TPER; it++) {
+                uint32_t i = tid + it * QW_WG_DN;
+                if (i >= QW_LUT_BYTES / 16) i -= QW_WG_DN;
+                tat[it] = (i + blockIdx.x * 320u) & (QW_LUT_BYTES / 16 - 1);
+                tabv[it] = ((const u4 *)a.glut)[tat[it]];
+            }
+        }
+        if (rec) {
+            uint32_t s4 = 0;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+                if (j < nt) s4 |= r_sl[j] << (8 * j);
+            L.ue[tid] = r_ue, L.mask[tid] = (uint16_t)r_mk, L.slot4[tid] = s4;
+        }
+        if (hasw) L.wl[tid] = r_w;
+        if (tid == 0) L.U = r_U, L.q[0] = qw_threads() >> 6, L.q[1] = 0;
+    }
+    __syncthreads();
+    QW_DSTAMP(7);
+    // the unique experts this quarter's tokens picked, in record order: every wave makes the whole list (all write the
+    // same values to the same places), so that none waits for another before it asks for its first weights
+    uint32_t nv = 0;
+    {
+        uint32_t U = L.U;
+        if (U > GU) U = GU;
+        const uint32_t want = (1u << nt) - 1;
+        for (uint32_t u0 = 0; u0 < U; u0 += 64) {
+            const uint32_t u = u0 + lane;
+            const bool on = u < U && (((uint32_t)L.mask[u] >> t0) & want);
+            const unsigned long long bal = __ballot(on);
+            const uint32_t at = nv + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0));
+            if (on && at < 48) L.vlist[at] = (uint16_t)u;
+            nv += (uint32_t)__popcll(bal);
+        }
+        if (nv > 48) nv = 48; // (four tokens of ten experts: 40 at most)
+    }
+    const uint32_t nsh = (FSD != 0 && a.Wsd) ? 1 : 0;
+    bool staged = false;
+    auto ready = [&] { // called by every wave once it has asked for its first tile
+        if (staged) return;
+        staged = true;
+#pragma unroll
+        for (uint32_t it = 0; it < RPER; it++)
+            if (at[it] != ~0u) L.hrows[at[it]] = rowv[it];
+        if constexpr (TAB) {
+#pragma unroll
+            for (uint32_t it = 0; it < TPER; it++) ((u4 *)lut)[tat[it]] = tabv[it];
+        }
+        __syncthreads();
+        QW_DSTAMP(8);
     };
-    uint32_t z = JOINED ? from(0) : 0;
-    bool tabled = false;
-    if (!JOINED || (AHEAD && z < QW_JOIN_MAX)) dnq_ask((&a0)[z], dnq_work((&a0)[z]), r);
-    if (JOINED && TAB) qw_lut_copy_issue(lut, (const u2 *)a0.glut); // (in registers it would hold them through the whole loop, which then spills)
-    if constexpr (TAB && !JOINED) { // every workgroup starts at another place of the table (as qw_lut_copy_issue); the last piece of some threads repeats an earlier one
-#pragma unroll
-        for (uint32_t it = 0; it < TPER; it++) {
-            uint32_t i = tid + it * QW_WG_DN;
-            if (i >= QW_LUT_BYTES / 16) i -= QW_WG_DN;
-            tat[it] = (i + blockIdx.x * 320u) & (QW_LUT_BYTES / 16 - 1);
-            tabv[it] = ((const u4 *)a0.glut)[tat[it]];
-        }
+    // the routed experts first; the shared expert's tiles go to the waves that leave the routed ones first
+    const qw_dnq_view V = {L.hrows, L.part, L.ue, L.slot4, L.mask, L.vlist, L.q};
+    dnq_run<F, CH, false, QW_DNQ_ROWS>(a, lut, V, g, t0, nt, nv, ready);
+    if (FSD != 0) {
+        if (nsh) dnq_run<FSD == 0 ? F : FSD, CHSD, true, QW_DNQ_ROWS>(a, lut, V, g, t0, nt, 1, ready);
     }
-    while (!JOINED || z < QW_JOIN_MAX) {
-        const qwk_dn_args &a = (&a0)[z];
-        const uint32_t K = a.topk, tpw = a.tpw, rw = 16 * tpw;
-        const qw_dnq_work k = dnq_work(a);
-        const uint32_t g = k.g, t0 = k.t0, nt = k.nt, GU = k.GU, next = JOINED ? from(z + 1) : 0;
-        if (JOINED && !AHEAD) dnq_ask(a, k, r);
-        {
-            const bool rec = tid < GU, hasw = tid < nt * (K + 1);
-            if (rec) {
-                uint32_t s4 = 0;
-#pragma unroll
-                for (uint32_t j = 0; j < 4; j++)
-                    if (j < nt) s4 |= r.sl[j] << (8 * j);
-                L.ue[tid] = r.ue, L.mask[tid] = (uint16_t)r.mk, L.slot4[tid] = s4;
-            }
-            if (hasw) L.wl[tid] = r.w;
-            if (tid == 0) L.U = r.U, L.q[0] = qw_threads() >> 6, L.q[1] = 0;
-        }
-        __syncthreads();
-        QW_DSTAMP(7);
-        // the unique experts this quarter's tokens picked, in record order: every wave makes the whole list (all write the
-        // same values to the same places), so that none waits for another before it asks for its first weights
-        uint32_t nv = 0;
-        {
-            uint32_t U = L.U;
-            if (U > GU) U = GU;
-            const uint32_t want = (1u << nt) - 1;
-            for (uint32_t u0 = 0; u0 < U; u0 += 64) {
-                const uint32_t u = u0 + lane;
-                const bool on = u < U && (((uint32_t)L.mask[u] >> t0) & want);
-                const unsigned long long bal = __ballot(on);
-                const uint32_t at = nv + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0));
-                if (on && at < 48) L.vlist[at] = (uint16_t)u;
-                nv += (uint32_t)__popcll(bal);
-            }
-            if (nv > 48) nv = 48; // (four tokens of ten experts: 40 at most)
-        }
-        const uint32_t nsh = (FSD != 0 && a.Wsd) ? 1 : 0;
-        bool staged = false;
-        auto ready = [&] { // called by every wave once it has asked for its first tile
-            if (staged) return;
-            staged = true;
-#pragma unroll
-            for (uint32_t it = 0; it < QW_DNQ_RPER; it++)
-                if (r.at[it] != ~0u) L.hrows[r.at[it]] = r.rowv[it];
-            if constexpr (TAB && JOINED) {
-                if (!tabled) qw_lds_arrive();
-                tabled = true;
-            } else if constexpr (TAB) {
-#pragma unroll
-                for (uint32_t it = 0; it < TPER; it++) ((u4 *)lut)[tat[it]] = tabv[it];
-            }
-            __syncthreads();
-            if (JOINED && AHEAD) dnq_ask((&a0)[next < QW_JOIN_MAX ? next : z], dnq_work((&a0)[next < QW_JOIN_MAX ? next : z]), r); // (without a next one this one's again: a load under a condition would have the arrays in scratch memory)
-            QW_DSTAMP(8);
-        };
-        // the routed experts first; the shared expert's tiles go to the waves that leave the routed ones first
-        const qw_dnq_view V = {L.hrows, L.part, L.ue, L.slot4, L.mask, L.vlist, L.q};
-        dnq_run<F, CH, false, QW_DNQ_ROWS>(a, lut, V, g, t0, nt, nv, ready);
-        if (FSD != 0) {
-            if (nsh) dnq_run<FSD == 0 ? F : FSD, CHSD, true, QW_DNQ_ROWS>(a, lut, V, g, t0, nt, 1, ready);
-        }
-        QW_DSTAMP(9);
-        __syncthreads();
-        for (uint32_t j = tid; j < nt * rw; j += qw_threads()) { // rank order, then the shared expert (qwk_cmb's arithmetic)
-            const uint32_t t = j >> (4 + __builtin_ctz(tpw)), i = j & (rw - 1), r = g * rw + i;
-            const float *w = L.wl + t * (K + 1), *p = L.part + t * (K + 1) * rw + i;
-            float o = 0;
-            for (uint32_t s = 0; s < K; s++) o = __builtin_fmaf(w[s], p[s * rw], o);
-            float sh;
-            if (nsh) sh = p[K * rw];
-            else sh = a.Psh[(size_t)(t0 + t) * a.D + r]; // the caller's own shared product
-            o = __builtin_fmaf(w[K], sh, o);
-            a.out[(size_t)(t0 + t) * a.D + r] = qw_f2h(o);
-            if (a.outh) qw_store_host(a.outh + (size_t)(t0 + t) * a.D + r, qw_f2h(o));
-        }
-        QW_DSTAMP(14);
-        if (!JOINED) return qw_back_fin(a.back, a.fin);
-        z = next;
-        __syncthreads(); // (the places that the next one fills have been read)
+    QW_DSTAMP(9);
+    __syncthreads();
+    for (uint32_t j = tid; j < nt * rw; j += qw_threads()) { // rank order, then the shared expert (qwk_cmb's arithmetic)
+        const uint32_t t = j >> (4 + __builtin_ctz(tpw)), i = j & (rw - 1), r = g * rw + i;
+        const float *w = L.wl + t * (K + 1), *p = L.part + t * (K + 1) * rw + i;
+        float o = 0;
+        for (uint32_t s = 0; s < K; s++) o = __builtin_fmaf(w[s], p[s * rw], o);
+        float sh;
+        if (nsh) sh = p[K * rw];
+        else sh = a.Psh[(size_t)(t0 + t) * a.D + r]; // the caller's own shared product
+        o = __builtin_fmaf(w[K], sh, o);
+        a.out[(size_t)(t0 + t) * a.D + r] = qw_f2h(o);
+        if (a.outh) qw_store_host(a.outh + (size_t)(t0 + t) * a.D + r, qw_f2h(o));
     }
-    qw_back_fin(a0.back, a0.fin);
+    QW_DSTAMP(14);
+    qw_back_fin(a.back, a.fin);
 }
 #define QW_DNQ(F, CH, FSD, CHSD, NAME)                                                              \
     extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_args a) { QW_THREADS(QW_WG_DN); \
         __shared__ struct { u2 lut[qw_has_lut(F) || qw_has_lut(FSD) ? QW_LUT_ENTRIES : 1]; qw_dnq_lds d; } L; \
         dnq_body<F, CH, FSD, CHSD>(a, L.lut, L.d);                                                  \
-    }
-#define QW_DNQ_J(F, CH, FSD, CHSD, NAME)                                                            \
-    extern "C" __global__ __launch_bounds__(QW_WG_DN) void NAME(qwk_dn_join a) { QW_THREADS(QW_WG_DN); \
-        __shared__ struct { u2 lut[qw_has_lut(F) || qw_has_lut(FSD) ? QW_LUT_ENTRIES : 1]; qw_dnq_lds d; } L; \
-        dnq_body<F, CH, FSD, CHSD, true>(QW_JOINED(dn).g[0], L.lut, L.d, QW_JOINED(dn).gx);         \
     }
 #if QW_IN_PART(4)
 QW_DNQ(121, 2, 0, 1, qwk_dnq_f121_c2) QW_DNQ(121, 2, 121, 2, qwk_dnq_f121_c2_s121_c2) QW_DNQ(121, 2, 8, 4, qwk_dnq_f121_c2_s8_c4)
@@ -3063,7 +2968,8 @@ QW_PFR(2, qwk_pfr_f121_c2) QW_PFR(1, qwk_pfr_f121_c1)
 // ================================================================ combine (kernels/moe_gg.metal:655-663)
 // Rank order, then the shared expert. One thread per (token, row).
 #if QW_IN_PART(5)
-__device__ __forceinline__ void cmb_body(const qwk_cmb_args &a) { // grid: 256 rows, tokens
+extern "C" __global__ __launch_bounds__(QW_WG_CMB) void qwk_cmb(qwk_cmb_args a) { // grid: 256 rows, tokens
+    QW_THREADS(QW_WG_CMB);
     const uint32_t t = blockIdx.y, row = blockIdx.x * QW_WG_CMB + threadIdx.x, K = a.topk;
     if (row >= a.D) return;
     const float *w = (const float *)(a.sel + QW_SEL_OFF_W(a.gnb, K)) + t * (K + 1);
@@ -3084,10 +2990,6 @@ __device__ __forceinline__ void cmb_body(const qwk_cmb_args &a) { // grid: 256 r
         if (s < K) o = __builtin_fmaf(wv[s], pg[s], o);
     o = __builtin_fmaf(wk, ps, o);
     a.out[(size_t)t * a.D + row] = qw_f2h(o);
-}
-extern "C" __global__ __launch_bounds__(QW_WG_CMB) void qwk_cmb(qwk_cmb_args a) {
-    QW_THREADS(QW_WG_CMB);
-    cmb_body(a);
 }
 #endif
 
@@ -3547,21 +3449,6 @@ extern "C" __global__ __launch_bounds__(256) void qwk_fill_blocks(qwk_fill_args 
 }
 #endif
 
-// ================================================================ several groups of a ragged step in one launch (QW_JOIN)
-// (At the end of the file, so that the kernels before lie beside each other as they did.)
 #if QW_IN_PART(6)
-QW_GU_J(121, 2, 0, 1, qwk_gu_f121_c2_j) QW_GU_J(8, 16, 0, 1, qwk_gu_f8_c16_j)
-QW_GU_J(108, 2, 0, 1, qwk_gu_f108_c2_j) QW_GU_J(112, 2, 0, 1, qwk_gu_f112_c2_j) QW_GU_J(QW_F_RT, 1, 0, 1, qwk_gu_rt_j)
-QW_PRE_J(1, QW_F_PACKED, qwk_pre_w1_s121_j) QW_PRE_J(1, 8, qwk_pre_w1_s8_j) QW_PRE_J(1, QW_F_RT, qwk_pre_w1_kq_j)
-QW_PRE_J(30, QW_F_PACKED, qwk_pre_w30_s121_j) QW_PRE_J(30, 8, qwk_pre_w30_s8_j) QW_PRE_J(30, QW_F_RT, qwk_pre_w30_kq_j)
-QW_DN_RANGE_NLP_J(QW_F_PACKED_NL, 10, qwk_dnr_f120_c10_s120_c10_j)
-QW_DNQ_J(121, 2, 121, 2, qwk_dnq_f121_c2_s121_c2_j) QW_DNQ_J(121, 2, 8, 4, qwk_dnq_f121_c2_s8_c4_j) QW_DNQ_J(121, 1, 121, 1, qwk_dnq_f121_c1_s121_c1_j) QW_DNQ_J(121, 1, 8, 4, qwk_dnq_f121_c1_s8_c4_j)
-QW_DNQ_J(108, 1, 108, 1, qwk_dnq_f108_c1_s108_c1_j) QW_DNQ_J(114, 1, 114, 1, qwk_dnq_f114_c1_s114_c1_j)
-extern "C" __global__ __launch_bounds__(QW_WG_CMB) void qwk_cmb_j(qwk_cmb_join a) {
-    QW_THREADS(QW_WG_CMB);
-    {
-        QW_JOIN(cmb);
-        if (!idle && blockIdx.y < a.nbr) cmb_body(a);
-    }
-}
+#include "qw_joined.hip.h"
 #endif
