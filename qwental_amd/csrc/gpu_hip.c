@@ -162,7 +162,8 @@ struct qw_batch {
     hipEvent_t ev[2 * 9]; // profiled batches, and those for which no slot was free: start/stop per submitted segment (end + at most 8 flushes)
     bool events;
     bool fin;            // the last launch raises the flag itself
-    int nparts, part_l[QW_PARTS_MAX]; // qw_hip_batch_part: the first launch of every part
+    int nparts, part_l[QW_PARTS_MAX]; // qw_hip_batch_part: the first launch of every part,
+    double part_work[QW_PARTS_MAX];   // and its work beside the others'
     int part_join;       // parts that come in sets of so many whose parts touch nothing of each other's (0: not known)
     double *part_s;      // where the seconds of the parts go (qw_hip_batch_end_parts)
     hipEvent_t *pev;      // profiling: 2 events per launch
@@ -2741,9 +2742,29 @@ static bool host_write_ok(const qw_batch *b, const qw_hbuf *h, bool last) { retu
 // part's. All or none: a part of which only some launches ran with another part's would have no time of its own for what it could not share.
 // Three groups of 15 tokens (benchmark's layer, IQ3_S, us): front 3 x 5.3 -> 10.4, gate/up 3 x 32.4 -> 73.7, down + combine 3 x 26.9 -> 72.3.
 // Grids: those that follow from the shape stay; gate/up and down by ranges deal their tiles over whatever grid they get, and get the compute
-// units shared out evenly.
+// units shared out (share_units).
 static bool same_launch(const qw_launch *l, const qw_launch *f) {
     return !l->side && l->gz == 1 && !l->lds && l->fname == f->fname && l->bx == f->bx && l->argsz == f->argsz && (l->gy == 1 || !strcmp(l->fname, "qwk_cmb"));
+}
+// Launches whose tiles go over any grid; joined, their workgroups lie behind one another
+static bool dealt(const qw_launch *l) { return !strncmp(l->fname, "qwk_gu_", 7) || !strncmp(l->fname, "qwk_dnr_", 8); }
+// The compute units among m parts by their work: in even shares a part of two rows holds half of them for nothing while one of sixteen takes
+// as long as both one after the other. In eights, one for each XCD, so that workgroups of the same number in two parts lie on one XCD and a tile
+// that both want is found in its L2. us a step, one group after the other -> even shares -> by work -> by work in eights: IQ3_S, 512 experts of
+// 2048 x 512, groups of 15 and 3 86 -> 94 -> 82 -> 83, of 16, 16, 16 and 2 212 -> 191 -> 180 -> 181; Q8_0, 64 experts, 16, 16, 16 and 2 171 -> 110 -> 127 -> 114,
+// of 15, 15 and 15 148 -> 115 -> 115 -> 98.
+static void share_units(unsigned units, const double *work, int m, unsigned *share) {
+    double all = 0;
+    int left = (int)units / 8;
+    for (int j = 0; j < m; j++) all += work[j];
+    for (int j = 0; j < m; j++) left -= (int)(share[j] = work[j] * (units / 8) >= all ? (unsigned)(work[j] * (units / 8) / all) : 1);
+    for (; left; left += left < 0 ? 1 : -1) { // the rest to those that are shortest of their due, one each; what the least took, from the one with the most
+        int at = 0;
+        for (int j = 1; j < m; j++)
+            if (left < 0 ? share[j] > share[at] : work[j] * (units / 8) / all - share[j] > work[at] * (units / 8) / all - share[at]) at = j;
+        share[at] += left < 0 ? -1 : 1;
+    }
+    for (int j = 0; j < m; j++) share[j] *= 8;
 }
 static void join_parts(qw_batch *b) {
     for (int s = 0, m; s < b->nparts; s += m) {
@@ -2756,16 +2777,15 @@ static void join_parts(qw_batch *b) {
             for (int k = 0; same && k < n; k++) same = same_launch(&b->l[at + k], &b->l[first + k]);
             if (!same) break;
         }
+        unsigned share[QW_JOIN_MAX];
+        if (m > 1) share_units((unsigned)b->g->ncu, b->part_work + s, m, share);
         for (int k = 0; m > 1 && k < n; k++) {
             qw_launch *f = &b->l[first + k];
-            const bool dealt = !strncmp(f->fname, "qwk_gu_", 7) || !strncmp(f->fname, "qwk_dnr_", 8);
-            unsigned gx = (unsigned)b->g->ncu / (unsigned)m;
-            for (int j = 0; j < m; j++) gx = umin(gx, b->l[b->part_l[s + j] + k].gx);
             f->nj = m;
             for (int j = 0; j < m; j++) {
                 qw_launch *l = &b->l[f->jl[j] = b->part_l[s + j] + k];
                 l->joined = true;
-                if (dealt) l->gx = gx;
+                if (dealt(l)) l->gx = umin(l->gx, share[j]);
             }
         }
     }
@@ -2773,16 +2793,17 @@ static void join_parts(qw_batch *b) {
 // The launches f->jl as one: their records side by side, then their grids (qwk_*_join)
 static bool launch_joined(qw_batch *b, const qw_launch *f, hipStream_t st) {
     _Alignas(16) unsigned char rec[QW_JOIN_MAX * QW_MAX_ARGS + 4 * QW_JOIN_MAX] = {0};
-    uint32_t *gx = (uint32_t *)(rec + QW_JOIN_MAX * f->argsz), most = 0, gy = 1;
+    uint32_t *gx = (uint32_t *)(rec + QW_JOIN_MAX * f->argsz), most = 0, all = 0, gy = 1;
     for (int j = 0; j < f->nj; j++) {
         const qw_launch *l = &b->l[f->jl[j]];
         memcpy(rec + (size_t)j * f->argsz, l->args, f->argsz);
-        gx[j] = l->gx;
+        all += gx[j] = l->gx;
         if (l->gx > most) most = l->gx;
         if (l->gy > gy) gy = l->gy;
     }
     void *params[] = {rec};
-    return HIPOK(b->g, hipModuleLaunchKernel(f->fj, most, gy, strncmp(f->fname, "qwk_dnq_", 8) ? (unsigned)f->nj : 1, f->bx, 1, 1, 0, st, params, NULL));
+    const bool flat = dealt(f), walked = !strncmp(f->fname, "qwk_dnq_", 8);
+    return HIPOK(b->g, hipModuleLaunchKernel(f->fj, flat ? all : most, gy, flat || walked ? 1 : (unsigned)f->nj, f->bx, 1, 1, 0, st, params, NULL));
 }
 
 // last: the caller waits for the batch at once, and its last launch also carries the outputs back (qw_batch_wait).
@@ -3043,8 +3064,8 @@ double qw_batch_wait(qw_batch *b) {
 
 // A batch recorded in parts (csrc/qw_internal.h)
 bool qw_hip_parts_ok(const qw_gpu *g) { return !g->prof && g->io_used != ~0u; }
-void qw_hip_batch_part(qw_batch *b) {
-    if (b->nparts < QW_PARTS_MAX) b->part_l[b->nparts++] = b->nl;
+void qw_hip_batch_part(qw_batch *b, double work) {
+    if (b->nparts < QW_PARTS_MAX) b->part_work[b->nparts] = work, b->part_l[b->nparts++] = b->nl;
 }
 void qw_hip_batch_join(qw_batch *b, int n) { b->part_join = n < (int)QW_JOIN_MAX ? n : (int)QW_JOIN_MAX; }
 double qw_hip_batch_end_parts(qw_batch *b, double *secs) {

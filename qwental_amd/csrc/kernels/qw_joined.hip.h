@@ -10,6 +10,12 @@
 #define QW_JOIN(T)                                                                                         \
     const qwk_##T##_args &a = QW_JOINED(T).g[blockIdx.z];                                                   \
     const bool idle = blockIdx.x >= QW_JOINED(T).gx[blockIdx.z]
+// The same where the workgroups of all launches lie behind one another: wg, this one's number among the nwg of its launch
+#define QW_JOIN_DEALT(T)                                                                                   \
+    uint32_t z = 0, wg = blockIdx.x;                                                                        \
+    for (; z < QW_JOIN_MAX - 1 && wg >= QW_JOINED(T).gx[z]; z++) wg -= QW_JOINED(T).gx[z];                  \
+    const qwk_##T##_args &a = QW_JOINED(T).g[z];                                                            \
+    const uint32_t nwg = QW_JOINED(T).gx[z]
 
 // The experts of the selection in the order of their numbers instead of that of the record, which has gone to memory as it is (all
 // threads; sc is complete before and after; results go by token and slot, so their places and bits do not depend on it). Groups that run beside
@@ -34,16 +40,20 @@ __device__ __forceinline__ void qw_sel_by_expert(qw_sel_cache &sc, uint32_t gnb)
     }
     __syncthreads();
 }
-// Several groups' gate/up: the compute units are shared out evenly among the groups, so that one start and one end serve all of them. Three groups
-// of 15 tokens (512 experts of 2048 x 512, IQ3_S): 3 x 32.4 us one after the other, 76.6 like this, 73.7 with the experts in order (350 MB). What
-// bounds it is the stream of a compute unit's twelve waves: 80 workgroups a group instead of 85, so that an expert's tile meets the
-// same XCD's L2 in every group, took 76.2.
+// Several groups' gate/up: the compute units are shared out among the groups by their work (share_units on the host), so that one start and one
+// end serve all of them. Three groups of 15 tokens (512 experts of 2048 x 512, IQ3_S): 3 x 32.4 us one after the other, 76.6 like this, 73.7 with the
+// experts in order (350 MB); groups of 15 and 3 52.8 in even shares, 39.9 by work. What bounds it is the stream of a compute unit's twelve waves.
+struct qw_h_joined : qw_h_global {
+    uint32_t wg, nwg;
+    static constexpr bool shared_grid = true;
+    __device__ __forceinline__ uint32_t workgroup() const { return wg; }
+    __device__ __forceinline__ uint32_t workgroups() const { return nwg; }
+};
 #define QW_GU_J(FGU, CHGU, NAME)                                                                            \
     extern "C" __global__ __launch_bounds__(QW_WG_GU) void NAME(qwk_gu_join a) { QW_THREADS(QW_WG_GU); \
         __shared__ struct { u2 lut[(qw_has_lut(FGU) ? QW_LUT_ENTRIES : 0) + (FGU == QW_F_RT ? QW_KQ_TAB / 2 : 1)]; u4 xf[QW_XF_MAXK * 2]; qw_sel_cache sc; qw_sel_scratch ss; } L; \
-        { QW_JOIN(gu);                                                                                       \
-        if (idle) return;                                                                                     \
-        qw_h_global hs = {a.H, a.hplane};                                                                      \
+        { QW_JOIN_DEALT(gu);                                                                                 \
+        qw_h_joined hs = {{a.H, a.hplane}, wg, nwg};                                                          \
         gu_body<FGU, CHGU, 0, 1>(a, L.lut, L.xf, (float *)&L.ss, &L.sc, &L.ss, hs, false, [&] { qw_sel_by_expert(L.sc, a.gnb); }); \
     } }
 QW_GU_J(121, 2, qwk_gu_f121_c2_j) QW_GU_J(8, 16, qwk_gu_f8_c16_j) QW_GU_J(108, 2, qwk_gu_f108_c2_j) QW_GU_J(112, 2, qwk_gu_f112_c2_j) QW_GU_J(QW_F_RT, 1, qwk_gu_rt_j)
@@ -63,9 +73,8 @@ QW_PRE_J(30, QW_F_PACKED, qwk_pre_w30_s121_j) QW_PRE_J(30, 8, qwk_pre_w30_s8_j) 
 extern "C" __global__ __launch_bounds__(QW_WG_DN) void qwk_dnr_f120_c10_s120_c10_j(qwk_dn_join a) { QW_THREADS(QW_WG_DN);
     __shared__ struct { u2 lut[QW_KQ_TAB / 2]; uint16_t arows[2 * 16 * 2 * 640]; qw_sel_cache sc; } L;
     {
-        QW_JOIN(dn);
-        if (idle) return;
-        dn_range_body<QW_F_PACKED_NL, 10, QW_F_PACKED_NL, 10>(a, L.lut, L.arows, &L.sc);
+        QW_JOIN_DEALT(dn);
+        dn_range_body<QW_F_PACKED_NL, 10, QW_F_PACKED_NL, 10, true>(a, L.lut, L.arows, &L.sc, wg, nwg);
     }
 }
 

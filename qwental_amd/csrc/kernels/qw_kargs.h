@@ -216,7 +216,8 @@ typedef struct { /* out[t][row] = half(sum_s w[t][s] * Pg[t][s][row] + w[t][topk
 } qwk_cmb_args;
 
 /* Several launches of one kernel as one (the _j entry points): launch z has record g[z] and gx[z] workgroups (0: there is none).
- * z is the grid's z, but in down + combine by token shares, whose workgroups go through the launches one after the other. */
+ * z is the grid's z; but gate/up and down by ranges, which deal their tiles over whatever grid they get, have the workgroups of all launches
+ * behind one another in x, and those of down + combine by token shares go through the launches one after the other. */
 #define QW_JOIN_MAX 4u
 typedef struct { qwk_pre_args g[QW_JOIN_MAX]; uint32_t gx[QW_JOIN_MAX]; } qwk_pre_join;
 typedef struct { qwk_gu_args g[QW_JOIN_MAX]; uint32_t gx[QW_JOIN_MAX]; } qwk_gu_join;

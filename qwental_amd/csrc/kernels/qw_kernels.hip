@@ -1076,6 +1076,10 @@ __device__ __forceinline__ void qw_sum32(const u4 *xf, float *xs, uint32_t K) {
 struct qw_h_global {
     uint16_t *H;
     uint32_t hplane;
+    // this workgroup's number, and of how many, among those that share the tiles (shared_grid: not all of the launch)
+    static constexpr bool shared_grid = false;
+    __device__ __forceinline__ uint32_t workgroup() const { return blockIdx.x; }
+    __device__ __forceinline__ uint32_t workgroups() const { return gridDim.x; }
     // a tile is done: m = the tokens that picked its expert (wave-uniform)
     __device__ __forceinline__ void tile(uint32_t) const {}
     __device__ __forceinline__ void stamp(uint32_t k) const { QW_DSTAMP(k); }
@@ -1086,7 +1090,7 @@ struct qw_h_global {
         qw_store_u16(H + o + hplane, lo);
     }
 };
-// QUEUE: the workgroup's tiles (blockIdx.x, blockIdx.x + gridDim.x, ...) go to its waves from the counter sc->qnext, which
+// QUEUE: the workgroup's tiles (its number among the launch's workgroups, that plus their count, ...) go to its waves from the counter sc->qnext, which
 // the caller has set to the number of waves before a barrier (wave w starts with the w-th of them); else wave w0 of nw takes
 // tiles w0, w0 + nw, ...
 template <int F, int CH, bool QUEUE, class S, class HS>
@@ -1141,10 +1145,11 @@ __device__ __forceinline__ void gu_tasks(const qwk_gu_args &a, const u2 *lut, co
         auto next = [&]() -> uint32_t {
             uint32_t j = 0;
             if (lane == 0) j = atomicAdd(&sc->qnext, 1u);
-            // (a workgroup's tiles lie gridDim.x tiles apart: neighbouring tiles on one compute unit measured slower, 38.4 -> 40.3 us)
-            return blockIdx.x + gridDim.x * (uint32_t)__builtin_amdgcn_readfirstlane((int)j);
+            // (a workgroup's tiles lie a whole grid apart: neighbouring tiles on one compute unit measured slower, 38.4 -> 40.3 us)
+            if constexpr (HS::shared_grid) return hs.workgroup() + hs.workgroups() * (uint32_t)__builtin_amdgcn_readfirstlane((int)j);
+            else return blockIdx.x + gridDim.x * (uint32_t)__builtin_amdgcn_readfirstlane((int)j);
         };
-        qw_task_queue<C>(ntasks, blockIdx.x + gridDim.x * qw_wave(), next, cpr, CH * C::BLK_B, kl, rowp, use, ready, spare);
+        qw_task_queue<C>(ntasks, hs.workgroup() + hs.workgroups() * qw_wave(), next, cpr, CH * C::BLK_B, kl, rowp, use, ready, spare);
     } else qw_task_stream<C>(ntasks, w0, nw, cpr, CH * C::BLK_B, kl, rowp, use, ready, spare);
 }
 
@@ -1172,7 +1177,7 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, f
             constexpr bool lutp = qw_has_lut(FGU) || qw_has_lut(FSG);
             const bool early = a.D * 2 + (QW_WG_GU / 64) * 288 / 4 <= QW_XF_MAXK * 2;
             // (four of the twelve waves ask for the table and the activations, the others make the selection meanwhile)
-            select_all<4>(sa, *ss, *sc, (float *)(early ? xf + a.D * 2 : xf), blockIdx.x == 0, [&](uint32_t part, uint32_t nparts) {
+            select_all<4>(sa, *ss, *sc, (float *)(early ? xf + a.D * 2 : xf), hs.workgroup() == 0, [&](uint32_t part, uint32_t nparts) {
                 if (lutp) qw_lut_copy_issue(lut, (const u2 *)a.glut, part, nparts);
                 if (early) qw_stage_x_issue(xf, a.x, a.D, a.D, a.nbr, part, nparts);
             }, all_w);
@@ -1183,7 +1188,7 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, f
             tabled = true;
         } else { // other expert counts need 1024 floats of scratch per wave: everything lies where x is staged afterwards
             qw_sel_scratch &so = *(qw_sel_scratch *)xf;
-            select_all(sa, so, *sc, (float *)(xf + (sizeof(qw_sel_scratch) + 15) / 16), blockIdx.x == 0, [](uint32_t, uint32_t) {}, all_w);
+            select_all(sa, so, *sc, (float *)(xf + (sizeof(qw_sel_scratch) + 15) / 16), hs.workgroup() == 0, [](uint32_t, uint32_t) {}, all_w);
             if (all_w) { // (the caller reads the weights from ss)
                 for (uint32_t i = threadIdx.x; i < a.gnb * (a.topk + 1); i += qw_threads()) ss->w[i] = so.w[i];
                 __syncthreads();
@@ -1211,6 +1216,7 @@ __device__ __forceinline__ void gu_body(const qwk_gu_args &a, u2 *lut, u4 *xf, f
     // Waves are numbered wave-major (wave w of workgroup b is number w * gridDim.x + b), so that when the tiles do not
     // divide evenly the waves with one tile more are spread over all compute units instead of filling the first ones.
     const uint32_t nw = gridDim.x * (qw_threads() >> 6), w0 = qw_wave() * gridDim.x + blockIdx.x;
+    static_assert(FSG == 0 || !HS::shared_grid, "a joint launch has no shared expert's tiles");
     if (FSG != 0) {
         if (a.Wsg) { // the shared expert's tiles go to the first waves
             qwk_gu_args sa = a;
@@ -1723,7 +1729,9 @@ template <int F, int CH, class S> __device__ __forceinline__ void dn_range_run(c
         },
         ready, qw_has_lut(F) ? (const uint8_t *)a.glut : nullptr);
 }
-template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_range_body(const qwk_dn_args &a, u2 *lut, uint16_t *arows /* [2][16][2][I] */, qw_sel_cache *sc) {
+// wg of nwg: the workgroup among those that share the tasks; all of a launch's unless JOINED.
+template <int F, int CH, int FSD, int CHSD, bool JOINED = false>
+__device__ __forceinline__ void dn_range_body(const qwk_dn_args &a, u2 *lut, uint16_t *arows /* [2][16][2][I] */, qw_sel_cache *sc, uint32_t wg = 0, uint32_t nwg = 0) {
     const uint32_t K = a.topk, gnb = a.gnb, GU = gnb * K, tpe = a.D / 16;
     auto div_tpe = [&](uint32_t x) { return qw_div(x, a.tpe_mul); };
     qw_sel_load(*sc, a.sel, K, gnb); // one memory round trip for everything the ranges depend on
@@ -1738,9 +1746,9 @@ template <int F, int CH, int FSD, int CHSD> __device__ __forceinline__ void dn_r
     const uint32_t tb = qw_tiled(F) ? a.rowbytes : 16 * a.rowbytes, stb = qw_tiled(FSD) ? a.sd_rowbytes : 16 * a.sd_rowbytes; // bytes of a tile
     const uint32_t nsh = (FSD != 0 && a.Wsd) ? 1 : 0, shw = FSD != F && nsh ? (stb + tb - 1) / tb : 1, vsh = nsh * shw * tpe;
     const uint32_t V = vsh + U * tpe;
-    uint32_t per = (V + gridDim.x - 1) / gridDim.x;
+    uint32_t per = (V + (JOINED ? nwg : gridDim.x) - 1) / (JOINED ? nwg : gridDim.x);
     if (per > tpe) per = tpe;
-    for (uint32_t base = blockIdx.x * per; base < V; base += gridDim.x * per) { // one round unless the grid is small
+    for (uint32_t base = (JOINED ? wg : blockIdx.x) * per; base < V; base += (JOINED ? nwg : gridDim.x) * per) { // one round unless the grid is small
         const uint32_t end = base + per < V ? base + per : V;
         // virtual expert of a position: 0 = shared (positions below vsh), then the routed experts
         const uint32_t v0 = base < vsh ? 0 : nsh + div_tpe(base - vsh), v1 = end - 1 < vsh ? 0 : nsh + div_tpe(end - 1 - vsh);
@@ -2272,6 +2280,9 @@ struct qw_h_lds { // the gate/up phase's SwiGLU values in LDS: entry = one (tile
     uint32_t *count, *off, *val; // val: hi | lo << 16
     uint16_t *H;
     uint32_t hplane, base;
+    static constexpr bool shared_grid = false;
+    __device__ __forceinline__ uint32_t workgroup() const { return blockIdx.x; }
+    __device__ __forceinline__ uint32_t workgroups() const { return gridDim.x; }
     __device__ __forceinline__ void stamp(uint32_t k) const { QW_DSTAMP(k); }
     __device__ __forceinline__ void tile(uint32_t m) {
         uint32_t b = 0;

@@ -501,7 +501,9 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
             const size_t k = sets ? (size_t)(ng - 1 - gi) % QW_JOIN_MAX : 0, o = k ? (k - 1) * set : 0;
             const qw_buf *v = &p->vset;
             const moe_scratch s = k ? (moe_scratch){v, v, v, v, v, o + at[0], o + at[1], o + at[2], o + at[3], o + at[4]} : (moe_scratch){.lg = &p->vlg, .sel = &p->vsel, .H = &p->H, .psh = &p->psh, .pd = &p->pd};
-            qw_hip_batch_part(b);
+            double none = 1; // the share of the experts that none of the group's rows picks, were all as likely: the group reads the others, and the shared one
+            for (int r = 0; r < grp[gi]; r++) none *= 1 - (double)p->topk / p->E;
+            qw_hip_batch_part(b, 1 + (1 - none) * p->E);
             rec = gg_moe_at(p, b, M, grp[gi], x, (size_t)c * (size_t)p->D * 2, &s, out, (size_t)c * (size_t)p->D * 2, false);
         }
         if (sets) qw_hip_batch_join(b, QW_JOIN_MAX);

@@ -32,3 +32,102 @@ def test_the_joined_kernels_lie_in_a_code_object_of_their_own(tmp_path):
     assert entry_points(build.JOINED) == sorted(joined)
     main = entry_points(build.HSACO)
     assert len(main) > 150 and not [n for n in main if n.endswith("_j")] and all(n[:-2] in main for n in joined)
+
+
+# Ragged steps of given layers and cuts: every launch with its grid, and of a joint one the workgroups of each group
+STEPS = r"""
+hipError_t hipMemGetInfo(size_t *avail, size_t *total) { return *avail = *total = (size_t)1 << 38, hipSuccess; }
+static bool listen;
+static void on_launch(const char *fname, unsigned gx, unsigned bx, const void *args) {
+    (void)bx;
+    if (!listen || !strcmp(fname, "qwk_io") || !strcmp(fname, "qwk_tab_init") || !strncmp(fname, "qwk_pack", 8)) return;
+    printf(" %s:%u", fname, gx);
+    const size_t n = strlen(fname), size = !strncmp(fname, "qwk_pre", 7) ? sizeof(qwk_pre_args) : !strncmp(fname, "qwk_gu", 6) ? sizeof(qwk_gu_args) : !strncmp(fname, "qwk_cmb", 7) ? sizeof(qwk_cmb_args) : sizeof(qwk_dn_args);
+    if (n < 2 || strcmp(fname + n - 2, "_j")) return;
+    for (unsigned j = 0; j < QW_JOIN_MAX; j++) {
+        unsigned g;
+        memcpy(&g, (const char *)args + QW_JOIN_MAX * size + 4 * j, 4);
+        printf("%c%u", j ? '+' : '=', g);
+    }
+}
+static const struct { int gu, dn, sg, su, sd, router, D, I, E, K, before, cut[9]; } steps[] = {
+@steps
+};
+int main(void) {
+    qw_gpu *g = device();
+    g->repack = true, g->copy_uses = QW_HIP_COPY_USES, g->copy_budget = (size_t)1 << 37;
+    for (size_t i = 0; i < sizeof steps / sizeof *steps; i++) {
+        const size_t D = (size_t)steps[i].D, I = (size_t)steps[i].I, E = (size_t)steps[i].E;
+        qw_path *p = qw_path_open(g, (int)D, (int)I, (int)E, steps[i].K, 16, true);
+        const int types[] = {steps[i].gu, steps[i].gu, steps[i].dn, steps[i].sg, steps[i].su, steps[i].sd, steps[i].router, steps[i].router};
+        const size_t values[] = {E * I * D, E * I * D, E * D * I, I * D, I * D, D * I, E * D, D};
+        qw_buf w[8], x, out;
+        qw_tensor t[8];
+        for (int k = 0; k < 8; k++) {
+            if (!qw_hip_buf_new_device(g, values[k] * 2, &w[k])) return printf("no memory\n"), 1; // (enough for all of these types)
+            t[k] = (qw_tensor){.buf = &w[k], .type = types[k]};
+        }
+        if (!p || !qw_buf_new(g, 64 * D * 2, &x) || !qw_buf_new(g, 64 * D * 2, &out)) return printf("no buffers\n"), 1;
+        const qw_moe_layer M = {.router = t[6], .sh_gate_w = t[7], .gate = t[0], .up = t[1], .down = t[2], .sh_gate = t[3], .sh_up = t[4], .sh_down = t[5]};
+        int R = 0, ng = 0;
+        qw_par *par = qw_par_new();
+        for (; steps[i].cut[ng]; ng++) R += steps[i].cut[ng];
+        for (int b = 1; b <= 16; b++) {
+            bool in = false;
+            for (int k = 0; k < ng; k++) in |= steps[i].cut[k] == b;
+            for (int k = 0; k < 2; k++) qw_par_observe(par, b, in ? 1e-3 : 50);
+        }
+        int n[64], cut[64];
+        for (int r = 0; r < R; r++) n[r] = 1;
+        if (qw_par_split(par, R, cut) != ng) return printf("another cut\n"), 1;
+        for (int k = 0; k <= steps[i].before; k++) {
+            listen = k == steps[i].before;
+            qw_vstep_info info;
+            qw_par *one = qw_par_new();
+            for (int b = 1; b <= 16; b++)
+                for (int q = 0; q < 2; q++) qw_par_observe(one, b, qw_par_group_cost(par, b));
+            if (!qw_path_par_vstep(p, one, &M, n, R, &x, &out, &info)) return printf("%s\n", g->err), 1;
+            if (listen) {
+                printf(" |");
+                for (int q = 0; q < info.ngroups; q++) printf(" %d", info.groups[q]);
+                printf("\n");
+            }
+            qw_par_free(one);
+        }
+        qw_par_free(par);
+        qw_path_close(p);
+        qw_buf_free(&x), qw_buf_free(&out);
+        for (int k = 0; k < 8; k++) qw_buf_free(&w[k]);
+    }
+    return 0;
+}
+"""
+
+
+def launches(tmp_path, steps):
+    """Of every step (types, router type, D, I, E, K, like steps before it, cut): [(kernel, grid, workgroups of each group or None)] and the groups."""
+    rows = ["{%s, {%s}}," % (", ".join(map(str, (*s[0], *s[1:7]))), ", ".join(map(str, s[7]))) for s in steps]
+    out = []
+    for line in hostrt.run(tmp_path, STEPS.replace("@steps", "\n".join(rows))).splitlines():
+        made, cut = line.split("|")
+        found = re.findall(r"(\w+):(\d+)(?:=([\d+]+))?", made)
+        out.append(([(k, int(gx), [int(v) for v in per.split("+") if v != "0"] if per else None) for k, gx, per in found], list(map(int, cut.split()))))
+    assert len(out) == len(steps)
+    return out
+
+
+IQ3, IQ3_Q8, NL, K4, Q8 = (21, 21, 21, 21, 21), (21, 21, 8, 8, 8), (21, 20, 12, 23, 20), (12, 14, 12, 12, 14), (8, 8, 8, 8, 8)
+
+
+def test_compute_units_by_the_groups_work(tmp_path):
+    """A group of two rows reads a seventh of the experts that one of sixteen reads, and gets about that many of the workgroups."""
+    steps = [(IQ3, 1, 512, 256, 512, 10, 1, c) for c in ([16, 2], [15, 3], [16, 16, 16, 2], [9, 9], [15, 15, 15], [16, 15, 7])] + [(NL, 1, 1024, 640, 128, 4, 1, [15, 3])]
+    for (made, cut), (E, K) in zip(launches(tmp_path, steps), (s[4:6] for s in steps)):
+        work = [1 + E * (1 - (1 - K / E) ** r) for r in cut]
+        for kernel, gx, per in made:
+            assert kernel.endswith("_j") and len(per) == len(cut)
+            if not kernel.startswith(("qwk_gu_", "qwk_dnr_")):
+                continue
+            assert gx == sum(per) <= 256 and all(p % 8 == 0 for p in per)  # behind one another, eights for the eight XCDs
+            for p, w in zip(per, work):
+                assert abs(p - 256 * w / sum(work)) <= 12, (cut, kernel, per)
