@@ -70,6 +70,9 @@ QW_GU_J(121, 2, qwk_gu_f121_c2_j) QW_GU_J(8, 16, qwk_gu_f8_c16_j) QW_GU_J(108, 2
 QW_PRE_J(1, QW_F_PACKED, qwk_pre_w1_s121_j) QW_PRE_J(1, 8, qwk_pre_w1_s8_j) QW_PRE_J(1, QW_F_RT, qwk_pre_w1_kq_j)
 QW_PRE_J(30, QW_F_PACKED, qwk_pre_w30_s121_j) QW_PRE_J(30, 8, qwk_pre_w30_s8_j) QW_PRE_J(30, QW_F_RT, qwk_pre_w30_kq_j)
 
+// Down by ranges: a workgroup takes at most one expert's tiles a round, and there are more experts than a group has workgroups. In rounds that are
+// filled evenly (QW_RANGE_PER): full ones, and 132 experts on 128 workgroups took two rounds of which the second was all but empty. Two groups
+// of 16 tokens (512 experts of 2560 x 640, IQ4_NL): 2 x 34.8 us one after the other, 107.1 in full rounds, 67.5 like this; three of 15 3 x 33.1, 106.8, 92.6.
 extern "C" __global__ __launch_bounds__(QW_WG_DN) void qwk_dnr_f120_c10_s120_c10_j(qwk_dn_join a) { QW_THREADS(QW_WG_DN);
     __shared__ struct { u2 lut[QW_KQ_TAB / 2]; uint16_t arows[2 * 16 * 2 * 640]; qw_sel_cache sc; } L;
     {

@@ -138,6 +138,9 @@ typedef struct {
     uint32_t fgu;
     uint32_t tpe_mul; /* QW_DIV_MUL(I / 8) */
 } qwk_gu_args;
+/* per tasks of a workgroup in rounds of at most `most`: those of a round, as few rounds as that takes and evenly filled */
+#define QW_ROUNDS(per, most) (((per) + (most) - 1) / (most))
+#define QW_RANGE_PER(per, most) (((per) + QW_ROUNDS(per, most) - 1) / QW_ROUNDS(per, most))
 /* For qw_div: x / d = x * QW_DIV_MUL(d) >> 32, d >= 2, x * d < 2^32 */
 #define QW_DIV_MUL(d) ((uint32_t)((((uint64_t)1) << 32) / (d) + 1))
 

@@ -1747,7 +1747,7 @@ __device__ __forceinline__ void dn_range_body(const qwk_dn_args &a, u2 *lut, uin
     const uint32_t nsh = (FSD != 0 && a.Wsd) ? 1 : 0, shw = FSD != F && nsh ? (stb + tb - 1) / tb : 1, vsh = nsh * shw * tpe;
     const uint32_t V = vsh + U * tpe;
     uint32_t per = (V + (JOINED ? nwg : gridDim.x) - 1) / (JOINED ? nwg : gridDim.x);
-    if (per > tpe) per = tpe;
+    if (per > tpe) per = JOINED ? QW_RANGE_PER(per, tpe) : tpe; // (JOINED: a few workgroups for up to 161 experts)
     for (uint32_t base = (JOINED ? wg : blockIdx.x) * per; base < V; base += (JOINED ? nwg : gridDim.x) * per) { // one round unless the grid is small
         const uint32_t end = base + per < V ? base + per : V;
         // virtual expert of a position: 0 = shared (positions below vsh), then the routed experts

@@ -131,3 +131,24 @@ def test_compute_units_by_the_groups_work(tmp_path):
             assert gx == sum(per) <= 256 and all(p % 8 == 0 for p in per)  # behind one another, eights for the eight XCDs
             for p, w in zip(per, work):
                 assert abs(p - 256 * w / sum(work)) <= 12, (cut, kernel, per)
+
+
+ROUNDS = r"""
+static void on_launch(const char *fname, unsigned gx, unsigned bx, const void *args) { (void)fname, (void)gx, (void)bx, (void)args; }
+int main(void) {
+    for (unsigned tpe = 16; tpe <= 160; tpe += 16)
+        for (unsigned U = 1; U <= 161; U++)
+            for (unsigned nwg = 1; nwg <= 256; nwg++) { // (dn_range_body's loop)
+                const unsigned V = U * tpe, all = (V + nwg - 1) / nwg, per = all > tpe ? QW_RANGE_PER(all, tpe) : all;
+                unsigned rounds = 0, most = 0;
+                for (unsigned base = 0; base < V; base += nwg * per) rounds++, most += per;
+                if (per > tpe || rounds != QW_ROUNDS(all, tpe) || most >= all + rounds) return printf("%u experts of %u tiles, %u workgroups: %u rounds of %u\n", U, tpe, nwg, rounds, per), 1;
+            }
+    return 0;
+}
+"""
+
+
+def test_rounds_of_down_by_ranges_are_filled_evenly(tmp_path):
+    """No workgroup has more than its share and a tile a round, and none more than an expert's tiles in a round."""
+    hostrt.run(tmp_path, ROUNDS)
