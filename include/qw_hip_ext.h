@@ -119,6 +119,7 @@ unsigned qw_hip_graph_launches(const qw_gpu *g);
  *                             Q8_0 and Q6_K down rows (default 2; 0: never)
  *   QW_HIP_PK_SPLIT           the packing sequence (p_zero, moe_count, moe_plan_t, moe_scatter, moe_pf_gg x 2, p_act2) one launch per
  *                             dispatch instead of one launch for the first four and SwiGLU inside the gate / up launch
+ *   QW_HIP_NO_JOIN            the groups of a ragged step (qw_path_par_vstep) one after the other instead of side by side
  *   QW_HIP_SIDE=1             a shared expert's gate/up in the K-quant / IQ4 / plain formats runs on a side stream beside the router
  *   QW_HIP_DN_ANY             IQ4_NL, K-quant and IQ4_XS down rows take the any-shape kernel instead of the range kernel (and, like Q8_0 rows,
  *                             no tile-major copy)
@@ -132,6 +133,10 @@ unsigned qw_hip_graph_launches(const qw_gpu *g);
  * goes to stderr as it is set) and QW_HIP_QUIET (qw_batch_wait prints none). QW_HIP_REPACK=0 and QW_HIP_GRAPH=1 are
  * read by qw_gpu_open() only (see above); afterwards qw_hip_set_repack / qw_hip_set_graphs change them. */
 void qw_hip_reload_switches(qw_gpu *g);
+/* Launches so far that stood for several groups of a ragged step, and the entry point of the back-th last one (back < 4, 0: the last; NULL: there
+ * were not that many): a group's own launches of that kernel, which went out together. */
+unsigned qw_hip_joint_launches(const qw_gpu *g);
+const char *qw_hip_joint_kernel(const qw_gpu *g, unsigned back);
 /* Whether the host can write the device's memory itself (small uploads then need no launch), and how many bytes it has uploaded so. */
 bool qw_hip_host_uploads(const qw_gpu *g, size_t *bytes);
 /* The device's synchronisation words (the first 384 are the barrier's: all zero between launches except word 0, the

@@ -136,7 +136,7 @@ enum { QW_IO_SLOTS = 32 };
 _Static_assert(QW_IO_SLOTS % QW_FIN_LINE == 0, "the counters behind the words begin a line");
 
 // measurement switches: read from the environment by qw_gpu_open (and again by qw_hip_reload_switches), never per batch
-typedef struct { unsigned dnc_nb, dnq_min, spin_limit, hc_rows; int side, load_threads; bool dn_any, nl_c4, no_swiglu_matvec, shared_in_gu, split_select, pk_split, kq_own, no_fuse, ablate, no_host_up, verbose, quiet; } qw_switches;
+typedef struct { unsigned dnc_nb, dnq_min, spin_limit, hc_rows; int side, load_threads; bool dn_any, nl_c4, no_swiglu_matvec, shared_in_gu, split_select, pk_split, kq_own, no_fuse, ablate, no_host_up, no_join, verbose, quiet; } qw_switches;
 
 struct qw_batch {
     qw_gpu *g;
@@ -267,6 +267,8 @@ struct qw_gpu {
     // that were launched eagerly (a graph is built only when a sequence repeats). Off unless QW_HIP_GRAPH=1 / qw_hip_set_graphs.
     struct qw_graph { uint64_t hash; int nl; size_t bytes; unsigned char *key; hipGraphExec_t exec; } graphs[8];
     unsigned ngraph_next, ngraph_launches;
+    unsigned njoint;             // launches for several groups so far,
+    const char *joint_fname[4];  // and the kernels of the last of them
     uint64_t seen_hash[8];
     unsigned nseen;
     bool use_graphs;
@@ -336,6 +338,7 @@ static void read_switches(qw_gpu *g) {
     e = getenv("QW_HIP_LOAD_THREADS");
     w->load_threads = e && atoi(e) > 0 ? (atoi(e) > QW_LD_MAX ? QW_LD_MAX : atoi(e)) : 4;
     w->no_host_up = getenv("QW_HIP_NO_HOST_UP") != NULL; // uploads always by a launch
+    w->no_join = getenv("QW_HIP_NO_JOIN") != NULL; // groups of a ragged step one after the other
     w->verbose = getenv("QW_HIP_VERBOSE") != NULL, w->quiet = getenv("QW_HIP_QUIET") != NULL;
 }
 bool qw_hip_sync_words(qw_gpu *g, uint32_t *dst, size_t nwords) {
@@ -906,6 +909,8 @@ size_t qw_hip_copy_budget(const qw_gpu *g, size_t *used) {
     return g->copy_budget;
 }
 unsigned qw_hip_graph_launches(const qw_gpu *g) { return g->ngraph_launches; }
+unsigned qw_hip_joint_launches(const qw_gpu *g) { return g->njoint; }
+const char *qw_hip_joint_kernel(const qw_gpu *g, unsigned back) { return back < 4 && back < g->njoint ? g->joint_fname[(g->njoint - 1 - back) % 4] : NULL; }
 bool qw_hip_host_uploads(const qw_gpu *g, size_t *bytes) { return *bytes = g->host_up_bytes, g->host_up; }
 void qw_hip_set_graphs(qw_gpu *g, bool on) { g->use_graphs = on; }
 size_t qw_hip_packed_bytes(const qw_gpu *g) { return g->pack_bytes; }
@@ -2802,6 +2807,7 @@ static bool launch_joined(qw_batch *b, const qw_launch *f, hipStream_t st) {
         if (l->gy > gy) gy = l->gy;
     }
     void *params[] = {rec};
+    b->g->joint_fname[b->g->njoint++ % 4] = f->fname;
     const bool flat = dealt(f), walked = !strncmp(f->fname, "qwk_dnq_", 8);
     return HIPOK(b->g, hipModuleLaunchKernel(f->fj, flat ? all : most, gy, flat || walked ? 1 : (unsigned)f->nj, f->bx, 1, 1, 0, st, params, NULL));
 }
@@ -2812,7 +2818,7 @@ static bool submit_segment(qw_batch *b, bool last) {
     hipStream_t st = g->stream[b->stream];
     if (b->failed || !flush_select(b) || !flush_tw(b, NULL, NULL) || !flush_pf(b) || !flush_gu(b) || !flush_dn(b) || !flush_pk(b)) return false;
     if (b->nseg >= 9) return fail(b, "too many flushes in one batch");
-    if (b->part_join > 1 && last && !b->prof && b->nseg == 0) join_parts(b);
+    if (b->part_join > 1 && last && !b->prof && b->nseg == 0 && !b->sw.no_join) join_parts(b);
     io_take(b);
     // host -> device for what this segment binds
     const unsigned mark = ++g->mark;

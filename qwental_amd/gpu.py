@@ -74,7 +74,7 @@ SYMBOLS = [
     ("qw_hip_buf_write_fd", _b, [_pb, _sz, _i, C.c_uint64, _sz]),
     ("qw_hip_reload_switches", None, [_vp]), ("qw_hip_sync_words", _b, [_vp, _vp, _sz]),
     ("qw_hip_set_repack", None, [_vp, _b]), ("qw_hip_set_copy_uses", None, [_vp, C.c_uint]),
-    ("qw_hip_set_copy_budget", None, [_vp, _sz]), ("qw_hip_copy_budget", _sz, [_vp, C.POINTER(_sz)]), ("qw_hip_graph_launches", C.c_uint, [_vp]), ("qw_hip_host_uploads", _b, [_vp, C.POINTER(_sz)]), ("qw_hip_set_graphs", None, [_vp, _b]),
+    ("qw_hip_set_copy_budget", None, [_vp, _sz]), ("qw_hip_copy_budget", _sz, [_vp, C.POINTER(_sz)]), ("qw_hip_graph_launches", C.c_uint, [_vp]), ("qw_hip_joint_launches", C.c_uint, [_vp]), ("qw_hip_joint_kernel", C.c_char_p, [_vp, C.c_uint]), ("qw_hip_host_uploads", _b, [_vp, C.POINTER(_sz)]), ("qw_hip_set_graphs", None, [_vp, _b]),
     ("qw_hip_packed_bytes", _sz, [_vp]), ("qw_hip_buf_release_source", _b, [_pb]), ("qw_hip_released_bytes", _sz, [_vp]),
     ("qw_hip_compile_check", _b, [C.c_char_p, _sz, C.c_char_p, _sz, C.c_char_p, _sz]),
     ("qw_hip_last_error", C.c_char_p, [_vp]), ("qw_hip_cu_count", _i, [_vp]), ("qw_hip_arch", C.c_char_p, []),
@@ -343,6 +343,11 @@ class Gpu:
                 else:
                     os.environ[name] = v
             self.L.qw_hip_reload_switches(self.g)
+
+    def joint_kernels(self, since):
+        """Entry points of the (last four) launches for several groups of a ragged step that came after the first `since`, in their order."""
+        n = self.L.qw_hip_joint_launches(self.g) - since
+        return [self.L.qw_hip_joint_kernel(self.g, i).decode() for i in reversed(range(min(n, 4)))]
 
     def profile_entries(self, entry_points=True):
         """(name, microseconds) per launch of the last profiled batch; entry-point names, or the callers' kernel names."""

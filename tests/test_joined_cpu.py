@@ -7,6 +7,7 @@ import subprocess
 import pytest
 
 import hostrt
+import test_gpu_joined
 from qwental_amd import build
 
 NAMES = r"""
@@ -152,3 +153,30 @@ int main(void) {
 def test_rounds_of_down_by_ranges_are_filled_evenly(tmp_path):
     """No workgroup has more than its share and a tile a round, and none more than an expert's tiles in a round."""
     hostrt.run(tmp_path, ROUNDS)
+
+
+def test_every_joined_kernel_has_a_test_that_sees_it_run(tmp_path):
+    cases = next(m for m in test_gpu_joined.test_groups_that_go_out_together.pytestmark if m.name == "parametrize").args[1]
+    seen = {"qwk_%s_j" % k for c in cases for k in c[8] + (c[9] or [])}
+    assert seen == set(hostrt.run(tmp_path, NAMES).split())
+
+
+def test_which_launches_a_step_makes(tmp_path):
+    """Sets of up to four neighbouring groups of the same kernels, launch for launch; all launches of a group are joined, or none."""
+    iq3, kq = (IQ3, 1, 512, 256, 64, 4, 1), (K4, 1, 512, 256, 64, 4, 1)  # (Q6_K rows of less than 64 MB: not joined)
+    j3 = ["qwk_pre_w1_s121_j", "qwk_gu_f121_c2_j", "qwk_dnq_f121_c1_s121_c1_j"]
+    one = ["qwk_pre_w1_s121", "qwk_gu_f121_c2", "qwk_dnc_f121_c1_s121_c1"]
+    alone = [k[:-2] for k in j3]
+    nl = ["qwk_pre_w1_kq_j", "qwk_gu_f121_c2_j", "qwk_dnr_f120_c10_s120_c10_j", "qwk_cmb_j"]
+    steps = [((*iq3, [16]), alone), ((*iq3, [9, 9]), j3), ((*iq3, [16] * 4), j3), ((*iq3, [12] * 5), j3 + alone), ((*iq3, [8] * 6), j3 + j3), ((*iq3, [16, 16, 1]), None),
+             ((*iq3[:-1], 0, [9, 9]), None), ((IQ3_Q8, *iq3[1:], [7, 7, 7]), ["qwk_pre_w1_s8_j", j3[1], "qwk_dnq_f121_c1_s8_c4_j"]), ((NL, 1, 512, 640, 64, 4, 1, [16] * 3), nl),
+             ((*kq, [9, 9]), ["qwk_pre_w1_kq", "qwk_gu_f112_c2", "qwk_dnr_f14_c1_s14_c1", "qwk_cmb"] * 2)]
+    for (step, want), (made, cut) in zip(steps, launches(tmp_path, [s for s, _ in steps])):
+        if want is None and step[-1] == [9, 9]:  # the first step of a path: its first group also makes the path's table, and is another sequence of launches
+            want = alone + alone
+        elif want is None:  # a group of one row has a form of its own
+            at = cut.index(1)
+            want = {0: one + j3, 1: alone + one + alone, 2: j3 + one}[at]
+        assert [k for k, _, _ in made] == want, (step, cut)
+        for k, _, per in made:
+            assert (per is not None) == k.endswith("_j")
