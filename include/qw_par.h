@@ -30,8 +30,15 @@ qw_par *qw_par_new(void);
 void qw_par_free(qw_par *p);
 /* One measured group of b rows (1 .. QW_PAR_VBMAX) took ms. */
 void qw_par_observe(qw_par *p, int b, double ms);
-/* The table entry of size b: the running average, 0 when not measured yet. */
+/* Groups of b[0 .. n) rows that the device ran side by side took ms together (n = 1: qw_par_observe). Each is given its share of ms, in
+ * proportion to what the table expects of its size (before anything is known, half evenly and half by rows), and the share averages in an entry
+ * of its own, of a group beside others: the price of a size differs between the two, since groups side by side share one start. */
+void qw_par_observe_set(qw_par *p, const int *b, int n, double ms);
+/* The table entry of size b: the running average of a group by itself (where one only ever ran beside others: of those), 0 when not measured
+ * yet; and that of a group beside others, 0 when never measured so. A step of one group is priced at the first, the groups of any other step at
+ * the second, or where that is 0 the first. */
 double qw_par_group_cost(const qw_par *p, int b);
+double qw_par_joint_cost(const qw_par *p, int b);
 /* What a step took beside its groups, whose times are then the device's alone: upload, recording, submission and wait come once
  * a step, however many groups it has. Averaged as the groups' times are, and added once to the estimate of a step; the cut does not
  * depend on it. For whoever runs the groups of a step in one batch (qw_path_par_vstep); never called, it is 0: a group's

@@ -2795,6 +2795,8 @@ static void join_parts(qw_batch *b) {
         }
     }
 }
+// Part k went out with the one before it
+static bool part_follows(const qw_batch *b, int k) { return b->part_l[k] < b->nl && b->l[b->part_l[k]].joined && !b->l[b->part_l[k]].nj; }
 // The launches f->jl as one: their records side by side, then their grids (qwk_*_join)
 static bool launch_joined(qw_batch *b, const qw_launch *f, hipStream_t st) {
     _Alignas(16) unsigned char rec[QW_JOIN_MAX * QW_MAX_ARGS + 4 * QW_JOIN_MAX] = {0};
@@ -3039,9 +3041,10 @@ static double batch_wait(qw_batch *b, bool ended) { // ended: submitted by qw_ba
             secs += (double)ms * 1e-3;
         }
     }
-    if (b->part_s) { // from one part's start to the next one's; 0 where a stamp is missing
-        for (int k = 0; k < b->nparts; k++) {
-            const uint64_t t0 = !ok || !b->io ? 0 : k ? b->io->part[k] : b->io->t0[0], t1 = !ok || !b->io ? 0 : k + 1 < b->nparts ? b->io->part[k + 1] : b->io->t1[0];
+    if (b->part_s) { // from the start of a part, and those that went out with it, to the next one's; 0 where a stamp is missing
+        for (int k = 0, e; k < b->nparts; k = e) {
+            for (e = k + 1; e < b->nparts && part_follows(b, e); e++) b->part_s[e] = -1;
+            const uint64_t t0 = !ok || !b->io ? 0 : k ? b->io->part[k] : b->io->t0[0], t1 = !ok || !b->io ? 0 : e < b->nparts ? b->io->part[e] : b->io->t1[0];
             b->part_s[k] = t0 && t1 > t0 ? (double)(t1 - t0) * g->tick : 0;
         }
     }

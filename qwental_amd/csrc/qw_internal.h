@@ -32,11 +32,11 @@ QW_INTERNAL qw_batch *qw_hip_batch_begin_static(qw_gpu *g, void *stream);
 QW_INTERNAL bool qw_hip_batch_launch_static(qw_batch *b, bool recorded);
 
 /* A batch in parts: qw_hip_batch_part before the dispatches of each part (up to 64), qw_hip_batch_end_parts instead of qw_batch_end;
- * work: the part's beside the others', in any unit (> 0). secs[k]: device time of part k (0: its first launch takes no stamp). Only while qw_hip_parts_ok: profiled batches have no stamps. */
+ * work: the part's beside the others', in any unit (> 0). secs[k]: device time of part k and of the parts after it that went out with it, which have
+ * -1 (0: its first launch takes no stamp). Only while qw_hip_parts_ok: profiled batches have no stamps. */
 QW_INTERNAL bool qw_hip_parts_ok(const qw_gpu *g);
 QW_INTERNAL void qw_hip_batch_part(qw_batch *b, double work);
-/* Of n neighbouring parts (0 .. n - 1, n .. 2 n - 1, ...; at most QW_JOIN_MAX) none touches what another writes: their launches may go out together. Those that
- * did have no stamps of their own. */
+/* Of any n parts in a row (at most QW_JOIN_MAX) none touches what another writes: the launches of up to n in a row, from any one on, may go out together. */
 QW_INTERNAL void qw_hip_batch_join(qw_batch *b, int n);
 QW_INTERNAL double qw_hip_batch_end_parts(qw_batch *b, double *secs);
 

@@ -5,8 +5,8 @@
 #define NBUCKET (QW_PAR_PACK_MAX / 16)
 
 struct qw_par {
-    double cost[QW_PAR_VBMAX + 1];
-    int seen[QW_PAR_VBMAX + 1];
+    double cost[QW_PAR_VBMAX + 1], joint[QW_PAR_VBMAX + 1]; // of a group by itself, and beside others
+    int seen[QW_PAR_VBMAX + 1], jseen[QW_PAR_VBMAX + 1];
     double step; // once a step, whatever its groups
     int step_seen;
     double pcost[NBUCKET + 1]; // bucket k: rows 16 (k - 1) + 1 .. 16 k
@@ -27,7 +27,12 @@ void qw_par_observe_step(qw_par *p, double ms) {
     if (ms > 0) observe(&p->step, &p->step_seen, ms);
 }
 double qw_par_step_cost(const qw_par *p) { return p->step; }
-double qw_par_group_cost(const qw_par *p, int b) { return b >= 1 && b <= QW_PAR_VBMAX ? p->cost[b] : 0; }
+double qw_par_joint_cost(const qw_par *p, int b) { return b >= 1 && b <= QW_PAR_VBMAX ? p->joint[b] : 0; }
+double qw_par_group_cost(const qw_par *p, int b) { return b >= 1 && b <= QW_PAR_VBMAX && p->cost[b] > 0 ? p->cost[b] : qw_par_joint_cost(p, b); }
+// The prices that a cut reckons with: an entry that was never measured takes the other one's value
+static void prices(const qw_par *p, double *lone, double *joint) {
+    for (int b = 0; b <= QW_PAR_VBMAX; b++) lone[b] = qw_par_group_cost(p, b), joint[b] = p->joint[b] > 0 ? p->joint[b] : p->cost[b];
+}
 
 // Sizes never measured, filled in on the line through the smallest and the largest measured size (one size: flat).
 // Two measured sizes close together can give the line any slope (a launch's time varies by a few per cent): a falling
@@ -55,6 +60,23 @@ static bool fill_line(const double *c, int n, double *out) {
     return true;
 }
 
+void qw_par_observe_set(qw_par *p, const int *b, int n, double ms) {
+    if (n == 1) qw_par_observe(p, b[0], ms);
+    if (n < 2 || n > QW_PAR_MAX || !(ms > 0)) return;
+    double lone[QW_PAR_VBMAX + 1], joint[QW_PAR_VBMAX + 1], full[QW_PAR_VBMAX + 1], part[QW_PAR_MAX], all = 0;
+    int rows = 0;
+    for (int i = 0; i < n; i++) {
+        if (b[i] < 1 || b[i] > QW_PAR_VBMAX) return;
+        rows += b[i];
+    }
+    prices(p, lone, joint);
+    const bool known = fill_line(p->joint, QW_PAR_VBMAX, full) || fill_line(joint, QW_PAR_VBMAX, full);
+    for (int i = 0; i < n; i++) all += part[i] = known ? full[b[i]] : 1.0 / n + (double)b[i] / rows;
+    bool had[QW_PAR_VBMAX + 1] = {false};
+    for (int i = 0; i < n; i++) // (one sample a size: those of a set are the same)
+        if (!had[b[i]]) had[b[i]] = true, observe(&p->joint[b[i]], &p->jseen[b[i]], ms * part[i] / all);
+}
+
 // One dynamic programme serves both questions (src/engine.c:8764-8797). cheapest[n]: least total of group costs c[]
 // that covers n rows; last[n]: the size of the group that completes it. Among equal totals the larger group wins.
 static void cover(const double *c, int B, double *cheapest, int *last) {
@@ -69,22 +91,35 @@ static void cover(const double *c, int B, double *cheapest, int *last) {
     }
 }
 
+// The best cut of B rows: one group by itself, or several beside one another. Returns its cost, and in *group the size that completes it (with
+// last[] what completes the rest of several); as in cover(), of equals the larger group.
+static double best_cut(const double *lone, const double *joint, int B, int *last, int *group) {
+    double cheapest[QW_PAR_MAX + 1], least = 1e30;
+    *group = 1;
+    cover(joint, B, cheapest, last);
+    for (int b = 1; b <= QW_PAR_VBMAX && b < B; b++)
+        if (cheapest[B - b] + joint[b] <= least) least = cheapest[B - b] + joint[b], *group = b;
+    if (B <= QW_PAR_VBMAX && lone[B] <= least) least = lone[B], *group = B;
+    return least;
+}
+
 double qw_par_cost(const qw_par *p, int B) { // the estimate: sizes never measured lie on the line through the measured ones
     if (B < 1) return 0;
-    double c[QW_PAR_VBMAX + 1], cheapest[QW_PAR_MAX + 1];
-    int last[QW_PAR_MAX + 1];
-    if (!fill_line(p->cost, QW_PAR_VBMAX, c)) return 0;
-    if (B > QW_PAR_MAX) B = QW_PAR_MAX;
-    cover(c, B, cheapest, last);
-    return cheapest[B] + p->step;
+    double lone[QW_PAR_VBMAX + 1], joint[QW_PAR_VBMAX + 1], l[QW_PAR_VBMAX + 1], j[QW_PAR_VBMAX + 1];
+    int last[QW_PAR_MAX + 1], group;
+    prices(p, lone, joint);
+    if (!fill_line(lone, QW_PAR_VBMAX, l) || !fill_line(joint, QW_PAR_VBMAX, j)) return 0;
+    return best_cut(l, j, B > QW_PAR_MAX ? QW_PAR_MAX : B, last, &group) + p->step;
 }
 
 int qw_par_split(const qw_par *p, int B, int *g) { // the cut: a size never measured costs 0, so that it gets tried
     if (B < 1 || B > QW_PAR_MAX) return 0;
-    double cheapest[QW_PAR_MAX + 1];
-    int last[QW_PAR_MAX + 1], ng = 0;
-    cover(p->cost, B, cheapest, last);
-    for (int n = B; n > 0; n -= last[n]) g[ng++] = last[n];
+    double lone[QW_PAR_VBMAX + 1], joint[QW_PAR_VBMAX + 1];
+    int last[QW_PAR_MAX + 1], ng = 0, group;
+    prices(p, lone, joint);
+    best_cut(lone, joint, B, last, &group);
+    g[ng++] = group;
+    for (int n = B - group; n > 0; n -= last[n]) g[ng++] = last[n];
     return ng;
 }
 

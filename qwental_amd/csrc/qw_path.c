@@ -456,9 +456,9 @@ bool qw_path_hyper_moe_stack(qw_path *p, qw_batch *b, const qw_hyper_w *H, const
 // ---------------------------------------------------------------- a ragged step (src/engine.c:8783-8814, :9138-9161, :9037)
 // Slot i brings n[i] rows; its first row is r0[i] = n[0] + ... + n[i - 1] (src/engine.c:9150-9161). The R rows are cut
 // into groups by the measured table (qw_par_split: the reference's par_split with groups of up to 16 rows), the
-// groups go through the layer one after the other (the reference's par_step, src/engine.c:8805-8812, each reading
-// the weights once), and each group's time goes back into the table (src/engine.c:9037): the device's alone, which does not depend on how many
-// groups the step has. What the host adds comes once a step, and goes back as that.
+// groups go through the layer (the reference's par_step, src/engine.c:8805-8812, each reading the weights of its experts once), one after the
+// other or in sets side by side, and the times go back into the table (src/engine.c:9037): the device's alone, of a group that ran by
+// itself as its own, of a set as that of the groups in it (qw_par_observe_set). What the host adds comes once a step, and goes back as that.
 bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int *n, int B, const qw_buf *x, const qw_buf *out, qw_vstep_info *info) {
     if (!p || !par || !M || !n || !x || !out || B < 1 || B > QW_PAR_MAX) return false;
     int R = 0, r0[QW_PAR_MAX];
@@ -511,11 +511,12 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
         if (!rec || t < 0) return false;
         gpu = t * 1e3, wall = (qw_now() - t0) * 1e3;
         bool stamped = true;
-        for (int gi = 0; gi < ng; gi++) stamped = stamped && part[gi] > 0;
-        // Without stamps of their own (groups that ran together, a front launch that takes none) the groups share the batch's time, a share being what
-        // a group takes by itself to first order: a part that does not depend on its rows, as long as eight rows' reads take, and one that does.
-        for (int gi = 0; gi < ng; gi++) sum += part[gi] = stamped ? part[gi] * 1e3 : gpu * (8 + grp[gi]) / (8 * ng + R);
-        for (int gi = 0; gi < ng; gi++) qw_par_observe(par, grp[gi], part[gi]);
+        for (int gi = 0; gi < ng; gi++) stamped = stamped && part[gi] != 0, sum += part[gi] > 0 ? part[gi] * 1e3 : 0;
+        if (!stamped) sum = gpu; // (a front launch that takes no stamp: the batch's time, as that of one set)
+        for (int gi = 0, e; gi < ng; gi = e) {
+            for (e = gi + 1; e < ng && (!stamped || part[e] < 0); e++) {}
+            qw_par_observe_set(par, grp + gi, e - gi, stamped ? part[gi] * 1e3 : gpu);
+        }
         qw_par_observe_step(par, wall - sum);
         if (info) info->gpu_ms = gpu, info->wall_ms = wall;
         return true;

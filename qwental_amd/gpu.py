@@ -108,7 +108,7 @@ SYMBOLS = [
     ("qw_gguf_hyper", _b, [_vp, _i, _i, C.POINTER(QwHyperW), _pi, C.c_char_p, _sz]),
     ("qw_gguf_tensor_at", _b, [_vp, _pg, _pt]), ("qw_gguf_moe_layer", _b, [_vp, _i, _pm, _pi, _pi, _pi, C.c_char_p, _sz]),
     # qw_par.h
-    ("qw_par_new", _vp, []), ("qw_par_free", None, [_vp]), ("qw_par_observe", None, [_vp, _i, _d]), ("qw_par_group_cost", _d, [_vp, _i]),
+    ("qw_par_new", _vp, []), ("qw_par_free", None, [_vp]), ("qw_par_observe", None, [_vp, _i, _d]), ("qw_par_observe_set", None, [_vp, _pi, _i, _d]), ("qw_par_group_cost", _d, [_vp, _i]), ("qw_par_joint_cost", _d, [_vp, _i]),
     ("qw_par_observe_step", None, [_vp, _d]), ("qw_par_step_cost", _d, [_vp]),
     ("qw_par_cost", _d, [_vp, _i]), ("qw_par_split", _i, [_vp, _i, _pi]), ("qw_par_observe_packed", None, [_vp, _i, _d]),
     ("qw_par_packed_cost", _d, [_vp, _i]), ("qw_par_choose", _b, [_vp, _i, _pi, _pi]),
@@ -597,6 +597,12 @@ class Par:
 
     def observe(self, b, ms):
         self.L.qw_par_observe(self.p, b, ms)
+
+    def observe_set(self, sizes, ms):
+        self.L.qw_par_observe_set(self.p, (C.c_int * len(sizes))(*sizes), len(sizes), ms)
+
+    def joint_cost(self, b):
+        return self.L.qw_par_joint_cost(self.p, b)
 
     def observe_step(self, ms):
         self.L.qw_par_observe_step(self.p, ms)

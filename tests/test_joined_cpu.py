@@ -8,6 +8,7 @@ import pytest
 
 import hostrt
 import test_gpu_joined
+import qwental_amd as q
 from qwental_amd import build
 
 NAMES = r"""
@@ -180,3 +181,130 @@ def test_which_launches_a_step_makes(tmp_path):
         assert [k for k, _, _ in made] == want, (step, cut)
         for k, _, per in made:
             assert (per is not None) == k.endswith("_j")
+
+
+# A device on which groups side by side take F + sum(a + r rows), one by itself F + a + r rows: steps of `rows` again and again, then the cut of each
+PLANNED = r"""
+static double F, A, Rr;
+static void on_launch(const char *fname, unsigned gx, unsigned bx, const void *args) {
+    (void)gx, (void)bx;
+    if (strncmp(fname, "qwk_gu", 6)) return;
+    const bool joint = fname[strlen(fname) - 1] == 'j' && fname[strlen(fname) - 2] == '_';
+    const qwk_gu_args *a = args;
+    const unsigned *gxs = (const unsigned *)(a + QW_JOIN_MAX);
+    double t = F;
+    for (unsigned j = 0; j < (joint ? QW_JOIN_MAX : 1); j++) t += joint && !gxs[j] ? 0 : A + Rr * a[j].nbr;
+    static uint32_t noise = 1; // two per cent either way
+    noise = noise * 1664525u + 1013904223u;
+    device_clock += (uint64_t)(t * 1000 * (0.98 + 0.04 * (noise >> 8) / (1 << 24)));
+}
+int main(void) {
+    qw_gpu *g = device();
+    g->repack = true;
+    qw_path *p = qw_path_open(g, 512, 256, 64, 4, 16, true);
+    qw_buf w, x, out;
+    if (!qw_hip_buf_new_device(g, (size_t)64 * 512 * 256 * 2, &w) || !qw_buf_new(g, 64 * 1024, &x) || !qw_buf_new(g, 64 * 1024, &out)) return printf("no buffers\n"), 1;
+    const qw_tensor W = {.buf = &w, .type = 21}, R = {.buf = &w, .type = 1};
+    const qw_moe_layer M = {.router = R, .sh_gate_w = R, .gate = W, .up = W, .down = W, .sh_gate = W, .sh_up = W, .sh_down = W};
+    const double layers[][3] = {@layers};
+    const int rows[] = {@rows};
+    enum { NR = sizeof rows / sizeof *rows };
+    for (size_t l = 0; l < sizeof layers / sizeof *layers; l++) {
+        F = layers[l][0], A = layers[l][1], Rr = layers[l][2];
+        qw_par *par = qw_par_new();
+        uint32_t seed = 1;
+        qw_vstep_info info;
+        for (int step = 0; step < 600; step++) {
+            seed = seed * 1664525u + 1013904223u;
+            const int n = rows[(seed >> 16) % NR], ones[64] = {[0 ... 63] = 1};
+            if (!qw_path_par_vstep(p, par, &M, ones, n, &x, &out, &info)) return printf("%s\n", g->err), 1;
+        }
+        for (int i = 0; i < NR; i++) {
+            int cut[64];
+            const int ng = qw_par_split(par, rows[i], cut);
+            printf("%.6g ", (qw_par_cost(par, rows[i]) - qw_par_step_cost(par)) * 1e3);
+            for (int k = 0; k < ng; k++) printf("%d ", cut[k]);
+            printf("\n");
+        }
+        qw_par_free(par);
+    }
+    return 0;
+}
+"""
+
+
+def test_the_cut_and_the_estimate_that_a_layers_times_ask_for(tmp_path):
+    """Layers whose groups cost from next to nothing to 120 rows' worth beside their rows, in steps of one group, of one set and of several."""
+    layers, rows = [(1, 2, 5), (1, 20, 2.5), (10, 4, 0.5), (1, 60, 0.5), (40, 10, 0.25)], [2, 5, 16, 18, 20, 31, 45, 64]
+    out = hostrt.run(tmp_path, PLANNED.replace("@layers", ", ".join("{%g, %g, %g}" % l for l in layers)).replace("@rows", ", ".join(map(str, rows)))).splitlines()
+    made = iter([list(map(float, line.split())) for line in out])
+    for F, a, r in layers:
+        for R in rows:
+            estimate, *cut = next(made)
+            time = lambda sizes: sum(F for i in range(0, len(sizes), 4)) + sum(a + r * b for b in sizes)  # (no time depends on the order)
+            assert sum(cut) == R
+            # as good as the fewest groups, which is the best there is (a group's cost beside its rows is never negative)
+            assert time(cut) <= 1.04 * time([16] * (R // 16) + [R % 16] * (R % 16 > 0)), (F, a, r, cut)
+            # a group by itself: its own time; groups side by side: what they share is priced as in the sets that its sizes came in
+            assert estimate == pytest.approx(time(cut), rel=0.03, abs=F if len(cut) > 1 else 0), (F, a, r, cut)
+
+
+def test_times_of_sets_in_the_planners_table():
+    p = q.Par()
+    p.observe_set([12, 12, 8], 1e6)      # the first sample of a size is dropped, as of a group by itself
+    assert [p.joint_cost(b) for b in (12, 8)] == [0, 0] and p.cost(20) == 0
+    p.observe_set([12, 12, 8], 60.0)     # nothing known: half evenly, half by rows; one sample a size
+    assert p.joint_cost(12) == pytest.approx(60 * (1 / 3 + 12 / 32) / 2) and p.joint_cost(8) == pytest.approx(60 * (1 / 3 + 8 / 32) / 2)
+    assert 2 * p.joint_cost(12) + p.joint_cost(8) == pytest.approx(60.0)
+    before = p.joint_cost(12), p.joint_cost(8)
+    p.observe_set([12, 12, 8], 120.0)    # in proportion to what is known
+    assert p.joint_cost(12) == pytest.approx(1.1 * before[0]) and p.joint_cost(8) == pytest.approx(1.1 * before[1])
+    assert p.group_cost(12) == p.joint_cost(12)  # never by itself
+    for bad in ([], [0, 4], [17, 4], [4] * 65):
+        p.observe_set(bad, 10.0)
+    p.observe_set([12, 8], -1.0)
+    p.observe_set([12, 8], 0.0)
+    assert p.joint_cost(12) == pytest.approx(1.1 * before[0]) and p.joint_cost(4) == 0
+    for _ in range(2):
+        p.observe_set([5], 7.0)          # a set of one is a group by itself
+    assert p.group_cost(5) == 7.0 and p.joint_cost(5) == 0
+    p.free()
+    p = q.Par()                          # sixteen rows: one group at the price of a lone one, or several at theirs
+    for b in range(1, 17):
+        for _ in range(2):
+            p.observe(b, 10.0 + b)
+    assert p.split(16) == [16] and p.cost(16) == 26.0 and p.split(18) == [16, 2]
+    for _ in range(2):
+        p.observe_set([8, 8], 24.0)
+    assert p.joint_cost(8) == 12.0 and p.group_cost(8) == 18.0
+    assert p.split(16) == [8, 8] and p.cost(16) == 24.0 and p.split(8) == [8] and p.cost(8) == 18.0
+    p.free()
+
+
+FED = r"""
+static void on_launch(const char *fname, unsigned gx, unsigned bx, const void *args) { (void)fname, (void)gx, (void)bx, (void)args; }
+int main(void) {
+    qw_gpu *g = device();
+    g->repack = true;
+    qw_path *p = qw_path_open(g, 512, 256, 64, 4, 16, true);
+    qw_buf w, x, out;
+    if (!qw_hip_buf_new_device(g, (size_t)64 * 512 * 256 * 2, &w) || !qw_buf_new(g, 64 * 1024, &x) || !qw_buf_new(g, 64 * 1024, &out)) return printf("no buffers\n"), 1;
+    const qw_tensor W = {.buf = &w, .type = 21}, R = {.buf = &w, .type = 1};
+    const qw_moe_layer M = {.router = R, .sh_gate_w = R, .gate = W, .up = W, .down = W, .sh_gate = W, .sh_up = W, .sh_down = W};
+    qw_par *par = qw_par_new();
+    for (int b = 1; b <= 16; b++)
+        for (int i = 0; i < 2; i++) qw_par_observe(par, b, b == 12 ? 1e-9 : 50);
+    const int ones[60] = {[0 ... 59] = 1};
+    qw_vstep_info info;
+    for (int step = 0; step < 400; step++)
+        if (!qw_path_par_vstep(p, par, &M, ones, 60, &x, &out, &info) || info.ngroups != 5) return printf("%d groups: %s\n", info.ngroups, g->err), 1;
+    printf("%.6g %.6g %.6g", qw_par_group_cost(par, 12), qw_par_joint_cost(par, 12), info.gpu_ms);
+    return 0;
+}
+"""
+
+
+def test_a_set_has_its_own_time_and_so_has_the_group_left_over(tmp_path):
+    """Five groups of twelve: four of them as three launches of ten nanoseconds, the fifth as three of its own."""
+    alone, beside, step = map(float, hostrt.run(tmp_path, FED).split())
+    assert alone == pytest.approx(3e-5, rel=1e-3) and beside == pytest.approx(3e-5 / 4, rel=1e-3) and step == pytest.approx(6e-5, rel=1e-3)
