@@ -24,6 +24,7 @@ struct qw_path {
     uint64_t flush_mask; // bit l: submit what is recorded after layer l of a stack (src/engine.c:142, :5997 vb_flush)
     qw_buf vlg, vsel;    // logits and selection record of one group of a ragged step (qw_path_par_vstep), made at first use
     qw_buf vset;         // and all that a group needs, for each of the others that go through the layer together
+    bool vset_refused;   // there was no memory for it: not asked for again, step after step
     // Kernels by what their names are made of (kernel_memo): the names are text, and three of them printed and looked up a
     // dispatch were most of what recording a layer cost (24 layers, 72 launches: 108 us with the names and a search of all
     // tile-major copies, 30 without; all of a batch is recorded before its first launch goes out)
@@ -492,7 +493,8 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
         size_t at[5], set = 0;
         for (int i = 0; i < 5; i++) at[i] = set, set += (sz[i] + 255) & ~(size_t)255;
         bool sets = ng > 1 && p->device_scratch;
-        if (sets && !p->vset.handle) sets = qw_hip_buf_new_device(p->g, (QW_JOIN_MAX - 1) * set, &p->vset); // (no memory for it: one after the other)
+        if (sets && !p->vset.handle) p->vset_refused = p->vset_refused || !qw_hip_buf_new_device(p->g, (QW_JOIN_MAX - 1) * set, &p->vset);
+        sets = sets && !p->vset_refused; // (otherwise one after the other)
         const double t0 = qw_now();
         qw_batch *b = qw_batch_begin(p->g, false);
         if (!b) return false;

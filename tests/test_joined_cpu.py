@@ -308,3 +308,43 @@ def test_a_set_has_its_own_time_and_so_has_the_group_left_over(tmp_path):
     """Five groups of twelve: four of them as three launches of ten nanoseconds, the fifth as three of its own."""
     alone, beside, step = map(float, hostrt.run(tmp_path, FED).split())
     assert alone == pytest.approx(3e-5, rel=1e-3) and beside == pytest.approx(3e-5 / 4, rel=1e-3) and step == pytest.approx(6e-5, rel=1e-3)
+
+
+NO_MEMORY = r"""
+static unsigned joint;
+static void on_launch(const char *fname, unsigned gx, unsigned bx, const void *args) { (void)gx, (void)bx, (void)args, joint += !strncmp(fname + strlen(fname) - 2, "_j", 2); }
+int main(void) {
+    qw_gpu *g = device();
+    g->repack = true;
+    qw_path *p = qw_path_open(g, 512, 256, 64, 4, 16, true);
+    qw_buf w, x, out;
+    if (!qw_hip_buf_new_device(g, (size_t)64 * 512 * 256 * 2, &w) || !qw_buf_new(g, 64 * 1024, &x) || !qw_buf_new(g, 64 * 1024, &out)) return printf("no buffers\n"), 1;
+    const qw_tensor W = {.buf = &w, .type = 21}, R = {.buf = &w, .type = 1};
+    const qw_moe_layer M = {.router = R, .sh_gate_w = R, .gate = W, .up = W, .down = W, .sh_gate = W, .sh_up = W, .sh_down = W};
+    const int ones[64] = {[0 ... 63] = 1};
+    for (int step = 0; step < 6; step++) {
+        qw_vstep_info info;
+        qw_par *par = qw_par_new();
+        if (!qw_path_par_vstep(p, par, &M, ones, step ? 40 : 16, &x, &out, &info)) return printf("step %d: %s\n", step, g->err), 1;
+        qw_par_free(par);
+        allocations_left = step >= 3 ? -1 : 0; // none for the first steps of several groups
+        if (step == 1 && allocations_refused != 1) return printf("%u refused\n", allocations_refused), 1;
+    }
+    return printf("%u %u", joint, allocations_refused), 0;
+}
+"""
+
+
+def test_no_memory_for_groups_side_by_side(tmp_path):
+    """One group after the other then, and the memory is asked for once and not at every step."""
+    (tmp_path / "alloc.h").write_text("""#define _GNU_SOURCE
+#include <stdlib.h>
+static int allocations_left = -1;
+static unsigned allocations_refused;
+static inline void *tested_alloc(size_t a, size_t n) {
+    if (allocations_left == 0) return allocations_refused++, NULL;
+    return aligned_alloc(a, n);
+}
+#define aligned_alloc tested_alloc
+""")
+    assert hostrt.run(tmp_path, NO_MEMORY, "-include", str(tmp_path / "alloc.h")).split() == ["0", "1"]
