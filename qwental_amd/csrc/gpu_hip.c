@@ -165,6 +165,7 @@ struct qw_batch {
     int nparts, part_l[QW_PARTS_MAX]; // qw_hip_batch_part: the first launch of every part,
     double part_work[QW_PARTS_MAX];   // and its work beside the others'
     int part_join;       // parts that come in sets of so many whose parts touch nothing of each other's (0: not known)
+    bool copies_to_come, copies_made; // tile-major copies that a dispatch did without, since they are not due yet, and that were made for one
     double *part_s;      // where the seconds of the parts go (qw_hip_batch_end_parts)
     hipEvent_t *pev;      // profiling: 2 events per launch
     int npev;
@@ -1537,7 +1538,11 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
     }
     const size_t bytes = (size_t)ntiles * nblk * pack_of(fmt).slab;
     const qw_want key = {.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .fmt = fmt};
-    if (beside && !copy_due(g, &key, bytes)) return NULL;
+    if (beside && !copy_due(g, &key, bytes)) {
+        const int i = want_find(g, &key);
+        if (i >= 0 && !g->wants[i].refused) b->copies_to_come = true;
+        return NULL;
+    }
     for (int i = 0; i < 2; i++)
         if (hs[i] && hs[i]->dirty && hs[i]->host) { // what the next submit would do for this buffer
             if (hipMemcpyAsync(hs[i]->dptr, hs[i]->host, hs[i]->size, hipMemcpyHostToDevice, g->stream[b->stream]) != hipSuccess) return NULL;
@@ -1565,6 +1570,7 @@ static const uint8_t *get_pack(qw_batch *b, uint32_t fmt, qw_hbuf *ha, const voi
     }
     g->packs[g->npacks++] = (qw_pack){.A = A, .B = B, .ha = ha, .hb = hb, .ntiles = ntiles, .nblk = nblk, .fmt = fmt, .split = split, .dst = dst, .bytes = bytes, .beside = beside, .pf = pf};
     g->pack_bytes += bytes;
+    b->copies_made = true;
     if (beside) {
         g->beside_bytes += bytes;
         const int i = want_find(g, &key);
@@ -3077,6 +3083,8 @@ void qw_hip_batch_part(qw_batch *b, double work) {
     if (b->nparts < QW_PARTS_MAX) b->part_work[b->nparts] = work, b->part_l[b->nparts++] = b->nl;
 }
 void qw_hip_batch_join(qw_batch *b, int n) { b->part_join = n < (int)QW_JOIN_MAX ? n : (int)QW_JOIN_MAX; }
+bool qw_hip_batch_copies_to_come(const qw_batch *b) { return b->copies_to_come; }
+bool qw_hip_batch_copies_made(const qw_batch *b) { return b->copies_made; }
 double qw_hip_batch_end_parts(qw_batch *b, double *secs) {
     for (int k = 0; k < b->nparts; k++) secs[k] = 0;
     b->part_s = secs;

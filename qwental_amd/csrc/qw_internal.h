@@ -38,6 +38,10 @@ QW_INTERNAL bool qw_hip_parts_ok(const qw_gpu *g);
 QW_INTERNAL void qw_hip_batch_part(qw_batch *b, double work);
 /* Of any n parts in a row (at most QW_JOIN_MAX) none touches what another writes: the launches of up to n in a row, from any one on, may go out together. */
 QW_INTERNAL void qw_hip_batch_join(qw_batch *b, int n);
+/* What the dispatches recorded so far did without a tile-major copy that will be made once its weights have come often enough (other kernels run from
+ * then on), or had one made (the recording took as long as that). */
+QW_INTERNAL bool qw_hip_batch_copies_to_come(const qw_batch *b);
+QW_INTERNAL bool qw_hip_batch_copies_made(const qw_batch *b);
 QW_INTERNAL double qw_hip_batch_end_parts(qw_batch *b, double *secs);
 
 #ifdef __cplusplus

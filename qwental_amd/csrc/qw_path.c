@@ -460,6 +460,8 @@ bool qw_path_hyper_moe_stack(qw_path *p, qw_batch *b, const qw_hyper_w *H, const
 // groups go through the layer (the reference's par_step, src/engine.c:8805-8812, each reading the weights of its experts once), one after the
 // other or in sets side by side, and the times go back into the table (src/engine.c:9037): the device's alone, of a group that ran by
 // itself as its own, of a set as that of the groups in it (qw_par_observe_set). What the host adds comes once a step, and goes back as that.
+// Times of a step in which tile-major copies were still to come do not: other kernels run once they are there, and a size that had its time
+// taken before would not be tried again.
 bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int *n, int B, const qw_buf *x, const qw_buf *out, qw_vstep_info *info) {
     if (!p || !par || !M || !n || !x || !out || B < 1 || B > QW_PAR_MAX) return false;
     int R = 0, r0[QW_PAR_MAX];
@@ -509,32 +511,36 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
             rec = gg_moe_at(p, b, M, grp[gi], x, (size_t)c * (size_t)p->D * 2, &s, out, (size_t)c * (size_t)p->D * 2, false);
         }
         if (sets) qw_hip_batch_join(b, QW_JOIN_MAX);
+        const bool passing = qw_hip_batch_copies_to_come(b), made = qw_hip_batch_copies_made(b);
         const double t = qw_hip_batch_end_parts(b, part);
         if (!rec || t < 0) return false;
         gpu = t * 1e3, wall = (qw_now() - t0) * 1e3;
         bool stamped = true;
         for (int gi = 0; gi < ng; gi++) stamped = stamped && part[gi] != 0, sum += part[gi] > 0 ? part[gi] * 1e3 : 0;
         if (!stamped) sum = gpu; // (a front launch that takes no stamp: the batch's time, as that of one set)
-        for (int gi = 0, e; gi < ng; gi = e) {
+        for (int gi = 0, e; gi < ng && !passing; gi = e) {
             for (e = gi + 1; e < ng && (!stamped || part[e] < 0); e++) {}
             qw_par_observe_set(par, grp + gi, e - gi, stamped ? part[gi] * 1e3 : gpu);
         }
-        qw_par_observe_step(par, wall - sum);
+        if (!passing && !made) qw_par_observe_step(par, wall - sum);
         if (info) info->gpu_ms = gpu, info->wall_ms = wall;
         return true;
     }
+    bool passing = false, made = false;
     const moe_scratch s = {.lg = &p->vlg, .sel = &p->vsel, .H = &p->H, .psh = &p->psh, .pd = &p->pd};
     for (int gi = 0, c = 0; gi < ng; c += grp[gi++]) {
         const double t0 = qw_now();
         qw_batch *b = qw_batch_begin(p->g, false);
         if (!b) return false;
         const bool rec = gg_moe_at(p, b, M, grp[gi], x, (size_t)c * (size_t)p->D * 2, &s, out, (size_t)c * (size_t)p->D * 2, false);
+        const bool to_come = qw_hip_batch_copies_to_come(b);
+        passing |= to_come, made |= qw_hip_batch_copies_made(b);
         const double t = qw_batch_end(b);
         if (!rec || t < 0) return false;
-        qw_par_observe(par, grp[gi], t * 1e3);
+        if (!to_come) qw_par_observe(par, grp[gi], t * 1e3);
         gpu += t * 1e3, wall += (qw_now() - t0) * 1e3;
     }
-    qw_par_observe_step(par, wall - gpu);
+    if (!passing && !made) qw_par_observe_step(par, wall - gpu);
     if (info) info->gpu_ms = gpu, info->wall_ms = wall;
     return true;
 }
