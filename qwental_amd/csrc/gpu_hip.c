@@ -1,6 +1,6 @@
 // HIP implementation of the GPU interface in include/gpu.h (the reference's src/gpu.h, implemented there by
-// src/gpu_metal.m). C23 over the HIP runtime's C API; the gfx950 code object built from kernels/qw_kernels.hip is
-// embedded below and loaded with hipModuleLoadData. No kernel is compiled at run time.
+// src/gpu_metal.m). C23 over the HIP runtime's C API; the gfx950 code objects built from kernels/qw_kernels.hip are
+// embedded below and in qw_joined.c and loaded with hipModuleLoadData. No kernel is compiled at run time.
 //
 // What a dispatch means here: callers record dispatches in Metal terms (kernel by name, sticky bindings by index,
 // grid in threadgroups of 32-wide SIMD groups). Each kernel name was registered by qw_gpu_compile() from the
@@ -513,7 +513,12 @@ const char *qw_hip_last_error(const qw_gpu *g) { return g->err; }
 int qw_hip_cu_count(const qw_gpu *g) { return g->ncu; }
 const char *qw_hip_arch(void) { return "gfx950"; }
 
-// Kernels that have a form for several launches in one (name + "_j"): what the layers of a ragged step are made of
+// Kernels that have a form for several launches in one (name + "_j"): what the layers of a ragged step are made of. Groups one after the other ->
+// side by side, us a step of three groups of 15 rows (512 experts of 2048 x 512): IQ3_S 176 -> 160, Q8_0 301 -> 231, Q4_K with Q6_K 234 -> 200, gate/up
+// rows in IQ4_XS (qwk_gu_rt) 226 -> 207, IQ4_NL down rows (2560 x 640) 271 -> 217; 64 experts in Q8_0 146 -> 95, in GGUF order (qwk_gu_f8_c16) 177 -> 124;
+// 128 of 1024 x 256 in IQ3_S 72 -> 50; four groups of four rows 116 -> 83, 156 -> 118, 146 -> 102, 137 -> 103, 167 -> 97, 122 -> 71, 142 -> 91, 70 -> 39.
+// No cut of two to six groups in any of these formats takes longer side by side. Forms that nothing here names (Q6_K down rows of less than 64 MB,
+// D not a multiple of 512, one row a group) have not been made: such groups run one after the other.
 static const char *const joinable[] = {
     "qwk_pre_w1_s121", "qwk_pre_w1_s8", "qwk_pre_w1_kq", "qwk_pre_w30_s121", "qwk_pre_w30_s8", "qwk_pre_w30_kq",
     "qwk_gu_f121_c2", "qwk_gu_f8_c16", "qwk_gu_f108_c2", "qwk_gu_f112_c2", "qwk_gu_rt",
@@ -2751,7 +2756,7 @@ static bool host_write_ok(const qw_batch *b, const qw_hbuf *h, bool last) { retu
 // Neighbouring parts of a batch that touch nothing of each other's (qw_hip_batch_join): where they are the same kernels launch for launch, and
 // all of these have a form for several launches in one, the k-th launches of up to part_join parts go out as one, at the place of the first
 // part's. All or none: a part of which only some launches ran with another part's would have no time of its own for what it could not share.
-// Three groups of 15 tokens (benchmark's layer, IQ3_S, us): front 3 x 5.3 -> 10.4, gate/up 3 x 32.4 -> 73.7, down + combine 3 x 26.9 -> 72.3.
+// Three groups of 15 tokens (512 experts of 2048 x 512, IQ3_S, us): front 3 x 5.3 -> 10.4, gate/up 3 x 32.4 -> 73.7, down + combine 3 x 26.9 -> 72.3.
 // Grids: those that follow from the shape stay; gate/up and down by ranges deal their tiles over whatever grid they get, and get the compute
 // units shared out (share_units).
 static bool same_launch(const qw_launch *l, const qw_launch *f) {
@@ -2773,6 +2778,7 @@ static void share_units(unsigned units, const double *work, int m, unsigned *sha
         int at = 0;
         for (int j = 1; j < m; j++)
             if (left < 0 ? share[j] > share[at] : work[j] * (units / 8) / all - share[j] > work[at] * (units / 8) / all - share[at]) at = j;
+        if (left < 0 && share[at] == 1) break; // (a device of less than eight units a part)
         share[at] += left < 0 ? -1 : 1;
     }
     for (int j = 0; j < m; j++) share[j] *= 8;

@@ -368,3 +368,30 @@ static inline void *tested_alloc(size_t a, size_t n) {
 #define aligned_alloc tested_alloc
 """)
     assert hostrt.run(tmp_path, NO_MEMORY, "-include", str(tmp_path / "alloc.h")).split() == ["0", "1"]
+
+
+SHARES = r"""
+static void on_launch(const char *fname, unsigned gx, unsigned bx, const void *args) { (void)fname, (void)gx, (void)bx, (void)args; }
+int main(void) {
+    uint32_t seed = 7;
+    for (unsigned units = 16; units <= 304; units += 16)
+        for (int i = 0; i < 2000; i++) {
+            const int m = 2 + i % 3;
+            double work[4], all = 0;
+            unsigned share[4], sum = 0;
+            for (int j = 0; j < m; j++) all += work[j] = 1 + ((seed = seed * 1664525u + 1013904223u) >> 22) % (i % 7 ? 200 : 1000);
+            share_units(units, work, m, share);
+            for (int j = 0; j < m; j++) {
+                sum += share[j];
+                if (!share[j] || share[j] % 8 || (units >= 64 && share[j] + 16 < units * work[j] / all)) return printf("%u units, %d parts: %u\n", units, m, share[j]), 1;
+            }
+            if (units / 8 >= (unsigned)m && sum != units) return printf("%u units, %d parts: %u in all\n", units, m, sum), 1;
+        }
+    return 0;
+}
+"""
+
+
+def test_every_part_gets_compute_units(tmp_path):
+    """All of them are shared out, in eights, about as the work asks; and none goes without, however few there are."""
+    hostrt.run(tmp_path, SHARES)
