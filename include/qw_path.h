@@ -82,11 +82,13 @@ void qw_path_set_flush(qw_path *p, uint64_t mask);
  * and qw_engine_par_step, :8798-8814): slot i contributes n[i] >= 1 consecutive rows of x [R][D] (binary16), its first row
  * being r0[i] = n[0] + ... + n[i - 1]; R = sum n[i] <= QW_PAR_MAX. The rows are cut into groups of at most 16 by par's
  * measured table (qw_par_split), each group runs the layer (the weights of the experts it picks are read once per group)
- * into the same rows of out [R][D], all groups in one batch, and the time of every group is fed back to par: the device's from
- * the group's first launch to the next group's (qw_par_observe; the first sample of a size is dropped, as src/engine.c:9037 does), or where
- * up to four groups of like sizes run side by side (a path opened with device scratch) a share of the batch's, by 8 + rows; and
- * what the host added to the step (qw_par_observe_step). The first step of several groups takes scratch for the three further ones (a few MB). On a device under qw_profile_enable it is a batch a group, with the same two figures. A row's result does not depend on
- * the group it falls into (bit for bit). The path must have been opened for 16 tokens. info (may be NULL) receives the cut.
+ * into the same rows of out [R][D], all groups in one batch, and the times are fed back to par: the device's, from
+ * a group's first launch to the next group's (qw_par_observe; the first sample of a size is dropped, as src/engine.c:9037 does), or where
+ * up to four neighbouring groups run side by side that of the set (qw_par_observe_set), and
+ * what the host added to the step (qw_par_observe_step). Steps that run without tile-major copies which are still to come feed nothing back.
+ * Groups run side by side in a path opened with device scratch, where the kernels are the same launch for launch and have a form for it; the first
+ * step of several groups takes scratch for three further ones (a few MB; without that memory the groups run one after the other). On a device under
+ * qw_profile_enable it is a batch a group. A row's result does not depend on the group it falls into (bit for bit), nor on what ran beside it. The path must have been opened for 16 tokens. info (may be NULL) receives the cut.
  * The packing path (qw_path_pf_moe) is the other form of such a step when the routing is known to the caller;
  * qw_par_choose() weighs the two. */
 typedef struct {

@@ -487,9 +487,9 @@ bool qw_path_par_vstep(qw_path *p, qw_par *par, const qw_moe_layer *M, const int
     double gpu = 0, wall = 0;
     if (qw_hip_parts_ok(p->g)) {
         // All groups in one batch: one upload, one wait, the rows written to the host by the last launches. Up to QW_JOIN_MAX groups go through the
-        // layer side by side, each in a scratch set of its own (the last one in the path's own), three launches for all of them.
-        // (A batch a group, each waited for: 232.9 us for sixteen slots and 45 rows of the benchmark's layer; one batch, one group after the other
-        // 207.9, and on another box 198.2 against 174.2 side by side.)
+        // layer side by side, each in a scratch set of its own (the last one in the path's own; any four in a row have different ones), three
+        // launches for all of them. (A batch a group, each waited for: 232.9 us for sixteen slots and 45 rows of 512 experts of 2048 x 512, IQ3_S;
+        // one batch, one group after the other 207.9; in turn on one device 206.7 against 186.3 side by side.)
         double part[QW_PAR_MAX], sum = 0;
         const size_t sz[5] = {qw_path_logits_bytes(p, QW_PAR_VBMAX), qw_path_sel_bytes(p, QW_PAR_VBMAX), p->H.size, p->psh.size, p->pd.size};
         size_t at[5], set = 0;
